@@ -6,7 +6,7 @@
 //   gemm_tiled.hip : BM x BN block tiles through two LDS stages
 //   gemm_pipe.hip  : 256x256 tile, one wave per SIMD, explicit software pipeline
 //   gemm_stream.hip: the same pipeline running across tile boundaries, epilogue under the
-//                    next tile's MFMAs (M, N, K multiples of 128); with a split over K for
+//                    next tile's MFMAs (any M; N, K multiples of 128); with a split over K for
 //                    outputs of few tiles, summed by splitk_reduce_kernel below
 //   here           : generic one-wave-per-32x32-tile kernel for any M, N, K % 16 == 0
 #include "gemm_common.h"
@@ -97,7 +97,7 @@ static const Variant kVariants[] = {
     {"128x128x128 4 waves (64x64 per wave)", 128, 128, 256, 0.70f},
     {"256x256x128 4 waves, software-pipelined, persistent (K % 256 == 0)", 256, 256, 256, 1.10f},
     {"256x256x128 4 waves, software-pipelined, one tile per block", 256, 256, 256, 0.50f},
-    {"256x256x128 4 waves, streaming across tiles, folded epilogue (M, N, K multiples of 128)", 256, 256, 256, 1.25f},
+    {"256x256x128 4 waves, streaming across tiles, folded epilogue (N, K multiples of 128)", 256, 256, 256, 1.25f},
 };
 constexpr int kPipeVariant = 5, kPipeOneTileVariant = 6, kStreamVariant = 7;
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
@@ -216,7 +216,7 @@ extern "C" int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, in
     const bool lim32 = (double)(M + 256) * (double)K < 2147483648.0 && (double)(N + 256) * (double)K < 2147483648.0;
     // C = C + product is an epilogue of the kernels whose tiles end in a separate output phase; the streaming kernel
     // stores a tile under the next tile's MFMAs, where nothing can wait for the old values of C
-    const bool stream_ok = tiled_ok && lim32 && M % 128 == 0 && N % 128 == 0 && K >= 512 && !accumulate;
+    const bool stream_ok = tiled_ok && lim32 && N % 128 == 0 && K >= 512 && !accumulate;
     int variant = t_forced_variant >= 0 ? t_forced_variant : (tiled_ok ? choose_variant(M, N, stream_ok) : 0);
     if (variant != 0 && !tiled_ok) variant = 0;
     // the pipelined kernel walks K in pairs of 128-byte steps
@@ -236,7 +236,7 @@ extern "C" int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, in
     g.tiles_m = (int)tm; g.tiles_n = (int)tn;
 
     if (variant == kStreamVariant && !(stream_ok && gemm_stream_accepts(g))) {
-        // the streaming kernel wants M, N in multiples of 128: next best kernel instead
+        // the streaming kernel wants N in multiples of 128: next best kernel instead
         variant = pipe_ok ? kPipeVariant : 2;
     }
     if (variant == 0) launch_gemm_generic(fmt_a, fmt_b, g, stream);
@@ -315,9 +315,9 @@ extern "C" int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t 
     g.out_dtype = out_dtype;
     g.ta = layout_a == ODL_K_SLOW;
     g.tb = layout_b == ODL_K_SLOW;
-    const bool sizes_ok = M > 0 && N > 0 && K >= 512 && M % 256 == 0 && N % 256 == 0 && K % 256 == 0 &&
+    const bool sizes_ok = M > 0 && N > 0 && K >= 512 && M % 256 == 0 && N % 256 == 0 && K % 128 == 0 &&
                           (double)(M + 256) * (double)K < 2147483648.0 && (double)(N + 256) * (double)K < 2147483648.0;
-    if (!sizes_ok) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_layouts: M, N, K must be multiples of 256 (K >= 512) and each operand under 2 GiB; got %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
+    if (!sizes_ok) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_layouts: M, N must be multiples of 256, K of 128 (K >= 512) and each operand under 2 GiB; got %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
     g.tiles_m = (int)(M / 256); g.tiles_n = (int)(N / 256);
     if (!gemm_stream_accepts(g)) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_layouts: shape not taken by the streaming kernel");
     attach_clock_probe(g);

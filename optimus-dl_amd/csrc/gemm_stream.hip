@@ -1,7 +1,7 @@
 // FP8 GEMM, 256x256 block tile, 4 waves (one per SIMD, 128x128 each), persistent,
 // with the epilogue of every tile folded under the first MFMAs of the next one.
 // C = (A[M,K] . B[N,K]^T) * (sa_inv * sb_inv) (+ bias) in bf16 or fp32, for the shapes training uses:
-// M % 128 == 0, N % 128 == 0, K % 128 == 0, K >= 512; scales per tensor or per row of A / B.
+// any M, N % 128 == 0, K % 128 == 0, K >= 512; scales per tensor or per row of A / B (block scales: M % 128 == 0).
 // Everything else goes to gemm_pipe.hip, whose K step this kernel shares:
 //
 //   per K step of 128 bytes (two halves h0, h1 of 64 bytes = one MFMA K each)
@@ -322,7 +322,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
 
     // ---- output side of the folded epilogue
     const int n2 = (int)g.N * ESZ;                // bytes per output row
-    const int c_soff0 = (wm0 * (int)g.N + wn0) * ESZ;
+    const int c_off0 = (wm0 * (int)g.N + wn0) * ESZ;
     auto uniform = [](float v) { return bits_to_float((uint32_t)__builtin_amdgcn_readfirstlane((int)float_to_bits(v))); };
     // SEG: between pair s and s + 1 the accumulators take sRatio[s] = (scale product of s) / (that of s + 1); kept in
     // LDS (read once per pair) rather than in scalar registers, of which the K loop leaves none to spare
@@ -333,28 +333,34 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
     }
     const float s_tensor = g.splits > 1 ? 1.0f :       // partial results leave unscaled
         SEG ? uniform(gp.sa[gp.count - 1][0] * gp.sb[gp.count - 1][0]) : uniform(g.sa[0] * g.sb[0]);
-    // M and N are multiples of 128 = the wave tile: in the last tile row / column of a matrix that is not a
-    // multiple of 256 a wave is either wholly inside or wholly outside.  One that is outside computes on the
-    // zeros that the bounded operand loads deliver and stores through the empty descriptor (nothing is written).
+    // N is a multiple of 128 = the width of a wave tile: in the last tile column a wave is either wholly inside or wholly
+    // outside.  One that is outside computes on the zeros that the bounded operand loads deliver and stores through the
+    // empty descriptor (nothing is written).  M is free: the descriptor of the output ends behind the tile's last row
+    // inside the matrix, and the row of a store is part of its per-lane offset, which the hardware checks against that
+    // end (the scalar offset it does not check).  The last tile row costs what a whole one does and no more: 4016 tokens
+    // are 16 tile rows like 4096; before, such a product took the tiled kernels (4016 x 5632 x 2048: 92.0 us, here 48.9).
     auto wave_inside = [&](int tm0, int tn0) { return tm0 + wm0 < (int)g.M && tn0 + wn0 < (int)g.N; };
     auto rsrc_out = [&](int item, int tm0, int tn0) -> v4i {
         const int split = __builtin_amdgcn_readfirstlane(item / tiles);
         const uint64_t addr = reinterpret_cast<uint64_t>(reinterpret_cast<uint8_t *>(g.c) +
                                                          ((int64_t)split * g.M * g.N + (int64_t)tm0 * g.N + tn0) * ESZ);
-        const v4i whole = {(int)(uint32_t)addr, (int)(uint32_t)(addr >> 32), (int)0x80000000u, 0x00020000};
+        const int bytes = min((int)g.M - tm0, BM) * n2;          // < 2 GiB (checked by the caller)
+        const v4i whole = {(int)(uint32_t)addr, (int)(uint32_t)(addr >> 32), bytes, 0x00020000};
         return wave_inside(tm0, tn0) ? whole : empty;
     };
     // `us`: the slab's position in the wave tile's row, in slabs of 128 bytes
-    auto store_slab = [](const u32x4 (&data)[4], int vo, const v4i &rsrc, int so_base, int row_bytes, int t, int us) {
+    auto store_slab = [](const u32x4 (&data)[4], int vo, const v4i &rsrc, int row_bytes, int t, int us) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int so = so_base + (32 * t + 8 * j) * row_bytes + 128 * us;
+            const int at = vo + (32 * t + 8 * j) * row_bytes, so = 128 * us;
             // s_nop 4: a scalar register written by a vector instruction (the compiler restores
             // spilled scalars that way) must not be read by a vector-memory instruction for 5
             // cycles, and the compiler does not look inside asm statements for that hazard.
             // nt: the output is not an operand of the next kernel; stored normally it sits dirty in the
             // memory-side cache and its write-back competes with the amax / cast pass that follows
-            asm volatile("s_nop 4\n\tbuffer_store_dwordx4 %0, %1, %2, %3 offen nt" ::"v"(data[j]), "v"(vo), "s"(rsrc), "s"(so));
+            // the scalar offset is a register on purpose: a 16-byte store without one needs a wait state before its data
+            // registers are written again, which nobody would insert here either
+            asm volatile("s_nop 4\n\tbuffer_store_dwordx4 %0, %1, %2, %3 offen nt" ::"v"(data[j]), "v"(at), "s"(rsrc), "s"(so));
         }
     };
     auto lds_w = [](uint32_t addr) { return (__attribute__((address_space(3))) u32x2 *)addr; };
@@ -423,7 +429,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         const uint32_t slab = lds_addr_of(sEpi) + wave_e * SLAB;
         const uint32_t epi_w = slab + (lane_e % 32) * PITCH + (lane_e / 32) * (F32 ? 16 : 8);
         const uint32_t epi_r = slab + (lane_e / 8) * PITCH + (lane_e % 8) * 16;
-        const int c_voff = (lane_e / 8) * n2 + (lane_e % 8) * 16;
+        const int c_voff = c_off0 + (lane_e / 8) * n2 + (lane_e % 8) * 16;
         const uint32_t vec_row = lds_addr_of(sVec) + wave_e * VEC_BYTES + (lane_e % 32) * 4;          // sa of row lr
         const uint32_t vec_col = lds_addr_of(sVec) + wave_e * VEC_BYTES + 512 + (lane_e / 32) * 16;   // sb of columns 4 lg ..
         float sa_next = 0.0f;
@@ -467,7 +473,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
                 if (i < 15) read_vectors((i + 1) / 4, (i + 1) % 4);
             }
             if constexpr (F32) {
-                if (i > 0) store_slab(back, c_voff, rsrc_c, c_soff0, n2, (i - 1) / 4, (i - 1) % 4);
+                if (i > 0) store_slab(back, c_voff, rsrc_c, n2, (i - 1) / 4, (i - 1) % 4);
                 // lane (lr, lg) holds columns 8q + 4lg + {0..3} of row lr: 16 bytes at 32q + 16lg, as two 8-byte
                 // writes (the row pitch of 34 dwords spreads the 32 rows of a half-wave over all 64 banks)
 #pragma unroll
@@ -490,14 +496,14 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
 #pragma unroll
                     for (int j = 0; j < 4; ++j) back[j] = lds_r(epi_r + j * 8 * PITCH);
                 } else if (i > 0) {
-                    store_slab(back, c_voff, rsrc_c, c_soff0, n2, (i - 2) / 4, ((i - 2) % 4) / 2);   // completed one MFMA ago
+                    store_slab(back, c_voff, rsrc_c, n2, (i - 2) / 4, ((i - 2) % 4) / 2);   // completed one MFMA ago
                 }
             }
             if (i < 4) a1[i] = read_a(sa_cur, i, 1);
             else if (i < 8) b1[i - 4] = read_b(sb_cur, i - 4, 1);
             __builtin_amdgcn_sched_barrier(0);
         }
-        store_slab(back, c_voff, rsrc_c, c_soff0, n2, 3, F32 ? 3 : 1);
+        store_slab(back, c_voff, rsrc_c, n2, 3, F32 ? 3 : 1);
         __builtin_amdgcn_sched_barrier(0);
     };
     // EPI > 0: this wave's 128 row scales, 128 column scales (and 128 bias values) of the tile at (tm0, tn0)
@@ -510,13 +516,14 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
             return v4i{(int)(uint32_t)addr, (int)(uint32_t)(addr >> 32), (int)(count * 4), 0x00020000};
         };
         // the bounds of a descriptor cover the per-lane offset only, not the scalar one: a wave outside the matrix
-        // must not request its (non-existent) slices at all
+        // must not request its (non-existent) slices at all, and the row goes into the per-lane offset (rows past the
+        // end, in the last tile row of an M that is not a multiple of 128, read as zero)
         const bool inside = wave_inside(tm0, tn0);
         const v4i ra_ = inside ? rsrc_vec(g.sa, g.sa_vec ? g.M : 1) : empty, rb_ = inside ? rsrc_vec(g.sb, g.sb_vec ? g.N : 1) : empty;
-        const int va = lane * 4 * g.sa_vec, vb = lane * 4 * g.sb_vec;
+        const int vb = lane * 4 * g.sb_vec;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            dma4(ra_, dst + j * 256, va, (tm0 + wm0 + 64 * j) * 4 * g.sa_vec);
+            dma4(ra_, dst + j * 256, (tm0 + wm0 + 64 * j + lane) * 4 * g.sa_vec, 0);
             dma4(rb_, dst + 512 + j * 256, vb, (tn0 + wn0 + 64 * j) * 4 * g.sb_vec);
         }
         if constexpr (EPI == 2) {
@@ -727,13 +734,14 @@ void launch_fmt(const GemmArgs &g, int blocks_per_xcd, hipStream_t stream) {
 
 // Shapes this kernel takes (the caller checks the 32-bit offset limits shared with gemm_pipe.hip).
 // An operand stored [K, rows] must fill whole tiles: the loads of a partial tile would run past the
-// end of its last K-row.  One stored [rows, K] may end after half a tile (see wave_inside).
+// end of its last K-row.  Stored [rows, K], A may end anywhere and B after half a tile (see wave_inside); block
+// scales are fetched for 128 rows at a time.
 bool gemm_stream_accepts(const GemmArgs &g) {
     const double esz = (g.out_dtype == ODL_F32 || g.splits > 1) ? 4.0 : 2.0;
     const bool vectors = g.splits == 1 && (g.sa_vec || g.sb_vec || g.bias != nullptr);   // only with both operands stored [rows, K]
     if (g.mx_sa && (g.ta || g.tb || g.sa_vec || g.sb_vec || !g.mx_sb)) return false;
     return !g.accumulate && (g.out_dtype == ODL_BF16 || g.out_dtype == ODL_F32) && !(vectors && (g.ta || g.tb)) &&
-           g.M % (g.ta ? BM : WM) == 0 && g.N % (g.tb ? BN : WN) == 0 && g.K % 128 == 0 && g.K >= 512 && (double)g.N * esz * (BM + 8) < 2147483648.0;
+           g.M % (g.ta ? BM : g.mx_sa ? WM : 1) == 0 && g.N % (g.tb ? BN : WN) == 0 && g.K % 128 == 0 && g.K >= 512 && (double)g.N * esz * (BM + 8) < 2147483648.0;
 }
 
 // Operand pairs: each a whole even number of K steps, four at least (the load pipeline is two steps deep and crosses
@@ -747,7 +755,7 @@ bool gemm_stream_accepts_pairs(const GemmArgs &g, const GemmPairs &gp) {
         if (!gp.a[s] || !gp.b[s] || !gp.sa[s] || !gp.sb[s] || k < 512 || k % 256 != 0) return false;
         if ((double)(g.M + 256) * k >= 2147483648.0 || (double)(g.N + 256) * k >= 2147483648.0) return false;
     }
-    return (g.out_dtype == ODL_BF16 || g.out_dtype == ODL_F32) && g.M > 0 && g.N > 0 && g.M % WM == 0 && g.N % WN == 0 &&
+    return (g.out_dtype == ODL_BF16 || g.out_dtype == ODL_F32) && g.M > 0 && g.N > 0 && g.N % WN == 0 &&
            (double)g.N * esz * (BM + 8) < 2147483648.0;
 }
 

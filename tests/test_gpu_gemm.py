@@ -692,3 +692,34 @@ def test_sum_of_products_shape_sweep_against_the_per_pair_route(N):
             # still a hundredth of the GEMM tolerance and far below what a wrong pair, ratio or pitch would give
             ref = O.t_gemm_nt_sum(list(zip(a, b, sa, sb)), O.E5M2, O.E4M3, want_f32=True)[1]
             assert max_rel_err(one, ref) <= 1e-4, (case, M, Nn, ks)
+
+
+# ------------------------------------------------------------------ streaming kernel, rows that fill no tile
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("epilogue", ["tensor", "rowwise", "bias"])
+@pytest.mark.parametrize("M", [1, 16, 127, 129, 255, 257, 400, 1021])
+def test_streaming_kernel_any_number_of_rows(N, M, epilogue, out_dtype):
+    """The last tile row ends anywhere (inside the first 128 rows of a tile, inside the second, one row before and after
+    both edges): the bits are those of the tiled kernel, which adds in the same order, and the rows behind the matrix
+    are left alone."""
+    Nn, K = 384, 640
+    aq, _ = quantised((M, K), O.E4M3, 1.0, 90)
+    bq, _ = quantised((Nn, K), O.E4M3, 0.02, 91)
+    g = torch.Generator().manual_seed(M)
+    n_a, n_b = (1, 1) if epilogue == "tensor" else (M, Nn)
+    sa, sb = torch.rand(n_a, generator=g) + 0.5, torch.rand(n_b, generator=g) + 0.5
+    bias = torch.randn(Nn, generator=g).cuda() if epilogue == "bias" else None
+    outs = []
+    for v in (7, 4):
+        room = torch.full((M + 256, Nn), 7.0, dtype=out_dtype, device="cuda")
+        N.gemm_set_variant(v)
+        N.gemm_nt(aq.cuda(), bq.cuda(), O.E4M3, O.E4M3, sa.cuda(), sb.cuda(), bias=bias, out=room[:M])
+        assert (room[M:] == 7.0).all()
+        outs.append(room[:M])
+    N.gemm_set_variant(-1)
+    assert torch.equal(outs[0], outs[1])
+    if epilogue == "tensor":
+        summed = N.gemm_nt_sum([aq.cuda()[:, :512].contiguous()] * 2, [bq.cuda()[:, :512].contiguous()] * 2, O.E4M3, O.E4M3,
+                               [sa.cuda()] * 2, [sb.cuda()] * 2, out_dtype=out_dtype)
+        ref = O.t_gemm_nt(aq[:, :512].contiguous(), bq[:, :512].contiguous(), O.E4M3, O.E4M3, sa, sb, want_f32=True)[1]
+        assert max_rel_err(summed, 2 * ref) <= TOL
