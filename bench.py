@@ -122,9 +122,9 @@ class KernelTimer:
         wrap("amax", lambda x, *r, **kw: float(x.numel() * esz(x)))                                       # bytes
         wrap("amax_scale", lambda x, *r, **kw: float(x.numel() * esz(x)), record_as="amax")       # amax + scale, one launch
         wrap("amax_parts", lambda x, *r, **kw: float(x.numel() * esz(x)), record_as="amax")
-        wrap("cast_dynamic", lambda x, parts, fmt, margin=0, want_rowmajor=True, want_transposed=True, out_t=None:
+        wrap("cast_dynamic", lambda x, parts, fmt, margin=0, want_rowmajor=True, want_transposed=True, out_t=None, rows_out=None:
              float(x.numel() * (esz(x) + int(want_rowmajor) + int(want_transposed or out_t is not None))),
-             record_as=lambda x, parts, fmt, margin=0, want_rowmajor=True, want_transposed=True, out_t=None:
+             record_as=lambda x, parts, fmt, margin=0, want_rowmajor=True, want_transposed=True, out_t=None, rows_out=None:
              "cast_transpose" if (want_transposed or out_t is not None) else "cast")
         wrap("cast", lambda x, *r, **kw: float(x.numel() * (esz(x) + 1)))
         wrap("cast_transpose",

@@ -529,14 +529,16 @@ __device__ __forceinline__ void record_scale_inv(float s, float *__restrict__ sc
 // quarter (fp32) of each 64-byte request, and non-temporal loads are not merged across instructions: fp32 sources ran
 // at 0.49 of the HBM peak that way (4096 x 14336, bf16 0.68).  cols % 16 == 0 and 16-byte aligned pointers
 // (host-checked), so a piece never crosses a row.
+// rows_out >= rows: `out` has that many rows, the ones behind x hold zero codes (a GEMM that contracts over the rows of x
+// then runs on whole K steps whatever their number).
 template <int SRC, int FMT, int MODE, bool AMAX>
-__global__ __launch_bounds__(AMAX ? kFatThreads : kThreads) void cast_kernel(const void *__restrict__ x, int64_t rows, int64_t cols,
+__global__ __launch_bounds__(AMAX ? kFatThreads : kThreads) void cast_kernel(const void *__restrict__ x, int64_t rows, int64_t cols, int64_t rows_out,
                                                          const float *__restrict__ scale, uint8_t *__restrict__ out,
                                                          float *__restrict__ amax_out, int margin, float *__restrict__ dyn_out,
                                                          int amax_mask) {
     constexpr int kT = AMAX ? kFatThreads : kThreads;
     __shared__ uint32_t red[kT / kWave];
-    const int64_t n = rows * cols;
+    const int64_t n = rows * cols, n_out = rows_out * cols;
     float s_t = 1.0f;
     if constexpr (MODE == ODL_SCALE_TENSOR) {
         s_t = scale[0];
@@ -587,7 +589,7 @@ __global__ __launch_bounds__(AMAX ? kFatThreads : kThreads) void cast_kernel(con
     };
     const char *px = reinterpret_cast<const char *>(x);
     constexpr int ESZ = SRC == ODL_BF16 ? 2 : 4;
-    const int64_t nspan = (n + 1023) / 1024;
+    const int64_t nspan = (n_out + 1023) / 1024;
     const int64_t stride = (int64_t)gridDim.x * (kT / kWave);
     int64_t sp = (int64_t)blockIdx.x * (kT / kWave) + threadIdx.x / kWave;
     for (; sp + (U - 1) * stride < nspan; sp += U * stride) {
@@ -604,7 +606,7 @@ __global__ __launch_bounds__(AMAX ? kFatThreads : kThreads) void cast_kernel(con
 #pragma unroll
             for (int h = 0; h < VP; ++h) {
                 const int64_t e = (sp + u * stride) * 1024 + (h * kWave + lane) * EPP;
-                if (e < n) one(e, v[u][h]);
+                if (e < n_out) one(e, v[u][h]);
             }
     }
     for (; sp < nspan; sp += stride) {
@@ -617,7 +619,7 @@ __global__ __launch_bounds__(AMAX ? kFatThreads : kThreads) void cast_kernel(con
 #pragma unroll
         for (int h = 0; h < VP; ++h) {
             const int64_t e = sp * 1024 + (h * kWave + lane) * EPP;
-            if (e < n) one(e, v[h]);
+            if (e < n_out) one(e, v[h]);
         }
     }
     if constexpr (AMAX) {
@@ -629,23 +631,25 @@ __global__ __launch_bounds__(AMAX ? kFatThreads : kThreads) void cast_kernel(con
 
 // element-at-a-time cast (+ optional transposed copy) for any shape / alignment
 template <int SRC, int FMT>
-__global__ __launch_bounds__(kThreads) void cast_generic_kernel(const void *__restrict__ x, int64_t rows, int64_t cols,
+__global__ __launch_bounds__(kThreads) void cast_generic_kernel(const void *__restrict__ x, int64_t rows, int64_t cols, int64_t rows_out,
                                                                  const float *__restrict__ scale, int mode,
                                                                  uint8_t *__restrict__ out, uint8_t *__restrict__ out_t,
                                                                  float *__restrict__ amax_out) {
     __shared__ uint32_t red[kThreads / kWave];
     uint32_t am = 0;
-    const int64_t n = rows * cols;
+    const int64_t n = rows_out * cols;
     for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
         const int64_t r = i / cols, c = i % cols;
-        float f;
-        if constexpr (SRC == ODL_BF16) f = bits_to_float((uint32_t) reinterpret_cast<const uint16_t *>(x)[i] << 16);
-        else f = reinterpret_cast<const float *>(x)[i];
+        float f = 0.0f;
+        if (r < rows) {
+            if constexpr (SRC == ODL_BF16) f = bits_to_float((uint32_t) reinterpret_cast<const uint16_t *>(x)[i] << 16);
+            else f = reinterpret_cast<const float *>(x)[i];
+        }
         am = max(am, float_to_bits(f) & 0x7fffffffu);
-        const float s = mode == ODL_SCALE_TENSOR ? scale[0] : (mode == ODL_SCALE_ROW ? scale[r] : scale[c]);
+        const float s = mode == ODL_SCALE_TENSOR ? scale[0] : (mode == ODL_SCALE_ROW ? scale[min(r, rows - 1)] : scale[c]);
         const uint8_t q = (uint8_t)(quantise4<FMT>(f, 0.f, 0.f, 0.f, s, 1.f, 1.f, 1.f) & 0xffu);
         if (out) out[i] = q;
-        if (out_t) out_t[c * rows + r] = q;
+        if (out_t) out_t[c * rows_out + r] = q;
     }
     if (amax_out) {
         am = block_max_u32(am, red);
@@ -667,6 +671,8 @@ __global__ __launch_bounds__(kThreads) void cast_generic_kernel(const void *__re
 // One 128 x 64 tile (tr, tc) of x: convert, write the row-major codes, transpose through `tile` (LDS), write the
 // transposed codes.  `st` is the per-tensor scale (modes TENSOR and parts), `scale` the vector of the ROW / COL modes.
 // Ends after the transposed stores: a caller that reuses `tile` puts a barrier in between.
+// rows_out >= rows, a multiple of 16: rows of `out` and pitch of `out_t`; what lies behind x holds zero codes.  The tiles
+// read such rows as zero anyway, so the padding costs its stores only.
 // first tile column of the lane's group g (0 / 1) of 4 columns
 template <int SRC>
 __device__ __forceinline__ int ct_group_col(int tx, int g) { return SRC == ODL_BF16 ? tx * 8 + 4 * g : tx * 4 + 32 * g; }
@@ -685,9 +691,9 @@ __device__ __forceinline__ void ct_load_row(const void *__restrict__ x, int64_t 
 
 // the lane's 8 row-major codes of row r
 template <int SRC>
-__device__ __forceinline__ void ct_store_row(uint8_t *__restrict__ out, int64_t r, int64_t rows, int64_t cols, int64_t cA, int64_t cB,
+__device__ __forceinline__ void ct_store_row(uint8_t *__restrict__ out, int64_t r, int64_t rows_out, int64_t cols, int64_t cA, int64_t cB,
                                              bool okA, bool okB, uint32_t lo, uint32_t hi) {
-    if (r >= rows) return;
+    if (r >= rows_out) return;
     if constexpr (SRC == ODL_BF16) {
         if (okA) ODL_CODE_STORE((u32x2{lo, hi}), reinterpret_cast<u32x2 *>(out + r * cols + cA));
     } else {
@@ -697,7 +703,7 @@ __device__ __forceinline__ void ct_store_row(uint8_t *__restrict__ out, int64_t 
 }
 
 template <int SRC, int FMT, int MODE, bool AMAX, bool WRITE_ROWMAJOR>
-__device__ __forceinline__ void ct_one_tile(const void *__restrict__ x, int64_t rows, int64_t cols, const float *__restrict__ scale,
+__device__ __forceinline__ void ct_one_tile(const void *__restrict__ x, int64_t rows, int64_t cols, int64_t rows_out, const float *__restrict__ scale,
                                             float st, uint8_t *__restrict__ out, uint8_t *__restrict__ out_t, int64_t tr,
                                             int64_t tc, uint8_t *tile, uint32_t &am) {
     constexpr int ESZ = SRC == ODL_BF16 ? 2 : 4;
@@ -761,7 +767,7 @@ __device__ __forceinline__ void ct_one_tile(const void *__restrict__ x, int64_t 
         }
         lo[i] = quantise4<FMT>(f[0], f[1], f[2], f[3], s[0], s[1], s[2], s[3]);
         hi[i] = quantise4<FMT>(f[4], f[5], f[6], f[7], s[4], s[5], s[6], s[7]);
-        if constexpr (WRITE_ROWMAJOR) ct_store_row<SRC>(out, r0 + i, rows, cols, cA, cB, okA, okB, lo[i], hi[i]);
+        if constexpr (WRITE_ROWMAJOR) ct_store_row<SRC>(out, r0 + i, rows_out, cols, cA, cB, okA, okB, lo[i], hi[i]);
     }
 
     // ---- transpose in registers, stage through LDS
@@ -780,15 +786,15 @@ __device__ __forceinline__ void ct_one_tile(const void *__restrict__ x, int64_t 
         const int chunk = threadIdx.x + it * kThreads;
         const int k = chunk / 8, m16 = chunk % 8;
         const int64_t oc = tc * kTileC + k, orow = tr * kTileR + m16 * 16;
-        if (oc < cols && orow < rows) {             // rows % 16 == 0 (host-checked)
+        if (oc < cols && orow < rows_out) {         // rows_out % 16 == 0 (host-checked)
             const u32x4 v = ct_lds_read(tile, k, m16);
-            __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(out_t + oc * rows + orow));
+            __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(out_t + oc * rows_out + orow));
         }
     }
 }
 
 template <int SRC, int FMT, int MODE, bool AMAX, bool WRITE_ROWMAJOR>
-__global__ __launch_bounds__(kThreads) void cast_transpose_kernel(const void *__restrict__ x, int64_t rows, int64_t cols,
+__global__ __launch_bounds__(kThreads) void cast_transpose_kernel(const void *__restrict__ x, int64_t rows, int64_t cols, int64_t rows_out,
                                                                    const float *__restrict__ scale,
                                                                    uint8_t *__restrict__ out, uint8_t *__restrict__ out_t,
                                                                    float *__restrict__ amax_out, int margin, float *__restrict__ dyn_out,
@@ -802,7 +808,7 @@ __global__ __launch_bounds__(kThreads) void cast_transpose_kernel(const void *__
         record_scale_inv(st, dyn_out);
     }
     const int64_t tiles_c = (cols + kTileC - 1) / kTileC;
-    const int64_t ntiles = tiles_c * ((rows + kTileR - 1) / kTileR);
+    const int64_t ntiles = tiles_c * ((rows_out + kTileR - 1) / kTileR);
     uint32_t am = 0;
     // With a maximum folded into one word the grid is small and each block walks several tiles, so
     // that the kernel ends in few atomics; otherwise one tile per block.
@@ -810,8 +816,8 @@ __global__ __launch_bounds__(kThreads) void cast_transpose_kernel(const void *__
         // Tiles are walked from the end of the tensor: the amax pass that ran just before read it front
         // to back, so its tail is what the memory-side cache still holds.
         int64_t tr, tc;
-        ct_tile_of(ntiles - 1 - tile_id, (rows + kTileR - 1) / kTileR, tiles_c, tr, tc);
-        ct_one_tile<SRC, FMT, MODE, AMAX, WRITE_ROWMAJOR>(x, rows, cols, scale, st, out, out_t, tr, tc, tile, am);
+        ct_tile_of(ntiles - 1 - tile_id, (rows_out + kTileR - 1) / kTileR, tiles_c, tr, tc);
+        ct_one_tile<SRC, FMT, MODE, AMAX, WRITE_ROWMAJOR>(x, rows, cols, rows_out, scale, st, out, out_t, tr, tc, tile, am);
         if (tile_id + gridDim.x < ntiles) __syncthreads();  // the LDS tile is reused by the next trip
     }
     if constexpr (AMAX) {
@@ -829,7 +835,7 @@ __global__ __launch_bounds__(kThreads) void cast_transpose_kernel(const void *__
 // scales and 64 column scales of a tile are derived once per block (IEEE division) and kept in
 // LDS; the blocks of the first tile column / row also record 1/scale for the GEMM epilogues.
 template <int SRC, int FMT>
-__global__ __launch_bounds__(kThreads) void cast_rowcol_kernel(const void *__restrict__ x, int64_t rows, int64_t cols,
+__global__ __launch_bounds__(kThreads) void cast_rowcol_kernel(const void *__restrict__ x, int64_t rows, int64_t cols, int64_t rows_out,
                                                                 const float *__restrict__ amax_row, const float *__restrict__ amax_col,
                                                                 int margin, uint8_t *__restrict__ out, uint8_t *__restrict__ out_t,
                                                                 float *__restrict__ s_row_out, float *__restrict__ s_row_inv,
@@ -841,7 +847,7 @@ __global__ __launch_bounds__(kThreads) void cast_rowcol_kernel(const void *__res
     const int ty = threadIdx.x / 8;                 // 32 lane-rows, 4 rows each
     const int64_t tiles_c = (cols + kTileC - 1) / kTileC;
     int64_t tr, tc;
-    ct_tile_of(blockIdx.x, (rows + kTileR - 1) / kTileR, tiles_c, tr, tc);
+    ct_tile_of(blockIdx.x, (rows_out + kTileR - 1) / kTileR, tiles_c, tr, tc);
     if (threadIdx.x < kTileR) {
         const int64_t r = tr * kTileR + threadIdx.x;
         const float sc = r < rows ? scale_rule(amax_row[r], Fp8Lim<FMT>::max, margin, 1.0f) : 1.0f;
@@ -880,7 +886,7 @@ __global__ __launch_bounds__(kThreads) void cast_rowcol_kernel(const void *__res
         const float sr = s_row[ty * 4 + i];
         const uint32_t rlo = quantise4<FMT>(f[0], f[1], f[2], f[3], sr, sr, sr, sr);
         const uint32_t rhi = quantise4<FMT>(f[4], f[5], f[6], f[7], sr, sr, sr, sr);
-        ct_store_row<SRC>(out, r0 + i, rows, cols, cA, cB, okA, okB, rlo, rhi);
+        ct_store_row<SRC>(out, r0 + i, rows_out, cols, cA, cB, okA, okB, rlo, rhi);
         lo[i] = quantise4<FMT>(f[0], f[1], f[2], f[3], sc_col[0], sc_col[1], sc_col[2], sc_col[3]);
         hi[i] = quantise4<FMT>(f[4], f[5], f[6], f[7], sc_col[4], sc_col[5], sc_col[6], sc_col[7]);
     }
@@ -899,9 +905,9 @@ __global__ __launch_bounds__(kThreads) void cast_rowcol_kernel(const void *__res
         const int chunk = threadIdx.x + it * kThreads;
         const int k = chunk / 8, m16 = chunk % 8;
         const int64_t oc = tc * kTileC + k, orow = tr * kTileR + m16 * 16;
-        if (oc < cols && orow < rows) {             // rows % 16 == 0 (host-checked)
+        if (oc < cols && orow < rows_out) {         // rows_out % 16 == 0 (host-checked)
             const u32x4 v = ct_lds_read(tile, k, m16);
-            __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(out_t + oc * rows + orow));
+            __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(out_t + oc * rows_out + orow));
         }
     }
 }
@@ -1024,40 +1030,40 @@ extern "C" int odl_fp8_delayed_update(float *history, int64_t H, int64_t R, int6
 namespace odl {
 
 template <int SRC, int FMT, int MODE>
-static void launch_cast(const void *x, int64_t rows, int64_t cols, const float *scale, uint8_t *out, float *amax_out,
+static void launch_cast(const void *x, int64_t rows, int64_t cols, int64_t rows_out, const float *scale, uint8_t *out, float *amax_out,
                         hipStream_t stream, int margin = 0, float *dyn_out = nullptr, int amax_mask = 0) {
     if (amax_out) {
-        const int64_t g = grid_for(rows * cols / 16, kFatThreads, 2);
-        hipLaunchKernelGGL((cast_kernel<SRC, FMT, MODE, true>), dim3((unsigned)g), dim3(kFatThreads), 0, stream, x, rows, cols, scale, out, amax_out, margin, dyn_out, amax_mask);
+        const int64_t g = grid_for(rows_out * cols / 16, kFatThreads, 2);
+        hipLaunchKernelGGL((cast_kernel<SRC, FMT, MODE, true>), dim3((unsigned)g), dim3(kFatThreads), 0, stream, x, rows, cols, rows_out, scale, out, amax_out, margin, dyn_out, amax_mask);
     } else {
-        const int64_t g = grid_for(rows * cols / 16, kThreads, 16);
-        hipLaunchKernelGGL((cast_kernel<SRC, FMT, MODE, false>), dim3((unsigned)g), dim3(kThreads), 0, stream, x, rows, cols, scale, out, amax_out, margin, dyn_out, amax_mask);
+        const int64_t g = grid_for(rows_out * cols / 16, kThreads, 16);
+        hipLaunchKernelGGL((cast_kernel<SRC, FMT, MODE, false>), dim3((unsigned)g), dim3(kThreads), 0, stream, x, rows, cols, rows_out, scale, out, amax_out, margin, dyn_out, amax_mask);
     }
 }
 
 template <int SRC, int FMT>
 static void launch_cast_mode(int mode, const void *x, int64_t rows, int64_t cols, const float *scale, uint8_t *out,
                              float *amax_out, hipStream_t stream) {
-    if (mode == ODL_SCALE_TENSOR) launch_cast<SRC, FMT, ODL_SCALE_TENSOR>(x, rows, cols, scale, out, amax_out, stream);
-    else if (mode == ODL_SCALE_ROW) launch_cast<SRC, FMT, ODL_SCALE_ROW>(x, rows, cols, scale, out, amax_out, stream);
-    else launch_cast<SRC, FMT, ODL_SCALE_COL>(x, rows, cols, scale, out, amax_out, stream);
+    if (mode == ODL_SCALE_TENSOR) launch_cast<SRC, FMT, ODL_SCALE_TENSOR>(x, rows, cols, rows, scale, out, amax_out, stream);
+    else if (mode == ODL_SCALE_ROW) launch_cast<SRC, FMT, ODL_SCALE_ROW>(x, rows, cols, rows, scale, out, amax_out, stream);
+    else launch_cast<SRC, FMT, ODL_SCALE_COL>(x, rows, cols, rows, scale, out, amax_out, stream);
 }
 
 template <int SRC, int FMT>
-static void launch_generic(const void *x, int64_t rows, int64_t cols, const float *scale, int mode, uint8_t *out,
+static void launch_generic(const void *x, int64_t rows, int64_t cols, int64_t rows_out, const float *scale, int mode, uint8_t *out,
                            uint8_t *out_t, float *amax_out, hipStream_t stream) {
-    const int64_t g = grid_for(rows * cols, kThreads * 4, 8);
-    hipLaunchKernelGGL((cast_generic_kernel<SRC, FMT>), dim3((unsigned)g), dim3(kThreads), 0, stream, x, rows, cols, scale, mode, out, out_t, amax_out);
+    const int64_t g = grid_for(rows_out * cols, kThreads * 4, 8);
+    hipLaunchKernelGGL((cast_generic_kernel<SRC, FMT>), dim3((unsigned)g), dim3(kThreads), 0, stream, x, rows, cols, rows_out, scale, mode, out, out_t, amax_out);
 }
 
 template <int SRC, int FMT, int MODE>
-static void launch_ct(const void *x, int64_t rows, int64_t cols, const float *scale, uint8_t *out, uint8_t *out_t,
+static void launch_ct(const void *x, int64_t rows, int64_t cols, int64_t rows_out, const float *scale, uint8_t *out, uint8_t *out_t,
                       float *amax_out, hipStream_t stream, int margin = 0, float *dyn_out = nullptr, int amax_mask = 0) {
-    int64_t g = ((rows + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
+    int64_t g = ((rows_out + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
     // maxima folded into ONE word: few blocks that walk several tiles each, so that the kernel ends in few
     // atomics on that word; spread over many words (amax_mask != 0), one tile per block as without a maximum
     if (amax_out && amax_mask == 0 && g > (int64_t)num_cus() * 4) g = (int64_t)num_cus() * 4;
-#define ODL_CT(AM, RM) hipLaunchKernelGGL((cast_transpose_kernel<SRC, FMT, MODE, AM, RM>), dim3((unsigned)g), dim3(kThreads), 0, stream, x, rows, cols, scale, out, out_t, amax_out, margin, dyn_out, amax_mask)
+#define ODL_CT(AM, RM) hipLaunchKernelGGL((cast_transpose_kernel<SRC, FMT, MODE, AM, RM>), dim3((unsigned)g), dim3(kThreads), 0, stream, x, rows, cols, rows_out, scale, out, out_t, amax_out, margin, dyn_out, amax_mask)
     if (amax_out) { if (out) ODL_CT(true, true); else ODL_CT(true, false); }
     else { if (out) ODL_CT(false, true); else ODL_CT(false, false); }
 #undef ODL_CT
@@ -1066,9 +1072,9 @@ static void launch_ct(const void *x, int64_t rows, int64_t cols, const float *sc
 template <int SRC, int FMT>
 static void launch_ct_mode(int mode, const void *x, int64_t rows, int64_t cols, const float *scale, uint8_t *out,
                            uint8_t *out_t, float *amax_out, hipStream_t stream) {
-    if (mode == ODL_SCALE_TENSOR) launch_ct<SRC, FMT, ODL_SCALE_TENSOR>(x, rows, cols, scale, out, out_t, amax_out, stream);
-    else if (mode == ODL_SCALE_ROW) launch_ct<SRC, FMT, ODL_SCALE_ROW>(x, rows, cols, scale, out, out_t, amax_out, stream);
-    else launch_ct<SRC, FMT, ODL_SCALE_COL>(x, rows, cols, scale, out, out_t, amax_out, stream);
+    if (mode == ODL_SCALE_TENSOR) launch_ct<SRC, FMT, ODL_SCALE_TENSOR>(x, rows, cols, rows, scale, out, out_t, amax_out, stream);
+    else if (mode == ODL_SCALE_ROW) launch_ct<SRC, FMT, ODL_SCALE_ROW>(x, rows, cols, rows, scale, out, out_t, amax_out, stream);
+    else launch_ct<SRC, FMT, ODL_SCALE_COL>(x, rows, cols, rows, scale, out, out_t, amax_out, stream);
 }
 
 static int check_cast_args(const char *who, const void *x, int src_dtype, int64_t rows, int64_t cols, const float *scale,
@@ -1102,7 +1108,7 @@ extern "C" int odl_fp8_cast(const void *x, int src_dtype, int64_t rows, int64_t 
     if (!out) return set_error(ODL_ERR_ARG, "odl_fp8_cast: out is null");
     const bool fast = cols % 16 == 0 && aligned16(x) && aligned16(out) && (mode != ODL_SCALE_COL || aligned16(scale));
     if (fast) ODL_DISPATCH_SRC_FMT(launch_cast_mode, mode, x, rows, cols, scale, out, amax_out, stream);
-    else ODL_DISPATCH_SRC_FMT(launch_generic, x, rows, cols, scale, mode, out, (uint8_t *)nullptr, amax_out, stream);
+    else ODL_DISPATCH_SRC_FMT(launch_generic, x, rows, cols, rows, scale, mode, out, (uint8_t *)nullptr, amax_out, stream);
     return check_launch("odl_fp8_cast");
 }
 
@@ -1117,7 +1123,7 @@ extern "C" int odl_fp8_cast_transpose(const void *x, int src_dtype, int64_t rows
                       (!out || (reinterpret_cast<uintptr_t>(out) & 7) == 0) &&
                       (mode != ODL_SCALE_COL || aligned16(scale)) && tiles <= 0x7fffffffLL;
     if (fast) ODL_DISPATCH_SRC_FMT(launch_ct_mode, mode, x, rows, cols, scale, out, out_t, amax_out, stream);
-    else ODL_DISPATCH_SRC_FMT(launch_generic, x, rows, cols, scale, mode, out, out_t, amax_out, stream);
+    else ODL_DISPATCH_SRC_FMT(launch_generic, x, rows, cols, rows, scale, mode, out, out_t, amax_out, stream);
     return check_launch("odl_fp8_cast_transpose");
 }
 
@@ -1127,51 +1133,57 @@ __global__ void scale_inv_kernel(const float *__restrict__ scale, float *__restr
 }
 
 template <int SRC, int FMT>
-static void launch_delayed(const void *x, int64_t rows, int64_t cols, const float *scale, uint8_t *out, uint8_t *out_t,
+static void launch_delayed(const void *x, int64_t rows, int64_t cols, int64_t rows_out, const float *scale, uint8_t *out, uint8_t *out_t,
                            float *amax_parts, float *scale_inv_out, bool fast, hipStream_t stream) {
     if (!fast) {
         // element-at-a-time route: the whole maximum goes into amax_parts[0]
-        launch_generic<SRC, FMT>(x, rows, cols, scale, ODL_SCALE_TENSOR, out, out_t, amax_parts, stream);
+        launch_generic<SRC, FMT>(x, rows, cols, rows_out, scale, ODL_SCALE_TENSOR, out, out_t, amax_parts, stream);
         if (scale_inv_out) hipLaunchKernelGGL(scale_inv_kernel, dim3(1), dim3(1), 0, stream, scale, scale_inv_out);
     } else if (out_t) {
-        launch_ct<SRC, FMT, ODL_SCALE_TENSOR>(x, rows, cols, scale, out, out_t, amax_parts, stream, 0, scale_inv_out, kAmaxParts - 1);
+        launch_ct<SRC, FMT, ODL_SCALE_TENSOR>(x, rows, cols, rows_out, scale, out, out_t, amax_parts, stream, 0, scale_inv_out, kAmaxParts - 1);
     } else {
-        launch_cast<SRC, FMT, ODL_SCALE_TENSOR>(x, rows, cols, scale, out, amax_parts, stream, 0, scale_inv_out, kAmaxParts - 1);
+        launch_cast<SRC, FMT, ODL_SCALE_TENSOR>(x, rows, cols, rows_out, scale, out, amax_parts, stream, 0, scale_inv_out, kAmaxParts - 1);
     }
 }
 }  // namespace odl
 
 extern "C" int odl_fp8_cast_delayed(const void *x, int src_dtype, int64_t rows, int64_t cols, const float *scale, int fmt,
                                     uint8_t *out, uint8_t *out_t, float *amax_parts, float *scale_inv_out, odl_stream_t stream_) {
+    return odl_fp8_cast_delayed_padded(x, src_dtype, rows, cols, rows, scale, fmt, out, out_t, amax_parts, scale_inv_out, stream_);
+}
+
+extern "C" int odl_fp8_cast_delayed_padded(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, const float *scale, int fmt,
+                                           uint8_t *out, uint8_t *out_t, float *amax_parts, float *scale_inv_out, odl_stream_t stream_) {
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
     if (int e = check_cast_args("odl_fp8_cast_delayed", x, src_dtype, rows, cols, scale, ODL_SCALE_TENSOR, fmt)) return e;
+    if (rows_out < rows) return set_error(ODL_ERR_ARG, "odl_fp8_cast_delayed: rows_out %lld < rows %lld", (long long)rows_out, (long long)rows);
     if (!scale) return set_error(ODL_ERR_ARG, "odl_fp8_cast_delayed: scale is null");
     if (rows * cols == 0) {                       // nothing to cast and nothing to record: only the inverse scale
         if (scale_inv_out) hipLaunchKernelGGL(scale_inv_kernel, dim3(1), dim3(1), 0, stream, scale, scale_inv_out);
         return check_launch("odl_fp8_cast_delayed");
     }
     if (!out && !out_t) return set_error(ODL_ERR_ARG, "odl_fp8_cast_delayed: out and out_t are both null");
-    const int64_t tiles = ((rows + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
-    const bool fast = out_t ? (cols % 8 == 0 && rows % 16 == 0 && aligned16(x) && aligned16(out_t) &&
+    const int64_t tiles = ((rows_out + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
+    const bool fast = out_t ? (cols % 8 == 0 && rows_out % 16 == 0 && aligned16(x) && aligned16(out_t) &&
                                (!out || (reinterpret_cast<uintptr_t>(out) & 7) == 0) && tiles <= 0x7fffffffLL)
                             : (cols % 16 == 0 && aligned16(x) && aligned16(out));
-    ODL_DISPATCH_SRC_FMT(launch_delayed, x, rows, cols, scale, out, out_t, amax_parts, scale_inv_out, fast, stream);
+    ODL_DISPATCH_SRC_FMT(launch_delayed, x, rows, cols, rows_out, scale, out, out_t, amax_parts, scale_inv_out, fast, stream);
     return check_launch("odl_fp8_cast_delayed");
 }
 
 namespace odl {
 
 template <int SRC, int FMT>
-static void launch_dynamic(const void *x, int64_t rows, int64_t cols, const float *parts, int margin, uint8_t *out,
+static void launch_dynamic(const void *x, int64_t rows, int64_t cols, int64_t rows_out, const float *parts, int margin, uint8_t *out,
                            uint8_t *out_t, float *dyn_out, bool fast, hipStream_t stream) {
     if (!fast) {
         // element-at-a-time route: scale first (one block), then the generic kernel reads it from dyn_out[1]
         hipLaunchKernelGGL((parts_to_scale_kernel<FMT>), dim3(1), dim3(kThreads), 0, stream, parts, margin, dyn_out);
-        launch_generic<SRC, FMT>(x, rows, cols, dyn_out + 1, ODL_SCALE_TENSOR, out, out_t, nullptr, stream);
+        launch_generic<SRC, FMT>(x, rows, cols, rows_out, dyn_out + 1, ODL_SCALE_TENSOR, out, out_t, nullptr, stream);
     } else if (out_t) {
-        launch_ct<SRC, FMT, kScaleParts>(x, rows, cols, parts, out, out_t, nullptr, stream, margin, dyn_out);
+        launch_ct<SRC, FMT, kScaleParts>(x, rows, cols, rows_out, parts, out, out_t, nullptr, stream, margin, dyn_out);
     } else {
-        launch_cast<SRC, FMT, kScaleParts>(x, rows, cols, parts, out, nullptr, stream, margin, dyn_out);
+        launch_cast<SRC, FMT, kScaleParts>(x, rows, cols, rows_out, parts, out, nullptr, stream, margin, dyn_out);
     }
 }
 
@@ -1199,8 +1211,14 @@ extern "C" int odl_fp8_amax_parts(const void *x, int src_dtype, int64_t rows, in
 
 extern "C" int odl_fp8_cast_dynamic(const void *x, int src_dtype, int64_t rows, int64_t cols, const float *parts, int fmt, int margin,
                                     uint8_t *out, uint8_t *out_t, float *dyn_out, odl_stream_t stream_) {
+    return odl_fp8_cast_dynamic_padded(x, src_dtype, rows, cols, rows, parts, fmt, margin, out, out_t, dyn_out, stream_);
+}
+
+extern "C" int odl_fp8_cast_dynamic_padded(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, const float *parts, int fmt,
+                                           int margin, uint8_t *out, uint8_t *out_t, float *dyn_out, odl_stream_t stream_) {
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
     if (int e = check_cast_args("odl_fp8_cast_dynamic", x, src_dtype, rows, cols, parts, ODL_SCALE_TENSOR, fmt)) return e;
+    if (rows_out < rows) return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic: rows_out %lld < rows %lld", (long long)rows_out, (long long)rows);
     if (!parts || !dyn_out) return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic: null pointer");
     if (rows * cols == 0) {                       // nothing to cast: only the three numbers
         if (fmt == ODL_FP8_E4M3) hipLaunchKernelGGL((parts_to_scale_kernel<ODL_FP8_E4M3>), dim3(1), dim3(kThreads), 0, stream, parts, margin, dyn_out);
@@ -1210,13 +1228,13 @@ extern "C" int odl_fp8_cast_dynamic(const void *x, int src_dtype, int64_t rows, 
     if (!out && !out_t) return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic: out and out_t are both null");
     bool fast;
     if (out_t) {
-        const int64_t tiles = ((rows + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
-        fast = cols % 8 == 0 && rows % 16 == 0 && aligned16(x) && aligned16(out_t) && (!out || (reinterpret_cast<uintptr_t>(out) & 7) == 0) &&
+        const int64_t tiles = ((rows_out + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
+        fast = cols % 8 == 0 && rows_out % 16 == 0 && aligned16(x) && aligned16(out_t) && (!out || (reinterpret_cast<uintptr_t>(out) & 7) == 0) &&
                tiles <= 0x7fffffffLL && rows * cols > 0;
     } else {
         fast = cols % 16 == 0 && aligned16(x) && aligned16(out) && rows * cols > 0;
     }
-    ODL_DISPATCH_SRC_FMT(launch_dynamic, x, rows, cols, parts, margin, out, out_t, dyn_out, fast, stream);
+    ODL_DISPATCH_SRC_FMT(launch_dynamic, x, rows, cols, rows_out, parts, margin, out, out_t, dyn_out, fast, stream);
     return check_launch("odl_fp8_cast_dynamic");
 }
 
@@ -1260,8 +1278,8 @@ __global__ __launch_bounds__(kThreads) void multi_cast_dynamic_kernel(const odl_
     int64_t tr, tc;
     ct_tile_of(tiles_r * tiles_c - 1 - local, tiles_r, tiles_c, tr, tc);
     uint32_t am = 0;
-    if (e.src_dtype == ODL_BF16) ct_one_tile<ODL_BF16, FMT, kScaleParts, false, true>(e.x, e.rows, e.cols, nullptr, st, e.out, e.out_t, tr, tc, tile, am);
-    else ct_one_tile<ODL_F32, FMT, kScaleParts, false, true>(e.x, e.rows, e.cols, nullptr, st, e.out, e.out_t, tr, tc, tile, am);
+    if (e.src_dtype == ODL_BF16) ct_one_tile<ODL_BF16, FMT, kScaleParts, false, true>(e.x, e.rows, e.cols, e.rows, nullptr, st, e.out, e.out_t, tr, tc, tile, am);
+    else ct_one_tile<ODL_F32, FMT, kScaleParts, false, true>(e.x, e.rows, e.cols, e.rows, nullptr, st, e.out, e.out_t, tr, tc, tile, am);
 }
 
 template <int FMT>
@@ -1281,10 +1299,10 @@ __global__ __launch_bounds__(kThreads) void multi_cast_delayed_kernel(const odl_
     ct_tile_of(tiles_r * tiles_c - 1 - local, tiles_r, tiles_c, tr, tc);
     uint32_t am = 0;
     if (e.src_dtype == ODL_BF16) {
-        ct_one_tile<ODL_BF16, FMT, ODL_SCALE_TENSOR, true, true>(e.x, e.rows, e.cols, nullptr, st, e.out, e.out_t, tr, tc, tile, am);
+        ct_one_tile<ODL_BF16, FMT, ODL_SCALE_TENSOR, true, true>(e.x, e.rows, e.cols, e.rows, nullptr, st, e.out, e.out_t, tr, tc, tile, am);
         am = fold_u16x2_to_f32bits(am);
     } else {
-        ct_one_tile<ODL_F32, FMT, ODL_SCALE_TENSOR, true, true>(e.x, e.rows, e.cols, nullptr, st, e.out, e.out_t, tr, tc, tile, am);
+        ct_one_tile<ODL_F32, FMT, ODL_SCALE_TENSOR, true, true>(e.x, e.rows, e.cols, e.rows, nullptr, st, e.out, e.out_t, tr, tc, tile, am);
     }
     am = block_max_u32(am, red);
     if (threadIdx.x == 0 && am != 0) atomicMax(reinterpret_cast<uint32_t *>(e.parts) + (local & (kAmaxParts - 1)), am);
@@ -1438,33 +1456,47 @@ extern "C" int odl_fp8_amax_rowcol(const void *x, int src_dtype, int64_t rows, i
 }
 
 template <int SRC, int FMT>
-static void launch_rowcol(const void *x, int64_t rows, int64_t cols, const float *amax_row, const float *amax_col, int margin,
+static void launch_rowcol(const void *x, int64_t rows, int64_t cols, int64_t rows_out, const float *amax_row, const float *amax_col, int margin,
                           uint8_t *out, uint8_t *out_t, float *s_row, float *s_row_inv, float *s_col, float *s_col_inv, hipStream_t stream) {
-    const int64_t g = ((rows + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
-    hipLaunchKernelGGL((cast_rowcol_kernel<SRC, FMT>), dim3((unsigned)g), dim3(kThreads), 0, stream, x, rows, cols, amax_row, amax_col,
+    const int64_t g = ((rows_out + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
+    hipLaunchKernelGGL((cast_rowcol_kernel<SRC, FMT>), dim3((unsigned)g), dim3(kThreads), 0, stream, x, rows, cols, rows_out, amax_row, amax_col,
                        margin, out, out_t, s_row, s_row_inv, s_col, s_col_inv);
 }
 
 extern "C" int odl_fp8_cast_rowcol(const void *x, int src_dtype, int64_t rows, int64_t cols, const float *amax_row,
                                    const float *amax_col, int fmt, int margin, uint8_t *out, uint8_t *out_t, float *s_row,
                                    float *s_row_inv, float *s_col, float *s_col_inv, odl_stream_t stream_) {
+    return odl_fp8_cast_rowcol_padded(x, src_dtype, rows, cols, rows, amax_row, amax_col, fmt, margin, out, out_t, s_row, s_row_inv, s_col,
+                                      s_col_inv, stream_);
+}
+
+extern "C" int odl_fp8_cast_rowcol_padded(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, const float *amax_row,
+                                          const float *amax_col, int fmt, int margin, uint8_t *out, uint8_t *out_t, float *s_row,
+                                          float *s_row_inv, float *s_col, float *s_col_inv, odl_stream_t stream_) {
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
     if (rows < 0 || cols < 0) return set_error(ODL_ERR_ARG, "odl_fp8_cast_rowcol: negative shape");
+    if (rows_out < rows) return set_error(ODL_ERR_ARG, "odl_fp8_cast_rowcol: rows_out %lld < rows %lld", (long long)rows_out, (long long)rows);
     if (src_dtype != ODL_BF16 && src_dtype != ODL_F32) return set_error(ODL_ERR_ARG, "odl_fp8_cast_rowcol: src_dtype %d", src_dtype);
     if (fmt != ODL_FP8_E4M3 && fmt != ODL_FP8_E5M2) return set_error(ODL_ERR_ARG, "odl_fp8_cast_rowcol: fmt %d", fmt);
     if ((rows > 0 && (!amax_row || !s_row || !s_row_inv)) || (cols > 0 && (!amax_col || !s_col || !s_col_inv)))
         return set_error(ODL_ERR_ARG, "odl_fp8_cast_rowcol: null scale pointer");
     if (rows * cols > 0 && (!x || !out || !out_t)) return set_error(ODL_ERR_ARG, "odl_fp8_cast_rowcol: null pointer");
-    const int64_t tiles = ((rows + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
-    const bool fast = rowcol_fast(x, rows, cols) && aligned16(out_t) && (reinterpret_cast<uintptr_t>(out) & 7) == 0 && tiles <= 0x7fffffffLL;
+    const int64_t tiles = ((rows_out + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
+    const bool fast = rowcol_fast(x, rows_out, cols) && rows > 0 && aligned16(out_t) && (reinterpret_cast<uintptr_t>(out) & 7) == 0 && tiles <= 0x7fffffffLL;
     if (!fast) {
         // the step-by-step route: scales first, then the two casts
         int rc = odl_fp8_scale_from_amax(amax_row, rows, fmt, margin, s_row, s_row_inv, stream_);
         if (rc == ODL_OK) rc = odl_fp8_scale_from_amax(amax_col, cols, fmt, margin, s_col, s_col_inv, stream_);
-        if (rc == ODL_OK && rows * cols > 0) rc = odl_fp8_cast(x, src_dtype, rows, cols, s_row, ODL_SCALE_ROW, fmt, out, nullptr, stream_);
-        if (rc == ODL_OK && rows * cols > 0) rc = odl_fp8_cast_transpose(x, src_dtype, rows, cols, s_col, ODL_SCALE_COL, fmt, nullptr, out_t, nullptr, stream_);
+        if (rc != ODL_OK || rows * cols == 0) return rc;
+        if (rows_out != rows) {
+            ODL_DISPATCH_SRC_FMT(launch_generic, x, rows, cols, rows_out, s_row, ODL_SCALE_ROW, out, (uint8_t *)nullptr, (float *)nullptr, stream);
+            ODL_DISPATCH_SRC_FMT(launch_generic, x, rows, cols, rows_out, s_col, ODL_SCALE_COL, (uint8_t *)nullptr, out_t, (float *)nullptr, stream);
+            return check_launch("odl_fp8_cast_rowcol");
+        }
+        rc = odl_fp8_cast(x, src_dtype, rows, cols, s_row, ODL_SCALE_ROW, fmt, out, nullptr, stream_);
+        if (rc == ODL_OK) rc = odl_fp8_cast_transpose(x, src_dtype, rows, cols, s_col, ODL_SCALE_COL, fmt, nullptr, out_t, nullptr, stream_);
         return rc;
     }
-    ODL_DISPATCH_SRC_FMT(launch_rowcol, x, rows, cols, amax_row, amax_col, margin, out, out_t, s_row, s_row_inv, s_col, s_col_inv, stream);
+    ODL_DISPATCH_SRC_FMT(launch_rowcol, x, rows, cols, rows_out, amax_row, amax_col, margin, out, out_t, s_row, s_row_inv, s_col, s_col_inv, stream);
     return check_launch("odl_fp8_cast_rowcol");
 }

@@ -85,14 +85,15 @@ def _kept_stamp(weight: torch.Tensor, pol) -> tuple:
 
 
 def _quantise_dynamic(x2d: torch.Tensor, fmt: int, margin: int, need_t: bool, need_rowmajor: bool = True,
-                      recipe: FP8Recipe | None = None, parts: torch.Tensor | None = None, out_t: torch.Tensor | None = None):
+                      recipe: FP8Recipe | None = None, parts: torch.Tensor | None = None, out_t: torch.Tensor | None = None,
+                      rows_out: int | None = None):
     """Per-tensor current scaling: amax pass, scale, cast (+transpose) pass.  The amax pass is
     skipped when the caller has the partial maxima, or when the kernel that produced x2d left them
     with the recipe."""
     if parts is None and recipe is not None:
         parts = recipe.take_parts(x2d)
     q, q_t, amax, _, scale_inv = native.quantize_dynamic(x2d, fmt, margin, want_rowmajor=need_rowmajor or not need_t,
-                                                        want_transposed=need_t, parts=parts, out_t=out_t)
+                                                        want_transposed=need_t, parts=parts, out_t=out_t, rows_out=rows_out)
     return q, q_t, scale_inv, amax
 
 
@@ -104,14 +105,16 @@ def _quantise_input_shared(recipe: FP8Recipe, x2d: torch.Tensor, fmt: int, margi
     """Per-tensor quantisation of a Linear's input, reused by the next Linear that is fed the
     very same tensor (gate and up of an MLP, q/k/v of an attention block).  The entry keeps
     the tensor alive, so its address cannot be handed to another tensor while it is cached;
-    an in-place change bumps ``_version`` and misses."""
+    an in-place change bumps ``_version`` and misses.  With need_t the codes are padded to whole K steps of the wgrad GEMM
+    (``native.padded_rows``)."""
+    rows_out = native.padded_rows(x2d.shape[0]) if need_t else None
     if not recipe.share_inputs:
-        return _quantise_dynamic(x2d, fmt, margin, need_t, recipe=recipe)[:3]
+        return _quantise_dynamic(x2d, fmt, margin, need_t, recipe=recipe, rows_out=rows_out)[:3]
     key = _input_key(x2d, "tensor", fmt, margin)
     hit = recipe.shared_input
     if hit is not None and hit["key"] == key and (hit["q_t"] is not None or not need_t):
         return hit["q"], hit["q_t"], hit["s_inv"]
-    q, q_t, s_inv, _ = _quantise_dynamic(x2d, fmt, margin, need_t, recipe=recipe)
+    q, q_t, s_inv, _ = _quantise_dynamic(x2d, fmt, margin, need_t, recipe=recipe, rows_out=rows_out)
     entry = {"key": key, "x": x2d, "q": q, "q_t": q_t, "s_inv": s_inv}
     if hit is not None and hit.get("x") is x2d:          # keep the record of the conversion that produced x2d
         entry["src_key"], entry["src"] = hit.get("src_key"), hit.get("src")
@@ -149,13 +152,14 @@ def _mx_input_shared(recipe: FP8Recipe, x2d: torch.Tensor, fmt: int, need_t: boo
 def _rowwise_input_shared(recipe: FP8Recipe, x2d: torch.Tensor, fmt: int, margin: int, need_t: bool):
     """Rowwise codes of a Linear's input: per-row scales for the forward GEMM and, with need_t, the transposed codes with
     per-column scales for wgrad, made once for the Linears fed by the very same tensor (two passes over x for q / k / v
-    together instead of two each).  -> (xq, sx_inv, xq_t or None, sx_inv_t or None)."""
+    together instead of two each).  The codes are padded like those of ``_quantise_input_shared``.
+    -> (xq, sx_inv, xq_t or None, sx_inv_t or None)."""
     key = _input_key(x2d, "rowwise", fmt, margin)
     hit = recipe.shared_input if recipe.share_inputs else None
     if hit is not None and hit["key"] == key and (hit["q_t"] is not None or not need_t):
         return hit["q"], hit["s_inv"], hit["q_t"], hit["s_t"]
     if need_t:
-        q, s_inv, q_t, s_t, _, _ = native.quantize_rowcol(x2d, fmt, margin)
+        q, s_inv, q_t, s_t, _, _ = native.quantize_rowcol(x2d, fmt, margin, rows_out=native.padded_rows(x2d.shape[0]))
     else:
         (q, s_inv), q_t, s_t = _quantise_axis(x2d, fmt, margin, R, False), None, None
     if recipe.share_inputs:
@@ -184,21 +188,26 @@ def _converted_input(recipe: FP8Recipe, x2d: torch.Tensor, dtype: torch.dtype) -
 
 def _quantise_delayed(x2d: torch.Tensor, fmt: int, meta: "_state.ScalingMeta | None", role: int, need_t: bool,
                       need_rowmajor: bool = True, recipe: FP8Recipe | None = None, record: bool = True, margin: int = 0,
-                      out_t: torch.Tensor | None = None):
+                      out_t: torch.Tensor | None = None, rows_out: int | None = None):
     """Delayed scaling: one pass with the scale from the history, this step's partial maxima recorded with the role.
     record=False (a module in eval mode): the scales that training arrived at are used as they are and
     the histories are left alone; roles that do not exist yet (meta None) or have never been through a
     refresh still stand at the initial scale 1 (a weight of std 0.02 would land in the subnormals), so
     such a tensor is scaled from its own amax instead."""
     if not record and (meta is None or not meta.trained):
-        q, q_t, scale_inv, _ = _quantise_dynamic(x2d, fmt, margin, need_t, need_rowmajor, out_t=out_t)
+        q, q_t, scale_inv, _ = _quantise_dynamic(x2d, fmt, margin, need_t, need_rowmajor, out_t=out_t, rows_out=rows_out)
         return q, q_t, scale_inv
     slot = meta.amax_slot(role) if record else None
     if record:
         meta.note_record(recipe._store)
     # the scale is refreshed in place after the step; the cast hands back the inverse of the one it used
     return native.cast_delayed(x2d, meta.scale_of(role), fmt, amax_parts=slot, want_rowmajor=need_rowmajor or not need_t,
-                               want_transposed=need_t, out_t=out_t)
+                               want_transposed=need_t, out_t=out_t, rows_out=rows_out)
+
+
+def _rows(codes: torch.Tensor, n: int) -> torch.Tensor:
+    """The first n rows of codes that were cast with padding behind them."""
+    return codes if codes.shape[0] == n else codes[:n]
 
 
 def _quantise_axis(x2d: torch.Tensor, fmt: int, margin: int, mode: int, transposed: bool):
@@ -242,13 +251,14 @@ class _Fp8LinearFn(torch.autograd.Function):
             if not recipe.cache_weights:
                 module._wcache_rowwise.clear()          # the backward of this call still finds what is made now
             wq, sw_inv = module._rowwise_weight(weight, pol, "row", both=need_dgrad)
-            y = native.gemm_nt(xq, wq, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sw_inv, bias=bias_f32, out_dtype=out_dtype)
+            y = native.gemm_nt(_rows(xq, x2d.shape[0]), wq, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sw_inv, bias=bias_f32, out_dtype=out_dtype)
         else:
             # With whole 256 x 256 tiles wgrad reads the ROW-MAJOR codes of dy with the tokens as the slow
             # axis (native.gemm_layouts): dy, the largest tensor of the backward, gets no transposed copy.
             # x and w keep theirs: they are cold by the time the backward runs, and reading a cold operand
             # K-slow costs the GEMM more than the copy (measured), while dy has just been written.
-            tokens, n_in, n_out = x2d.shape[0], x2d.shape[1], weight.shape[0]
+            # The codes of x and dy are cast with zero codes behind the last token, up to whole K steps of wgrad.
+            tokens, n_in, n_out = native.padded_rows(x2d.shape[0]), x2d.shape[1], weight.shape[0]
             fp8_wgrad = need_wgrad and recipe.wgrad
             # (not when weight gradients are added into .grad by the GEMM: the kernel that reads dy as stored cannot
             # accumulate, and the detour through a workspace costs what the fusion saves: measured 500 us against
@@ -263,11 +273,11 @@ class _Fp8LinearFn(torch.autograd.Function):
                 record = module._records()
                 meta = module._meta(recipe, x2d.device, "fwd", create=record)
                 xq, xq_t, sx_inv = _quantise_delayed(x2d, pol.fmt_fwd, meta, ROLE_X, fp8_wgrad, recipe=recipe,
-                                                     record=record, margin=pol.margin)
+                                                     record=record, margin=pol.margin, rows_out=tokens if fp8_wgrad else None)
             else:
                 xq, xq_t, sx_inv = _quantise_input_shared(recipe, x2d, pol.fmt_fwd, pol.margin, fp8_wgrad)
             wq, wq_t, sw_inv = module._tensor_weight(weight, recipe, need_t=need_dgrad)
-            y = native.gemm_nt(xq, wq, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sw_inv, bias=bias_f32, out_dtype=out_dtype)
+            y = native.gemm_nt(_rows(xq, x2d.shape[0]), wq, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sw_inv, bias=bias_f32, out_dtype=out_dtype)
             if fp8_wgrad:
                 saved["xq_t"], saved["sx_inv_t"] = xq_t, sx_inv
             if need_dgrad:
@@ -298,6 +308,8 @@ class _Fp8LinearFn(torch.autograd.Function):
             dy2d = dy2d.to(torch.bfloat16)
         dx = dw = db = None
         fp8_wgrad = ctx.need_wgrad and recipe.wgrad
+        tokens = dy2d.shape[0]
+        rows_out = native.padded_rows(tokens) if fp8_wgrad else None       # whole K steps for wgrad, as the codes of x
 
         if pol.kind in ("mxfp8", "blockwise"):
             if ctx.need_dgrad or fp8_wgrad:
@@ -309,11 +321,12 @@ class _Fp8LinearFn(torch.autograd.Function):
                 dw = native.mx_gemm_nt(gq_t, gs_t, saved["xq_t"], saved["xs_t"], pol.fmt_bwd, pol.fmt_fwd, out_dtype=ctx.w_dtype)
         elif pol.kind == "rowwise":
             if ctx.need_dgrad and fp8_wgrad:
-                gq, sg_inv, gq_t, sg_inv_t, _, _ = native.quantize_rowcol(dy2d, pol.fmt_bwd, pol.margin)
+                gq, sg_inv, gq_t, sg_inv_t, _, _ = native.quantize_rowcol(dy2d, pol.fmt_bwd, pol.margin, rows_out=rows_out)
+                gq = _rows(gq, tokens)
             elif ctx.need_dgrad:
                 gq, sg_inv = _quantise_axis(dy2d, pol.fmt_bwd, pol.margin, R, False)
             elif fp8_wgrad:
-                gq_t, sg_inv_t = _quantise_axis(dy2d, pol.fmt_bwd, pol.margin, C, True)
+                _, _, gq_t, sg_inv_t, _, _ = native.quantize_rowcol(dy2d, pol.fmt_bwd, pol.margin, rows_out=rows_out)
             if ctx.need_dgrad:
                 wq_t, sw_inv_t = module._rowwise_weight(saved["weight"], pol, "col")
                 dx_into = getattr(ctx, "dx_into", None)      # a later member of a sibling group adds into the group's dx
@@ -336,7 +349,8 @@ class _Fp8LinearFn(torch.autograd.Function):
                 if pol.kind == "delayed":
                     meta = module._meta(recipe, dy2d.device, "bwd", create=module.training)
                     gq, gq_t, sg_inv = _quantise_delayed(dy2d, pol.fmt_bwd, meta, ROLE_G, g_t_needed, g_rm_needed,
-                                                         recipe=recipe, record=module.training, margin=pol.margin, out_t=gq_t_out)
+                                                         recipe=recipe, record=module.training, margin=pol.margin, out_t=gq_t_out,
+                                                         rows_out=rows_out)
                 else:
                     parts = recipe.take_parts(dy2d)
                     if ctx.has_bias and native.colsum_supported(dy2d):
@@ -346,20 +360,21 @@ class _Fp8LinearFn(torch.autograd.Function):
                         parts, colsum = native.amax_parts_colsum(dy2d)
                         db = colsum.to(ctx.bias_dtype)
                     gq, gq_t, sg_inv, _ = _quantise_dynamic(dy2d, pol.fmt_bwd, pol.margin, g_t_needed, g_rm_needed,
-                                                            parts=parts, out_t=gq_t_out)
+                                                            parts=parts, out_t=gq_t_out, rows_out=rows_out)
             if ctx.need_dgrad:
+                gq_rows = _rows(gq, tokens)
                 # a member of a group of Linears fed by one tensor leaves its operands to the group's one GEMM over
                 # all members, or adds its share into the group's gradient (the GEMM's accumulate flag), instead of
                 # leaving the sum to a separate pass
                 dx_pairs = getattr(ctx, "dx_pairs", None)
                 dx_into = getattr(ctx, "dx_into", None)
                 if dx_pairs is not None:
-                    dx_pairs.append((gq, saved["wq_t"], sg_inv, saved["sw_inv_t"]))
+                    dx_pairs.append((gq_rows, saved["wq_t"], sg_inv, saved["sw_inv_t"]))
                 elif dx_into is not None:
-                    dx = native.gemm_nt(gq, saved["wq_t"], pol.fmt_bwd, pol.fmt_fwd, sg_inv, saved["sw_inv_t"],
+                    dx = native.gemm_nt(gq_rows, saved["wq_t"], pol.fmt_bwd, pol.fmt_fwd, sg_inv, saved["sw_inv_t"],
                                         out=dx_into, accumulate=True)
                 else:
-                    dx = native.gemm_nt(gq, saved["wq_t"], pol.fmt_bwd, pol.fmt_fwd, sg_inv, saved["sw_inv_t"],
+                    dx = native.gemm_nt(gq_rows, saved["wq_t"], pol.fmt_bwd, pol.fmt_fwd, sg_inv, saved["sw_inv_t"],
                                         out_dtype=ctx.x_dtype)
             if fp8_wgrad and joint is not None:
                 joint["sg_inv"] = sg_inv             # the group multiplies: dW rows of this member = dY^T codes . X^T codes

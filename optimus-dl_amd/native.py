@@ -24,7 +24,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 16
+ABI_VERSION = 17
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -41,6 +41,9 @@ EXPORTS = (
     "odl_fp8_amax_parts",
     "odl_fp8_cast_dynamic",
     "odl_fp8_cast_dynamic_noalloc",
+    "odl_fp8_cast_dynamic_padded",
+    "odl_fp8_cast_delayed_padded",
+    "odl_fp8_cast_rowcol_padded",
     "odl_fp8_multi_plan",
     "odl_fp8_multi_amax_parts",
     "odl_fp8_multi_cast_dynamic",
@@ -111,6 +114,9 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_amax_scale.argtypes = [vp, i32, i64, i64, i32, i32, vp, vp, vp, vp, vp]
         L.odl_fp8_amax_parts.argtypes = [vp, i32, i64, i64, vp, vp]
         L.odl_fp8_cast_dynamic.argtypes = [vp, i32, i64, i64, vp, i32, i32, vp, vp, vp, vp]
+        L.odl_fp8_cast_dynamic_padded.argtypes = [vp, i32, i64, i64, i64, vp, i32, i32, vp, vp, vp, vp]
+        L.odl_fp8_cast_delayed_padded.argtypes = [vp, i32, i64, i64, i64, vp, i32, vp, vp, vp, vp, vp]
+        L.odl_fp8_cast_rowcol_padded.argtypes = [vp, i32, i64, i64, i64, vp, vp, i32, i32, vp, vp, vp, vp, vp, vp, vp]
         L.odl_fp8_cast_dynamic_noalloc.argtypes = [vp, i32, i64, i64, i32, i32, vp, vp, vp, vp]
         L.odl_fp8_multi_plan.argtypes = [vp, i64, i32, vp, i64]
         L.odl_fp8_multi_plan.restype = ctypes.c_int64
@@ -307,11 +313,18 @@ def _codes_out(t: torch.Tensor, shape: tuple, device, what: str) -> torch.Tensor
     return t
 
 
+def padded_rows(rows: int) -> int:
+    """The next multiple of 128, the K step of the GEMM kernels: what a tensor that a GEMM contracts over its rows (the
+    tokens of a weight gradient) is cast with as ``rows_out``."""
+    return (rows + 127) // 128 * 128
+
+
 def cast_dynamic(x: torch.Tensor, parts: torch.Tensor, fmt: int, margin: int = 0, want_rowmajor: bool = True,
-                 want_transposed: bool = True, out_t: torch.Tensor | None = None):
+                 want_transposed: bool = True, out_t: torch.Tensor | None = None, rows_out: int | None = None):
     """Cast with the per-tensor scale derived inside the kernel from the partial maxima.  out_t: where the transposed
     codes go (a [cols, rows] uint8 tensor of the caller's, e.g. a run of rows of a larger buffer that holds the codes of
-    several tensors); implies want_transposed.
+    several tensors); implies want_transposed.  rows_out: the codes get that many rows (q [rows_out, cols], q_t
+    [cols, rows_out]), zero codes behind those of x (see :func:`padded_rows`).
     -> (q or None, q_t or None, amax, scale, scale_inv); the last three are fp32[1]."""
     want_transposed = want_transposed or out_t is not None
     if not (want_rowmajor or want_transposed):
@@ -319,15 +332,16 @@ def cast_dynamic(x: torch.Tensor, parts: torch.Tensor, fmt: int, margin: int = 0
     x = _as_2d(x)
     rows, cols = x.shape
     _f32_dev(parts, AMAX_PARTS, "cast_dynamic parts")
-    q = torch.empty((rows, cols), dtype=torch.uint8, device=x.device) if want_rowmajor else None
+    n = rows if rows_out is None else rows_out
+    q = torch.empty((n, cols), dtype=torch.uint8, device=x.device) if want_rowmajor else None
     if out_t is not None:
-        q_t = _codes_out(out_t, (cols, rows), x.device, "cast_dynamic out_t")
+        q_t = _codes_out(out_t, (cols, n), x.device, "cast_dynamic out_t")
     else:
-        q_t = torch.empty((cols, rows), dtype=torch.uint8, device=x.device) if want_transposed else None
+        q_t = torch.empty((cols, n), dtype=torch.uint8, device=x.device) if want_transposed else None
     dyn = torch.empty(3, dtype=torch.float32, device=x.device)
-    _check(load().odl_fp8_cast_dynamic(x.data_ptr(), _src_dtype(x), rows, cols, parts.data_ptr(), fmt, margin,
-                                       q.data_ptr() if q is not None else None, q_t.data_ptr() if q_t is not None else None,
-                                       dyn.data_ptr(), _stream()), "odl_fp8_cast_dynamic")
+    _check(load().odl_fp8_cast_dynamic_padded(x.data_ptr(), _src_dtype(x), rows, cols, n, parts.data_ptr(), fmt, margin,
+                                              q.data_ptr() if q is not None else None, q_t.data_ptr() if q_t is not None else None,
+                                              dyn.data_ptr(), _stream()), "odl_fp8_cast_dynamic")
     return q, q_t, dyn[0:1], dyn[1:2], dyn[2:3]
 
 
@@ -445,11 +459,12 @@ class MultiTensorPlan:
 
 
 def quantize_dynamic(x: torch.Tensor, fmt: int, margin: int = 0, want_rowmajor: bool = True, want_transposed: bool = True,
-                     parts: torch.Tensor | None = None, out_t: torch.Tensor | None = None):
+                     parts: torch.Tensor | None = None, out_t: torch.Tensor | None = None, rows_out: int | None = None):
     """Current scaling of one tensor in two launches: partial maxima, then a cast that derives the
     scale itself.  parts: the partial maxima, when the kernel that produced x already delivered
-    them (one launch then).  -> (q or None, q_t or None, amax, scale, scale_inv)."""
-    return cast_dynamic(x, amax_parts(x) if parts is None else parts, fmt, margin, want_rowmajor, want_transposed, out_t=out_t)
+    them (one launch then).  out_t, rows_out: as in :func:`cast_dynamic`.  -> (q or None, q_t or None, amax, scale, scale_inv)."""
+    return cast_dynamic(x, amax_parts(x) if parts is None else parts, fmt, margin, want_rowmajor, want_transposed, out_t=out_t,
+                        rows_out=rows_out)
 
 
 def _bf16_dense(t: torch.Tensor, what: str) -> torch.Tensor:
@@ -650,10 +665,10 @@ def gelu_bwd_amax_parts(dy: torch.Tensor, x: torch.Tensor):
     return dx, parts
 
 
-def quantize_rowcol(x: torch.Tensor, fmt: int, margin: int = 0):
+def quantize_rowcol(x: torch.Tensor, fmt: int, margin: int = 0, rows_out: int | None = None):
     """Rowwise recipe, both operands of one tensor in two passes over it:
     -> (q [rows, cols] scaled per row, s_row_inv [rows], q_t [cols, rows] scaled per column, s_col_inv [cols],
-        amax_row, amax_col)."""
+        amax_row, amax_col).  rows_out: as in :func:`cast_dynamic`."""
     x = _as_2d(x)
     rows, cols = x.shape
     pr, pc = -(-rows // 4) * 4, -(-cols // 4) * 4            # every vector starts on a 16-byte boundary (the GEMM wants that)
@@ -663,14 +678,15 @@ def quantize_rowcol(x: torch.Tensor, fmt: int, margin: int = 0):
     s_row, s_col = buf[o:o + rows], buf[o + pr:o + pr + cols]
     o = 2 * (pr + pc)
     s_row_inv, s_col_inv = buf[o:o + rows], buf[o + pr:o + pr + cols]
-    q = torch.empty((rows, cols), dtype=torch.uint8, device=x.device)
-    q_t = torch.empty((cols, rows), dtype=torch.uint8, device=x.device)
+    n = rows if rows_out is None else rows_out
+    q = torch.empty((n, cols), dtype=torch.uint8, device=x.device)
+    q_t = torch.empty((cols, n), dtype=torch.uint8, device=x.device)
     L, stream = load(), _stream()
     _check(L.odl_fp8_amax_rowcol(x.data_ptr(), _src_dtype(x), rows, cols, a_row.data_ptr(), a_col.data_ptr(), stream),
            "odl_fp8_amax_rowcol")
-    _check(L.odl_fp8_cast_rowcol(x.data_ptr(), _src_dtype(x), rows, cols, a_row.data_ptr(), a_col.data_ptr(), fmt, margin,
-                                 q.data_ptr(), q_t.data_ptr(), s_row.data_ptr(), s_row_inv.data_ptr(), s_col.data_ptr(),
-                                 s_col_inv.data_ptr(), stream), "odl_fp8_cast_rowcol")
+    _check(L.odl_fp8_cast_rowcol_padded(x.data_ptr(), _src_dtype(x), rows, cols, n, a_row.data_ptr(), a_col.data_ptr(), fmt, margin,
+                                        q.data_ptr(), q_t.data_ptr(), s_row.data_ptr(), s_row_inv.data_ptr(), s_col.data_ptr(),
+                                        s_col_inv.data_ptr(), stream), "odl_fp8_cast_rowcol")
     return q, s_row_inv, q_t, s_col_inv, a_row, a_col
 
 
@@ -716,31 +732,34 @@ def cast_transpose(x: torch.Tensor, scale: torch.Tensor, fmt: int, mode: int = S
 
 
 def cast_delayed(x: torch.Tensor, scale: torch.Tensor, fmt: int, amax_parts: torch.Tensor | None = None,
-                 want_rowmajor: bool = True, want_transposed: bool = False, out_t: torch.Tensor | None = None):
+                 want_rowmajor: bool = True, want_transposed: bool = False, out_t: torch.Tensor | None = None,
+                 rows_out: int | None = None):
     """The cast of the delayed-scaling recipe, one launch: codes with the per-tensor ``scale`` in force
     (row-major, transposed, or both), this step's partial maxima folded into ``amax_parts``
     (AMAX_PARTS floats of a role, accumulated, cleared by the next ``delayed_update``; None: nothing is
-    recorded), and 1/scale in a fresh 1-element tensor that later refreshes of ``scale`` do not touch.
+    recorded), and 1/scale in a fresh 1-element tensor that later refreshes of ``scale`` do not touch.  out_t, rows_out:
+    as in :func:`cast_dynamic`.
     -> (codes or None, codes_t or None, scale_inv[1])."""
     x = _as_2d(x)
     rows, cols = x.shape
     _f32_dev(scale, 1, "cast_delayed scale")
     if amax_parts is not None:
         _f32_dev(amax_parts, AMAX_PARTS, "cast_delayed amax_parts")
-    want_transposed = want_transposed or out_t is not None       # out_t: the caller's [cols, rows] buffer, as in cast_dynamic
+    want_transposed = want_transposed or out_t is not None
     if not (want_rowmajor or want_transposed):
         raise NativeError("cast_delayed: neither layout asked for")
-    out = torch.empty((rows, cols), dtype=torch.uint8, device=x.device) if want_rowmajor else None
+    n = rows if rows_out is None else rows_out
+    out = torch.empty((n, cols), dtype=torch.uint8, device=x.device) if want_rowmajor else None
     if out_t is not None:
-        _codes_out(out_t, (cols, rows), x.device, "cast_delayed out_t")
+        _codes_out(out_t, (cols, n), x.device, "cast_delayed out_t")
     else:
-        out_t = torch.empty((cols, rows), dtype=torch.uint8, device=x.device) if want_transposed else None
+        out_t = torch.empty((cols, n), dtype=torch.uint8, device=x.device) if want_transposed else None
     scale_inv = torch.empty(1, dtype=torch.float32, device=x.device)
-    _check(load().odl_fp8_cast_delayed(x.data_ptr(), _src_dtype(x), rows, cols, scale.data_ptr(), fmt,
-                                       out.data_ptr() if out is not None else None,
-                                       out_t.data_ptr() if out_t is not None else None,
-                                       amax_parts.data_ptr() if amax_parts is not None else None, scale_inv.data_ptr(), _stream()),
-           "odl_fp8_cast_delayed")
+    _check(load().odl_fp8_cast_delayed_padded(x.data_ptr(), _src_dtype(x), rows, cols, n, scale.data_ptr(), fmt,
+                                              out.data_ptr() if out is not None else None,
+                                              out_t.data_ptr() if out_t is not None else None,
+                                              amax_parts.data_ptr() if amax_parts is not None else None, scale_inv.data_ptr(),
+                                              _stream()), "odl_fp8_cast_delayed")
     return out, out_t, scale_inv
 
 

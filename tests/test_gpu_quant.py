@@ -432,3 +432,35 @@ def test_kernels_against_the_committed_golden_vectors(N, name, fmt):
             N.delayed_update(hist, scale, scale_inv, fmts, 0, N.AMAX_MAX if case["algo"] == "max" else N.AMAX_MOST_RECENT)
             assert_f32_bits_equal(scale, torch.tensor([after[t]]), f"scale after step {t}")
         assert_f32_bits_equal(hist[:, 0], torch.from_numpy(_f32(case["final_history_f32_hex"]).copy()), "final history")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols,rows_out", [(16, 8, 128), (48, 72, 128), (112, 64, 128), (144, 136, 256), (1008, 80, 1024),
+                                                (128, 64, 128), (7, 13, 16), (130, 24, 256)])
+def test_padded_casts_are_the_plain_ones_with_zero_codes_behind(N, rows, cols, rows_out, dtype):
+    """Row counts on both sides of the 128-row tile and of the 1024-element spans, shapes that take the element-at-a-time
+    route (13 columns), the three casts with both layouts and each alone."""
+    x = seeded_bf16((rows, cols), seed=rows + cols).to(dtype).cuda()
+    parts, scale = N.amax_parts(x), torch.full((1,), 3.0, device="cuda")
+
+    def check(got, got_t, ref, ref_t):
+        for g, r in ((got, ref), (got_t, None if ref_t is None else ref_t)):
+            assert (g is None) == (r is None)
+        if got is not None:
+            assert got.shape == (rows_out, cols) and torch.equal(got[:rows], ref) and not got[rows:].any()
+        if got_t is not None:
+            assert got_t.shape == (cols, rows_out) and torch.equal(got_t[:, :rows], ref_t) and not got_t[:, rows:].any()
+
+    for want, want_t in ((True, True), (True, False), (False, True)):
+        ref = N.cast_dynamic(x, parts, O.E5M2, 0, want, want_t)
+        got = N.cast_dynamic(x, parts, O.E5M2, 0, want, want_t, rows_out=rows_out)
+        check(got[0], got[1], ref[0], ref[1])
+        assert all(torch.equal(a, b) for a, b in zip(got[2:], ref[2:]))
+        strips = [torch.zeros(N.AMAX_PARTS, device="cuda") for _ in range(2)]
+        ref = N.cast_delayed(x, scale, O.E4M3, strips[0], want, want_t)
+        got = N.cast_delayed(x, scale, O.E4M3, strips[1], want, want_t, rows_out=rows_out)
+        check(got[0], got[1], ref[0], ref[1])
+        assert torch.equal(strips[0].max(), strips[1].max()) and torch.equal(got[2], ref[2])
+    ref, got = N.quantize_rowcol(x, O.E4M3), N.quantize_rowcol(x, O.E4M3, rows_out=rows_out)
+    check(got[0], got[2], ref[0], ref[2])
+    assert torch.equal(got[1], ref[1]) and torch.equal(got[3], ref[3])
