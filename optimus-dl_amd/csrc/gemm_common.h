@@ -255,8 +255,11 @@ __device__ __forceinline__ void epilogue_staged_accumulate(const GemmArgs &g, v1
     }
 }
 
-// launchers implemented in gemm_tiled.hip / gemm_pipe.hip / gemm_stream.hip (fa, fb: odl_fp8_format of A and B)
+// launchers implemented in gemm_tiled.hip / gemm_thin.hip / gemm_pipe.hip / gemm_stream.hip (fa, fb: odl_fp8_format of A and B)
 void launch_gemm_tiled(int variant, int fa, int fb, const GemmArgs &g, hipStream_t stream);
+// operand rows that the busiest compute unit of a thin launch fetches per K step: what the launch costs (gemm_thin.hip)
+int gemm_thin_rows(int64_t M, int64_t N, int num_cus);
+void launch_gemm_thin(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
 void launch_gemm_pipe(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
 bool gemm_stream_accepts(const GemmArgs &g);
 void launch_gemm_stream(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);

@@ -4,6 +4,7 @@
 //
 // Both operands are K-contiguous 8-bit codes ("NT").  Kernels:
 //   gemm_tiled.hip : BM x BN block tiles through two LDS stages
+//   gemm_thin.hip  : small tiles, the waves of a block share K: outputs of few tiles (N % 4 == 0, K % 128 == 0)
 //   gemm_pipe.hip  : 256x256 tile, one wave per SIMD, explicit software pipeline
 //   gemm_stream.hip: the same pipeline running across tile boundaries, epilogue under the
 //                    next tile's MFMAs (any M; N, K multiples of 128); with a split over K for
@@ -98,8 +99,9 @@ static const Variant kVariants[] = {
     {"256x256x128 4 waves, software-pipelined, persistent (K % 256 == 0)", 256, 256, 256, 1.10f},
     {"256x256x128 4 waves, software-pipelined, one tile per block", 256, 256, 256, 0.50f},
     {"256x256x128 4 waves, streaming across tiles, folded epilogue (N, K multiples of 128)", 256, 256, 256, 1.25f},
+    {"thin tiles, 8 waves sharing K (N % 4 == 0, K % 128 == 0)", 64, 64, 512, 0.0f},
 };
-constexpr int kPipeVariant = 5, kPipeOneTileVariant = 6, kStreamVariant = 7;
+constexpr int kPipeVariant = 5, kPipeOneTileVariant = 6, kStreamVariant = 7, kThinVariant = 8;
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 // Forced kernel variant of the calling host thread (-1: choose by shape).  Thread-local: a test or a tuning
 // sweep that pins a variant cannot change the kernels another thread (e.g. the autograd worker) launches.
@@ -123,15 +125,29 @@ static void launch_gemm_generic(int fa, int fb, const GemmArgs &g, hipStream_t s
 
 static int cu_count() { return device_cu_count(); }
 
-static int choose_variant(int64_t M, int64_t N, bool stream_ok) {
+// Whether the waves of a block sharing K (gemm_thin.hip) beat one 128 x 128 tile per compute unit.  A K step takes the thin
+// kernel 2.7 ns per operand row that the busiest unit fetches, the four-stage 128 x 128 kernel 0.43 us: even at 160 rows,
+// and the line is drawn 10 % below.  Measured on both sides, thin against 128 x 128: 128 rows (32 x 14336 x 4096) 18.6
+// against 21.1 us, 96 rows (512 x 768 x 3072) 10.1 against 13.8, 48 rows (32 x 4096 x 14336) 19.2 against 53.4; 192 rows
+// (768 x 768 x 2048) 13.1 against 10.3, (256 x 4096 x 4096) 22.1 against 17.5.  K under 2048 (fewer than two steps per
+// wave) is left to the tiled kernels: there is no chain to shorten (128 x 3072 x 768: 5.6 against 5.9).
+static bool thin_ok(int64_t M, int64_t N) { return N % 4 == 0 && ((M + 127) / 128) * ((N + 127) / 128) <= cu_count(); }
+
+static bool thin_pays(int64_t M, int64_t N, int64_t K) {
     const int cus = cu_count();
+    return K >= 2048 && thin_ok(M, N) && gemm_thin_rows(M, N, cus) < 145;
+}
+
+static int choose_variant(int64_t M, int64_t N, int64_t K, bool stream_ok) {
+    const int cus = cu_count();
+    if (thin_pays(M, N, K)) return kThinVariant;
     // an output of at most cus / 2 tiles of 256 x 256 leaves half the chip idle with the big tiles: the 128 x 128
     // kernel (two blocks per compute unit) spreads it four times wider (measured 15-20 % faster than either
     // 256-wide kernel at 8192 x 1024, 8192 x 768 and 2048 x 4096 outputs, K = 768 .. 4096)
     if (((M + 255) / 256) * ((N + 255) / 256) * 2 <= cus) return 4;
     int best = 2;
     double best_score = -1.0;
-    for (int v = 2; v < kNumVariants; ++v) {                       // variant 1 (one wave per SIMD) only by explicit request
+    for (int v = 2; v <= kStreamVariant; ++v) {                       // variant 1 (one wave per SIMD) only by explicit request
         if (v == kStreamVariant && !stream_ok) continue;
         const Variant &cfg = kVariants[v];
         const int64_t tiles = ((M + cfg.bm - 1) / cfg.bm) * ((N + cfg.bn - 1) / cfg.bn);
@@ -217,11 +233,13 @@ extern "C" int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, in
     // C = C + product is an epilogue of the kernels whose tiles end in a separate output phase; the streaming kernel
     // stores a tile under the next tile's MFMAs, where nothing can wait for the old values of C
     const bool stream_ok = tiled_ok && lim32 && N % 128 == 0 && K >= 512 && !accumulate;
-    int variant = t_forced_variant >= 0 ? t_forced_variant : (tiled_ok ? choose_variant(M, N, stream_ok) : 0);
+    int variant = t_forced_variant >= 0 ? t_forced_variant : (tiled_ok ? choose_variant(M, N, K, stream_ok) : 0);
     if (variant != 0 && !tiled_ok) variant = 0;
     // the pipelined kernel walks K in pairs of 128-byte steps
     const bool pipe_ok = tiled_ok && K % 256 == 0 && lim32;
     if ((variant == kPipeVariant || variant == kPipeOneTileVariant) && !pipe_ok) variant = 2;
+
+    if (variant == kThinVariant && !thin_ok(M, N)) variant = 4;
 
     GemmArgs g;
     g.a = a; g.b = b; g.c = c; g.sa = sa_inv; g.sb = sb_inv; g.bias = bias;
@@ -240,6 +258,7 @@ extern "C" int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, in
         variant = pipe_ok ? kPipeVariant : 2;
     }
     if (variant == 0) launch_gemm_generic(fmt_a, fmt_b, g, stream);
+    else if (variant == kThinVariant) launch_gemm_thin(fmt_a, fmt_b, g, cu_count(), stream);
     else if (variant == kPipeVariant) launch_gemm_pipe(fmt_a, fmt_b, g, cu_count(), stream);
     else if (variant == kPipeOneTileVariant) launch_gemm_pipe(fmt_a, fmt_b, g, 1 << 30, stream);
     else if (variant == kStreamVariant) { attach_clock_probe(g); launch_gemm_stream(fmt_a, fmt_b, g, cu_count(), stream); }
@@ -334,6 +353,7 @@ extern "C" int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t 
 //   split                       : 0.96 us per step of a run + 9 us (pipeline fill, the fp32 epilogue, the second launch)
 //                                 + the partial results, splits x M x N floats written and read back, at 2.7 TB/s in all
 //   each bounded below by its operand traffic (tiles x panel bytes) at about 12 TB/s out of the caches.
+//   one launch, thin tiles      : 4 us + 2.7 ns per K step and operand row of the busiest compute unit (see thin_pays)
 // The runs of a split must fit the compute units at once, and a split must win by 10 %.
 // k_slow: an operand is stored with the contraction index slow (odl_fp8_gemm_layouts), which only the streaming
 // kernel reads: the 128 x 128 kernel is then not an alternative.
@@ -353,6 +373,10 @@ extern "C" int odl_fp8_gemm_split_count(int64_t M, int64_t N, int64_t K, int k_s
         const double small_traffic_us = (double)small_tiles * 256.0 * (double)K / 12.0e6;
         if (small < small_traffic_us) small = small_traffic_us;
         if (small < whole) whole = small;
+    }
+    if (!k_slow && thin_pays(M, N, K)) {
+        const double thin = 4.0 + 0.0027 * (double)gemm_thin_rows(M, N, cus) * (double)steps;
+        if (thin < whole) whole = thin;
     }
     double best = whole;
     int best_splits = 1;

@@ -723,3 +723,47 @@ def test_streaming_kernel_any_number_of_rows(N, M, epilogue, out_dtype):
                                [sa.cuda()] * 2, [sb.cuda()] * 2, out_dtype=out_dtype)
         ref = O.t_gemm_nt(aq[:, :512].contiguous(), bq[:, :512].contiguous(), O.E4M3, O.E4M3, sa, sb, want_f32=True)[1]
         assert max_rel_err(summed, 2 * ref) <= TOL
+
+
+@pytest.mark.parametrize("shape", [(1, 4, 128), (16, 4096, 1024), (17, 60, 1152), (32, 14336, 640), (33, 132, 3072), (48, 768, 8192),
+                                   (250, 764, 2048), (512, 768, 3072)])
+@pytest.mark.parametrize("fmts", [(O.E4M3, O.E4M3), (O.E5M2, O.E4M3)])
+def test_thin_tiles(N, shape, fmts):
+    """Waves that share K (outputs of few tiles): every tile form, ragged edges, fewer K steps than waves and counts that
+    are no multiple of them.  Exactly summable operands, so the bits have to be those of the generic kernel; row scales,
+    a bias and the sum into an existing output take the same fp32 steps in both."""
+    M, Nn, K = shape
+    fa, fb = fmts
+    g = torch.Generator().manual_seed(M + Nn + K)
+    vals = torch.tensor([0.0, 1.0, -1.0, 2.0, -2.0, 0.5, -0.5, 4.0])
+    a = vals[torch.randint(0, 8, (M, K), generator=g)].to(O.TORCH_FP8[fa]).view(torch.uint8).cuda()
+    b = vals[torch.randint(0, 8, (Nn, K), generator=g)].to(O.TORCH_FP8[fb]).view(torch.uint8).cuda()
+    sa, sb = (torch.rand(M, generator=g) + 0.5).cuda(), (torch.rand(Nn, generator=g) + 0.5).cuda()
+    bias, old = torch.randn(Nn, generator=g).cuda(), torch.randn((M, Nn), generator=g).cuda()
+    got = {}
+    for variant in (0, 8):
+        N.gemm_set_variant(variant)
+        assert variant == 0 or "thin" in N.gemm_variants()[variant]
+        got[variant] = [N.gemm_nt(a, b, fa, fb, sa[:1].contiguous(), sb[:1].contiguous(), out_dtype=torch.float32)]
+        for dtype in (torch.bfloat16, torch.float32):
+            got[variant].append(N.gemm_nt(a, b, fa, fb, sa, sb, bias=bias, out_dtype=dtype))
+            got[variant].append(N.gemm_nt(a, b, fa, fb, sa, sb, out=old.to(dtype, copy=True), accumulate=True))
+    N.gemm_set_variant(-1)
+    for k, (want, out) in enumerate(zip(got[0], got[8])):
+        assert torch.equal(want, out), f"output {k}: {(want.float() - out.float()).abs().max()}"
+
+
+@pytest.mark.parametrize("k_steps", [1, 2, 3, 4, 5, 6, 7, 9, 13])
+def test_four_stage_tiles_at_every_pipeline_depth(N, k_steps):
+    """One 128 x 128 tile per compute unit where the waves do not share K: as test_few_tile_outputs_at_every_pipeline_depth,
+    with the kernel pinned."""
+    M, Nn, K = 384, 200, 128 * k_steps
+    one = torch.ones(1)
+    a = torch.zeros((M, K), dtype=torch.uint8)
+    cols = (7 * torch.arange(M)) % K
+    a[torch.arange(M), cols] = 0x38                                    # 1.0 in E4M3
+    b = O.t_cast(seeded_bf16((Nn, K), 1.0, 80 + k_steps).float(), one, O.E4M3)
+    N.gemm_set_variant(4)
+    got = N.gemm_nt(a.cuda(), b.cuda(), O.E4M3, O.E4M3, one.cuda(), one.cuda(), out_dtype=torch.float32).cpu()
+    N.gemm_set_variant(-1)
+    assert torch.equal(got, O.t_decode(b, O.E4M3)[:, cols].t())
