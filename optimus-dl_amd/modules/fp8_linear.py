@@ -45,6 +45,7 @@ import torch.nn.functional as F
 from .. import native
 from .amp import state as _state
 from .amp.fp8 import FP8Recipe
+from .calls import apply, untraced
 
 logger = logging.getLogger(__name__)
 _warned: set[str] = set()
@@ -532,7 +533,7 @@ class _Fp8LinearGroupFn(torch.autograd.Function):
         return (dx, None, None, None, *grads)
 
 
-@torch.compiler.disable
+@untraced
 def linear_group(x: torch.Tensor, modules: "tuple[FP8Linear, ...]") -> tuple[torch.Tensor, ...] | None:
     """``tuple(m(x) for m in modules)`` as one autograd node (see ``_Fp8LinearGroupFn``), or None where the members
     cannot run that way (no recipe, a block-scaled recipe, shapes the FP8 path refuses): the caller
@@ -554,7 +555,7 @@ def linear_group(x: torch.Tensor, modules: "tuple[FP8Linear, ...]") -> tuple[tor
         m.fp8_calls += 1
         m._note_grad_mode()
         params += [m.weight, m.bias]
-    outs = _Fp8LinearGroupFn.apply(x2d, recipe, compute_dtype, tuple(modules), *params)
+    outs = apply(_Fp8LinearGroupFn, x2d, recipe, compute_dtype, tuple(modules), *params)
     return tuple(y.reshape(*x.shape[:-1], m.out_features) for y, m in zip(outs, modules))
 
 
@@ -580,8 +581,10 @@ class SiblingGroup:
     def clear(self) -> None:
         self.pending, self.key, self.x = {}, None, None
 
-    @torch.compiler.disable          # like FP8Linear._forward_fp8: runs as written, between the compiled parts of a model
+    @untraced          # like FP8Linear._forward_fp8: runs as written, between the compiled parts of a model
     def forward(self, member: "FP8Linear", x: torch.Tensor) -> torch.Tensor:
+        if not self.pending and (self.misses or not torch.is_grad_enabled() or not x.requires_grad):
+            return member._forward_fp8(x)
         # the same values at the same address: the same tensor object, or another handle on it (a graph compiler hands
         # the pieces of a model it runs separately fresh handles on the same storage)
         key = (x.data_ptr(), _state.tensor_version(x), tuple(x.shape), tuple(x.stride()), x.dtype, x.requires_grad)
@@ -815,7 +818,7 @@ class FP8Linear(nn.Linear):
     # The FP8 path calls the native library through ctypes and keeps per-step state on the recipe: a graph
     # compiler (the reference has a torch.compile transform, model_transforms/compile.py) must not trace into
     # it.  Marked like this it runs as written, between the compiled parts of the model.
-    @torch.compiler.disable
+    @untraced
     def _forward_fp8(self, x: torch.Tensor) -> torch.Tensor:
         recipe = _state.active_recipe()
         if recipe is None or not self._fp8_eligible(x):
@@ -831,7 +834,7 @@ class FP8Linear(nn.Linear):
             x2d = _converted_input(recipe, x2d, compute_dtype)
         self.fp8_calls += 1
         self._note_grad_mode()
-        y = _Fp8LinearFn.apply(x2d, self.weight, self.bias, self, recipe, compute_dtype)
+        y = apply(_Fp8LinearFn, x2d, self.weight, self.bias, self, recipe, compute_dtype)
         return y.reshape(*x.shape[:-1], self.out_features)
 
     def extra_repr(self) -> str:

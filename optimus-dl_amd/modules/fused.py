@@ -22,6 +22,7 @@ import torch.nn.functional as F
 from .. import native
 from .amp import state as _state
 from .amp.fp8 import FP8Recipe
+from .calls import apply, untraced
 from .fp8_linear import FP8Linear
 
 
@@ -53,13 +54,13 @@ class _SwiGLUFn(torch.autograd.Function):
         return dgate, dup, None
 
 
-@torch.compiler.disable
+@untraced
 def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """silu(gate) * up; fused (and feeding the next FP8 Linear) when an FP8 recipe is active."""
     recipe = _state.active_recipe()
     if recipe is None or not _bf16_cuda(gate, up) or gate.shape != up.shape or gate.numel() % 8:
         return F.silu(gate) * up
-    return _SwiGLUFn.apply(gate, up, recipe)
+    return apply(_SwiGLUFn, gate, up, recipe)
 
 
 # ---------------------------------------------------------------- in-place re-classing
@@ -133,7 +134,7 @@ class _RMSNormFn(torch.autograd.Function):
         return (dx if ctx.needs_input_grad[0] else None), (dw.to(weight.dtype) if ctx.needs_input_grad[1] else None), None, None
 
 
-@torch.compiler.disable
+@untraced
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor | None:
     """Fused RMSNorm when an FP8 recipe is active and the kernel takes the input; else None."""
     recipe = _state.active_recipe()
@@ -144,7 +145,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor |
     cols = x.shape[-1]
     if cols % 8 or cols < 8 or cols > 8192 or weight.numel() != cols or x.numel() == 0:
         return None
-    return _RMSNormFn.apply(x, weight, float(eps), recipe)
+    return apply(_RMSNormFn, x, weight, float(eps), recipe)
 
 
 class _FusedRMSNormForward(_Reclassed):
@@ -194,7 +195,7 @@ class _LayerNormFn(torch.autograd.Function):
                 db.to(ctx.bias_dtype) if ctx.bias_dtype is not None and ctx.needs_input_grad[2] else None, None, None)
 
 
-@torch.compiler.disable
+@untraced
 def layernorm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, eps: float) -> torch.Tensor | None:
     """Fused LayerNorm when an FP8 recipe is active and the kernel takes the input; else None."""
     recipe = _state.active_recipe()
@@ -205,7 +206,7 @@ def layernorm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, 
     cols = x.shape[-1]
     if cols % 8 or cols < 8 or cols > 4096 or weight is None or weight.numel() != cols or x.numel() == 0:
         return None
-    return _LayerNormFn.apply(x, weight, bias, float(eps), recipe)
+    return apply(_LayerNormFn, x, weight, bias, float(eps), recipe)
 
 
 class _FusedLayerNormForward(_Reclassed):
@@ -256,13 +257,13 @@ class _GeluFn(torch.autograd.Function):
         return dx, None
 
 
-@torch.compiler.disable
+@untraced
 def gelu(x: torch.Tensor) -> torch.Tensor | None:
     """Fused GELU when an FP8 recipe is active and the input is a bf16 GPU tensor; else None."""
     recipe = _state.active_recipe()
     if recipe is None or not _bf16_cuda(x) or x.numel() % 8 or x.numel() == 0:
         return None
-    return _GeluFn.apply(x, recipe)
+    return apply(_GeluFn, x, recipe)
 
 
 class _FusedGeluForward(_Reclassed):

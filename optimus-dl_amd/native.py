@@ -195,11 +195,13 @@ def _check(status: int, what: str) -> None:
 # the handle of the current stream without building a torch.cuda.Stream object around it: that constructor and the
 # device look-ups on its way cost 10 us a call, 0.4 ms over the 40 launches of a small step
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+# (whoever asks for a stream already holds a GPU tensor: no lazy initialisation to look after)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def _stream() -> int:
     if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
+        return _raw_stream(_current_device())
     return torch.cuda.current_stream().cuda_stream
 
 
@@ -338,11 +340,11 @@ def cast_dynamic(x: torch.Tensor, parts: torch.Tensor, fmt: int, margin: int = 0
         q_t = _codes_out(out_t, (cols, n), x.device, "cast_dynamic out_t")
     else:
         q_t = torch.empty((cols, n), dtype=torch.uint8, device=x.device) if want_transposed else None
-    dyn = torch.empty(3, dtype=torch.float32, device=x.device)
+    dyn = torch.empty((3, 1), dtype=torch.float32, device=x.device)
     _check(load().odl_fp8_cast_dynamic_padded(x.data_ptr(), _src_dtype(x), rows, cols, n, parts.data_ptr(), fmt, margin,
                                               q.data_ptr() if q is not None else None, q_t.data_ptr() if q_t is not None else None,
                                               dyn.data_ptr(), _stream()), "odl_fp8_cast_dynamic")
-    return q, q_t, dyn[0:1], dyn[1:2], dyn[2:3]
+    return (q, q_t, *dyn.unbind())
 
 
 NOALLOC_MAX_ELEMS = 1 << 31            # ODL_FP8_NOALLOC_MAX_ELEMS

@@ -418,3 +418,59 @@ def test_forward_context_fallbacks_follow_the_reference_evaluator(monkeypatch):
     assert len(made) == 2                                          # another configuration, another recipe
     with tc.forward_context(cfg, cpu):                             # a recipe off the GPU: ordinary bf16 autocast (fp8.py:488)
         assert torch.get_autocast_dtype("cpu") == torch.bfloat16
+
+
+def test_functions_without_a_graph_run_their_forward_only():
+    """No graph recorded: the forward alone, with nothing reported as needing a gradient; anything that has to see the
+    autograd function still does."""
+    from optimus_dl_amd.modules.calls import apply
+
+    class Double(torch.autograd.Function):
+        seen = []
+
+        @staticmethod
+        def forward(ctx, x, w):
+            Double.seen.append((type(ctx).__name__, tuple(ctx.needs_input_grad)))
+            ctx.save_for_backward(x, w)
+            return x * w
+
+        @staticmethod
+        def backward(ctx, dy):
+            x, w = ctx.saved_tensors
+            return dy * w, dy * x
+
+    x, w = torch.randn(3), torch.randn(3, requires_grad=True)
+    with torch.no_grad():
+        y = apply(Double, x, w)
+    assert Double.seen.pop() == ("_NoGraph", (False, False)) and not y.requires_grad and torch.equal(y, x * w.detach())
+    apply(Double, x, w).sum().backward()
+    assert Double.seen.pop()[1] == (False, True) and torch.equal(w.grad, x)
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        apply(Double, x, w)
+    assert Double.seen.pop()[0] != "_NoGraph"
+    with torch.no_grad(), pytest.raises(RuntimeError, match="setup_context|vmap"):
+        torch.vmap(lambda a: apply(Double, a, w))(torch.randn(2, 3))
+
+
+def test_untraced_functions_stay_out_of_compiled_graphs():
+    from optimus_dl_amd.modules.calls import untraced
+
+    seen = []
+
+    @untraced
+    def inner(x):
+        seen.append(torch.compiler.is_compiling())
+        return x + 1
+
+    graphs = []
+
+    def backend(gm, _):
+        graphs.append(gm)
+        return gm.forward
+
+    def model(x):
+        return inner(x * 2) * 3
+
+    x = torch.ones(4)
+    assert torch.equal(torch.compile(model, backend=backend)(x), model(x))
+    assert seen == [False, False] and len(graphs) == 2          # what lies before and behind the call, never the call
