@@ -161,6 +161,21 @@ static int choose_variant(int64_t M, int64_t N, int64_t K, bool stream_ok) {
     return best;
 }
 
+// Rows of A that the streaming kernel should leave to a second launch (0: none).  Its 256 x 256 tiles go round the chip one
+// per compute unit, and a last round of few tiles costs as much as a full one.  Those rows as 128 x 128 tiles take about half
+// a round with one tile per unit, 0.7 with two, and 4 us for the launch.  With one tile that pays from 16 K steps on
+// (5000 x 4096 x 2048: 47.8 -> 43.4 us, x 14336: 256 -> 216; 4096 x 4864 x 4096: 82.2 -> 68.8), with two from 32
+// (11264 x 2048 x 4096: 91.5 -> 86.2, 50304 x 768 x 8192: 292 -> 272; 4016 x 5632 x 2048 would go from 49.1 to 53.7).
+// Same K order, same bits.
+static int64_t tail_rows(int64_t M, int64_t N, int64_t K) {
+    const int cus = cu_count();
+    const int64_t tiles_n = (N + 255) / 256, tiles = ((M + 255) / 256) * tiles_n;
+    if (K < 2048 || tiles <= cus || tiles_n > cus || tiles % cus == 0) return 0;
+    const int64_t rest = M - tiles / cus * cus / tiles_n * 256;
+    const int64_t rest_tiles = ((rest + 127) / 128) * ((N + 127) / 128);
+    return rest > 0 && rest_tiles <= (K >= 4096 ? 2 : 1) * (int64_t)cus ? rest : 0;
+}
+
 }  // namespace odl
 
 using namespace odl;
@@ -206,40 +221,35 @@ extern "C" int odl_fp8_gemm_set_variant(int variant) {
     return ODL_OK;
 }
 
-extern "C" int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b,
-                               const float *sa_inv, int64_t sa_n, const float *sb_inv, int64_t sb_n, const void *bias,
-                               int bias_dtype, void *c, int out_dtype, int accumulate, odl_stream_t stream_) {
-    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
-    if (!a || !b || !c || !sa_inv || !sb_inv) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: null pointer");
-    if (M < 0 || N < 0 || K < 0) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: negative size");
-    if ((fmt_a != ODL_FP8_E4M3 && fmt_a != ODL_FP8_E5M2) || (fmt_b != ODL_FP8_E4M3 && fmt_b != ODL_FP8_E5M2))
-        return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: formats %d, %d", fmt_a, fmt_b);
-    if (sa_n != 1 && sa_n != M) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: sa_n=%lld is neither 1 nor M", (long long)sa_n);
-    if (sb_n != 1 && sb_n != N) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: sb_n=%lld is neither 1 nor N", (long long)sb_n);
-    if (out_dtype != ODL_BF16 && out_dtype != ODL_F32) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: out_dtype %d", out_dtype);
-    if (bias && bias_dtype != ODL_F32) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: bias must be fp32 (bias_dtype %d)", bias_dtype);
-    if (K % 16 != 0) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt: K=%lld must be a multiple of 16", (long long)K);
-    if ((reinterpret_cast<uintptr_t>(a) & 15) || (reinterpret_cast<uintptr_t>(b) & 15))
-        return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt: operands must be 16-byte aligned");
-    if (reinterpret_cast<uintptr_t>(c) & 15) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt: output must be 16-byte aligned");
-    if ((sa_n > 1 && (reinterpret_cast<uintptr_t>(sa_inv) & 15)) || (sb_n > 1 && (reinterpret_cast<uintptr_t>(sb_inv) & 15)) ||
-        (bias && (reinterpret_cast<uintptr_t>(bias) & 15)))
-        return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt: scale vectors and bias must be 16-byte aligned");
-    if (M == 0 || N == 0) return ODL_OK;
-
+// The launch of checked arguments.  launch_as: the variant to use (-1: the forced one, or the choice by shape).
+static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b, const float *sa_inv, int64_t sa_n,
+                           const float *sb_inv, int64_t sb_n, const void *bias, void *c, int out_dtype, int accumulate, int launch_as,
+                           hipStream_t stream) {
     const bool tiled_ok = K >= 128 && K % 128 == 0 && (double)M * (double)K < 4294967296.0 && (double)N * (double)K < 4294967296.0;
     // the pipelined and the streaming kernel address rows with 32-bit byte offsets
     const bool lim32 = (double)(M + 256) * (double)K < 2147483648.0 && (double)(N + 256) * (double)K < 2147483648.0;
     // C = C + product is an epilogue of the kernels whose tiles end in a separate output phase; the streaming kernel
     // stores a tile under the next tile's MFMAs, where nothing can wait for the old values of C
     const bool stream_ok = tiled_ok && lim32 && N % 128 == 0 && K >= 512 && !accumulate;
-    int variant = t_forced_variant >= 0 ? t_forced_variant : (tiled_ok ? choose_variant(M, N, K, stream_ok) : 0);
+    int variant = launch_as >= 0 ? launch_as : t_forced_variant >= 0 ? t_forced_variant : (tiled_ok ? choose_variant(M, N, K, stream_ok) : 0);
     if (variant != 0 && !tiled_ok) variant = 0;
     // the pipelined kernel walks K in pairs of 128-byte steps
     const bool pipe_ok = tiled_ok && K % 256 == 0 && lim32;
     if ((variant == kPipeVariant || variant == kPipeOneTileVariant) && !pipe_ok) variant = 2;
 
     if (variant == kThinVariant && !thin_ok(M, N)) variant = 4;
+
+    if (variant == kStreamVariant && t_forced_variant < 0 && launch_as < 0) {
+        const int64_t rest = tail_rows(M, N, K), head = M - rest;
+        if (rest > 0) {
+            const int64_t esz = out_dtype == ODL_BF16 ? 2 : 4;
+            const int rc = gemm_nt_checked(a, b, head, N, K, fmt_a, fmt_b, sa_inv, sa_n == 1 ? 1 : head, sb_inv, sb_n, bias, c, out_dtype, accumulate,
+                                           kStreamVariant, stream);
+            if (rc != ODL_OK) return rc;
+            return gemm_nt_checked(a + head * K, b, rest, N, K, fmt_a, fmt_b, sa_n == 1 ? sa_inv : sa_inv + head, sa_n == 1 ? 1 : rest, sb_inv, sb_n,
+                                   bias, reinterpret_cast<uint8_t *>(c) + head * N * esz, out_dtype, accumulate, 4, stream);
+        }
+    }
 
     GemmArgs g;
     g.a = a; g.b = b; g.c = c; g.sa = sa_inv; g.sb = sb_inv; g.bias = bias;
@@ -264,6 +274,29 @@ extern "C" int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, in
     else if (variant == kStreamVariant) { attach_clock_probe(g); launch_gemm_stream(fmt_a, fmt_b, g, cu_count(), stream); }
     else launch_gemm_tiled(variant, fmt_a, fmt_b, g, stream);
     return check_launch("odl_fp8_gemm_nt");
+}
+
+extern "C" int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b,
+                               const float *sa_inv, int64_t sa_n, const float *sb_inv, int64_t sb_n, const void *bias,
+                               int bias_dtype, void *c, int out_dtype, int accumulate, odl_stream_t stream_) {
+    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+    if (!a || !b || !c || !sa_inv || !sb_inv) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: null pointer");
+    if (M < 0 || N < 0 || K < 0) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: negative size");
+    if ((fmt_a != ODL_FP8_E4M3 && fmt_a != ODL_FP8_E5M2) || (fmt_b != ODL_FP8_E4M3 && fmt_b != ODL_FP8_E5M2))
+        return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: formats %d, %d", fmt_a, fmt_b);
+    if (sa_n != 1 && sa_n != M) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: sa_n=%lld is neither 1 nor M", (long long)sa_n);
+    if (sb_n != 1 && sb_n != N) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: sb_n=%lld is neither 1 nor N", (long long)sb_n);
+    if (out_dtype != ODL_BF16 && out_dtype != ODL_F32) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: out_dtype %d", out_dtype);
+    if (bias && bias_dtype != ODL_F32) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: bias must be fp32 (bias_dtype %d)", bias_dtype);
+    if (K % 16 != 0) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt: K=%lld must be a multiple of 16", (long long)K);
+    if ((reinterpret_cast<uintptr_t>(a) & 15) || (reinterpret_cast<uintptr_t>(b) & 15))
+        return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt: operands must be 16-byte aligned");
+    if (reinterpret_cast<uintptr_t>(c) & 15) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt: output must be 16-byte aligned");
+    if ((sa_n > 1 && (reinterpret_cast<uintptr_t>(sa_inv) & 15)) || (sb_n > 1 && (reinterpret_cast<uintptr_t>(sb_inv) & 15)) ||
+        (bias && (reinterpret_cast<uintptr_t>(bias) & 15)))
+        return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt: scale vectors and bias must be 16-byte aligned");
+    if (M == 0 || N == 0) return ODL_OK;
+    return gemm_nt_checked(a, b, M, N, K, fmt_a, fmt_b, sa_inv, sa_n, sb_inv, sb_n, bias, c, out_dtype, accumulate, -1, stream);
 }
 
 extern "C" int odl_fp8_gemm_nt_sum(int pairs, const uint8_t *const *a, const uint8_t *const *b, const int64_t *K, int64_t M, int64_t N,

@@ -767,3 +767,22 @@ def test_four_stage_tiles_at_every_pipeline_depth(N, k_steps):
     got = N.gemm_nt(a.cuda(), b.cuda(), O.E4M3, O.E4M3, one.cuda(), one.cuda(), out_dtype=torch.float32).cpu()
     N.gemm_set_variant(-1)
     assert torch.equal(got, O.t_decode(b, O.E4M3)[:, cols].t())
+
+
+@pytest.mark.parametrize("shape", [(4016, 5632, 4096), (6784, 2816, 2048), (5000, 4096, 2176), (50304, 768, 4096)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_last_round_in_smaller_tiles_has_the_same_bits(N, shape, out_dtype):
+    """Outputs whose last round of 256 x 256 tiles would leave most of the chip idle are finished by a second launch:
+    the rows meet without a gap, row scales and bias go along, nothing behind the output is written."""
+    M, Nn, K = shape
+    aq, bq = (torch.randint(0, 0x78, (r, K), dtype=torch.uint8, device="cuda") for r in (M, Nn))
+    g = torch.Generator().manual_seed(M)
+    sa, sb = (torch.rand(M, generator=g) + 0.5).cuda(), (torch.rand(Nn, generator=g) + 0.5).cuda()
+    bias = torch.randn(Nn, generator=g).cuda()
+    for args, kw in (((sa[:1].contiguous(), sb[:1].contiguous()), {}), ((sa, sb), {"bias": bias})):
+        guarded = torch.full((M + 128, Nn), 7.0, dtype=out_dtype, device="cuda")
+        auto = N.gemm_nt(aq, bq, O.E4M3, O.E4M3, *args, out=guarded[:M], **kw)
+        assert (guarded[M:] == 7.0).all()
+        N.gemm_set_variant(2)
+        assert torch.equal(auto, N.gemm_nt(aq, bq, O.E4M3, O.E4M3, *args, out_dtype=out_dtype, **kw))
+        N.gemm_set_variant(-1)
