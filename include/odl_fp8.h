@@ -385,7 +385,7 @@ int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, in
  * multiplying them by (scale product of pair s) / (scale product of pair s + 1) where it passes from one pair
  * to the next, and applies the last pair's scale product in its epilogue:
  *   C = round(((acc_0 r_0 + acc_1) r_1 + ... + acc_last) s_last), every step in fp32, ONE rounding to out_dtype.
- * That route is taken for 2 .. 4 pairs with N % 128 == 0, every K[s] % 256 == 0 and >= 512 and
+ * That route is taken for 2 .. 4 pairs with M % 128 == 0, N % 128 == 0, every K[s] % 256 == 0 and >= 512 and
  * every operand under 2 GiB.  Anything else (up to 64 pairs, K[s] % 16 == 0) runs as one odl_fp8_gemm_nt per
  * pair, the second and later ones with accumulate set: one rounding to out_dtype per pair.  The two routes
  * agree within those roundings and bit for bit where every partial sum and every scale ratio is exact

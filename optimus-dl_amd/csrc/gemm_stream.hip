@@ -745,7 +745,9 @@ bool gemm_stream_accepts(const GemmArgs &g) {
 }
 
 // Operand pairs: each a whole even number of K steps, four at least (the load pipeline is two steps deep and crosses
-// from one pair to the next in its last two), every operand addressed with 32-bit byte offsets.
+// from one pair to the next in its last two), every operand addressed with 32-bit byte offsets.  Rows in whole wave tiles:
+// the kernel could end anywhere, but its one rounding and the rounding per pair of the other route are results that lie
+// 3e-3 (2-norm, bf16, contractions 4096 + 1024 + 1024) apart, and which of them a size gets is part of the contract.
 bool gemm_stream_accepts_pairs(const GemmArgs &g, const GemmPairs &gp) {
     const double esz = g.out_dtype == ODL_F32 ? 4.0 : 2.0;
     if (gp.count < 1 || gp.count > 4 || g.accumulate || g.ta || g.tb || g.sa_vec || g.sb_vec || g.bias || g.mx_sa || g.mx_sb || g.splits > 1)
@@ -755,7 +757,7 @@ bool gemm_stream_accepts_pairs(const GemmArgs &g, const GemmPairs &gp) {
         if (!gp.a[s] || !gp.b[s] || !gp.sa[s] || !gp.sb[s] || k < 512 || k % 256 != 0) return false;
         if ((double)(g.M + 256) * k >= 2147483648.0 || (double)(g.N + 256) * k >= 2147483648.0) return false;
     }
-    return (g.out_dtype == ODL_BF16 || g.out_dtype == ODL_F32) && g.M > 0 && g.N > 0 && g.N % WN == 0 &&
+    return (g.out_dtype == ODL_BF16 || g.out_dtype == ODL_F32) && g.M > 0 && g.N > 0 && g.M % WM == 0 && g.N % WN == 0 &&
            (double)g.N * esz * (BM + 8) < 2147483648.0;
 }
 

@@ -806,7 +806,7 @@ def gemm_nt(a: torch.Tensor, b: torch.Tensor, fmt_a: int, fmt_b: int, sa_inv: to
 def gemm_nt_sum(a: "list[torch.Tensor]", b: "list[torch.Tensor]", fmt_a: int, fmt_b: int, sa_inv: "list[torch.Tensor]",
                 sb_inv: "list[torch.Tensor]", out_dtype: torch.dtype = torch.bfloat16, out: torch.Tensor | None = None) -> torch.Tensor:
     """out[M,N] = sum_s (a[s][M,K_s] . b[s][N,K_s]^T) * (sa_inv[s] * sb_inv[s]); uint8 FP8 codes, one scale per operand.
-    One launch where the shapes suit the streaming kernel (2 .. 4 pairs, N a multiple of 128, every K_s a multiple
+    One launch where the shapes suit the streaming kernel (2 .. 4 pairs, M and N multiples of 128, every K_s a multiple
     of 256 and at least 512), otherwise one GEMM per pair, the later ones adding into ``out``."""
     n = len(a)
     if n < 1 or len(b) != n or len(sa_inv) != n or len(sb_inv) != n:
@@ -1050,7 +1050,7 @@ def dgrad_sum_in_one_launch(tokens: int, n_in: int, n_outs: "list[int]") -> bool
     as ONE launch of :func:`gemm_nt_sum` (the streaming kernel carrying its accumulators from one pair to the next): the
     shapes that kernel takes, and an output of more 256 x 256 tiles than half the 256 compute units (smaller ones are better
     served by the per-pair GEMMs that add into dX: those pick 128 x 128 tiles or split the contraction)."""
-    if not 2 <= len(n_outs) <= 4 or n_in % 128 or any(k % 256 or k < 512 for k in n_outs):
+    if not 2 <= len(n_outs) <= 4 or tokens % 128 or n_in % 128 or any(k % 256 or k < 512 for k in n_outs):
         return False
     tiles = ((tokens + 255) // 256) * ((n_in + 255) // 256)
     return tiles > 128 and all((tokens + 256) * k < 2**31 and (n_in + 256) * k < 2**31 for k in n_outs)

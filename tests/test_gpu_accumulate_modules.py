@@ -236,6 +236,27 @@ def test_sibling_group_data_gradient_from_one_gemm(amp, kind, monkeypatch):
         assert (got[1].float() - want[1].float()).abs().max().item() <= 3 * 2.0 ** -8 * want[1].float().abs().max().item()
 
 
+@pytest.mark.parametrize("kind", ["tensorwise", "delayed"])
+def test_sibling_group_data_gradient_of_ragged_token_counts(amp, kind, monkeypatch):
+    """4016 tokens (no multiple of 128) x 2304 features: the members add into dx one by one, with the bits of
+    ``fuse_dgrad_gemm = False``; outputs and weight gradients are the bits of the separate Linears."""
+    from optimus_dl_amd import native as N
+
+    kw = {"amax_history_len": 4} if kind == "delayed" else {}
+    grouped, stepwise, plain = build_wide(), build_wide(), build_wide(False)
+    r1, r2, r3 = (amp.create_fp8_recipe(kind, "hybrid", **kw) for _ in range(3))
+    r2.fuse_dgrad_gemm = False
+    sums, real_sum = [], N.gemm_nt_sum
+    monkeypatch.setattr(N, "gemm_nt_sum", lambda *a, **k: (sums.append(len(a[0])), real_sum(*a, **k))[1])
+    x = seeded_bf16((4, 1004, 2304), 1.0, 940).cuda()
+    dys = [seeded_bf16((4, 1004, n), 1e-3 * (4.0 ** i), 941 + i).cuda() for i, n in enumerate((1024, 512, 512))]
+    got, mid, want = run(grouped, r1, x, dys), run(stepwise, r2, x, dys), run(plain, r3, x, dys)
+    assert sums == [] and grouped.wq._siblings.groups_run == 1
+    assert torch.equal(got[1], mid[1])
+    for a, b in zip(got[0] + got[2], want[0] + want[2]):
+        assert torch.equal(a, b)
+
+
 def test_one_gemm_data_gradient_replays_from_a_graph(amp):
     """The call that sums the members' products takes host arrays of device pointers and hands them to the kernel by value:
     captured in a graph it must replay on new data like everything else (three replays, eager work and synchronisations

@@ -694,6 +694,37 @@ def test_sum_of_products_shape_sweep_against_the_per_pair_route(N):
             assert max_rel_err(one, ref) <= 1e-4, (case, M, Nn, ks)
 
 
+@pytest.mark.parametrize("M", [1, 127, 400, 4016])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_sum_of_products_with_rows_that_fill_no_wave_tile(N, M, out_dtype):
+    """Row counts that are no multiple of 128 take a GEMM per pair, each rounding to the output type: the bits of the chain
+    of gemm_nt calls (the one-launch route lies 3e-3 away in bf16), for pairs of different lengths whose scale products lie
+    up to 2^10 apart; nothing behind the output is written.  Against 64 bits every rounding is off by at most 2^-9 (bf16,
+    of the running sum, which the sum of the parts' magnitudes bounds) and the products by 7 * 2^-14 of sum |a||b|."""
+    Nn, ks = 384, (1024, 512, 768)
+    a, b, sa, sb = [], [], [], []
+    for i, k in enumerate(ks):
+        for lst, inv, shape, fmt, std, seed in ((a, sa, (M, k), O.E5M2, 1e-3 * 4.0 ** i, 100), (b, sb, (Nn, k), O.E4M3, 0.02 * 8.0 ** i, 200)):
+            q, s_inv = quantised(shape, fmt, std, seed + i)
+            lst.append(q.cuda())
+            inv.append(s_inv.cuda())
+    room = torch.full((M + 128, Nn), 7.0, dtype=out_dtype, device="cuda")
+    got = N.gemm_nt_sum(a, b, O.E5M2, O.E4M3, sa, sb, out=room[:M])
+    assert (room[M:] == 7.0).all()
+    chain = N.gemm_nt(a[0], b[0], O.E5M2, O.E4M3, sa[0], sb[0], out_dtype=out_dtype)
+    for s in range(1, len(ks)):
+        N.gemm_nt(a[s], b[s], O.E5M2, O.E4M3, sa[s], sb[s], out=chain, accumulate=True)
+    assert torch.equal(got, chain)
+    exact, parts, magnitude = 0, 0, 0
+    for x, y, p, q in zip(a, b, sa, sb):
+        x64, y64 = x.view(torch.float8_e5m2).double(), y.view(torch.float8_e4m3fn).double()
+        product = (x64 @ y64.t()) * (p.double() * q.double())
+        exact, parts = exact + product, parts + product.abs()
+        magnitude = magnitude + (x64.abs() @ y64.abs().t()) * (p.double() * q.double())
+    bound = 7 * 2.0 ** -14 * magnitude + (len(ks) * 2.0 ** -8 * parts if out_dtype == torch.bfloat16 else 0)
+    assert bool(((got.double() - exact).abs() <= bound).all())
+
+
 # ------------------------------------------------------------------ streaming kernel, rows that fill no tile
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("epilogue", ["tensor", "rowwise", "bias"])

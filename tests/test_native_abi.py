@@ -144,6 +144,19 @@ def test_split_count_is_a_host_side_decision_with_the_documented_shape_rules():
         assert count(M, N, K) == 1                          # not multiples of 128, or too short to split
 
 
+def test_data_gradient_sums_run_in_one_launch_only_for_whole_wave_tiles():
+    """Whether the members' products are rounded once or one by one depends on the token count like this and no other way:
+    multiples of 128 with more than 128 output tiles go in one launch."""
+    from optimus_dl_amd import native
+
+    qkv = [4096, 1024, 1024]
+    assert native.dgrad_sum_in_one_launch(4096, 4096, qkv) and native.dgrad_sum_in_one_launch(4224, 4096, qkv)
+    for tokens in (4016, 4112, 4095, 8176):
+        assert not native.dgrad_sum_in_one_launch(tokens, 4096, qkv)
+    assert not native.dgrad_sum_in_one_launch(2048, 4096, qkv)                  # 128 tiles
+    assert not native.dgrad_sum_in_one_launch(4096, 4096, [4096]) and not native.dgrad_sum_in_one_launch(4096, 4096, [4096, 640])
+
+
 def test_block_scaled_entry_points_refuse_bad_arguments_before_touching_a_device():
     """Argument and shape checks of the MXFP8 / blockwise entry points are host code that runs before any HIP call: they
     answer with an error code and a message here, where no GPU exists."""
