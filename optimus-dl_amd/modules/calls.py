@@ -35,6 +35,12 @@ class _NoGraph:
     def save_for_backward(self, *tensors: torch.Tensor) -> None:
         pass
 
+    # what else a forward may tell its context is about the node
+    mark_dirty = mark_non_differentiable = save_for_forward = save_for_backward
+
+    def set_materialize_grads(self, value: bool) -> None:
+        pass
+
 
 def apply(function: "type[torch.autograd.Function]", *args):
     """``function.apply(*args)``; only its forward where no graph is recorded.

@@ -90,6 +90,19 @@ def test_sibling_group_equals_separate_linears(amp, kind, bias):
     assert grouped.wq.fp8_calls == 3 and grouped.wk.fp8_calls == 3
 
 
+@pytest.mark.parametrize("kind", ["tensorwise", "delayed", "rowwise"])
+@pytest.mark.parametrize("mode", [torch.no_grad, torch.inference_mode])
+def test_group_without_a_graph_gives_the_members_outputs(amp, kind, mode):
+    from optimus_dl_amd.modules.fp8_linear import linear_group
+
+    net, recipe = build(bias=True), amp.create_fp8_recipe(kind, "hybrid")
+    x = seeded_bf16((2, 96, 512), 1.0, 760).cuda()
+    with mode(), recipe.autocast():
+        together = linear_group(x, (net.wq, net.wk, net.wv))
+        apart = net(x)
+    assert len(together) == 3 and all(torch.equal(a, b) and not a.requires_grad for a, b in zip(together, apart))
+
+
 def test_sibling_group_launches_no_separate_adds(amp, monkeypatch):
     """Two of the three dgrad GEMMs run with the accumulate flag, and an unused output costs nothing in the backward."""
     from optimus_dl_amd import native as N

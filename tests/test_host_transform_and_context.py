@@ -452,6 +452,34 @@ def test_functions_without_a_graph_run_their_forward_only():
         torch.vmap(lambda a: apply(Double, a, w))(torch.randn(2, 3))
 
 
+def test_a_forward_without_a_graph_may_use_every_method_of_its_context():
+    """And the group of sibling Linears, whose forward does, runs without a graph like with one."""
+    from optimus_dl_amd.modules import fp8_linear
+    from optimus_dl_amd.modules.calls import apply
+
+    class Busy(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            ctx.set_materialize_grads(False)
+            y, order = x.sort()
+            ctx.mark_non_differentiable(order)
+            ctx.mark_dirty()
+            ctx.save_for_forward(x)
+            ctx.save_for_backward(order)
+            return y, order
+
+        @staticmethod
+        def backward(ctx, dy, _):
+            return dy
+
+    x = torch.randn(5, requires_grad=True)
+    with torch.no_grad():
+        got = apply(Busy, x)
+        want = Busy.apply(x)
+        assert fp8_linear.apply(fp8_linear._Fp8LinearGroupFn, x, None, torch.bfloat16, ()) == ()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 def test_untraced_functions_stay_out_of_compiled_graphs():
     from optimus_dl_amd.modules.calls import untraced
 
