@@ -18,10 +18,10 @@ def untraced(fn):
     disabled = torch.compiler.disable(fn)
 
     @functools.wraps(fn)
-    def call(*args):
+    def call(*args, **kwargs):
         if torch.compiler.is_compiling() or _compiler_callback() is not None:
-            return disabled(*args)
-        return fn(*args)
+            return disabled(*args, **kwargs)
+        return fn(*args, **kwargs)
 
     return call
 

@@ -480,6 +480,18 @@ def test_a_forward_without_a_graph_may_use_every_method_of_its_context():
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+def test_untraced_functions_take_keyword_arguments():
+    """Off the GPU each of them falls back: to the plain expression, or to None."""
+    from optimus_dl_amd.modules import fp8_linear, fused
+
+    x, w = torch.randn(4, 8), torch.ones(8)
+    assert torch.equal(fused.swiglu(gate=x, up=x), torch.nn.functional.silu(x) * x)
+    assert fused.rmsnorm(x, weight=w, eps=1e-5) is None and fused.layernorm(x, w, bias=None, eps=1e-5) is None
+    assert fused.gelu(x=x) is None and fp8_linear.linear_group(x, modules=()) is None
+    compiled = torch.compile(lambda t: fused.swiglu(t, up=t) * 2, backend="eager")
+    assert torch.equal(compiled(x), fused.swiglu(x, x) * 2)
+
+
 def test_untraced_functions_stay_out_of_compiled_graphs():
     from optimus_dl_amd.modules.calls import untraced
 
