@@ -10,7 +10,18 @@ import functools
 
 import torch
 import torch.autograd.forward_ad as _forward_ad
-from torch._C._dynamo.eval_frame import get_eval_frame_callback as _compiler_callback
+
+# Whether a graph compiler, a functorch transform, forward-mode differentiation or a tracer is at work is known to private
+# parts of torch only.  Where a version of torch lacks one of them, every call takes the long way.
+try:
+    from torch._C._dynamo.eval_frame import get_eval_frame_callback as _compiler_callback
+except ImportError:
+    def _compiler_callback():
+        return False
+
+_functorch_stack = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", None)
+_tracing_state = getattr(torch._C, "_get_tracing_state", None)
+_graph_state_known = _functorch_stack is not None and _tracing_state is not None and hasattr(_forward_ad, "_current_level")
 
 
 def untraced(fn):
@@ -48,7 +59,7 @@ def apply(function: "type[torch.autograd.Function]", *args):
     ``Function.apply`` reports parameters that require gradients as needing one also under ``torch.no_grad()``: a forward
     that prepares operands of the backward (transposed codes) would make them for nobody.  Whatever else looks at an
     autograd function still finds it: functorch transforms, forward-mode differentiation and the tracer of torch.jit."""
-    if (torch.is_grad_enabled() or _forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch._C._get_tracing_state() is not None):
+    if (not _graph_state_known or torch.is_grad_enabled() or _forward_ad._current_level >= 0 or _functorch_stack() is not None
+            or _tracing_state() is not None):
         return function.apply(*args)
     return function.forward(_NoGraph(len(args)), *args)

@@ -492,6 +492,40 @@ def test_untraced_functions_take_keyword_arguments():
     assert torch.equal(compiled(x), fused.swiglu(x, x) * 2)
 
 
+@pytest.mark.parametrize("missing", ["compiler callback", "functorch stack", "tracing state", "forward level"])
+def test_calls_take_the_long_way_where_torch_does_not_tell(monkeypatch, missing):
+    import importlib.util
+    import sys
+
+    from optimus_dl_amd.modules import calls
+
+    if missing == "compiler callback":
+        monkeypatch.setitem(sys.modules, "torch._C._dynamo.eval_frame", None)
+    elif missing == "functorch stack":
+        monkeypatch.delattr(torch._C._functorch, "peek_interpreter_stack")
+    elif missing == "tracing state":
+        monkeypatch.delattr(torch._C, "_get_tracing_state")
+    else:
+        monkeypatch.delattr(torch.autograd.forward_ad, "_current_level")
+    spec = importlib.util.spec_from_file_location("calls_without", calls.__file__)
+    without = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(without)
+    monkeypatch.undo()
+    x = torch.randn(3)
+    assert torch.equal(without.untraced(lambda t, *, by: t * by)(x, by=2), x * 2)
+    seen = []
+
+    class Note(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, t):
+            seen.append(type(ctx).__name__)
+            return t.clone()
+
+    with torch.no_grad():
+        assert torch.equal(without.apply(Note, x), x)
+    assert (seen == ["_NoGraph"]) == (missing == "compiler callback")
+
+
 def test_untraced_functions_stay_out_of_compiled_graphs():
     from optimus_dl_amd.modules.calls import untraced
 
