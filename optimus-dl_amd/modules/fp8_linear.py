@@ -232,11 +232,16 @@ class _Fp8LinearFn(torch.autograd.Function):
         bias_f32 = None if bias is None else bias.detach().float()
         saved: dict[str, Any] = {}
         ctx.wgrad_direct = False
+        # Both layouts of a weight whose codes are kept are made for a forward without a graph too if its input needs a
+        # gradient: reentrant activation checkpointing runs such a forward first, and its second one finds them (4096 x 14336
+        # MLP, 1024 tokens, per step: 1207 us with the weights quantised twice, 1108 with both layouts at once).  Not in training
+        # under delayed scaling, whose forwards with a graph record the maxima and make codes of their own.
+        both_w = need_dgrad or (recipe.cache_weights and x2d.requires_grad and not (pol.kind == "delayed" and module.training))
 
         if pol.kind in ("mxfp8", "blockwise"):
             fp8_wgrad = need_wgrad and recipe.wgrad
             xq, xs, xq_t, xs_t = _mx_input_shared(recipe, x2d, pol.fmt_fwd, fp8_wgrad)
-            wq, ws, wq_t, ws_t = module._mx_weight(weight, recipe, need_t=need_dgrad)
+            wq, ws, wq_t, ws_t = module._mx_weight(weight, recipe, need_t=both_w)
             y = native.mx_gemm_nt(xq, xs, wq, ws, pol.fmt_fwd, pol.fmt_fwd, bias=bias_f32, out_dtype=out_dtype)
             if fp8_wgrad:
                 saved["xq_t"], saved["xs_t"] = xq_t, xs_t
@@ -251,7 +256,7 @@ class _Fp8LinearFn(torch.autograd.Function):
                 saved["xq_t"], saved["sx_inv_t"] = xq_t, sx_inv_t
             if not recipe.cache_weights:
                 module._wcache_rowwise.clear()          # the backward of this call still finds what is made now
-            wq, sw_inv = module._rowwise_weight(weight, pol, "row", both=need_dgrad)
+            wq, sw_inv = module._rowwise_weight(weight, pol, "row", both=both_w)
             y = native.gemm_nt(_rows(xq, x2d.shape[0]), wq, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sw_inv, bias=bias_f32, out_dtype=out_dtype)
         else:
             # With whole 256 x 256 tiles wgrad reads the ROW-MAJOR codes of dy with the tokens as the slow
@@ -277,7 +282,7 @@ class _Fp8LinearFn(torch.autograd.Function):
                                                      record=record, margin=pol.margin, rows_out=tokens if fp8_wgrad else None)
             else:
                 xq, xq_t, sx_inv = _quantise_input_shared(recipe, x2d, pol.fmt_fwd, pol.margin, fp8_wgrad)
-            wq, wq_t, sw_inv = module._tensor_weight(weight, recipe, need_t=need_dgrad)
+            wq, wq_t, sw_inv = module._tensor_weight(weight, recipe, need_t=both_w)
             y = native.gemm_nt(_rows(xq, x2d.shape[0]), wq, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sw_inv, bias=bias_f32, out_dtype=out_dtype)
             if fp8_wgrad:
                 saved["xq_t"], saved["sx_inv_t"] = xq_t, sx_inv

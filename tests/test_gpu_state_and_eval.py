@@ -283,3 +283,45 @@ def test_first_use_under_stream_capture_is_refused_until_the_device_is_set_up(mo
     N.cast_dynamic_noalloc(x, N.E4M3, 0, out, None, dyn)
     want, _, _, _, _ = N.quantize_dynamic(x, N.E4M3, 0, want_transposed=False)
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("kind", ["tensorwise", "rowwise", "mxfp8", "blockwise"])
+def test_reentrant_checkpointing_quantises_a_weight_once_per_step(amp, kind, monkeypatch):
+    """The first of the two forwards has no graph, the second has one: kept weight codes serve both (and the backward), and
+    the gradients are those without checkpointing."""
+    from torch.utils.checkpoint import checkpoint
+
+    from optimus_dl_amd import native as N
+    from optimus_dl_amd.modules import fp8_linear as L
+
+    w, x, dy = seeded_bf16((384, 256), 0.02, 801), seeded_bf16((128, 256), 1.0, 800), seeded_bf16((128, 384), 1e-3, 802)
+    lin, plain = make_linear(w), make_linear(w)
+    made = []
+
+    def spy(owner, name, at):
+        real = getattr(owner, name)
+
+        def call(*args, **kw):
+            if args[at].data_ptr() == lin.weight.data_ptr():
+                made.append(name)
+            return real(*args, **kw)
+
+        monkeypatch.setattr(owner, name, call)
+
+    for owner, name, at in ((L, "_quantise_dynamic", 0), (L, "_quantise_axis", 0), (L, "_block_cast", 1), (N, "quantize_rowcol", 0)):
+        spy(owner, name, at)
+    recipe = amp.create_fp8_recipe(kind, "hybrid")
+    for _ in range(2):
+        xd, lin.weight.grad = x.cuda().requires_grad_(True), None
+        with recipe.autocast():
+            y = checkpoint(lin, xd, use_reentrant=True)
+        with recipe.backward():
+            y.backward(dy.cuda())
+        want = train_step(plain, amp.create_fp8_recipe(kind, "hybrid"), x, dy)
+        for a, b in zip((y.detach(), xd.grad, lin.weight.grad), want):
+            assert torch.equal(a, b)
+        assert len(made) == 1, made
+        made.clear()
+        with torch.no_grad():
+            for m in (lin, plain):
+                m.weight.mul_(1.25)
