@@ -646,7 +646,7 @@ __global__ __launch_bounds__(kThreads) void cast_generic_kernel(const void *__re
             else f = reinterpret_cast<const float *>(x)[i];
         }
         am = max(am, float_to_bits(f) & 0x7fffffffu);
-        const float s = mode == ODL_SCALE_TENSOR ? scale[0] : (mode == ODL_SCALE_ROW ? scale[min(r, rows - 1)] : scale[c]);
+        const float s = mode == ODL_SCALE_TENSOR ? scale[0] : (mode == ODL_SCALE_ROW ? (r < rows ? scale[r] : 1.0f) : scale[c]);
         const uint8_t q = (uint8_t)(quantise4<FMT>(f, 0.f, 0.f, 0.f, s, 1.f, 1.f, 1.f) & 0xffu);
         if (out) out[i] = q;
         if (out_t) out_t[c * rows_out + r] = q;
@@ -1158,7 +1158,7 @@ extern "C" int odl_fp8_cast_delayed_padded(const void *x, int src_dtype, int64_t
     if (int e = check_cast_args("odl_fp8_cast_delayed", x, src_dtype, rows, cols, scale, ODL_SCALE_TENSOR, fmt)) return e;
     if (rows_out < rows) return set_error(ODL_ERR_ARG, "odl_fp8_cast_delayed: rows_out %lld < rows %lld", (long long)rows_out, (long long)rows);
     if (!scale) return set_error(ODL_ERR_ARG, "odl_fp8_cast_delayed: scale is null");
-    if (rows * cols == 0) {                       // nothing to cast and nothing to record: only the inverse scale
+    if (rows_out * cols == 0) {                   // nothing to cast and nothing to record: only the inverse scale
         if (scale_inv_out) hipLaunchKernelGGL(scale_inv_kernel, dim3(1), dim3(1), 0, stream, scale, scale_inv_out);
         return check_launch("odl_fp8_cast_delayed");
     }
@@ -1220,7 +1220,7 @@ extern "C" int odl_fp8_cast_dynamic_padded(const void *x, int src_dtype, int64_t
     if (int e = check_cast_args("odl_fp8_cast_dynamic", x, src_dtype, rows, cols, parts, ODL_SCALE_TENSOR, fmt)) return e;
     if (rows_out < rows) return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic: rows_out %lld < rows %lld", (long long)rows_out, (long long)rows);
     if (!parts || !dyn_out) return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic: null pointer");
-    if (rows * cols == 0) {                       // nothing to cast: only the three numbers
+    if (rows_out * cols == 0) {                   // nothing to cast: only the three numbers
         if (fmt == ODL_FP8_E4M3) hipLaunchKernelGGL((parts_to_scale_kernel<ODL_FP8_E4M3>), dim3(1), dim3(kThreads), 0, stream, parts, margin, dyn_out);
         else hipLaunchKernelGGL((parts_to_scale_kernel<ODL_FP8_E5M2>), dim3(1), dim3(kThreads), 0, stream, parts, margin, dyn_out);
         return check_launch("odl_fp8_cast_dynamic(empty)");
@@ -1480,14 +1480,14 @@ extern "C" int odl_fp8_cast_rowcol_padded(const void *x, int src_dtype, int64_t 
     if (fmt != ODL_FP8_E4M3 && fmt != ODL_FP8_E5M2) return set_error(ODL_ERR_ARG, "odl_fp8_cast_rowcol: fmt %d", fmt);
     if ((rows > 0 && (!amax_row || !s_row || !s_row_inv)) || (cols > 0 && (!amax_col || !s_col || !s_col_inv)))
         return set_error(ODL_ERR_ARG, "odl_fp8_cast_rowcol: null scale pointer");
-    if (rows * cols > 0 && (!x || !out || !out_t)) return set_error(ODL_ERR_ARG, "odl_fp8_cast_rowcol: null pointer");
+    if ((rows * cols > 0 && !x) || (rows_out * cols > 0 && (!out || !out_t))) return set_error(ODL_ERR_ARG, "odl_fp8_cast_rowcol: null pointer");
     const int64_t tiles = ((rows_out + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
     const bool fast = rowcol_fast(x, rows_out, cols) && rows > 0 && aligned16(out_t) && (reinterpret_cast<uintptr_t>(out) & 7) == 0 && tiles <= 0x7fffffffLL;
     if (!fast) {
         // the step-by-step route: scales first, then the two casts
         int rc = odl_fp8_scale_from_amax(amax_row, rows, fmt, margin, s_row, s_row_inv, stream_);
         if (rc == ODL_OK) rc = odl_fp8_scale_from_amax(amax_col, cols, fmt, margin, s_col, s_col_inv, stream_);
-        if (rc != ODL_OK || rows * cols == 0) return rc;
+        if (rc != ODL_OK || rows_out * cols == 0) return rc;
         if (rows_out != rows) {
             ODL_DISPATCH_SRC_FMT(launch_generic, x, rows, cols, rows_out, s_row, ODL_SCALE_ROW, out, (uint8_t *)nullptr, (float *)nullptr, stream);
             ODL_DISPATCH_SRC_FMT(launch_generic, x, rows, cols, rows_out, s_col, ODL_SCALE_COL, (uint8_t *)nullptr, out_t, (float *)nullptr, stream);

@@ -464,3 +464,33 @@ def test_padded_casts_are_the_plain_ones_with_zero_codes_behind(N, rows, cols, r
     ref, got = N.quantize_rowcol(x, O.E4M3), N.quantize_rowcol(x, O.E4M3, rows_out=rows_out)
     check(got[0], got[2], ref[0], ref[2])
     assert torch.equal(got[1], ref[1]) and torch.equal(got[3], ref[3])
+
+
+@pytest.mark.parametrize("cols", [64, 13])
+def test_padded_casts_of_no_rows_write_zero_codes(N, cols):
+    """A tensor without rows: every code belongs to no row, so all of them are zero, on both routes."""
+    for dtype in (torch.bfloat16, torch.float32):
+        x, scale = torch.empty((0, cols), dtype=dtype, device="cuda"), torch.full((1,), 3.0, device="cuda")
+        for want, want_t in ((True, True), (True, False), (False, True)):
+            # the allocator hands out what was just freed: codes that nothing writes are not zero
+            for _ in range(4):
+                torch.full((128 * cols,), 9, dtype=torch.uint8, device="cuda")
+            got = N.cast_dynamic(x, N.amax_parts(x), O.E4M3, 0, want, want_t, rows_out=128)
+            later = N.cast_delayed(x, scale, O.E5M2, torch.zeros(N.AMAX_PARTS, device="cuda"), want, want_t, rows_out=128)
+            for codes, shape in ((got[0], (128, cols)), (got[1], (cols, 128)), (later[0], (128, cols)), (later[1], (cols, 128))):
+                assert codes is None or (codes.shape == shape and not codes.any())
+            assert got[2].item() == 0.0 and got[3].item() == 1.0 and later[2].item() == 1.0 / torch.tensor(3.0)
+        out_t = torch.full((cols, 128), 9, dtype=torch.uint8, device="cuda")
+        N.cast_dynamic(x, N.amax_parts(x), O.E4M3, 0, False, out_t=out_t, rows_out=128)
+        assert not out_t.any()
+        out_t.fill_(9)
+        N.cast_delayed(x, scale, O.E4M3, None, False, out_t=out_t, rows_out=128)
+        assert not out_t.any()
+        L = N.load()
+        amax_col, one = torch.zeros(cols, device="cuda"), torch.zeros(1, device="cuda")
+        s_col, s_col_inv = torch.empty_like(amax_col), torch.empty_like(amax_col)
+        out, out_t = (torch.full(s, 9, dtype=torch.uint8, device="cuda") for s in ((128, cols), (cols, 128)))
+        assert L.odl_fp8_cast_rowcol_padded(None, N._src_dtype(x), 0, cols, 128, one.data_ptr(), amax_col.data_ptr(), O.E4M3, 0,
+                                            out.data_ptr(), out_t.data_ptr(), one.data_ptr(), one.data_ptr(), s_col.data_ptr(),
+                                            s_col_inv.data_ptr(), N._stream()) == 0
+        assert not out.any() and not out_t.any() and (s_col == 1).all() and (s_col_inv == 1).all()
