@@ -114,7 +114,7 @@ int odl_fp8_cast_dynamic(const void *x, int src_dtype, int64_t rows, int64_t col
                          odl_stream_t stream);
 
 /*
- * The casts of odl_fp8_cast_dynamic, odl_fp8_cast_delayed and odl_fp8_cast_rowcol with room behind the rows of x:
+ * The casts of odl_fp8_cast_dynamic, odl_fp8_cast_delayed, odl_fp8_cast_rowcol and odl_fp8_cast_transpose with room behind the rows of x:
  * out is [rows_out, cols] and out_t [cols, rows_out], rows_out >= rows (a multiple of 16 for the fast kernels), and
  * codes that belong to no row of x are zero.  A weight gradient contracts over the tokens: with rows_out the next
  * multiple of 128 it runs on whole K steps of the GEMM kernels whatever the number of tokens, and the zeros add
@@ -130,6 +130,9 @@ int odl_fp8_cast_rowcol_padded(const void *x, int src_dtype, int64_t rows, int64
                                const float *amax_row, const float *amax_col, int fmt, int margin, uint8_t *out,
                                uint8_t *out_t, float *s_row, float *s_row_inv, float *s_col, float *s_col_inv,
                                odl_stream_t stream);
+int odl_fp8_cast_transpose_padded(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out,
+                                  const float *scale, int mode, int fmt, uint8_t *out, uint8_t *out_t,
+                                  float *amax_out, odl_stream_t stream);
 
 /*
  * MANY tensors per launch: every weight of a model after an optimizer step (what te.pytorch.Linear does per

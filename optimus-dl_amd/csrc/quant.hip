@@ -1070,11 +1070,11 @@ static void launch_ct(const void *x, int64_t rows, int64_t cols, int64_t rows_ou
 }
 
 template <int SRC, int FMT>
-static void launch_ct_mode(int mode, const void *x, int64_t rows, int64_t cols, const float *scale, uint8_t *out,
+static void launch_ct_mode(int mode, const void *x, int64_t rows, int64_t cols, int64_t rows_out, const float *scale, uint8_t *out,
                            uint8_t *out_t, float *amax_out, hipStream_t stream) {
-    if (mode == ODL_SCALE_TENSOR) launch_ct<SRC, FMT, ODL_SCALE_TENSOR>(x, rows, cols, rows, scale, out, out_t, amax_out, stream);
-    else if (mode == ODL_SCALE_ROW) launch_ct<SRC, FMT, ODL_SCALE_ROW>(x, rows, cols, rows, scale, out, out_t, amax_out, stream);
-    else launch_ct<SRC, FMT, ODL_SCALE_COL>(x, rows, cols, rows, scale, out, out_t, amax_out, stream);
+    if (mode == ODL_SCALE_TENSOR) launch_ct<SRC, FMT, ODL_SCALE_TENSOR>(x, rows, cols, rows_out, scale, out, out_t, amax_out, stream);
+    else if (mode == ODL_SCALE_ROW) launch_ct<SRC, FMT, ODL_SCALE_ROW>(x, rows, cols, rows_out, scale, out, out_t, amax_out, stream);
+    else launch_ct<SRC, FMT, ODL_SCALE_COL>(x, rows, cols, rows_out, scale, out, out_t, amax_out, stream);
 }
 
 static int check_cast_args(const char *who, const void *x, int src_dtype, int64_t rows, int64_t cols, const float *scale,
@@ -1114,16 +1114,23 @@ extern "C" int odl_fp8_cast(const void *x, int src_dtype, int64_t rows, int64_t 
 
 extern "C" int odl_fp8_cast_transpose(const void *x, int src_dtype, int64_t rows, int64_t cols, const float *scale, int mode,
                                       int fmt, uint8_t *out, uint8_t *out_t, float *amax_out, odl_stream_t stream_) {
+    return odl_fp8_cast_transpose_padded(x, src_dtype, rows, cols, rows, scale, mode, fmt, out, out_t, amax_out, stream_);
+}
+
+extern "C" int odl_fp8_cast_transpose_padded(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, const float *scale,
+                                             int mode, int fmt, uint8_t *out, uint8_t *out_t, float *amax_out, odl_stream_t stream_) {
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
     if (int e = check_cast_args("odl_fp8_cast_transpose", x, src_dtype, rows, cols, scale, mode, fmt)) return e;
-    if (rows * cols == 0) return ODL_OK;
+    if (rows_out < rows) return set_error(ODL_ERR_ARG, "odl_fp8_cast_transpose: rows_out %lld < rows %lld", (long long)rows_out, (long long)rows);
+    if (rows_out * cols == 0) return ODL_OK;
+    if (!scale && mode != ODL_SCALE_ROW) return set_error(ODL_ERR_ARG, "odl_fp8_cast_transpose: scale is null");
     if (!out_t) return set_error(ODL_ERR_ARG, "odl_fp8_cast_transpose: out_t is null");
-    const int64_t tiles = ((rows + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
-    const bool fast = cols % 8 == 0 && rows % 16 == 0 && aligned16(x) && aligned16(out_t) &&
+    const int64_t tiles = ((rows_out + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
+    const bool fast = cols % 8 == 0 && rows_out % 16 == 0 && aligned16(x) && aligned16(out_t) &&
                       (!out || (reinterpret_cast<uintptr_t>(out) & 7) == 0) &&
                       (mode != ODL_SCALE_COL || aligned16(scale)) && tiles <= 0x7fffffffLL;
-    if (fast) ODL_DISPATCH_SRC_FMT(launch_ct_mode, mode, x, rows, cols, scale, out, out_t, amax_out, stream);
-    else ODL_DISPATCH_SRC_FMT(launch_generic, x, rows, cols, rows, scale, mode, out, out_t, amax_out, stream);
+    if (fast) ODL_DISPATCH_SRC_FMT(launch_ct_mode, mode, x, rows, cols, rows_out, scale, out, out_t, amax_out, stream);
+    else ODL_DISPATCH_SRC_FMT(launch_generic, x, rows, cols, rows_out, scale, mode, out, out_t, amax_out, stream);
     return check_launch("odl_fp8_cast_transpose");
 }
 

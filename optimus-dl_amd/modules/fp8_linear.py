@@ -211,13 +211,14 @@ def _rows(codes: torch.Tensor, n: int) -> torch.Tensor:
     return codes if codes.shape[0] == n else codes[:n]
 
 
-def _quantise_axis(x2d: torch.Tensor, fmt: int, margin: int, mode: int, transposed: bool):
+def _quantise_axis(x2d: torch.Tensor, fmt: int, margin: int, mode: int, transposed: bool, rows_out: int | None = None):
     """Rowwise recipe: one scale per row (mode R) or per column (mode C) of x2d.
-    Returns the codes (transposed when asked) and the inverse scale vector."""
+    Returns the codes (transposed when asked, then with room behind the rows: ``native.padded_rows``) and the inverse
+    scale vector."""
     amax = native.amax(x2d, mode)
     scale, scale_inv = native.scale_from_amax(amax, fmt, margin)
     if transposed:
-        _, q = native.cast_transpose(x2d, scale, fmt, mode, want_rowmajor=False)
+        _, q = native.cast_transpose(x2d, scale, fmt, mode, want_rowmajor=False, rows_out=rows_out)
     else:
         q = native.cast(x2d, scale, fmt, mode)
     return q, scale_inv
@@ -332,7 +333,8 @@ class _Fp8LinearFn(torch.autograd.Function):
             elif ctx.need_dgrad:
                 gq, sg_inv = _quantise_axis(dy2d, pol.fmt_bwd, pol.margin, R, False)
             elif fp8_wgrad:
-                _, _, gq_t, sg_inv_t, _, _ = native.quantize_rowcol(dy2d, pol.fmt_bwd, pol.margin, rows_out=rows_out)
+                # no data gradient: only the columns are needed (4096 -> 14336, 8192 tokens: 870 us a step, with both axes 919)
+                gq_t, sg_inv_t = _quantise_axis(dy2d, pol.fmt_bwd, pol.margin, C, True, rows_out=rows_out)
             if ctx.need_dgrad:
                 wq_t, sw_inv_t = module._rowwise_weight(saved["weight"], pol, "col")
                 dx_into = getattr(ctx, "dx_into", None)      # a later member of a sibling group adds into the group's dx

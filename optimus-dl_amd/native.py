@@ -24,7 +24,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 17
+ABI_VERSION = 18
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -44,6 +44,7 @@ EXPORTS = (
     "odl_fp8_cast_dynamic_padded",
     "odl_fp8_cast_delayed_padded",
     "odl_fp8_cast_rowcol_padded",
+    "odl_fp8_cast_transpose_padded",
     "odl_fp8_multi_plan",
     "odl_fp8_multi_amax_parts",
     "odl_fp8_multi_cast_dynamic",
@@ -117,6 +118,7 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_cast_dynamic_padded.argtypes = [vp, i32, i64, i64, i64, vp, i32, i32, vp, vp, vp, vp]
         L.odl_fp8_cast_delayed_padded.argtypes = [vp, i32, i64, i64, i64, vp, i32, vp, vp, vp, vp, vp]
         L.odl_fp8_cast_rowcol_padded.argtypes = [vp, i32, i64, i64, i64, vp, vp, i32, i32, vp, vp, vp, vp, vp, vp, vp]
+        L.odl_fp8_cast_transpose_padded.argtypes = [vp, i32, i64, i64, i64, vp, i32, i32, vp, vp, vp, vp]
         L.odl_fp8_cast_dynamic_noalloc.argtypes = [vp, i32, i64, i64, i32, i32, vp, vp, vp, vp]
         L.odl_fp8_multi_plan.argtypes = [vp, i64, i32, vp, i64]
         L.odl_fp8_multi_plan.restype = ctypes.c_int64
@@ -717,18 +719,19 @@ def cast(x: torch.Tensor, scale: torch.Tensor, fmt: int, mode: int = SCALE_TENSO
 
 
 def cast_transpose(x: torch.Tensor, scale: torch.Tensor, fmt: int, mode: int = SCALE_TENSOR,
-                   amax_out: torch.Tensor | None = None, want_rowmajor: bool = True):
-    """Returns (codes[rows, cols] or None, codes_t[cols, rows])."""
+                   amax_out: torch.Tensor | None = None, want_rowmajor: bool = True, rows_out: int | None = None):
+    """Returns (codes[rows, cols] or None, codes_t[cols, rows]).  rows_out: as in :func:`cast_dynamic`."""
     x = _as_2d(x)
     rows, cols = x.shape
     _f32_dev(scale, _n_scales(mode, rows, cols), "cast_transpose scale")
-    out = torch.empty((rows, cols), dtype=torch.uint8, device=x.device) if want_rowmajor else None
-    out_t = torch.empty((cols, rows), dtype=torch.uint8, device=x.device)
+    n = rows if rows_out is None else rows_out
+    out = torch.empty((n, cols), dtype=torch.uint8, device=x.device) if want_rowmajor else None
+    out_t = torch.empty((cols, n), dtype=torch.uint8, device=x.device)
     if amax_out is not None:
         _f32_dev(amax_out, 1, "cast_transpose amax_out")
-    _check(load().odl_fp8_cast_transpose(x.data_ptr(), _src_dtype(x), rows, cols, scale.data_ptr(), mode, fmt,
-                                         out.data_ptr() if out is not None else None, out_t.data_ptr(),
-                                         amax_out.data_ptr() if amax_out is not None else None, _stream()),
+    _check(load().odl_fp8_cast_transpose_padded(x.data_ptr(), _src_dtype(x), rows, cols, n, scale.data_ptr(), mode, fmt,
+                                                out.data_ptr() if out is not None else None, out_t.data_ptr(),
+                                                amax_out.data_ptr() if amax_out is not None else None, _stream()),
            "odl_fp8_cast_transpose")
     return out, out_t
 

@@ -683,3 +683,29 @@ def test_seeded_random_linears_match_the_oracle(amp, seed):
         want_db = dy.float().sum(0)
         err = (lin.bias.grad.float().cpu() - want_db).abs().max().item() / max(want_db.abs().max().item(), 1e-30)
         assert err <= (1e-2 if lin.bias.dtype == torch.bfloat16 else 1e-5), f"{what}: db {err}"
+
+
+@pytest.mark.parametrize("tokens", [128, 144, 1008])
+def test_rowwise_backward_without_a_data_gradient_casts_one_axis(tokens, monkeypatch):
+    """An input that needs no gradient: dy is scaled per column only, and dW has the bits of the pass that needs both."""
+    from optimus_dl_amd import native as N
+    from optimus_dl_amd.modules.amp import create_fp8_recipe
+    from optimus_dl_amd.modules.fp8_linear import FP8Linear
+
+    torch.manual_seed(0)
+    lin = FP8Linear(256, 384, bias=False, device="cuda", dtype=torch.bfloat16)
+    x, dy = seeded_bf16((tokens, 256), 1.0, 850).cuda(), seeded_bf16((tokens, 384), 1e-3, 851).cuda()
+    both_axes, real = [], N.quantize_rowcol
+    monkeypatch.setattr(N, "quantize_rowcol", lambda t, *a, **k: (both_axes.append(tuple(t.shape)), real(t, *a, **k))[1])
+    grads = []
+    for needs in (True, False):
+        recipe = create_fp8_recipe("rowwise", "hybrid")
+        lin.weight.grad = None
+        both_axes.clear()
+        with recipe.autocast():
+            y = lin(x.clone().requires_grad_(needs))
+        with recipe.backward():
+            y.backward(dy)
+        grads.append(lin.weight.grad)
+        assert ((tokens, 384) in both_axes) == needs
+    assert torch.equal(grads[0], grads[1])

@@ -494,3 +494,27 @@ def test_padded_casts_of_no_rows_write_zero_codes(N, cols):
                                             out.data_ptr(), out_t.data_ptr(), one.data_ptr(), one.data_ptr(), s_col.data_ptr(),
                                             s_col_inv.data_ptr(), N._stream()) == 0
         assert not out.any() and not out_t.any() and (s_col == 1).all() and (s_col_inv == 1).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols,rows_out", [(16, 8, 128), (112, 72, 128), (144, 136, 256), (1008, 80, 1024), (7, 13, 16), (130, 24, 256), (0, 8, 16)])
+@pytest.mark.parametrize("mode", [O.SCALE_TENSOR, O.SCALE_ROW, O.SCALE_COL])
+def test_padded_cast_transpose_is_the_plain_one_with_zero_codes_behind(N, rows, cols, rows_out, dtype, mode):
+    """Every scale mode, both routes (13 columns: element at a time), with and without the row-major codes and the maximum."""
+    x = seeded_bf16((rows, cols), seed=rows + cols).to(dtype).cuda()
+    n = {O.SCALE_TENSOR: 1, O.SCALE_ROW: rows, O.SCALE_COL: cols}[mode]
+    scale = (torch.rand(n, generator=torch.Generator().manual_seed(cols)) + 0.5).cuda()
+    for want in (True, False):
+        amax = [torch.zeros(1, device="cuda") if want else None for _ in range(2)]
+        ref, ref_t = N.cast_transpose(x, scale, O.E5M2, mode, amax[0], want)
+        for _ in range(4):                                         # what nothing writes is not zero
+            torch.full((rows_out * cols,), 9, dtype=torch.uint8, device="cuda")
+        got, got_t = N.cast_transpose(x, scale, O.E5M2, mode, amax[1], want, rows_out=rows_out)
+        assert got_t.shape == (cols, rows_out) and torch.equal(got_t[:, :rows], ref_t) and not got_t[:, rows:].any()
+        assert (got is None) == (not want)
+        if want:
+            assert got.shape == (rows_out, cols) and torch.equal(got[:rows], ref) and not got[rows:].any()
+            assert torch.equal(amax[0], amax[1])
+    if rows:
+        with pytest.raises(N.NativeError):
+            N.cast_transpose(x, scale, O.E5M2, mode, rows_out=rows - 1)
