@@ -315,6 +315,43 @@ def test_k_slow_layouts_index_check_with_one_hot_operands(N):
     assert torch.equal(out.cpu(), want)
 
 
+def _any_codes(shape, fmt, seed):
+    """Codes drawn uniformly from a format's finite values: products of all sizes, so that another order of addition shows."""
+    c = torch.randint(0, 256, shape, generator=torch.Generator().manual_seed(seed), dtype=torch.uint8)
+    if fmt == O.E5M2:
+        c[(c & 0x7C) == 0x7C] = 0x3C
+    else:
+        c[(c & 0x7F) == 0x7F] = 0x38
+    return c
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape", [(256, 256, 640), (512, 256, 1152), (256, 768, 2176), (4352, 4096, 640)])
+def test_k_slow_layouts_with_an_odd_number_of_k_steps(N, shape, out_dtype):
+    """K an odd multiple of 128: the kernel rounds its K steps up to pairs, and the step it adds multiplies zeros.  What lies
+    behind each operand here is NaN; one shape has 272 tiles, so that blocks go on to a second one.  The bits of the 256 x 256
+    tiled kernel, which walks K in the same order, in every layout; nothing behind the output is written."""
+    M, Nn, K = shape
+    one = torch.tensor([0.25]).cuda(), torch.tensor([0.5]).cuda()
+    nan = {O.E4M3: 0x7F, O.E5M2: 0x7E}
+    a, b = _any_codes((M, K), O.E5M2, 1).cuda(), _any_codes((Nn, K), O.E4M3, 2).cuda()
+    N.gemm_set_variant(2)
+    ref = N.gemm_nt(a, b, O.E5M2, O.E4M3, *one, out_dtype=out_dtype)
+    N.gemm_set_variant(-1)
+    assert torch.isfinite(ref).all()
+
+    def stored(t, slow, fmt):
+        t = t.t().contiguous() if slow else t
+        room = torch.full((t.shape[0] + 256, t.shape[1]), nan[fmt], dtype=torch.uint8, device="cuda")
+        room[:t.shape[0]] = t
+        return room[:t.shape[0]]
+
+    for la, lb in ((N.K_FAST, N.K_FAST), (N.K_FAST, N.K_SLOW), (N.K_SLOW, N.K_FAST), (N.K_SLOW, N.K_SLOW)):
+        room = torch.full((M + 128, Nn), 7.0, dtype=out_dtype, device="cuda")
+        N.gemm_layouts(stored(a, la, O.E5M2), stored(b, lb, O.E4M3), O.E5M2, O.E4M3, la, lb, *one, out=room[:M])
+        assert torch.equal(room[:M], ref) and (room[M:] == 7.0).all(), f"layouts {la}{lb}"
+
+
 def test_k_slow_layouts_refusals(N):
     one = torch.ones(1, device="cuda")
     a = torch.zeros((256, 512), dtype=torch.uint8, device="cuda")
@@ -782,6 +819,30 @@ def test_thin_tiles(N, shape, fmts):
     N.gemm_set_variant(-1)
     for k, (want, out) in enumerate(zip(got[0], got[8])):
         assert torch.equal(want, out), f"output {k}: {(want.float() - out.float()).abs().max()}"
+
+
+@pytest.mark.parametrize("shape", [(16, 4096, 4096), (32, 4096, 14336), (250, 764, 2048), (512, 768, 3072), (32, 768, 50304)])
+@pytest.mark.parametrize("fmts", [(O.E4M3, O.E4M3), (O.E5M2, O.E4M3)])
+def test_thin_tiles_are_as_exact_as_the_tiled_kernel(N, shape, fmts):
+    """Operands that do not sum exactly (Gaussian, quantised), fp32 output, against 64 bits: every element within
+    7 * 2^-14 of sum |a||b| (what the matrix instruction's adder drops) plus the fp32 additions' 2^-24 each, and the error as
+    a whole no larger than that of the 128 x 128 tiles (they differ in the order of the fp32 additions only, which is a
+    hundredth of the adder's share)."""
+    M, Nn, K = shape
+    fa, fb = fmts
+    (a, sa), (b, sb) = quantised((M, K), fa, 1.0, 21), quantised((Nn, K), fb, 0.02, 22)
+    a, b, sa, sb = a.cuda(), b.cuda(), sa.cuda(), sb.cuda()
+    a64, b64 = a.view(O.TORCH_FP8[fa]).double(), b.view(O.TORCH_FP8[fb]).double()
+    s = sa.double() * sb.double()
+    exact, magnitude = (a64 @ b64.t()) * s, (a64.abs() @ b64.abs().t()) * s
+    off = {}
+    for variant in (8, 4):
+        N.gemm_set_variant(variant)
+        diff = (N.gemm_nt(a, b, fa, fb, sa, sb, out_dtype=torch.float32).double() - exact).abs()
+        N.gemm_set_variant(-1)
+        assert bool((diff <= (7 * 2.0 ** -14 + K * 2.0 ** -24) * magnitude).all())
+        off[variant] = (diff.norm() / exact.norm()).item()
+    assert off[8] <= 1.02 * off[4], off
 
 
 @pytest.mark.parametrize("k_steps", [1, 2, 3, 4, 5, 6, 7, 9, 13])

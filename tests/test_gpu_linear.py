@@ -633,6 +633,35 @@ def test_wgrad_reads_dy_as_stored_and_matches_the_transposed_copy_route(amp, mon
         assert max_rel_err(results[True][2], ref["dw"]) <= TOL
 
 
+@pytest.mark.parametrize("wdtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("recipe_name", ["tensorwise", "delayed"])
+@pytest.mark.parametrize("tokens", [624, 1008, 1104])
+def test_wgrad_of_ragged_tokens_reads_dy_as_stored(amp, monkeypatch, tokens, recipe_name, wdtype):
+    """Token counts that are padded to an odd (640, 1152) and an even (1024) number of K steps: the weight gradient comes from
+    the padded row-major codes of dy, with the bits of the route over the transposed copy, and is the oracle's over the
+    tokens there are (under delayed scaling too: the second step of the same tensors runs on their own maxima)."""
+    from optimus_dl_amd import native
+
+    K, N = 512, 768
+    x, w, dy = seeded_bf16((tokens, K), 1.0, 70), seeded_bf16((N, K), 0.02, 71), seeded_bf16((tokens, N), 1e-3, 72)
+    results = {}
+    for direct in (True, False):
+        recipe = amp.create_fp8_recipe(recipe_name, "hybrid", amax_history_len=4)
+        recipe.direct_layouts = direct
+        lin = make_linear(w, dtype=wdtype)
+        run_step(lin, recipe, x, dy)
+        seen, real = [], native.gemm_layouts
+        monkeypatch.setattr(native, "gemm_layouts", lambda a, *r, **k: (seen.append(tuple(a.shape)), real(a, *r, **k))[1])
+        results[direct] = run_step(lin, recipe, x, dy)
+        monkeypatch.setattr(native, "gemm_layouts", real)
+        assert seen == ([(native.padded_rows(tokens), N)] if direct else [])
+    for got, want in zip(results[True], results[False]):
+        assert torch.equal(got, want)
+    ref = O.linear_fwd_bwd(x, w, dy)
+    for got, name in zip(results[True], ("y", "dx", "dw")):
+        assert max_rel_err(got, ref[name]) <= TOL, name
+
+
 def test_mid_sized_weight_gradients_take_the_transposed_copy(amp, monkeypatch):
     """A gradient whose 256 x 256 tiles neither fill the chip nor are few enough not to matter is computed from a
     transposed copy of dy (native.wgrad_direct_pays); the two routes give the same bits."""
