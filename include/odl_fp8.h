@@ -369,6 +369,11 @@ int odl_fp8_cast_delayed(const void *x, int src_dtype, int64_t rows, int64_t col
  * Covers fwd (A=Xq, B=Wq), dgrad (A=dYq, B=Wq^T) and wgrad (A=dYq^T, B=Xq^T):
  * the three GEMMs of te.pytorch.Linear forward/backward.
  * K must be a multiple of 16; any M, N >= 1.
+ * Order of the fp32 additions: along K in 128-byte steps (K % 128 == 0), the same for every kernel and so the same
+ * bits, but for outputs of few tiles with K >= 2048 (decode steps, small gradients): their K steps are dealt to
+ * eight waves whose partial sums are added in wave order.  Which outputs those are depends on M, N, K and the
+ * number of compute units, so a row of a product may differ in its last bits between batch sizes (2-norm, operands
+ * of any finite codes: 2e-7 .. 5e-7 before the rounding to out_dtype).  For given sizes a result is reproducible.
  */
 int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K,
                     int fmt_a, int fmt_b,
@@ -406,8 +411,8 @@ int odl_fp8_gemm_nt_sum(int pairs, const uint8_t *const *a, const uint8_t *const
  *   fwd   Y  = X . W^T      a = X  (K_FAST), b = W  (K_FAST)
  *   dgrad dX = dY . W       a = dY (K_FAST), b = W  (K_SLOW: contraction over N, W is [N, K])
  *   wgrad dW = dY^T . X     a = dY (K_SLOW), b = X  (K_SLOW: contraction over M)
- * Results equal those of odl_fp8_gemm_nt on the transposed copies bit for bit (same order of
- * accumulation).  One scale per operand, no bias, out_dtype ODL_BF16 or ODL_F32 (weight gradients
+ * K is walked in one run, in steps: results equal those of odl_fp8_gemm_nt on the transposed copies bit for
+ * bit where that adds in the same order (all but its outputs of few tiles, see there).  One scale per operand, no bias, out_dtype ODL_BF16 or ODL_F32 (weight gradients
  * of fp32 master weights); M, N multiples of 256, K of 128, K >= 512: anything else is refused with
  * ODL_ERR_SHAPE (make the transposed copy and use odl_fp8_gemm_nt).  There is no accumulate flag here
  * (only the streaming kernel reads K-slow operands): C = C + product with such operands is

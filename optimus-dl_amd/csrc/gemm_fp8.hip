@@ -125,12 +125,12 @@ static void launch_gemm_generic(int fa, int fb, const GemmArgs &g, hipStream_t s
 
 static int cu_count() { return device_cu_count(); }
 
-// Whether the waves of a block sharing K (gemm_thin.hip) beat one 128 x 128 tile per compute unit.  A K step takes the thin
-// kernel 2.7 ns per operand row that the busiest unit fetches, the four-stage 128 x 128 kernel 0.43 us: even at 160 rows,
-// and the line is drawn 10 % below.  Measured on both sides, thin against 128 x 128: 128 rows (32 x 14336 x 4096) 18.6
-// against 21.1 us, 96 rows (512 x 768 x 3072) 10.1 against 13.8, 48 rows (32 x 4096 x 14336) 19.2 against 53.4; 192 rows
-// (768 x 768 x 2048) 13.1 against 10.3, (256 x 4096 x 4096) 22.1 against 17.5.  K under 2048 (fewer than two steps per
-// wave) is left to the tiled kernels: there is no chain to shorten (128 x 3072 x 768: 5.6 against 5.9).
+// Whether the waves of a block sharing K (gemm_thin.hip) beat one 128 x 128 tile per compute unit.  The line in operand
+// rows of the busiest unit lies between what was measured on both sides, thin against 128 x 128: 128 rows (32 x 14336 x
+// 4096) 18.6 against 21.1 us, 96 rows (512 x 768 x 3072) 10.1 against 13.8, 48 rows (32 x 4096 x 14336) 19.2 against 53.4;
+// 192 rows (768 x 768 x 2048) 13.1 against 10.3, (256 x 4096 x 4096) 22.1 against 17.5, though also (64 x 14336 x 4096) 23.9
+// against 25.8.  K under 2048 (fewer than two steps per wave) is left to the tiled kernels: there is no chain to shorten
+// (128 x 3072 x 768: 5.6 against 5.9).
 static bool thin_ok(int64_t M, int64_t N) { return N % 4 == 0 && ((M + 127) / 128) * ((N + 127) / 128) <= cu_count(); }
 
 static bool thin_pays(int64_t M, int64_t N, int64_t K) {
@@ -386,7 +386,8 @@ extern "C" int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t 
 //   split                       : 0.96 us per step of a run + 9 us (pipeline fill, the fp32 epilogue, the second launch)
 //                                 + the partial results, splits x M x N floats written and read back, at 2.7 TB/s in all
 //   each bounded below by its operand traffic (tiles x panel bytes) at about 12 TB/s out of the caches.
-//   one launch, thin tiles      : 4 us + 2.7 ns per K step and operand row of the busiest compute unit (see thin_pays)
+//   one launch, thin tiles      : 4 us + 2.7 ns per K step and operand row of the busiest compute unit (how well that
+//                                 fits: gemm_thin.hip)
 // The runs of a split must fit the compute units at once, and a split must win by 10 %.
 // k_slow: an operand is stored with the contraction index slow (odl_fp8_gemm_layouts), which only the streaming
 // kernel reads: the 128 x 128 kernel is then not an alternative.

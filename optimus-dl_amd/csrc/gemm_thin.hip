@@ -161,9 +161,12 @@ static void launch_thin_fmt(int mt, int nt, const GemmArgs &g, hipStream_t strea
     else launch_thin<4, 2, FA, FB>(g, stream);
 }
 
-// The tile with the least operand rows fetched by the busiest compute unit, rows of a tile x rounds of blocks: a launch
-// takes 4 us + 2.7 ns per such row and K step, whatever the tile (32 x 4096 x 14336 with 16 x 16, 32 x 16, 32 x 32 and
-// 64 x 32 tiles, 64, 48, 64 and 96 rows: 22.3, 19.2, 22.5 and 24.3 us).
+// The tile with the least operand rows fetched by the busiest compute unit, rows of a tile x rounds of blocks (32 x 4096 x
+// 14336 with 16 x 16, 32 x 16, 32 x 32 and 64 x 32 tiles, 64, 48, 64 and 96 rows: 22.3, 19.2, 22.5 and 24.3 us).  With
+// the tile picked so and K >= 2048 a launch takes about 4 us + 2.7 ns per such row and K step: over 16 measured shapes
+// within 14 % but for 32 x 14336 x 4096 (15.1 by the rule, 18.6 measured), 128 x 4096 x 14336 (33.0, 28.5) and 32 x 768 x
+// 50304 (38.0, 29.3).  It says nothing of tiles that are not picked (up to 65 % too much: one round of large tiles) nor of
+// several rounds over a short K (half of what they take).  At all 16 shapes the picked tile was the fastest of the five, or tied.
 static int thin_tile(int64_t M, int64_t N, int num_cus, int *mt_out, int *nt_out) {
     static const int tiles[][2] = {{4, 2}, {2, 2}, {2, 1}, {1, 2}, {1, 1}};
     int64_t best = INT32_MAX;
