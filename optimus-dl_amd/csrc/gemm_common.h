@@ -28,7 +28,7 @@ struct GemmArgs {
     // streaming kernel only, measurement aid: when set, the first wave of block 0 writes {shader-clock counter,
     // 100 MHz counter} on entry and on exit (4 x uint64): the average clock the board granted this launch
     unsigned long long *clock_out = nullptr;
-    // streaming kernel only: block scales of A and B (E8M0 bytes, one per 32 K-bytes), stored K-step-major:
+    // streaming kernel and gemm_deep.hip only: block scales of A and B (E8M0 bytes, one per 32 K-bytes), stored K-step-major:
     // dword [K / 128][rows] = the 4 scale bytes of a row in one 128-byte K step.  Set: the MFMAs apply them.
     const uint8_t *mx_sa = nullptr, *mx_sb = nullptr;
 };
@@ -112,20 +112,22 @@ __device__ __forceinline__ void store_tile(const GemmArgs &g, const v16f &acc, i
 
 
 // ---------------------------------------------------------------- staged epilogue
-// Output path for a wave tile that lies wholly inside the matrix.  The MFMA leaves
+// Output path for a wave tile that lies inside the matrix; with RAGGED its rows may end anywhere.  The MFMA leaves
 // each lane with 4-column fragments of 32 different rows, which as direct stores
 // touch 32 cache lines per instruction.  Instead every slab of 32 rows x (TNS*32)
 // columns of the wave tile is scaled, rounded and written to a private LDS region
 // (rows padded by 16 bytes), then read back 16 bytes per lane along the rows and
 // stored so that a wave instruction writes whole 128-byte lines.
 //   value = acc * (sa_inv[m] * sb_inv[n]) (+ bias[n]); fp32 steps, one final rounding.
-// Requires: N % 8 == 0, n_wave % 8 == 0, 16-byte aligned output / scale vectors / bias,
+// Rows past the last one are not stored (with direct stores instead for the last tile row, 4016 x 2048 x 5632 took 53.7 us
+// in 256 x 128 tiles, the whole 4096 rows 41).
+// Requires: N % 8 == 0, n_wave % 8 == 0, n_wave + 32 TN <= N, 16-byte aligned output / scale vectors / bias,
 // and that nobody else touches `wave_lds` (staged_epilogue_bytes<> bytes).  LDS
 // operations of one wave execute in order, so write -> read -> next write needs no barrier.
 template <bool OUT_BF16, int TNS>
 constexpr int staged_epilogue_bytes() { return 32 * (TNS * 32 * (OUT_BF16 ? 2 : 4) + 16); }
 
-template <bool OUT_BF16, int TM, int TN, int TNS>
+template <bool OUT_BF16, int TM, int TN, int TNS, bool RAGGED = false>
 __device__ __forceinline__ void epilogue_staged(const GemmArgs &g, v16f (&acc)[TM][TN], uint8_t *wave_lds,
                                                 int64_t m_wave, int64_t n_wave, int lane) {
     static_assert(TN % TNS == 0, "slab width must divide the wave tile");
@@ -138,10 +140,12 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs &g, v16f (&acc)[T
     const float s_tensor = g.sa[0] * g.sb[0];
     const float *bias = reinterpret_cast<const float *>(g.bias);
     uint8_t *out = reinterpret_cast<uint8_t *>(g.c);
+    const int rows = RAGGED ? (int)min(g.M - m_wave, (int64_t)(32 * TM)) : 32 * TM;          // of this wave tile
+    if (RAGGED && rows <= 0) return;
 #pragma unroll
     for (int t = 0; t < TM; ++t) {
         float sa = 1.0f;
-        if (vec) sa = g.sa[(m_wave + 32 * t + lr) * g.sa_vec];
+        if (vec) sa = g.sa[(m_wave + (RAGGED ? min(32 * t + lr, rows - 1) : 32 * t + lr)) * g.sa_vec];
 #pragma unroll
         for (int us = 0; us < TN; us += TNS) {
 #pragma unroll
@@ -173,7 +177,7 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs &g, v16f (&acc)[T
                 uint8_t *dst = out + ((m_wave + 32 * t + r) * g.N + n_wave + 32 * us) * ESZ + chunk * 16;
                 // non-temporal: the output is not read by the next kernel, and written through the memory-side
                 // cache it would still be draining to HBM while the next (memory-bound) kernel runs
-                __builtin_nontemporal_store(val, reinterpret_cast<u32x4 *>(dst));
+                if (!RAGGED || 32 * t + r < rows) __builtin_nontemporal_store(val, reinterpret_cast<u32x4 *>(dst));
             }
         }
     }
@@ -183,7 +187,7 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs &g, v16f (&acc)[T
 // once), TNS sub-tiles wide (32 * (TNS * 128 + 16) bytes of `wave_lds`), and a lane that has read back four values of
 // a row adds the four old values of C, which it requested one slab earlier (the loads of slab k + 1 are in flight
 // while slab k is scaled, staged and stored).  Ordinary stores: what is accumulated into is read again.
-template <bool OUT_BF16, int TM, int TN, int TNS>
+template <bool OUT_BF16, int TM, int TN, int TNS, bool RAGGED = false>
 __device__ __forceinline__ void epilogue_staged_accumulate(const GemmArgs &g, v16f (&acc)[TM][TN], uint8_t *wave_lds,
                                                            int64_t m_wave, int64_t n_wave, int lane) {
     static_assert(TN % TNS == 0, "slab width must divide the wave tile");
@@ -197,10 +201,13 @@ __device__ __forceinline__ void epilogue_staged_accumulate(const GemmArgs &g, v1
     const float s_tensor = g.sa[0] * g.sb[0];
     const float *bias = reinterpret_cast<const float *>(g.bias);
     uint8_t *out = reinterpret_cast<uint8_t *>(g.c);
-    auto c_ptr = [&](int slab, int i) -> uint8_t * {   // where this lane's four values of instruction i of a slab live
-        const int t = slab / (TN / TNS), us = (slab % (TN / TNS)) * TNS;
-        const int r = i * RPI + lane / LPR, chunk = lane % LPR;
-        return out + ((m_wave + 32 * t + r) * g.N + n_wave + 32 * us + 4 * chunk) * ESZ;
+    const int rows = RAGGED ? (int)min(g.M - m_wave, (int64_t)(32 * TM)) : 32 * TM;          // of this wave tile
+    if (RAGGED && rows <= 0) return;
+    auto row_of = [&](int slab, int i) { return 32 * (slab / (TN / TNS)) + i * RPI + lane / LPR; };
+    // where this lane's four values of instruction i of a slab live (rows past the last one: the last one, read but not written)
+    auto c_ptr = [&](int slab, int i) -> uint8_t * {
+        const int us = (slab % (TN / TNS)) * TNS, chunk = lane % LPR;
+        return out + ((m_wave + (RAGGED ? min(row_of(slab, i), rows - 1) : row_of(slab, i))) * g.N + n_wave + 32 * us + 4 * chunk) * ESZ;
     };
     auto fetch_old = [&](float (&old)[NI][4], int slab) {
 #pragma unroll
@@ -222,7 +229,7 @@ __device__ __forceinline__ void epilogue_staged_accumulate(const GemmArgs &g, v1
         const int t = slab / (TN / TNS), us = (slab % (TN / TNS)) * TNS;
         if (slab + 1 < SLABS) fetch_old(old[(slab + 1) & 1], slab + 1);
         float sa = 1.0f;
-        if (vec) sa = g.sa[(m_wave + 32 * t + lr) * g.sa_vec];
+        if (vec) sa = g.sa[(m_wave + (RAGGED ? min(32 * t + lr, rows - 1) : 32 * t + lr)) * g.sa_vec];
 #pragma unroll
         for (int uu = 0; uu < TNS; ++uu) {
 #pragma unroll
@@ -249,17 +256,23 @@ __device__ __forceinline__ void epilogue_staged_accumulate(const GemmArgs &g, v1
             const float4 val = *reinterpret_cast<const float4 *>(wave_lds + r * PITCH + chunk * 16);
             const float (&o)[4] = old[slab & 1][i];
             const float w[4] = {o[0] + val.x, o[1] + val.y, o[2] + val.z, o[3] + val.w};
+            if (RAGGED && row_of(slab, i) >= rows) continue;
             if constexpr (OUT_BF16) *reinterpret_cast<u32x2 *>(c_ptr(slab, i)) = u32x2{pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3])};
             else *reinterpret_cast<float4 *>(c_ptr(slab, i)) = float4{w[0], w[1], w[2], w[3]};
         }
     }
 }
 
-// launchers implemented in gemm_tiled.hip / gemm_thin.hip / gemm_pipe.hip / gemm_stream.hip (fa, fb: odl_fp8_format of A and B)
+// launchers implemented in gemm_tiled.hip / gemm_thin.hip / gemm_deep.hip / gemm_pipe.hip / gemm_stream.hip (fa, fb: odl_fp8_format of A and B)
 void launch_gemm_tiled(int variant, int fa, int fb, const GemmArgs &g, hipStream_t stream);
 // operand rows that the busiest compute unit of a thin launch fetches per K step: what the launch costs (gemm_thin.hip)
 int gemm_thin_rows(int64_t M, int64_t N, int num_cus);
 void launch_gemm_thin(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
+// the kernel for outputs of few tiles (gemm_fp8.hip); operands under 2 GiB each, K % 128 == 0
+enum FewTiles { kManyTiles, kTwoBlocks, kDeepWide, kDeep };
+FewTiles gemm_few_tiles(int64_t M, int64_t N, int64_t K, int num_cus);
+// wide: 256 x 128 tiles, else 128 x 128
+void launch_gemm_deep(bool wide, int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
 void launch_gemm_pipe(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
 bool gemm_stream_accepts(const GemmArgs &g);
 void launch_gemm_stream(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);

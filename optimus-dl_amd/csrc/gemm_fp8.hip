@@ -5,6 +5,7 @@
 // Both operands are K-contiguous 8-bit codes ("NT").  Kernels:
 //   gemm_tiled.hip : BM x BN block tiles through two LDS stages
 //   gemm_thin.hip  : small tiles, the waves of a block share K: outputs of few tiles (N % 4 == 0, K % 128 == 0)
+//   gemm_deep.hip  : 256x128 and 128x128 tiles, one block per compute unit, three LDS stages: outputs of about one tile per unit
 //   gemm_pipe.hip  : 256x256 tile, one wave per SIMD, explicit software pipeline
 //   gemm_stream.hip: the same pipeline running across tile boundaries, epilogue under the
 //                    next tile's MFMAs (any M; N, K multiples of 128); with a split over K for
@@ -100,8 +101,10 @@ static const Variant kVariants[] = {
     {"256x256x128 4 waves, software-pipelined, one tile per block", 256, 256, 256, 0.50f},
     {"256x256x128 4 waves, streaming across tiles, folded epilogue (N, K multiples of 128)", 256, 256, 256, 1.25f},
     {"thin tiles, 8 waves sharing K (N % 4 == 0, K % 128 == 0)", 64, 64, 512, 0.0f},
+    {"256x128x128 4 waves (128x64 per wave), three stages, software-pipelined", 256, 128, 256, 0.0f},
+    {"128x128x128 4 waves (64x64 per wave), three stages, software-pipelined", 128, 128, 256, 0.0f},
 };
-constexpr int kPipeVariant = 5, kPipeOneTileVariant = 6, kStreamVariant = 7, kThinVariant = 8;
+constexpr int kPipeVariant = 5, kPipeOneTileVariant = 6, kStreamVariant = 7, kThinVariant = 8, kDeepWideVariant = 9, kDeepVariant = 10;
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 // Forced kernel variant of the calling host thread (-1: choose by shape).  Thread-local: a test or a tuning
 // sweep that pins a variant cannot change the kernels another thread (e.g. the autograd worker) launches.
@@ -138,13 +141,28 @@ static bool thin_pays(int64_t M, int64_t N, int64_t K) {
     return K >= 2048 && thin_ok(M, N) && gemm_thin_rows(M, N, cus) < 145;
 }
 
-static int choose_variant(int64_t M, int64_t N, int64_t K, bool stream_ok) {
+// The kernel for an output of at most num_cus / 2 tiles of 256 x 256, which the big tiles would leave half the chip idle on
+// (kManyTiles: the output has more).  At most one 128 x 128 tile per unit: the pipelined kernel of gemm_deep.hip.  More: 256 x
+// 128 tiles of the same kernel, one per unit, from 24 K steps on (2048 x 4096 x 8192 52.9 us against 60.5 with two 128 x 128
+// blocks per unit, x 4096 30.3 against 32.4); with fewer steps the blocks that hide each other's fill and drain win (x 2048:
+// 18.0 against 18.4, x 1024 11.6 against 12.7).
+FewTiles gemm_few_tiles(int64_t M, int64_t N, int64_t K, int num_cus) {
+    if (((M + 127) / 128) * ((N + 127) / 128) <= num_cus) return kDeep;
+    if (((M + 255) / 256) * ((N + 255) / 256) * 2 > num_cus) return kManyTiles;
+    return K >= 3072 && ((M + 255) / 256) * ((N + 127) / 128) <= num_cus ? kDeepWide : kTwoBlocks;
+}
+
+// ... as a variant (0: many tiles)
+static int few_tiles_variant(int64_t M, int64_t N, int64_t K, bool lim32) {
+    const FewTiles few = gemm_few_tiles(M, N, K, cu_count());
+    if (few == kManyTiles) return 0;
+    return few == kTwoBlocks || !lim32 ? 4 : few == kDeep ? kDeepVariant : kDeepWideVariant;
+}
+
+static int choose_variant(int64_t M, int64_t N, int64_t K, bool stream_ok, bool lim32) {
     const int cus = cu_count();
     if (thin_pays(M, N, K)) return kThinVariant;
-    // an output of at most cus / 2 tiles of 256 x 256 leaves half the chip idle with the big tiles: the 128 x 128
-    // kernel (two blocks per compute unit) spreads it four times wider (measured 15-20 % faster than either
-    // 256-wide kernel at 8192 x 1024, 8192 x 768 and 2048 x 4096 outputs, K = 768 .. 4096)
-    if (((M + 255) / 256) * ((N + 255) / 256) * 2 <= cus) return 4;
+    if (const int small = few_tiles_variant(M, N, K, lim32)) return small;
     int best = 2;
     double best_score = -1.0;
     for (int v = 2; v <= kStreamVariant; ++v) {                       // variant 1 (one wave per SIMD) only by explicit request
@@ -231,13 +249,14 @@ static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_
     // C = C + product is an epilogue of the kernels whose tiles end in a separate output phase; the streaming kernel
     // stores a tile under the next tile's MFMAs, where nothing can wait for the old values of C
     const bool stream_ok = tiled_ok && lim32 && N % 128 == 0 && K >= 512 && !accumulate;
-    int variant = launch_as >= 0 ? launch_as : t_forced_variant >= 0 ? t_forced_variant : (tiled_ok ? choose_variant(M, N, K, stream_ok) : 0);
+    int variant = launch_as >= 0 ? launch_as : t_forced_variant >= 0 ? t_forced_variant : (tiled_ok ? choose_variant(M, N, K, stream_ok, lim32) : 0);
     if (variant != 0 && !tiled_ok) variant = 0;
     // the pipelined kernel walks K in pairs of 128-byte steps
     const bool pipe_ok = tiled_ok && K % 256 == 0 && lim32;
     if ((variant == kPipeVariant || variant == kPipeOneTileVariant) && !pipe_ok) variant = 2;
 
     if (variant == kThinVariant && !thin_ok(M, N)) variant = 4;
+    if ((variant == kDeepVariant || variant == kDeepWideVariant) && !lim32) variant = 4;
 
     if (variant == kStreamVariant && t_forced_variant < 0 && launch_as < 0) {
         const int64_t rest = tail_rows(M, N, K), head = M - rest;
@@ -247,7 +266,8 @@ static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_
                                            kStreamVariant, stream);
             if (rc != ODL_OK) return rc;
             return gemm_nt_checked(a + head * K, b, rest, N, K, fmt_a, fmt_b, sa_n == 1 ? sa_inv : sa_inv + head, sa_n == 1 ? 1 : rest, sb_inv, sb_n,
-                                   bias, reinterpret_cast<uint8_t *>(c) + head * N * esz, out_dtype, accumulate, 4, stream);
+                                   bias, reinterpret_cast<uint8_t *>(c) + head * N * esz, out_dtype, accumulate,
+                                   few_tiles_variant(rest, N, K, lim32), stream);
         }
     }
 
@@ -269,6 +289,7 @@ static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_
     }
     if (variant == 0) launch_gemm_generic(fmt_a, fmt_b, g, stream);
     else if (variant == kThinVariant) launch_gemm_thin(fmt_a, fmt_b, g, cu_count(), stream);
+    else if (variant == kDeepWideVariant || variant == kDeepVariant) launch_gemm_deep(variant == kDeepWideVariant, fmt_a, fmt_b, g, cu_count(), stream);
     else if (variant == kPipeVariant) launch_gemm_pipe(fmt_a, fmt_b, g, cu_count(), stream);
     else if (variant == kPipeOneTileVariant) launch_gemm_pipe(fmt_a, fmt_b, g, 1 << 30, stream);
     else if (variant == kStreamVariant) { attach_clock_probe(g); launch_gemm_stream(fmt_a, fmt_b, g, cu_count(), stream); }
@@ -380,12 +401,15 @@ extern "C" int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t 
 // How many runs to cut K into for an output of few tiles (1 = do not split).  A model in microseconds, fitted to
 // measurements on this GPU (outputs 768 x 768 .. 8192 x 1024, K = 8192 .. 151936):
 //   one launch, 256 x 256 tiles : 0.92 us per K step of 128 (few compute units busy: high clock) + 3 steps of overhead
-//   one launch, 128 x 128 tiles : 0.55 us per step where every block has a compute unit to itself (the four-stage form
-//                                 of the kernel), 0.62 with two blocks per unit (what odl_fp8_gemm_nt takes for outputs
-//                                 of <= cus / 2 big tiles); it reads every operand panel twice as often
+//   one launch, smaller tiles   : what odl_fp8_gemm_nt takes for outputs of <= cus / 2 big tiles (few_tiles_variant).
+//                                 128 x 128 with a unit each 0.37 us per step + 6 us (3072 x 768 x 16384: 45 - 50 us, in
+//                                 six runs 52 and the reduction's launch); 256 x 128 with a unit each 0.70 + 7 (0.82 where the
+//                                 operands outgrow the 256 MB memory-side cache: 8192 x 768 x 50304 328 us); two 128 x 128
+//                                 blocks per unit 0.62 (it reads every operand panel twice as often)
 //   split                       : 0.96 us per step of a run + 9 us (pipeline fill, the fp32 epilogue, the second launch)
 //                                 + the partial results, splits x M x N floats written and read back, at 2.7 TB/s in all
-//   each bounded below by its operand traffic (tiles x panel bytes) at about 12 TB/s out of the caches.
+//   each bounded below by its operand traffic (tiles x panel bytes) at about 12 TB/s out of the caches (the kernels of
+//   gemm_deep.hip: 18).
 //   one launch, thin tiles      : 4 us + 2.7 ns per K step and operand row of the busiest compute unit (how well that
 //                                 fits: gemm_thin.hip)
 // The runs of a split must fit the compute units at once, and a split must win by 10 %.
@@ -401,10 +425,13 @@ extern "C" int odl_fp8_gemm_split_count(int64_t M, int64_t N, int64_t K, int k_s
     const double traffic_us = (double)tiles * 512.0 * (double)K / 12.0e6;
     double whole = 0.92 * ((double)steps + 3.0);
     if (whole < traffic_us) whole = traffic_us;
-    if (tiles * 2 <= cus && !k_slow) {
-        const int64_t small_tiles = ((M + 127) / 128) * ((N + 127) / 128);
-        double small = (small_tiles <= cus ? 0.55 : 0.62) * ((double)steps + 3.0);
-        const double small_traffic_us = (double)small_tiles * 256.0 * (double)K / 12.0e6;
+    if (!k_slow) {
+        const int variant = few_tiles_variant(M, N, K, (double)(M + 256) * (double)K < 2147483648.0 && (double)(N + 256) * (double)K < 2147483648.0);
+        const double panels = (double)((M + 127) / 128) * (double)((N + 127) / 128) * (double)K;         // of 128 rows, once per tile
+        double small = whole, small_traffic_us = 0.0;
+        if (variant == kDeepVariant) { small = 0.37 * (double)steps + 6.0; small_traffic_us = panels * 256.0 / 18.0e6; }
+        else if (variant == kDeepWideVariant) { small = ((double)(M + N) * (double)K > 268435456.0 ? 0.82 : 0.70) * (double)steps + 7.0; small_traffic_us = panels * 192.0 / 18.0e6; }
+        else if (variant) { small = 0.62 * ((double)steps + 3.0); small_traffic_us = panels * 256.0 / 12.0e6; }
         if (small < small_traffic_us) small = small_traffic_us;
         if (small < whole) whole = small;
     }

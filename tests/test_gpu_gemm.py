@@ -878,3 +878,33 @@ def test_last_round_in_smaller_tiles_has_the_same_bits(N, shape, out_dtype):
         N.gemm_set_variant(2)
         assert torch.equal(auto, N.gemm_nt(aq, bq, O.E4M3, O.E4M3, *args, out_dtype=out_dtype, **kw))
         N.gemm_set_variant(-1)
+
+
+@pytest.mark.parametrize("variant", [4, 9, 10])
+@pytest.mark.parametrize("M,Nn,K", [(16, 16, 128), (129, 144, 256), (200, 136, 384), (255, 264, 512), (300, 20, 640), (513, 392, 1152), (64, 1000, 2176)])
+def test_few_tile_kernels_at_ragged_edges(N, variant, M, Nn, K):
+    """128 x 128 and 256 x 128 tiles that end inside the matrix, in rows and in columns, for every form of the output: one
+    scale, scales per row and column with a bias, added to what is there.  Lengths of K shorter than the pipeline and odd in
+    steps; far fewer tiles than compute units.  Codes, scales, bias and old values are small multiples of powers of two:
+    every sum is exact in fp32, so the result is known to the bit."""
+    g = torch.Generator().manual_seed(M + Nn + K + variant)
+    values = torch.tensor([0.0, 0.5, 1.0, -1.0, 2.0, -0.5])
+    a, b = values[torch.randint(0, 6, (M, K), generator=g)], values[torch.randint(0, 6, (Nn, K), generator=g)]
+    ac, bc = (t.to(torch.float8_e4m3fn).view(torch.uint8).cuda() for t in (a, b))
+    product = a.double() @ b.double().t()
+    one, half = torch.tensor([0.5]), torch.tensor([0.25])
+    sa, sb = 2.0 ** torch.randint(-1, 2, (M,), generator=g), 2.0 ** torch.randint(-1, 2, (Nn,), generator=g)
+    bias = torch.randint(-8, 8, (Nn,), generator=g).float()
+    old = torch.randint(-64, 64, (M, Nn), generator=g).float()
+    N.gemm_set_variant(variant)
+    try:
+        for dtype in (torch.bfloat16, torch.float32):
+            got = N.gemm_nt(ac, bc, O.E4M3, O.E4M3, one.cuda(), half.cuda(), out_dtype=dtype)
+            assert torch.equal(got.cpu(), (product * 0.125).float().to(dtype))
+            got = N.gemm_nt(ac, bc, O.E4M3, O.E4M3, sa.cuda(), sb.cuda(), bias=bias.cuda(), out_dtype=dtype)
+            assert torch.equal(got.cpu(), (product * sa[:, None].double() * sb[None].double() + bias.double()).float().to(dtype))
+            out = old.to(dtype).cuda()
+            N.gemm_nt(ac, bc, O.E4M3, O.E4M3, one.cuda(), half.cuda(), out=out, accumulate=True)
+            assert torch.equal(out.cpu(), (product * 0.125 + old.double()).float().to(dtype))
+    finally:
+        N.gemm_set_variant(-1)
