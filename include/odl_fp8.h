@@ -524,6 +524,13 @@ int odl_fp8_gemm_set_clock_probe(uint64_t *records_dev, int capacity);
 #define ODL_MX_SCALE_CEIL 1
 int odl_fp8_mx_cast(const void *x, int src_dtype, int64_t rows, int64_t cols, int fmt, uint8_t *out, uint8_t *scales,
                     int scales_layout, uint8_t *out_t, uint8_t *scales_t, int scales_t_layout, int scale_rule, odl_stream_t stream);
+/* The same with the transposed pair padded: out_t is [cols, rows_out], scales_t for [cols, rows_out / 32] blocks, zero codes
+ * with scale byte 0 behind those of x (rows_out >= rows; rows and rows_out multiples of 32, rows_out of 128 for K-step-major
+ * scales_t).  A weight gradient contracts the rows: with rows_out a multiple of 128 it finds whole K steps at any token
+ * count, and what was added contributes nothing.  out and scales are those of odl_fp8_mx_cast. */
+int odl_fp8_mx_cast_padded(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, int fmt, uint8_t *out,
+                           uint8_t *scales, int scales_layout, uint8_t *out_t, uint8_t *scales_t, int scales_t_layout,
+                           int scale_rule, odl_stream_t stream);
 
 /*
  * C[M, N] = sum over blocks kb of 2^(sa[m, kb] - 127) * 2^(sb[n, kb] - 127) * dot(A[m, 32 kb .. +32], B[n, 32 kb .. +32])

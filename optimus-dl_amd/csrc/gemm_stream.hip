@@ -1,7 +1,7 @@
 // FP8 GEMM, 256x256 block tile, 4 waves (one per SIMD, 128x128 each), persistent,
 // with the epilogue of every tile folded under the first MFMAs of the next one.
 // C = (A[M,K] . B[N,K]^T) * (sa_inv * sb_inv) (+ bias) in bf16 or fp32, for the shapes training uses:
-// any M, N % 128 == 0, K % 128 == 0, K >= 512; scales per tensor or per row of A / B (block scales: M % 128 == 0).
+// any M, N % 128 == 0, K % 128 == 0, K >= 512; scales per tensor, per row of A / B, or per block.
 // Everything else goes to gemm_pipe.hip, whose K step this kernel shares:
 //
 //   per K step of 128 bytes (two halves h0, h1 of 64 bytes = one MFMA K each)
@@ -734,14 +734,15 @@ void launch_fmt(const GemmArgs &g, int blocks_per_xcd, hipStream_t stream) {
 
 // Shapes this kernel takes (the caller checks the 32-bit offset limits shared with gemm_pipe.hip).
 // An operand stored [K, rows] must fill whole tiles: the loads of a partial tile would run past the
-// end of its last K-row.  Stored [rows, K], A may end anywhere and B after half a tile (see wave_inside); block
-// scales are fetched for 128 rows at a time.
+// end of its last K-row.  Stored [rows, K], A may end anywhere and B after half a tile (see wave_inside).
+// Block scales are fetched for 128 rows at a time: behind the last row lie the next K step's, and what they scale is zero and
+// not stored.
 bool gemm_stream_accepts(const GemmArgs &g) {
     const double esz = (g.out_dtype == ODL_F32 || g.splits > 1) ? 4.0 : 2.0;
     const bool vectors = g.splits == 1 && (g.sa_vec || g.sb_vec || g.bias != nullptr);   // only with both operands stored [rows, K]
     if (g.mx_sa && (g.ta || g.tb || g.sa_vec || g.sb_vec || !g.mx_sb)) return false;
     return !g.accumulate && (g.out_dtype == ODL_BF16 || g.out_dtype == ODL_F32) && !(vectors && (g.ta || g.tb)) &&
-           g.M % (g.ta ? BM : g.mx_sa ? WM : 1) == 0 && g.N % (g.tb ? BN : WN) == 0 && g.K % 128 == 0 && g.K >= 512 && (double)g.N * esz * (BM + 8) < 2147483648.0;
+           g.M % (g.ta ? BM : 1) == 0 && g.N % (g.tb ? BN : WN) == 0 && g.K % 128 == 0 && g.K >= 512 && (double)g.N * esz * (BM + 8) < 2147483648.0;
 }
 
 // Operand pairs: each a whole even number of K steps, four at least (the load pipeline is two steps deep and crosses

@@ -136,11 +136,13 @@ __device__ __forceinline__ uint32_t cvt_scaled4(uint32_t p0, uint32_t p1, uint32
 // neighbouring lanes; fp32 source, columns 4 tx .. + 3 and 32 + 4 tx .. + 3 (every load instruction contiguous over the
 // 8 lanes of a row), so the first groups of the 8 lanes are one block and the second groups the other.  A block along
 // the rows (32 of them) is held by the 8 lanes of a wave that share tx.  All maxima are exchanges inside the wave.
+// The transposed codes are rows_t >= rows long: zero codes with scale byte 0 behind those of x, so that a GEMM that contracts
+// the rows finds whole K steps.
 template <int SRC, int FMT, bool WANT_ROW, bool WANT_COL>
 __global__ __launch_bounds__(kMxThreads) void mx_cast_kernel(const void *__restrict__ x, int64_t rows, int64_t cols,
                                                               uint8_t *__restrict__ out, uint8_t *__restrict__ scales,
                                                               uint8_t *__restrict__ out_t, uint8_t *__restrict__ scales_t,
-                                                              int layout, int layout_t, int rule) {
+                                                              int layout, int layout_t, int rule, int64_t rows_t) {
     __shared__ __attribute__((aligned(16))) uint8_t tile[kTileC * kTileR];
     // K-step-major scale bytes leave the block as whole runs: the tile's 4 row blocks are one dword per column (256
     // contiguous bytes per tile), its 2 column blocks one 16-bit half of a dword per row.  Stored a byte at a time from
@@ -150,8 +152,8 @@ __global__ __launch_bounds__(kMxThreads) void mx_cast_kernel(const void *__restr
     saturate_fp8_conversions();
     constexpr int ESZ = SRC == ODL_BF16 ? 2 : 4;
     const int tx = threadIdx.x % 8, ty = threadIdx.x / 8;
-    const int64_t tiles_r = (rows + kTileR - 1) / kTileR, tiles_c = (cols + kTileC - 1) / kTileC;
-    // (K-step-major implies whole dwords: cols % 128 == 0 for `scales`, rows % 128 == 0 for `scales_t`; host-checked)
+    const int64_t tiles_r = ((WANT_COL ? rows_t : rows) + kTileR - 1) / kTileR, tiles_c = (cols + kTileC - 1) / kTileC;
+    // (K-step-major implies whole dwords: cols % 128 == 0 for `scales`, rows_t % 128 == 0 for `scales_t`; host-checked)
     const bool staged_r = WANT_ROW && WANT_COL && layout == ODL_MX_SCALES_KSTEP;
     const bool staged_t = WANT_COL && layout_t == ODL_MX_SCALES_KSTEP;
     int64_t tr, tc;
@@ -248,7 +250,7 @@ __global__ __launch_bounds__(kMxThreads) void mx_cast_kernel(const void *__restr
     }
 
     if constexpr (WANT_COL) {
-        const int64_t nbt = rows / kMxBlock;
+        const int64_t nbt = rows_t / kMxBlock;
         float mul_c[8], e8_c[8];
         uint32_t col_bytes[2] = {0u, 0u};                                // the scale bytes of the lane's 8 columns, packed
         uint32_t cmax[8];                                                // fp32 magnitude bits per column, over the 32 rows
@@ -270,9 +272,9 @@ __global__ __launch_bounds__(kMxThreads) void mx_cast_kernel(const void *__restr
             uint32_t byte;
             mx_scale_of<FMT>(cmax[j], rule, byte, mul_c[j]);
             e8_c[j] = bits_to_float(byte << 23);
-            // rows % 32 == 0 (host-checked): a row block is inside the matrix as a whole or not at all
+            // rows_t % 32 == 0 (host-checked): a row block is inside the matrix as a whole or not at all
             col_bytes[j / 4] |= byte << (8 * (j % 4));
-            if (!staged_t && (ty & 7) == 0 && (j < 4 ? okA : okB) && r0 < rows)
+            if (!staged_t && (ty & 7) == 0 && (j < 4 ? okA : okB) && r0 < rows_t)
                 scales_t[mx_scale_at(layout_t, col_of(j), r0 / kMxBlock, cols, nbt)] = (uint8_t)byte;
         }
         // staged: the wave's row block is one plane of 64 bytes, a lane's two groups of 4 columns a 4-byte write each
@@ -323,15 +325,15 @@ __global__ __launch_bounds__(kMxThreads) void mx_cast_kernel(const void *__restr
             const int chunk = threadIdx.x + it * kMxThreads;
             const int k = chunk / 8, m16 = chunk % 8;
             const int64_t oc = tc * kTileC + k, orow = tr * kTileR + m16 * 16;
-            if (oc < cols && orow < rows)
-                __builtin_nontemporal_store(ct_lds_read(tile, k, m16), reinterpret_cast<u32x4 *>(out_t + oc * rows + orow));
+            if (oc < cols && orow < rows_t)
+                __builtin_nontemporal_store(ct_lds_read(tile, k, m16), reinterpret_cast<u32x4 *>(out_t + oc * rows_t + orow));
         }
         // the staged scale bytes: dword [tile row][column] of scales_t from the first wave, the 16-bit half
         // [tile column / 2][row] of scales from the next two
         if (staged_t && threadIdx.x < kTileC) {
             const int64_t oc = tc * kTileC + threadIdx.x;
             const int c = threadIdx.x;
-            if (oc < cols && tr * kTileR < rows)
+            if (oc < cols && tr * kTileR < rows_t)
                 reinterpret_cast<uint32_t *>(scales_t)[tr * cols + oc] = (uint32_t)stage_t[c] | ((uint32_t)stage_t[kTileC + c] << 8) |
                                                                          ((uint32_t)stage_t[2 * kTileC + c] << 16) | ((uint32_t)stage_t[3 * kTileC + c] << 24);
         }
@@ -804,9 +806,9 @@ const float *unit_scale_for_current_device(const char *who) {
 
 template <int SRC, int FMT>
 static void launch_mx_cast(const void *x, int64_t rows, int64_t cols, uint8_t *out, uint8_t *scales, uint8_t *out_t, uint8_t *scales_t,
-                           int layout, int layout_t, int rule, hipStream_t stream) {
-    const int64_t g = ((rows + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
-#define ODL_MX(R, C) hipLaunchKernelGGL((mx_cast_kernel<SRC, FMT, R, C>), dim3((unsigned)g), dim3(kMxThreads), 0, stream, x, rows, cols, out, scales, out_t, scales_t, layout, layout_t, rule)
+                           int layout, int layout_t, int rule, int64_t rows_t, hipStream_t stream) {
+    const int64_t g = (((out_t ? rows_t : rows) + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
+#define ODL_MX(R, C) hipLaunchKernelGGL((mx_cast_kernel<SRC, FMT, R, C>), dim3((unsigned)g), dim3(kMxThreads), 0, stream, x, rows, cols, out, scales, out_t, scales_t, layout, layout_t, rule, rows_t)
     if (out && out_t) ODL_MX(true, true);
     else if (out) ODL_MX(true, false);
     else ODL_MX(false, true);
@@ -872,40 +874,46 @@ static void launch_block_cast(const void *x, int64_t rows, int64_t cols, int mar
 
 using namespace odl;
 
-extern "C" int odl_fp8_mx_cast(const void *x, int src_dtype, int64_t rows, int64_t cols, int fmt, uint8_t *out, uint8_t *scales,
+extern "C" int odl_fp8_mx_cast_padded(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, int fmt, uint8_t *out, uint8_t *scales,
                                int scales_layout, uint8_t *out_t, uint8_t *scales_t, int scales_t_layout, int scale_rule,
                                odl_stream_t stream_) {
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
-    if (rows < 0 || cols < 0) return set_error(ODL_ERR_ARG, "odl_fp8_mx_cast: negative shape");
+    if (rows < 0 || cols < 0 || rows_out < rows) return set_error(ODL_ERR_ARG, "odl_fp8_mx_cast: negative shape");
     if (scale_rule != ODL_MX_SCALE_FLOOR && scale_rule != ODL_MX_SCALE_CEIL) return set_error(ODL_ERR_ARG, "odl_fp8_mx_cast: scale_rule %d", scale_rule);
     if (src_dtype != ODL_BF16 && src_dtype != ODL_F32) return set_error(ODL_ERR_ARG, "odl_fp8_mx_cast: src_dtype %d", src_dtype);
     if (fmt != ODL_FP8_E4M3 && fmt != ODL_FP8_E5M2) return set_error(ODL_ERR_ARG, "odl_fp8_mx_cast: fmt %d", fmt);
-    if (rows * cols == 0) return ODL_OK;
+    if (cols == 0 || rows_out == 0 || (rows == 0 && !out_t)) return ODL_OK;
     if ((out == nullptr) != (scales == nullptr) || (out_t == nullptr) != (scales_t == nullptr))
         return set_error(ODL_ERR_ARG, "odl_fp8_mx_cast: codes and scale bytes of a layout go together");
     if (!out && !out_t) return set_error(ODL_ERR_ARG, "odl_fp8_mx_cast: neither layout asked for");
     auto bad_layout = [](int l) { return l != ODL_MX_SCALES_ROWMAJOR && l != ODL_MX_SCALES_KSTEP; };
     if ((out && bad_layout(scales_layout)) || (out_t && bad_layout(scales_t_layout)))
         return set_error(ODL_ERR_ARG, "odl_fp8_mx_cast: scale layouts %d, %d", scales_layout, scales_t_layout);
-    if ((out && scales_layout == ODL_MX_SCALES_KSTEP && cols % 128 != 0) || (out_t && scales_t_layout == ODL_MX_SCALES_KSTEP && rows % 128 != 0))
+    if ((out && scales_layout == ODL_MX_SCALES_KSTEP && cols % 128 != 0) || (out_t && scales_t_layout == ODL_MX_SCALES_KSTEP && rows_out % 128 != 0))
         return set_error(ODL_ERR_SHAPE, "odl_fp8_mx_cast: K-step-major scales need the blocked axis to be a multiple of 128 (%lld x %lld)",
                          (long long)rows, (long long)cols);
-    if (!x) return set_error(ODL_ERR_ARG, "odl_fp8_mx_cast: x is null");
-    if (cols % 8 != 0 || (out && cols % kMxBlock != 0) || (out_t && rows % kMxBlock != 0))
+    if (!x && rows > 0) return set_error(ODL_ERR_ARG, "odl_fp8_mx_cast: x is null");
+    if (cols % 8 != 0 || (out && cols % kMxBlock != 0) || (out_t && (rows % kMxBlock != 0 || rows_out % kMxBlock != 0)))
         return set_error(ODL_ERR_SHAPE, "odl_fp8_mx_cast: %lld x %lld: the blocked axis must be a multiple of 32 (cols for out, rows for out_t) and cols of 8",
                          (long long)rows, (long long)cols);
     auto mis = [](const void *p, uintptr_t a) { return p && (reinterpret_cast<uintptr_t>(p) & (a - 1)); };
     if (mis(x, 16) || mis(out, 8) || mis(out_t, 16)) return set_error(ODL_ERR_SHAPE, "odl_fp8_mx_cast: x and out_t must be 16-byte aligned, out 8-byte");
-    const int64_t tiles = ((rows + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
+    const int64_t tiles = (((out_t ? rows_out : rows) + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC);
     if (tiles > 0x7fffffffLL) return set_error(ODL_ERR_SHAPE, "odl_fp8_mx_cast: too many tiles for one launch");
     if (src_dtype == ODL_BF16) {
-        if (fmt == ODL_FP8_E4M3) launch_mx_cast<ODL_BF16, ODL_FP8_E4M3>(x, rows, cols, out, scales, out_t, scales_t, scales_layout, scales_t_layout, scale_rule, stream);
-        else launch_mx_cast<ODL_BF16, ODL_FP8_E5M2>(x, rows, cols, out, scales, out_t, scales_t, scales_layout, scales_t_layout, scale_rule, stream);
+        if (fmt == ODL_FP8_E4M3) launch_mx_cast<ODL_BF16, ODL_FP8_E4M3>(x, rows, cols, out, scales, out_t, scales_t, scales_layout, scales_t_layout, scale_rule, rows_out, stream);
+        else launch_mx_cast<ODL_BF16, ODL_FP8_E5M2>(x, rows, cols, out, scales, out_t, scales_t, scales_layout, scales_t_layout, scale_rule, rows_out, stream);
     } else {
-        if (fmt == ODL_FP8_E4M3) launch_mx_cast<ODL_F32, ODL_FP8_E4M3>(x, rows, cols, out, scales, out_t, scales_t, scales_layout, scales_t_layout, scale_rule, stream);
-        else launch_mx_cast<ODL_F32, ODL_FP8_E5M2>(x, rows, cols, out, scales, out_t, scales_t, scales_layout, scales_t_layout, scale_rule, stream);
+        if (fmt == ODL_FP8_E4M3) launch_mx_cast<ODL_F32, ODL_FP8_E4M3>(x, rows, cols, out, scales, out_t, scales_t, scales_layout, scales_t_layout, scale_rule, rows_out, stream);
+        else launch_mx_cast<ODL_F32, ODL_FP8_E5M2>(x, rows, cols, out, scales, out_t, scales_t, scales_layout, scales_t_layout, scale_rule, rows_out, stream);
     }
     return check_launch("odl_fp8_mx_cast");
+}
+
+extern "C" int odl_fp8_mx_cast(const void *x, int src_dtype, int64_t rows, int64_t cols, int fmt, uint8_t *out, uint8_t *scales,
+                               int scales_layout, uint8_t *out_t, uint8_t *scales_t, int scales_t_layout, int scale_rule,
+                               odl_stream_t stream_) {
+    return odl_fp8_mx_cast_padded(x, src_dtype, rows, cols, rows, fmt, out, scales, scales_layout, out_t, scales_t, scales_t_layout, scale_rule, stream_);
 }
 
 extern "C" int odl_fp8_mx_gemm_nt(const uint8_t *a, const uint8_t *sa, const uint8_t *b, const uint8_t *sb, int scales_layout, int64_t M,

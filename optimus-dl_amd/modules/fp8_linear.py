@@ -125,10 +125,11 @@ def _quantise_input_shared(recipe: FP8Recipe, x2d: torch.Tensor, fmt: int, margi
 
 def _block_cast(pol, x2d: torch.Tensor, fmt: int, want_rowmajor: bool, want_transposed: bool, weight: bool = False):
     """Codes and E8M0 scale bytes of the two block-scaled recipes: 32-element blocks (mxfp8) or 128-element blocks with
-    128 x 128 ones for a weight (blockwise)."""
+    128 x 128 ones for a weight (blockwise).  The transposed codes of activations and gradients, which a weight gradient
+    contracts over the tokens, are padded to whole K steps (``native.padded_rows``; blockwise takes whole blocks of 128 only)."""
     if pol.kind == "mxfp8":
         return native.mx_cast(x2d, fmt, want_rowmajor=want_rowmajor, want_transposed=want_transposed,
-                              scale_rule=pol.mx_scale_rule)
+                              scale_rule=pol.mx_scale_rule, rows_out=None if weight else native.padded_rows(x2d.shape[0]))
     return native.block_cast(x2d, fmt, pol.margin, two_d=weight, want_rowmajor=want_rowmajor, want_transposed=want_transposed)
 
 

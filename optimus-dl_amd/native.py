@@ -24,7 +24,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 18
+ABI_VERSION = 19
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -75,6 +75,7 @@ EXPORTS = (
     "odl_fp8_gemm_set_variant",
     "odl_fp8_gemm_set_clock_probe",
     "odl_fp8_mx_cast",
+    "odl_fp8_mx_cast_padded",
     "odl_fp8_mx_gemm_nt",
     "odl_fp8_block_cast",
     "odl_fp8_mx_gemm_splitk",
@@ -152,6 +153,7 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_gemm_variant_name.restype = ctypes.c_char_p
         L.odl_fp8_gemm_set_variant.argtypes = [i32]
         L.odl_fp8_gemm_set_clock_probe.argtypes = [vp, i32]
+        L.odl_fp8_mx_cast_padded.argtypes = [vp, i32, i64, i64, i64, i32, vp, vp, i32, vp, vp, i32, i32, vp]
         L.odl_fp8_mx_cast.argtypes = [vp, i32, i64, i64, i32, vp, vp, i32, vp, vp, i32, i32, vp]
         L.odl_fp8_mx_gemm_nt.argtypes = [vp, vp, vp, vp, i32, i64, i64, i64, i32, i32, vp, vp, i32, i32, vp]
         L.odl_fp8_block_cast.argtypes = [vp, i32, i64, i64, i32, i32, i32, vp, vp, vp, vp, vp]
@@ -866,28 +868,30 @@ def mx_scales_rowmajor(scales: torch.Tensor) -> torch.Tensor:
 
 
 def mx_cast(x: torch.Tensor, fmt: int, want_rowmajor: bool = True, want_transposed: bool = False, layout: int | None = None,
-            scale_rule: int = MX_FLOOR):
+            scale_rule: int = MX_FLOOR, rows_out: int | None = None):
     """MXFP8 conversion of ``x`` [rows, cols] in one launch -> (codes [rows, cols], their scales, codes_t [cols, rows],
     their scales); the pair that was not asked for is (None, None).  Scales are E8M0 bytes, one per 32 elements along
     the last axis of the codes they belong to, stored as ``_mx_scales`` describes (layout None: K-step-major where the
     blocked axis allows it).  scale_rule: MX_FLOOR (the OCP formula; a block amax in the top eighth of its binade
-    saturates) or MX_CEIL (the exponent rounded up: nothing saturates)."""
+    saturates) or MX_CEIL (the exponent rounded up: nothing saturates).  rows_out: the transposed codes and their scales are
+    that many rows of x long, zero codes with scale byte 0 behind those of x (see :func:`padded_rows`)."""
     x = _as_2d(x)
     rows, cols = x.shape
     if not (want_rowmajor or want_transposed):
         raise NativeError("mx_cast: neither layout asked for")
     dev = x.device
+    n = rows if rows_out is None else rows_out
     out = sc = out_t = sc_t = None
     lay = lay_t = MX_ROWMAJOR
     if want_rowmajor:
         out = torch.empty((rows, cols), dtype=torch.uint8, device=dev)
         sc, lay = _mx_scales(rows, cols, layout, dev)
     if want_transposed:
-        out_t = torch.empty((cols, rows), dtype=torch.uint8, device=dev)
-        sc_t, lay_t = _mx_scales(cols, rows, layout, dev)
+        out_t = torch.empty((cols, n), dtype=torch.uint8, device=dev)
+        sc_t, lay_t = _mx_scales(cols, n, layout, dev)
     ptr = lambda t: t.data_ptr() if t is not None else None
-    _check(load().odl_fp8_mx_cast(x.data_ptr(), _src_dtype(x), rows, cols, fmt, ptr(out), ptr(sc), lay, ptr(out_t), ptr(sc_t), lay_t,
-                                  int(scale_rule), _stream()), "odl_fp8_mx_cast")
+    _check(load().odl_fp8_mx_cast_padded(x.data_ptr(), _src_dtype(x), rows, cols, n, fmt, ptr(out), ptr(sc), lay, ptr(out_t), ptr(sc_t),
+                                         lay_t, int(scale_rule), _stream()), "odl_fp8_mx_cast")
     return out, sc, out_t, sc_t
 
 

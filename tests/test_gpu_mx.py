@@ -537,3 +537,55 @@ def test_mx_gemm_split_over_k_matches_the_single_launch(N, shape):
     rc = real(aq.data_ptr(), asc.data_ptr(), bq.data_ptr(), bsc.data_ptr(), M, N_, K, E5M2, E4M3, None, out.data_ptr(), 1, 0, 4,
               ws.data_ptr(), 64, None)
     assert rc != 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols,rows_out", [(32, 64, 128), (96, 200, 128), (160, 72, 256), (288, 128, 384), (128, 96, 128), (64, 64, 320)])
+def test_mx_cast_pads_the_transposed_codes(N, dtype, rows, cols, rows_out):
+    x = seeded_bf16((rows, cols), 1.0, rows + cols).to(dtype).cuda()
+    row = cols % 32 == 0
+    q, s, qt, st = N.mx_cast(x, E4M3, row, True, scale_rule=N.MX_CEIL, rows_out=rows_out)
+    want_q, want_s, want_t, want_st = N.mx_cast(x, E4M3, row, True, layout=N.MX_ROWMAJOR, scale_rule=N.MX_CEIL)
+    if row:
+        assert torch.equal(q, want_q) and torch.equal(N.mx_scales_rowmajor(s), want_s)
+    assert qt.shape == (cols, rows_out)
+    assert torch.equal(qt[:, :rows], want_t) and not qt[:, rows:].any()
+    st = N.mx_scales_rowmajor(st)
+    assert torch.equal(st[:, :rows // 32], want_st) and not st[:, rows // 32:].any()
+
+
+@pytest.mark.parametrize("M,N_,K", [(4000, 4480, 640), (4128, 4352, 512)])
+def test_mx_streaming_kernel_ends_at_any_row(N, M, N_, K):
+    """The last 128 rows of A partly outside: behind them lie the scale dwords of the next K step (a NaN scale there must not
+    reach a row that is stored)."""
+    ac, asc, bc, bsc = _operands(M, N_, K, E5M2, E4M3, seed=M)
+    got = N.mx_gemm_nt(ac.cuda(), _kstep(asc).cuda(), bc.cuda(), _kstep(bsc).cuda(), E5M2, E4M3, out_dtype=torch.float32).cpu()
+    _assert_within_hardware_sum(got, ac, asc, bc, bsc, E5M2, E4M3)
+    asc[: M % 128 or 128] = 255                          # what follows the last row in the array
+    got2 = N.mx_gemm_nt(ac.cuda(), _kstep(asc).cuda(), bc.cuda(), _kstep(bsc).cuda(), E5M2, E4M3, out_dtype=torch.float32).cpu()
+    keep = slice(M % 128 or 128, None)
+    assert torch.equal(got[keep], got2[keep]) and got2[: M % 128 or 128].isnan().all()
+
+
+@pytest.mark.parametrize("tokens", [32, 160, 544])
+def test_mx_linear_at_token_counts_without_whole_k_steps(N, tokens):
+    """Forward and both gradients equal those of the same codes multiplied without padding (the plain kernel for the weight
+    gradient), up to the order of fp32 sums: 2e-5 of the largest entry at these lengths."""
+    from optimus_dl_amd.modules.amp import create_fp8_recipe
+    from optimus_dl_amd.modules.fp8_linear import FP8Linear
+
+    lin = FP8Linear.from_linear(torch.nn.Linear(256, 384, bias=False).cuda())
+    x = seeded_bf16((tokens, 256), 1.0, 5).cuda().requires_grad_(True)
+    dy = seeded_bf16((tokens, 384), 1e-3, 6).cuda()
+    recipe = create_fp8_recipe("mxfp8", "hybrid")
+    with recipe.autocast(), torch.autocast("cuda", dtype=torch.bfloat16):
+        y = lin(x)
+    with recipe.backward():
+        y.backward(dy)
+    rule, layout = N.MX_CEIL, N.MX_ROWMAJOR
+    xq, xs, xt, xts = N.mx_cast(x.detach(), E4M3, True, True, layout=layout, scale_rule=rule)
+    wq, ws, wt, wts = N.mx_cast(lin.weight.detach(), E4M3, True, True, layout=layout, scale_rule=rule)
+    gq, gs, gt, gts = N.mx_cast(dy, E5M2, True, True, layout=layout, scale_rule=rule)
+    assert max_rel_err(lin.weight.grad.cpu(), N.mx_gemm_nt(gt, gts, xt, xts, E5M2, E4M3, out_dtype=torch.float32).cpu()) <= 2e-5
+    for got, want in ((y, N.mx_gemm_nt(xq, xs, wq, ws, E4M3, E4M3)), (x.grad, N.mx_gemm_nt(gq, gs, wt, wts, E5M2, E4M3))):
+        assert max_rel_err(got.detach().float().cpu(), want.float().cpu()) <= 2.0 ** -7
