@@ -122,6 +122,36 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
     return v;
 }
 
+// A lane's value against that of another lane of its row of 16 (a DPP control word): no LDS crossbar.
+template <int CTRL>
+__device__ __forceinline__ uint32_t max_with_dpp(uint32_t m) {
+    return max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ __forceinline__ uint32_t max_u16x2_with_dpp(uint32_t m) {
+    return max_u16x2(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, CTRL, 0xf, 0xf, false));
+}
+
+// Max over each half of a wave (32 lanes), in every lane; PAIRS: of two 16-bit values per lane.
+template <bool PAIRS>
+__device__ __forceinline__ uint32_t half_wave_max(uint32_t m) {
+    if constexpr (PAIRS) {
+        m = max_u16x2_with_dpp<0xB1>(m);          // lane ^ 1
+        m = max_u16x2_with_dpp<0x4E>(m);          // lane ^ 2
+        m = max_u16x2_with_dpp<0x141>(m);         // the other quad of 8 lanes
+        m = max_u16x2_with_dpp<0x140>(m);         // the other half of 16 lanes
+        const auto r = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+        return max_u16x2(r[0], r[1]);
+    } else {
+        m = max_with_dpp<0xB1>(m);
+        m = max_with_dpp<0x4E>(m);
+        m = max_with_dpp<0x141>(m);
+        m = max_with_dpp<0x140>(m);
+        const auto r = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+        return max(r[0], r[1]);
+    }
+}
+
 // Block-wide max of fp32 magnitude bits; result valid in thread 0.
 // `red` is LDS scratch with one slot per wave.
 __device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t *red) {

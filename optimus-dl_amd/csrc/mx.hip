@@ -64,10 +64,6 @@ __device__ __forceinline__ void mx_scale_of(uint32_t amax_bits, int rule, uint32
 // Maxima across lanes without the LDS crossbar: DPP inside a row of 16 lanes, and the two swap instructions of gfx950
 // (v_permlane16_swap exchanges the odd rows of one register with the even rows of another, v_permlane32_swap the wave's
 // halves: applied to two copies of a value they leave "mine" in one and "my partner's" in the other).
-template <int CTRL>
-__device__ __forceinline__ uint32_t max_with_dpp(uint32_t m) {
-    return max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, CTRL, 0xf, 0xf, false));
-}
 // over the 4 lanes l ^ {0, 1, 2, 3}
 __device__ __forceinline__ uint32_t max_quad(uint32_t m) {
     m = max_with_dpp<0xB1>(m);            // quad_perm [1, 0, 3, 2]

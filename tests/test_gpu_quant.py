@@ -518,3 +518,21 @@ def test_padded_cast_transpose_is_the_plain_one_with_zero_codes_behind(N, rows, 
     if rows:
         with pytest.raises(N.NativeError):
             N.cast_transpose(x, scale, O.E5M2, mode, rows_out=rows - 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols", [(16, 8), (16, 264), (48, 136), (80, 1000), (1040, 520)])
+def test_row_and_column_maxima_of_one_pass(N, dtype, rows, cols):
+    """Every row and column has its maximum at its own place; one row and one column of zeros, one infinity and one NaN (which
+    sorts above it)."""
+    x = seeded_bf16((rows, cols), 1.0, rows * cols)
+    x[3] = 0
+    x[:, 5] = 0
+    x[7, 1], x[9, 2] = float("inf"), float("nan")
+    x = x.to(dtype)
+    _, _, _, _, row, col = N.quantize_rowcol(x.cuda(), O.E4M3)
+    want = x.float().abs()
+    for got, dim in ((row, 1), (col, 0)):
+        ref = want.nan_to_num(nan=0.0).amax(dim)
+        nan = want.isnan().any(dim)
+        assert torch.equal(got.cpu().isnan(), nan) and torch.equal(got.cpu()[~nan], ref[~nan])
