@@ -1,4 +1,5 @@
-"""Compiles the HIP sources under csrc/ into one C-ABI shared library for gfx950.
+"""Compiles the HIP sources under csrc/ into one C-ABI shared library for gfx950, and the host side of its Python
+wrappers (csrc/host.cpp) into an extension module.
 
 Run as ``python -m optimus_dl_amd.build`` (or call :func:`build`).  The library
 lands beside this file as ``libodl_fp8.so``; it is built in-tree so that it
@@ -13,11 +14,14 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libodl_fp8.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
+HOST_NAME = "_host"
+HOST_PATH = os.path.join(HERE, HOST_NAME + ".so")
 SOURCES = ["api.hip", "quant.hip", "gemm_fp8.hip", "gemm_tiled.hip", "gemm_thin.hip", "gemm_deep.hip", "gemm_pipe.hip", "gemm_stream.hip", "fused.hip", "mx.hip"]
 
 # Per-source additions.  The compiler-scheduled tiled GEMMs: left to its own choice the compiler computes in vector
@@ -123,9 +127,22 @@ def check_saturating_conversions(asm_text: str, name: str = "") -> list[str]:
     return problems
 
 
+def host_command() -> list[str]:
+    """The command that compiles csrc/host.cpp against the installed torch."""
+    import torch
+    from torch.utils import cpp_extension
+
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-DTORCH_EXTENSION_NAME=" + HOST_NAME,
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+            *["-isystem" + p for p in cpp_extension.include_paths()], "-isystem" + sysconfig.get_paths()["include"],
+            os.path.join(CSRC, "host.cpp"), "-o", HOST_PATH + ".tmp",
+            *["-L" + p for p in cpp_extension.library_paths()], "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
+
+
 def build(verbose: bool = False, keep_asm: bool = False) -> str:
     """Compile every source and link ``libodl_fp8.so``.  Always recompiles."""
     hipcc = hipcc_path()
+    host = subprocess.Popen(host_command(), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     objdir = os.path.join(HERE, "csrc", "_obj")
     os.makedirs(objdir, exist_ok=True)
     for stale in glob.glob(os.path.join(objdir, "*.s")):
@@ -163,6 +180,10 @@ def build(verbose: bool = False, keep_asm: bool = False) -> str:
     r = subprocess.run(link, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}")
+    out, _ = host.communicate()
+    if host.returncode != 0:
+        raise RuntimeError(f"g++ failed on host.cpp:\n{out}")
+    os.replace(HOST_PATH + ".tmp", HOST_PATH)
     os.replace(tmp, LIB_PATH)
     return LIB_PATH
 

@@ -56,8 +56,11 @@ def pop_recipe() -> int:
 
 
 def active_recipe() -> "FP8Recipe | None":
-    with _lock:
-        return _stack[-1] if _stack else None
+    # (asked several times per module call; one look at the end of a list needs no lock)
+    try:
+        return _stack[-1]
+    except IndexError:
+        return None
 
 
 def is_fp8_active() -> bool:

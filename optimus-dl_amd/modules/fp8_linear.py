@@ -560,7 +560,7 @@ def linear_group(x: torch.Tensor, modules: "tuple[FP8Linear, ...]") -> tuple[tor
         x2d = _converted_input(recipe, x2d, compute_dtype)
     params: list = []
     for m in modules:
-        m.fp8_calls += 1
+        m.__dict__["fp8_calls"] += 1
         m._note_grad_mode()
         params += [m.weight, m.bias]
     outs = apply(_Fp8LinearGroupFn, x2d, recipe, compute_dtype, tuple(modules), *params)
@@ -840,7 +840,7 @@ class FP8Linear(nn.Linear):
         x2d = x.reshape(-1, self.in_features)
         if x2d.dtype != compute_dtype or not x2d.is_contiguous():
             x2d = _converted_input(recipe, x2d, compute_dtype)
-        self.fp8_calls += 1
+        self.__dict__["fp8_calls"] += 1      # (nn.Module.__setattr__ costs a microsecond)
         self._note_grad_mode()
         y = apply(_Fp8LinearFn, x2d, self.weight, self.bias, self, recipe, compute_dtype)
         return y.reshape(*x.shape[:-1], self.out_features)

@@ -12,6 +12,7 @@ synchronises with the host.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 
@@ -25,6 +26,7 @@ AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
 ABI_VERSION = 19
+_OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -81,6 +83,9 @@ EXPORTS = (
     "odl_fp8_mx_gemm_splitk",
 )
 
+# csrc/host.cpp: the plain case of the wrappers below (see there); None until the library is loaded
+HOST_NAME = "_host"
+_host = None
 _lib = None
 _lock = threading.Lock()
 
@@ -162,8 +167,33 @@ def load() -> ctypes.CDLL:
             getattr(L, name)  # AttributeError here = the library does not match the header
         if L.odl_fp8_abi_version() != ABI_VERSION:
             raise NativeError(f"{LIB_PATH}: ABI {L.odl_fp8_abi_version()} != expected {ABI_VERSION}; rebuild")
+        _load_host(L)
         _lib = L
     return _lib
+
+
+def _load_host(L: ctypes.CDLL) -> None:
+    """The C++ side of the wrappers (built beside the library), bound to the entries of the library that was loaded."""
+    global _host
+    path = os.path.join(_HERE, HOST_NAME + ".so")
+    if not os.path.exists(path):
+        raise NativeError(f"{path} is missing: build it with `python -m optimus_dl_amd.build`")
+    spec = importlib.util.spec_from_file_location(HOST_NAME, path)
+    host = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(host)
+    host.bind({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in EXPORTS})
+    _host = host
+
+
+def _done(r, what: str):
+    """What the C++ side answered: a result, or the status of an entry that refused."""
+    if r.__class__ is int:
+        _check(r, what)
+    return r
+
+
+def _may_split() -> bool:
+    return split_k and getattr(_tls, "forced_variant", -1) < 0
 
 
 _devices_ready: set[int] = set()
@@ -283,6 +313,10 @@ def amax_parts(x: torch.Tensor) -> torch.Tensor:
     """AMAX_PARTS partial maxima of |x| (no atomics); input of :func:`cast_dynamic`.  The kernel
     writes every entry, so the buffer is a fresh allocation per call: callers on several threads
     cannot get each other's partials."""
+    load()
+    r = _host.amax_parts(x, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_amax_parts")
     x = _as_2d(x)
     rows, cols = x.shape
     parts = torch.empty(AMAX_PARTS, dtype=torch.float32, device=x.device)
@@ -303,6 +337,10 @@ def colsum_supported(x: torch.Tensor) -> bool:
 
 def amax_parts_colsum(x: torch.Tensor):
     """Partial maxima of |x| and the fp32 column sums of x in one pass.  -> (parts, colsum[cols])."""
+    load()
+    r = _host.amax_colsum(x, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_amax_parts_colsum")
     x = _as_2d(x)
     rows, cols = x.shape
     parts = torch.empty(AMAX_PARTS, dtype=torch.float32, device=x.device)
@@ -332,6 +370,10 @@ def cast_dynamic(x: torch.Tensor, parts: torch.Tensor, fmt: int, margin: int = 0
     several tensors); implies want_transposed.  rows_out: the codes get that many rows (q [rows_out, cols], q_t
     [cols, rows_out]), zero codes behind those of x (see :func:`padded_rows`).
     -> (q or None, q_t or None, amax, scale, scale_inv); the last three are fp32[1]."""
+    load()
+    r = _host.cast_dynamic(x, parts, fmt, margin, want_rowmajor, want_transposed, out_t, rows_out, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_cast_dynamic")
     want_transposed = want_transposed or out_t is not None
     if not (want_rowmajor or want_transposed):
         raise NativeError("cast_dynamic: nothing to produce")
@@ -488,6 +530,10 @@ def _bf16_dense(t: torch.Tensor, what: str) -> torch.Tensor:
 def swiglu_amax_parts(gate: torch.Tensor, up: torch.Tensor):
     """h = silu(gate) * up as eager bf16 arithmetic leaves it, and the partial maxima of |h| for
     :func:`cast_dynamic`.  -> (h, parts)."""
+    load()
+    r = _host.swiglu(gate, up, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_swiglu_amax_parts")
     gate, up = _bf16_dense(gate, "swiglu gate"), _bf16_dense(up, "swiglu up")
     if gate.shape != up.shape:
         raise NativeError(f"swiglu: gate {tuple(gate.shape)} and up {tuple(up.shape)} differ")
@@ -503,6 +549,10 @@ def swiglu_amax_parts(gate: torch.Tensor, up: torch.Tensor):
 def swiglu_bwd_amax_parts(dh: torch.Tensor, gate: torch.Tensor, up: torch.Tensor):
     """Gradients of silu(gate) * up for grad_output dh, with their partial maxima.
     -> (d_gate, d_up, parts_d_gate, parts_d_up)."""
+    load()
+    r = _host.swiglu_bwd(dh, gate, up, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_swiglu_bwd_amax_parts")
     dh, gate, up = _bf16_dense(dh, "swiglu dh"), _bf16_dense(gate, "swiglu gate"), _bf16_dense(up, "swiglu up")
     if not (dh.shape == gate.shape == up.shape):
         raise NativeError(f"swiglu backward: shapes {tuple(dh.shape)}, {tuple(gate.shape)}, {tuple(up.shape)} differ")
@@ -520,6 +570,10 @@ def swiglu_bwd_amax_parts(dh: torch.Tensor, gate: torch.Tensor, up: torch.Tensor
 def rmsnorm_amax_parts(x: torch.Tensor, weight: torch.Tensor, eps: float):
     """y = bf16(x * rsqrt(mean(x^2, -1) + eps) * weight) over the last axis, the per-row
     1/rms, and the partial maxima of |y|.  x: bf16 or fp32.  -> (y bf16, rstd fp32, parts)."""
+    load()
+    r = _host.rmsnorm(x, weight, eps, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_rmsnorm_amax_parts")
     if not x.is_cuda:
         raise NativeError(f"rmsnorm: the kernels run on the GPU only; got a tensor on {x.device}")
     src = _src_dtype(x)
@@ -541,6 +595,10 @@ RMSNORM_BWD_SLABS = 512
 def rmsnorm_bwd(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, rstd: torch.Tensor):
     """Gradients of :func:`rmsnorm_amax_parts`'s y for grad_output dy (bf16).
     -> (dx in the dtype of x, d_weight fp32[cols])."""
+    load()
+    r = _host.rmsnorm_bwd(dy, x, weight, rstd, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_rmsnorm_bwd")
     dy = _bf16_dense(dy, "rmsnorm dy")
     src = _src_dtype(x)
     x = _dense_16(x)
@@ -585,6 +643,10 @@ def _dense_16(x: torch.Tensor) -> torch.Tensor:
 def layernorm_amax_parts(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, eps: float):
     """y = bf16(layer_norm(x) * weight + bias) over the last axis, per-row mean and 1/std, and the
     partial maxima of |y|.  x: bf16 or fp32.  -> (y bf16, mean fp32, rstd fp32, parts)."""
+    load()
+    r = _host.layernorm(x, weight, bias, eps, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_layernorm_amax_parts")
     if not x.is_cuda:
         raise NativeError(f"layernorm: the kernels run on the GPU only; got a tensor on {x.device}")
     src = _src_dtype(x)
@@ -605,6 +667,10 @@ def layernorm_amax_parts(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tens
 def layernorm_bwd(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, mean: torch.Tensor, rstd: torch.Tensor):
     """Gradients of :func:`layernorm_amax_parts`'s y for grad_output dy (bf16).
     -> (dx in the dtype of x, d_weight fp32[cols], d_bias fp32[cols])."""
+    load()
+    r = _host.layernorm_bwd(dy, x, weight, mean, rstd, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_layernorm_bwd")
     dy = _bf16_dense(dy, "layernorm dy")
     src = _src_dtype(x)
     x = _dense_16(x)
@@ -647,6 +713,11 @@ def gelu_table(device: torch.device) -> torch.Tensor:
 
 def gelu_amax_parts(x: torch.Tensor):
     """Exact GELU of a bf16 tensor and the partial maxima of the result.  -> (y, parts)."""
+    if x.is_cuda:
+        load()
+        r = _host.gelu(x, gelu_table(x.device), _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_gelu_amax_parts")
     x = _bf16_dense(x, "gelu x")
     cols = x.shape[-1] if x.dim() else 1
     rows = x.numel() // max(cols, 1)
@@ -659,6 +730,11 @@ def gelu_amax_parts(x: torch.Tensor):
 
 def gelu_bwd_amax_parts(dy: torch.Tensor, x: torch.Tensor):
     """dx = dy * gelu'(x) in bf16 and its partial maxima.  -> (dx, parts)."""
+    if x.is_cuda:
+        load()
+        r = _host.gelu_bwd(dy, x, gelu_table(x.device), _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_gelu_bwd_amax_parts")
     dy, x = _bf16_dense(dy, "gelu dy"), _bf16_dense(x, "gelu x")
     if dy.shape != x.shape:
         raise NativeError(f"gelu backward: dy {tuple(dy.shape)} and x {tuple(x.shape)} differ")
@@ -675,6 +751,10 @@ def quantize_rowcol(x: torch.Tensor, fmt: int, margin: int = 0, rows_out: int | 
     """Rowwise recipe, both operands of one tensor in two passes over it:
     -> (q [rows, cols] scaled per row, s_row_inv [rows], q_t [cols, rows] scaled per column, s_col_inv [cols],
         amax_row, amax_col).  rows_out: as in :func:`cast_dynamic`."""
+    load()
+    r = _host.quantize_rowcol(x, fmt, margin, rows_out, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_amax_rowcol / odl_fp8_cast_rowcol")
     x = _as_2d(x)
     rows, cols = x.shape
     pr, pc = -(-rows // 4) * 4, -(-cols // 4) * 4            # every vector starts on a 16-byte boundary (the GEMM wants that)
@@ -747,6 +827,10 @@ def cast_delayed(x: torch.Tensor, scale: torch.Tensor, fmt: int, amax_parts: tor
     recorded), and 1/scale in a fresh 1-element tensor that later refreshes of ``scale`` do not touch.  out_t, rows_out:
     as in :func:`cast_dynamic`.
     -> (codes or None, codes_t or None, scale_inv[1])."""
+    load()
+    r = _host.cast_delayed(x, scale, fmt, amax_parts, want_rowmajor, want_transposed, out_t, rows_out, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_cast_delayed")
     x = _as_2d(x)
     rows, cols = x.shape
     _f32_dev(scale, 1, "cast_delayed scale")
@@ -775,6 +859,12 @@ def gemm_nt(a: torch.Tensor, b: torch.Tensor, fmt_a: int, fmt_b: int, sa_inv: to
             out: torch.Tensor | None = None, accumulate: bool = False) -> torch.Tensor:
     """out[M,N] = (a[M,K] . b[N,K]^T) * (sa_inv x sb_inv) (+ bias); a, b uint8 FP8 codes.  A given ``out`` decides the
     output type.  accumulate: out = out + product (needs ``out``; the old value joins the fp32 sum, one rounding)."""
+    load()
+    odt = _OUT_DTYPES.get(out_dtype, -1)
+    if odt >= 0:
+        r = _host.gemm_nt(a, b, fmt_a, fmt_b, sa_inv, sb_inv, bias, odt, out, accumulate, _may_split(), _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_gemm_nt")
     if accumulate and out is None:
         raise NativeError("gemm_nt(accumulate=True) needs the `out` tensor to add into")
     if out is not None:
@@ -875,6 +965,11 @@ def mx_cast(x: torch.Tensor, fmt: int, want_rowmajor: bool = True, want_transpos
     blocked axis allows it).  scale_rule: MX_FLOOR (the OCP formula; a block amax in the top eighth of its binade
     saturates) or MX_CEIL (the exponent rounded up: nothing saturates).  rows_out: the transposed codes and their scales are
     that many rows of x long, zero codes with scale byte 0 behind those of x (see :func:`padded_rows`)."""
+    load()
+    if layout is None:
+        r = _host.mx_cast(x, fmt, want_rowmajor, want_transposed, int(scale_rule), rows_out, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_mx_cast")
     x = _as_2d(x)
     rows, cols = x.shape
     if not (want_rowmajor or want_transposed):
@@ -905,6 +1000,10 @@ def block_cast(x: torch.Tensor, fmt: int, margin: int = 0, two_d: bool = False, 
     per 128 x 128 block (two_d True, weights).  -> (codes [rows, cols], scales [cols/128, rows, 4], codes_t [cols, rows],
     scales_t [rows/128, cols, 4]); the scale tensors hold E8M0 bytes in the K-step-major layout, each block's byte four
     times, and go to ``mx_gemm_nt`` as they are.  The pair that was not asked for is (None, None)."""
+    load()
+    r = _host.block_cast(x, fmt, margin, two_d, want_rowmajor, want_transposed, _stream())
+    if r is not None:
+        return _done(r, "odl_fp8_block_cast")
     x = _as_2d(x)
     rows, cols = x.shape
     if not (want_rowmajor or want_transposed):
@@ -931,6 +1030,14 @@ def mx_gemm_nt(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Ten
     """out[M,N] = sum over 32-blocks of 2^(sa-127) 2^(sb-127) (a_block . b_block) (+ bias); a [M,K], b [N,K] codes,
     sa, sb their E8M0 scale bytes as ``mx_cast`` returns them (both row-major [rows, K/32] or both K-step-major
     [K/128, rows, 4])."""
+    load()
+    if a.is_cuda:
+        init_device(a.device)
+    odt = _OUT_DTYPES.get(out_dtype, -1)
+    if odt >= 0:
+        r = _host.mx_gemm_nt(a, sa, b, sb, fmt_a, fmt_b, bias, odt, out, accumulate, _may_split(), _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_mx_gemm_nt")
     for t, what in ((a, "a"), (b, "b"), (sa, "sa"), (sb, "sb")):
         if t.dtype != torch.uint8 or not t.is_cuda or not t.is_contiguous():
             raise NativeError(f"mx_gemm_nt: {what} must be a dense uint8 device tensor")
@@ -1071,6 +1178,12 @@ def gemm_layouts(a: torch.Tensor, b: torch.Tensor, fmt_a: int, fmt_b: int, layou
     ``out`` decides the output type, else ``out_dtype`` does.  accumulate: out = out + product (needs ``out``); the
     product then passes through an fp32 workspace (``odl_fp8_gemm_splitk``, with one run where K is not worth cutting),
     because the kernel that reads K-slow operands stores a tile where nothing can wait for the old values."""
+    load()
+    odt = _OUT_DTYPES.get(out_dtype, -1)
+    if odt >= 0 and not accumulate:
+        r = _host.gemm_layouts(a, b, fmt_a, fmt_b, layout_a == K_SLOW, layout_b == K_SLOW, sa_inv, sb_inv, out, odt, _may_split(), _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_gemm_layouts")
     if accumulate and out is None:
         raise NativeError("gemm_layouts(accumulate=True) needs the `out` tensor to add into")
     if a.dtype != torch.uint8 or b.dtype != torch.uint8:
