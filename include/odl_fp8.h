@@ -532,6 +532,25 @@ int odl_fp8_mx_cast_padded(const void *x, int src_dtype, int64_t rows, int64_t c
                            uint8_t *scales, int scales_layout, uint8_t *out_t, uint8_t *scales_t, int scales_t_layout,
                            int scale_rule, odl_stream_t stream);
 
+/* h = silu(gate) * up (the arithmetic of odl_fp8_swiglu_amax_parts, rounded to bf16 as there) and its codes, and d_gate and d_up of
+ * odl_fp8_swiglu_bwd_amax_parts and theirs, in one pass: the bf16 tensors in between are never written.  Codes and scales
+ * are bit for bit those of the producer followed by the cast.  rows > 0 does something, cols > 0 too.
+ *   _mx_cast       odl_fp8_mx_cast_padded with both layouts and K-step-major scales (rows % 32 == 0, cols and rows_out % 128 == 0;
+ *                  every pointer 16-byte aligned)
+ *   _cast_delayed  odl_fp8_cast_delayed_padded (cols % 8 == 0, rows_out % 16 == 0); amax_parts and scale_inv are required; the
+ *                  transposed codes of both tensors may be NULL together */
+int odl_fp8_swiglu_mx_cast(const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out, int fmt, uint8_t *out,
+                           uint8_t *scales, uint8_t *out_t, uint8_t *scales_t, int scale_rule, odl_stream_t stream);
+int odl_fp8_swiglu_bwd_mx_cast(const void *dh, const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out,
+                               int fmt, uint8_t *dg, uint8_t *dg_scales, uint8_t *dg_t, uint8_t *dg_scales_t, uint8_t *du,
+                               uint8_t *du_scales, uint8_t *du_t, uint8_t *du_scales_t, int scale_rule, odl_stream_t stream);
+int odl_fp8_swiglu_cast_delayed(const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out, const float *scale,
+                                int fmt, uint8_t *out, uint8_t *out_t, float *amax_parts, float *scale_inv, odl_stream_t stream);
+int odl_fp8_swiglu_bwd_cast_delayed(const void *dh, const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out,
+                                    int fmt, const float *scale_g, uint8_t *dg, uint8_t *dg_t, float *parts_g, float *inv_g,
+                                    const float *scale_u, uint8_t *du, uint8_t *du_t, float *parts_u, float *inv_u,
+                                    odl_stream_t stream);
+
 /*
  * C[M, N] = sum over blocks kb of 2^(sa[m, kb] - 127) * 2^(sb[n, kb] - 127) * dot(A[m, 32 kb .. +32], B[n, 32 kb .. +32])
  * (+ bias[n]), accumulated in fp32 by the scaled MFMA (V_MFMA_SCALE_F32_32X32X64_F8F6F4 applies the two block scales to

@@ -8,7 +8,7 @@
 // a plain-C restatement gives the same bits: fused multiply-adds are spelled out, nothing is left
 // to contraction, no hardware approximation (v_exp_f32, v_rcp_f32, v_rsq_f32) is used.  Sums over
 // rows (d_weight, column sums) are fp32 partial sums in a fixed order.
-#include "common.h"
+#include "swiglu.h"
 
 #pragma clang fp contract(off)
 
@@ -16,61 +16,6 @@ namespace odl {
 
 constexpr int kFusedThreads = 1024;
 constexpr int kParts = ODL_FP8_AMAX_PARTS;
-
-// 1 / d for 1 <= d < 2^120: integer first guess, three Newton steps in fused multiply-adds.
-__device__ __forceinline__ float recip_newton(float d) {
-    float y = bits_to_float(0x7EF311C7u - float_to_bits(d));
-    y = __fmaf_rn(y, __fmaf_rn(-d, y, 1.0f), y);
-    y = __fmaf_rn(y, __fmaf_rn(-d, y, 1.0f), y);
-    y = __fmaf_rn(y, __fmaf_rn(-d, y, 1.0f), y);
-    return y;
-}
-
-// logistic function 1 / (1 + exp(-g)): range reduction by ln 2 in two pieces, degree-5 polynomial
-// for (exp(r) - 1 - r) / r^2, exact scaling by 2^k, reciprocal as above.  A NaN argument is
-// evaluated as 0 here (every use below multiplies by the argument again, which restores the NaN).
-__device__ __forceinline__ float sigmoid_det(float g) {
-    float t = (g != g) ? 0.0f : -g;
-    const bool zero = t > 80.0f;                 // exp(-g) beyond 2^115: the quotient is taken as 0
-    t = __builtin_amdgcn_fmed3f(t, -80.0f, 80.0f);
-    const float kf = __builtin_rintf(__fmul_rn(t, 1.44269504f));
-    float r = __fmaf_rn(kf, -0.693359375f, t);
-    r = __fmaf_rn(kf, 2.12194440e-4f, r);
-    float p = 1.9875691500e-4f;
-    p = __fmaf_rn(p, r, 1.3981999507e-3f);
-    p = __fmaf_rn(p, r, 8.3334519073e-3f);
-    p = __fmaf_rn(p, r, 4.1665795894e-2f);
-    p = __fmaf_rn(p, r, 1.6666665459e-1f);
-    p = __fmaf_rn(p, r, 5.0000001201e-1f);
-    const float z = __fmul_rn(r, r);
-    const float y = __fadd_rn(__fmaf_rn(p, z, r), 1.0f);
-    const float e = __fmul_rn(y, bits_to_float((uint32_t)((int)kf + 127) << 23));
-    const float s = recip_newton(__fadd_rn(1.0f, e));
-    return zero ? 0.0f : s;
-}
-
-// Roundings to bf16 use the hardware's round-to-nearest-even conversion of a pair (subnormal
-// results are kept: the kernels run with fp32 denormals enabled).
-
-// h = bf16( bf16(g * sigmoid(g)) * u ), the two roundings of silu(gate) * up evaluated in bf16, for
-// the two elements of a packed pair
-__device__ __forceinline__ uint32_t swiglu_fwd_pair(uint32_t gw, uint32_t uw) {
-    const float g0 = bf16_lo(gw), g1 = bf16_hi(gw);
-    const uint32_t s = pack_bf16x2(__fmul_rn(g0, sigmoid_det(g0)), __fmul_rn(g1, sigmoid_det(g1)));
-    return pack_bf16x2(__fmul_rn(bf16_lo(s), bf16_lo(uw)), __fmul_rn(bf16_hi(s), bf16_hi(uw)));
-}
-
-// d_up = bf16(dh * s), d_gate = bf16( bf16(dh * u) * (sig * (1 + g * (1 - sig))) ), s = bf16(g * sig)
-__device__ __forceinline__ void swiglu_bwd_pair(uint32_t dw, uint32_t gw, uint32_t uw, uint32_t &dg, uint32_t &du) {
-    const float g0 = bf16_lo(gw), g1 = bf16_hi(gw), d0 = bf16_lo(dw), d1 = bf16_hi(dw);
-    const float sig0 = sigmoid_det(g0), sig1 = sigmoid_det(g1);
-    const uint32_t s = pack_bf16x2(__fmul_rn(g0, sig0), __fmul_rn(g1, sig1));
-    du = pack_bf16x2(__fmul_rn(d0, bf16_lo(s)), __fmul_rn(d1, bf16_hi(s)));
-    const uint32_t ds = pack_bf16x2(__fmul_rn(d0, bf16_lo(uw)), __fmul_rn(d1, bf16_hi(uw)));
-    const float ds0 = __fmul_rn(sig0, __fmaf_rn(g0, __fsub_rn(1.0f, sig0), 1.0f));
-    const float ds1 = __fmul_rn(sig1, __fmaf_rn(g1, __fsub_rn(1.0f, sig1), 1.0f));
-    dg = pack_bf16x2(__fmul_rn(bf16_lo(ds), ds0), __fmul_rn(bf16_hi(ds), ds1));
-}
 
 __device__ __forceinline__ uint32_t pack2(float a, float b) { return pack_bf16x2(a, b); }
 

@@ -25,9 +25,12 @@
 // that hold Inf / NaN are converted step by step.
 #include <hip/hip_runtime.h>
 
+#include <initializer_list>
+
 #include "common.h"
 #include "ct_tile.h"
 #include "gemm_common.h"
+#include "swiglu.h"
 
 namespace odl {
 
@@ -134,47 +137,32 @@ __device__ __forceinline__ uint32_t cvt_scaled4(uint32_t p0, uint32_t p1, uint32
 // the rows (32 of them) is held by the 8 lanes of a wave that share tx.  All maxima are exchanges inside the wave.
 // The transposed codes are rows_t >= rows long: zero codes with scale byte 0 behind those of x, so that a GEMM that contracts
 // the rows finds whole K steps.
-template <int SRC, int FMT, bool WANT_ROW, bool WANT_COL>
-__global__ __launch_bounds__(kMxThreads) void mx_cast_kernel(const void *__restrict__ x, int64_t rows, int64_t cols,
-                                                              uint8_t *__restrict__ out, uint8_t *__restrict__ scales,
-                                                              uint8_t *__restrict__ out_t, uint8_t *__restrict__ scales_t,
-                                                              int layout, int layout_t, int rule, int64_t rows_t) {
-    __shared__ __attribute__((aligned(16))) uint8_t tile[kTileC * kTileR];
+// What a lane knows of its tile, and the tile's LDS.
+struct MxShared {
+    __attribute__((aligned(16))) uint8_t tile[kTileC * kTileR];
     // K-step-major scale bytes leave the block as whole runs: the tile's 4 row blocks are one dword per column (256
     // contiguous bytes per tile), its 2 column blocks one 16-bit half of a dword per row.  Stored a byte at a time from
     // the lanes that hold them they were hundreds of masked one-byte writes per tile and cost a tenth of the kernel.
-    __shared__ __attribute__((aligned(16))) uint8_t stage_t[kTileC * 4];
-    __shared__ __attribute__((aligned(16))) uint8_t stage_r[kTileR * 2];
-    saturate_fp8_conversions();
-    constexpr int ESZ = SRC == ODL_BF16 ? 2 : 4;
+    __attribute__((aligned(16))) uint8_t stage_t[kTileC * 4];
+    __attribute__((aligned(16))) uint8_t stage_r[kTileR * 2];
+};
+
+// One tile of which every lane holds its 4 x 8 patch as loaded (bf16: 4 dwords a row; it is widened row by row where it is
+// used, and magnitudes of bf16 pairs are compared as packed 16-bit integers, two columns at a time).
+template <int SRC, int FMT, bool WANT_ROW, bool WANT_COL>
+__device__ __forceinline__ void mx_cast_tile(const uint32_t (&raw)[4][SRC == ODL_BF16 ? 4 : 8], int64_t tr, int64_t tc, int64_t rows, int64_t cols,
+                                             uint8_t *__restrict__ out, uint8_t *__restrict__ scales, uint8_t *__restrict__ out_t,
+                                             uint8_t *__restrict__ scales_t, int layout, int layout_t, int rule, int64_t rows_t, MxShared &lds) {
+    uint8_t *tile = lds.tile, *stage_t = lds.stage_t, *stage_r = lds.stage_r;
     const int tx = threadIdx.x % 8, ty = threadIdx.x / 8;
-    const int64_t tiles_r = ((WANT_COL ? rows_t : rows) + kTileR - 1) / kTileR, tiles_c = (cols + kTileC - 1) / kTileC;
     // (K-step-major implies whole dwords: cols % 128 == 0 for `scales`, rows_t % 128 == 0 for `scales_t`; host-checked)
     const bool staged_r = WANT_ROW && WANT_COL && layout == ODL_MX_SCALES_KSTEP;
     const bool staged_t = WANT_COL && layout_t == ODL_MX_SCALES_KSTEP;
-    int64_t tr, tc;
-    ct_tile_of(blockIdx.x, tiles_r, tiles_c, tr, tc);
     const int kA = SRC == ODL_BF16 ? tx * 8 : tx * 4, kB = SRC == ODL_BF16 ? tx * 8 + 4 : 32 + tx * 4;   // tile columns of the two groups
     const int64_t r0 = tr * kTileR + ty * 4, cA = tc * kTileC + kA, cB = tc * kTileC + kB;
     // cols % 32 == 0 where codes along the rows are wanted, % 8 otherwise (host-checked): a group of 4 is in or out as a whole
     const bool okA = cA < cols, okB = cB < cols;
     [[maybe_unused]] auto col_of = [&](int j) { return j < 4 ? cA + j : cB + j - 4; };      // matrix column of the lane's column j
-
-    // The patch stays in registers as loaded (bf16: 4 dwords a row) and is widened row by row where it is used; magnitudes
-    // of bf16 pairs are compared as packed 16-bit integers, two columns at a time.
-    constexpr int DW = SRC == ODL_BF16 ? 4 : 8;
-    uint32_t raw[4][DW];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const bool row_ok = (r0 + i) < rows;
-        const char *row = reinterpret_cast<const char *>(x) + (r0 + i) * cols * ESZ;
-#pragma unroll
-        for (int h = 0; h < DW / 4; ++h) {
-            const bool ok = row_ok && (h == 0 ? okA : okB);
-            const u32x4 v = ok ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(row + (h == 0 ? cA : cB) * ESZ)) : u32x4{0, 0, 0, 0};
-            raw[i][4 * h] = v.x; raw[i][4 * h + 1] = v.y; raw[i][4 * h + 2] = v.z; raw[i][4 * h + 3] = v.w;
-        }
-    }
     auto widen = [&](int i, float (&f)[8]) {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
@@ -340,6 +328,84 @@ __global__ __launch_bounds__(kMxThreads) void mx_cast_kernel(const void *__restr
                 reinterpret_cast<uint16_t *>(scales)[((tc >> 1) * rows + orow) * 2 + (tc & 1)] = reinterpret_cast<const uint16_t *>(stage_r)[r];
         }
     }
+}
+
+template <int SRC, int FMT, bool WANT_ROW, bool WANT_COL>
+__global__ __launch_bounds__(kMxThreads) void mx_cast_kernel(const void *__restrict__ x, int64_t rows, int64_t cols,
+                                                              uint8_t *__restrict__ out, uint8_t *__restrict__ scales,
+                                                              uint8_t *__restrict__ out_t, uint8_t *__restrict__ scales_t,
+                                                              int layout, int layout_t, int rule, int64_t rows_t) {
+    __shared__ MxShared lds;
+    saturate_fp8_conversions();
+    constexpr int ESZ = SRC == ODL_BF16 ? 2 : 4, DW = SRC == ODL_BF16 ? 4 : 8;
+    const int tx = threadIdx.x % 8, ty = threadIdx.x / 8;
+    const int64_t tiles_r = ((WANT_COL ? rows_t : rows) + kTileR - 1) / kTileR, tiles_c = (cols + kTileC - 1) / kTileC;
+    int64_t tr, tc;
+    ct_tile_of(blockIdx.x, tiles_r, tiles_c, tr, tc);
+    const int64_t r0 = tr * kTileR + ty * 4, cA = tc * kTileC + (SRC == ODL_BF16 ? tx * 8 : tx * 4), cB = tc * kTileC + (SRC == ODL_BF16 ? tx * 8 + 4 : 32 + tx * 4);
+    uint32_t raw[4][DW];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const bool row_ok = (r0 + i) < rows;
+        const char *row = reinterpret_cast<const char *>(x) + (r0 + i) * cols * ESZ;
+#pragma unroll
+        for (int h = 0; h < DW / 4; ++h) {
+            const bool ok = row_ok && (h == 0 ? cA < cols : cB < cols);
+            const u32x4 v = ok ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(row + (h == 0 ? cA : cB) * ESZ)) : u32x4{0, 0, 0, 0};
+            raw[i][4 * h] = v.x; raw[i][4 * h + 1] = v.y; raw[i][4 * h + 2] = v.z; raw[i][4 * h + 3] = v.w;
+        }
+    }
+    mx_cast_tile<SRC, FMT, WANT_ROW, WANT_COL>(raw, tr, tc, rows, cols, out, scales, out_t, scales_t, layout, layout_t, rule, rows_t, lds);
+}
+
+// The same of h = silu(gate) * up, and of d_gate and d_up, without the bf16 tensors in between: both layouts, K-step-major scales,
+// cols and rows_t multiples of 128.  HBM-bound: 4 + 2 (1 + 1/32) and 6 + 4 (1 + 1/32) bytes an element, where a producer
+// that writes bf16 and the casts that read it again move 10 and 18.
+struct MxOut { uint8_t *out, *scales, *out_t, *scales_t; };
+
+template <int FMT>
+__global__ __launch_bounds__(kMxThreads) void swiglu_mx_cast_kernel(const uint8_t *__restrict__ gate, const uint8_t *__restrict__ up, int64_t rows,
+                                                                     int64_t cols, MxOut h, int rule, int64_t rows_t) {
+    __shared__ MxShared lds;
+    saturate_fp8_conversions();
+    const int tx = threadIdx.x % 8, ty = threadIdx.x / 8;
+    int64_t tr, tc;
+    ct_tile_of(blockIdx.x, rows_t / kTileR, cols / kTileC, tr, tc);
+    uint32_t raw[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int64_t r = tr * kTileR + ty * 4 + i, at = (r * cols + tc * kTileC + tx * 8) * 2;
+        u32x4 v = {0, 0, 0, 0};
+        if (r < rows)
+            v = swiglu_fwd8(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(gate + at)), __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(up + at)));
+        raw[i][0] = v.x; raw[i][1] = v.y; raw[i][2] = v.z; raw[i][3] = v.w;
+    }
+    mx_cast_tile<ODL_BF16, FMT, true, true>(raw, tr, tc, rows, cols, h.out, h.scales, h.out_t, h.scales_t, ODL_MX_SCALES_KSTEP, ODL_MX_SCALES_KSTEP, rule, rows_t, lds);
+}
+
+template <int FMT>
+__global__ __launch_bounds__(kMxThreads) void swiglu_bwd_mx_cast_kernel(const uint8_t *__restrict__ dh, const uint8_t *__restrict__ gate,
+                                                                         const uint8_t *__restrict__ up, int64_t rows, int64_t cols, MxOut dg,
+                                                                         MxOut du, int rule, int64_t rows_t) {
+    __shared__ MxShared lds;
+    saturate_fp8_conversions();
+    const int tx = threadIdx.x % 8, ty = threadIdx.x / 8;
+    int64_t tr, tc;
+    ct_tile_of(blockIdx.x, rows_t / kTileR, cols / kTileC, tr, tc);
+    uint32_t rg[4][4], ru[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int64_t r = tr * kTileR + ty * 4 + i, at = (r * cols + tc * kTileC + tx * 8) * 2;
+        u32x4 g = {0, 0, 0, 0}, u = {0, 0, 0, 0};
+        if (r < rows)
+            swiglu_bwd8(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(dh + at)), __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(gate + at)),
+                        __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(up + at)), g, u);
+        rg[i][0] = g.x; rg[i][1] = g.y; rg[i][2] = g.z; rg[i][3] = g.w;
+        ru[i][0] = u.x; ru[i][1] = u.y; ru[i][2] = u.z; ru[i][3] = u.w;
+    }
+    mx_cast_tile<ODL_BF16, FMT, true, true>(rg, tr, tc, rows, cols, dg.out, dg.scales, dg.out_t, dg.scales_t, ODL_MX_SCALES_KSTEP, ODL_MX_SCALES_KSTEP, rule, rows_t, lds);
+    __syncthreads();                       // the tile's LDS is reused
+    mx_cast_tile<ODL_BF16, FMT, true, true>(ru, tr, tc, rows, cols, du.out, du.scales, du.out_t, du.scales_t, ODL_MX_SCALES_KSTEP, ODL_MX_SCALES_KSTEP, rule, rows_t, lds);
 }
 
 // ------------------------------------------------------------------ blockwise recipe
@@ -910,6 +976,49 @@ extern "C" int odl_fp8_mx_cast(const void *x, int src_dtype, int64_t rows, int64
                                int scales_layout, uint8_t *out_t, uint8_t *scales_t, int scales_t_layout, int scale_rule,
                                odl_stream_t stream_) {
     return odl_fp8_mx_cast_padded(x, src_dtype, rows, cols, rows, fmt, out, scales, scales_layout, out_t, scales_t, scales_t_layout, scale_rule, stream_);
+}
+
+static int check_swiglu_mx(const char *who, int64_t rows, int64_t cols, int64_t rows_out, int fmt, int rule, std::initializer_list<const void *> all) {
+    if (rows < 0 || cols < 0 || rows_out < rows) return set_error(ODL_ERR_ARG, "%s: shape %lld x %lld, rows_out %lld", who, (long long)rows, (long long)cols, (long long)rows_out);
+    if (fmt != ODL_FP8_E4M3 && fmt != ODL_FP8_E5M2) return set_error(ODL_ERR_ARG, "%s: fmt %d", who, fmt);
+    if (rule != ODL_MX_SCALE_FLOOR && rule != ODL_MX_SCALE_CEIL) return set_error(ODL_ERR_ARG, "%s: scale_rule %d", who, rule);
+    if (rows % kMxBlock != 0 || cols % 128 != 0 || rows_out % 128 != 0)
+        return set_error(ODL_ERR_SHAPE, "%s: %lld x %lld, rows_out %lld: rows must be a multiple of 32, cols and rows_out of 128", who, (long long)rows, (long long)cols, (long long)rows_out);
+    if ((rows_out / kTileR) * (cols / kTileC) > 0x7fffffffLL) return set_error(ODL_ERR_SHAPE, "%s: too many tiles for one launch", who);
+    if (rows == 0 || cols == 0) return ODL_OK;
+    for (const void *p : all) {
+        if (!p) return set_error(ODL_ERR_ARG, "%s: null pointer", who);
+        if (reinterpret_cast<uintptr_t>(p) & 15) return set_error(ODL_ERR_SHAPE, "%s: every pointer must be 16-byte aligned", who);
+    }
+    return ODL_OK;
+}
+
+extern "C" int odl_fp8_swiglu_mx_cast(const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out, int fmt, uint8_t *out,
+                                      uint8_t *scales, uint8_t *out_t, uint8_t *scales_t, int scale_rule, odl_stream_t stream_) {
+    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+    if (int e = check_swiglu_mx("odl_fp8_swiglu_mx_cast", rows, cols, rows_out, fmt, scale_rule, {gate, up, out, scales, out_t, scales_t})) return e;
+    if (rows == 0 || cols == 0) return ODL_OK;
+    const dim3 grid((unsigned)((rows_out / kTileR) * (cols / kTileC))), block(kMxThreads);
+    const uint8_t *g = static_cast<const uint8_t *>(gate), *u = static_cast<const uint8_t *>(up);
+    const MxOut h = {out, scales, out_t, scales_t};
+    if (fmt == ODL_FP8_E4M3) hipLaunchKernelGGL((swiglu_mx_cast_kernel<ODL_FP8_E4M3>), grid, block, 0, stream, g, u, rows, cols, h, scale_rule, rows_out);
+    else hipLaunchKernelGGL((swiglu_mx_cast_kernel<ODL_FP8_E5M2>), grid, block, 0, stream, g, u, rows, cols, h, scale_rule, rows_out);
+    return check_launch("odl_fp8_swiglu_mx_cast");
+}
+
+extern "C" int odl_fp8_swiglu_bwd_mx_cast(const void *dh, const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out, int fmt,
+                                          uint8_t *dg, uint8_t *dg_scales, uint8_t *dg_t, uint8_t *dg_scales_t, uint8_t *du, uint8_t *du_scales,
+                                          uint8_t *du_t, uint8_t *du_scales_t, int scale_rule, odl_stream_t stream_) {
+    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+    if (int e = check_swiglu_mx("odl_fp8_swiglu_bwd_mx_cast", rows, cols, rows_out, fmt, scale_rule,
+                                {dh, gate, up, dg, dg_scales, dg_t, dg_scales_t, du, du_scales, du_t, du_scales_t})) return e;
+    if (rows == 0 || cols == 0) return ODL_OK;
+    const dim3 grid((unsigned)((rows_out / kTileR) * (cols / kTileC))), block(kMxThreads);
+    const uint8_t *d = static_cast<const uint8_t *>(dh), *g = static_cast<const uint8_t *>(gate), *u = static_cast<const uint8_t *>(up);
+    const MxOut og = {dg, dg_scales, dg_t, dg_scales_t}, ou = {du, du_scales, du_t, du_scales_t};
+    if (fmt == ODL_FP8_E4M3) hipLaunchKernelGGL((swiglu_bwd_mx_cast_kernel<ODL_FP8_E4M3>), grid, block, 0, stream, d, g, u, rows, cols, og, ou, scale_rule, rows_out);
+    else hipLaunchKernelGGL((swiglu_bwd_mx_cast_kernel<ODL_FP8_E5M2>), grid, block, 0, stream, d, g, u, rows, cols, og, ou, scale_rule, rows_out);
+    return check_launch("odl_fp8_swiglu_bwd_mx_cast");
 }
 
 extern "C" int odl_fp8_mx_gemm_nt(const uint8_t *a, const uint8_t *sa, const uint8_t *b, const uint8_t *sb, int scales_layout, int64_t M,

@@ -9,6 +9,7 @@
 //     the tail is short.
 #include "common.h"
 #include "ct_tile.h"
+#include "swiglu.h"
 
 #include <float.h>
 
@@ -717,11 +718,11 @@ __device__ __forceinline__ void ct_store_row(uint8_t *__restrict__ out, int64_t 
     }
 }
 
-template <int SRC, int FMT, int MODE, bool AMAX, bool WRITE_ROWMAJOR>
-__device__ __forceinline__ void ct_one_tile(const void *__restrict__ x, int64_t rows, int64_t cols, int64_t rows_out, const float *__restrict__ scale,
-                                            float st, uint8_t *__restrict__ out, uint8_t *__restrict__ out_t, int64_t tr,
+// ... of which every lane holds its 4 x 8 patch.  WRITE_T: transposed codes are wanted.
+template <int SRC, int FMT, int MODE, bool AMAX, bool WRITE_ROWMAJOR, bool WRITE_T>
+__device__ __forceinline__ void ct_quantise_tile(const u32x4 (&raw)[4][SRC == ODL_BF16 ? 1 : 2], int64_t rows, int64_t cols, int64_t rows_out,
+                                            const float *__restrict__ scale, float st, uint8_t *__restrict__ out, uint8_t *__restrict__ out_t, int64_t tr,
                                             int64_t tc, uint8_t *tile, uint32_t &am) {
-    constexpr int ESZ = SRC == ODL_BF16 ? 2 : 4;
     const int tx = threadIdx.x % 8;                 // 8 lanes across 64 columns
     const int ty = threadIdx.x / 8;                 // 32 lane-rows, 4 rows each
     // tile columns of the lane's two groups of 4 (codes lo / hi below)
@@ -745,11 +746,6 @@ __device__ __forceinline__ void ct_one_tile(const void *__restrict__ x, int64_t 
             s_col[4] = t1.x; s_col[5] = t1.y; s_col[6] = t1.z; s_col[7] = t1.w;
         }
     }
-
-    // ---- load the 4 x 8 patch (rows beyond the matrix read as zero)
-    u32x4 raw[4][ESZ / 2];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ct_load_row<SRC>(x, r0 + i, rows, cols, cA, cB, okA, okB, raw[i]);
 
     uint32_t lo[4], hi[4];                          // codes of columns 0..3 / 4..7 for each of the 4 rows
 #pragma unroll
@@ -785,6 +781,7 @@ __device__ __forceinline__ void ct_one_tile(const void *__restrict__ x, int64_t 
         if constexpr (WRITE_ROWMAJOR) ct_store_row<SRC>(out, r0 + i, rows_out, cols, cA, cB, okA, okB, lo[i], hi[i]);
     }
 
+    if constexpr (!WRITE_T) return;
     // ---- transpose in registers, stage through LDS
     uint32_t tl[4], th[4];
     transpose4x4(lo, tl);                           // tl[k] = rows r0..r0+3 of column c0+k
@@ -805,6 +802,65 @@ __device__ __forceinline__ void ct_one_tile(const void *__restrict__ x, int64_t 
             const u32x4 v = ct_lds_read(tile, k, m16);
             __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(out_t + oc * rows_out + orow));
         }
+    }
+}
+
+template <int SRC, int FMT, int MODE, bool AMAX, bool WRITE_ROWMAJOR>
+__device__ __forceinline__ void ct_one_tile(const void *__restrict__ x, int64_t rows, int64_t cols, int64_t rows_out, const float *__restrict__ scale,
+                                            float st, uint8_t *__restrict__ out, uint8_t *__restrict__ out_t, int64_t tr,
+                                            int64_t tc, uint8_t *tile, uint32_t &am) {
+    // ---- load the 4 x 8 patch (rows beyond the matrix read as zero)
+    const int tx = threadIdx.x % 8, ty = threadIdx.x / 8;
+    const int64_t r0 = tr * kTileR + ty * 4, cA = tc * kTileC + ct_group_col<SRC>(tx, 0), cB = tc * kTileC + ct_group_col<SRC>(tx, 1);
+    u32x4 raw[4][SRC == ODL_BF16 ? 1 : 2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ct_load_row<SRC>(x, r0 + i, rows, cols, cA, cB, cA < cols, cB < cols, raw[i]);
+    ct_quantise_tile<SRC, FMT, MODE, AMAX, WRITE_ROWMAJOR, true>(raw, rows, cols, rows_out, scale, st, out, out_t, tr, tc, tile, am);
+}
+
+// ------------------------------------- SwiGLU and its gradients straight to codes, delayed scaling
+// h = silu(gate) * up, or d_gate and d_up, are quantised with the scales in force as they are computed, and their partial maxima
+// folded into the roles' strips; the bf16 tensors in between are never written.  HBM-bound: 4 + 2 and 6 + 4 bytes an element
+// (6 + 2 where the transposed codes are not wanted) instead of the 10 and 18 (16) of a bf16 producer and the casts behind it.
+struct DelayedOut {
+    const float *scale;
+    uint8_t *out, *out_t;                            // out_t: null unless T
+    float *parts, *scale_inv;
+};
+
+template <int FMT, bool BWD, bool T>
+__global__ __launch_bounds__(kThreads) void swiglu_cast_delayed_kernel(const uint8_t *__restrict__ dh, const uint8_t *__restrict__ gate,
+                                                                        const uint8_t *__restrict__ up, int64_t rows, int64_t cols, int64_t rows_out,
+                                                                        DelayedOut first, DelayedOut second) {
+    __shared__ __attribute__((aligned(16))) uint8_t tile[T ? kTileC * kTileR : 16];
+    __shared__ uint32_t red[kThreads / kWave];
+    const int tx = threadIdx.x % 8, ty = threadIdx.x / 8;
+    int64_t tr, tc;
+    ct_tile_of(blockIdx.x, (rows_out + kTileR - 1) / kTileR, (cols + kTileC - 1) / kTileC, tr, tc);
+    const int64_t c = tc * kTileC + tx * 8;
+    u32x4 a[4][1], b[4][1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int64_t r = tr * kTileR + ty * 4 + i, at = (r * cols + c) * 2;
+        a[i][0] = b[i][0] = u32x4{0, 0, 0, 0};
+        if (r < rows && c < cols) {                  // cols % 8 == 0 (host-checked)
+            const u32x4 g = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(gate + at)), u = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(up + at));
+            if constexpr (BWD) swiglu_bwd8(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(dh + at)), g, u, a[i][0], b[i][0]);
+            else a[i][0] = swiglu_fwd8(g, u);
+        }
+    }
+    auto finish = [&](const u32x4 (&raw)[4][1], const DelayedOut &o) {
+        const float st = o.scale[0];
+        record_scale_inv(st, o.scale_inv);
+        uint32_t am = 0;
+        ct_quantise_tile<ODL_BF16, FMT, ODL_SCALE_TENSOR, true, true, T>(raw, rows, cols, rows_out, nullptr, st, o.out, o.out_t, tr, tc, tile, am);
+        am = block_max_u32(fold_u16x2_to_f32bits(am), red);
+        if (threadIdx.x == 0 && am != 0) atomicMax(reinterpret_cast<uint32_t *>(o.parts) + (blockIdx.x & (kAmaxParts - 1)), am);
+    };
+    finish(a, first);
+    if constexpr (BWD) {
+        __syncthreads();                             // tile and red are reused
+        finish(b, second);
     }
 }
 
@@ -1443,6 +1499,58 @@ extern "C" int odl_fp8_cast_dynamic_noalloc(const void *x, int src_dtype, int64_
     // the amax pass writes all ODL_FP8_AMAX_PARTS entries (unused ones as 0), so what the last call left is overwritten
     if (int e = odl_fp8_amax_parts(x, src_dtype, rows, cols, parts, stream_)) return e;
     return odl_fp8_cast_dynamic(x, src_dtype, rows, cols, parts, fmt, margin, out, out_t, dyn_out, stream_);
+}
+
+// ------------------------------------------------------------------ SwiGLU straight to codes, delayed scaling
+namespace odl {
+template <int FMT, bool BWD>
+static void launch_swiglu_delayed(const void *dh, const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out, const DelayedOut &a,
+                                  const DelayedOut &b, hipStream_t stream) {
+    const dim3 grid((unsigned)(((rows_out + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC))), block(kThreads);
+    const uint8_t *d = static_cast<const uint8_t *>(dh), *g = static_cast<const uint8_t *>(gate), *u = static_cast<const uint8_t *>(up);
+    if (a.out_t) hipLaunchKernelGGL((swiglu_cast_delayed_kernel<FMT, BWD, true>), grid, block, 0, stream, d, g, u, rows, cols, rows_out, a, b);
+    else hipLaunchKernelGGL((swiglu_cast_delayed_kernel<FMT, BWD, false>), grid, block, 0, stream, d, g, u, rows, cols, rows_out, a, b);
+}
+
+static int check_swiglu_delayed(const char *who, int64_t rows, int64_t cols, int64_t rows_out, int fmt, const void *dh, const void *gate, const void *up,
+                                const DelayedOut *o, int n) {
+    if (rows < 0 || cols < 0 || rows_out < rows) return set_error(ODL_ERR_ARG, "%s: shape %lld x %lld, rows_out %lld", who, (long long)rows, (long long)cols, (long long)rows_out);
+    if (fmt != ODL_FP8_E4M3 && fmt != ODL_FP8_E5M2) return set_error(ODL_ERR_ARG, "%s: fmt %d", who, fmt);
+    if (cols % 8 != 0 || rows_out % 16 != 0) return set_error(ODL_ERR_SHAPE, "%s: cols must be a multiple of 8 and rows_out of 16", who);
+    if (((rows_out + kTileR - 1) / kTileR) * ((cols + kTileC - 1) / kTileC) > 0x7fffffffLL) return set_error(ODL_ERR_SHAPE, "%s: too many tiles for one launch", who);
+    if (rows == 0 || cols == 0) return ODL_OK;
+    if (!gate || !up || (n == 2 && !dh)) return set_error(ODL_ERR_ARG, "%s: null pointer", who);
+    if (!aligned16(gate) || !aligned16(up) || !aligned16(dh)) return set_error(ODL_ERR_SHAPE, "%s: sources must be 16-byte aligned", who);
+    for (int i = 0; i < n; ++i) {
+        if (!o[i].scale || !o[i].out || !o[i].parts || !o[i].scale_inv || (o[i].out_t == nullptr) != (o[0].out_t == nullptr))
+            return set_error(ODL_ERR_ARG, "%s: null pointer", who);
+        if ((reinterpret_cast<uintptr_t>(o[i].out) & 7) || !aligned16(o[i].out_t)) return set_error(ODL_ERR_SHAPE, "%s: codes must be 8-byte, transposed ones 16-byte aligned", who);
+    }
+    return ODL_OK;
+}
+}  // namespace odl
+
+extern "C" int odl_fp8_swiglu_cast_delayed(const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out, const float *scale, int fmt,
+                                           uint8_t *out, uint8_t *out_t, float *amax_parts, float *scale_inv_out, odl_stream_t stream_) {
+    const DelayedOut o[1] = {{scale, out, out_t, amax_parts, scale_inv_out}};
+    if (int e = check_swiglu_delayed("odl_fp8_swiglu_cast_delayed", rows, cols, rows_out, fmt, nullptr, gate, up, o, 1)) return e;
+    if (rows == 0 || cols == 0) return ODL_OK;
+    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+    if (fmt == ODL_FP8_E4M3) launch_swiglu_delayed<ODL_FP8_E4M3, false>(nullptr, gate, up, rows, cols, rows_out, o[0], o[0], stream);
+    else launch_swiglu_delayed<ODL_FP8_E5M2, false>(nullptr, gate, up, rows, cols, rows_out, o[0], o[0], stream);
+    return check_launch("odl_fp8_swiglu_cast_delayed");
+}
+
+extern "C" int odl_fp8_swiglu_bwd_cast_delayed(const void *dh, const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out, int fmt,
+                                               const float *scale_g, uint8_t *dg, uint8_t *dg_t, float *parts_g, float *inv_g, const float *scale_u,
+                                               uint8_t *du, uint8_t *du_t, float *parts_u, float *inv_u, odl_stream_t stream_) {
+    const DelayedOut o[2] = {{scale_g, dg, dg_t, parts_g, inv_g}, {scale_u, du, du_t, parts_u, inv_u}};
+    if (int e = check_swiglu_delayed("odl_fp8_swiglu_bwd_cast_delayed", rows, cols, rows_out, fmt, dh, gate, up, o, 2)) return e;
+    if (rows == 0 || cols == 0) return ODL_OK;
+    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+    if (fmt == ODL_FP8_E4M3) launch_swiglu_delayed<ODL_FP8_E4M3, true>(dh, gate, up, rows, cols, rows_out, o[0], o[1], stream);
+    else launch_swiglu_delayed<ODL_FP8_E5M2, true>(dh, gate, up, rows, cols, rows_out, o[0], o[1], stream);
+    return check_launch("odl_fp8_swiglu_bwd_cast_delayed");
 }
 
 // ------------------------------------------------------------------ rowwise recipe, fused passes

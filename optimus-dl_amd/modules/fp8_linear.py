@@ -231,6 +231,9 @@ class _Fp8LinearFn(torch.autograd.Function):
                 recipe: FP8Recipe, out_dtype: torch.dtype):
         pol = recipe.recipe
         need_dgrad, need_wgrad = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+        # the codes of x where the kernel that computed x has already made them (SwiGLUMLPFn; x2d then holds no values, only
+        # its shape and type count)
+        given = getattr(ctx, "given_input", None)
         bias_f32 = None if bias is None else bias.detach().float()
         saved: dict[str, Any] = {}
         ctx.wgrad_direct = False
@@ -242,7 +245,7 @@ class _Fp8LinearFn(torch.autograd.Function):
 
         if pol.kind in ("mxfp8", "blockwise"):
             fp8_wgrad = need_wgrad and recipe.wgrad
-            xq, xs, xq_t, xs_t = _mx_input_shared(recipe, x2d, pol.fmt_fwd, fp8_wgrad)
+            xq, xs, xq_t, xs_t = given or _mx_input_shared(recipe, x2d, pol.fmt_fwd, fp8_wgrad)
             wq, ws, wq_t, ws_t = module._mx_weight(weight, recipe, need_t=both_w)
             y = native.mx_gemm_nt(xq, xs, wq, ws, pol.fmt_fwd, pol.fmt_fwd, bias=bias_f32, out_dtype=out_dtype)
             if fp8_wgrad:
@@ -280,7 +283,7 @@ class _Fp8LinearFn(torch.autograd.Function):
                 # pass under torch.no_grad() without model.eval() reads the scales and leaves the histories alone
                 record = module._records()
                 meta = module._meta(recipe, x2d.device, "fwd", create=record)
-                xq, xq_t, sx_inv = _quantise_delayed(x2d, pol.fmt_fwd, meta, ROLE_X, fp8_wgrad, recipe=recipe,
+                xq, xq_t, sx_inv = given or _quantise_delayed(x2d, pol.fmt_fwd, meta, ROLE_X, fp8_wgrad, recipe=recipe,
                                                      record=record, margin=pol.margin, rows_out=tokens if fp8_wgrad else None)
             else:
                 xq, xq_t, sx_inv = _quantise_input_shared(recipe, x2d, pol.fmt_fwd, pol.margin, fp8_wgrad)
@@ -311,7 +314,9 @@ class _Fp8LinearFn(torch.autograd.Function):
         module, recipe = ctx.module, ctx.recipe
         saved = dict(zip(ctx.saved_names, ctx.saved_tensors))
         pol = recipe.recipe
-        dy2d = dy if dy.is_contiguous() else dy.contiguous()
+        # codes of dy where the kernel that computed dy has already made them (dy then holds no values, only its shape counts)
+        given = getattr(ctx, "given_grad", None)
+        dy2d = dy if given is not None or dy.is_contiguous() else dy.contiguous()
         if dy2d.dtype not in (torch.bfloat16, torch.float32):
             dy2d = dy2d.to(torch.bfloat16)
         dx = dw = db = None
@@ -322,7 +327,7 @@ class _Fp8LinearFn(torch.autograd.Function):
         if pol.kind in ("mxfp8", "blockwise"):
             if ctx.need_dgrad or fp8_wgrad:
                 # one pass over dy: blocks along the output features for dgrad, along the tokens (transposed) for wgrad
-                gq, gs, gq_t, gs_t = _block_cast(pol, dy2d, pol.fmt_bwd, ctx.need_dgrad, fp8_wgrad)
+                gq, gs, gq_t, gs_t = given or _block_cast(pol, dy2d, pol.fmt_bwd, ctx.need_dgrad, fp8_wgrad)
             if ctx.need_dgrad:
                 dx = native.mx_gemm_nt(gq, gs, saved["wq_t"], saved["ws_t"], pol.fmt_bwd, pol.fmt_fwd, out_dtype=ctx.x_dtype)
             if fp8_wgrad:
@@ -355,7 +360,9 @@ class _Fp8LinearFn(torch.autograd.Function):
             joint = getattr(ctx, "wgrad_joint", None)
             gq_t_out = joint["codes_t"] if joint is not None else None
             if ctx.need_dgrad or fp8_wgrad:
-                if pol.kind == "delayed":
+                if given is not None:
+                    gq, gq_t, sg_inv = given
+                elif pol.kind == "delayed":
                     meta = module._meta(recipe, dy2d.device, "bwd", create=module.training)
                     gq, gq_t, sg_inv = _quantise_delayed(dy2d, pol.fmt_bwd, meta, ROLE_G, g_t_needed, g_rm_needed,
                                                          recipe=recipe, record=module.training, margin=pol.margin, out_t=gq_t_out,

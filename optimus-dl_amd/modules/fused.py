@@ -23,7 +23,7 @@ from .. import native
 from .amp import state as _state
 from .amp.fp8 import FP8Recipe
 from .calls import apply, untraced
-from .fp8_linear import FP8Linear
+from .fp8_linear import ROLE_G, ROLE_X, FP8Linear, _converted_input, _Fp8LinearFn, _Fp8LinearGroupFn, _MemberCtx
 
 
 def _bf16_cuda(*tensors: torch.Tensor) -> bool:
@@ -63,6 +63,128 @@ def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return apply(_SwiGLUFn, gate, up, recipe)
 
 
+# -------------------------------------------------------------- a whole SwiGLU MLP
+class _SwiGLUMLPFn(torch.autograd.Function):
+    """``c_proj(silu(w1 x) * w2 x)`` as one node, for the recipes that need no amax before they cast (delayed scaling, mxfp8).
+
+    The product and its gradients go from the registers of the kernel that computes them straight into codes: h, d_gate and
+    d_up are never written in bf16.  Between separate nodes they have to be, since autograd hands tensors over.  Everything
+    else is what the three Linears do by themselves (their own forwards and backwards run, on their own saved tensors)."""
+
+    @staticmethod
+    def forward(ctx, x2d: torch.Tensor, recipe: FP8Recipe, modules: tuple, *weights: torch.Tensor):
+        pol = recipe.recipe
+        subs, saved = [], []
+
+        def member(x, module, weight, need_x, given=None):
+            sub = _MemberCtx((need_x, True, False, False, False, False))
+            sub.given_input = given
+            y = _Fp8LinearFn.forward(sub, x, weight, None, module, recipe, torch.bfloat16)
+            sub.given_input = None
+            sub.span = (len(saved), len(sub.saved_tensors))
+            saved.extend(sub.saved_tensors)
+            sub.saved_tensors = ()
+            subs.append(sub)
+            return y
+
+        w1, w2, down = modules
+        gate, up = member(x2d, w1, weights[0], ctx.needs_input_grad[0]), member(x2d, w2, weights[1], ctx.needs_input_grad[0])
+        if pol.kind == "mxfp8":
+            h = native.swiglu_mx_cast(gate, up, pol.fmt_fwd, pol.mx_scale_rule)
+        else:
+            meta = down._meta(recipe, x2d.device, "fwd")
+            meta.note_record(recipe._store)
+            h = native.swiglu_cast_delayed(gate, up, meta.scale_of(ROLE_X), pol.fmt_fwd, meta.amax_slot(ROLE_X))
+        y = member(gate, down, weights[2], True, given=h)         # (gate: the shape and type of the product)
+        ctx.save_for_backward(gate, up, *saved)
+        ctx.subs, ctx.recipe = subs, recipe
+        return y
+
+    @staticmethod
+    def backward(ctx, dy: torch.Tensor):
+        gate, up, *tensors = ctx.saved_tensors
+        recipe, pol = ctx.recipe, ctx.recipe.recipe
+        sub_g, sub_u, sub_d = ctx.subs
+        for sub in ctx.subs:
+            sub.saved_tensors = tuple(tensors[sub.span[0]:sub.span[0] + sub.span[1]])
+        dh, dw_d, *_ = _Fp8LinearFn.backward(sub_d, dy)
+        mods = (sub_g.module, sub_u.module)
+        if pol.kind == "mxfp8":
+            given = native.swiglu_bwd_mx_cast(dh, gate, up, pol.fmt_bwd, pol.mx_scale_rule)
+        elif all(m.training for m in mods):
+            metas = [m._meta(recipe, dh.device, "bwd") for m in mods]
+            for meta in metas:
+                meta.note_record(recipe._store)
+            given = native.swiglu_bwd_cast_delayed(dh, gate, up, pol.fmt_bwd, tuple(m.scale_of(ROLE_G) for m in metas),
+                                                   tuple(m.amax_slot(ROLE_G) for m in metas), want_transposed=not (sub_g.wgrad_direct and sub_u.wgrad_direct))
+        else:                                # put into eval mode since the forward: their histories are left alone
+            given = None
+        dgate, dup = (gate, up) if given is not None else native.swiglu_bwd_amax_parts(dh, gate, up)[:2]
+        pairs = _Fp8LinearGroupFn._dgrad_in_one_gemm(ctx, (dgate, dup))
+        dx, grads = None, []
+        for i, (sub, g) in enumerate(zip((sub_g, sub_u), (dgate, dup))):
+            sub.given_grad = given[i] if given is not None else None
+            sub.dx_pairs = pairs
+            # (block scales: the GEMM that adds into what is there is not the streaming one; a sum of its own is cheaper)
+            sub.dx_into = dx if dx is not None and pol.kind == "delayed" else None
+            dxi, dw, *_ = _Fp8LinearFn.backward(sub, g)
+            sub.given_grad = sub.dx_pairs = sub.dx_into = None
+            if dx is None:
+                dx = dxi
+            elif dxi is not None and pol.kind != "delayed":
+                dx = dx + dxi
+            grads.append(dw)
+        if pairs:
+            gqs, wq_ts, sg_invs, sw_invs = zip(*pairs)
+            dx = native.gemm_nt_sum(list(gqs), list(wq_ts), pol.fmt_bwd, pol.fmt_fwd, list(sg_invs), list(sw_invs), out_dtype=sub_g.x_dtype)
+        for sub in ctx.subs:
+            sub.saved_tensors = ()
+        return dx, None, None, *grads, dw_d
+
+
+_any_global_hook = getattr(torch.nn.modules.module, "_has_any_global_hook", None)
+
+
+def _runs_as_written(m: FP8Linear) -> bool:
+    """Nothing looks at this Linear's input, output or their gradients, and nothing stands in for its forward."""
+    return (type(m) is FP8Linear and m.fp8_enabled and m.bias is None and "forward" not in m.__dict__
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
+
+
+@untraced
+def swiglu_mlp(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
+    """``mlp(x)`` as one node (``_SwiGLUMLPFn``), or None where its parts have to run on their own: a recipe that
+    casts with the amax of the tensor itself, no graph, biases, hooks, a Linear switched off or in eval mode, sizes that
+    the kernels do not take, weight gradients that are not FP8 or go straight into ``.grad``."""
+    recipe = _state.active_recipe()
+    if recipe is None or recipe.recipe.kind not in ("delayed", "mxfp8") or _any_global_hook is None or _any_global_hook():
+        return None
+    if not torch.is_grad_enabled() or not x.requires_grad or not recipe.wgrad or recipe.fuse_wgrad_accumulation or not recipe.fuse_dgrad_sum:
+        return None
+    mods = (mlp.w1, mlp.w2, mlp.c_proj)
+    w1, w2, down = mods
+    if not all(_runs_as_written(m) and m.weight.requires_grad for m in mods):
+        return None
+    if (torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype) != torch.bfloat16:
+        return None
+    hidden = w1.out_features
+    if w2.out_features != hidden or down.in_features != hidden or w1._siblings is None or w1._siblings.misses or w1._siblings is not w2._siblings:
+        return None
+    if not (w1._fp8_eligible(x) and w2._fp8_eligible(x)) or not down.weight.is_cuda or down.weight.dtype not in (torch.bfloat16, torch.float32):
+        return None
+    mx = recipe.recipe.kind == "mxfp8"
+    if hidden % (128 if mx else 16) or down.out_features % (32 if mx else 16) or not (mx or all(m.training for m in mods)):
+        return None
+    x2d = x.reshape(-1, w1.in_features)
+    if x2d.dtype != torch.bfloat16 or not x2d.is_contiguous():
+        x2d = _converted_input(recipe, x2d, torch.bfloat16)
+    for m in mods:
+        m.__dict__["fp8_calls"] += 1
+        m._note_grad_mode()
+    y = apply(_SwiGLUMLPFn, x2d, recipe, mods, w1.weight, w2.weight, down.weight)
+    return y.reshape(*x.shape[:-1], down.out_features)
+
+
 # ---------------------------------------------------------------- in-place re-classing
 # A module is fused by giving it a subclass of its own class with the fused forward mixed in: same object, same
 # parameters, same state-dict keys, isinstance() checks keep working.  The subclass is made on the fly, so pickling
@@ -99,7 +221,8 @@ class _FusedSwiGLUForward(_Reclassed):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if _state.active_recipe() is None or not x.is_cuda:
             return super().forward(x)
-        return self.c_proj(swiglu(self.w1(x), self.w2(x)))
+        y = swiglu_mlp(self, x)
+        return self.c_proj(swiglu(self.w1(x), self.w2(x))) if y is None else y
 
 
 def fuse_swiglu_mlp(mlp: nn.Module) -> bool:

@@ -25,7 +25,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 19
+ABI_VERSION = 20
 _OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
@@ -78,6 +78,10 @@ EXPORTS = (
     "odl_fp8_gemm_set_clock_probe",
     "odl_fp8_mx_cast",
     "odl_fp8_mx_cast_padded",
+    "odl_fp8_swiglu_mx_cast",
+    "odl_fp8_swiglu_bwd_mx_cast",
+    "odl_fp8_swiglu_cast_delayed",
+    "odl_fp8_swiglu_bwd_cast_delayed",
     "odl_fp8_mx_gemm_nt",
     "odl_fp8_block_cast",
     "odl_fp8_mx_gemm_splitk",
@@ -158,6 +162,10 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_gemm_variant_name.restype = ctypes.c_char_p
         L.odl_fp8_gemm_set_variant.argtypes = [i32]
         L.odl_fp8_gemm_set_clock_probe.argtypes = [vp, i32]
+        L.odl_fp8_swiglu_mx_cast.argtypes = [vp, vp, i64, i64, i64, i32, vp, vp, vp, vp, i32, vp]
+        L.odl_fp8_swiglu_bwd_mx_cast.argtypes = [vp, vp, vp, i64, i64, i64, i32, vp, vp, vp, vp, vp, vp, vp, vp, i32, vp]
+        L.odl_fp8_swiglu_cast_delayed.argtypes = [vp, vp, i64, i64, i64, vp, i32, vp, vp, vp, vp, vp]
+        L.odl_fp8_swiglu_bwd_cast_delayed.argtypes = [vp, vp, vp, i64, i64, i64, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
         L.odl_fp8_mx_cast_padded.argtypes = [vp, i32, i64, i64, i64, i32, vp, vp, i32, vp, vp, i32, i32, vp]
         L.odl_fp8_mx_cast.argtypes = [vp, i32, i64, i64, i32, vp, vp, i32, vp, vp, i32, i32, vp]
         L.odl_fp8_mx_gemm_nt.argtypes = [vp, vp, vp, vp, i32, i64, i64, i64, i32, i32, vp, vp, i32, i32, vp]
@@ -988,6 +996,78 @@ def mx_cast(x: torch.Tensor, fmt: int, want_rowmajor: bool = True, want_transpos
     _check(load().odl_fp8_mx_cast_padded(x.data_ptr(), _src_dtype(x), rows, cols, n, fmt, ptr(out), ptr(sc), lay, ptr(out_t), ptr(sc_t),
                                          lay_t, int(scale_rule), _stream()), "odl_fp8_mx_cast")
     return out, sc, out_t, sc_t
+
+
+def _swiglu_sources(tensors: tuple, what: str) -> tuple:
+    tensors = tuple(_bf16_dense(t, what) for t in tensors)
+    if any(t.dim() != 2 or t.shape != tensors[0].shape for t in tensors):
+        raise NativeError(f"{what}: 2-D tensors of one shape expected, got {[tuple(t.shape) for t in tensors]}")
+    return tensors
+
+
+def _mx_pair(rows: int, cols: int, n: int, device) -> tuple:
+    new = lambda *size: torch.empty(size, dtype=torch.uint8, device=device)
+    return new(rows, cols), new(cols // 128, rows, 4), new(cols, n), new(n // 128, cols, 4)
+
+
+def swiglu_mx_cast(gate: torch.Tensor, up: torch.Tensor, fmt: int, scale_rule: int):
+    """``mx_cast`` of silu(gate) * up, both layouts, without writing the product (bit for bit that of
+    :func:`swiglu_amax_parts`).  rows % 32 == 0, cols % 128 == 0; the transposed codes are padded to whole K steps.
+    -> (codes, scales, codes_t, scales_t)."""
+    gate, up = _swiglu_sources((gate, up), "swiglu_mx_cast")
+    rows, cols = gate.shape
+    n = padded_rows(rows)
+    h = _mx_pair(rows, cols, n, gate.device)
+    _check(load().odl_fp8_swiglu_mx_cast(gate.data_ptr(), up.data_ptr(), rows, cols, n, fmt, *[t.data_ptr() for t in h], scale_rule, _stream()),
+           "odl_fp8_swiglu_mx_cast")
+    return h
+
+
+def swiglu_bwd_mx_cast(dh: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, fmt: int, scale_rule: int):
+    """The same of the gradients of silu(gate) * up.  -> (what :func:`swiglu_mx_cast` returns) for d_gate, and for d_up."""
+    dh, gate, up = _swiglu_sources((dh, gate, up), "swiglu_bwd_mx_cast")
+    rows, cols = gate.shape
+    n = padded_rows(rows)
+    dg, du = _mx_pair(rows, cols, n, gate.device), _mx_pair(rows, cols, n, gate.device)
+    _check(load().odl_fp8_swiglu_bwd_mx_cast(dh.data_ptr(), gate.data_ptr(), up.data_ptr(), rows, cols, n, fmt,
+                                             *[t.data_ptr() for t in dg + du], scale_rule, _stream()), "odl_fp8_swiglu_bwd_mx_cast")
+    return dg, du
+
+
+def swiglu_cast_delayed(gate: torch.Tensor, up: torch.Tensor, scale: torch.Tensor, fmt: int, amax_parts: torch.Tensor):
+    """``cast_delayed`` of silu(gate) * up, both layouts padded to whole K steps, without writing the product.
+    -> (codes, codes_t, scale_inv[1])."""
+    gate, up = _swiglu_sources((gate, up), "swiglu_cast_delayed")
+    rows, cols = gate.shape
+    n = padded_rows(rows)
+    _f32_dev(scale, 1, "swiglu_cast_delayed scale")
+    _f32_dev(amax_parts, AMAX_PARTS, "swiglu_cast_delayed amax_parts")
+    q, q_t = (torch.empty(size, dtype=torch.uint8, device=gate.device) for size in ((n, cols), (cols, n)))
+    inv = torch.empty(1, dtype=torch.float32, device=gate.device)
+    _check(load().odl_fp8_swiglu_cast_delayed(gate.data_ptr(), up.data_ptr(), rows, cols, n, scale.data_ptr(), fmt, q.data_ptr(), q_t.data_ptr(),
+                                              amax_parts.data_ptr(), inv.data_ptr(), _stream()), "odl_fp8_swiglu_cast_delayed")
+    return q, q_t, inv
+
+
+def swiglu_bwd_cast_delayed(dh: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, fmt: int, scales: tuple, amax_parts: tuple,
+                            want_transposed: bool = True):
+    """The same of the gradients of silu(gate) * up; scales and amax_parts: of d_gate and of d_up.
+    -> ((codes, codes_t or None, scale_inv), the same of d_up)."""
+    dh, gate, up = _swiglu_sources((dh, gate, up), "swiglu_bwd_cast_delayed")
+    rows, cols = gate.shape
+    n = padded_rows(rows)
+    outs, args = [], []
+    for scale, parts in zip(scales, amax_parts):
+        _f32_dev(scale, 1, "swiglu_bwd_cast_delayed scale")
+        _f32_dev(parts, AMAX_PARTS, "swiglu_bwd_cast_delayed amax_parts")
+        q = torch.empty((n, cols), dtype=torch.uint8, device=gate.device)
+        q_t = torch.empty((cols, n), dtype=torch.uint8, device=gate.device) if want_transposed else None
+        inv = torch.empty(1, dtype=torch.float32, device=gate.device)
+        outs.append((q, q_t, inv))
+        args += [scale.data_ptr(), q.data_ptr(), q_t.data_ptr() if q_t is not None else None, parts.data_ptr(), inv.data_ptr()]
+    _check(load().odl_fp8_swiglu_bwd_cast_delayed(dh.data_ptr(), gate.data_ptr(), up.data_ptr(), rows, cols, n, fmt, *args, _stream()),
+           "odl_fp8_swiglu_bwd_cast_delayed")
+    return tuple(outs)
 
 
 BLOCK = 128

@@ -438,3 +438,70 @@ def test_inference_mode_forward_equals_the_no_grad_forward(amp, fuse):
         got = m(ids)["logits"]
     assert sum(mod.fp8_calls for mod in m.modules() if hasattr(mod, "fp8_calls")) - before == 2 * 15
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tokens,width,hidden", [(32, 128, 256), (160, 192, 384), (1056, 256, 640), (2048, 1024, 4096)])
+@pytest.mark.parametrize("kind", ["delayed", "mxfp8"])
+def test_whole_mlp_node_changes_no_bit(amp, monkeypatch, kind, tokens, width, hidden):
+    """SwiGLU straight to codes against the same MLP as separate nodes, over steps that move the delayed scales: outputs, all
+    gradients, histories.  The sizes end inside tiles and K steps; the last one takes wgrad from dY as stored and dX from one GEMM."""
+    from optimus_dl_amd.modules import fused
+    from optimus_dl_amd.modules.model.blocks import SwiGLUMLP
+    from optimus_dl_amd.modules.model_transforms import build_model_transform
+
+    nodes = []
+    real = fused.swiglu_mlp
+    results = {}
+    for whole in (True, False):
+        monkeypatch.setattr(fused, "swiglu_mlp", (lambda m, x: (nodes.append(1), real(m, x))[1]) if whole else (lambda m, x: None))
+        torch.manual_seed(7)
+        mlp = build_model_transform({"_name": "fp8_linear"}).apply(SwiGLUMLP(width, hidden).cuda())
+        recipe = amp.create_fp8_recipe(kind, "hybrid", amax_history_len=4)
+        seen = []
+        for step in range(3):
+            x = (seeded_bf16((2, tokens // 2, width), 1.0 + step, 3 + step)).cuda().requires_grad_(True)
+            mlp.zero_grad()
+            with recipe.autocast(), torch.autocast("cuda", dtype=torch.bfloat16):
+                y = mlp(x)
+            assert (type(y.grad_fn.next_functions[0][0]).__name__ == "_SwiGLUMLPFnBackward") == whole
+            with recipe.backward():
+                y.backward(seeded_bf16(tuple(y.shape), 1e-3 * (1 + step), 9 + step).cuda())
+            seen += [y.detach().clone(), x.grad.clone()] + [p.grad.clone() for p in mlp.parameters()]
+        if kind == "delayed":
+            seen += [meta.amax_history.clone() for m in (mlp.w1, mlp.w2, mlp.c_proj) for meta in m.fp8_meta.values()]
+        results[whole] = seen
+    assert nodes and len(results[True]) == len(results[False])
+    for a, b in zip(results[True], results[False]):
+        assert torch.equal(a, b)
+
+
+def test_whole_mlp_node_stands_back_for_hooks_and_eval_mode(amp):
+    from optimus_dl_amd.modules.fused import swiglu_mlp
+    from optimus_dl_amd.modules.model.blocks import SwiGLUMLP
+    from optimus_dl_amd.modules.model_transforms import build_model_transform
+
+    mlp = build_model_transform({"_name": "fp8_linear"}).apply(SwiGLUMLP(128, 256).cuda())
+    x = seeded_bf16((64, 128), 1.0, 1).cuda().requires_grad_(True)
+    seen = []
+
+    def taken(kind="delayed", data=x):
+        recipe = amp.create_fp8_recipe(kind, "hybrid", amax_history_len=4)
+        with recipe.autocast(), torch.autocast("cuda", dtype=torch.bfloat16):
+            return swiglu_mlp(mlp, data) is not None
+
+    assert taken() and taken("mxfp8") and not taken("tensorwise") and not taken("rowwise") and not taken(data=x.detach())
+    with torch.no_grad():
+        assert not taken()
+    hook = mlp.c_proj.register_forward_pre_hook(lambda m, a: seen.append(a[0].shape))
+    assert not taken()
+    recipe = amp.create_fp8_recipe("delayed", "hybrid", amax_history_len=4)
+    with recipe.autocast(), torch.autocast("cuda", dtype=torch.bfloat16):
+        mlp(x)
+    assert seen == [torch.Size([64, 256])]
+    hook.remove()
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, a, o: None)
+    assert not taken()
+    handle.remove()
+    assert taken()
+    mlp.w2.eval()
+    assert not taken() and taken("mxfp8")
