@@ -263,6 +263,39 @@ __device__ __forceinline__ void epilogue_staged_accumulate(const GemmArgs &g, v1
     }
 }
 
+// ---------------------------------------------------------------- warming
+// What blocks of 256 lanes without a tile do, where the tiles leave compute units idle: read the operands (both K-contiguous)
+// through, ahead of the blocks that multiply them.  An operand of a backward pass was written long ago and lies in HBM, and
+// what one compute unit gets from there is bounded by its latency: 64 KB in flight a microsecond, 0.53 us per K step of a 128 x
+// 128 tile however many stages wait for it and however few units ask.  The idle units bring the whole of it to the
+// memory-side cache in a fraction of the launch.  Cold operands, us without and with: 128 x 128 tiles, 3072 x 768 x 16384 71.5 ->
+// 57.8, 3072 x 1024 x 8192 38.8 -> 33.4, 1024 x 1024 x 4096 21.5 -> 15.9, 512 x 3072 x 768 8.1 -> 7.2 (warm ones 51.7 -> 54.8, 29.4 ->
+// 30.0, 15.9 -> 15.8, 6.4 -> 6.5).
+// A helper reads kb_per_step KB per K step at most (what it can while a step is multiplied); where that does not cover the
+// operands, their last K bytes are read.
+__device__ __forceinline__ void warm_operands(const GemmArgs &g, int helper, int helpers, int kb_per_step) {
+    constexpr int SPAN = 1024, BURST = 16;                // bytes of a row that a wave reads at once; loads in flight
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int M = (int)g.M, rows = M + (int)g.N, K = (int)g.K, spans = (K + SPAN - 1) / SPAN;
+    const int covered = min(spans, (int)((int64_t)(K / 128) * kb_per_step * helpers / rows));
+    const int items = covered * rows, first = spans - covered, waves = helpers * 4;
+    for (int i = helper * 4 + wave; i < items; i += waves * BURST) {
+        u32x4 v[BURST];
+#pragma unroll
+        for (int j = 0; j < BURST; ++j) {
+            const int item = min(i + j * waves, items - 1);
+            const int row = item % rows, k = (first + item / rows) * SPAN + 16 * lane;
+            const uint8_t *p = row < M ? g.a + (int64_t)row * K : g.b + (int64_t)(row - M) * K;
+            v[j] = *reinterpret_cast<const u32x4 *>(p + (k < K ? k : 0));
+        }
+#pragma unroll
+        for (int j = 0; j < BURST; ++j) asm volatile("" ::"v"(v[j]));       // only the reading counts
+    }
+}
+
+// Operands that outgrow the memory-side cache are left alone (8192 x 768 x 50304: 324 us without, 331 with).
+inline bool warming_pays(const GemmArgs &g) { return (g.M + g.N) * g.K <= (int64_t)256 << 20; }
+
 // launchers implemented in gemm_tiled.hip / gemm_thin.hip / gemm_deep.hip / gemm_pipe.hip / gemm_stream.hip (fa, fb: odl_fp8_format of A and B)
 void launch_gemm_tiled(int variant, int fa, int fb, const GemmArgs &g, hipStream_t stream);
 // operand rows that the busiest compute unit of a thin launch fetches per K step: what the launch costs (gemm_thin.hip)

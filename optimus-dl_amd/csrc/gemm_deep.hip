@@ -33,34 +33,6 @@ namespace {
 
 constexpr int NW = 4, STAGES = 3;
 
-// What the blocks without a tile do, where the tiles leave compute units idle: read the operands through, ahead of the
-// blocks that multiply them.  An operand of a backward pass was written long ago and lies in HBM, and what one compute unit
-// gets from there is bounded by its latency: 64 KB in flight a microsecond, 0.53 us per K step however many stages wait for
-// it and however few units ask.  The idle units bring the whole of it to the memory-side cache in a fraction of the launch.
-// Cold operands, us without and with: 3072 x 768 x 16384 71.5 -> 57.8, 3072 x 1024 x 8192 38.8 -> 33.4, 1024 x 1024 x 4096
-// 21.5 -> 15.9, 512 x 3072 x 768 8.1 -> 7.2; warm ones 51.7 -> 54.8, 29.4 -> 30.0, 15.9 -> 15.8, 6.4 -> 6.5.
-// A helper reads 10 KB per K step at most (what it can while a step is multiplied); where that does not cover the
-// operands, their last K bytes are read.  Operands larger than the cache are left alone (8192 x 768 x 50304: 324 -> 331).
-__device__ __forceinline__ void warm_operands(const GemmArgs &g, int helper, int helpers) {
-    constexpr int SPAN = 1024, BURST = 16;                // bytes of a row that a wave reads at once; loads in flight
-    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-    const int M = (int)g.M, rows = M + (int)g.N, K = (int)g.K, spans = (K + SPAN - 1) / SPAN;
-    const int covered = min(spans, (int)((int64_t)(K / 128) * 10 * helpers / rows));
-    const int items = covered * rows, first = spans - covered, waves = helpers * NW;
-    for (int i = helper * NW + wave; i < items; i += waves * BURST) {
-        u32x4 v[BURST];
-#pragma unroll
-        for (int j = 0; j < BURST; ++j) {
-            const int item = min(i + j * waves, items - 1);
-            const int row = item % rows, k = (first + item / rows) * SPAN + 16 * lane;
-            const uint8_t *p = row < M ? g.a + (int64_t)row * K : g.b + (int64_t)(row - M) * K;
-            v[j] = *reinterpret_cast<const u32x4 *>(p + (k < K ? k : 0));
-        }
-#pragma unroll
-        for (int j = 0; j < BURST; ++j) asm volatile("" ::"v"(v[j]));       // only the reading counts
-    }
-}
-
 // MX: block scales (g.mx_sa / g.mx_sb, K-step-major: dword [step][row] = the four scale bytes of a row in that step).  A wave
 // brings 64 dwords of A and B rows to LDS beside its operand loads; a lane reads the dwords of its rows with the fragments
 // and shifts them so that byte 0 / byte 2 are what it supplies in the first / second half (lanes 32 .. 63 hold the odd
@@ -80,7 +52,7 @@ __global__ __launch_bounds__(256) void gemm_nt_deep_kernel(const GemmArgs g) {
     const int per_xcd = (total + 7) / 8;
     const int pid = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if ((int)blockIdx.x >= 8 * per_xcd) {
-        warm_operands(g, (int)blockIdx.x - 8 * per_xcd, (int)gridDim.x - 8 * per_xcd);
+        warm_operands(g, (int)blockIdx.x - 8 * per_xcd, (int)gridDim.x - 8 * per_xcd, 10);
         return;
     }
     if (pid >= total) return;
@@ -257,8 +229,7 @@ template <int FA, int FB>
 void launch_deep_fmt(bool wide, const GemmArgs &g, int num_cus, hipStream_t stream) {
     const int total = g.tiles_m * g.tiles_n;
     const int whole = (total + 7) / 8 * 8;                // a multiple of 8, as is the launch: see the placement in the kernel
-    const bool warm = whole < num_cus && (g.M + g.N) * g.K <= (int64_t)256 << 20;         // idle units, operands that fit the cache
-    const dim3 grid((unsigned)(warm ? num_cus : whole)), block(256);
+    const dim3 grid((unsigned)(whole < num_cus && warming_pays(g) ? num_cus : whole)), block(256);
     if (g.mx_sa) {
         if (wide) hipLaunchKernelGGL((gemm_nt_deep_kernel<4, 2, FA, FB, true>), grid, block, 0, stream, g);
         else hipLaunchKernelGGL((gemm_nt_deep_kernel<2, 2, FA, FB, true>), grid, block, 0, stream, g);
