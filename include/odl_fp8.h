@@ -532,6 +532,19 @@ int odl_fp8_mx_cast_padded(const void *x, int src_dtype, int64_t rows, int64_t c
                            uint8_t *scales, int scales_layout, uint8_t *out_t, uint8_t *scales_t, int scales_t_layout,
                            int scale_rule, odl_stream_t stream);
 
+/* Current scaling of a tensor of at most ODL_FP8_SMALL_BYTES (a multiple of 16 elements, 16-byte aligned) in one launch:
+ * row-major codes and dyn_out = {amax, scale, 1/scale}, bit for bit those of odl_fp8_amax_parts + odl_fp8_cast_dynamic. */
+#define ODL_FP8_SMALL_BYTES 262144
+int odl_fp8_quantise_small(const void *x, int src_dtype, int64_t n, int fmt, int margin, uint8_t *out, float *dyn_out,
+                           odl_stream_t stream);
+
+/* h [M, N] = silu(x . gate^T) * (x . up^T) in bf16 with the roundings of two odl_fp8_gemm_nt (bf16 outputs) and
+ * odl_fp8_swiglu_amax_parts, and the partial maxima of |h|, in one launch.  x [M, K], gate, up [N, K] codes with one scale
+ * each; M <= 64, N % 4 == 0, K % 128 == 0; the products add up as the thin kernel of odl_fp8_gemm_nt adds them. */
+int odl_fp8_gemm_swiglu(const uint8_t *x, const uint8_t *gate, const uint8_t *up, int64_t M, int64_t N, int64_t K, int fmt_x,
+                        int fmt_w, const float *sx_inv, const float *sg_inv, const float *su_inv, void *h, float *parts,
+                        odl_stream_t stream);
+
 /* h = silu(gate) * up (the arithmetic of odl_fp8_swiglu_amax_parts, rounded to bf16 as there) and its codes, and d_gate and d_up of
  * odl_fp8_swiglu_bwd_amax_parts and theirs, in one pass: the bf16 tensors in between are never written.  Codes and scales
  * are bit for bit those of the producer followed by the cast.  rows > 0 does something, cols > 0 too.

@@ -12,6 +12,7 @@
 // The eight partial tiles are added in wave order through LDS at the end: the result does not depend on scheduling, and
 // there is no workspace and no second launch.
 #include "gemm_common.h"
+#include "swiglu.h"
 
 namespace odl {
 
@@ -26,17 +27,19 @@ __device__ __forceinline__ v4f mfma_16x16x128(v8i first, v8i second, v4f acc) {
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(first, second, acc, F1, F2, 0, 0, 0, 0);
 }
 
-template <int MT, int NT, int FA, int FB>
-__global__ __launch_bounds__(64 * kThinWaves) void gemm_nt_thin_kernel(const GemmArgs g) {
-    constexpr int ROWS = 16 * (MT + NT);                  // operand rows of a K step: NT tiles of B, then MT tiles of A
+// operand rows of a K step: NT tiles of B, then MT tiles of A; LDS of a block: a stage, later a set of partial tiles, per wave
+template <int MT, int NT>
+constexpr int thin_lds_bytes() { return kThinWaves * (16 * (MT + NT) * 128 > MT * NT * 1024 ? 16 * (MT + NT) * 128 : MT * NT * 1024); }
+
+// GATED: the first column tile comes from g.b and the second from `up`, 16 columns of each.
+template <int MT, int NT, int FA, int FB, bool GATED>
+__device__ __forceinline__ void thin_partial_tiles(const GemmArgs &g, const uint8_t *up, int64_t m0, int64_t n0, uint8_t *lds) {
+    constexpr int ROWS = 16 * (MT + NT);
     constexpr int LOADS = ROWS / 8;                       // a wave instruction fetches whole 128-byte lines of 8 rows
     constexpr int DEPTH = 3;                              // K steps held in registers
-    constexpr int STAGE = ROWS * 128, PARTIAL = MT * NT * 1024;
-    __shared__ __align__(1024) uint8_t lds[kThinWaves * (STAGE > PARTIAL ? STAGE : PARTIAL)];
+    constexpr int STAGE = ROWS * 128;
     const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int row = lane % 16, group = lane / 16;
-    // the row tiles of one column tile run side by side: they read the same rows of B
-    const int64_t m0 = (int64_t)(blockIdx.x % g.tiles_m) * (16 * MT), n0 = (int64_t)(blockIdx.x / g.tiles_m) * (16 * NT);
 
     // Memory -> registers: lane l reads chunk l % 8 of row l / 8 of each group of eight rows (rows past the end are read
     // as the last row; what they give is not stored).  Registers -> the wave's own LDS, chunks swizzled so that the
@@ -47,13 +50,13 @@ __global__ __launch_bounds__(64 * kThinWaves) void gemm_nt_thin_kernel(const Gem
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) {
         const int r = 8 * j + lane / 8, chunk = lane % 8;
-        src[j] = (uint32_t)((j < 2 * NT ? min(n0 + r, g.N - 1) : min(m0 + r - 16 * NT, g.M - 1)) * g.K) + 16 * chunk;
+        src[j] = (uint32_t)((j < 2 * NT ? min(n0 + (GATED ? r % 16 : r), g.N - 1) : min(m0 + r - 16 * NT, g.M - 1)) * g.K) + 16 * chunk;
         dst[j] = r * 128 + ((chunk ^ swz(r)) << 4);
     }
     struct Lines { u32x4 v[LOADS]; };
     auto fetch = [&](Lines &f, int64_t k) {
 #pragma unroll
-        for (int j = 0; j < LOADS; ++j) f.v[j] = *reinterpret_cast<const u32x4 *>((j < 2 * NT ? g.b : g.a) + k + src[j]);
+        for (int j = 0; j < LOADS; ++j) f.v[j] = *reinterpret_cast<const u32x4 *>((j < 2 * NT ? (GATED && j >= 2 ? up : g.b) : g.a) + k + src[j]);
     };
     v4f acc[MT][NT];
 #pragma unroll
@@ -108,15 +111,34 @@ __global__ __launch_bounds__(64 * kThinWaves) void gemm_nt_thin_kernel(const Gem
 #pragma unroll
         for (int u = 0; u < NT; ++u) partial[wave][t * NT + u][lane] = acc[t][u];
     __syncthreads();
+}
+
+// the eight waves' sums of a tile, in wave order
+template <int MT, int NT>
+__device__ __forceinline__ v4f thin_sum(const uint8_t *lds, int tile) {
+    const v4f(*partial)[MT * NT][64] = reinterpret_cast<const v4f (*)[MT * NT][64]>(lds);
+    const int lane = threadIdx.x % 64;
+    v4f sum = partial[0][tile][lane];
+#pragma unroll
+    for (int w = 1; w < kThinWaves; ++w) {
+        const v4f p = partial[w][tile][lane];
+        sum.x = sum.x + p.x; sum.y = sum.y + p.y; sum.z = sum.z + p.z; sum.w = sum.w + p.w;
+    }
+    return sum;
+}
+
+template <int MT, int NT, int FA, int FB>
+__global__ __launch_bounds__(64 * kThinWaves) void gemm_nt_thin_kernel(const GemmArgs g) {
+    __shared__ __align__(1024) uint8_t lds[thin_lds_bytes<MT, NT>()];
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int row = lane % 16, group = lane / 16;
+    // the row tiles of one column tile run side by side: they read the same rows of B
+    const int64_t m0 = (int64_t)(blockIdx.x % g.tiles_m) * (16 * MT), n0 = (int64_t)(blockIdx.x / g.tiles_m) * (16 * NT);
+    thin_partial_tiles<MT, NT, FA, FB, false>(g, nullptr, m0, n0, lds);
 
     const float *bias = reinterpret_cast<const float *>(g.bias);
     for (int tile = wave; tile < MT * NT; tile += kThinWaves) {
-        v4f sum = partial[0][tile][lane];
-#pragma unroll
-        for (int w = 1; w < kThinWaves; ++w) {
-            const v4f p = partial[w][tile][lane];
-            sum.x = sum.x + p.x; sum.y = sum.y + p.y; sum.z = sum.z + p.z; sum.w = sum.w + p.w;
-        }
+        const v4f sum = thin_sum<MT, NT>(lds, tile);
         const int64_t m = m0 + 16 * (tile / NT) + row, n = n0 + 16 * (tile % NT) + 4 * group;
         if (m >= g.M || n >= g.N) continue;               // N % 4 == 0: the four columns are in or out together
         const float sa = g.sa[m * g.sa_vec];
@@ -142,6 +164,48 @@ __global__ __launch_bounds__(64 * kThinWaves) void gemm_nt_thin_kernel(const Gem
             *c = float4{v[0], v[1], v[2], v[3]};
         }
     }
+}
+
+// ---------------------------------------------------------------- gate and up of a SwiGLU MLP, and their product
+// h = bf16( silu(bf16(x . gate^T)) * bf16(x . up^T) ) for a few rows, and the partial maxima of |h| that odl_fp8_cast_dynamic
+// takes: a block owns 16 columns of both weights.  Bound by reading them (32 x 14336 x 4096 twice: 117 MB).  As two products
+// and a third launch for the activation: 16.5 + 15.4 + 6 us, here 33, and two more launches for the host to issue, of the
+// seven that a decode step of the MLP took.  At most kParts blocks, each its own entry of `parts`, so that nobody has to
+// zero them; the same sums and roundings as the three launches.
+template <int MT, int FA, int FB>
+__global__ __launch_bounds__(64 * kThinWaves) void gemm_thin_swiglu_kernel(const GemmArgs g, const uint8_t *up, const float *s_up, float *parts) {
+    __shared__ __align__(1024) uint8_t lds[thin_lds_bytes<MT, 2>()];
+    __shared__ uint32_t red[MT];
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int row = lane % 16, group = lane / 16;
+    const float sg = g.sa[0] * g.sb[0], su = g.sa[0] * s_up[0];
+    uint32_t am = 0;
+    const int tiles = g.tiles_m * g.tiles_n;
+    for (int p = blockIdx.x; p < tiles; p += gridDim.x) {
+        const int64_t m0 = (int64_t)(p % g.tiles_m) * (16 * MT), n0 = (int64_t)(p / g.tiles_m) * 16;
+        thin_partial_tiles<MT, 2, FA, FB, true>(g, up, m0, n0, lds);
+        if (wave < MT) {
+            const v4f a = thin_sum<MT, 2>(lds, 2 * wave), b = thin_sum<MT, 2>(lds, 2 * wave + 1);
+            const int64_t m = m0 + 16 * wave + row, n = n0 + 4 * group;
+            if (m < g.M && n < g.N) {
+                const u32x2 h = {swiglu_fwd_pair(pack_bf16x2(a.x * sg, a.y * sg), pack_bf16x2(b.x * su, b.y * su)),
+                                 swiglu_fwd_pair(pack_bf16x2(a.z * sg, a.w * sg), pack_bf16x2(b.z * su, b.w * su))};
+                *reinterpret_cast<u32x2 *>(reinterpret_cast<uint16_t *>(g.c) + m * g.N + n) = h;
+                am = max_u16x2(am, max_u16x2(abs_bf16x2(h.x), abs_bf16x2(h.y)));
+            }
+        }
+        __syncthreads();                                  // the partial tiles lie where the next tile's operands go
+    }
+    am = wave_max_u32(fold_u16x2_to_f32bits(am));
+    if (wave < MT && lane == 0) red[wave] = am;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < MT; ++w) am = max(am, red[w]);
+        parts[blockIdx.x] = bits_to_float(am);
+    }
+    if (blockIdx.x == 0)
+        for (int j = (int)gridDim.x + threadIdx.x; j < ODL_FP8_AMAX_PARTS; j += 64 * kThinWaves) parts[j] = 0.0f;
 }
 
 template <int MT, int NT, int FA, int FB>
@@ -192,4 +256,41 @@ void launch_gemm_thin(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_
     else launch_thin_fmt<ODL_FP8_E5M2, ODL_FP8_E5M2>(mt, nt, g, stream);
 }
 
+template <int FA, int FB>
+static void launch_thin_swiglu(const GemmArgs &args, const uint8_t *up, const float *s_up, float *parts, hipStream_t stream) {
+    GemmArgs g = args;
+    const int mt = g.M <= 16 ? 1 : g.M <= 32 ? 2 : 4;
+    g.tiles_m = (int)((g.M + 16 * mt - 1) / (16 * mt));
+    g.tiles_n = (int)((g.N + 15) / 16);
+    const int tiles = g.tiles_m * g.tiles_n;
+    const dim3 grid((unsigned)(tiles < ODL_FP8_AMAX_PARTS ? tiles : ODL_FP8_AMAX_PARTS)), block(64 * kThinWaves);
+    if (mt == 1) hipLaunchKernelGGL((gemm_thin_swiglu_kernel<1, FA, FB>), grid, block, 0, stream, g, up, s_up, parts);
+    else if (mt == 2) hipLaunchKernelGGL((gemm_thin_swiglu_kernel<2, FA, FB>), grid, block, 0, stream, g, up, s_up, parts);
+    else hipLaunchKernelGGL((gemm_thin_swiglu_kernel<4, FA, FB>), grid, block, 0, stream, g, up, s_up, parts);
+}
+
 }  // namespace odl
+
+using namespace odl;
+
+extern "C" int odl_fp8_gemm_swiglu(const uint8_t *x, const uint8_t *gate, const uint8_t *up, int64_t M, int64_t N, int64_t K, int fmt_x, int fmt_w,
+                                   const float *sx_inv, const float *sg_inv, const float *su_inv, void *h, float *parts, odl_stream_t stream_) {
+    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+    if (!x || !gate || !up || !sx_inv || !sg_inv || !su_inv || !h || !parts) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_swiglu: null pointer");
+    if ((fmt_x != ODL_FP8_E4M3 && fmt_x != ODL_FP8_E5M2) || (fmt_w != ODL_FP8_E4M3 && fmt_w != ODL_FP8_E5M2))
+        return set_error(ODL_ERR_ARG, "odl_fp8_gemm_swiglu: formats %d, %d", fmt_x, fmt_w);
+    if (M <= 0 || N <= 0 || K <= 0 || M > 64 || N % 4 != 0 || K % 128 != 0 || (double)N * (double)K >= 4294967296.0 || (double)M * (double)K >= 4294967296.0)
+        return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_swiglu: at most 64 rows, N %% 4 == 0, K %% 128 == 0, operands under 4 GiB; got %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
+    for (const void *p : {(const void *)x, (const void *)gate, (const void *)up, (const void *)h})
+        if (reinterpret_cast<uintptr_t>(p) & 15) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_swiglu: operands and output must be 16-byte aligned");
+    GemmArgs g;
+    g.a = x; g.b = gate; g.c = h; g.sa = sx_inv; g.sb = sg_inv; g.bias = nullptr;
+    g.M = M; g.N = N; g.K = K;
+    g.sa_vec = g.sb_vec = 0;
+    g.out_dtype = ODL_BF16;
+    if (fmt_x == ODL_FP8_E4M3 && fmt_w == ODL_FP8_E4M3) launch_thin_swiglu<ODL_FP8_E4M3, ODL_FP8_E4M3>(g, up, su_inv, parts, stream);
+    else if (fmt_x == ODL_FP8_E5M2 && fmt_w == ODL_FP8_E4M3) launch_thin_swiglu<ODL_FP8_E5M2, ODL_FP8_E4M3>(g, up, su_inv, parts, stream);
+    else if (fmt_x == ODL_FP8_E4M3 && fmt_w == ODL_FP8_E5M2) launch_thin_swiglu<ODL_FP8_E4M3, ODL_FP8_E5M2>(g, up, su_inv, parts, stream);
+    else launch_thin_swiglu<ODL_FP8_E5M2, ODL_FP8_E5M2>(g, up, su_inv, parts, stream);
+    return check_launch("odl_fp8_gemm_swiglu");
+}

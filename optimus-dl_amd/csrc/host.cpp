@@ -16,11 +16,14 @@ using i64 = int64_t;
 namespace {
 
 constexpr i64 kParts = 512;                 // ODL_FP8_AMAX_PARTS
+constexpr i64 kSmall = 262144;              // ODL_FP8_SMALL_BYTES
 constexpr i64 kColsumFloats = 512 * 256, kNormSlabs = 512;
 
 // entries of the C library, by address (native.py loads it and hands them over)
 int (*amax_parts_c)(const void *, int, i64, i64, void *, void *);
 int (*cast_dynamic_c)(const void *, int, i64, i64, i64, const void *, int, int, void *, void *, void *, void *);
+int (*quantise_small_c)(const void *, int, i64, int, int, void *, void *, void *);
+int (*gemm_swiglu_c)(const void *, const void *, const void *, i64, i64, i64, int, int, const void *, const void *, const void *, void *, void *, void *);
 int (*cast_delayed_c)(const void *, int, i64, i64, i64, const void *, int, void *, void *, void *, void *, void *);
 int (*amax_colsum_c)(const void *, int, i64, i64, void *, void *, void *, void *);
 int (*swiglu_c)(const void *, const void *, i64, i64, void *, void *, void *);
@@ -46,6 +49,8 @@ void take(F &f, const py::dict &d, const char *name) { f = reinterpret_cast<F>(p
 void bind(const py::dict &d) {
     take(amax_parts_c, d, "odl_fp8_amax_parts");
     take(cast_dynamic_c, d, "odl_fp8_cast_dynamic_padded");
+    take(quantise_small_c, d, "odl_fp8_quantise_small");
+    take(gemm_swiglu_c, d, "odl_fp8_gemm_swiglu");
     take(cast_delayed_c, d, "odl_fp8_cast_delayed_padded");
     take(amax_colsum_c, d, "odl_fp8_amax_parts_colsum");
     take(swiglu_c, d, "odl_fp8_swiglu_amax_parts");
@@ -117,6 +122,26 @@ py::object cast_dynamic(const Tensor &x, const Tensor &parts, int fmt, int margi
     const int rc = call(cast_dynamic_c, ptr(x), src_of(x), rows, cols, n, ptr(parts), fmt, margin, ptr(q), ptr(q_t), ptr(dyn), str(stream));
     if (rc) return status(rc);
     return py::make_tuple(obj(q), obj(q_t), dyn.select(0, 0), dyn.select(0, 1), dyn.select(0, 2));
+}
+
+// a small tensor in one launch, row-major codes only
+py::object quantise_small(const Tensor &x, int fmt, int margin, i64 stream) {
+    const i64 n = x.numel();
+    if (!source2d(x) || n == 0 || n * x.element_size() > kSmall || n % 16 || !aligned(x)) return none();
+    Tensor q = bytes(x, {x.size(0), x.size(1)}), dyn = f32(x, {3, 1});
+    const int rc = call(quantise_small_c, ptr(x), src_of(x), n, fmt, margin, ptr(q), ptr(dyn), str(stream));
+    return rc ? status(rc) : py::make_tuple(q, py::none(), dyn.select(0, 0), dyn.select(0, 1), dyn.select(0, 2));
+}
+
+py::object gemm_swiglu(const Tensor &x, const Tensor &gate, const Tensor &up, int fx, int fw, const Tensor &sx, const Tensor &sg, const Tensor &su,
+                       i64 stream) {
+    if (!codes2d(x) || !codes2d(gate) || !codes2d(up) || gate.sizes() != up.sizes() || x.size(1) != gate.size(1) || !floats(sx, 1) || !floats(sg, 1) ||
+        !floats(su, 1))
+        return none();
+    Tensor h = at::empty({x.size(0), gate.size(0)}, x.options().dtype(at::kBFloat16)), parts = f32(x, {kParts});
+    const int rc = call(gemm_swiglu_c, ptr(x), ptr(gate), ptr(up), x.size(0), gate.size(0), x.size(1), fx, fw, ptr(sx), ptr(sg), ptr(su), ptr(h),
+                        ptr(parts), str(stream));
+    return rc ? status(rc) : py::make_tuple(h, parts);
 }
 
 py::object cast_delayed(const Tensor &x, const Tensor &scale, int fmt, const OptTensor &parts, bool want_q, bool want_t, const OptTensor &out_t,
@@ -312,6 +337,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("bind", &bind);
     m.def("amax_parts", &amax_parts);
     m.def("cast_dynamic", &cast_dynamic);
+    m.def("quantise_small", &quantise_small);
+    m.def("gemm_swiglu", &gemm_swiglu);
     m.def("cast_delayed", &cast_delayed);
     m.def("amax_colsum", &amax_colsum);
     m.def("swiglu", &swiglu);

@@ -53,13 +53,18 @@ class _NoGraph:
         pass
 
 
+def no_graph() -> bool:
+    """Whether nothing records, transforms or traces what runs now."""
+    return not (not _graph_state_known or torch.is_grad_enabled() or _forward_ad._current_level >= 0 or _functorch_stack() is not None
+                or _tracing_state() is not None)
+
+
 def apply(function: "type[torch.autograd.Function]", *args):
     """``function.apply(*args)``; only its forward where no graph is recorded.
 
     ``Function.apply`` reports parameters that require gradients as needing one also under ``torch.no_grad()``: a forward
     that prepares operands of the backward (transposed codes) would make them for nobody.  Whatever else looks at an
     autograd function still finds it: functorch transforms, forward-mode differentiation and the tracer of torch.jit."""
-    if (not _graph_state_known or torch.is_grad_enabled() or _forward_ad._current_level >= 0 or _functorch_stack() is not None
-            or _tracing_state() is not None):
+    if not no_graph():
         return function.apply(*args)
     return function.forward(_NoGraph(len(args)), *args)

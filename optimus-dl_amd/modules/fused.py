@@ -22,7 +22,7 @@ import torch.nn.functional as F
 from .. import native
 from .amp import state as _state
 from .amp.fp8 import FP8Recipe
-from .calls import apply, untraced
+from .calls import apply, no_graph, untraced
 from .fp8_linear import ROLE_G, ROLE_X, FP8Linear, _converted_input, _Fp8LinearFn, _Fp8LinearGroupFn, _MemberCtx
 
 
@@ -185,6 +185,40 @@ def swiglu_mlp(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
     return y.reshape(*x.shape[:-1], down.out_features)
 
 
+@untraced
+def swiglu_few_rows(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
+    """``silu(w1 x) * w2 x`` of a decode step in one launch (``native.gemm_swiglu``), or None: only per-tensor current scaling,
+    no graph, at most 64 rows, no biases, no hooks."""
+    recipe = _state.active_recipe()
+    if recipe is None or recipe.recipe.kind != "tensorwise" or not no_graph() or _any_global_hook is None or _any_global_hook():
+        return None
+    w1, w2 = mlp.w1, mlp.w2
+    k = w1.in_features
+    if x.numel() > 64 * k or k % 128 or w2.out_features != w1.out_features or w2.in_features != k or not (_runs_as_written(w1) and _runs_as_written(w2)):
+        return None
+    if (torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype) != torch.bfloat16:
+        return None
+    if not (w1._fp8_eligible(x) and w2._fp8_eligible(x)):
+        return None
+    x2d = x.reshape(-1, k)
+    if x2d.dtype != torch.bfloat16 or not x2d.is_contiguous():
+        x2d = _converted_input(recipe, x2d, torch.bfloat16)
+    pol = recipe.recipe
+    parts = recipe.take_parts(x2d)
+    xq, _, _, _, sx_inv = (native.quantise_small(x2d, pol.fmt_fwd, pol.margin) if parts is None
+                           else native.cast_dynamic(x2d, parts, pol.fmt_fwd, pol.margin, want_transposed=False))
+    codes = []
+    for m in (w1, w2):
+        m.__dict__["fp8_calls"] += 1
+        m._note_grad_mode()
+        codes.append(m._tensor_weight(m.weight, recipe, need_t=recipe.cache_weights and x2d.requires_grad))
+    (g, _, sg_inv), (u, _, su_inv) = codes
+    h, parts = native.gemm_swiglu(xq, g, u, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sg_inv, su_inv)
+    h = h.reshape(*x.shape[:-1], w1.out_features)
+    recipe.offer_parts(h, parts)
+    return h
+
+
 # ---------------------------------------------------------------- in-place re-classing
 # A module is fused by giving it a subclass of its own class with the fused forward mixed in: same object, same
 # parameters, same state-dict keys, isinstance() checks keep working.  The subclass is made on the fly, so pickling
@@ -221,8 +255,14 @@ class _FusedSwiGLUForward(_Reclassed):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if _state.active_recipe() is None or not x.is_cuda:
             return super().forward(x)
-        y = swiglu_mlp(self, x)
-        return self.c_proj(swiglu(self.w1(x), self.w2(x))) if y is None else y
+        if torch.is_grad_enabled():
+            y = swiglu_mlp(self, x)
+            if y is not None:
+                return y
+            h = None
+        else:
+            h = swiglu_few_rows(self, x)
+        return self.c_proj(swiglu(self.w1(x), self.w2(x)) if h is None else h)
 
 
 def fuse_swiglu_mlp(mlp: nn.Module) -> bool:

@@ -25,7 +25,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 20
+ABI_VERSION = 21
 _OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
@@ -42,6 +42,8 @@ EXPORTS = (
     "odl_fp8_amax_scale",
     "odl_fp8_amax_parts",
     "odl_fp8_cast_dynamic",
+    "odl_fp8_quantise_small",
+    "odl_fp8_gemm_swiglu",
     "odl_fp8_cast_dynamic_noalloc",
     "odl_fp8_cast_dynamic_padded",
     "odl_fp8_cast_delayed_padded",
@@ -124,6 +126,8 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_scale_from_amax.argtypes = [vp, i64, i32, i32, vp, vp, vp]
         L.odl_fp8_amax_scale.argtypes = [vp, i32, i64, i64, i32, i32, vp, vp, vp, vp, vp]
         L.odl_fp8_amax_parts.argtypes = [vp, i32, i64, i64, vp, vp]
+        L.odl_fp8_quantise_small.argtypes = [vp, i32, i64, i32, i32, vp, vp, vp]
+        L.odl_fp8_gemm_swiglu.argtypes = [vp, vp, vp, i64, i64, i64, i32, i32, vp, vp, vp, vp, vp, vp]
         L.odl_fp8_cast_dynamic.argtypes = [vp, i32, i64, i64, vp, i32, i32, vp, vp, vp, vp]
         L.odl_fp8_cast_dynamic_padded.argtypes = [vp, i32, i64, i64, i64, vp, i32, i32, vp, vp, vp, vp]
         L.odl_fp8_cast_delayed_padded.argtypes = [vp, i32, i64, i64, i64, vp, i32, vp, vp, vp, vp, vp]
@@ -521,6 +525,16 @@ def quantize_dynamic(x: torch.Tensor, fmt: int, margin: int = 0, want_rowmajor: 
     them (one launch then).  out_t, rows_out: as in :func:`cast_dynamic`.  -> (q or None, q_t or None, amax, scale, scale_inv)."""
     return cast_dynamic(x, amax_parts(x) if parts is None else parts, fmt, margin, want_rowmajor, want_transposed, out_t=out_t,
                         rows_out=rows_out)
+
+
+def quantise_small(x: torch.Tensor, fmt: int, margin: int = 0):
+    """Row-major codes of :func:`quantize_dynamic` in one launch (one block: at most 256 KB, a multiple of 16 elements), or by
+    that function where the tensor is larger or not dense.  -> (q, None, amax, scale, scale_inv)."""
+    load()
+    r = _host.quantise_small(x, fmt, margin, _stream())
+    if r is None:
+        return quantize_dynamic(x, fmt, margin, want_transposed=False)
+    return _done(r, "odl_fp8_quantise_small")
 
 
 def _bf16_dense(t: torch.Tensor, what: str) -> torch.Tensor:
@@ -938,6 +952,17 @@ def gemm_nt_sum(a: "list[torch.Tensor]", b: "list[torch.Tensor]", fmt_a: int, fm
                                       ptrs(*[t.data_ptr() for t in sa_inv]), ptrs(*[t.data_ptr() for t in sb_inv]), out.data_ptr(),
                                       odt, _stream()), "odl_fp8_gemm_nt_sum")
     return out
+
+
+def gemm_swiglu(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, fmt_x: int, fmt_w: int, sx_inv: torch.Tensor, sg_inv: torch.Tensor,
+                su_inv: torch.Tensor):
+    """h = silu(x . gate^T) * (x . up^T) in bf16 for at most 64 rows (the roundings of two products and :func:`swiglu_amax_parts`),
+    in one launch; x, gate, up uint8 FP8 codes [M, K], [N, K], [N, K] with one inverse scale each.  -> (h, partial maxima of |h|)."""
+    load()
+    r = _host.gemm_swiglu(x, gate, up, fmt_x, fmt_w, sx_inv, sg_inv, su_inv, _stream())
+    if r is None:
+        raise NativeError("gemm_swiglu: dense uint8 codes [M, K], [N, K], [N, K] and one fp32 scale each expected")
+    return _done(r, "odl_fp8_gemm_swiglu")
 
 
 MX_BLOCK = 32

@@ -505,3 +505,46 @@ def test_whole_mlp_node_stands_back_for_hooks_and_eval_mode(amp):
     assert taken()
     mlp.w2.eval()
     assert not taken() and taken("mxfp8")
+
+
+@pytest.mark.parametrize("rows", [16, 32, 48, 64])
+@pytest.mark.parametrize("width,hidden", [(128, 48), (768, 2048), (2048, 5632), (1152, 14336)])
+def test_gate_up_and_product_of_a_few_rows_in_one_launch(rows, width, hidden):
+    """Bit for bit the two products of the thin kernel (which adds in the same order) and the SwiGLU kernel."""
+    from optimus_dl_amd import native as N
+
+    x, g, u = seeded_bf16((rows, width), 1.0, rows), seeded_bf16((hidden, width), 0.02, 2), seeded_bf16((hidden, width), 0.02, 3)
+    (xq, _, _, _, sx), (gq, _, _, _, sg), (uq, _, _, _, su) = (N.quantize_dynamic(t.cuda(), O.E4M3, 0, True, False) for t in (x, g, u))
+    h, parts = N.gemm_swiglu(xq, gq, uq, O.E4M3, O.E4M3, sx, sg, su)
+    N.gemm_set_variant(next(i for i, name in enumerate(N.gemm_variants()) if name.startswith("thin")))
+    try:
+        gate, up = N.gemm_nt(xq, gq, O.E4M3, O.E4M3, sx, sg), N.gemm_nt(xq, uq, O.E4M3, O.E4M3, sx, su)
+    finally:
+        N.gemm_set_variant(-1)
+    assert torch.equal(h, N.swiglu_amax_parts(gate, up)[0])
+    assert parts.max().item() == h.float().abs().max().item() and (parts >= 0).all()
+
+
+def test_decode_step_of_a_swiglu_mlp(amp):
+    """Evaluation of a few rows takes the one launch; more rows, hooks and other recipes do not."""
+    from optimus_dl_amd.modules import fused
+
+    mlp, _ = make_mlp(256, 512)
+    x = seeded_bf16((32, 1, 256), 1.0, 4).cuda()
+    recipe = amp.create_fp8_recipe("tensorwise", "hybrid")
+    with recipe.autocast(), torch.no_grad():
+        h = fused.swiglu_few_rows(mlp, x)
+        y = mlp(x)
+        many = mlp(x.expand(32, 8, 256).contiguous())
+        assert fused.swiglu_few_rows(mlp, x.expand(32, 8, 256)) is None
+        seen = []
+        hook = mlp.w2.register_forward_hook(lambda m, a, o: seen.append(o.shape))
+        assert fused.swiglu_few_rows(mlp, x) is None
+        mlp(x)
+        hook.remove()
+    assert h.shape == (32, 1, 512) and seen == [torch.Size([32, 1, 512])]
+    assert max_rel_err(y.float().cpu(), many[:, :1].float().cpu()) <= 1e-2
+    with recipe.autocast():
+        assert fused.swiglu_few_rows(mlp, x) is None          # a graph is recorded
+    with amp.create_fp8_recipe("rowwise", "hybrid").autocast(), torch.no_grad():
+        assert fused.swiglu_few_rows(mlp, x) is None

@@ -536,3 +536,19 @@ def test_row_and_column_maxima_of_one_pass(N, dtype, rows, cols):
         ref = want.masked_fill(want.isnan(), 0.0).amax(dim)
         nan = want.isnan().any(dim)
         assert torch.equal(got.cpu().isnan(), nan) and torch.equal(got.cpu()[~nan], ref[~nan])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("fmt", [O.E4M3, O.E5M2])
+@pytest.mark.parametrize("rows,cols", [(1, 16), (16, 17), (32, 4096), (48, 1008), (16, 8192), (32, 4112)])
+def test_small_tensors_in_one_launch(N, dtype, fmt, rows, cols):
+    x = seeded_bf16((rows, cols), 3.0, rows + cols).to(dtype)
+    for special in (None, 0.0, float("inf"), float("nan")):
+        if special is not None:
+            x = x.clone() if special != 0.0 else torch.zeros_like(x)
+            x[0, cols // 2] = special
+        one = N.quantise_small(x.cuda(), fmt, 1)
+        two = N.cast_dynamic(x.cuda(), N.amax_parts(x.cuda()), fmt, 1, True, False)
+        assert_bytes_equal(one[0].cpu(), two[0].cpu(), f"codes, {special}")
+        for a, b in zip(one[2:], two[2:]):
+            assert_f32_bits_equal(a.cpu(), b.cpu(), f"scales, {special}")
