@@ -550,6 +550,7 @@ int odl_fp8_gemm_swiglu(const uint8_t *x, const uint8_t *gate, const uint8_t *up
  * are bit for bit those of the producer followed by the cast.  rows > 0 does something, cols > 0 too.
  *   _mx_cast       odl_fp8_mx_cast_padded with both layouts and K-step-major scales (rows % 32 == 0, cols and rows_out % 128 == 0;
  *                  every pointer 16-byte aligned)
+ *   _block_cast    odl_fp8_block_cast with 1-D blocks and both layouts (rows % 128 == 0, cols % 128 == 0; every pointer 16-byte aligned)
  *   _cast_delayed  odl_fp8_cast_delayed_padded (cols % 8 == 0, rows_out % 16 == 0); amax_parts and scale_inv are required; the
  *                  transposed codes of both tensors may be NULL together */
 int odl_fp8_swiglu_mx_cast(const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out, int fmt, uint8_t *out,
@@ -557,6 +558,11 @@ int odl_fp8_swiglu_mx_cast(const void *gate, const void *up, int64_t rows, int64
 int odl_fp8_swiglu_bwd_mx_cast(const void *dh, const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out,
                                int fmt, uint8_t *dg, uint8_t *dg_scales, uint8_t *dg_t, uint8_t *dg_scales_t, uint8_t *du,
                                uint8_t *du_scales, uint8_t *du_t, uint8_t *du_scales_t, int scale_rule, odl_stream_t stream);
+int odl_fp8_swiglu_block_cast(const void *gate, const void *up, int64_t rows, int64_t cols, int fmt, int margin, uint8_t *out,
+                              uint8_t *scales, uint8_t *out_t, uint8_t *scales_t, odl_stream_t stream);
+int odl_fp8_swiglu_bwd_block_cast(const void *dh, const void *gate, const void *up, int64_t rows, int64_t cols, int fmt, int margin,
+                                  uint8_t *dg, uint8_t *dg_scales, uint8_t *dg_t, uint8_t *dg_scales_t, uint8_t *du,
+                                  uint8_t *du_scales, uint8_t *du_t, uint8_t *du_scales_t, odl_stream_t stream);
 int odl_fp8_swiglu_cast_delayed(const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out, const float *scale,
                                 int fmt, uint8_t *out, uint8_t *out_t, float *amax_parts, float *scale_inv, odl_stream_t stream);
 int odl_fp8_swiglu_bwd_cast_delayed(const void *dh, const void *gate, const void *up, int64_t rows, int64_t cols, int64_t rows_out,

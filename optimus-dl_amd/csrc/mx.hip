@@ -442,40 +442,42 @@ __device__ __forceinline__ int block_lds_off(int col, int dw) {
 // neighbouring 16-byte pieces leaves every instruction a half (quarter) of each 64-byte request (a read-only loop over
 // 8192 x 14336 bf16 measured 5.1 TB/s that way against 6.2 TB/s with contiguous instructions).  TWO_D: one scale for the whole tile (weights); else one per row of the tile for the row-major
 // codes and one per column for the transposed codes.  rows, cols multiples of 128.
-template <int SRC, int FMT, bool TWO_D, bool WANT_ROW, bool WANT_COL>
-__global__ __launch_bounds__(256, SRC == ODL_BF16 ? 8 : 4) void block_cast_kernel(const void *__restrict__ x, int64_t rows, int64_t cols, int margin,
-                                                         uint8_t *__restrict__ out, uint32_t *__restrict__ scales,
-                                                         uint8_t *__restrict__ out_t, uint32_t *__restrict__ scales_t) {
-    __shared__ __attribute__((aligned(16))) uint8_t tile[WANT_COL ? 128 * 128 : 16];
+struct BlockOut {
+    uint8_t *out;
+    uint32_t *scales;
+    uint8_t *out_t;
+    uint32_t *scales_t;
+};
+
+template <bool WANT_COL>
+struct BlockShared {
+    __attribute__((aligned(16))) uint8_t tile[WANT_COL ? 128 * 128 : 16];
     // red and col_e8 hold one value per column at block_col_slot(column): every 32 columns sit four dwords further on.
     // The 8-byte write of the column maxima is served 16 lanes at a time over 32 banks (measured: with the 8 lanes tx
     // on dwords 8 tx + j, lanes tx and tx + 4 met, 4 conflict cycles per wave); with the pitch the 16 lanes (8 tx, two
     // neighbouring column pairs each) cover 32 consecutive dwords.  The 16-byte reads of col_e8 stay on 32 different banks.
-    __shared__ __attribute__((aligned(16))) uint32_t red[4][144];       // per wave: column maxima (1-D), or slot 0: the wave's maximum (2-D)
-    __shared__ __attribute__((aligned(16))) float col_e8[144];          // per column: its E8M0 byte where a float keeps its exponent
-    __shared__ int odd_tile;                                       // 1-D blocks: some column of the tile holds Inf / NaN
-    __shared__ uint32_t row_dw[128];                               // 1-D blocks, both outputs: the scale dwords of the tile's rows
-    saturate_fp8_conversions();
+    __attribute__((aligned(16))) uint32_t red[4][144];       // per wave: column maxima (1-D), or slot 0: the wave's maximum (2-D)
+    __attribute__((aligned(16))) float col_e8[144];          // per column: its E8M0 byte where a float keeps its exponent
+    int odd_tile;                                            // 1-D blocks: some column of the tile holds Inf / NaN
+    uint32_t row_dw[128];                                    // 1-D blocks, both outputs: the scale dwords of the tile's rows
+};
+
+// One tile of which every lane holds its patch: raw[i] is row 4 ty + i, the groups of 4 columns in the order of group_col.
+template <int SRC, int FMT, bool TWO_D, bool WANT_ROW, bool WANT_COL>
+__device__ __forceinline__ void block_cast_tile(const uint32_t (&raw)[4][SRC == ODL_BF16 ? 8 : 16], int64_t tr, int64_t tc, int64_t rows, int64_t cols,
+                                                int margin, const BlockOut &o, BlockShared<WANT_COL> &lds) {
+    uint8_t *__restrict__ out = o.out, *__restrict__ out_t = o.out_t;
+    uint32_t *__restrict__ scales = o.scales, *__restrict__ scales_t = o.scales_t;
+    auto &tile = lds.tile;
+    auto &red = lds.red;
+    auto &col_e8 = lds.col_e8;
+    auto &odd_tile = lds.odd_tile;
+    auto &row_dw = lds.row_dw;
     constexpr int ESZ = SRC == ODL_BF16 ? 2 : 4, DW = 16 * ESZ / 4;
     const int tx = threadIdx.x % 8, ty = threadIdx.x / 8, wave = threadIdx.x / 64;
-    const int64_t tiles_r = rows / 128, tiles_c = cols / 128;
-    int64_t tr, tc;
-    ct_tile_of(blockIdx.x, tiles_r, tiles_c, tr, tc);
     const int64_t r0 = tr * 128 + ty * 4;
     // first tile column of the lane's group g of 4 columns; raw[i] holds the groups in this order
     auto group_col = [&](int g) { return SRC == ODL_BF16 ? 8 * tx + 4 * (g & 1) + 64 * (g >> 1) : 4 * tx + 32 * g; };
-
-    uint32_t raw[4][DW];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const char *row = reinterpret_cast<const char *>(x) + ((r0 + i) * cols + tc * 128) * ESZ;
-#pragma unroll
-        for (int h = 0; h < DW / 4; ++h) {
-            const int byte = 16 * tx + 128 * h;
-            const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(row + byte));
-            raw[i][4 * h] = v.x; raw[i][4 * h + 1] = v.y; raw[i][4 * h + 2] = v.z; raw[i][4 * h + 3] = v.w;
-        }
-    }
     auto widen4 = [&](int i, int g, float (&f)[4]) {            // the lane's column group g of row i
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -648,6 +650,68 @@ __global__ __launch_bounds__(256, SRC == ODL_BF16 ? 8 : 4) void block_cast_kerne
             const u32x4 v = *reinterpret_cast<const u32x4 *>(&tile[block_lds_off(col, 4 * m16)]);
             __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(out_t + (tc * 128 + col) * rows + tr * 128 + m16 * 16));
         }
+    }
+}
+
+template <int SRC, int FMT, bool TWO_D, bool WANT_ROW, bool WANT_COL>
+__global__ __launch_bounds__(256, SRC == ODL_BF16 ? 8 : 4) void block_cast_kernel(const void *__restrict__ x, int64_t rows, int64_t cols, int margin,
+                                                                                   BlockOut o) {
+    __shared__ BlockShared<WANT_COL> lds;
+    saturate_fp8_conversions();
+    constexpr int ESZ = SRC == ODL_BF16 ? 2 : 4, DW = 16 * ESZ / 4;
+    const int tx = threadIdx.x % 8, ty = threadIdx.x / 8;
+    int64_t tr, tc;
+    ct_tile_of(blockIdx.x, rows / 128, cols / 128, tr, tc);
+    uint32_t raw[4][DW];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const char *row = reinterpret_cast<const char *>(x) + ((tr * 128 + ty * 4 + i) * cols + tc * 128) * ESZ;
+#pragma unroll
+        for (int h = 0; h < DW / 4; ++h) {
+            const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(row + 16 * tx + 128 * h));
+            raw[i][4 * h] = v.x; raw[i][4 * h + 1] = v.y; raw[i][4 * h + 2] = v.z; raw[i][4 * h + 3] = v.w;
+        }
+    }
+    block_cast_tile<SRC, FMT, TWO_D, WANT_ROW, WANT_COL>(raw, tr, tc, rows, cols, margin, o, lds);
+}
+
+// The same of h = silu(gate) * up, and of d_gate and d_up, without the bf16 tensors in between (1-D blocks, both layouts).
+// HBM-bound: 4 + 2 and 6 + 4 bytes an element, where a producer and the casts behind it move 10 and 18.  Measured, the
+// separate launches against this one: 8192 x 14336 h 233 -> 158 us, gradients 397 -> 214 us; 1024 x 5632 21 -> 15.5 and
+// 32 -> 21.6 us.
+template <int FMT, bool BWD>
+__global__ __launch_bounds__(256, 4) void swiglu_block_cast_kernel(const uint8_t *__restrict__ dh, const uint8_t *__restrict__ gate,
+                                                                             const uint8_t *__restrict__ up, int64_t rows, int64_t cols, int margin,
+                                                                             BlockOut first, BlockOut second) {
+    __shared__ BlockShared<true> lds;
+    saturate_fp8_conversions();
+    const int tx = threadIdx.x % 8, ty = threadIdx.x / 8;
+    int64_t tr, tc;
+    ct_tile_of(blockIdx.x, rows / 128, cols / 128, tr, tc);
+    uint32_t a[4][8], b[4][8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int64_t at = ((tr * 128 + ty * 4 + i) * cols + tc * 128) * 2 + 16 * tx + 128 * h;
+            const u32x4 g = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(gate + at)), u = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(up + at));
+            u32x4 v, w = {0, 0, 0, 0};
+            if constexpr (BWD) swiglu_bwd8(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(dh + at)), g, u, v, w);
+            else v = swiglu_fwd8(g, u);
+            a[i][4 * h] = v.x; a[i][4 * h + 1] = v.y; a[i][4 * h + 2] = v.z; a[i][4 * h + 3] = v.w;
+            b[i][4 * h] = w.x; b[i][4 * h + 1] = w.y; b[i][4 * h + 2] = w.z; b[i][4 * h + 3] = w.w;
+            // Opaque from here: the compiler otherwise keeps the halves of the packed pairs apart, two registers a pair, and
+            // spills (560 bytes a lane for the gradients).
+#pragma unroll
+            for (int d = 4 * h; d < 4 * h + 4; ++d) {
+                asm volatile("" : "+v"(a[i][d]));
+                if constexpr (BWD) asm volatile("" : "+v"(b[i][d]));
+            }
+        }
+    block_cast_tile<ODL_BF16, FMT, false, true, true>(a, tr, tc, rows, cols, margin, first, lds);
+    if constexpr (BWD) {
+        __syncthreads();                   // the tile's LDS is reused
+        block_cast_tile<ODL_BF16, FMT, false, true, true>(b, tr, tc, rows, cols, margin, second, lds);
     }
 }
 
@@ -924,8 +988,8 @@ template <int SRC, int FMT, bool TWO_D>
 static void launch_block_cast(const void *x, int64_t rows, int64_t cols, int margin, uint8_t *out, uint8_t *scales, uint8_t *out_t,
                               uint8_t *scales_t, hipStream_t stream) {
     const dim3 grid((unsigned)((rows / 128) * (cols / 128))), block(256);
-    uint32_t *s = reinterpret_cast<uint32_t *>(scales), *st = reinterpret_cast<uint32_t *>(scales_t);
-#define ODL_BLK(R, C) hipLaunchKernelGGL((block_cast_kernel<SRC, FMT, TWO_D, R, C>), grid, block, 0, stream, x, rows, cols, margin, out, s, out_t, st)
+    const BlockOut o = {out, reinterpret_cast<uint32_t *>(scales), out_t, reinterpret_cast<uint32_t *>(scales_t)};
+#define ODL_BLK(R, C) hipLaunchKernelGGL((block_cast_kernel<SRC, FMT, TWO_D, R, C>), grid, block, 0, stream, x, rows, cols, margin, o)
     if (out && out_t) ODL_BLK(true, true);
     else if (out) ODL_BLK(true, false);
     else ODL_BLK(false, true);
@@ -1019,6 +1083,42 @@ extern "C" int odl_fp8_swiglu_bwd_mx_cast(const void *dh, const void *gate, cons
     if (fmt == ODL_FP8_E4M3) hipLaunchKernelGGL((swiglu_bwd_mx_cast_kernel<ODL_FP8_E4M3>), grid, block, 0, stream, d, g, u, rows, cols, og, ou, scale_rule, rows_out);
     else hipLaunchKernelGGL((swiglu_bwd_mx_cast_kernel<ODL_FP8_E5M2>), grid, block, 0, stream, d, g, u, rows, cols, og, ou, scale_rule, rows_out);
     return check_launch("odl_fp8_swiglu_bwd_mx_cast");
+}
+
+static int swiglu_block_cast(const char *who, bool bwd, const void *dh, const void *gate, const void *up, int64_t rows, int64_t cols, int fmt, int margin,
+                             const BlockOut &a, const BlockOut &b, hipStream_t stream) {
+    if (rows < 0 || cols < 0) return set_error(ODL_ERR_ARG, "%s: negative shape", who);
+    if (fmt != ODL_FP8_E4M3 && fmt != ODL_FP8_E5M2) return set_error(ODL_ERR_ARG, "%s: fmt %d", who, fmt);
+    if (margin < -64 || margin > 64) return set_error(ODL_ERR_ARG, "%s: margin %d", who, margin);
+    if (rows % 128 != 0 || cols % 128 != 0) return set_error(ODL_ERR_SHAPE, "%s: %lld x %lld: both sizes must be multiples of 128", who, (long long)rows, (long long)cols);
+    if ((rows / 128) * (cols / 128) > 0x7fffffffLL) return set_error(ODL_ERR_SHAPE, "%s: too many tiles for one launch", who);
+    if (rows == 0 || cols == 0) return ODL_OK;
+    for (const void *p : {bwd ? dh : gate, gate, up, (const void *)a.out, (const void *)a.scales, (const void *)a.out_t, (const void *)a.scales_t, (const void *)b.out,
+                          (const void *)b.scales, (const void *)b.out_t, (const void *)b.scales_t}) {
+        if (!p) return set_error(ODL_ERR_ARG, "%s: null pointer", who);
+        if (reinterpret_cast<uintptr_t>(p) & 15) return set_error(ODL_ERR_SHAPE, "%s: every pointer must be 16-byte aligned", who);
+    }
+    const dim3 grid((unsigned)((rows / 128) * (cols / 128))), block(256);
+    const uint8_t *d = static_cast<const uint8_t *>(dh), *g = static_cast<const uint8_t *>(gate), *u = static_cast<const uint8_t *>(up);
+#define ODL_SB(F, B) hipLaunchKernelGGL((swiglu_block_cast_kernel<F, B>), grid, block, 0, stream, d, g, u, rows, cols, margin, a, b)
+    if (fmt == ODL_FP8_E4M3) { if (bwd) ODL_SB(ODL_FP8_E4M3, true); else ODL_SB(ODL_FP8_E4M3, false); }
+    else { if (bwd) ODL_SB(ODL_FP8_E5M2, true); else ODL_SB(ODL_FP8_E5M2, false); }
+#undef ODL_SB
+    return check_launch(who);
+}
+
+extern "C" int odl_fp8_swiglu_block_cast(const void *gate, const void *up, int64_t rows, int64_t cols, int fmt, int margin, uint8_t *out, uint8_t *scales,
+                                         uint8_t *out_t, uint8_t *scales_t, odl_stream_t stream_) {
+    const BlockOut o = {out, reinterpret_cast<uint32_t *>(scales), out_t, reinterpret_cast<uint32_t *>(scales_t)};
+    return swiglu_block_cast("odl_fp8_swiglu_block_cast", false, nullptr, gate, up, rows, cols, fmt, margin, o, o, reinterpret_cast<hipStream_t>(stream_));
+}
+
+extern "C" int odl_fp8_swiglu_bwd_block_cast(const void *dh, const void *gate, const void *up, int64_t rows, int64_t cols, int fmt, int margin, uint8_t *dg,
+                                             uint8_t *dg_scales, uint8_t *dg_t, uint8_t *dg_scales_t, uint8_t *du, uint8_t *du_scales, uint8_t *du_t,
+                                             uint8_t *du_scales_t, odl_stream_t stream_) {
+    const BlockOut a = {dg, reinterpret_cast<uint32_t *>(dg_scales), dg_t, reinterpret_cast<uint32_t *>(dg_scales_t)};
+    const BlockOut b = {du, reinterpret_cast<uint32_t *>(du_scales), du_t, reinterpret_cast<uint32_t *>(du_scales_t)};
+    return swiglu_block_cast("odl_fp8_swiglu_bwd_block_cast", true, dh, gate, up, rows, cols, fmt, margin, a, b, reinterpret_cast<hipStream_t>(stream_));
 }
 
 extern "C" int odl_fp8_mx_gemm_nt(const uint8_t *a, const uint8_t *sa, const uint8_t *b, const uint8_t *sb, int scales_layout, int64_t M,

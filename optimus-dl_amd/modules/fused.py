@@ -65,7 +65,8 @@ def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 
 # -------------------------------------------------------------- a whole SwiGLU MLP
 class _SwiGLUMLPFn(torch.autograd.Function):
-    """``c_proj(silu(w1 x) * w2 x)`` as one node, for the recipes that need no amax before they cast (delayed scaling, mxfp8).
+    """``c_proj(silu(w1 x) * w2 x)`` as one node, for the recipes that need no amax of the whole tensor before they cast (delayed
+    scaling, mxfp8, blockwise).
 
     The product and its gradients go from the registers of the kernel that computes them straight into codes: h, d_gate and
     d_up are never written in bf16.  Between separate nodes they have to be, since autograd hands tensors over.  Everything
@@ -91,6 +92,8 @@ class _SwiGLUMLPFn(torch.autograd.Function):
         gate, up = member(x2d, w1, weights[0], ctx.needs_input_grad[0]), member(x2d, w2, weights[1], ctx.needs_input_grad[0])
         if pol.kind == "mxfp8":
             h = native.swiglu_mx_cast(gate, up, pol.fmt_fwd, pol.mx_scale_rule)
+        elif pol.kind == "blockwise":
+            h = native.swiglu_block_cast(gate, up, pol.fmt_fwd, pol.margin)
         else:
             meta = down._meta(recipe, x2d.device, "fwd")
             meta.note_record(recipe._store)
@@ -111,6 +114,8 @@ class _SwiGLUMLPFn(torch.autograd.Function):
         mods = (sub_g.module, sub_u.module)
         if pol.kind == "mxfp8":
             given = native.swiglu_bwd_mx_cast(dh, gate, up, pol.fmt_bwd, pol.mx_scale_rule)
+        elif pol.kind == "blockwise":
+            given = native.swiglu_bwd_block_cast(dh, gate, up, pol.fmt_bwd, pol.margin)
         elif all(m.training for m in mods):
             metas = [m._meta(recipe, dh.device, "bwd") for m in mods]
             for meta in metas:
@@ -157,7 +162,7 @@ def swiglu_mlp(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
     casts with the amax of the tensor itself, no graph, biases, hooks, a Linear switched off or in eval mode, sizes that
     the kernels do not take, weight gradients that are not FP8 or go straight into ``.grad``."""
     recipe = _state.active_recipe()
-    if recipe is None or recipe.recipe.kind not in ("delayed", "mxfp8") or _any_global_hook is None or _any_global_hook():
+    if recipe is None or recipe.recipe.kind not in ("delayed", "mxfp8", "blockwise") or _any_global_hook is None or _any_global_hook():
         return None
     if not torch.is_grad_enabled() or not x.requires_grad or not recipe.wgrad or recipe.fuse_wgrad_accumulation or not recipe.fuse_dgrad_sum:
         return None
@@ -172,8 +177,9 @@ def swiglu_mlp(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
         return None
     if not (w1._fp8_eligible(x) and w2._fp8_eligible(x)) or not down.weight.is_cuda or down.weight.dtype not in (torch.bfloat16, torch.float32):
         return None
-    mx = recipe.recipe.kind == "mxfp8"
-    if hidden % (128 if mx else 16) or down.out_features % (32 if mx else 16) or not (mx or all(m.training for m in mods)):
+    delayed = recipe.recipe.kind == "delayed"
+    out_mult = {"delayed": 16, "mxfp8": 32, "blockwise": 128}[recipe.recipe.kind]
+    if hidden % (16 if delayed else 128) or down.out_features % out_mult or (delayed and not all(m.training for m in mods)):
         return None
     x2d = x.reshape(-1, w1.in_features)
     if x2d.dtype != torch.bfloat16 or not x2d.is_contiguous():

@@ -25,7 +25,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 21
+ABI_VERSION = 22
 _OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
@@ -82,6 +82,8 @@ EXPORTS = (
     "odl_fp8_mx_cast_padded",
     "odl_fp8_swiglu_mx_cast",
     "odl_fp8_swiglu_bwd_mx_cast",
+    "odl_fp8_swiglu_block_cast",
+    "odl_fp8_swiglu_bwd_block_cast",
     "odl_fp8_swiglu_cast_delayed",
     "odl_fp8_swiglu_bwd_cast_delayed",
     "odl_fp8_mx_gemm_nt",
@@ -168,6 +170,8 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_gemm_set_clock_probe.argtypes = [vp, i32]
         L.odl_fp8_swiglu_mx_cast.argtypes = [vp, vp, i64, i64, i64, i32, vp, vp, vp, vp, i32, vp]
         L.odl_fp8_swiglu_bwd_mx_cast.argtypes = [vp, vp, vp, i64, i64, i64, i32, vp, vp, vp, vp, vp, vp, vp, vp, i32, vp]
+        L.odl_fp8_swiglu_block_cast.argtypes = [vp, vp, i64, i64, i32, i32, vp, vp, vp, vp, vp]
+        L.odl_fp8_swiglu_bwd_block_cast.argtypes = [vp, vp, vp, i64, i64, i32, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp]
         L.odl_fp8_swiglu_cast_delayed.argtypes = [vp, vp, i64, i64, i64, vp, i32, vp, vp, vp, vp, vp]
         L.odl_fp8_swiglu_bwd_cast_delayed.argtypes = [vp, vp, vp, i64, i64, i64, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
         L.odl_fp8_mx_cast_padded.argtypes = [vp, i32, i64, i64, i64, i32, vp, vp, i32, vp, vp, i32, i32, vp]
@@ -1056,6 +1060,26 @@ def swiglu_bwd_mx_cast(dh: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, f
     dg, du = _mx_pair(rows, cols, n, gate.device), _mx_pair(rows, cols, n, gate.device)
     _check(load().odl_fp8_swiglu_bwd_mx_cast(dh.data_ptr(), gate.data_ptr(), up.data_ptr(), rows, cols, n, fmt,
                                              *[t.data_ptr() for t in dg + du], scale_rule, _stream()), "odl_fp8_swiglu_bwd_mx_cast")
+    return dg, du
+
+
+def swiglu_block_cast(gate: torch.Tensor, up: torch.Tensor, fmt: int, margin: int = 0):
+    """``block_cast`` of silu(gate) * up (1-D blocks, both layouts) without writing the product.  rows, cols % 128 == 0."""
+    gate, up = _swiglu_sources((gate, up), "swiglu_block_cast")
+    rows, cols = gate.shape
+    h = _mx_pair(rows, cols, rows, gate.device)
+    _check(load().odl_fp8_swiglu_block_cast(gate.data_ptr(), up.data_ptr(), rows, cols, fmt, margin, *[t.data_ptr() for t in h], _stream()),
+           "odl_fp8_swiglu_block_cast")
+    return h
+
+
+def swiglu_bwd_block_cast(dh: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, fmt: int, margin: int = 0):
+    """The same of the gradients of silu(gate) * up.  -> (what :func:`swiglu_block_cast` returns) for d_gate, and for d_up."""
+    dh, gate, up = _swiglu_sources((dh, gate, up), "swiglu_bwd_block_cast")
+    rows, cols = gate.shape
+    dg, du = _mx_pair(rows, cols, rows, gate.device), _mx_pair(rows, cols, rows, gate.device)
+    _check(load().odl_fp8_swiglu_bwd_block_cast(dh.data_ptr(), gate.data_ptr(), up.data_ptr(), rows, cols, fmt, margin,
+                                                *[t.data_ptr() for t in dg + du], _stream()), "odl_fp8_swiglu_bwd_block_cast")
     return dg, du
 
 

@@ -64,6 +64,21 @@ def test_block_cast_one_dimensional_blocks_bit_exact(N, shape, fmt, dtype):
     assert_bytes_equal(_bytes(sc), ts, "scale bytes (torch restatement)")
 
 
+@pytest.mark.parametrize("shape", [(128, 128), (384, 512), (2048, 256)])
+@pytest.mark.parametrize("fmt", [E4M3, E5M2])
+def test_swiglu_straight_to_block_codes(N, shape, fmt):
+    """Bit for bit the bf16 results of the SwiGLU kernels and their cast, also of tiles that hold Inf and NaN."""
+    gate, up, dh = (_mixed(shape, seed=s).clamp(-1e15, 1e15).cuda() for s in (1, 2, 3))
+    gate[-1, -3], up[3, 1], dh[-1, 5] = float("nan"), float("inf"), -float("inf")
+    for margin in (0, 2):
+        pairs = [(N.swiglu_block_cast(gate, up, fmt, margin), N.swiglu_amax_parts(gate, up)[0])]
+        dg, du = N.swiglu_bwd_amax_parts(dh, gate, up)[:2]
+        pairs += list(zip(N.swiglu_bwd_block_cast(dh, gate, up, fmt, margin), (dg, du)))
+        for k, (got, plain) in enumerate(pairs):
+            for a, b, what in zip(got, N.block_cast(plain, fmt, margin, False, True, True), ("codes", "scales", "codes_t", "scales_t")):
+                assert_bytes_equal(a, b, f"{what} of result {k}, {shape} fmt {fmt} margin {margin}")
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("fmt", [E4M3, E5M2])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

@@ -441,7 +441,7 @@ def test_inference_mode_forward_equals_the_no_grad_forward(amp, fuse):
 
 
 @pytest.mark.parametrize("tokens,width,hidden", [(32, 128, 256), (160, 192, 384), (1056, 256, 640), (2048, 1024, 4096)])
-@pytest.mark.parametrize("kind", ["delayed", "mxfp8"])
+@pytest.mark.parametrize("kind", ["delayed", "mxfp8", "blockwise"])
 def test_whole_mlp_node_changes_no_bit(amp, monkeypatch, kind, tokens, width, hidden):
     """SwiGLU straight to codes against the same MLP as separate nodes, over steps that move the delayed scales: outputs, all
     gradients, histories.  The sizes end inside tiles and K steps; the last one takes wgrad from dY as stored and dX from one GEMM."""
@@ -449,6 +449,8 @@ def test_whole_mlp_node_changes_no_bit(amp, monkeypatch, kind, tokens, width, hi
     from optimus_dl_amd.modules.model.blocks import SwiGLUMLP
     from optimus_dl_amd.modules.model_transforms import build_model_transform
 
+    if kind == "blockwise":                       # whole blocks of 128 only
+        tokens, width = (tokens + 127) // 128 * 128, (width + 127) // 128 * 128
     nodes = []
     real = fused.swiglu_mlp
     results = {}
