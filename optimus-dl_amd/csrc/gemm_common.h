@@ -302,10 +302,10 @@ void launch_gemm_tiled(int variant, int fa, int fb, const GemmArgs &g, hipStream
 int gemm_thin_rows(int64_t M, int64_t N, int num_cus);
 void launch_gemm_thin(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
 // the kernel for outputs of few tiles (gemm_fp8.hip); operands under 2 GiB each, K % 128 == 0
-enum FewTiles { kManyTiles, kTwoBlocks, kDeepWide, kDeep };
+enum FewTiles { kManyTiles, kTwoBlocks, kDeepWide, kDeep192, kDeep };
 FewTiles gemm_few_tiles(int64_t M, int64_t N, int64_t K, int num_cus);
-// wide: 256 x 128 tiles, else 128 x 128
-void launch_gemm_deep(bool wide, int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
+// bm x bn: 128 x 128, 128 x 192 or 256 x 128
+void launch_gemm_deep(int bm, int bn, int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
 void launch_gemm_pipe(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
 bool gemm_stream_accepts(const GemmArgs &g);
 void launch_gemm_stream(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);

@@ -1,4 +1,4 @@
-// FP8 GEMM for outputs of about one tile per compute unit: 256 x 128 or 128 x 128 tiles, four waves, three LDS stages,
+// FP8 GEMM for outputs of about one tile per compute unit: 256 x 128, 128 x 192 or 128 x 128 tiles, four waves, three LDS stages,
 // explicit software pipeline.  Both operands K-contiguous, K % 128 == 0, any M and N, every scale form (block scales
 // K-step-major), `accumulate`.
 //
@@ -6,11 +6,14 @@
 // bytes a cycle, for 512 cycles of MFMA; of a 256 x 128 tile 96 + 48 KB, 1152 cycles for 1024.  With the whole chip busy
 // the caches come into it: 18 - 20 TB/s of operand panels is the most they were seen to deliver.  Measured per K step
 // (slope over K = 2048 .. 8192): 128 x 128 0.29 us (705 cycles) with 24 units busy, 0.35 with 192, 0.40 with 256; 256 x 128
-// 0.52 and 0.71.  A launch costs 5.5 - 7 us beside its steps.
+// 0.52 and 0.71.  A launch costs 5.5 - 7 us beside its steps.  128 x 192 tiles lie between: 0.66 us with 256 units busy and
+// operands from HBM, which is what 40 KB a step take there (see warm_operands; nobody is left to warm).  They fill the
+// chip where 256 x 128 tiles leave a quarter of it idle: 8192 x 768 x 3072 26.1 -> 24.4 us, x 50304 327 -> 285.  (256 x 192 in two
+// stages does not fit the registers: 2.7 us a step.)
 //
 // A block that has a compute unit to itself has nobody to hide its waits behind, so nothing here waits for what was
 // asked for recently:
-//   * a wave tile is 64 x 64 or 128 x 64, four waves: with eight waves of 64 x 32 LDS would deliver half as much again;
+//   * a wave tile is 64 x 64, 64 x 96 or 128 x 64, four waves: with eight waves of 64 x 32 LDS would deliver half as much again;
 //   * the fragments of step kt + 1 (both halves) stream from LDS into one set of registers while the MFMAs of step kt
 //     work on the other.  Half a step ahead, as the 256 x 256 kernels do it, is 256 cycles of MFMA here and less than
 //     LDS takes (0.39 us a step instead of 0.29);
@@ -43,7 +46,7 @@ __global__ __launch_bounds__(256) void gemm_nt_deep_kernel(const GemmArgs g) {
     constexpr int BM = 64 * TM, BN = 64 * TN, WM = 32 * TM, WN = 32 * TN;
     constexpr int A_BYTES = BM * 128, CODES = (BM + BN) * 128, STAGE = CODES + (MX ? (BM + BN + 255) / 256 * 1024 : 0);
     constexpr int LA = BM / 32, LB = BN / 32, SC = MX ? (BM + BN + 255) / 256 : 0, PER = LA + LB + SC;         // direct-to-LDS loads per wave and step
-    constexpr int MFMAS = TM * TN;
+    constexpr int MFMAS = TM * TN, TNS = TN % 2 ? 1 : TN;             // TNS: sub-tiles of a row staged together
     constexpr int GM = BM == 256 ? 4 : 8;                             // tile rows walked together
     static_assert(PER * (STAGES - 1) <= 63, "the counter holds 63 loads");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[STAGES * STAGE];
@@ -212,8 +215,8 @@ __global__ __launch_bounds__(256) void gemm_nt_deep_kernel(const GemmArgs g) {
         if (g.accumulate) {
             if (g.out_dtype == ODL_BF16) epilogue_staged_accumulate<true, TM, TN, 1, true>(g, acc, wave_lds, m0 + wm0, n0 + wn0, lane);
             else epilogue_staged_accumulate<false, TM, TN, 1, true>(g, acc, wave_lds, m0 + wm0, n0 + wn0, lane);
-        } else if (g.out_dtype == ODL_BF16) epilogue_staged<true, TM, TN, TN, true>(g, acc, wave_lds, m0 + wm0, n0 + wn0, lane);
-        else epilogue_staged<false, TM, TN, TN, true>(g, acc, wave_lds, m0 + wm0, n0 + wn0, lane);
+        } else if (g.out_dtype == ODL_BF16) epilogue_staged<true, TM, TN, TNS, true>(g, acc, wave_lds, m0 + wm0, n0 + wn0, lane);
+        else epilogue_staged<false, TM, TN, TNS, true>(g, acc, wave_lds, m0 + wm0, n0 + wn0, lane);
     } else {
 #pragma unroll
         for (int t = 0; t < TM; ++t)
@@ -225,27 +228,29 @@ __global__ __launch_bounds__(256) void gemm_nt_deep_kernel(const GemmArgs g) {
     }
 }
 
-template <int FA, int FB>
-void launch_deep_fmt(bool wide, const GemmArgs &g, int num_cus, hipStream_t stream) {
+template <int FA, int FB, bool MX>
+void launch_deep_tile(int bm, int bn, const GemmArgs &g, int num_cus, hipStream_t stream) {
     const int total = g.tiles_m * g.tiles_n;
     const int whole = (total + 7) / 8 * 8;                // a multiple of 8, as is the launch: see the placement in the kernel
     const dim3 grid((unsigned)(whole < num_cus && warming_pays(g) ? num_cus : whole)), block(256);
-    if (g.mx_sa) {
-        if (wide) hipLaunchKernelGGL((gemm_nt_deep_kernel<4, 2, FA, FB, true>), grid, block, 0, stream, g);
-        else hipLaunchKernelGGL((gemm_nt_deep_kernel<2, 2, FA, FB, true>), grid, block, 0, stream, g);
-    } else {
-        if (wide) hipLaunchKernelGGL((gemm_nt_deep_kernel<4, 2, FA, FB, false>), grid, block, 0, stream, g);
-        else hipLaunchKernelGGL((gemm_nt_deep_kernel<2, 2, FA, FB, false>), grid, block, 0, stream, g);
-    }
+    if (bm == 128 && bn == 128) hipLaunchKernelGGL((gemm_nt_deep_kernel<2, 2, FA, FB, MX>), grid, block, 0, stream, g);
+    else if (bm == 128) hipLaunchKernelGGL((gemm_nt_deep_kernel<2, 3, FA, FB, MX>), grid, block, 0, stream, g);
+    else hipLaunchKernelGGL((gemm_nt_deep_kernel<4, 2, FA, FB, MX>), grid, block, 0, stream, g);
+}
+
+template <int FA, int FB>
+void launch_deep_fmt(int bm, int bn, const GemmArgs &g, int num_cus, hipStream_t stream) {
+    if (g.mx_sa) launch_deep_tile<FA, FB, true>(bm, bn, g, num_cus, stream);
+    else launch_deep_tile<FA, FB, false>(bm, bn, g, num_cus, stream);
 }
 
 }  // namespace
 
-void launch_gemm_deep(bool wide, int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream) {
-    if (fa == ODL_FP8_E4M3 && fb == ODL_FP8_E4M3) launch_deep_fmt<ODL_FP8_E4M3, ODL_FP8_E4M3>(wide, g, num_cus, stream);
-    else if (fa == ODL_FP8_E5M2 && fb == ODL_FP8_E4M3) launch_deep_fmt<ODL_FP8_E5M2, ODL_FP8_E4M3>(wide, g, num_cus, stream);
-    else if (fa == ODL_FP8_E4M3 && fb == ODL_FP8_E5M2) launch_deep_fmt<ODL_FP8_E4M3, ODL_FP8_E5M2>(wide, g, num_cus, stream);
-    else launch_deep_fmt<ODL_FP8_E5M2, ODL_FP8_E5M2>(wide, g, num_cus, stream);
+void launch_gemm_deep(int bm, int bn, int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream) {
+    if (fa == ODL_FP8_E4M3 && fb == ODL_FP8_E4M3) launch_deep_fmt<ODL_FP8_E4M3, ODL_FP8_E4M3>(bm, bn, g, num_cus, stream);
+    else if (fa == ODL_FP8_E5M2 && fb == ODL_FP8_E4M3) launch_deep_fmt<ODL_FP8_E5M2, ODL_FP8_E4M3>(bm, bn, g, num_cus, stream);
+    else if (fa == ODL_FP8_E4M3 && fb == ODL_FP8_E5M2) launch_deep_fmt<ODL_FP8_E4M3, ODL_FP8_E5M2>(bm, bn, g, num_cus, stream);
+    else launch_deep_fmt<ODL_FP8_E5M2, ODL_FP8_E5M2>(bm, bn, g, num_cus, stream);
 }
 
 }  // namespace odl

@@ -103,8 +103,9 @@ static const Variant kVariants[] = {
     {"thin tiles, 8 waves sharing K (N % 4 == 0, K % 128 == 0)", 64, 64, 512, 0.0f},
     {"256x128x128 4 waves (128x64 per wave), three stages, software-pipelined", 256, 128, 256, 0.0f},
     {"128x128x128 4 waves (64x64 per wave), three stages, software-pipelined", 128, 128, 256, 0.0f},
+    {"128x192x128 4 waves (64x96 per wave), three stages, software-pipelined", 128, 192, 256, 0.0f},
 };
-constexpr int kPipeVariant = 5, kPipeOneTileVariant = 6, kStreamVariant = 7, kThinVariant = 8, kDeepWideVariant = 9, kDeepVariant = 10;
+constexpr int kPipeVariant = 5, kPipeOneTileVariant = 6, kStreamVariant = 7, kThinVariant = 8, kDeepWideVariant = 9, kDeepVariant = 10, kDeep192Variant = 11;
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 // Forced kernel variant of the calling host thread (-1: choose by shape).  Thread-local: a test or a tuning
 // sweep that pins a variant cannot change the kernels another thread (e.g. the autograd worker) launches.
@@ -142,13 +143,16 @@ static bool thin_pays(int64_t M, int64_t N, int64_t K) {
 }
 
 // The kernel for an output of at most num_cus / 2 tiles of 256 x 256, which the big tiles would leave half the chip idle on
-// (kManyTiles: the output has more).  At most one 128 x 128 tile per unit: the pipelined kernel of gemm_deep.hip.  More: 256 x
-// 128 tiles of the same kernel, one per unit, from 24 K steps on (2048 x 4096 x 8192 52.9 us against 60.5 with two 128 x 128
+// (kManyTiles: the output has more).  At most one 128 x 128 tile per unit: the pipelined kernel of gemm_deep.hip.  At most one of
+// 128 x 192 and 8 K steps or more: those (against the better of the other two, cold operands: 8192 x 768 x 2048 19.1 -> 17.0 us, x 16384
+// 104 -> 93.8; 3072 x 1536 x 4096 fp32 27.0 -> 23.8; 5120 x 1152 x 1024 13.2 -> 12.4; but 3072 x 1920 x 768 9.6 -> 9.8, 8192 x 768 x 512 8.4
+// -> 8.7, where two blocks per unit hide each other's ends).  More: 256 x 128 tiles of the same kernel, one per unit, from 24 K steps on (2048 x 4096 x 8192 52.9 us against 60.5 with two 128 x 128
 // blocks per unit, x 4096 30.3 against 32.4); with fewer steps the blocks that hide each other's fill and drain win (x 2048:
 // 18.0 against 18.4, x 1024 11.6 against 12.7).
 FewTiles gemm_few_tiles(int64_t M, int64_t N, int64_t K, int num_cus) {
     if (((M + 127) / 128) * ((N + 127) / 128) <= num_cus) return kDeep;
     if (((M + 255) / 256) * ((N + 255) / 256) * 2 > num_cus) return kManyTiles;
+    if (K >= 1024 && ((M + 127) / 128) * ((N + 191) / 192) <= num_cus) return kDeep192;
     return K >= 3072 && ((M + 255) / 256) * ((N + 127) / 128) <= num_cus ? kDeepWide : kTwoBlocks;
 }
 
@@ -156,7 +160,7 @@ FewTiles gemm_few_tiles(int64_t M, int64_t N, int64_t K, int num_cus) {
 static int few_tiles_variant(int64_t M, int64_t N, int64_t K, bool lim32) {
     const FewTiles few = gemm_few_tiles(M, N, K, cu_count());
     if (few == kManyTiles) return 0;
-    return few == kTwoBlocks || !lim32 ? 4 : few == kDeep ? kDeepVariant : kDeepWideVariant;
+    return few == kTwoBlocks || !lim32 ? 4 : few == kDeep ? kDeepVariant : few == kDeep192 ? kDeep192Variant : kDeepWideVariant;
 }
 
 static int choose_variant(int64_t M, int64_t N, int64_t K, bool stream_ok, bool lim32) {
@@ -183,7 +187,7 @@ static int choose_variant(int64_t M, int64_t N, int64_t K, bool stream_ok, bool 
 // per compute unit, and a last round of few tiles costs as much as a full one.  Those rows as 128 x 128 tiles take about half
 // a round with one tile per unit, 0.7 with two, and 4 us for the launch.  With one tile that pays from 16 K steps on
 // (5000 x 4096 x 2048: 47.8 -> 43.4 us, x 14336: 256 -> 216; 4096 x 4864 x 4096: 82.2 -> 68.8), with two from 32
-// (11264 x 2048 x 4096: 91.5 -> 86.2, 50304 x 768 x 8192: 292 -> 272; 4016 x 5632 x 2048 would go from 49.1 to 53.7).
+// (11264 x 2048 x 4096: 91.5 -> 86.2, 50304 x 768 x 8192: 290 -> 261; 4016 x 5632 x 2048 would go from 49.1 to 53.7).
 // Same K order, same bits.
 static int64_t tail_rows(int64_t M, int64_t N, int64_t K) {
     const int cus = cu_count();
@@ -256,7 +260,7 @@ static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_
     if ((variant == kPipeVariant || variant == kPipeOneTileVariant) && !pipe_ok) variant = 2;
 
     if (variant == kThinVariant && !thin_ok(M, N)) variant = 4;
-    if ((variant == kDeepVariant || variant == kDeepWideVariant) && !lim32) variant = 4;
+    if (variant >= kDeepWideVariant && !lim32) variant = 4;
 
     if (variant == kStreamVariant && t_forced_variant < 0 && launch_as < 0) {
         const int64_t rest = tail_rows(M, N, K), head = M - rest;
@@ -289,7 +293,7 @@ static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_
     }
     if (variant == 0) launch_gemm_generic(fmt_a, fmt_b, g, stream);
     else if (variant == kThinVariant) launch_gemm_thin(fmt_a, fmt_b, g, cu_count(), stream);
-    else if (variant == kDeepWideVariant || variant == kDeepVariant) launch_gemm_deep(variant == kDeepWideVariant, fmt_a, fmt_b, g, cu_count(), stream);
+    else if (variant >= kDeepWideVariant) launch_gemm_deep(bm, bn, fmt_a, fmt_b, g, cu_count(), stream);
     else if (variant == kPipeVariant) launch_gemm_pipe(fmt_a, fmt_b, g, cu_count(), stream);
     else if (variant == kPipeOneTileVariant) launch_gemm_pipe(fmt_a, fmt_b, g, 1 << 30, stream);
     else if (variant == kStreamVariant) { attach_clock_probe(g); launch_gemm_stream(fmt_a, fmt_b, g, cu_count(), stream); }
@@ -403,10 +407,12 @@ extern "C" int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t 
 //   one launch, 256 x 256 tiles : 0.92 us per K step of 128 (few compute units busy: high clock) + 3 steps of overhead
 //   one launch, smaller tiles   : what odl_fp8_gemm_nt takes for outputs of <= cus / 2 big tiles (few_tiles_variant).
 //                                 128 x 128 with a unit each 0.37 us per step + 6 us (3072 x 768 x 16384: 45 - 50 us, in
-//                                 six runs 52 and the reduction's launch); 256 x 128 with a unit each 0.70 + 7 (0.82 where the
-//                                 operands outgrow the 256 MB memory-side cache: 8192 x 768 x 50304 328 us); two 128 x 128
-//                                 blocks per unit 0.62 (it reads every operand panel twice as often)
+//                                 six runs 52 and the reduction's launch); 128 x 192 0.66 + 8; 256 x 128 with a unit each
+//                                 0.70 + 7; two 128 x 128 blocks per unit 0.62 (it reads every operand panel twice as often)
 //   split                       : 0.96 us per step of a run + 9 us (pipeline fill, the fp32 epilogue, the second launch)
+//   with operands that outgrow the 256 MB memory-side cache, per step 0.61 (128 x 128: 8192 x 512 x 50304 241 us, in three runs 234,
+//                                 in four 200), 0.71 (128 x 192: 8192 x 768 x 50304 285, in two runs 319), 0.88 (256 x 128: 8192 x 1024 x
+//                                 151936 1047, in two runs 961) and 1.45 (split)
 //                                 + the partial results, splits x M x N floats written and read back, at 2.7 TB/s in all
 //   each bounded below by its operand traffic (tiles x panel bytes) at about 12 TB/s out of the caches (the kernels of
 //   gemm_deep.hip: 18).
@@ -420,6 +426,7 @@ extern "C" int odl_fp8_gemm_split_count(int64_t M, int64_t N, int64_t K, int k_s
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
     const int cus = cu_count();
     const int64_t steps = K / 128;
+    const bool cold = (double)(M + N) * (double)K > 268435456.0;
     int64_t most = cus / tiles;
     if (most > 16) most = 16;
     const double traffic_us = (double)tiles * 512.0 * (double)K / 12.0e6;
@@ -429,8 +436,9 @@ extern "C" int odl_fp8_gemm_split_count(int64_t M, int64_t N, int64_t K, int k_s
         const int variant = few_tiles_variant(M, N, K, (double)(M + 256) * (double)K < 2147483648.0 && (double)(N + 256) * (double)K < 2147483648.0);
         const double panels = (double)((M + 127) / 128) * (double)((N + 127) / 128) * (double)K;         // of 128 rows, once per tile
         double small = whole, small_traffic_us = 0.0;
-        if (variant == kDeepVariant) { small = 0.37 * (double)steps + 6.0; small_traffic_us = panels * 256.0 / 18.0e6; }
-        else if (variant == kDeepWideVariant) { small = ((double)(M + N) * (double)K > 268435456.0 ? 0.82 : 0.70) * (double)steps + 7.0; small_traffic_us = panels * 192.0 / 18.0e6; }
+        if (variant == kDeepVariant) { small = (cold ? 0.61 : 0.37) * (double)steps + 6.0; small_traffic_us = panels * 256.0 / 18.0e6; }
+        else if (variant == kDeep192Variant) { small = (cold ? 0.71 : 0.66) * (double)steps + 8.0; small_traffic_us = panels * 213.4 / 18.0e6; }
+        else if (variant == kDeepWideVariant) { small = (cold ? 0.88 : 0.70) * (double)steps + 7.0; small_traffic_us = panels * 192.0 / 18.0e6; }
         else if (variant) { small = 0.62 * ((double)steps + 3.0); small_traffic_us = panels * 256.0 / 12.0e6; }
         if (small < small_traffic_us) small = small_traffic_us;
         if (small < whole) whole = small;
@@ -445,7 +453,7 @@ extern "C" int odl_fp8_gemm_split_count(int64_t M, int64_t N, int64_t K, int k_s
         const int64_t per = ((steps + splits - 1) / splits + 1) & ~(int64_t)1;
         const int64_t last = steps - (splits - 1) * per;
         if (per < 8 || last < 4) continue;
-        double run = 0.96 * (double)per + 9.0;
+        double run = (cold ? 1.45 : 0.96) * (double)per + 9.0;
         if (run < traffic_us) run = traffic_us;
         const double cost = run + (double)splits * (double)M * (double)N * 4.0 / 2.7e6;
         if (cost < 0.90 * whole && cost < best) { best = cost; best_splits = (int)splits; }

@@ -946,11 +946,11 @@ static void launch_mx_tiled(const GemmArgs &g, const uint8_t *sa, const uint8_t 
     GemmArgs t = g;
     // outputs of about one tile per compute unit: as for the per-tensor GEMMs
     const FewTiles few = gemm_few_tiles(g.M, g.N, g.K, cus);
-    if (KS && (few == kDeep || few == kDeepWide)) {
-        const int bm = few == kDeep ? 128 : 256;
+    if (KS && few >= kDeepWide) {
+        const int bm = few == kDeepWide ? 256 : 128, bn = few == kDeep192 ? 192 : 128;
         t.mx_sa = sa; t.mx_sb = sb;
-        t.tiles_m = (int)((g.M + bm - 1) / bm); t.tiles_n = (int)((g.N + 127) / 128);
-        launch_gemm_deep(few == kDeepWide, FA, FB, t, cus, stream);
+        t.tiles_m = (int)((g.M + bm - 1) / bm); t.tiles_n = (int)((g.N + bn - 1) / bn);
+        launch_gemm_deep(bm, bn, FA, FB, t, cus, stream);
         return;
     }
     // 256 x 256 tiles (8 waves of 128 x 64) when they fill the chip, else 128 x 128 (two blocks per compute unit)

@@ -880,10 +880,10 @@ def test_last_round_in_smaller_tiles_has_the_same_bits(N, shape, out_dtype):
         N.gemm_set_variant(-1)
 
 
-@pytest.mark.parametrize("variant", [4, 9, 10])
+@pytest.mark.parametrize("variant", [4, 9, 10, 11])
 @pytest.mark.parametrize("M,Nn,K", [(16, 16, 128), (129, 144, 256), (200, 136, 384), (255, 264, 512), (300, 20, 640), (513, 392, 1152), (64, 1000, 2176)])
 def test_few_tile_kernels_at_ragged_edges(N, variant, M, Nn, K):
-    """128 x 128 and 256 x 128 tiles that end inside the matrix, in rows and in columns, for every form of the output: one
+    """128 x 128, 256 x 128 and 128 x 192 tiles that end inside the matrix, in rows and in columns, for every form of the output: one
     scale, scales per row and column with a bias, added to what is there.  Lengths of K shorter than the pipeline and odd in
     steps; far fewer tiles than compute units.  Codes, scales, bias and old values are small multiples of powers of two:
     every sum is exact in fp32, so the result is known to the bit."""

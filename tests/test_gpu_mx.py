@@ -303,6 +303,20 @@ def test_mx_gemm_few_tile_outputs_at_every_pipeline_depth(N, k_steps):
         assert max_rel_err(got.float(), ref_bf16.float()) <= 1e-2
 
 
+@pytest.mark.parametrize("M,N_,K", [(8192, 768, 1024), (5000, 1136, 1152), (22000, 200, 1024)])
+def test_mx_gemm_outputs_of_one_128_by_192_tile_per_unit(N, M, N_, K):
+    """Against the kernel for scales as [rows, K / 32], which has other tiles.  Codes and scales are small powers of two and
+    their multiples: every sum is exact in fp32, in whatever order, so the results agree to the bit."""
+    g = torch.Generator().manual_seed(M)
+    values = torch.tensor([0.0, 0.5, 1.0, -1.0, 2.0, -0.5]).to(torch.float8_e4m3fn).view(torch.uint8)
+    ac, bc = (values[torch.randint(0, 6, (r, K), generator=g)].cuda() for r in (M, N_))
+    asc, bsc = (torch.randint(126, 129, (r, K // 32), generator=g, dtype=torch.uint8) for r in (M, N_))
+    for dtype in (torch.bfloat16, torch.float32):
+        want = N.mx_gemm_nt(ac, asc.cuda(), bc, bsc.cuda(), E4M3, E4M3, out_dtype=dtype)
+        got = N.mx_gemm_nt(ac, _kstep(asc).cuda(), bc, _kstep(bsc).cuda(), E4M3, E4M3, out_dtype=dtype)
+        assert torch.equal(got, want)
+
+
 def test_mx_gemm_small_case_against_the_c_oracle_and_bias(N):
     M, N_, K = 48, 40, 96
     ac, asc, bc, bsc = _operands(M, N_, K, E4M3, E4M3, seed=3)
