@@ -432,7 +432,8 @@ int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t M, int64_t 
  * is therefore taken in a different order than by odl_fp8_gemm_nt: equal within fp32 rounding,
  * bit-identical where every partial sum is exact.  odl_fp8_gemm_split_count proposes `splits`
  * for a shape (1 = not worth splitting; k_slow != 0: an operand will be passed K-slow); any 2 <= splits <= 64 that leaves every run at least 512
- * long is accepted.  M, N, K multiples of 128 (256 for an operand stored K-slow), K-run >= 512.
+ * long is accepted.  M, N, K multiples of 128 (256 for an operand stored K-slow), K-run >= 512.  `splits` is the most
+ * that is used: where one launch of smaller tiles is faster than two runs, that is what runs (the workspace stays unread).
  * accumulate != 0: the second kernel adds the old value of C to the sum before the one rounding
  * (C = C + product, as for odl_fp8_gemm_nt); splits == 1 is then accepted too, which is how a product
  * with an operand stored K-slow (a weight gradient that reads dY as stored) is added into C.

@@ -407,13 +407,13 @@ extern "C" int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t 
 //   one launch, 256 x 256 tiles : 0.92 us per K step of 128 (few compute units busy: high clock) + 3 steps of overhead
 //   one launch, smaller tiles   : what odl_fp8_gemm_nt takes for outputs of <= cus / 2 big tiles (few_tiles_variant).
 //                                 128 x 128 with a unit each 0.37 us per step + 6 us (3072 x 768 x 16384: 45 - 50 us, in
-//                                 six runs 52 and the reduction's launch); 128 x 192 0.66 + 8; 256 x 128 with a unit each
-//                                 0.70 + 7; two 128 x 128 blocks per unit 0.62 (it reads every operand panel twice as often)
+//                                 six runs 52 and the reduction's launch); 256 x 128 with a unit each 0.70 + 7 (128 x 192 in
+//                                 their place: 0.66 + 8; where two runs are proposed instead, odl_fp8_gemm_splitk looks
+//                                 again); two 128 x 128 blocks per unit 0.62 (it reads every operand panel twice as often)
 //   split                       : 0.96 us per step of a run + 9 us (pipeline fill, the fp32 epilogue, the second launch)
-//   with operands that outgrow the 256 MB memory-side cache, per step 0.61 (128 x 128: 8192 x 512 x 50304 241 us, in three runs 234,
-//                                 in four 200), 0.71 (128 x 192: 8192 x 768 x 50304 285, in two runs 319), 0.88 (256 x 128: 8192 x 1024 x
-//                                 151936 1047, in two runs 961) and 1.45 (split)
 //                                 + the partial results, splits x M x N floats written and read back, at 2.7 TB/s in all
+//   with operands that outgrow the 256 MB memory-side cache, per step 0.61 (128 x 128: 8192 x 512 x 50304 241 us, in three runs
+//                                 234, in four 200), 0.88 (256 x 128: 8192 x 1024 x 151936 1047, in two runs 961), 1.45 (split)
 //   each bounded below by its operand traffic (tiles x panel bytes) at about 12 TB/s out of the caches (the kernels of
 //   gemm_deep.hip: 18).
 //   one launch, thin tiles      : 4 us + 2.7 ns per K step and operand row of the busiest compute unit (how well that
@@ -437,8 +437,7 @@ extern "C" int odl_fp8_gemm_split_count(int64_t M, int64_t N, int64_t K, int k_s
         const double panels = (double)((M + 127) / 128) * (double)((N + 127) / 128) * (double)K;         // of 128 rows, once per tile
         double small = whole, small_traffic_us = 0.0;
         if (variant == kDeepVariant) { small = (cold ? 0.61 : 0.37) * (double)steps + 6.0; small_traffic_us = panels * 256.0 / 18.0e6; }
-        else if (variant == kDeep192Variant) { small = (cold ? 0.71 : 0.66) * (double)steps + 8.0; small_traffic_us = panels * 213.4 / 18.0e6; }
-        else if (variant == kDeepWideVariant) { small = (cold ? 0.88 : 0.70) * (double)steps + 7.0; small_traffic_us = panels * 192.0 / 18.0e6; }
+        else if (variant == kDeepWideVariant || variant == kDeep192Variant) { small = (cold ? 0.88 : 0.70) * (double)steps + 7.0; small_traffic_us = panels * 192.0 / 18.0e6; }
         else if (variant) { small = 0.62 * ((double)steps + 3.0); small_traffic_us = panels * 256.0 / 12.0e6; }
         if (small < small_traffic_us) small = small_traffic_us;
         if (small < whole) whole = small;
@@ -492,6 +491,11 @@ extern "C" int odl_fp8_gemm_splitk(const uint8_t *a, const uint8_t *b, int64_t M
     if (workspace_bytes < (int64_t)splits * M * N * 4)
         return set_error(ODL_ERR_ARG, "odl_fp8_gemm_splitk: workspace of %lld bytes, %lld needed", (long long)workspace_bytes,
                          (long long)splits * M * N * 4);
+    // One launch of 128 x 192 tiles that gives (nearly) every compute unit one beats two runs of big tiles and the addition
+    // behind them: 8192 x 768 x 50304 319 -> 283 us, 16384 x 384 x 50304 340 -> 308.
+    auto mis = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; };
+    if (splits == 2 && !ta && !tb && gemm_few_tiles(M, N, K, cu_count()) == kDeep192 && !mis(sa_inv) && !mis(sb_inv) && !mis(bias))
+        return gemm_nt_checked(a, b, M, N, K, fmt_a, fmt_b, sa_inv, sa_n, sb_inv, sb_n, bias, c, out_dtype, accumulate, kDeep192Variant, stream);
     GemmArgs g;
     g.a = a; g.b = b; g.c = workspace; g.sa = sa_inv; g.sb = sb_inv; g.bias = nullptr;
     g.M = M; g.N = N; g.K = K;
