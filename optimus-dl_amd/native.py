@@ -1278,14 +1278,15 @@ def gemm_layouts_supported(M: int, N: int, K: int, out_dtype: torch.dtype = torc
 def wgrad_direct_pays(n_out: int, n_in: int, tokens: int) -> bool:
     """Whether the weight gradient [n_out, n_in] = dY^T . X is better computed from the row-major codes of dY
     (:func:`gemm_layouts`, K-slow operand, no transposed copy of dY) than from a transposed copy with :func:`gemm_nt`.
-    The kernel that reads K-slow operands works on whole 256 x 256 tiles: it pays where those fill the chip, and for
-    small gradients, where both routes are a handful of short launches and the copy is one more.  In between it either
-    leaves compute units idle or splits the contraction and adds a reduction pass, and 128 x 128 tiles over the
-    transposed copy are faster.  Measured at 8192 tokens, cast of dY included, direct / transposed in us:
-    1024 x 4096 61.7 / 52.2, 2048 x 4096 90.3 / 81.2, 1024 x 3072 53.3 / 48.7, 3072 x 1024 68.2 / 64.6;
-    4096 x 4096 129.9 / 136.3, 2048 x 1024 54.2 / 56.2, 2304 x 768 53.8 / 58.7, 1024 x 1024 38.1 / 41.9."""
-    tiles = (n_out // 256) * (n_in // 256)
-    return tiles >= 192 or n_out * n_in < 2_200_000
+    The kernel that reads K-slow operands works on whole 256 x 256 tiles: it pays where those fill the chip.  Where they do
+    not it leaves compute units idle or splits the contraction and adds a reduction pass, and smaller tiles over the
+    transposed copy are faster.  Measured, cast of dY included, direct / transposed in us: at 8192 tokens 4096 x 4096 124 / 130;
+    1024 x 4096 61.7 / 52.2, 3072 x 768 55.3 / 52.9, 2048 x 1024 53.9 / 46.6; 1024 x 1024 at 512 tokens 17.1 / 11.7, 2048 29.7 / 17.7,
+    4096 31.8 / 24.9, 6144 35.8 / 32.7.  From 8192 tokens on, outputs of less than 1.8 million elements are equal either way
+    (2304 x 768 47.6 / 48.6, 1024 x 1024 37.9 / 38.8, 768 x 768 33.6 / 33.8), and the route without a second copy of dY is
+    taken; so it is for the smallest outputs (768 x 512), which give 5 to 10 us for that."""
+    tiles, elements = (n_out // 256) * (n_in // 256), n_out * n_in
+    return tiles >= 192 or (elements < 1_800_000 and tokens >= 8192) or elements < 400_000
 
 
 def dgrad_sum_in_one_launch(tokens: int, n_in: int, n_outs: "list[int]") -> bool:
