@@ -494,7 +494,8 @@ extern "C" int odl_fp8_gemm_splitk(const uint8_t *a, const uint8_t *b, int64_t M
     // One launch of 128 x 192 tiles that gives (nearly) every compute unit one beats two runs of big tiles and the addition
     // behind them: 8192 x 768 x 50304 319 -> 283 us, 16384 x 384 x 50304 340 -> 308.
     auto mis = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; };
-    if (splits == 2 && !ta && !tb && gemm_few_tiles(M, N, K, cu_count()) == kDeep192 && !mis(sa_inv) && !mis(sb_inv) && !mis(bias))
+    if (splits == 2 && !ta && !tb && gemm_few_tiles(M, N, K, cu_count()) == kDeep192 && !(sa_n > 1 && mis(sa_inv)) && !(sb_n > 1 && mis(sb_inv)) &&
+        !mis(bias))
         return gemm_nt_checked(a, b, M, N, K, fmt_a, fmt_b, sa_inv, sa_n, sb_inv, sb_n, bias, c, out_dtype, accumulate, kDeep192Variant, stream);
     GemmArgs g;
     g.a = a; g.b = b; g.c = workspace; g.sa = sa_inv; g.sb = sb_inv; g.bias = nullptr;

@@ -563,6 +563,24 @@ def test_accumulate_random_every_variant(N, shape, out_dtype):
     N.gemm_set_variant(-1)
 
 
+@pytest.mark.parametrize("M,Nn", [(8192, 768), (16384, 384)])
+def test_two_runs_proposed_where_one_launch_of_smaller_tiles_is_faster(N, M, Nn):
+    """The split entry with two runs and an output of one 128 x 192 tile per compute unit: one scale at an address off the
+    16-byte grid, scales per row and column with a bias, added to what is there.  Every sum is exact."""
+    K = 2048
+    g = torch.Generator().manual_seed(Nn)
+    values = torch.tensor([0.0, 0.5, 1.0, -1.0])
+    a, b = values[torch.randint(0, 4, (M, K), generator=g)], values[torch.randint(0, 4, (Nn, K), generator=g)]
+    ac, bc = (t.to(torch.float8_e4m3fn).view(torch.uint8).cuda() for t in (a, b))
+    product = a @ b.t()
+    half = torch.full((3,), 0.5).cuda()[2:]
+    sa, sb, bias = 2.0 ** torch.randint(-1, 2, (M,), generator=g), 2.0 ** torch.randint(-1, 2, (Nn,), generator=g), torch.randint(-8, 8, (Nn,), generator=g).float()
+    got = N.gemm_splitk(ac, bc, O.E4M3, O.E4M3, half, half, 2, out_dtype=torch.float32)
+    assert torch.equal(got.cpu(), product * 0.25)
+    got = N.gemm_splitk(ac, bc, O.E4M3, O.E4M3, sa.cuda(), sb.cuda(), 2, bias=bias.cuda(), out=got, accumulate=True)
+    assert torch.equal(got.cpu(), product * 0.25 + (product * sa[:, None] * sb[None] + bias))
+
+
 def test_accumulate_through_split_k_and_k_slow_layouts(N):
     """The routes that pass through the fp32 workspace: a split over K (few tiles, long contraction) and an operand
     stored K-slow (wgrad reading dY as stored), the latter also with a single run."""
