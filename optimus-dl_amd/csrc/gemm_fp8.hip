@@ -184,8 +184,8 @@ static int choose_variant(int64_t M, int64_t N, int64_t K, bool stream_ok, bool 
 }
 
 // Rows of A that the streaming kernel should leave to a second launch (0: none).  Its 256 x 256 tiles go round the chip one
-// per compute unit, and a last round of few tiles costs as much as a full one.  Those rows as 128 x 128 tiles take about half
-// a round with one tile per unit, 0.7 with two, and 4 us for the launch.  With one tile that pays from 16 K steps on
+// per compute unit, and a last round of few tiles costs as much as a full one.  Those rows in the tiles of few_tiles_variant take
+// about half a round with one 128 x 128 tile per unit, 0.6 with more, and 4 us for the launch.  With one tile that pays from 16 K steps on
 // (5000 x 4096 x 2048: 47.8 -> 43.4 us, x 14336: 256 -> 216; 4096 x 4864 x 4096: 82.2 -> 68.8), with two from 32
 // (11264 x 2048 x 4096: 91.5 -> 86.2, 50304 x 768 x 8192: 290 -> 261; 4016 x 5632 x 2048 would go from 49.1 to 53.7).
 // Same K order, same bits.
