@@ -45,7 +45,7 @@ enum odl_status {
     ODL_ERR_LAUNCH = 3    /* HIP reported an error at launch */
 };
 
-/* ABI version of this header (15); bumped when a signature changes or an entry point is added. */
+/* ABI version of this header; bumped when a signature changes or an entry point is added. */
 int odl_fp8_abi_version(void);
 
 /*
@@ -478,6 +478,11 @@ int odl_fp8_delayed_update(float *history, int64_t H, int64_t R, int64_t ld,
 int odl_fp8_gemm_num_variants(void);
 const char *odl_fp8_gemm_variant_name(int variant);
 int odl_fp8_gemm_set_variant(int variant);
+/*
+ * The variant that odl_fp8_gemm_nt takes for a shape, and, where the last rows go to a second launch, how many
+ * (*tail_rows, 0: none) and in which variant.  -1: bad arguments.  Without a GPU it plans for 256 compute units.
+ */
+int odl_fp8_gemm_route(int64_t M, int64_t N, int64_t K, int out_dtype, int accumulate, int64_t *tail_rows, int *tail_variant);
 /*
  * BENCH-ONLY hook; a production build may compile it out (-DODL_FP8_NO_BENCH_HOOKS removes the entry point and the
  * two clock reads it switches on in the streaming kernel).  Host thread-local, like odl_fp8_gemm_set_variant; NULL

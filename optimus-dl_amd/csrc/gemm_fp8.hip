@@ -156,17 +156,18 @@ FewTiles gemm_few_tiles(int64_t M, int64_t N, int64_t K, int num_cus) {
     return K >= 3072 && ((M + 255) / 256) * ((N + 127) / 128) <= num_cus ? kDeepWide : kTwoBlocks;
 }
 
-// ... as a variant (0: many tiles)
+// ... as a variant (kNoVariant: many tiles)
+constexpr int kNoVariant = -1;
 static int few_tiles_variant(int64_t M, int64_t N, int64_t K, bool lim32) {
     const FewTiles few = gemm_few_tiles(M, N, K, cu_count());
-    if (few == kManyTiles) return 0;
+    if (few == kManyTiles) return kNoVariant;
     return few == kTwoBlocks || !lim32 ? 4 : few == kDeep ? kDeepVariant : few == kDeep192 ? kDeep192Variant : kDeepWideVariant;
 }
 
 static int choose_variant(int64_t M, int64_t N, int64_t K, bool stream_ok, bool lim32) {
     const int cus = cu_count();
     if (thin_pays(M, N, K)) return kThinVariant;
-    if (const int small = few_tiles_variant(M, N, K, lim32)) return small;
+    if (const int small = few_tiles_variant(M, N, K, lim32); small != kNoVariant) return small;
     int best = 2;
     double best_score = -1.0;
     for (int v = 2; v <= kStreamVariant; ++v) {                       // variant 1 (one wave per SIMD) only by explicit request
@@ -243,10 +244,15 @@ extern "C" int odl_fp8_gemm_set_variant(int variant) {
     return ODL_OK;
 }
 
-// The launch of checked arguments.  launch_as: the variant to use (-1: the forced one, or the choice by shape).
-static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b, const float *sa_inv, int64_t sa_n,
-                           const float *sb_inv, int64_t sb_n, const void *bias, void *c, int out_dtype, int accumulate, int launch_as,
-                           hipStream_t stream) {
+// Which kernel runs a product of checked arguments, and which one its last rows where they go to a second launch.
+struct Route {
+    int variant;
+    int64_t tail;              // rows of the second launch (0: there is none)
+    int tail_variant;
+};
+
+// launch_as: the variant to use (-1: the forced one, or the choice by shape)
+static Route route_of(int64_t M, int64_t N, int64_t K, int out_dtype, int accumulate, int launch_as) {
     const bool tiled_ok = K >= 128 && K % 128 == 0 && (double)M * (double)K < 4294967296.0 && (double)N * (double)K < 4294967296.0;
     // the pipelined and the streaming kernel address rows with 32-bit byte offsets
     const bool lim32 = (double)(M + 256) * (double)K < 2147483648.0 && (double)(N + 256) * (double)K < 2147483648.0;
@@ -263,16 +269,36 @@ static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_
     if (variant >= kDeepWideVariant && !lim32) variant = 4;
 
     if (variant == kStreamVariant && t_forced_variant < 0 && launch_as < 0) {
-        const int64_t rest = tail_rows(M, N, K), head = M - rest;
-        if (rest > 0) {
-            const int64_t esz = out_dtype == ODL_BF16 ? 2 : 4;
-            const int rc = gemm_nt_checked(a, b, head, N, K, fmt_a, fmt_b, sa_inv, sa_n == 1 ? 1 : head, sb_inv, sb_n, bias, c, out_dtype, accumulate,
-                                           kStreamVariant, stream);
-            if (rc != ODL_OK) return rc;
-            return gemm_nt_checked(a + head * K, b, rest, N, K, fmt_a, fmt_b, sa_n == 1 ? sa_inv : sa_inv + head, sa_n == 1 ? 1 : rest, sb_inv, sb_n,
-                                   bias, reinterpret_cast<uint8_t *>(c) + head * N * esz, out_dtype, accumulate,
-                                   few_tiles_variant(rest, N, K, lim32), stream);
-        }
+        // Counted in 256 x 256 tiles those rows can be too many for the kernels of few tiles (half tiles at an edge count
+        // whole there): two 128 x 128 blocks per unit then (4224 x 5632 x 4096,
+        // rest 1408 rows: 84 us in all).
+        const int64_t rest = tail_rows(M, N, K);
+        const int small = rest > 0 ? few_tiles_variant(rest, N, K, lim32) : kNoVariant;
+        if (rest > 0) return {kStreamVariant, rest, small != kNoVariant ? small : 4};
+    }
+
+    GemmArgs g = {};
+    g.M = M; g.N = N; g.K = K;
+    g.out_dtype = out_dtype;
+    g.accumulate = accumulate != 0;
+    // the streaming kernel wants N in multiples of 128: next best kernel instead
+    if (variant == kStreamVariant && !(stream_ok && gemm_stream_accepts(g))) variant = pipe_ok ? kPipeVariant : 2;
+    return {variant, 0, 0};
+}
+
+// The launch of checked arguments.
+static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b, const float *sa_inv, int64_t sa_n,
+                           const float *sb_inv, int64_t sb_n, const void *bias, void *c, int out_dtype, int accumulate, int launch_as,
+                           hipStream_t stream) {
+    const Route route = route_of(M, N, K, out_dtype, accumulate, launch_as);
+    const int variant = route.variant;
+    if (route.tail > 0) {
+        const int64_t head = M - route.tail, esz = out_dtype == ODL_BF16 ? 2 : 4;
+        const int rc = gemm_nt_checked(a, b, head, N, K, fmt_a, fmt_b, sa_inv, sa_n == 1 ? 1 : head, sb_inv, sb_n, bias, c, out_dtype, accumulate,
+                                       kStreamVariant, stream);
+        if (rc != ODL_OK) return rc;
+        return gemm_nt_checked(a + head * K, b, route.tail, N, K, fmt_a, fmt_b, sa_n == 1 ? sa_inv : sa_inv + head, sa_n == 1 ? 1 : route.tail, sb_inv,
+                               sb_n, bias, reinterpret_cast<uint8_t *>(c) + head * N * esz, out_dtype, accumulate, route.tail_variant, stream);
     }
 
     GemmArgs g;
@@ -287,10 +313,6 @@ static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_
     if (tm * tn > 0x7ffffff0LL) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt: too many tiles");
     g.tiles_m = (int)tm; g.tiles_n = (int)tn;
 
-    if (variant == kStreamVariant && !(stream_ok && gemm_stream_accepts(g))) {
-        // the streaming kernel wants N in multiples of 128: next best kernel instead
-        variant = pipe_ok ? kPipeVariant : 2;
-    }
     if (variant == 0) launch_gemm_generic(fmt_a, fmt_b, g, stream);
     else if (variant == kThinVariant) launch_gemm_thin(fmt_a, fmt_b, g, cu_count(), stream);
     else if (variant >= kDeepWideVariant) launch_gemm_deep(bm, bn, fmt_a, fmt_b, g, cu_count(), stream);
@@ -299,6 +321,17 @@ static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_
     else if (variant == kStreamVariant) { attach_clock_probe(g); launch_gemm_stream(fmt_a, fmt_b, g, cu_count(), stream); }
     else launch_gemm_tiled(variant, fmt_a, fmt_b, g, stream);
     return check_launch("odl_fp8_gemm_nt");
+}
+
+extern "C" int odl_fp8_gemm_route(int64_t M, int64_t N, int64_t K, int out_dtype, int accumulate, int64_t *tail_rows_out, int *tail_variant_out) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 16 != 0 || (out_dtype != ODL_BF16 && out_dtype != ODL_F32) || !tail_rows_out || !tail_variant_out) {
+        set_error(ODL_ERR_ARG, "odl_fp8_gemm_route: %lld x %lld x %lld, out_dtype %d", (long long)M, (long long)N, (long long)K, out_dtype);
+        return -1;
+    }
+    const Route route = route_of(M, N, K, out_dtype, accumulate, -1);
+    *tail_rows_out = route.tail;
+    *tail_variant_out = route.tail_variant;
+    return route.variant;
 }
 
 extern "C" int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b,
@@ -438,7 +471,7 @@ extern "C" int odl_fp8_gemm_split_count(int64_t M, int64_t N, int64_t K, int k_s
         double small = whole, small_traffic_us = 0.0;
         if (variant == kDeepVariant) { small = (cold ? 0.61 : 0.37) * (double)steps + 6.0; small_traffic_us = panels * 256.0 / 18.0e6; }
         else if (variant == kDeepWideVariant || variant == kDeep192Variant) { small = (cold ? 0.88 : 0.70) * (double)steps + 7.0; small_traffic_us = panels * 192.0 / 18.0e6; }
-        else if (variant) { small = 0.62 * ((double)steps + 3.0); small_traffic_us = panels * 256.0 / 12.0e6; }
+        else if (variant != kNoVariant) { small = 0.62 * ((double)steps + 3.0); small_traffic_us = panels * 256.0 / 12.0e6; }
         if (small < small_traffic_us) small = small_traffic_us;
         if (small < whole) whole = small;
     }

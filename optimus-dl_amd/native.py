@@ -25,7 +25,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 22
+ABI_VERSION = 23
 _OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
@@ -77,6 +77,7 @@ EXPORTS = (
     "odl_fp8_gemm_num_variants",
     "odl_fp8_gemm_variant_name",
     "odl_fp8_gemm_set_variant",
+    "odl_fp8_gemm_route",
     "odl_fp8_gemm_set_clock_probe",
     "odl_fp8_mx_cast",
     "odl_fp8_mx_cast_padded",
@@ -167,6 +168,7 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_gemm_variant_name.argtypes = [i32]
         L.odl_fp8_gemm_variant_name.restype = ctypes.c_char_p
         L.odl_fp8_gemm_set_variant.argtypes = [i32]
+        L.odl_fp8_gemm_route.argtypes = [i64, i64, i64, i32, i32, vp, vp]
         L.odl_fp8_gemm_set_clock_probe.argtypes = [vp, i32]
         L.odl_fp8_swiglu_mx_cast.argtypes = [vp, vp, i64, i64, i64, i32, vp, vp, vp, vp, i32, vp]
         L.odl_fp8_swiglu_bwd_mx_cast.argtypes = [vp, vp, vp, i64, i64, i64, i32, vp, vp, vp, vp, vp, vp, vp, vp, i32, vp]
@@ -1369,6 +1371,16 @@ def delayed_update_raw(history: torch.Tensor, H: int, ld: int, R: int, scale: to
 def gemm_variants() -> list[str]:
     L = load()
     return [L.odl_fp8_gemm_variant_name(i).decode() for i in range(L.odl_fp8_gemm_num_variants())]
+
+
+def gemm_route(M: int, N: int, K: int, out_dtype: torch.dtype = torch.bfloat16, accumulate: bool = False) -> tuple[int, int, int]:
+    """What ``odl_fp8_gemm_nt`` runs for a shape (host code): the variant, the rows left to a second launch (0: none) and its
+    variant."""
+    tail_rows, tail_variant = ctypes.c_int64(), ctypes.c_int()
+    variant = load().odl_fp8_gemm_route(M, N, K, _OUT_DTYPES[out_dtype], int(accumulate), ctypes.byref(tail_rows), ctypes.byref(tail_variant))
+    if variant < 0:
+        _check(1, "odl_fp8_gemm_route")
+    return variant, tail_rows.value, tail_variant.value
 
 
 def gemm_set_variant(variant: int) -> None:

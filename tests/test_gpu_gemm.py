@@ -879,7 +879,7 @@ def test_four_stage_tiles_at_every_pipeline_depth(N, k_steps):
     assert torch.equal(got, O.t_decode(b, O.E4M3)[:, cols].t())
 
 
-@pytest.mark.parametrize("shape", [(4016, 5632, 4096), (6784, 2816, 2048), (5000, 4096, 2176), (50304, 768, 4096)])
+@pytest.mark.parametrize("shape", [(4016, 5632, 4096), (6784, 2816, 2048), (5000, 4096, 2176), (50304, 768, 4096), (4224, 5632, 4096), (16384, 1408, 4096)])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 def test_last_round_in_smaller_tiles_has_the_same_bits(N, shape, out_dtype):
     """Outputs whose last round of 256 x 256 tiles would leave most of the chip idle are finished by a second launch:

@@ -144,6 +144,31 @@ def test_split_count_is_a_host_side_decision_with_the_documented_shape_rules():
         assert count(M, N, K) == 1                          # not multiples of 128, or too short to split
 
 
+def test_whole_k_steps_never_run_the_generic_kernel():
+    """Neither a whole product nor the rows of its last round that go to a second launch: over every remainder of tiles that
+    the rows and columns can leave, the shapes among them whose rest is few 128 x 128 tiles and many of 256 x 256."""
+    from optimus_dl_amd import native
+
+    if not native.is_built():
+        pytest.skip("library not built")
+    generic = next(i for i, name in enumerate(native.gemm_variants()) if name.startswith("generic"))
+    tails = 0
+    shapes = [(4224, 5632, 4096), (16384, 1408, 4096), (612, 50304, 4096), (25088, 896, 4864), (8064, 3072, 4096), (32640, 768, 50304)]
+    for shape in shapes:
+        assert native.gemm_route(*shape)[1] > 0, "meant to have a second launch"
+    for N in (384, 768, 896, 1024, 1408, 2944, 3072, 4096, 5632, 14336, 50304):
+        for K in (128, 2048, 4096):
+            shapes += [(M, N, K) for M in [*range(16, 20000, 336), *range(25088, 33000, 128)]]
+    for M, N, K in shapes:
+        for dtype in native._OUT_DTYPES:
+            variant, rest, second = native.gemm_route(M, N, K, dtype)
+            tails += rest > 0
+            assert variant != generic and (rest == 0 or second != generic), (M, N, K, dtype)
+    assert tails > 1000
+    with pytest.raises(native.NativeError):
+        native.gemm_route(16, 16, 20)
+
+
 def test_data_gradient_sums_run_in_one_launch_only_for_whole_wave_tiles():
     """Whether the members' products are rounded once or one by one depends on the token count like this and no other way:
     multiples of 128 with more than 128 output tiles go in one launch."""
