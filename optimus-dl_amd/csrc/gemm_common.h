@@ -2,6 +2,8 @@
 // wrapper and the scaling epilogue.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace odl {
@@ -120,7 +122,8 @@ __device__ __forceinline__ void store_tile(const GemmArgs &g, const v16f &acc, i
 // stored so that a wave instruction writes whole 128-byte lines.
 //   value = acc * (sa_inv[m] * sb_inv[n]) (+ bias[n]); fp32 steps, one final rounding.
 // Rows past the last one are not stored (with direct stores instead for the last tile row, 4016 x 2048 x 5632 took 53.7 us
-// in 256 x 128 tiles, the whole 4096 rows 41).
+// in 256 x 128 tiles, the whole 4096 rows 41).  Only the slab in which the matrix ends asks row by row: a comparison in front
+// of every store costs the whole tiles up to 0.7 us (bf16, two blocks per unit: 2304 x 2048 x 512 8.3 -> 7.6 us without).
 // Requires: N % 8 == 0, n_wave % 8 == 0, n_wave + 32 TN <= N, 16-byte aligned output / scale vectors / bias,
 // and that nobody else touches `wave_lds` (staged_epilogue_bytes<> bytes).  LDS
 // operations of one wave execute in order, so write -> read -> next write needs no barrier.
@@ -144,6 +147,8 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs &g, v16f (&acc)[T
     if (RAGGED && rows <= 0) return;
 #pragma unroll
     for (int t = 0; t < TM; ++t) {
+        if (RAGGED && 32 * t >= rows) break;
+        const bool whole = !RAGGED || 32 * t + 32 <= rows;
         float sa = 1.0f;
         if (vec) sa = g.sa[(m_wave + (RAGGED ? min(32 * t + lr, rows - 1) : 32 * t + lr)) * g.sa_vec];
 #pragma unroll
@@ -170,15 +175,19 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs &g, v16f (&acc)[T
                     else *reinterpret_cast<float4 *>(dst) = float4{v[0], v[1], v[2], v[3]};
                 }
             }
+            auto store = [&](auto all) {
 #pragma unroll
-            for (int i = 0; i < 32 / RPI; ++i) {
-                const int r = i * RPI + lane / LPR, chunk = lane % LPR;
-                const u32x4 val = *reinterpret_cast<const u32x4 *>(wave_lds + r * PITCH + chunk * 16);
-                uint8_t *dst = out + ((m_wave + 32 * t + r) * g.N + n_wave + 32 * us) * ESZ + chunk * 16;
-                // non-temporal: the output is not read by the next kernel, and written through the memory-side
-                // cache it would still be draining to HBM while the next (memory-bound) kernel runs
-                if (!RAGGED || 32 * t + r < rows) __builtin_nontemporal_store(val, reinterpret_cast<u32x4 *>(dst));
-            }
+                for (int i = 0; i < 32 / RPI; ++i) {
+                    const int r = i * RPI + lane / LPR, chunk = lane % LPR;
+                    const u32x4 val = *reinterpret_cast<const u32x4 *>(wave_lds + r * PITCH + chunk * 16);
+                    uint8_t *dst = out + ((m_wave + 32 * t + r) * g.N + n_wave + 32 * us) * ESZ + chunk * 16;
+                    // non-temporal: the output is not read by the next kernel, and written through the memory-side
+                    // cache it would still be draining to HBM while the next (memory-bound) kernel runs
+                    if (all || 32 * t + r < rows) __builtin_nontemporal_store(val, reinterpret_cast<u32x4 *>(dst));
+                }
+            };
+            if (whole) store(std::true_type{});
+            else store(std::false_type{});
         }
     }
 }
@@ -222,12 +231,15 @@ __device__ __forceinline__ void epilogue_staged_accumulate(const GemmArgs &g, v1
             }
         }
     };
+    auto inside = [&](int slab) { return !RAGGED || 32 * (slab / (TN / TNS)) < rows; };
     float old[2][NI][4];
-    fetch_old(old[0], 0);
+    if (inside(0)) fetch_old(old[0], 0);
 #pragma unroll
     for (int slab = 0; slab < SLABS; ++slab) {
         const int t = slab / (TN / TNS), us = (slab % (TN / TNS)) * TNS;
-        if (slab + 1 < SLABS) fetch_old(old[(slab + 1) & 1], slab + 1);
+        if (slab + 1 < SLABS && inside(slab + 1)) fetch_old(old[(slab + 1) & 1], slab + 1);
+        if (!inside(slab)) continue;
+        const bool whole = !RAGGED || 32 * t + 32 <= rows;
         float sa = 1.0f;
         if (vec) sa = g.sa[(m_wave + (RAGGED ? min(32 * t + lr, rows - 1) : 32 * t + lr)) * g.sa_vec];
 #pragma unroll
@@ -250,16 +262,20 @@ __device__ __forceinline__ void epilogue_staged_accumulate(const GemmArgs &g, v1
                 *reinterpret_cast<float4 *>(wave_lds + lr * PITCH + col * 4) = float4{v[0], v[1], v[2], v[3]};
             }
         }
+        auto store = [&](auto all) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int r = i * RPI + lane / LPR, chunk = lane % LPR;
-            const float4 val = *reinterpret_cast<const float4 *>(wave_lds + r * PITCH + chunk * 16);
-            const float (&o)[4] = old[slab & 1][i];
-            const float w[4] = {o[0] + val.x, o[1] + val.y, o[2] + val.z, o[3] + val.w};
-            if (RAGGED && row_of(slab, i) >= rows) continue;
-            if constexpr (OUT_BF16) *reinterpret_cast<u32x2 *>(c_ptr(slab, i)) = u32x2{pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3])};
-            else *reinterpret_cast<float4 *>(c_ptr(slab, i)) = float4{w[0], w[1], w[2], w[3]};
-        }
+            for (int i = 0; i < NI; ++i) {
+                const int r = i * RPI + lane / LPR, chunk = lane % LPR;
+                const float4 val = *reinterpret_cast<const float4 *>(wave_lds + r * PITCH + chunk * 16);
+                const float (&o)[4] = old[slab & 1][i];
+                const float w[4] = {o[0] + val.x, o[1] + val.y, o[2] + val.z, o[3] + val.w};
+                if (!all && row_of(slab, i) >= rows) continue;
+                if constexpr (OUT_BF16) *reinterpret_cast<u32x2 *>(c_ptr(slab, i)) = u32x2{pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3])};
+                else *reinterpret_cast<float4 *>(c_ptr(slab, i)) = float4{w[0], w[1], w[2], w[3]};
+            }
+        };
+        if (whole) store(std::true_type{});
+        else store(std::false_type{});
     }
 }
 
