@@ -114,7 +114,8 @@ __device__ __forceinline__ void store_tile(const GemmArgs &g, const v16f &acc, i
 
 
 // ---------------------------------------------------------------- staged epilogue
-// Output path for a wave tile that lies inside the matrix; with RAGGED its rows may end anywhere.  The MFMA leaves
+// Output path for a wave tile that lies inside the matrix; with RAGGED its rows may end anywhere and its columns after any
+// slab.  The MFMA leaves
 // each lane with 4-column fragments of 32 different rows, which as direct stores
 // touch 32 cache lines per instruction.  Instead every slab of 32 rows x (TNS*32)
 // columns of the wave tile is scaled, rounded and written to a private LDS region
@@ -124,7 +125,8 @@ __device__ __forceinline__ void store_tile(const GemmArgs &g, const v16f &acc, i
 // Rows past the last one are not stored (with direct stores instead for the last tile row, 4016 x 2048 x 5632 took 53.7 us
 // in 256 x 128 tiles, the whole 4096 rows 41).  Only the slab in which the matrix ends asks row by row: a comparison in front
 // of every store costs the whole tiles up to 0.7 us (bf16, two blocks per unit: 2304 x 2048 x 512 8.3 -> 7.6 us without).
-// Requires: N % 8 == 0, n_wave % 8 == 0, n_wave + 32 TN <= N, 16-byte aligned output / scale vectors / bias,
+// Requires: N % 8 == 0, n_wave % 8 == 0, n_wave + 32 TN <= N (RAGGED: or N and n_wave multiples of 32 TNS), 16-byte aligned
+// output / scale vectors / bias,
 // and that nobody else touches `wave_lds` (staged_epilogue_bytes<> bytes).  LDS
 // operations of one wave execute in order, so write -> read -> next write needs no barrier.
 template <bool OUT_BF16, int TNS>
@@ -153,6 +155,7 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs &g, v16f (&acc)[T
         if (vec) sa = g.sa[(m_wave + (RAGGED ? min(32 * t + lr, rows - 1) : 32 * t + lr)) * g.sa_vec];
 #pragma unroll
         for (int us = 0; us < TN; us += TNS) {
+            if (RAGGED && n_wave + 32 * us >= g.N) break;
 #pragma unroll
             for (int uu = 0; uu < TNS; ++uu) {
 #pragma unroll
@@ -231,7 +234,7 @@ __device__ __forceinline__ void epilogue_staged_accumulate(const GemmArgs &g, v1
             }
         }
     };
-    auto inside = [&](int slab) { return !RAGGED || 32 * (slab / (TN / TNS)) < rows; };
+    auto inside = [&](int slab) { return !RAGGED || (32 * (slab / (TN / TNS)) < rows && n_wave + 32 * (slab % (TN / TNS)) * TNS < g.N); };
     float old[2][NI][4];
     if (inside(0)) fetch_old(old[0], 0);
 #pragma unroll

@@ -926,3 +926,33 @@ def test_few_tile_kernels_at_ragged_edges(N, variant, M, Nn, K):
             assert torch.equal(out.cpu(), (product * 0.125 + old.double()).float().to(dtype))
     finally:
         N.gemm_set_variant(-1)
+
+
+@pytest.mark.parametrize("variant", [9, 10, 11])
+@pytest.mark.parametrize("M,Nn", [(33, 32), (100, 160), (260, 256), (70, 352), (129, 448), (300, 576)])
+def test_few_tile_kernels_where_the_columns_end_between_slabs(N, variant, M, Nn):
+    """Columns that fill some of the 32-wide slabs of a wave tile and none of the others, rows that end inside a slab: every form
+    of the output (exact sums, as above), and nothing is written behind it."""
+    K = 384
+    g = torch.Generator().manual_seed(M + Nn + variant)
+    values = torch.tensor([0.0, 0.5, 1.0, -1.0, 2.0, -0.5])
+    a, b = values[torch.randint(0, 6, (M, K), generator=g)], values[torch.randint(0, 6, (Nn, K), generator=g)]
+    ac, bc = (t.to(torch.float8_e4m3fn).view(torch.uint8).cuda() for t in (a, b))
+    product = a.double() @ b.double().t()
+    one = torch.tensor([0.5]).cuda()
+    sa, sb = 2.0 ** torch.randint(-1, 2, (M,), generator=g), 2.0 ** torch.randint(-1, 2, (Nn,), generator=g)
+    bias = torch.randint(-8, 8, (Nn,), generator=g).float()
+    scaled = product * sa[:, None].double() * sb[None].double() + bias.double()
+    N.gemm_set_variant(variant)
+    try:
+        for dtype in (torch.bfloat16, torch.float32):
+            guarded = torch.full((M + 300, Nn), 7.0, dtype=dtype, device="cuda")
+            N.gemm_nt(ac, bc, O.E4M3, O.E4M3, one, one, out=guarded[:M])
+            assert torch.equal(guarded[:M].cpu(), (product * 0.25).float().to(dtype)) and (guarded[M:] == 7.0).all()
+            N.gemm_nt(ac, bc, O.E4M3, O.E4M3, sa.cuda(), sb.cuda(), bias=bias.cuda(), out=guarded[:M])
+            assert torch.equal(guarded[:M].cpu(), scaled.float().to(dtype)) and (guarded[M:] == 7.0).all()
+            old = guarded[:M].double().cpu()
+            N.gemm_nt(ac, bc, O.E4M3, O.E4M3, one, one, out=guarded[:M], accumulate=True)
+            assert torch.equal(guarded[:M].cpu(), (product * 0.25 + old).float().to(dtype)) and (guarded[M:] == 7.0).all()
+    finally:
+        N.gemm_set_variant(-1)
