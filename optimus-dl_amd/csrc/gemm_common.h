@@ -288,8 +288,7 @@ __device__ __forceinline__ void epilogue_staged_accumulate(const GemmArgs &g, v1
 // what one compute unit gets from there is bounded by its latency: 64 KB in flight a microsecond, 0.53 us per K step of a 128 x
 // 128 tile however many stages wait for it and however few units ask.  The idle units bring the whole of it to the
 // memory-side cache in a fraction of the launch.  Cold operands, us without and with: 128 x 128 tiles, 3072 x 768 x 16384 71.5 ->
-// 57.8, 3072 x 1024 x 8192 38.8 -> 33.4, 1024 x 1024 x 4096 21.5 -> 15.9, 512 x 3072 x 768 8.1 -> 7.2 (warm ones 51.7 -> 54.8, 29.4 ->
-// 30.0, 15.9 -> 15.8, 6.4 -> 6.5).
+// 57.8, 3072 x 1024 x 8192 38.8 -> 33.4, 1024 x 1024 x 4096 21.5 -> 15.9 (warm ones 51.7 -> 54.8, 29.4 -> 30.0, 15.9 -> 15.8).
 // A helper reads kb_per_step KB per K step at most (what it can while a step is multiplied); where that does not cover the
 // operands, their last K bytes are read.
 __device__ __forceinline__ void warm_operands(const GemmArgs &g, int helper, int helpers, int kb_per_step) {

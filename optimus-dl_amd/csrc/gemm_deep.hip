@@ -20,8 +20,8 @@
 //   * the loads of step kt + 3 go into the stage that step kt lay in, two whole steps ahead of their use;
 //   * one barrier per step.  Behind it everybody has read stage kt into registers and everybody's loads of stage kt + 1
 //     have landed: a wave's loads complete in order, so that is "at most one step's loads outstanding".
-// Against the kernel it replaces (eight waves, four stages, fragments read as they are needed), bf16 outputs in us:
-// 2048 x 2048 x 1024 8.1 -> 8.3, x 2048 12.1 -> 11.6, x 4096 20.8 -> 18.6, x 8192 36.4 -> 31.2; 3072 x 1024 x 8192 fp32
+// Against the four-stage tiled kernel (eight waves, fragments read as they are needed), which keeps the contractions of less
+// than 16 steps (gemm_few_tiles), bf16 outputs in us: 2048 x 2048 x 2048 12.1 -> 11.6, x 4096 20.8 -> 18.6, x 8192 36.4 -> 31.2; 3072 x 1024 x 8192 fp32
 // 35.3 -> 28.3; 1024 x 4096 x 14336 65.3 -> 52.5 (operands in the memory-side cache).  Four or five stages: the same but for
 // 0.2 us a launch and stage.
 //

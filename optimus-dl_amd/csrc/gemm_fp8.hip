@@ -143,14 +143,17 @@ static bool thin_pays(int64_t M, int64_t N, int64_t K) {
 }
 
 // The kernel for an output of at most num_cus / 2 tiles of 256 x 256, which the big tiles would leave half the chip idle on
-// (kManyTiles: the output has more).  At most one 128 x 128 tile per unit: the pipelined kernel of gemm_deep.hip.  At most one of
+// (kManyTiles: the output has more).  At most one 128 x 128 tile per unit: from 16 K steps on the pipelined kernel of
+// gemm_deep.hip; with fewer its longer way to the first MFMA (the second stage has to be there) costs more than its steps
+// gain, and the four-stage form of the tiled kernel runs (1024 x 1024, warm and cold operands, deep / four stages: x 512 6.5 / 5.9 and
+// 6.1 / 5.4 us, x 1024 7.6 / 7.6 and 7.5 / 7.2, x 1536 8.7 / 9.1 and 9.3 / 8.9, x 2048 9.7 / 10.7 and 10.4 / 10.7).  At most one of
 // 128 x 192 and 8 K steps or more: those (against the better of the other two, cold operands: 8192 x 768 x 2048 19.1 -> 17.0 us, x 16384
 // 104 -> 93.8; 3072 x 1536 x 4096 fp32 27.0 -> 23.8; 5120 x 1152 x 1024 13.2 -> 12.4; but 3072 x 1920 x 768 9.6 -> 9.8, 8192 x 768 x 512 8.4
 // -> 8.7, where two blocks per unit hide each other's ends).  More: 256 x 128 tiles of the same kernel, one per unit, from 24 K steps on (2048 x 4096 x 8192 52.9 us against 60.5 with two 128 x 128
 // blocks per unit, x 4096 30.3 against 32.4); with fewer steps the blocks that hide each other's fill and drain win (x 2048:
 // 18.0 against 18.4, x 1024 11.6 against 12.7).
 FewTiles gemm_few_tiles(int64_t M, int64_t N, int64_t K, int num_cus) {
-    if (((M + 127) / 128) * ((N + 127) / 128) <= num_cus) return kDeep;
+    if (((M + 127) / 128) * ((N + 127) / 128) <= num_cus) return K >= 2048 ? kDeep : kTwoBlocks;
     if (((M + 255) / 256) * ((N + 255) / 256) * 2 > num_cus) return kManyTiles;
     if (K >= 1024 && ((M + 127) / 128) * ((N + 191) / 192) <= num_cus) return kDeep192;
     return K >= 3072 && ((M + 255) / 256) * ((N + 127) / 128) <= num_cus ? kDeepWide : kTwoBlocks;

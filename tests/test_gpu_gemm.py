@@ -99,9 +99,10 @@ def test_random_gemm_within_tolerance_auto_variant(N, shape):
     assert err <= TOL, f"{shape}: max rel err {err}"
 
 
-@pytest.mark.parametrize("k_steps", [1, 2, 3, 4, 5, 6, 7, 9, 13])
+@pytest.mark.parametrize("k_steps", [1, 2, 3, 4, 5, 6, 7, 9, 13, 15, 16, 17])
 def test_few_tile_outputs_at_every_pipeline_depth(N, k_steps):
-    """Outputs of at most one 128 x 128 tile per compute unit take the four-stage form of the tiled kernel: every length
+    """Outputs of at most one 128 x 128 tile per compute unit take the four-stage form of the tiled kernel (from 16 steps on the
+    pipelined one): every length
     of its prologue and tail (1 .. 3 K steps in flight, a trip count that is not a multiple of four), interior and
     ragged tiles, one-hot rows so that a misplaced stage shows as a wrong element rather than as noise."""
     M, Nn, K = 384, 200, 128 * k_steps

@@ -287,9 +287,10 @@ def test_mx_gemm_matches_emulation(N, shape, fmts):
         assert torch.equal(got, got32.bfloat16())
 
 
-@pytest.mark.parametrize("k_steps", [1, 2, 3, 4, 5, 6, 7, 9, 13])
+@pytest.mark.parametrize("k_steps", [1, 2, 3, 4, 5, 6, 7, 9, 13, 15, 16, 17])
 def test_mx_gemm_few_tile_outputs_at_every_pipeline_depth(N, k_steps):
-    """The four-stage form of the tiled kernel (outputs of at most one 128 x 128 tile per compute unit): every length of
+    """The four-stage form of the tiled kernel (outputs of at most one 128 x 128 tile per compute unit; the pipelined kernel from 16
+    steps on): every length of
     its prologue and tail, with scale bytes that differ from K step to K step so that a scale dword that arrives with
     the wrong stage shows."""
     M, N_, K = 384, 200, 128 * k_steps

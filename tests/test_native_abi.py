@@ -169,6 +169,24 @@ def test_whole_k_steps_never_run_the_generic_kernel():
         native.gemm_route(16, 16, 20)
 
 
+def test_short_contractions_of_few_tiles_keep_the_four_stage_kernel():
+    """At most one 128 x 128 tile per compute unit: the tiled kernel below 16 K steps, the pipelined one from there on; more tiles
+    in 128 x 192 from 8 steps on."""
+    from optimus_dl_amd import native
+
+    if not native.is_built():
+        pytest.skip("library not built")
+    names = native.gemm_variants()
+    deep, wide = (next(i for i, n in enumerate(names) if n.startswith(tile) and "three stages" in n) for tile in ("128x128x128", "128x192x128"))
+    tiled = next(i for i, n in enumerate(names) if n.startswith("128x128x128") and "three stages" not in n)
+    for M, N in ((512, 768), (1024, 1024), (2048, 2048), (130, 16), (4016, 768)):
+        for K in (128, 512, 1920):
+            assert native.gemm_route(M, N, K) == (tiled, 0, 0), (M, N, K)
+        assert native.gemm_route(M, N, 2048, accumulate=True)[0] in (deep, 8)
+    assert native.gemm_route(1024, 1024, 2048) == (deep, 0, 0)
+    assert native.gemm_route(1024, 5632, 512)[0] == tiled and native.gemm_route(1024, 5632, 1024)[0] == wide
+
+
 def test_data_gradient_sums_run_in_one_launch_only_for_whole_wave_tiles():
     """Whether the members' products are rounded once or one by one depends on the token count like this and no other way:
     multiples of 128 with more than 128 output tiles go in one launch."""
