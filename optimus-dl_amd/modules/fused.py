@@ -199,8 +199,10 @@ def swiglu_few_rows(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
     if recipe is None or recipe.recipe.kind != "tensorwise" or not no_graph() or _any_global_hook is None or _any_global_hook():
         return None
     w1, w2 = mlp.w1, mlp.w2
+    if not (_runs_as_written(w1) and _runs_as_written(w2)):       # (whatever may have been put in their place, a wrapper say)
+        return None
     k = w1.in_features
-    if x.numel() > 64 * k or k % 128 or w2.out_features != w1.out_features or w2.in_features != k or not (_runs_as_written(w1) and _runs_as_written(w2)):
+    if x.numel() > 64 * k or k % 128 or w2.out_features != w1.out_features or w2.in_features != k:
         return None
     if (torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype) != torch.bfloat16:
         return None

@@ -548,3 +548,34 @@ def test_untraced_functions_stay_out_of_compiled_graphs():
     x = torch.ones(4)
     assert torch.equal(torch.compile(model, backend=backend)(x), model(x))
     assert seen == [False, False] and len(graphs) == 2          # what lies before and behind the call, never the call
+
+
+def test_decode_step_of_an_mlp_whose_linears_were_wrapped_stands_back():
+    """A wrapper put in the place of w1 after the MLP was fused (an adapter, say) has no sizes of its own to ask for."""
+    from types import SimpleNamespace
+
+    from optimus_dl_amd.modules.amp import state
+    from optimus_dl_amd.modules.fp8_linear import FP8Linear
+    from optimus_dl_amd.modules.fused import swiglu_few_rows, swiglu_mlp
+    from optimus_dl_amd.modules.model.blocks import SwiGLUMLP
+
+    class Adapter(nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, x):
+            return self.inner(x)
+
+    for name in ("w1", "w2"):
+        mlp = SwiGLUMLP(128, 256)
+        for n in ("w1", "w2", "c_proj"):
+            setattr(mlp, n, FP8Linear.from_linear(getattr(mlp, n)))
+        setattr(mlp, name, Adapter(getattr(mlp, name)))
+        for kind, call, grad in (("tensorwise", swiglu_few_rows, False), ("delayed", swiglu_mlp, True)):
+            state.push_recipe(SimpleNamespace(recipe=SimpleNamespace(kind=kind), wgrad=True, fuse_wgrad_accumulation=False, fuse_dgrad_sum=True))
+            try:
+                with torch.set_grad_enabled(grad):
+                    assert call(mlp, torch.zeros(16, 128, dtype=torch.bfloat16, requires_grad=grad)) is None
+            finally:
+                state.pop_recipe()
