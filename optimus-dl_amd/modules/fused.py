@@ -194,7 +194,7 @@ def swiglu_mlp(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
 @untraced
 def swiglu_few_rows(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
     """``silu(w1 x) * w2 x`` of a decode step in one launch (``native.gemm_swiglu``), or None: only per-tensor current scaling,
-    no graph, at most 64 rows, no biases, no hooks."""
+    no graph, few rows (``native.gemm_swiglu_pays``), no biases, no hooks."""
     recipe = _state.active_recipe()
     if recipe is None or recipe.recipe.kind != "tensorwise" or not no_graph() or _any_global_hook is None or _any_global_hook():
         return None
@@ -202,7 +202,7 @@ def swiglu_few_rows(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
     if not (_runs_as_written(w1) and _runs_as_written(w2)):       # (whatever may have been put in their place, a wrapper say)
         return None
     k = w1.in_features
-    if x.numel() > 64 * k or k % 128 or w2.out_features != w1.out_features or w2.in_features != k:
+    if w2.out_features != w1.out_features or w2.in_features != k or not native.gemm_swiglu_pays(x.numel() // max(k, 1), w1.out_features, k):
         return None
     if (torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype) != torch.bfloat16:
         return None

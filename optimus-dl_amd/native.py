@@ -960,6 +960,20 @@ def gemm_nt_sum(a: "list[torch.Tensor]", b: "list[torch.Tensor]", fmt_a: int, fm
     return out
 
 
+def gemm_swiglu_pays(M: int, N: int, K: int) -> bool:
+    """Whether :func:`gemm_swiglu` takes a shape and is faster than two :func:`gemm_nt` and the SwiGLU kernel.  A block owns 16
+    columns and, from 33 rows on, has a compute unit to itself: rounds of blocks cost it more than they cost the separate
+    products.  Up to 32 rows four rounds (N <= 16384): 1.1 to 3.9 times as fast over K = 256 .. 8192 (N = 28672 0.8 to 1.2, 50304 0.6 to
+    1.0).  Up to 64 rows one round, below K = 2048 (where separate products run the kernel of few rows, too): 1.3 to 1.7
+    times as fast, where two rounds are 0.6 to 0.9, 14336 columns 0.4 to 0.7, and K = 2048 .. 8192 in one round 0.9 to 1.2.  us,
+    one launch / three, cold weights: 32 x 1024 -> 3072 6.0 / 18.3, 32 x 4096 -> 14336 37.2 / 44.8, 64 x 1024 -> 3072 11.5 / 18.8, 64 x
+    2048 -> 5632 33.0 / 22.7, 64 x 4096 -> 14336 79.4 / 49.4."""
+    if not (0 < M <= 64 and N > 0 and N % 4 == 0 and K > 0 and K % 128 == 0 and N * K < 2**32 and M * K < 2**32):
+        return False
+    columns = (N + 15) // 16
+    return columns <= 4 * 256 if M <= 32 else (columns <= 256 and K < 2048)
+
+
 def gemm_swiglu(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, fmt_x: int, fmt_w: int, sx_inv: torch.Tensor, sg_inv: torch.Tensor,
                 su_inv: torch.Tensor):
     """h = silu(x . gate^T) * (x . up^T) in bf16 for at most 64 rows (the roundings of two products and :func:`swiglu_amax_parts`),

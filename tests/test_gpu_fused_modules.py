@@ -539,6 +539,10 @@ def test_decode_step_of_a_swiglu_mlp(amp):
         y = mlp(x)
         many = mlp(x.expand(32, 8, 256).contiguous())
         assert fused.swiglu_few_rows(mlp, x.expand(32, 8, 256)) is None
+        assert fused.swiglu_few_rows(mlp, x.expand(32, 2, 256)) is not None
+        wide, _ = make_mlp(256, 4352)                         # 64 rows and two rounds of blocks: the separate launches are faster
+        assert fused.swiglu_few_rows(wide, x.expand(32, 2, 256)) is None and wide(x.expand(32, 2, 256)).shape == (32, 2, 256)
+        assert fused.swiglu_few_rows(wide, x) is not None
         seen = []
         hook = mlp.w2.register_forward_hook(lambda m, a, o: seen.append(o.shape))
         assert fused.swiglu_few_rows(mlp, x) is None

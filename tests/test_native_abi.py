@@ -187,6 +187,18 @@ def test_short_contractions_of_few_tiles_keep_the_four_stage_kernel():
     assert native.gemm_route(1024, 5632, 512)[0] == tiled and native.gemm_route(1024, 5632, 1024)[0] == wide
 
 
+def test_gate_up_and_product_in_one_launch_only_where_that_is_faster():
+    """Up to 32 rows four rounds of 16-column blocks, up to 64 rows one round and a short contraction; never more than the entry
+    takes (operands under 4 GiB): what it would refuse goes to the separate products, as it always has."""
+    from optimus_dl_amd.native import gemm_swiglu_pays as pays
+
+    assert pays(32, 14336, 4096) and pays(16, 16384, 128) and pays(64, 3072, 1024) and pays(48, 4096, 1920) and pays(32, 14336, 8192)
+    assert not pays(16, 16388, 128) and not pays(32, 28672, 8192) and not pays(64, 4112, 1024) and not pays(48, 3072, 2048)
+    assert not pays(48, 5632, 2048) and not pays(64, 14336, 4096) and not pays(33, 14336, 1024)
+    assert not pays(65, 3072, 1024) and not pays(0, 3072, 1024) and not pays(32, 3074, 1024) and not pays(32, 3072, 1040)
+    assert not pays(16, 16384, 2**18)
+
+
 def test_data_gradient_sums_run_in_one_launch_only_for_whole_wave_tiles():
     """Whether the members' products are rounded once or one by one depends on the token count like this and no other way:
     multiples of 128 with more than 128 output tiles go in one launch."""
