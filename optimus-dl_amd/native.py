@@ -331,10 +331,11 @@ def amax_parts(x: torch.Tensor) -> torch.Tensor:
     """AMAX_PARTS partial maxima of |x| (no atomics); input of :func:`cast_dynamic`.  The kernel
     writes every entry, so the buffer is a fresh allocation per call: callers on several threads
     cannot get each other's partials."""
-    load()
-    r = _host.amax_parts(x, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_amax_parts")
+    if x.is_cuda:
+        load()
+        r = _host.amax_parts(x, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_amax_parts")
     x = _as_2d(x)
     rows, cols = x.shape
     parts = torch.empty(AMAX_PARTS, dtype=torch.float32, device=x.device)
@@ -355,10 +356,11 @@ def colsum_supported(x: torch.Tensor) -> bool:
 
 def amax_parts_colsum(x: torch.Tensor):
     """Partial maxima of |x| and the fp32 column sums of x in one pass.  -> (parts, colsum[cols])."""
-    load()
-    r = _host.amax_colsum(x, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_amax_parts_colsum")
+    if x.is_cuda:
+        load()
+        r = _host.amax_colsum(x, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_amax_parts_colsum")
     x = _as_2d(x)
     rows, cols = x.shape
     parts = torch.empty(AMAX_PARTS, dtype=torch.float32, device=x.device)
@@ -388,10 +390,11 @@ def cast_dynamic(x: torch.Tensor, parts: torch.Tensor, fmt: int, margin: int = 0
     several tensors); implies want_transposed.  rows_out: the codes get that many rows (q [rows_out, cols], q_t
     [cols, rows_out]), zero codes behind those of x (see :func:`padded_rows`).
     -> (q or None, q_t or None, amax, scale, scale_inv); the last three are fp32[1]."""
-    load()
-    r = _host.cast_dynamic(x, parts, fmt, margin, want_rowmajor, want_transposed, out_t, rows_out, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_cast_dynamic")
+    if x.is_cuda:
+        load()
+        r = _host.cast_dynamic(x, parts, fmt, margin, want_rowmajor, want_transposed, out_t, rows_out, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_cast_dynamic")
     want_transposed = want_transposed or out_t is not None
     if not (want_rowmajor or want_transposed):
         raise NativeError("cast_dynamic: nothing to produce")
@@ -536,11 +539,12 @@ def quantize_dynamic(x: torch.Tensor, fmt: int, margin: int = 0, want_rowmajor: 
 def quantise_small(x: torch.Tensor, fmt: int, margin: int = 0):
     """Row-major codes of :func:`quantize_dynamic` in one launch (one block: at most 256 KB, a multiple of 16 elements), or by
     that function where the tensor is larger or not dense.  -> (q, None, amax, scale, scale_inv)."""
-    load()
-    r = _host.quantise_small(x, fmt, margin, _stream())
-    if r is None:
-        return quantize_dynamic(x, fmt, margin, want_transposed=False)
-    return _done(r, "odl_fp8_quantise_small")
+    if x.is_cuda:
+        load()
+        r = _host.quantise_small(x, fmt, margin, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_quantise_small")
+    return quantize_dynamic(x, fmt, margin, want_transposed=False)
 
 
 def _bf16_dense(t: torch.Tensor, what: str) -> torch.Tensor:
@@ -558,10 +562,11 @@ def _bf16_dense(t: torch.Tensor, what: str) -> torch.Tensor:
 def swiglu_amax_parts(gate: torch.Tensor, up: torch.Tensor):
     """h = silu(gate) * up as eager bf16 arithmetic leaves it, and the partial maxima of |h| for
     :func:`cast_dynamic`.  -> (h, parts)."""
-    load()
-    r = _host.swiglu(gate, up, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_swiglu_amax_parts")
+    if gate.is_cuda:
+        load()
+        r = _host.swiglu(gate, up, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_swiglu_amax_parts")
     gate, up = _bf16_dense(gate, "swiglu gate"), _bf16_dense(up, "swiglu up")
     if gate.shape != up.shape:
         raise NativeError(f"swiglu: gate {tuple(gate.shape)} and up {tuple(up.shape)} differ")
@@ -577,10 +582,11 @@ def swiglu_amax_parts(gate: torch.Tensor, up: torch.Tensor):
 def swiglu_bwd_amax_parts(dh: torch.Tensor, gate: torch.Tensor, up: torch.Tensor):
     """Gradients of silu(gate) * up for grad_output dh, with their partial maxima.
     -> (d_gate, d_up, parts_d_gate, parts_d_up)."""
-    load()
-    r = _host.swiglu_bwd(dh, gate, up, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_swiglu_bwd_amax_parts")
+    if gate.is_cuda:
+        load()
+        r = _host.swiglu_bwd(dh, gate, up, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_swiglu_bwd_amax_parts")
     dh, gate, up = _bf16_dense(dh, "swiglu dh"), _bf16_dense(gate, "swiglu gate"), _bf16_dense(up, "swiglu up")
     if not (dh.shape == gate.shape == up.shape):
         raise NativeError(f"swiglu backward: shapes {tuple(dh.shape)}, {tuple(gate.shape)}, {tuple(up.shape)} differ")
@@ -598,10 +604,11 @@ def swiglu_bwd_amax_parts(dh: torch.Tensor, gate: torch.Tensor, up: torch.Tensor
 def rmsnorm_amax_parts(x: torch.Tensor, weight: torch.Tensor, eps: float):
     """y = bf16(x * rsqrt(mean(x^2, -1) + eps) * weight) over the last axis, the per-row
     1/rms, and the partial maxima of |y|.  x: bf16 or fp32.  -> (y bf16, rstd fp32, parts)."""
-    load()
-    r = _host.rmsnorm(x, weight, eps, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_rmsnorm_amax_parts")
+    if x.is_cuda:
+        load()
+        r = _host.rmsnorm(x, weight, eps, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_rmsnorm_amax_parts")
     if not x.is_cuda:
         raise NativeError(f"rmsnorm: the kernels run on the GPU only; got a tensor on {x.device}")
     src = _src_dtype(x)
@@ -623,10 +630,11 @@ RMSNORM_BWD_SLABS = 512
 def rmsnorm_bwd(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, rstd: torch.Tensor):
     """Gradients of :func:`rmsnorm_amax_parts`'s y for grad_output dy (bf16).
     -> (dx in the dtype of x, d_weight fp32[cols])."""
-    load()
-    r = _host.rmsnorm_bwd(dy, x, weight, rstd, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_rmsnorm_bwd")
+    if x.is_cuda:
+        load()
+        r = _host.rmsnorm_bwd(dy, x, weight, rstd, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_rmsnorm_bwd")
     dy = _bf16_dense(dy, "rmsnorm dy")
     src = _src_dtype(x)
     x = _dense_16(x)
@@ -671,10 +679,11 @@ def _dense_16(x: torch.Tensor) -> torch.Tensor:
 def layernorm_amax_parts(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, eps: float):
     """y = bf16(layer_norm(x) * weight + bias) over the last axis, per-row mean and 1/std, and the
     partial maxima of |y|.  x: bf16 or fp32.  -> (y bf16, mean fp32, rstd fp32, parts)."""
-    load()
-    r = _host.layernorm(x, weight, bias, eps, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_layernorm_amax_parts")
+    if x.is_cuda:
+        load()
+        r = _host.layernorm(x, weight, bias, eps, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_layernorm_amax_parts")
     if not x.is_cuda:
         raise NativeError(f"layernorm: the kernels run on the GPU only; got a tensor on {x.device}")
     src = _src_dtype(x)
@@ -695,10 +704,11 @@ def layernorm_amax_parts(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tens
 def layernorm_bwd(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, mean: torch.Tensor, rstd: torch.Tensor):
     """Gradients of :func:`layernorm_amax_parts`'s y for grad_output dy (bf16).
     -> (dx in the dtype of x, d_weight fp32[cols], d_bias fp32[cols])."""
-    load()
-    r = _host.layernorm_bwd(dy, x, weight, mean, rstd, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_layernorm_bwd")
+    if x.is_cuda:
+        load()
+        r = _host.layernorm_bwd(dy, x, weight, mean, rstd, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_layernorm_bwd")
     dy = _bf16_dense(dy, "layernorm dy")
     src = _src_dtype(x)
     x = _dense_16(x)
@@ -779,10 +789,11 @@ def quantize_rowcol(x: torch.Tensor, fmt: int, margin: int = 0, rows_out: int | 
     """Rowwise recipe, both operands of one tensor in two passes over it:
     -> (q [rows, cols] scaled per row, s_row_inv [rows], q_t [cols, rows] scaled per column, s_col_inv [cols],
         amax_row, amax_col).  rows_out: as in :func:`cast_dynamic`."""
-    load()
-    r = _host.quantize_rowcol(x, fmt, margin, rows_out, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_amax_rowcol / odl_fp8_cast_rowcol")
+    if x.is_cuda:
+        load()
+        r = _host.quantize_rowcol(x, fmt, margin, rows_out, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_amax_rowcol / odl_fp8_cast_rowcol")
     x = _as_2d(x)
     rows, cols = x.shape
     pr, pc = -(-rows // 4) * 4, -(-cols // 4) * 4            # every vector starts on a 16-byte boundary (the GEMM wants that)
@@ -855,10 +866,11 @@ def cast_delayed(x: torch.Tensor, scale: torch.Tensor, fmt: int, amax_parts: tor
     recorded), and 1/scale in a fresh 1-element tensor that later refreshes of ``scale`` do not touch.  out_t, rows_out:
     as in :func:`cast_dynamic`.
     -> (codes or None, codes_t or None, scale_inv[1])."""
-    load()
-    r = _host.cast_delayed(x, scale, fmt, amax_parts, want_rowmajor, want_transposed, out_t, rows_out, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_cast_delayed")
+    if x.is_cuda:
+        load()
+        r = _host.cast_delayed(x, scale, fmt, amax_parts, want_rowmajor, want_transposed, out_t, rows_out, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_cast_delayed")
     x = _as_2d(x)
     rows, cols = x.shape
     _f32_dev(scale, 1, "cast_delayed scale")
@@ -887,9 +899,9 @@ def gemm_nt(a: torch.Tensor, b: torch.Tensor, fmt_a: int, fmt_b: int, sa_inv: to
             out: torch.Tensor | None = None, accumulate: bool = False) -> torch.Tensor:
     """out[M,N] = (a[M,K] . b[N,K]^T) * (sa_inv x sb_inv) (+ bias); a, b uint8 FP8 codes.  A given ``out`` decides the
     output type.  accumulate: out = out + product (needs ``out``; the old value joins the fp32 sum, one rounding)."""
-    load()
     odt = _OUT_DTYPES.get(out_dtype, -1)
-    if odt >= 0:
+    if odt >= 0 and a.is_cuda:
+        load()
         r = _host.gemm_nt(a, b, fmt_a, fmt_b, sa_inv, sb_inv, bias, odt, out, accumulate, _may_split(), _stream())
         if r is not None:
             return _done(r, "odl_fp8_gemm_nt")
@@ -978,8 +990,10 @@ def gemm_swiglu(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, fmt_x: in
                 su_inv: torch.Tensor):
     """h = silu(x . gate^T) * (x . up^T) in bf16 for at most 64 rows (the roundings of two products and :func:`swiglu_amax_parts`),
     in one launch; x, gate, up uint8 FP8 codes [M, K], [N, K], [N, K] with one inverse scale each.  -> (h, partial maxima of |h|)."""
-    load()
-    r = _host.gemm_swiglu(x, gate, up, fmt_x, fmt_w, sx_inv, sg_inv, su_inv, _stream())
+    r = None
+    if x.is_cuda:
+        load()
+        r = _host.gemm_swiglu(x, gate, up, fmt_x, fmt_w, sx_inv, sg_inv, su_inv, _stream())
     if r is None:
         raise NativeError("gemm_swiglu: dense uint8 codes [M, K], [N, K], [N, K] and one fp32 scale each expected")
     return _done(r, "odl_fp8_gemm_swiglu")
@@ -1018,8 +1032,8 @@ def mx_cast(x: torch.Tensor, fmt: int, want_rowmajor: bool = True, want_transpos
     blocked axis allows it).  scale_rule: MX_FLOOR (the OCP formula; a block amax in the top eighth of its binade
     saturates) or MX_CEIL (the exponent rounded up: nothing saturates).  rows_out: the transposed codes and their scales are
     that many rows of x long, zero codes with scale byte 0 behind those of x (see :func:`padded_rows`)."""
-    load()
-    if layout is None:
+    if layout is None and x.is_cuda:
+        load()
         r = _host.mx_cast(x, fmt, want_rowmajor, want_transposed, int(scale_rule), rows_out, _stream())
         if r is not None:
             return _done(r, "odl_fp8_mx_cast")
@@ -1145,10 +1159,11 @@ def block_cast(x: torch.Tensor, fmt: int, margin: int = 0, two_d: bool = False, 
     per 128 x 128 block (two_d True, weights).  -> (codes [rows, cols], scales [cols/128, rows, 4], codes_t [cols, rows],
     scales_t [rows/128, cols, 4]); the scale tensors hold E8M0 bytes in the K-step-major layout, each block's byte four
     times, and go to ``mx_gemm_nt`` as they are.  The pair that was not asked for is (None, None)."""
-    load()
-    r = _host.block_cast(x, fmt, margin, two_d, want_rowmajor, want_transposed, _stream())
-    if r is not None:
-        return _done(r, "odl_fp8_block_cast")
+    if x.is_cuda:
+        load()
+        r = _host.block_cast(x, fmt, margin, two_d, want_rowmajor, want_transposed, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_block_cast")
     x = _as_2d(x)
     rows, cols = x.shape
     if not (want_rowmajor or want_transposed):
@@ -1175,11 +1190,10 @@ def mx_gemm_nt(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Ten
     """out[M,N] = sum over 32-blocks of 2^(sa-127) 2^(sb-127) (a_block . b_block) (+ bias); a [M,K], b [N,K] codes,
     sa, sb their E8M0 scale bytes as ``mx_cast`` returns them (both row-major [rows, K/32] or both K-step-major
     [K/128, rows, 4])."""
-    load()
-    if a.is_cuda:
-        init_device(a.device)
     odt = _OUT_DTYPES.get(out_dtype, -1)
-    if odt >= 0:
+    if odt >= 0 and a.is_cuda:
+        load()
+        init_device(a.device)
         r = _host.mx_gemm_nt(a, sa, b, sb, fmt_a, fmt_b, bias, odt, out, accumulate, _may_split(), _stream())
         if r is not None:
             return _done(r, "odl_fp8_mx_gemm_nt")
@@ -1324,9 +1338,9 @@ def gemm_layouts(a: torch.Tensor, b: torch.Tensor, fmt_a: int, fmt_b: int, layou
     ``out`` decides the output type, else ``out_dtype`` does.  accumulate: out = out + product (needs ``out``); the
     product then passes through an fp32 workspace (``odl_fp8_gemm_splitk``, with one run where K is not worth cutting),
     because the kernel that reads K-slow operands stores a tile where nothing can wait for the old values."""
-    load()
     odt = _OUT_DTYPES.get(out_dtype, -1)
-    if odt >= 0 and not accumulate:
+    if odt >= 0 and not accumulate and a.is_cuda:
+        load()
         r = _host.gemm_layouts(a, b, fmt_a, fmt_b, layout_a == K_SLOW, layout_b == K_SLOW, sa_inv, sb_inv, out, odt, _may_split(), _stream())
         if r is not None:
             return _done(r, "odl_fp8_gemm_layouts")

@@ -91,6 +91,30 @@ def test_cpu_tensors_are_refused_not_emulated():
         native.amax(torch.zeros((4, 4), dtype=torch.bfloat16))
 
 
+def test_every_wrapper_refuses_cpu_tensors_with_an_error_of_its_own():
+    """Also where no GPU is visible, where asking torch for the current stream would raise something else."""
+    import torch
+
+    from optimus_dl_amd import native as N
+
+    x, codes, one = torch.zeros((128, 128), dtype=torch.bfloat16), torch.zeros((128, 512), dtype=torch.uint8), torch.ones(1)
+    parts, row = torch.ones(N.AMAX_PARTS), torch.ones(128)
+    scales = torch.zeros((4, 128, 4), dtype=torch.uint8)
+    calls = {
+        "amax_parts": (x,), "amax_parts_colsum": (x,), "cast_dynamic": (x, parts, N.E4M3), "quantise_small": (x, N.E4M3),
+        "swiglu_amax_parts": (x, x), "swiglu_bwd_amax_parts": (x, x, x), "rmsnorm_amax_parts": (x, row, 1e-5), "rmsnorm_bwd": (x, x, row, row),
+        "layernorm_amax_parts": (x, row, row, 1e-5), "layernorm_bwd": (x, x, row, row, row), "gelu_amax_parts": (x,), "gelu_bwd_amax_parts": (x, x),
+        "quantize_rowcol": (x, N.E4M3), "cast_delayed": (x, one, N.E4M3), "gemm_nt": (codes, codes, N.E4M3, N.E4M3, one, one),
+        "gemm_layouts": (codes, codes, N.E4M3, N.E4M3, N.K_FAST, N.K_FAST, one, one), "gemm_swiglu": (codes, codes, codes, N.E4M3, N.E4M3, one, one, one),
+        "mx_cast": (x, N.E4M3), "block_cast": (x, N.E4M3), "mx_gemm_nt": (codes, scales, codes, scales, N.E4M3, N.E4M3),
+        "swiglu_mx_cast": (x, x, N.E4M3, N.MX_CEIL), "swiglu_block_cast": (x, x, N.E4M3), "swiglu_cast_delayed": (x, x, one, N.E4M3, parts),
+    }
+    for name, args in calls.items():
+        with pytest.raises(N.NativeError):
+            getattr(N, name)(*args)
+            raise AssertionError(name)
+
+
 def test_build_rejects_asm_that_reads_a_scalar_too_soon_after_a_vector_write():
     from optimus_dl_amd.build import check_asm_hazards
 
