@@ -46,6 +46,7 @@ enum odl_status {
 };
 
 /* ABI version of this header; bumped when a signature changes or an entry point is added. */
+#define ODL_FP8_ABI_VERSION 23
 int odl_fp8_abi_version(void);
 
 /*

@@ -5,8 +5,11 @@
 // which copies or refuses.  An int is the status of a C entry that refused.  A step of a few hundred tokens waits for
 // the host, and of its time a third went into the wrappers: per call 5 to 9 us of Python around 3.7 us of launch, here 1 to 2.
 #include <torch/extension.h>
+#include <torch/version.h>
 
 #include <cstdint>
+
+#include "../../include/odl_fp8.h"
 
 namespace py = pybind11;
 using at::Tensor;
@@ -15,33 +18,31 @@ using i64 = int64_t;
 
 namespace {
 
-constexpr i64 kParts = 512;                 // ODL_FP8_AMAX_PARTS
-constexpr i64 kSmall = 262144;              // ODL_FP8_SMALL_BYTES
-constexpr i64 kColsumFloats = 512 * 256, kNormSlabs = 512;
+constexpr i64 kParts = ODL_FP8_AMAX_PARTS;
 
-// entries of the C library, by address (native.py loads it and hands them over)
-int (*amax_parts_c)(const void *, int, i64, i64, void *, void *);
-int (*cast_dynamic_c)(const void *, int, i64, i64, i64, const void *, int, int, void *, void *, void *, void *);
-int (*quantise_small_c)(const void *, int, i64, int, int, void *, void *, void *);
-int (*gemm_swiglu_c)(const void *, const void *, const void *, i64, i64, i64, int, int, const void *, const void *, const void *, void *, void *, void *);
-int (*cast_delayed_c)(const void *, int, i64, i64, i64, const void *, int, void *, void *, void *, void *, void *);
-int (*amax_colsum_c)(const void *, int, i64, i64, void *, void *, void *, void *);
-int (*swiglu_c)(const void *, const void *, i64, i64, void *, void *, void *);
-int (*swiglu_bwd_c)(const void *, const void *, const void *, i64, i64, void *, void *, void *, void *, void *);
-int (*gelu_c)(const void *, i64, i64, const void *, void *, void *, void *);
-int (*gelu_bwd_c)(const void *, const void *, i64, i64, const void *, void *, void *, void *);
-int (*rmsnorm_c)(const void *, int, const void *, i64, i64, float, void *, void *, void *, void *);
-int (*rmsnorm_bwd_c)(const void *, const void *, int, const void *, const void *, i64, i64, void *, void *, void *, void *);
-int (*layernorm_c)(const void *, int, const void *, const void *, i64, i64, float, void *, void *, void *, void *, void *);
-int (*layernorm_bwd_c)(const void *, const void *, int, const void *, const void *, const void *, i64, i64, void *, void *, void *, void *, void *);
-int (*amax_rowcol_c)(const void *, int, i64, i64, void *, void *, void *);
-int (*cast_rowcol_c)(const void *, int, i64, i64, i64, const void *, const void *, int, int, void *, void *, void *, void *, void *, void *, void *);
-int (*gemm_nt_c)(const void *, const void *, i64, i64, i64, int, int, const void *, i64, const void *, i64, const void *, int, void *, int, int, void *);
-int (*gemm_layouts_c)(const void *, const void *, i64, i64, i64, int, int, int, int, const void *, const void *, void *, int, void *);
-int (*split_count_c)(i64, i64, i64, int);
-int (*mx_cast_c)(const void *, int, i64, i64, i64, int, void *, void *, int, void *, void *, int, int, void *);
-int (*block_cast_c)(const void *, int, i64, i64, int, int, int, void *, void *, void *, void *, void *);
-int (*mx_gemm_nt_c)(const void *, const void *, const void *, const void *, int, i64, i64, i64, int, int, const void *, void *, int, int, void *);
+// entries of the C library: their types from the header, their addresses from native.py, which has loaded it
+decltype(&odl_fp8_amax_parts) amax_parts_c;
+decltype(&odl_fp8_cast_dynamic_padded) cast_dynamic_c;
+decltype(&odl_fp8_quantise_small) quantise_small_c;
+decltype(&odl_fp8_gemm_swiglu) gemm_swiglu_c;
+decltype(&odl_fp8_cast_delayed_padded) cast_delayed_c;
+decltype(&odl_fp8_amax_parts_colsum) amax_colsum_c;
+decltype(&odl_fp8_swiglu_amax_parts) swiglu_c;
+decltype(&odl_fp8_swiglu_bwd_amax_parts) swiglu_bwd_c;
+decltype(&odl_fp8_gelu_amax_parts) gelu_c;
+decltype(&odl_fp8_gelu_bwd_amax_parts) gelu_bwd_c;
+decltype(&odl_fp8_rmsnorm_amax_parts) rmsnorm_c;
+decltype(&odl_fp8_rmsnorm_bwd) rmsnorm_bwd_c;
+decltype(&odl_fp8_layernorm_amax_parts) layernorm_c;
+decltype(&odl_fp8_layernorm_bwd) layernorm_bwd_c;
+decltype(&odl_fp8_amax_rowcol) amax_rowcol_c;
+decltype(&odl_fp8_cast_rowcol_padded) cast_rowcol_c;
+decltype(&odl_fp8_gemm_nt) gemm_nt_c;
+decltype(&odl_fp8_gemm_layouts) gemm_layouts_c;
+decltype(&odl_fp8_gemm_split_count) split_count_c;
+decltype(&odl_fp8_mx_cast_padded) mx_cast_c;
+decltype(&odl_fp8_block_cast) block_cast_c;
+decltype(&odl_fp8_mx_gemm_nt) mx_gemm_nt_c;
 
 template <class F>
 void take(F &f, const py::dict &d, const char *name) { f = reinterpret_cast<F>(py::cast<uintptr_t>(d[name])); }
@@ -78,9 +79,15 @@ int call(F entry, A... args) {
     return entry(args...);
 }
 
-void *ptr(const Tensor &t) { return t.data_ptr(); }
-void *ptr(const OptTensor &t) { return t ? t->data_ptr() : nullptr; }
-void *str(i64 stream) { return reinterpret_cast<void *>(stream); }
+// an address, as whatever pointer the entry takes
+struct Address {
+    void *p;
+    template <class T>
+    operator T *() const { return static_cast<T *>(p); }
+};
+Address ptr(const Tensor &t) { return {t.data_ptr()}; }
+Address ptr(const OptTensor &t) { return {t ? t->data_ptr() : nullptr}; }
+Address str(i64 stream) { return {reinterpret_cast<void *>(stream)}; }
 bool aligned(const Tensor &t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
 int src_of(const Tensor &t) { return t.scalar_type() == at::kBFloat16 ? 0 : t.scalar_type() == at::kFloat ? 1 : -1; }
 bool dense(const Tensor &t) { return t.is_cuda() && t.is_contiguous() && t.layout() == at::kStrided; }
@@ -127,7 +134,7 @@ py::object cast_dynamic(const Tensor &x, const Tensor &parts, int fmt, int margi
 // a small tensor in one launch, row-major codes only
 py::object quantise_small(const Tensor &x, int fmt, int margin, i64 stream) {
     const i64 n = x.numel();
-    if (!source2d(x) || n == 0 || n * x.element_size() > kSmall || n % 16 || !aligned(x)) return none();
+    if (!source2d(x) || n == 0 || n * x.element_size() > ODL_FP8_SMALL_BYTES || n % 16 || !aligned(x)) return none();
     Tensor q = bytes(x, {x.size(0), x.size(1)}), dyn = f32(x, {3, 1});
     const int rc = call(quantise_small_c, ptr(x), src_of(x), n, fmt, margin, ptr(q), ptr(dyn), str(stream));
     return rc ? status(rc) : py::make_tuple(q, py::none(), dyn.select(0, 0), dyn.select(0, 1), dyn.select(0, 2));
@@ -158,7 +165,7 @@ py::object cast_delayed(const Tensor &x, const Tensor &scale, int fmt, const Opt
 
 py::object amax_colsum(const Tensor &x, i64 stream) {
     if (!source2d(x)) return none();
-    Tensor parts = f32(x, {kParts}), sums = f32(x, {x.size(1)}), ws = f32(x, {kColsumFloats});
+    Tensor parts = f32(x, {kParts}), sums = f32(x, {x.size(1)}), ws = f32(x, {ODL_FP8_COLSUM_WORKSPACE});
     const int rc = call(amax_colsum_c, ptr(x), src_of(x), x.size(0), x.size(1), ptr(parts), ptr(sums), ptr(ws), str(stream));
     return rc ? status(rc) : py::make_tuple(parts, sums);
 }
@@ -214,7 +221,7 @@ py::object rmsnorm_bwd(const Tensor &dy, const Tensor &x, const Tensor &w, const
     if (!bf16(dy) || !norm_input(x) || dy.sizes() != x.sizes() || !norm_vector(w, x)) return none();
     const i64 cols = x.size(-1), rows = x.numel() / std::max<i64>(cols, 1);
     if (!floats(rstd, rows)) return none();
-    Tensor dx = at::empty_like(x), dw = f32(x, {cols}), ws = f32(x, {kNormSlabs * cols});
+    Tensor dx = at::empty_like(x), dw = f32(x, {cols}), ws = f32(x, {ODL_FP8_RMSNORM_BWD_SLABS * cols});
     const int rc = call(rmsnorm_bwd_c, ptr(dy), ptr(x), src_of(x), ptr(w), ptr(rstd), rows, cols, ptr(dx), ptr(dw), ptr(ws), str(stream));
     return rc ? status(rc) : py::make_tuple(dx, dw);
 }
@@ -234,7 +241,7 @@ py::object layernorm_bwd(const Tensor &dy, const Tensor &x, const Tensor &w, con
     if (!bf16(dy) || !norm_input(x) || dy.sizes() != x.sizes() || !norm_vector(w, x)) return none();
     const i64 cols = x.size(-1), rows = x.numel() / std::max<i64>(cols, 1);
     if (!floats(mean, rows) || !floats(rstd, rows)) return none();
-    Tensor dx = at::empty_like(x), dwb = f32(x, {2 * cols}), ws = f32(x, {2 * kNormSlabs * cols});
+    Tensor dx = at::empty_like(x), dwb = f32(x, {2 * cols}), ws = f32(x, {2 * ODL_FP8_RMSNORM_BWD_SLABS * cols});
     Tensor dw = dwb.narrow(0, 0, cols), db = dwb.narrow(0, cols, cols);
     const int rc = call(layernorm_bwd_c, ptr(dy), ptr(x), src_of(x), ptr(w), ptr(mean), ptr(rstd), rows, cols, ptr(dx), ptr(dw), ptr(db), ptr(ws),
                                    str(stream));
@@ -334,6 +341,8 @@ py::object mx_gemm_nt(const Tensor &a, const Tensor &sa, const Tensor &b, const 
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    m.attr("abi_version") = ODL_FP8_ABI_VERSION;        // of the header this was compiled with
+    m.attr("torch_version") = TORCH_VERSION;
     m.def("bind", &bind);
     m.def("amax_parts", &amax_parts);
     m.def("cast_dynamic", &cast_dynamic);

@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import ctypes
 import importlib.util
+import logging
 import os
 import threading
 
@@ -92,6 +93,7 @@ EXPORTS = (
     "odl_fp8_mx_gemm_splitk",
 )
 
+logger = logging.getLogger(__name__)
 # csrc/host.cpp: the plain case of the wrappers below (see there); None until the library is loaded
 HOST_NAME = "_host"
 _host = None
@@ -110,7 +112,7 @@ def is_built() -> bool:
 def load() -> ctypes.CDLL:
     """Load the library once (torch is imported first so that its HIP runtime,
     which has the same SONAME, is the one the library binds to)."""
-    global _lib
+    global _lib, _host
     if _lib is not None:
         return _lib
     with _lock:
@@ -185,22 +187,36 @@ def load() -> ctypes.CDLL:
             getattr(L, name)  # AttributeError here = the library does not match the header
         if L.odl_fp8_abi_version() != ABI_VERSION:
             raise NativeError(f"{LIB_PATH}: ABI {L.odl_fp8_abi_version()} != expected {ABI_VERSION}; rebuild")
-        _load_host(L)
+        _host = _load_host(L)
         _lib = L
     return _lib
 
 
-def _load_host(L: ctypes.CDLL) -> None:
-    """The C++ side of the wrappers (built beside the library), bound to the entries of the library that was loaded."""
-    global _host
+class _NoHost:
+    """Stands in for the C++ side where it cannot be used: every call is left to the long way."""
+
+    def __getattr__(self, name: str):
+        return lambda *args: None
+
+
+def _load_host(L: ctypes.CDLL):
+    """The C++ side of the wrappers (built beside the library), bound to the entries of the library that was loaded.  Unlike the
+    library it belongs to one version of torch; where it is missing, or was built for another torch or another header,
+    the wrappers do its work in Python, 4 to 7 us slower a call."""
     path = os.path.join(_HERE, HOST_NAME + ".so")
-    if not os.path.exists(path):
-        raise NativeError(f"{path} is missing: build it with `python -m optimus_dl_amd.build`")
-    spec = importlib.util.spec_from_file_location(HOST_NAME, path)
-    host = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(host)
-    host.bind({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in EXPORTS})
-    _host = host
+    try:
+        spec = importlib.util.spec_from_file_location(HOST_NAME, path)
+        host = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(host)
+        built_for = getattr(host, "abi_version", None), getattr(host, "torch_version", None)
+        if built_for != (ABI_VERSION, torch.__version__.split("+")[0]):
+            raise ImportError(f"built for ABI {built_for[0]} and torch {built_for[1]}, this is {ABI_VERSION} and {torch.__version__}")
+        host.bind({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in EXPORTS})
+    except (ImportError, OSError) as e:
+        logger.warning("%s is not usable, calls into the FP8 library are slower on the host (rebuild with `python -m optimus_dl_amd.build`): %s",
+                       path, e)
+        return _NoHost()
+    return host
 
 
 def _done(r, what: str):
@@ -990,13 +1006,24 @@ def gemm_swiglu(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, fmt_x: in
                 su_inv: torch.Tensor):
     """h = silu(x . gate^T) * (x . up^T) in bf16 for at most 64 rows (the roundings of two products and :func:`swiglu_amax_parts`),
     in one launch; x, gate, up uint8 FP8 codes [M, K], [N, K], [N, K] with one inverse scale each.  -> (h, partial maxima of |h|)."""
-    r = None
     if x.is_cuda:
         load()
         r = _host.gemm_swiglu(x, gate, up, fmt_x, fmt_w, sx_inv, sg_inv, su_inv, _stream())
-    if r is None:
-        raise NativeError("gemm_swiglu: dense uint8 codes [M, K], [N, K], [N, K] and one fp32 scale each expected")
-    return _done(r, "odl_fp8_gemm_swiglu")
+        if r is not None:
+            return _done(r, "odl_fp8_gemm_swiglu")
+    for t in (x, gate, up):
+        if not (t.is_cuda and t.dtype == torch.uint8 and t.dim() == 2 and t.is_contiguous()):
+            raise NativeError("gemm_swiglu: dense uint8 codes [M, K], [N, K], [N, K] on the GPU expected")
+    (M, K), N = x.shape, gate.shape[0]
+    if gate.shape != up.shape or gate.shape[1] != K:
+        raise NativeError(f"gemm_swiglu: {tuple(x.shape)}, {tuple(gate.shape)}, {tuple(up.shape)} do not fit")
+    for t in (sx_inv, sg_inv, su_inv):
+        _f32_dev(t, 1, "gemm_swiglu scale")
+    h = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    parts = torch.empty(AMAX_PARTS, dtype=torch.float32, device=x.device)
+    _check(load().odl_fp8_gemm_swiglu(x.data_ptr(), gate.data_ptr(), up.data_ptr(), M, N, K, fmt_x, fmt_w, sx_inv.data_ptr(), sg_inv.data_ptr(),
+                                      su_inv.data_ptr(), h.data_ptr(), parts.data_ptr(), _stream()), "odl_fp8_gemm_swiglu")
+    return h, parts
 
 
 MX_BLOCK = 32

@@ -527,6 +527,30 @@ def test_gate_up_and_product_of_a_few_rows_in_one_launch(rows, width, hidden):
     assert parts.max().item() == h.float().abs().max().item() and (parts >= 0).all()
 
 
+@pytest.mark.parametrize("kind", ["tensorwise", "delayed", "rowwise", "mxfp8", "blockwise"])
+def test_modules_without_the_cpp_side_of_the_wrappers(amp, monkeypatch, kind):
+    """The long way through the wrappers gives the same bits: training step, evaluation and decode step of an MLP."""
+    from optimus_dl_amd import native as N
+
+    N.load()
+    results = []
+    for host in (N._host, N._NoHost()):
+        monkeypatch.setattr(N, "_host", host)
+        mlp, _ = make_mlp(256, 512)
+        recipe = amp.create_fp8_recipe(kind, "hybrid", amax_history_len=4)
+        x = seeded_bf16((256, 256), 1.0, 3).cuda().requires_grad_(True)
+        with recipe.autocast():
+            y = mlp(x)
+        with recipe.backward():
+            y.backward(seeded_bf16((256, 256), 1e-3, 4).cuda())
+        out = [y.detach(), x.grad, *(p.grad for p in mlp.parameters())]
+        mlp.eval()
+        with recipe.autocast(), torch.no_grad():
+            out += [mlp(x), mlp(x[:128]), mlp(x[:32])]
+        results.append(out)
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
 def test_decode_step_of_a_swiglu_mlp(amp):
     """Evaluation of a few rows takes the one launch; more rows, hooks and other recipes do not."""
     from optimus_dl_amd.modules import fused

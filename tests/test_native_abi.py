@@ -80,6 +80,47 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
         native.load()
 
 
+@pytest.mark.parametrize("why", ["missing", "not a module", "other header", "other torch"])
+def test_library_is_usable_without_the_cpp_side_of_its_wrappers(monkeypatch, tmp_path, caplog, why):
+    """The extension belongs to one torch and one header.  Without a fitting one the library still loads, says so once, and
+    every wrapper goes the long way; nothing of a module that does not fit is bound or called."""
+    from optimus_dl_amd import native
+
+    if not native.is_built():
+        pytest.skip("library not built")
+    native.load()
+    monkeypatch.setattr(native, "_lib", None)
+    monkeypatch.setattr(native, "_host", None)
+    monkeypatch.setattr(native, "_HERE", str(tmp_path))
+    if why == "not a module":
+        (tmp_path / "_host.so").write_bytes(b"not an ELF file")
+    elif why != "missing":
+        bound = []
+
+        class Module:
+            abi_version = native.ABI_VERSION - (why == "other header")
+            torch_version = "1.0.0" if why == "other torch" else __import__("torch").__version__.split("+")[0]
+            bind = bound.append
+
+        spec = type("Spec", (), {"loader": type("L", (), {"exec_module": lambda self, m: None})()})()
+        monkeypatch.setattr(native.importlib.util, "spec_from_file_location", lambda *a: spec)
+        monkeypatch.setattr(native.importlib.util, "module_from_spec", lambda s: Module)
+    with caplog.at_level("WARNING"):
+        assert native.load() is native.load() and native.is_built()
+    assert [r for r in caplog.records if "rebuild" in r.message] and len(caplog.records) == 1
+    assert native._host.amax_parts("anything", 0) is None and native._host.gemm_swiglu() is None
+    assert why in ("missing", "not a module") or not bound
+
+
+def test_cpp_side_of_the_wrappers_is_the_one_in_use():
+    from optimus_dl_amd import native
+
+    if not native.is_built():
+        pytest.skip("library not built")
+    native.load()
+    assert native._host.abi_version == native.ABI_VERSION and callable(native._host.gemm_nt)
+
+
 def test_cpu_tensors_are_refused_not_emulated():
     import torch
 
