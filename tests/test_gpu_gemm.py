@@ -957,3 +957,18 @@ def test_few_tile_kernels_where_the_columns_end_between_slabs(N, variant, M, Nn)
             assert torch.equal(guarded[:M].cpu(), (product * 0.25 + old).float().to(dtype)) and (guarded[M:] == 7.0).all()
     finally:
         N.gemm_set_variant(-1)
+
+
+@pytest.mark.parametrize("M,Nn,K,runs", [(3072, 768, 16384, 6), (1024, 1024, 8192, 8), (2048, 2048, 16384, 4), (8192, 768, 50304, 2)])
+def test_one_launch_in_place_of_a_split_is_as_precise(N, M, Nn, K, runs):
+    """fp32 results of the automatic choice against 64 bits: no further off than K cut into runs side by side, whose chains of
+    additions are shorter.  The error is that of the MFMA's own sum of 64 products (1e-5); were it that of the chain, 256 additions
+    in a row would be off by 1.7 times as much as 6 x 43.  Measured: 4e-7 (K = 16384) to 6e-6 (K = 50304) of the error apart."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    a = torch.randn((M, K), device="cuda", generator=g).to(torch.float8_e5m2)
+    b = torch.randn((Nn, K), device="cuda", generator=g).to(torch.float8_e4m3fn)
+    exact = a.double() @ b.double().t()
+    one = torch.ones(1, device="cuda")
+    args = (a.view(torch.uint8), b.view(torch.uint8), O.E5M2, O.E4M3, one, one)
+    rms = lambda out: (out.double() - exact).pow(2).mean().sqrt().item()
+    assert rms(N.gemm_nt(*args, out_dtype=torch.float32)) <= (1 + 3e-5) * rms(N.gemm_splitk(*args, runs, out_dtype=torch.float32))
