@@ -464,11 +464,12 @@ class _Fp8LinearGroupFn(torch.autograd.Function):
         into one buffer, the scales become a per-row vector, and dW comes out as one [sum N, K] matrix whose row ranges
         are the members' gradients: twice the tiles per launch fill the chip where each alone leaves every compute unit
         with one block (measured, 8192 tokens: 2 x [1024 x 4096] 83.0 us, one [2048 x 4096] 65.2 us).
+        Current scaling only: under delayed scaling every member casts x with a scale of its own, so no two contract the same codes.
         -> (indices, codes_t buffer, X^T codes, its inverse scale) or None."""
         recipe = ctx.subs[0].recipe
         if not getattr(recipe, "fuse_sibling_wgrad", True) or recipe.fuse_wgrad_accumulation or not recipe.wgrad:
             return None
-        if recipe.recipe.kind not in ("tensorwise", "delayed"):
+        if recipe.recipe.kind != "tensorwise":
             return None
         picked, xq_t, sx_inv_t, w_dtype = [], None, None, None
         for i, (sub, (first, count), dy) in enumerate(zip(ctx.subs, ctx.spans, dys)):

@@ -70,7 +70,11 @@ class _SwiGLUMLPFn(torch.autograd.Function):
 
     The product and its gradients go from the registers of the kernel that computes them straight into codes: h, d_gate and
     d_up are never written in bf16.  Between separate nodes they have to be, since autograd hands tensors over.  Everything
-    else is what the three Linears do by themselves (their own forwards and backwards run, on their own saved tensors)."""
+    else is what the three Linears do by themselves (their own forwards and backwards run, on their own saved tensors); gate and
+    up never share a weight-gradient GEMM here, nor do they as a sibling group under these recipes (``_joint_wgrad``).
+
+    What one node costs: its saved tensors live until all of it is done, the three weight gradients arrive together, and a
+    backward that asks for some of the gradients only (``torch.autograd.grad`` for ``c_proj.weight``, say) computes all of them."""
 
     @staticmethod
     def forward(ctx, x2d: torch.Tensor, recipe: FP8Recipe, modules: tuple, *weights: torch.Tensor):

@@ -578,3 +578,28 @@ def test_decode_step_of_a_swiglu_mlp(amp):
         assert fused.swiglu_few_rows(mlp, x) is None          # a graph is recorded
     with amp.create_fp8_recipe("rowwise", "hybrid").autocast(), torch.no_grad():
         assert fused.swiglu_few_rows(mlp, x) is None
+
+
+@pytest.mark.parametrize("whole", [True, False])
+def test_delayed_scaling_gives_gate_and_up_weight_gradients_of_their_own(amp, monkeypatch, whole):
+    """Every member of a group casts x with its own scale there, so the MLP as one node and the sibling group both multiply twice:
+    neither drops a joint product that the other has."""
+    from optimus_dl_amd import native
+    from optimus_dl_amd.modules import fused
+    from optimus_dl_amd.modules.model.blocks import SwiGLUMLP
+    from optimus_dl_amd.modules.model_transforms import build_model_transform
+
+    if not whole:
+        monkeypatch.setattr(fused, "swiglu_mlp", lambda m, x: None)
+    tokens, width, hidden = 560, 1024, 3072
+    mlp = build_model_transform({"_name": "fp8_linear"}).apply(SwiGLUMLP(width, hidden).cuda())
+    recipe = amp.create_fp8_recipe("delayed", "hybrid", amax_history_len=4)
+    x = seeded_bf16((tokens, width), 1.0, 3).cuda().requires_grad_(True)
+    with recipe.autocast(), torch.autocast("cuda", dtype=torch.bfloat16):
+        y = mlp(x)
+    outputs = []
+    real = native.gemm_nt
+    monkeypatch.setattr(native, "gemm_nt", lambda a, b, *args, **kw: (outputs.append((a.shape[0], b.shape[0])), real(a, b, *args, **kw))[1])
+    with recipe.backward():
+        y.backward(seeded_bf16((tokens, width), 1e-3, 9).cuda())
+    assert outputs.count((hidden, width)) == 2 and (2 * hidden, width) not in outputs
