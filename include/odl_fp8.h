@@ -46,7 +46,7 @@ enum odl_status {
 };
 
 /* ABI version of this header; bumped when a signature changes or an entry point is added. */
-#define ODL_FP8_ABI_VERSION 23
+#define ODL_FP8_ABI_VERSION 24
 int odl_fp8_abi_version(void);
 
 /*
@@ -381,6 +381,16 @@ int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, in
                     const float *sa_inv, int64_t sa_n, const float *sb_inv, int64_t sb_n,
                     const void *bias, int bias_dtype,
                     void *c, int out_dtype, int accumulate, odl_stream_t stream);
+/*
+ * The same product, with a word on where its operands lie.  fresh != 0: both have just been written (a forward product), so
+ * compute units that the output leaves idle need not read them ahead of the others, which they do for operands of
+ * unknown age (fresh = 0: odl_fp8_gemm_nt).  The same kernels, the same bits.
+ */
+int odl_fp8_gemm_nt_hinted(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K,
+                           int fmt_a, int fmt_b,
+                           const float *sa_inv, int64_t sa_n, const float *sb_inv, int64_t sb_n,
+                           const void *bias, int bias_dtype,
+                           void *c, int out_dtype, int accumulate, int fresh, odl_stream_t stream);
 
 /*
  * A sum of such products in one call:
@@ -591,6 +601,10 @@ int odl_fp8_swiglu_bwd_cast_delayed(const void *dh, const void *gate, const void
 int odl_fp8_mx_gemm_nt(const uint8_t *a, const uint8_t *sa, const uint8_t *b, const uint8_t *sb, int scales_layout, int64_t M,
                        int64_t N, int64_t K, int fmt_a, int fmt_b, const float *bias, void *c, int out_dtype, int accumulate,
                        odl_stream_t stream);
+/* fresh: as for odl_fp8_gemm_nt_hinted */
+int odl_fp8_mx_gemm_nt_hinted(const uint8_t *a, const uint8_t *sa, const uint8_t *b, const uint8_t *sb, int scales_layout, int64_t M,
+                              int64_t N, int64_t K, int fmt_a, int fmt_b, const float *bias, void *c, int out_dtype, int accumulate,
+                              int fresh, odl_stream_t stream);
 
 /*
  * odl_fp8_mx_gemm_nt with K cut into `splits` runs that are computed side by side, for outputs of few tiles and a long

@@ -33,6 +33,7 @@ struct GemmArgs {
     // streaming kernel and gemm_deep.hip only: block scales of A and B (E8M0 bytes, one per 32 K-bytes), stored K-step-major:
     // dword [K / 128][rows] = the 4 scale bytes of a row in one 128-byte K step.  Set: the MFMAs apply them.
     const uint8_t *mx_sa = nullptr, *mx_sb = nullptr;
+    int fresh = 0;               // the operands have just been written: see warming_pays
 };
 
 // A contraction that runs over several operand pairs (streaming kernel only):
@@ -311,8 +312,11 @@ __device__ __forceinline__ void warm_operands(const GemmArgs &g, int helper, int
     }
 }
 
-// Operands that outgrow the memory-side cache are left alone (8192 x 768 x 50304: 324 us without, 331 with).
-inline bool warming_pays(const GemmArgs &g) { return (g.M + g.N) * g.K <= (int64_t)256 << 20; }
+// Operands that outgrow the memory-side cache are left alone (8192 x 768 x 50304: 324 us without, 331 with), and so are those of a
+// forward product, which its casts have just written: us of the product behind both casts, without and with warming, 4096 x
+// 768 x 3072 14.3 / 15.0, 4096 x 768 x 4096 16.9 / 17.7, 2048 x 1024 x 4096 16.1 / 17.2, 16384 x 768 x 3072 36.4 / 37.4, 2048 x 5632 x 2048
+// 27.2 / 27.8; the same where the weight's codes are kept from an earlier call.
+inline bool warming_pays(const GemmArgs &g) { return !g.fresh && (g.M + g.N) * g.K <= (int64_t)256 << 20; }
 
 // launchers implemented in gemm_tiled.hip / gemm_thin.hip / gemm_deep.hip / gemm_pipe.hip / gemm_stream.hip (fa, fb: odl_fp8_format of A and B)
 void launch_gemm_tiled(int variant, int fa, int fb, const GemmArgs &g, hipStream_t stream);

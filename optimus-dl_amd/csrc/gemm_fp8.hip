@@ -292,16 +292,17 @@ static Route route_of(int64_t M, int64_t N, int64_t K, int out_dtype, int accumu
 // The launch of checked arguments.
 static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b, const float *sa_inv, int64_t sa_n,
                            const float *sb_inv, int64_t sb_n, const void *bias, void *c, int out_dtype, int accumulate, int launch_as,
-                           hipStream_t stream) {
+                           bool fresh, hipStream_t stream) {
     const Route route = route_of(M, N, K, out_dtype, accumulate, launch_as);
     const int variant = route.variant;
     if (route.tail > 0) {
         const int64_t head = M - route.tail, esz = out_dtype == ODL_BF16 ? 2 : 4;
         const int rc = gemm_nt_checked(a, b, head, N, K, fmt_a, fmt_b, sa_inv, sa_n == 1 ? 1 : head, sb_inv, sb_n, bias, c, out_dtype, accumulate,
-                                       kStreamVariant, stream);
+                                       kStreamVariant, fresh, stream);
         if (rc != ODL_OK) return rc;
         return gemm_nt_checked(a + head * K, b, route.tail, N, K, fmt_a, fmt_b, sa_n == 1 ? sa_inv : sa_inv + head, sa_n == 1 ? 1 : route.tail, sb_inv,
-                               sb_n, bias, reinterpret_cast<uint8_t *>(c) + head * N * esz, out_dtype, accumulate, route.tail_variant, stream);
+                               sb_n, bias, reinterpret_cast<uint8_t *>(c) + head * N * esz, out_dtype, accumulate, route.tail_variant,
+                               fresh, stream);
     }
 
     GemmArgs g;
@@ -311,6 +312,7 @@ static int gemm_nt_checked(const uint8_t *a, const uint8_t *b, int64_t M, int64_
     g.sb_vec = sb_n == N && N != 1;
     g.out_dtype = out_dtype;
     g.accumulate = accumulate != 0;
+    g.fresh = fresh;
     const int bm = variant == 0 ? 32 : kVariants[variant].bm, bn = variant == 0 ? 32 : kVariants[variant].bn;
     const int64_t tm = (M + bm - 1) / bm, tn = (N + bn - 1) / bn;
     if (tm * tn > 0x7ffffff0LL) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt: too many tiles");
@@ -337,9 +339,9 @@ extern "C" int odl_fp8_gemm_route(int64_t M, int64_t N, int64_t K, int out_dtype
     return route.variant;
 }
 
-extern "C" int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b,
-                               const float *sa_inv, int64_t sa_n, const float *sb_inv, int64_t sb_n, const void *bias,
-                               int bias_dtype, void *c, int out_dtype, int accumulate, odl_stream_t stream_) {
+extern "C" int odl_fp8_gemm_nt_hinted(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b,
+                                      const float *sa_inv, int64_t sa_n, const float *sb_inv, int64_t sb_n, const void *bias,
+                                      int bias_dtype, void *c, int out_dtype, int accumulate, int fresh, odl_stream_t stream_) {
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
     if (!a || !b || !c || !sa_inv || !sb_inv) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: null pointer");
     if (M < 0 || N < 0 || K < 0) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt: negative size");
@@ -357,7 +359,13 @@ extern "C" int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, in
         (bias && (reinterpret_cast<uintptr_t>(bias) & 15)))
         return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt: scale vectors and bias must be 16-byte aligned");
     if (M == 0 || N == 0) return ODL_OK;
-    return gemm_nt_checked(a, b, M, N, K, fmt_a, fmt_b, sa_inv, sa_n, sb_inv, sb_n, bias, c, out_dtype, accumulate, -1, stream);
+    return gemm_nt_checked(a, b, M, N, K, fmt_a, fmt_b, sa_inv, sa_n, sb_inv, sb_n, bias, c, out_dtype, accumulate, -1, fresh != 0, stream);
+}
+
+extern "C" int odl_fp8_gemm_nt(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b,
+                               const float *sa_inv, int64_t sa_n, const float *sb_inv, int64_t sb_n, const void *bias,
+                               int bias_dtype, void *c, int out_dtype, int accumulate, odl_stream_t stream_) {
+    return odl_fp8_gemm_nt_hinted(a, b, M, N, K, fmt_a, fmt_b, sa_inv, sa_n, sb_inv, sb_n, bias, bias_dtype, c, out_dtype, accumulate, 0, stream_);
 }
 
 extern "C" int odl_fp8_gemm_nt_sum(int pairs, const uint8_t *const *a, const uint8_t *const *b, const int64_t *K, int64_t M, int64_t N,
@@ -536,7 +544,7 @@ extern "C" int odl_fp8_gemm_splitk(const uint8_t *a, const uint8_t *b, int64_t M
     auto mis = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; };
     if (splits == 2 && !ta && !tb && gemm_few_tiles(M, N, K, cu_count()) == kDeep192 && !(sa_n > 1 && mis(sa_inv)) && !(sb_n > 1 && mis(sb_inv)) &&
         !mis(bias))
-        return gemm_nt_checked(a, b, M, N, K, fmt_a, fmt_b, sa_inv, sa_n, sb_inv, sb_n, bias, c, out_dtype, accumulate, kDeep192Variant, stream);
+        return gemm_nt_checked(a, b, M, N, K, fmt_a, fmt_b, sa_inv, sa_n, sb_inv, sb_n, bias, c, out_dtype, accumulate, kDeep192Variant, false, stream);
     GemmArgs g;
     g.a = a; g.b = b; g.c = workspace; g.sa = sa_inv; g.sb = sb_inv; g.bias = nullptr;
     g.M = M; g.N = N; g.K = K;

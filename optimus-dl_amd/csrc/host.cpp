@@ -37,12 +37,12 @@ decltype(&odl_fp8_layernorm_amax_parts) layernorm_c;
 decltype(&odl_fp8_layernorm_bwd) layernorm_bwd_c;
 decltype(&odl_fp8_amax_rowcol) amax_rowcol_c;
 decltype(&odl_fp8_cast_rowcol_padded) cast_rowcol_c;
-decltype(&odl_fp8_gemm_nt) gemm_nt_c;
+decltype(&odl_fp8_gemm_nt_hinted) gemm_nt_c;
 decltype(&odl_fp8_gemm_layouts) gemm_layouts_c;
 decltype(&odl_fp8_gemm_split_count) split_count_c;
 decltype(&odl_fp8_mx_cast_padded) mx_cast_c;
 decltype(&odl_fp8_block_cast) block_cast_c;
-decltype(&odl_fp8_mx_gemm_nt) mx_gemm_nt_c;
+decltype(&odl_fp8_mx_gemm_nt_hinted) mx_gemm_nt_c;
 
 template <class F>
 void take(F &f, const py::dict &d, const char *name) { f = reinterpret_cast<F>(py::cast<uintptr_t>(d[name])); }
@@ -64,12 +64,12 @@ void bind(const py::dict &d) {
     take(layernorm_bwd_c, d, "odl_fp8_layernorm_bwd");
     take(amax_rowcol_c, d, "odl_fp8_amax_rowcol");
     take(cast_rowcol_c, d, "odl_fp8_cast_rowcol_padded");
-    take(gemm_nt_c, d, "odl_fp8_gemm_nt");
+    take(gemm_nt_c, d, "odl_fp8_gemm_nt_hinted");
     take(gemm_layouts_c, d, "odl_fp8_gemm_layouts");
     take(split_count_c, d, "odl_fp8_gemm_split_count");
     take(mx_cast_c, d, "odl_fp8_mx_cast_padded");
     take(block_cast_c, d, "odl_fp8_block_cast");
-    take(mx_gemm_nt_c, d, "odl_fp8_mx_gemm_nt");
+    take(mx_gemm_nt_c, d, "odl_fp8_mx_gemm_nt_hinted");
 }
 
 // as ctypes does: other Python threads run while a launch waits for room in its queue
@@ -271,7 +271,7 @@ bool small(i64 M, i64 N, i64 K) { return (M + 256) * K < (i64)1 << 31 && (N + 25
 
 // odt: 0 = bf16, 1 = fp32 (where no `out` decides).  split: K may be cut into runs, which the long way does.
 py::object gemm_nt(const Tensor &a, const Tensor &b, int fa, int fb, const Tensor &sa, const Tensor &sb, const OptTensor &bias, int odt,
-                   const OptTensor &out, bool accumulate, bool split, i64 stream) {
+                   const OptTensor &out, bool accumulate, bool fresh, bool split, i64 stream) {
     if (!codes2d(a) || !codes2d(b) || a.size(1) != b.size(1)) return none();
     const i64 M = a.size(0), K = a.size(1), N = b.size(0), na = sa.numel(), nb = sb.numel();
     if ((na != 1 && na != M) || (nb != 1 && nb != N) || !floats(sa, na) || !floats(sb, nb) || (bias && !floats(*bias, N)) || !out_fits(out, M, N) ||
@@ -279,7 +279,7 @@ py::object gemm_nt(const Tensor &a, const Tensor &b, int fa, int fb, const Tenso
         return none();
     if (split && small(M, N, K) && split_count_c(M, N, K, 0) > 1) return none();
     Tensor c = result(out, a, M, N, odt);
-    const int rc = call(gemm_nt_c, ptr(a), ptr(b), M, N, K, fa, fb, ptr(sa), na, ptr(sb), nb, ptr(bias), 1, ptr(c), src_of(c), accumulate, str(stream));
+    const int rc = call(gemm_nt_c, ptr(a), ptr(b), M, N, K, fa, fb, ptr(sa), na, ptr(sb), nb, ptr(bias), 1, ptr(c), src_of(c), accumulate, fresh, str(stream));
     return rc ? status(rc) : py::cast(c);
 }
 
@@ -323,7 +323,7 @@ py::object block_cast(const Tensor &x, int fmt, int margin, bool two_d, bool wan
 }
 
 py::object mx_gemm_nt(const Tensor &a, const Tensor &sa, const Tensor &b, const Tensor &sb, int fa, int fb, const OptTensor &bias, int odt,
-                      const OptTensor &out, bool accumulate, bool split, i64 stream) {
+                      const OptTensor &out, bool accumulate, bool fresh, bool split, i64 stream) {
     if (!codes2d(a) || !codes2d(b) || a.size(1) != b.size(1) || !dense(sa) || !dense(sb) || sa.scalar_type() != at::kByte || sb.scalar_type() != at::kByte)
         return none();
     const i64 M = a.size(0), K = a.size(1), N = b.size(0);
@@ -334,7 +334,7 @@ py::object mx_gemm_nt(const Tensor &a, const Tensor &sa, const Tensor &b, const 
     if ((bias && !floats(*bias, N)) || !out_fits(out, M, N) || (accumulate && !out)) return none();
     if (split && small(M, N, K) && split_count_c(M, N, K, 0) > 1) return none();
     Tensor c = result(out, a, M, N, odt);
-    const int rc = call(mx_gemm_nt_c, ptr(a), ptr(sa), ptr(b), ptr(sb), 1, M, N, K, fa, fb, ptr(bias), ptr(c), src_of(c), accumulate, str(stream));
+    const int rc = call(mx_gemm_nt_c, ptr(a), ptr(sa), ptr(b), ptr(sb), 1, M, N, K, fa, fb, ptr(bias), ptr(c), src_of(c), accumulate, fresh, str(stream));
     return rc ? status(rc) : py::cast(c);
 }
 

@@ -1178,6 +1178,12 @@ extern "C" int odl_fp8_swiglu_bwd_block_cast(const void *dh, const void *gate, c
 
 extern "C" int odl_fp8_mx_gemm_nt(const uint8_t *a, const uint8_t *sa, const uint8_t *b, const uint8_t *sb, int scales_layout, int64_t M,
                                   int64_t N, int64_t K, int fmt_a, int fmt_b, const float *bias, void *c, int out_dtype, int accumulate, odl_stream_t stream_) {
+    return odl_fp8_mx_gemm_nt_hinted(a, sa, b, sb, scales_layout, M, N, K, fmt_a, fmt_b, bias, c, out_dtype, accumulate, 0, stream_);
+}
+
+extern "C" int odl_fp8_mx_gemm_nt_hinted(const uint8_t *a, const uint8_t *sa, const uint8_t *b, const uint8_t *sb, int scales_layout, int64_t M,
+                                         int64_t N, int64_t K, int fmt_a, int fmt_b, const float *bias, void *c, int out_dtype, int accumulate,
+                                         int fresh, odl_stream_t stream_) {
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
     if (M < 0 || N < 0 || K < 0) return set_error(ODL_ERR_ARG, "odl_fp8_mx_gemm_nt: negative shape");
     if ((fmt_a != ODL_FP8_E4M3 && fmt_a != ODL_FP8_E5M2) || (fmt_b != ODL_FP8_E4M3 && fmt_b != ODL_FP8_E5M2))
@@ -1199,6 +1205,7 @@ extern "C" int odl_fp8_mx_gemm_nt(const uint8_t *a, const uint8_t *sa, const uin
     g.a = a; g.b = b; g.c = c; g.sa = one; g.sb = one; g.bias = bias;
     g.M = M; g.N = N; g.K = K; g.sa_vec = 0; g.sb_vec = 0; g.out_dtype = out_dtype;
     g.accumulate = accumulate != 0;
+    g.fresh = fresh != 0;
     // the tiled and the streaming kernel address rows with 32-bit offsets and read whole scale dwords (4 blocks = one
     // 128-byte K step); the streaming kernel wants the scales K-step-major and the shapes of gemm_stream_accepts, and
     // pays only when more than half the compute units get one of its 256 x 256 tiles (at exactly half, outputs of

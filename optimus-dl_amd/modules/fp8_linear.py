@@ -247,7 +247,7 @@ class _Fp8LinearFn(torch.autograd.Function):
             fp8_wgrad = need_wgrad and recipe.wgrad
             xq, xs, xq_t, xs_t = given or _mx_input_shared(recipe, x2d, pol.fmt_fwd, fp8_wgrad)
             wq, ws, wq_t, ws_t = module._mx_weight(weight, recipe, need_t=both_w)
-            y = native.mx_gemm_nt(xq, xs, wq, ws, pol.fmt_fwd, pol.fmt_fwd, bias=bias_f32, out_dtype=out_dtype)
+            y = native.mx_gemm_nt(xq, xs, wq, ws, pol.fmt_fwd, pol.fmt_fwd, bias=bias_f32, out_dtype=out_dtype, fresh=True)
             if fp8_wgrad:
                 saved["xq_t"], saved["xs_t"] = xq_t, xs_t
             if need_dgrad:
@@ -262,7 +262,7 @@ class _Fp8LinearFn(torch.autograd.Function):
             if not recipe.cache_weights:
                 module._wcache_rowwise.clear()          # the backward of this call still finds what is made now
             wq, sw_inv = module._rowwise_weight(weight, pol, "row", both=both_w)
-            y = native.gemm_nt(_rows(xq, x2d.shape[0]), wq, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sw_inv, bias=bias_f32, out_dtype=out_dtype)
+            y = native.gemm_nt(_rows(xq, x2d.shape[0]), wq, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sw_inv, bias=bias_f32, out_dtype=out_dtype, fresh=True)
         else:
             # With whole 256 x 256 tiles wgrad reads the ROW-MAJOR codes of dy with the tokens as the slow
             # axis (native.gemm_layouts): dy, the largest tensor of the backward, gets no transposed copy.
@@ -288,7 +288,7 @@ class _Fp8LinearFn(torch.autograd.Function):
             else:
                 xq, xq_t, sx_inv = _quantise_input_shared(recipe, x2d, pol.fmt_fwd, pol.margin, fp8_wgrad)
             wq, wq_t, sw_inv = module._tensor_weight(weight, recipe, need_t=both_w)
-            y = native.gemm_nt(_rows(xq, x2d.shape[0]), wq, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sw_inv, bias=bias_f32, out_dtype=out_dtype)
+            y = native.gemm_nt(_rows(xq, x2d.shape[0]), wq, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sw_inv, bias=bias_f32, out_dtype=out_dtype, fresh=True)
             if fp8_wgrad:
                 saved["xq_t"], saved["sx_inv_t"] = xq_t, sx_inv
             if need_dgrad:

@@ -26,7 +26,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 23
+ABI_VERSION = 24
 _OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
@@ -70,6 +70,7 @@ EXPORTS = (
     "odl_fp8_cast_transpose",
     "odl_fp8_cast_delayed",
     "odl_fp8_gemm_nt",
+    "odl_fp8_gemm_nt_hinted",
     "odl_fp8_gemm_nt_sum",
     "odl_fp8_gemm_layouts",
     "odl_fp8_gemm_split_count",
@@ -89,6 +90,7 @@ EXPORTS = (
     "odl_fp8_swiglu_cast_delayed",
     "odl_fp8_swiglu_bwd_cast_delayed",
     "odl_fp8_mx_gemm_nt",
+    "odl_fp8_mx_gemm_nt_hinted",
     "odl_fp8_block_cast",
     "odl_fp8_mx_gemm_splitk",
 )
@@ -160,6 +162,7 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_cast_transpose.argtypes = [vp, i32, i64, i64, vp, i32, i32, vp, vp, vp, vp]
         L.odl_fp8_cast_delayed.argtypes = [vp, i32, i64, i64, vp, i32, vp, vp, vp, vp, vp]
         L.odl_fp8_gemm_nt.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, i64, vp, i64, vp, i32, vp, i32, i32, vp]
+        L.odl_fp8_gemm_nt_hinted.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, i64, vp, i64, vp, i32, vp, i32, i32, i32, vp]
         L.odl_fp8_gemm_nt_sum.argtypes = [i32, vp, vp, vp, i64, i64, i32, i32, vp, vp, vp, i32, vp]
         L.odl_fp8_gemm_layouts.argtypes = [vp, vp, i64, i64, i64, i32, i32, i32, i32, vp, vp, vp, i32, vp]
         L.odl_fp8_gemm_split_count.argtypes = [i64, i64, i64, i32]
@@ -181,6 +184,7 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_mx_cast_padded.argtypes = [vp, i32, i64, i64, i64, i32, vp, vp, i32, vp, vp, i32, i32, vp]
         L.odl_fp8_mx_cast.argtypes = [vp, i32, i64, i64, i32, vp, vp, i32, vp, vp, i32, i32, vp]
         L.odl_fp8_mx_gemm_nt.argtypes = [vp, vp, vp, vp, i32, i64, i64, i64, i32, i32, vp, vp, i32, i32, vp]
+        L.odl_fp8_mx_gemm_nt_hinted.argtypes = [vp, vp, vp, vp, i32, i64, i64, i64, i32, i32, vp, vp, i32, i32, i32, vp]
         L.odl_fp8_block_cast.argtypes = [vp, i32, i64, i64, i32, i32, i32, vp, vp, vp, vp, vp]
         L.odl_fp8_mx_gemm_splitk.argtypes = [vp, vp, vp, vp, i64, i64, i64, i32, i32, vp, vp, i32, i32, i32, vp, i64, vp]
         for name in EXPORTS:
@@ -912,13 +916,14 @@ def cast_delayed(x: torch.Tensor, scale: torch.Tensor, fmt: int, amax_parts: tor
 
 def gemm_nt(a: torch.Tensor, b: torch.Tensor, fmt_a: int, fmt_b: int, sa_inv: torch.Tensor, sb_inv: torch.Tensor,
             bias: torch.Tensor | None = None, out_dtype: torch.dtype = torch.bfloat16,
-            out: torch.Tensor | None = None, accumulate: bool = False) -> torch.Tensor:
+            out: torch.Tensor | None = None, accumulate: bool = False, fresh: bool = False) -> torch.Tensor:
     """out[M,N] = (a[M,K] . b[N,K]^T) * (sa_inv x sb_inv) (+ bias); a, b uint8 FP8 codes.  A given ``out`` decides the
-    output type.  accumulate: out = out + product (needs ``out``; the old value joins the fp32 sum, one rounding)."""
+    output type.  accumulate: out = out + product (needs ``out``; the old value joins the fp32 sum, one rounding).  fresh: a
+    and b have just been written (a forward product): nobody reads them ahead.  The same bits."""
     odt = _OUT_DTYPES.get(out_dtype, -1)
     if odt >= 0 and a.is_cuda:
         load()
-        r = _host.gemm_nt(a, b, fmt_a, fmt_b, sa_inv, sb_inv, bias, odt, out, accumulate, _may_split(), _stream())
+        r = _host.gemm_nt(a, b, fmt_a, fmt_b, sa_inv, sb_inv, bias, odt, out, accumulate, fresh, _may_split(), _stream())
         if r is not None:
             return _done(r, "odl_fp8_gemm_nt")
     if accumulate and out is None:
@@ -948,9 +953,9 @@ def gemm_nt(a: torch.Tensor, b: torch.Tensor, fmt_a: int, fmt_b: int, sa_inv: to
     splits = gemm_split_count(M, N, K)
     if splits > 1:
         return _gemm_splitk(a, b, M, N, K, fmt_a, fmt_b, K_FAST, K_FAST, sa_inv, sb_inv, bias, out, splits, accumulate)
-    _check(load().odl_fp8_gemm_nt(a.data_ptr(), b.data_ptr(), M, N, K, fmt_a, fmt_b, sa_inv.data_ptr(), sa_inv.numel(),
-                                  sb_inv.data_ptr(), sb_inv.numel(), bias.data_ptr() if bias is not None else None,
-                                  DT_F32, out.data_ptr(), odt, int(accumulate), _stream()), "odl_fp8_gemm_nt")
+    _check(load().odl_fp8_gemm_nt_hinted(a.data_ptr(), b.data_ptr(), M, N, K, fmt_a, fmt_b, sa_inv.data_ptr(), sa_inv.numel(),
+                                         sb_inv.data_ptr(), sb_inv.numel(), bias.data_ptr() if bias is not None else None,
+                                         DT_F32, out.data_ptr(), odt, int(accumulate), int(fresh), _stream()), "odl_fp8_gemm_nt")
     return out
 
 
@@ -1213,15 +1218,15 @@ def block_cast(x: torch.Tensor, fmt: int, margin: int = 0, two_d: bool = False, 
 
 def mx_gemm_nt(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Tensor, fmt_a: int, fmt_b: int,
                bias: torch.Tensor | None = None, out_dtype: torch.dtype = torch.bfloat16, out: torch.Tensor | None = None,
-               accumulate: bool = False) -> torch.Tensor:
+               accumulate: bool = False, fresh: bool = False) -> torch.Tensor:
     """out[M,N] = sum over 32-blocks of 2^(sa-127) 2^(sb-127) (a_block . b_block) (+ bias); a [M,K], b [N,K] codes,
     sa, sb their E8M0 scale bytes as ``mx_cast`` returns them (both row-major [rows, K/32] or both K-step-major
-    [K/128, rows, 4])."""
+    [K/128, rows, 4]).  accumulate, fresh: as for :func:`gemm_nt`."""
     odt = _OUT_DTYPES.get(out_dtype, -1)
     if odt >= 0 and a.is_cuda:
         load()
         init_device(a.device)
-        r = _host.mx_gemm_nt(a, sa, b, sb, fmt_a, fmt_b, bias, odt, out, accumulate, _may_split(), _stream())
+        r = _host.mx_gemm_nt(a, sa, b, sb, fmt_a, fmt_b, bias, odt, out, accumulate, fresh, _may_split(), _stream())
         if r is not None:
             return _done(r, "odl_fp8_mx_gemm_nt")
     for t, what in ((a, "a"), (b, "b"), (sa, "sa"), (sb, "sb")):
@@ -1262,8 +1267,8 @@ def mx_gemm_nt(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Ten
                                              splits, workspace.data_ptr(), workspace.numel() * 4, _stream()), "odl_fp8_mx_gemm_splitk")
         return out
     init_device(a.device)
-    _check(load().odl_fp8_mx_gemm_nt(a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), layout, M, N, K, fmt_a, fmt_b,
-                                     bias.data_ptr() if bias is not None else None, out.data_ptr(), odt, int(accumulate), _stream()),
+    _check(load().odl_fp8_mx_gemm_nt_hinted(a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), layout, M, N, K, fmt_a, fmt_b,
+                                            bias.data_ptr() if bias is not None else None, out.data_ptr(), odt, int(accumulate), int(fresh), _stream()),
            "odl_fp8_mx_gemm_nt")
     return out
 

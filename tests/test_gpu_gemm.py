@@ -972,3 +972,14 @@ def test_one_launch_in_place_of_a_split_is_as_precise(N, M, Nn, K, runs):
     args = (a.view(torch.uint8), b.view(torch.uint8), O.E5M2, O.E4M3, one, one)
     rms = lambda out: (out.double() - exact).pow(2).mean().sqrt().item()
     assert rms(N.gemm_nt(*args, out_dtype=torch.float32)) <= (1 + 3e-5) * rms(N.gemm_splitk(*args, runs, out_dtype=torch.float32))
+
+
+@pytest.mark.parametrize("M,Nn,K", [(4096, 768, 3072), (1004, 384, 2176), (2048, 5632, 2048), (4016, 896, 4096), (48, 256, 2048)])
+def test_fresh_operands_give_the_same_bits(N, M, Nn, K):
+    """Whether idle units read the operands ahead changes nothing in the result: 128 x 128 tiles, ragged rows, streaming tiles."""
+    a, b = (torch.randint(0, 0x78, (r, K), dtype=torch.uint8, device="cuda") for r in (M, Nn))
+    one = torch.ones(1, device="cuda")
+    for dtype in (torch.bfloat16, torch.float32):
+        assert torch.equal(N.gemm_nt(a, b, O.E4M3, O.E5M2, one, one, out_dtype=dtype, fresh=True), N.gemm_nt(a, b, O.E4M3, O.E5M2, one, one, out_dtype=dtype))
+    sa, sb = (torch.full((K // 128, r, 4), 120, dtype=torch.uint8, device="cuda") for r in (M, Nn))
+    assert torch.equal(N.mx_gemm_nt(a, sa, b, sb, O.E4M3, O.E5M2, fresh=True), N.mx_gemm_nt(a, sa, b, sb, O.E4M3, O.E5M2))

@@ -738,3 +738,17 @@ def test_rowwise_backward_without_a_data_gradient_casts_one_axis(tokens, monkeyp
         grads.append(lin.weight.grad)
         assert ((tokens, 384) in both_axes) == needs
     assert torch.equal(grads[0], grads[1])
+
+
+@pytest.mark.parametrize("kind", ["tensorwise", "delayed", "rowwise", "mxfp8"])
+def test_only_forward_products_say_that_their_operands_are_fresh(amp, monkeypatch, kind):
+    """Their codes have just been cast; a gradient product contracts at least one operand that the forward left behind."""
+    from optimus_dl_amd import native
+
+    said = []
+    for name in ("gemm_nt", "mx_gemm_nt"):
+        real = getattr(native, name)
+        monkeypatch.setattr(native, name, lambda *a, real=real, **kw: (said.append(kw.get("fresh", False)), real(*a, **kw))[1])
+    M, K, N = 256, 512, 384
+    run_step(make_linear(seeded_bf16((N, K), 0.02, 61)), amp.create_fp8_recipe(kind, "hybrid"), seeded_bf16((M, K), 1.0, 60), seeded_bf16((M, N), 1e-3, 62))
+    assert said[0] and len(said) > 1 and not any(said[1:])
