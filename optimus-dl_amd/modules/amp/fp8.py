@@ -210,9 +210,9 @@ class FP8Recipe:
         # optimizer step).  Code that rewrites weights through ``param.data`` does not move that counter:
         # set this to False there, and every forward quantises its weight again (what the reference does).
         self.cache_weights = True
-        # wgrad reads the row-major codes of dy with the tokens as the slow axis where the shapes allow
-        # (no transposed copy of dy); False keeps the cast+transpose route everywhere
-        self.direct_layouts = True
+        # wgrad reads the row-major codes of dy with the tokens as the slow axis (no transposed copy of dy): "auto" where the
+        # shapes allow and it is faster (native.wgrad_direct_pays), True wherever they allow, False nowhere
+        self.direct_layouts: "bool | str" = "auto"
         # partial maxima handed over by the kernel that produced a tensor (SwiGLU, RMSNorm), so that
         # the Linear that quantises this very tensor skips its amax pass; a handful of entries
         self.producer_parts: list[tuple[tuple, torch.Tensor, torch.Tensor]] = []

@@ -1346,9 +1346,10 @@ def wgrad_direct_pays(n_out: int, n_in: int, tokens: int) -> bool:
     1024 x 4096 61.7 / 52.2, 3072 x 768 55.3 / 52.9, 2048 x 1024 53.9 / 46.6; 1024 x 1024 at 512 tokens 17.1 / 11.7, 2048 29.7 / 17.7,
     4096 31.8 / 24.9, 6144 35.8 / 32.7.  From 8192 tokens on, outputs of less than 1.8 million elements are equal either way
     (2304 x 768 47.6 / 48.6, 1024 x 1024 37.9 / 38.8, 768 x 768 33.6 / 33.8), and the route without a second copy of dY is
-    taken; so it is for the smallest outputs (768 x 512), which give 5 to 10 us for that."""
+    taken.  The smallest outputs are thin tiles over the copy, and equal only at twice the tokens: 768 x 512 19.4 / 12.3 at 1024
+    tokens, 31.5 / 24.5 at 8192, 42.3 / 43.9 at 16384; 512 x 512 28.8 / 18.5 and 36.7 / 38.3; 512 x 256 28.4 / 16.1 and 36.6 / 25.0."""
     tiles, elements = (n_out // 256) * (n_in // 256), n_out * n_in
-    return tiles >= 192 or (elements < 1_800_000 and tokens >= 8192) or elements < 400_000
+    return tiles >= 192 or 262_144 <= elements < 1_800_000 and tokens >= (8192 if elements >= 400_000 else 16384)
 
 
 def dgrad_sum_in_one_launch(tokens: int, n_in: int, n_outs: "list[int]") -> bool:

@@ -307,3 +307,13 @@ def test_block_scaled_entry_points_refuse_bad_arguments_before_touching_a_device
     # blockwise cast: sizes must be multiples of 128, margin in range
     assert L.odl_fp8_block_cast(p, 0, 128, 192, 0, 0, 0, p, p, None, None, None) != 0 and "multiples of 128" in err()
     assert L.odl_fp8_block_cast(p, 0, 128, 128, 0, 1000, 0, p, p, None, None, None) != 0 and "margin" in err()
+
+
+def test_small_weight_gradients_read_dy_as_stored_only_where_that_is_no_slower():
+    """The line in output elements and tokens that the measurements beside the rule draw."""
+    from optimus_dl_amd.native import wgrad_direct_pays as pays
+
+    assert not pays(768, 512, 1024) and not pays(512, 768, 8192) and pays(768, 512, 16384) and pays(512, 512, 16384)
+    assert not pays(512, 256, 16384) and not pays(256, 256, 32768)
+    assert not pays(768, 768, 8064) and pays(768, 768, 8192) and pays(2304, 768, 8192) and not pays(2048, 1024, 16384)
+    assert pays(4096, 4096, 512) and pays(14336, 4096, 8192)
