@@ -46,7 +46,7 @@ enum odl_status {
 };
 
 /* ABI version of this header; bumped when a signature changes or an entry point is added. */
-#define ODL_FP8_ABI_VERSION 24
+#define ODL_FP8_ABI_VERSION 25
 int odl_fp8_abi_version(void);
 
 /*
@@ -443,14 +443,18 @@ int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t M, int64_t 
  * is therefore taken in a different order than by odl_fp8_gemm_nt: equal within fp32 rounding,
  * bit-identical where every partial sum is exact.  odl_fp8_gemm_split_count proposes `splits`
  * for a shape (1 = not worth splitting; k_slow != 0: an operand will be passed K-slow); any 2 <= splits <= 64 that leaves every run at least 512
- * long is accepted.  M, N, K multiples of 128 (256 for an operand stored K-slow), K-run >= 512.  `splits` is the most
- * that is used: where one launch of smaller tiles is faster than two runs, that is what runs (the workspace stays unread).
+ * long is accepted.  M, N, K multiples of 128 (256 for an operand stored K-slow), K-run >= 512.
  * accumulate != 0: the second kernel adds the old value of C to the sum before the one rounding
  * (C = C + product, as for odl_fp8_gemm_nt); splits == 1 is then accepted too, which is how a product
  * with an operand stored K-slow (a weight gradient that reads dY as stored) is added into C.
  * No counterpart in the reference, whose GEMMs are cuBLASLt's choice inside te.pytorch.Linear.
  */
 int odl_fp8_gemm_split_count(int64_t M, int64_t N, int64_t K, int k_slow);
+/*
+ * The runs worth a workspace: odl_fp8_gemm_split_count, but 1 where one launch of odl_fp8_gemm_nt (or odl_fp8_mx_gemm_nt) in 128 x 192
+ * tiles is faster than the two runs proposed.
+ */
+int odl_fp8_gemm_runs(int64_t M, int64_t N, int64_t K, int k_slow);
 int odl_fp8_gemm_splitk(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K,
                         int fmt_a, int fmt_b, int layout_a, int layout_b,
                         const float *sa_inv, int64_t sa_n, const float *sb_inv, int64_t sb_n,
@@ -609,7 +613,7 @@ int odl_fp8_mx_gemm_nt_hinted(const uint8_t *a, const uint8_t *sa, const uint8_t
 /*
  * odl_fp8_mx_gemm_nt with K cut into `splits` runs that are computed side by side, for outputs of few tiles and a long
  * contraction (weight gradients of small layers), exactly as odl_fp8_gemm_splitk does for per-tensor scales
- * (odl_fp8_gemm_split_count says when and how many): fp32 partial results in `workspace` (splits * M * N floats, 16-byte
+ * (odl_fp8_gemm_runs says when and how many): fp32 partial results in `workspace` (splits * M * N floats, 16-byte
  * aligned, caller-owned), added in run order, bias added, one rounding.  K-step-major scales only; M, N, K multiples of
  * 128; every run at least 512 long.
  */

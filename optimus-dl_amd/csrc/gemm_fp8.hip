@@ -452,7 +452,7 @@ extern "C" int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t 
 //   one launch, smaller tiles   : what odl_fp8_gemm_nt takes for outputs of <= cus / 2 big tiles (few_tiles_variant).
 //                                 128 x 128 with a unit each 0.37 us per step + 6 us (3072 x 768 x 16384: 45 - 50 us, in
 //                                 six runs 52 and the reduction's launch); 256 x 128 with a unit each 0.70 + 7 (128 x 192 in
-//                                 their place: 0.66 + 8; where two runs are proposed instead, odl_fp8_gemm_splitk looks
+//                                 their place: 0.66 + 8; where two runs are proposed instead, odl_fp8_gemm_runs looks
 //                                 again); two 128 x 128 blocks per unit 0.62 (it reads every operand panel twice as often)
 //   split                       : 0.96 us per step of a run + 9 us (pipeline fill, the fp32 epilogue, the second launch)
 //                                 + the partial results, splits x M x N floats written and read back, at 2.7 TB/s in all
@@ -508,6 +508,14 @@ extern "C" int odl_fp8_gemm_split_count(int64_t M, int64_t N, int64_t K, int k_s
     return best_splits;
 }
 
+// One launch of 128 x 192 tiles that gives (nearly) every compute unit one beats two runs of big tiles and the addition behind
+// them: 8192 x 768 x 50304 319 -> 283 us, 16384 x 384 x 50304 340 -> 308; with block scales 337 -> 308 and 359 -> 328.  Not three runs
+// (3072 x 1536 x 50304 229 against 231, with block scales 236 against 256).
+extern "C" int odl_fp8_gemm_runs(int64_t M, int64_t N, int64_t K, int k_slow) {
+    const int runs = odl_fp8_gemm_split_count(M, N, K, k_slow);
+    return runs == 2 && !k_slow && gemm_few_tiles(M, N, K, cu_count()) == kDeep192 ? 1 : runs;
+}
+
 extern "C" int odl_fp8_gemm_splitk(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b,
                                    int layout_a, int layout_b, const float *sa_inv, int64_t sa_n, const float *sb_inv,
                                    int64_t sb_n, const float *bias, void *c, int out_dtype, int accumulate, int splits, void *workspace,
@@ -539,12 +547,6 @@ extern "C" int odl_fp8_gemm_splitk(const uint8_t *a, const uint8_t *b, int64_t M
     if (workspace_bytes < (int64_t)splits * M * N * 4)
         return set_error(ODL_ERR_ARG, "odl_fp8_gemm_splitk: workspace of %lld bytes, %lld needed", (long long)workspace_bytes,
                          (long long)splits * M * N * 4);
-    // One launch of 128 x 192 tiles that gives (nearly) every compute unit one beats two runs of big tiles and the addition
-    // behind them: 8192 x 768 x 50304 319 -> 283 us, 16384 x 384 x 50304 340 -> 308.
-    auto mis = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; };
-    if (splits == 2 && !ta && !tb && gemm_few_tiles(M, N, K, cu_count()) == kDeep192 && !(sa_n > 1 && mis(sa_inv)) && !(sb_n > 1 && mis(sb_inv)) &&
-        !mis(bias))
-        return gemm_nt_checked(a, b, M, N, K, fmt_a, fmt_b, sa_inv, sa_n, sb_inv, sb_n, bias, c, out_dtype, accumulate, kDeep192Variant, false, stream);
     GemmArgs g;
     g.a = a; g.b = b; g.c = workspace; g.sa = sa_inv; g.sb = sb_inv; g.bias = nullptr;
     g.M = M; g.N = N; g.K = K;

@@ -39,7 +39,7 @@ decltype(&odl_fp8_amax_rowcol) amax_rowcol_c;
 decltype(&odl_fp8_cast_rowcol_padded) cast_rowcol_c;
 decltype(&odl_fp8_gemm_nt_hinted) gemm_nt_c;
 decltype(&odl_fp8_gemm_layouts) gemm_layouts_c;
-decltype(&odl_fp8_gemm_split_count) split_count_c;
+decltype(&odl_fp8_gemm_runs) runs_c;
 decltype(&odl_fp8_mx_cast_padded) mx_cast_c;
 decltype(&odl_fp8_block_cast) block_cast_c;
 decltype(&odl_fp8_mx_gemm_nt_hinted) mx_gemm_nt_c;
@@ -66,7 +66,7 @@ void bind(const py::dict &d) {
     take(cast_rowcol_c, d, "odl_fp8_cast_rowcol_padded");
     take(gemm_nt_c, d, "odl_fp8_gemm_nt_hinted");
     take(gemm_layouts_c, d, "odl_fp8_gemm_layouts");
-    take(split_count_c, d, "odl_fp8_gemm_split_count");
+    take(runs_c, d, "odl_fp8_gemm_runs");
     take(mx_cast_c, d, "odl_fp8_mx_cast_padded");
     take(block_cast_c, d, "odl_fp8_block_cast");
     take(mx_gemm_nt_c, d, "odl_fp8_mx_gemm_nt_hinted");
@@ -275,9 +275,9 @@ py::object gemm_nt(const Tensor &a, const Tensor &b, int fa, int fb, const Tenso
     if (!codes2d(a) || !codes2d(b) || a.size(1) != b.size(1)) return none();
     const i64 M = a.size(0), K = a.size(1), N = b.size(0), na = sa.numel(), nb = sb.numel();
     if ((na != 1 && na != M) || (nb != 1 && nb != N) || !floats(sa, na) || !floats(sb, nb) || (bias && !floats(*bias, N)) || !out_fits(out, M, N) ||
-        (accumulate && !out))
+        (accumulate && !out) || (na > 1 && !aligned(sa)) || (nb > 1 && !aligned(sb)) || (bias && !aligned(*bias)))
         return none();
-    if (split && small(M, N, K) && split_count_c(M, N, K, 0) > 1) return none();
+    if (split && small(M, N, K) && runs_c(M, N, K, 0) > 1) return none();
     Tensor c = result(out, a, M, N, odt);
     const int rc = call(gemm_nt_c, ptr(a), ptr(b), M, N, K, fa, fb, ptr(sa), na, ptr(sb), nb, ptr(bias), 1, ptr(c), src_of(c), accumulate, fresh, str(stream));
     return rc ? status(rc) : py::cast(c);
@@ -289,7 +289,7 @@ py::object gemm_layouts(const Tensor &a, const Tensor &b, int fa, int fb, bool a
     if (!codes2d(a) || !codes2d(b) || !floats(sa, 1) || !floats(sb, 1)) return none();
     const i64 M = a.size(a_slow ? 1 : 0), K = a.size(a_slow ? 0 : 1), N = b.size(b_slow ? 1 : 0);
     if (K != b.size(b_slow ? 0 : 1) || !out_fits(out, M, N) || M <= 0 || N <= 0 || M % 256 || N % 256 || K % 128 || K < 512 || !small(M, N, K)) return none();
-    if (N * (i64)4 * 264 >= (i64)1 << 31 || (split && split_count_c(M, N, K, a_slow || b_slow) > 1)) return none();
+    if (N * (i64)4 * 264 >= (i64)1 << 31 || (split && runs_c(M, N, K, a_slow || b_slow) > 1)) return none();
     Tensor c = result(out, a, M, N, odt);
     const int rc = call(gemm_layouts_c, ptr(a), ptr(b), M, N, K, fa, fb, a_slow, b_slow, ptr(sa), ptr(sb), ptr(c), src_of(c), str(stream));
     return rc ? status(rc) : py::cast(c);
@@ -332,7 +332,7 @@ py::object mx_gemm_nt(const Tensor &a, const Tensor &sa, const Tensor &b, const 
         sb.size(1) != N || sb.size(2) != 4)
         return none();
     if ((bias && !floats(*bias, N)) || !out_fits(out, M, N) || (accumulate && !out)) return none();
-    if (split && small(M, N, K) && split_count_c(M, N, K, 0) > 1) return none();
+    if (split && small(M, N, K) && runs_c(M, N, K, 0) > 1) return none();
     Tensor c = result(out, a, M, N, odt);
     const int rc = call(mx_gemm_nt_c, ptr(a), ptr(sa), ptr(b), ptr(sb), 1, M, N, K, fa, fb, ptr(bias), ptr(c), src_of(c), accumulate, fresh, str(stream));
     return rc ? status(rc) : py::cast(c);

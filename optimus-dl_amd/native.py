@@ -26,7 +26,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 24
+ABI_VERSION = 25
 _OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
@@ -74,6 +74,7 @@ EXPORTS = (
     "odl_fp8_gemm_nt_sum",
     "odl_fp8_gemm_layouts",
     "odl_fp8_gemm_split_count",
+    "odl_fp8_gemm_runs",
     "odl_fp8_gemm_splitk",
     "odl_fp8_delayed_update",
     "odl_fp8_gemm_num_variants",
@@ -167,6 +168,8 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_gemm_layouts.argtypes = [vp, vp, i64, i64, i64, i32, i32, i32, i32, vp, vp, vp, i32, vp]
         L.odl_fp8_gemm_split_count.argtypes = [i64, i64, i64, i32]
         L.odl_fp8_gemm_split_count.restype = i32
+        L.odl_fp8_gemm_runs.argtypes = [i64, i64, i64, i32]
+        L.odl_fp8_gemm_runs.restype = i32
         L.odl_fp8_gemm_splitk.argtypes = [vp, vp, i64, i64, i64, i32, i32, i32, i32, vp, i64, vp, i64, vp, vp, i32, i32, i32, vp, i64, vp]
         L.odl_fp8_delayed_update.argtypes = [vp, i64, i64, i64, vp, vp, vp, i32, i32, vp, vp]
         L.odl_fp8_gemm_num_variants.restype = i32
@@ -951,6 +954,9 @@ def gemm_nt(a: torch.Tensor, b: torch.Tensor, fmt_a: int, fmt_b: int, sa_inv: to
     elif out.shape != (M, N) or out.dtype != out_dtype or not out.is_contiguous():
         raise NativeError("gemm_nt: `out` has the wrong shape / dtype / layout")
     splits = gemm_split_count(M, N, K)
+    if splits == 1 and _may_split() and any(t is not None and t.numel() > 1 and t.data_ptr() % 16 for t in (sa_inv, sb_inv, bias)):
+        # vectors off the 16-byte grid, which only the split entry takes: its runs also where one launch would be faster
+        splits = int(load().odl_fp8_gemm_split_count(M, N, K, 0)) if max(M + 256, N + 256) * K < 2**31 else 1
     if splits > 1:
         return _gemm_splitk(a, b, M, N, K, fmt_a, fmt_b, K_FAST, K_FAST, sa_inv, sb_inv, bias, out, splits, accumulate)
     _check(load().odl_fp8_gemm_nt_hinted(a.data_ptr(), b.data_ptr(), M, N, K, fmt_a, fmt_b, sa_inv.data_ptr(), sa_inv.numel(),
@@ -1284,7 +1290,7 @@ def gemm_split_count(M: int, N: int, K: int, k_slow: bool = False) -> int:
     Always 1 while a kernel variant is forced or ``split_k`` is off."""
     if not split_k or getattr(_tls, "forced_variant", -1) >= 0 or (M + 256) * K >= 2**31 or (N + 256) * K >= 2**31:
         return 1
-    return int(load().odl_fp8_gemm_split_count(M, N, K, 1 if k_slow else 0))
+    return int(load().odl_fp8_gemm_runs(M, N, K, 1 if k_slow else 0))
 
 
 def _gemm_splitk(a, b, M, N, K, fmt_a, fmt_b, layout_a, layout_b, sa_inv, sb_inv, bias, out, splits, accumulate=False):

@@ -983,3 +983,29 @@ def test_fresh_operands_give_the_same_bits(N, M, Nn, K):
         assert torch.equal(N.gemm_nt(a, b, O.E4M3, O.E5M2, one, one, out_dtype=dtype, fresh=True), N.gemm_nt(a, b, O.E4M3, O.E5M2, one, one, out_dtype=dtype))
     sa, sb = (torch.full((K // 128, r, 4), 120, dtype=torch.uint8, device="cuda") for r in (M, Nn))
     assert torch.equal(N.mx_gemm_nt(a, sa, b, sb, O.E4M3, O.E5M2, fresh=True), N.mx_gemm_nt(a, sa, b, sb, O.E4M3, O.E5M2))
+
+
+def test_split_entry_runs_what_it_is_asked_for_where_one_launch_would_be_faster(N):
+    """8192 x 768 in two runs by hand: both partial results are in the workspace, and they add up."""
+    M, Nn, K = 8192, 768, 2048
+    g = torch.Generator().manual_seed(3)
+    values = torch.tensor([0.0, 0.5, 1.0, -1.0, 2.0, -0.5])
+    a, b = values[torch.randint(0, 6, (M, K), generator=g)].cuda(), values[torch.randint(0, 6, (Nn, K), generator=g)].cuda()
+    ac, bc = (t.to(torch.float8_e4m3fn).view(torch.uint8) for t in (a, b))
+    one, ws, out = torch.ones(1, device="cuda"), torch.full((2, M, Nn), float("nan"), device="cuda"), torch.empty((M, Nn), device="cuda")
+    assert N.load().odl_fp8_gemm_splitk(ac.data_ptr(), bc.data_ptr(), M, Nn, K, O.E4M3, O.E4M3, 0, 0, one.data_ptr(), 1, one.data_ptr(), 1, None,
+                                        out.data_ptr(), 1, 0, 2, ws.data_ptr(), ws.numel() * 4, torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(out, (a.double() @ b.double().t()).float()) and torch.equal(ws[0] + ws[1], out) and not torch.equal(ws[0], out)
+
+
+def test_vectors_off_the_16_byte_grid_still_go_through_the_split_entry(N):
+    """Row scales and a bias that start between 16-byte boundaries: only the entry that cuts K takes them, so where that is
+    proposed the product runs, one launch being faster or not; elsewhere it is refused, as ever."""
+    M, Nn, K = 8192, 768, 50304
+    a, b = (torch.randint(0, 0x70, (r, K), dtype=torch.uint8, device="cuda") for r in (M, Nn))
+    sa, sb, bias = torch.rand(M + 1, device="cuda") + 0.5, torch.rand(Nn + 1, device="cuda") + 0.5, torch.randn(Nn + 1, device="cuda")
+    got = N.gemm_nt(a, b, O.E4M3, O.E4M3, sa[1:], sb[1:], bias=bias[1:], out_dtype=torch.float32)
+    want = N.gemm_nt(a, b, O.E4M3, O.E4M3, sa[1:].clone(), sb[1:].clone(), bias=bias[1:].clone(), out_dtype=torch.float32)
+    assert max_rel_err(got, want) <= 1e-5
+    with pytest.raises(N.NativeError, match="16-byte"):
+        N.gemm_nt(a[:, :1024].contiguous(), b[:, :1024].contiguous(), O.E4M3, O.E4M3, sa[1:], sb[1:])

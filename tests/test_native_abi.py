@@ -317,3 +317,17 @@ def test_small_weight_gradients_read_dy_as_stored_only_where_that_is_no_slower()
     assert not pays(512, 256, 16384) and not pays(256, 256, 32768)
     assert not pays(768, 768, 8064) and pays(768, 768, 8192) and pays(2304, 768, 8192) and not pays(2048, 1024, 16384)
     assert pays(4096, 4096, 512) and pays(14336, 4096, 8192)
+
+
+def test_a_split_that_one_launch_beats_is_dropped_before_its_workspace_is_made():
+    """128 x 192 tiles in place of two runs, for every caller; the split entry itself runs what it is asked for."""
+    from optimus_dl_amd import native
+
+    if not native.is_built():
+        pytest.skip("library not built")
+    proposed = native.load().odl_fp8_gemm_split_count
+    for M, N, K in ((8192, 768, 50304), (16384, 384, 50304)):
+        assert proposed(M, N, K, 0) == 2 and native.gemm_split_count(M, N, K) == 1
+    for M, N, K in ((8192, 1024, 151936), (3072, 1536, 50304), (768, 768, 16384), (8192, 14336, 4096), (300, 512, 8192)):
+        assert native.gemm_split_count(M, N, K) == proposed(M, N, K, 0)
+    assert native.gemm_split_count(8192, 768, 50304, True) == proposed(8192, 768, 50304, 1)
