@@ -240,6 +240,8 @@ int odl_fp8_cast_rowcol(const void *x, int src_dtype, int64_t rows, int64_t cols
  *               e = (fma(p, r * r, r) + 1) * 2^k; d = 1 + e;
  *               y = bits(0x7EF311C7 - bits(d)); three times y = fma(y, fma(-d, y, 1), y);
  *               result y, 0 where -g > 80, NaN for NaN.
+ *               (coefficients and the split of ln 2: the single-precision exp of the Cephes Mathematical
+ *               Library, S. L. Moshier)
  *
  * odl_fp8_swiglu_amax_parts: h = bf16( bf16(gate * sigmoid(gate)) * up ), the value of
  *   silu(w1(x)) * w2(x) computed in bf16 (optimus_dl/modules/model/blocks/mlp.py:73-76);

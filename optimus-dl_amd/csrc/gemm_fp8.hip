@@ -3,9 +3,9 @@
 //   C[M,N] = (A[M,K] . B[N,K]^T) * (sa_inv[i] * sb_inv[j]) (+ bias[j])
 //
 // Both operands are K-contiguous 8-bit codes ("NT").  Kernels:
-//   gemm_tiled.hip : BM x BN block tiles through two LDS stages
+//   gemm_tiled.hip : BM x BN block tiles through two LDS stages (few 128x128 tiles and a short K: four)
 //   gemm_thin.hip  : small tiles, the waves of a block share K: outputs of few tiles (N % 4 == 0, K % 128 == 0)
-//   gemm_deep.hip  : 256x128 and 128x128 tiles, one block per compute unit, three LDS stages: outputs of about one tile per unit
+//   gemm_deep.hip  : 256x128, 128x192 and 128x128 tiles, one block per compute unit, three LDS stages: outputs of about one tile per unit
 //   gemm_pipe.hip  : 256x256 tile, one wave per SIMD, explicit software pipeline
 //   gemm_stream.hip: the same pipeline running across tile boundaries, epilogue under the
 //                    next tile's MFMAs (any M; N, K multiples of 128); with a split over K for

@@ -20,6 +20,8 @@ __device__ __forceinline__ float recip_newton(float d) {
 // logistic function 1 / (1 + exp(-g)): range reduction by ln 2 in two pieces, degree-5 polynomial
 // for (exp(r) - 1 - r) / r^2, exact scaling by 2^k, reciprocal as above.  A NaN argument is
 // evaluated as 0 here (every use below multiplies by the argument again, which restores the NaN).
+// The polynomial and the two pieces of ln 2 are those of the single-precision exp of the Cephes Mathematical Library
+// (S. L. Moshier, expf.c); the reciprocal's first guess is the exponent negated in the integer domain.
 __device__ __forceinline__ float sigmoid_det(float g) {
     float t = (g != g) ? 0.0f : -g;
     const bool zero = t > 80.0f;                 // exp(-g) beyond 2^115: the quotient is taken as 0

@@ -1016,7 +1016,9 @@ def gemm_swiglu_pays(M: int, N: int, K: int) -> bool:
 def gemm_swiglu(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, fmt_x: int, fmt_w: int, sx_inv: torch.Tensor, sg_inv: torch.Tensor,
                 su_inv: torch.Tensor):
     """h = silu(x . gate^T) * (x . up^T) in bf16 for at most 64 rows (the roundings of two products and :func:`swiglu_amax_parts`),
-    in one launch; x, gate, up uint8 FP8 codes [M, K], [N, K], [N, K] with one inverse scale each.  -> (h, partial maxima of |h|)."""
+    in one launch; x, gate, up uint8 FP8 codes [M, K], [N, K], [N, K] with one inverse scale each.  The products add up as the thin
+    kernel of :func:`gemm_nt` adds them: its bits from K = 2048 on, where it is chosen; below that the last places differ.
+    -> (h, partial maxima of |h|)."""
     if x.is_cuda:
         load()
         r = _host.gemm_swiglu(x, gate, up, fmt_x, fmt_w, sx_inv, sg_inv, su_inv, _stream())

@@ -512,7 +512,8 @@ def test_whole_mlp_node_stands_back_for_hooks_and_eval_mode(amp):
 @pytest.mark.parametrize("rows", [16, 32, 48, 64])
 @pytest.mark.parametrize("width,hidden", [(128, 48), (768, 2048), (2048, 5632), (1152, 14336)])
 def test_gate_up_and_product_of_a_few_rows_in_one_launch(rows, width, hidden):
-    """Bit for bit the two products of the thin kernel (which adds in the same order) and the SwiGLU kernel."""
+    """Bit for bit the two products of the thin kernel (which adds in the same order) and the SwiGLU kernel; from 2048 columns on
+    that is the kernel which separate products take by themselves."""
     from optimus_dl_amd import native as N
 
     x, g, u = seeded_bf16((rows, width), 1.0, rows), seeded_bf16((hidden, width), 0.02, 2), seeded_bf16((hidden, width), 0.02, 3)
@@ -603,3 +604,40 @@ def test_delayed_scaling_gives_gate_and_up_weight_gradients_of_their_own(amp, mo
     with recipe.backward():
         y.backward(seeded_bf16((tokens, width), 1e-3, 9).cuda())
     assert outputs.count((hidden, width)) == 2 and (2 * hidden, width) not in outputs
+
+
+@pytest.mark.parametrize("fmt_x,fmt_w", [(O.E5M2, O.E4M3), (O.E4M3, O.E5M2), (O.E5M2, O.E5M2)])
+@pytest.mark.parametrize("rows", [16, 32, 64])
+def test_gate_up_and_product_in_every_format(rows, fmt_x, fmt_w):
+    """The forms that no recipe asks for, on small multiples of powers of two: every sum of the products is exact."""
+    from optimus_dl_amd import native as N
+
+    g = torch.Generator().manual_seed(rows + fmt_x)
+    values = torch.tensor([0.0, 0.5, 1.0, -1.0, 2.0, -0.5])
+    codes = lambda t, fmt: t.to(O.TORCH_FP8[fmt]).view(torch.uint8).cuda()
+    x, gate, up = (values[torch.randint(0, 6, (n, 640), generator=g)] for n in (rows, 52, 52))
+    sx, sg, su = (torch.tensor([v]).cuda() for v in (0.125, 0.25, 0.5))
+    h, parts = N.gemm_swiglu(codes(x, fmt_x), codes(gate, fmt_w), codes(up, fmt_w), fmt_x, fmt_w, sx, sg, su)
+    want = N.swiglu_amax_parts(((x @ gate.t()) * 0.03125).bfloat16().cuda(), ((x @ up.t()) * 0.0625).bfloat16().cuda())[0]
+    assert torch.equal(h, want) and parts.max().item() == want.float().abs().max().item()
+
+
+@pytest.mark.parametrize("rows,hidden,width", [(32, 2048, 768), (64, 3072, 1024), (16, 5632, 1920)])
+def test_short_products_of_few_rows_are_as_precise_in_either_order(rows, hidden, width):
+    """Below 2048 columns gate and up in one launch add in another order than the separate products (eight partial sums of 128 products
+    at a time against one chain of 64 at a time): equally far from 64 bits.  Measured equal to 1e-4; were either sum's own
+    rounding to count, eight chains would be off by a third as much as one."""
+    from optimus_dl_amd import native as N
+
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    a = (torch.randn((rows, width), device="cuda", generator=g) * 20).to(torch.float8_e4m3fn)
+    b = (torch.randn((hidden, width), device="cuda", generator=g) * 20).to(torch.float8_e4m3fn)
+    exact, one, errors = a.double() @ b.double().t(), torch.ones(1, device="cuda"), []
+    for name in ("thin", "128x128x128 4 waves (64x64 per wave)"):
+        N.gemm_set_variant(N.gemm_variants().index(next(v for v in N.gemm_variants() if v.startswith(name) and "stages" not in v)))
+        try:
+            out = N.gemm_nt(a.view(torch.uint8), b.view(torch.uint8), O.E4M3, O.E4M3, one, one, out_dtype=torch.float32)
+        finally:
+            N.gemm_set_variant(-1)
+        errors.append((out.double() - exact).pow(2).mean().sqrt().item())
+    assert abs(errors[0] - errors[1]) <= 1e-3 * errors[1]
