@@ -211,7 +211,8 @@ class FP8Recipe:
         # set this to False there, and every forward quantises its weight again (what the reference does).
         self.cache_weights = True
         # wgrad reads the row-major codes of dy with the tokens as the slow axis (no transposed copy of dy): "auto" where the
-        # shapes allow and it is faster (native.wgrad_direct_pays), True wherever they allow, False nowhere
+        # shapes allow and it is faster (native.wgrad_direct_pays), True also for the
+        # smallest gradients (less than 0.4 million elements) at any token count, False nowhere
         self.direct_layouts: "bool | str" = "auto"
         # partial maxima handed over by the kernel that produced a tensor (SwiGLU, RMSNorm), so that
         # the Linear that quantises this very tensor skips its amax pass; a handful of entries

@@ -276,7 +276,8 @@ class _Fp8LinearFn(torch.autograd.Function):
             # 475 us unfused for a 14336 x 4096 fp32 gradient, where the transposed route with the flag takes 395)
             ctx.wgrad_direct = (fp8_wgrad and recipe.direct_layouts and not recipe.fuse_wgrad_accumulation
                                 and native.gemm_layouts_supported(n_out, n_in, tokens, weight.dtype)
-                                and (recipe.direct_layouts is True or native.wgrad_direct_pays(n_out, n_in, tokens)))
+                                and (native.wgrad_direct_pays(n_out, n_in, tokens)
+                                     or (recipe.direct_layouts is True and n_out * n_in < 400_000)))
             if pol.kind == "delayed":
                 # the histories see a forward only when it is part of training: the module in training mode AND
                 # grad mode on (the reference's backend refreshes its state on the same condition), so a validation

@@ -769,3 +769,15 @@ def test_smallest_weight_gradients_take_the_transposed_copy_unless_told_otherwis
             recipe.direct_layouts = told
         calls.clear()
         assert max_rel_err(run_step(make_linear(w), recipe, x, dy)[2], want) <= TOL and len(calls) == direct
+
+
+def test_middle_sized_weight_gradients_take_the_transposed_copy_whatever_the_smallest_are_told(amp, monkeypatch):
+    """``direct_layouts = True`` speaks of the smallest gradients only: 1024 x 4096 stays where it is faster."""
+    from optimus_dl_amd import native
+
+    x, w, dy = seeded_bf16((512, 4096), 1.0, 60), seeded_bf16((1024, 4096), 0.02, 61), seeded_bf16((512, 1024), 1e-3, 62)
+    calls = _count_calls(monkeypatch, native, "gemm_layouts")
+    recipe = amp.create_fp8_recipe("tensorwise", "hybrid")
+    recipe.direct_layouts = True
+    run_step(make_linear(w), recipe, x, dy)
+    assert not calls
