@@ -46,7 +46,7 @@ enum odl_status {
 };
 
 /* ABI version of this header; bumped when a signature changes or an entry point is added. */
-#define ODL_FP8_ABI_VERSION 25
+#define ODL_FP8_ABI_VERSION 26
 int odl_fp8_abi_version(void);
 
 /*
@@ -415,6 +415,21 @@ int odl_fp8_gemm_nt_hinted(const uint8_t *a, const uint8_t *b, int64_t M, int64_
 int odl_fp8_gemm_nt_sum(int pairs, const uint8_t *const *a, const uint8_t *const *b, const int64_t *K,
                         int64_t M, int64_t N, int fmt_a, int fmt_b, const float *const *sa_inv,
                         const float *const *sb_inv, void *c, int out_dtype, odl_stream_t stream);
+
+/*
+ * Several products of one contraction length, C_s[M_s, N_s] = (A_s . B_s^T) * (sa_inv[s][0] * sb_inv[s][0]): the forward products
+ * of Linears fed one tensor, or their weight gradients.  a .. c: HOST arrays of `count` device pointers, M and N host arrays (all
+ * read during the call); one scale per operand, no bias.  One launch over all their tiles where odl_fp8_gemm_group_route says so,
+ * else `count` calls of odl_fp8_gemm_nt_hinted; the bits of those either way, but that the last place of an fp32 sum may
+ * differ where a product alone takes the thin kernel (which adds eight partial sums).
+ * odl_fp8_gemm_group_route: the variant that one launch would use, or -1: one by one (always for fewer than 2 or more than 4
+ * products, K % 128 != 0, K < 768, operands of 2 GiB, or a product that odl_fp8_gemm_runs cuts; otherwise what is faster).
+ * With a variant forced (odl_fp8_gemm_set_variant) one launch of that one, if it is 4, 7 or 9 and up and takes the shapes.
+ */
+int odl_fp8_gemm_group_route(int count, const int64_t *M, const int64_t *N, int64_t K, int out_dtype);
+int odl_fp8_gemm_nt_group(int count, const uint8_t *const *a, const uint8_t *const *b, const int64_t *M, const int64_t *N, int64_t K,
+                          int fmt_a, int fmt_b, const float *const *sa_inv, const float *const *sb_inv, void *const *c, int out_dtype,
+                          int fresh, odl_stream_t stream);
 
 /*
  * The same product for operands that need no transposed copy.  layout_a / layout_b say how an

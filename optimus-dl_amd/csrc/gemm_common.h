@@ -46,6 +46,25 @@ struct GemmPairs {
     const float *sa[4] = {nullptr, nullptr, nullptr, nullptr}, *sb[4] = {nullptr, nullptr, nullptr, nullptr};
 };
 
+// Several products of one contraction length in one launch: the tiles of member s are [first[s], first[s + 1]) of the launch's.
+struct GemmGroup {
+    int count = 0, total = 0;                             // products, tiles
+    int first[4] = {0, 0x7fffffff, 0x7fffffff, 0x7fffffff};
+    GemmArgs m[4];
+    __device__ __forceinline__ int member(int tile) const { return (tile >= first[1]) + (tile >= first[2]) + (tile >= first[3]); }
+};
+
+// What a kernel of one tile per block is launched with, one product (GemmArgs) or several: the tiles in all, and the product and
+// the tile of it that a block works on.
+__device__ __forceinline__ int tile_count(const GemmArgs &g) { return g.tiles_m * g.tiles_n; }
+__device__ __forceinline__ int tile_count(const GemmGroup &gg) { return gg.total; }
+__device__ __forceinline__ const GemmArgs &product_of(const GemmArgs &g, int &) { return g; }
+__device__ __forceinline__ const GemmArgs &product_of(const GemmGroup &gg, int &tile) {
+    const int s = __builtin_amdgcn_readfirstlane(gg.member(tile));
+    tile -= gg.first[s];
+    return gg.m[s];
+}
+
 __device__ __forceinline__ int swz(int row) { return (row ^ (row >> 3)) & 7; }
 
 // D[i][j] += sum_k first[i][k] * second[j][k]; lane l supplies row l%32 and 32 K-bytes
@@ -326,12 +345,25 @@ void launch_gemm_thin(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_
 // the kernel for outputs of few tiles (gemm_fp8.hip); operands under 2 GiB each, K % 128 == 0
 enum FewTiles { kManyTiles, kTwoBlocks, kDeepWide, kDeep192, kDeep };
 FewTiles gemm_few_tiles(int64_t M, int64_t N, int64_t K, int num_cus);
+struct TileCounts {                 // of an output, or of several together
+    int64_t t128 = 0, t192 = 0, wide = 0, t256 = 0;        // 128 x 128, 128 x 192, 256 x 128, 256 x 256
+    TileCounts() = default;
+    TileCounts(int64_t M, int64_t N) {
+        const int64_t m1 = (M + 127) / 128, m2 = (M + 255) / 256, n1 = (N + 127) / 128;
+        t128 = m1 * n1; t192 = m1 * ((N + 191) / 192); wide = m2 * n1; t256 = m2 * ((N + 255) / 256);
+    }
+};
+FewTiles gemm_few_tiles(const TileCounts &tiles, int64_t K, int num_cus);
 // bm x bn: 128 x 128, 128 x 192 or 256 x 128
 void launch_gemm_deep(int bm, int bn, int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
 void launch_gemm_pipe(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
 bool gemm_stream_accepts(const GemmArgs &g);
 void launch_gemm_stream(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream);
 bool gemm_stream_accepts_pairs(const GemmArgs &g, const GemmPairs &pairs);
+bool gemm_stream_accepts_group(const GemmArgs &g);
+void launch_gemm_stream_group(int fa, int fb, const GemmGroup &gg, int num_cus, hipStream_t stream);
+void launch_gemm_deep_group(int bm, int bn, int fa, int fb, const GemmGroup &gg, int num_cus, hipStream_t stream);
+void launch_gemm_tiled_group(int fa, int fb, const GemmGroup &gg, hipStream_t stream);
 void launch_gemm_stream_pairs(int fa, int fb, const GemmArgs &g, const GemmPairs &pairs, int num_cus, hipStream_t stream);
 // gemm_fp8.hip: hands the calling thread's clock-probe record (odl_fp8_gemm_set_clock_probe), if any, to a streaming launch
 void attach_clock_probe(GemmArgs &g);

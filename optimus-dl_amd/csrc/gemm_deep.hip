@@ -41,8 +41,10 @@ constexpr int NW = 4, STAGES = 3;
 // and shifts them so that byte 0 / byte 2 are what it supplies in the first / second half (lanes 32 .. 63 hold the odd
 // blocks).  The instruction takes registers 0 .. 3 / 4 .. 7 as K 16 g .. / 32 + 16 g .., so the chunks of a fragment are lg and
 // 2 + lg; without scales any 32 of the 64 bytes do.
-template <int TM, int TN, int FA, int FB, bool MX>
-__global__ __launch_bounds__(256) void gemm_nt_deep_kernel(const GemmArgs g) {
+//
+// Args: one product, or several (GemmGroup)
+template <int TM, int TN, int FA, int FB, bool MX, class Args>
+__global__ __launch_bounds__(256) void gemm_nt_deep_kernel(const Args args) {
     constexpr int BM = 64 * TM, BN = 64 * TN, WM = 32 * TM, WN = 32 * TN;
     constexpr int A_BYTES = BM * 128, CODES = (BM + BN) * 128, STAGE = CODES + (MX ? (BM + BN + 255) / 256 * 1024 : 0);
     constexpr int LA = BM / 32, LB = BN / 32, SC = MX ? (BM + BN + 255) / 256 : 0, PER = LA + LB + SC;         // direct-to-LDS loads per wave and step
@@ -51,14 +53,17 @@ __global__ __launch_bounds__(256) void gemm_nt_deep_kernel(const GemmArgs g) {
     static_assert(PER * (STAGES - 1) <= 63, "the counter holds 63 loads");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[STAGES * STAGE];
 
-    const int total = g.tiles_m * g.tiles_n;
+    const int total = tile_count(args);
     const int per_xcd = (total + 7) / 8;
-    const int pid = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
+    int pid = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if ((int)blockIdx.x >= 8 * per_xcd) {
-        warm_operands(g, (int)blockIdx.x - 8 * per_xcd, (int)gridDim.x - 8 * per_xcd, 10);
+        const int spare = (int)blockIdx.x - 8 * per_xcd, spares = (int)gridDim.x - 8 * per_xcd;
+        if constexpr (std::is_same_v<Args, GemmArgs>) warm_operands(args, spare, spares, 10);
+        else warm_operands(args.m[spare % args.count], spare / args.count, spares / args.count, 10);
         return;
     }
     if (pid >= total) return;
+    const GemmArgs &g = product_of(args, pid);
     const int in_group = GM * g.tiles_n;
     const int first_m = (pid / in_group) * GM;
     const int group_rows = min(g.tiles_m - first_m, GM);
@@ -236,9 +241,9 @@ void launch_deep_tile(int bm, int bn, const GemmArgs &g, int num_cus, hipStream_
     const int total = g.tiles_m * g.tiles_n;
     const int whole = (total + 7) / 8 * 8;                // a multiple of 8, as is the launch: see the placement in the kernel
     const dim3 grid((unsigned)(whole < num_cus && warming_pays(g) ? num_cus : whole)), block(256);
-    if (bm == 128 && bn == 128) hipLaunchKernelGGL((gemm_nt_deep_kernel<2, 2, FA, FB, MX>), grid, block, 0, stream, g);
-    else if (bm == 128) hipLaunchKernelGGL((gemm_nt_deep_kernel<2, 3, FA, FB, MX>), grid, block, 0, stream, g);
-    else hipLaunchKernelGGL((gemm_nt_deep_kernel<4, 2, FA, FB, MX>), grid, block, 0, stream, g);
+    if (bm == 128 && bn == 128) hipLaunchKernelGGL((gemm_nt_deep_kernel<2, 2, FA, FB, MX, GemmArgs>), grid, block, 0, stream, g);
+    else if (bm == 128) hipLaunchKernelGGL((gemm_nt_deep_kernel<2, 3, FA, FB, MX, GemmArgs>), grid, block, 0, stream, g);
+    else hipLaunchKernelGGL((gemm_nt_deep_kernel<4, 2, FA, FB, MX, GemmArgs>), grid, block, 0, stream, g);
 }
 
 template <int FA, int FB>
@@ -247,7 +252,25 @@ void launch_deep_fmt(int bm, int bn, const GemmArgs &g, int num_cus, hipStream_t
     else launch_deep_tile<FA, FB, false>(bm, bn, g, num_cus, stream);
 }
 
+template <int FA, int FB>
+void launch_deep_group_fmt(int bm, int bn, const GemmGroup &gg, int num_cus, hipStream_t stream) {
+    const int whole = (gg.total + 7) / 8 * 8;
+    bool warm = whole < num_cus;
+    for (int s = 0; s < gg.count; ++s) warm = warm && warming_pays(gg.m[s]);
+    warm = warm && num_cus - whole >= gg.count;
+    const dim3 grid((unsigned)(warm ? num_cus : whole)), block(256);
+    if (bm == 128 && bn == 128) hipLaunchKernelGGL((gemm_nt_deep_kernel<2, 2, FA, FB, false, GemmGroup>), grid, block, 0, stream, gg);
+    else if (bm == 128) hipLaunchKernelGGL((gemm_nt_deep_kernel<2, 3, FA, FB, false, GemmGroup>), grid, block, 0, stream, gg);
+    else hipLaunchKernelGGL((gemm_nt_deep_kernel<4, 2, FA, FB, false, GemmGroup>), grid, block, 0, stream, gg);
+}
+
 }  // namespace
+
+void launch_gemm_deep_group(int bm, int bn, int fa, int fb, const GemmGroup &gg, int num_cus, hipStream_t stream) {
+    if (fa == ODL_FP8_E4M3 && fb == ODL_FP8_E4M3) launch_deep_group_fmt<ODL_FP8_E4M3, ODL_FP8_E4M3>(bm, bn, gg, num_cus, stream);
+    else if (fa == ODL_FP8_E5M2 && fb == ODL_FP8_E4M3) launch_deep_group_fmt<ODL_FP8_E5M2, ODL_FP8_E4M3>(bm, bn, gg, num_cus, stream);
+    else launch_deep_group_fmt<ODL_FP8_E5M2, ODL_FP8_E5M2>(bm, bn, gg, num_cus, stream);
+}
 
 void launch_gemm_deep(int bm, int bn, int fa, int fb, const GemmArgs &g, int num_cus, hipStream_t stream) {
     if (fa == ODL_FP8_E4M3 && fb == ODL_FP8_E4M3) launch_deep_fmt<ODL_FP8_E4M3, ODL_FP8_E4M3>(bm, bn, g, num_cus, stream);

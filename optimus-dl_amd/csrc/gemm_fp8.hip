@@ -152,11 +152,13 @@ static bool thin_pays(int64_t M, int64_t N, int64_t K) {
 // -> 8.7, where two blocks per unit hide each other's ends).  More: 256 x 128 tiles of the same kernel, one per unit, from 24 K steps on (2048 x 4096 x 8192 52.9 us against 60.5 with two 128 x 128
 // blocks per unit, x 4096 30.3 against 32.4); with fewer steps the blocks that hide each other's fill and drain win (x 2048:
 // 18.0 against 18.4, x 1024 11.6 against 12.7).
-FewTiles gemm_few_tiles(int64_t M, int64_t N, int64_t K, int num_cus) {
-    if (((M + 127) / 128) * ((N + 127) / 128) <= num_cus) return K >= 2048 ? kDeep : kTwoBlocks;
-    if (((M + 255) / 256) * ((N + 255) / 256) * 2 > num_cus) return kManyTiles;
-    if (K >= 1024 && ((M + 127) / 128) * ((N + 191) / 192) <= num_cus) return kDeep192;
-    return K >= 3072 && ((M + 255) / 256) * ((N + 127) / 128) <= num_cus ? kDeepWide : kTwoBlocks;
+FewTiles gemm_few_tiles(int64_t M, int64_t N, int64_t K, int num_cus) { return gemm_few_tiles(TileCounts(M, N), K, num_cus); }
+
+FewTiles gemm_few_tiles(const TileCounts &t, int64_t K, int num_cus) {
+    if (t.t128 <= num_cus) return K >= 2048 ? kDeep : kTwoBlocks;
+    if (t.t256 * 2 > num_cus) return kManyTiles;
+    if (K >= 1024 && t.t192 <= num_cus) return kDeep192;
+    return K >= 3072 && t.wide <= num_cus ? kDeepWide : kTwoBlocks;
 }
 
 // ... as a variant (kNoVariant: many tiles)
@@ -568,4 +570,113 @@ extern "C" int odl_fp8_gemm_splitk(const uint8_t *a, const uint8_t *b, int64_t M
     }
     launch_splitk_reduce((const float *)workspace, splits, M, N, sa_inv, sa_vec, sb_inv, sb_vec, bias, c, out_dtype, accumulate != 0, stream);
     return check_launch("odl_fp8_gemm_splitk");
+}
+
+// ------------------------------------------------------- several products in one launch
+// What launches cost, in microseconds: of `variant` over t tiles of its size in all, K in steps of 128.  Fitted to products of 256
+// to 14336 rows and columns, K = 768 .. 8192, within 15 % where it decides; the fill of a launch and its last stores are the
+// constants.  A last round of 256 x 256 tiles that leaves units idle runs faster than a full one (power, caches): 0.55 of
+// one and up.
+static double launch_us(int variant, const TileCounts &t, int64_t steps, int cus) {
+    const double k = (double)steps;
+    if (variant == kStreamVariant) {
+        const double rest = (double)(t.t256 % cus) / cus;
+        return ((double)(t.t256 / cus) + (rest > 0.0 ? 0.55 + 0.45 * rest : 0.0)) * k * 1.4 + 8.0;
+    }
+    if (variant == kDeepVariant) return 0.37 * k + 6.0;
+    if (variant == kDeepWideVariant || variant == kDeep192Variant) return 0.70 * k + 7.0;
+    return t.t128 <= cus ? 0.30 * k + 5.5 : (double)((t.t128 + 2 * cus - 1) / (2 * cus)) * 0.62 * (k + 3.0) + 4.0;
+}
+
+static int variant_of(FewTiles few) {
+    return few == kManyTiles ? kStreamVariant : few == kTwoBlocks ? 4 : few == kDeep ? kDeepVariant : few == kDeep192 ? kDeep192Variant : kDeepWideVariant;
+}
+
+// The kernel that computes several products of one contraction length in one launch, or kNoVariant: one by one.
+//
+// Products that a Linear's siblings need side by side (q / k / v, gate / up, and their weight gradients) each leave a last round of
+// tiles part empty, or are too small to fill the chip at all, and each pays a launch's fill and drain.  Together they are one
+// launch of gemm_few_tiles's kernel for all their tiles.  Same K order as alone, so the same bits (fp32 sums of products
+// that alone take the thin kernel add in that kernel's order instead: its error, gemm_fp8.hip).  us one by one / in one launch:
+//   8192 x (4096, 1024, 1024) x 4096 160.7 / 146.9   2048 x (4096, 1024, 1024) x 4096 64.4 / 44.3   256 x the same 32.1 / 15.7
+//   4016 x (5632, 5632) x 2048 93.2 / 76.9           8192 x (3072, 3072) x 1024 59.8 / 49.9        1024 x the same 14.4 / 11.0
+//   (3072, 3072) x 1024 x 8192 fp32 61.8 / 51.4      (5632, 5632) x 2048 x 4096 fp32 91.3 / 89.9   (14336 x 2) x 4096 x 4096 395 / 369
+//   8192 x (14336, 14336) x 4096 696 / 707: whole rounds either way, and the launches of their own are a little faster
+// so the model above has to promise 3 %.  K from 768 on, which is where it was measured.
+static int group_variant(int count, const int64_t *M, const int64_t *N, int64_t K, int out_dtype) {
+    if (count < 2 || count > 4 || K < 128 || K % 128 != 0) return kNoVariant;
+    const int cus = cu_count();
+    bool stream_ok = K >= 512;
+    TileCounts all;
+    double apart = 0.0;
+    for (int s = 0; s < count; ++s) {
+        if (M[s] <= 0 || N[s] <= 0 || (double)(M[s] + 256) * (double)K >= 2147483648.0 || (double)(N[s] + 256) * (double)K >= 2147483648.0) return kNoVariant;
+        GemmArgs g = {};
+        g.M = M[s]; g.N = N[s]; g.K = K;
+        g.out_dtype = out_dtype;
+        stream_ok = stream_ok && gemm_stream_accepts_group(g);
+        const TileCounts own(M[s], N[s]);
+        all.t128 += own.t128; all.t192 += own.t192; all.wide += own.wide; all.t256 += own.t256;
+        if (t_forced_variant >= 0) continue;
+        if (K < 768 || odl_fp8_gemm_runs(M[s], N[s], K, 0) > 1) return kNoVariant;         // (K in runs: a workspace, which the caller brings)
+        const Route route = route_of(M[s], N[s], K, out_dtype, 0, -1);
+        apart += route.variant == kThinVariant ? 4.0 + 0.0027 * gemm_thin_rows(M[s], N[s], cus) * (double)(K / 128)
+                 : route.tail > 0 ? launch_us(kStreamVariant, TileCounts(M[s] - route.tail, N[s]), K / 128, cus) +
+                                        launch_us(route.tail_variant, TileCounts(route.tail, N[s]), K / 128, cus)
+                                  : launch_us(route.variant, own, K / 128, cus);
+    }
+    if (all.t128 > 0x7ffffff0LL) return kNoVariant;
+    const int variant = t_forced_variant >= 0 ? t_forced_variant : variant_of(gemm_few_tiles(all, K, cus));
+    if (variant == kStreamVariant ? !stream_ok : variant != 4 && variant < kDeepWideVariant) return kNoVariant;
+    return t_forced_variant >= 0 || launch_us(variant, all, K / 128, cus) < 0.97 * apart ? variant : kNoVariant;
+}
+
+extern "C" int odl_fp8_gemm_group_route(int count, const int64_t *M, const int64_t *N, int64_t K, int out_dtype) {
+    if (!M || !N || (out_dtype != ODL_BF16 && out_dtype != ODL_F32)) {
+        set_error(ODL_ERR_ARG, "odl_fp8_gemm_group_route: null pointer, or out_dtype %d", out_dtype);
+        return -1;
+    }
+    return group_variant(count, M, N, K, out_dtype);
+}
+
+extern "C" int odl_fp8_gemm_nt_group(int count, const uint8_t *const *a, const uint8_t *const *b, const int64_t *M, const int64_t *N, int64_t K,
+                                     int fmt_a, int fmt_b, const float *const *sa_inv, const float *const *sb_inv, void *const *c, int out_dtype,
+                                     int fresh, odl_stream_t stream_) {
+    if (count < 1 || !a || !b || !M || !N || !sa_inv || !sb_inv || !c) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt_group: null pointer, or %d products", count);
+    const int variant = group_variant(count, M, N, K, out_dtype);
+    // (E4M3 times E5M2 is no product of a Linear: its kernels are not built)
+    bool one = variant != kNoVariant && (out_dtype == ODL_BF16 || out_dtype == ODL_F32) &&
+               (fmt_b == ODL_FP8_E4M3 ? fmt_a == ODL_FP8_E4M3 || fmt_a == ODL_FP8_E5M2 : fmt_b == ODL_FP8_E5M2 && fmt_a == ODL_FP8_E5M2);
+    for (int s = 0; one && s < count; ++s) {
+        one = a[s] && b[s] && sa_inv[s] && sb_inv[s] && c[s];
+        for (const void *p : {(const void *)a[s], (const void *)b[s], (const void *)c[s]}) one = one && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
+    }
+    if (!one) {                    // one by one, with the checks of that entry
+        for (int s = 0; s < count; ++s) {
+            const int rc = odl_fp8_gemm_nt_hinted(a[s], b[s], M[s], N[s], K, fmt_a, fmt_b, sa_inv[s], 1, sb_inv[s], 1, nullptr, ODL_F32, c[s], out_dtype,
+                                                  0, fresh, stream_);
+            if (rc != ODL_OK) return rc;
+        }
+        return ODL_OK;
+    }
+    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+    const int bm = kVariants[variant].bm, bn = kVariants[variant].bn;
+    GemmGroup gg;
+    gg.count = count;
+    for (int s = 0; s < count; ++s) {
+        GemmArgs &g = gg.m[s];
+        g.a = a[s]; g.b = b[s]; g.c = c[s]; g.sa = sa_inv[s]; g.sb = sb_inv[s]; g.bias = nullptr;
+        g.M = M[s]; g.N = N[s]; g.K = K;
+        g.sa_vec = g.sb_vec = 0;
+        g.out_dtype = out_dtype;
+        g.fresh = fresh != 0;
+        const int64_t tm = (M[s] + bm - 1) / bm, tn = (N[s] + bn - 1) / bn;
+        g.tiles_m = (int)tm; g.tiles_n = (int)tn;
+        gg.first[s] = gg.total;
+        gg.total += (int)(tm * tn);
+    }
+    if (variant == kStreamVariant) launch_gemm_stream_group(fmt_a, fmt_b, gg, cu_count(), stream);
+    else if (variant == 4) launch_gemm_tiled_group(fmt_a, fmt_b, gg, stream);
+    else launch_gemm_deep_group(bm, bn, fmt_a, fmt_b, gg, cu_count(), stream);
+    return check_launch("odl_fp8_gemm_nt_group");
 }

@@ -96,10 +96,14 @@ __device__ __forceinline__ v16f mma_step(const v8i &b, const v8i &a, const v16f 
 // ends with a fold, a pair ends with the accumulators multiplied by (scale product of this pair) / (that of the next)
 // under the first MFMAs of the next pair.  After the last pair the fold applies the last pair's scale product, so
 // C = ((acc_0 r_0 + acc_1) r_1 + ...) s_last in fp32 with one rounding to the output type.
-template <int FA, int FB, bool TA, bool TB, bool F32, int EPI, bool MX, bool SEG>
-__device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const GemmPairs &gp) {
+//
+// GRP: the tiles are those of up to four products (gg) with one contraction length and one scale per operand, g being the first:
+// where a tile begins or ends, its operands, output, row length and scale product are its own product's.
+template <int FA, int FB, bool TA, bool TB, bool F32, int EPI, bool MX, bool SEG, bool GRP>
+__device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const GemmPairs &gp, const GemmGroup &gg) {
     static_assert(!MX || (!TA && !TB && EPI != 1), "block scales: both operands stored [rows, K], no scale vectors");
     static_assert(!SEG || (!TA && !TB && EPI == 0 && !MX), "operand pairs: both stored [rows, K], one scale each");
+    static_assert(!GRP || (!TA && !TB && EPI == 0 && !MX && !SEG), "grouped products: operands stored [rows, K], one scale each");
     constexpr int ESZ = F32 ? 4 : 2;
     constexpr int VEC_BYTES = 3 * 128 * 4;     // per wave: 128 row scales, 128 column scales, 128 bias values
     __shared__ __attribute__((aligned(1024))) uint8_t sA0[REGION];
@@ -121,7 +125,9 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
     // partial result to slice `split` of the workspace that g.c then points to.
     int KT = 0;
     bool padded = false;
-    const int tiles = g.tiles_m * g.tiles_n;
+    const int tiles = GRP ? gg.total : g.tiles_m * g.tiles_n;
+    auto member_of = [&](int p) { return GRP ? __builtin_amdgcn_readfirstlane(gg.member(p)) : 0; };
+    auto args_of = [&](int member) -> const GemmArgs & { return GRP ? gg.m[member] : g; };
     auto item_steps = [&](int p, int &first_step, int &kt, bool &pad) {
         first_step = __builtin_amdgcn_readfirstlane((p / tiles) * g.split_steps);
         const int real = min(g.split_steps, (int)(g.K / 128) - first_step);
@@ -138,7 +144,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
     int pid = xcd * per_xcd + (int)(blockIdx.x / 8);
     if (pid >= pid_end) {
         // more blocks than tiles (launch_gemm_stream): the last ones of each XCD read the operands ahead of the others
-        if constexpr (!TA && !TB && !SEG)
+        if constexpr (!TA && !TB && !SEG && !GRP)
             if (stride > per_xcd && (int)(blockIdx.x / 8) >= per_xcd)
                 warm_operands(g, ((int)(blockIdx.x / 8) - per_xcd) * 8 + xcd, (stride - per_xcd) * 8, 30);
         return;
@@ -156,11 +162,11 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
     // ---- per-tile addressing: the tile's origin lives in the buffer resources, the
     // per-lane offsets are the same for every tile and for both operands
     const v4i empty = {0, 0, 0, 0x00020000};      // zero bytes: loads read as zero, stores are dropped
-    auto tile_origin = [&](int item, int &tm0, int &tn0) {
-        const int p = item % tiles;
-        const int in_group = GM * g.tiles_n;
+    auto tile_origin = [&](int item, int member, int &tm0, int &tn0) {
+        const int p = GRP ? item - gg.first[member] : item % tiles;
+        const int in_group = GM * args_of(member).tiles_n;
         const int first_m = (p / in_group) * GM;
-        const int group_rows = min(g.tiles_m - first_m, GM);
+        const int group_rows = min(args_of(member).tiles_m - first_m, GM);
         // (integer division runs on the vector unit: readfirstlane states that the results are uniform)
         tm0 = __builtin_amdgcn_readfirstlane((first_m + (p % in_group) % group_rows) * BM);
         tn0 = __builtin_amdgcn_readfirstlane(((p % in_group) / group_rows) * BN);
@@ -328,7 +334,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
 
     // ---- output side of the folded epilogue
     const int n2 = (int)g.N * ESZ;                // bytes per output row
-    const int c_off0 = (wm0 * (int)g.N + wn0) * ESZ;
+    const int c_off0 = (wm0 * (int)g.N + wn0) * ESZ;          // (GRP: of the first product; see phase_a_fold)
     auto uniform = [](float v) { return bits_to_float((uint32_t)__builtin_amdgcn_readfirstlane((int)float_to_bits(v))); };
     // SEG: between pair s and s + 1 the accumulators take sRatio[s] = (scale product of s) / (that of s + 1); kept in
     // LDS (read once per pair) rather than in scalar registers, of which the K loop leaves none to spare
@@ -337,7 +343,11 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         if (s + 1 < gp.count) sRatio[s] = (gp.sa[s][0] * gp.sb[s][0]) / (gp.sa[s + 1][0] * gp.sb[s + 1][0]);
         // (first read after the K loop of the first pair, many barriers from here)
     }
-    const float s_tensor = g.splits > 1 ? 1.0f :       // partial results leave unscaled
+    if constexpr (GRP) {                          // (first read behind the first tile's K loop)
+        const int s = (int)threadIdx.x;
+        if (s <= member_of(tiles - 1)) sRatio[s] = gg.m[s].sa[0] * gg.m[s].sb[0];
+    }
+    const float s_tensor = g.splits > 1 || GRP ? 1.0f :       // partial results leave unscaled
         SEG ? uniform(gp.sa[gp.count - 1][0] * gp.sb[gp.count - 1][0]) : uniform(g.sa[0] * g.sb[0]);
     // N is a multiple of 128 = the width of a wave tile: in the last tile column a wave is either wholly inside or wholly
     // outside.  One that is outside computes on the zeros that the bounded operand loads deliver and stores through the
@@ -345,14 +355,14 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
     // inside the matrix, and the row of a store is part of its per-lane offset, which the hardware checks against that
     // end (the scalar offset it does not check).  The last tile row costs what a whole one does and no more: 4016 tokens
     // are 16 tile rows like 4096; before, such a product took the tiled kernels (4016 x 5632 x 2048: 92.0 us, here 48.9).
-    auto wave_inside = [&](int tm0, int tn0) { return tm0 + wm0 < (int)g.M && tn0 + wn0 < (int)g.N; };
-    auto rsrc_out = [&](int item, int tm0, int tn0) -> v4i {
+    auto wave_inside = [&](int tm0, int tn0, const GemmArgs &o) { return tm0 + wm0 < (int)o.M && tn0 + wn0 < (int)o.N; };
+    auto rsrc_out = [&](int item, int tm0, int tn0, const GemmArgs &o, int row_bytes) -> v4i {
         const int split = __builtin_amdgcn_readfirstlane(item / tiles);
-        const uint64_t addr = reinterpret_cast<uint64_t>(reinterpret_cast<uint8_t *>(g.c) +
-                                                         ((int64_t)split * g.M * g.N + (int64_t)tm0 * g.N + tn0) * ESZ);
-        const int bytes = min((int)g.M - tm0, BM) * n2;          // < 2 GiB (checked by the caller)
+        const uint64_t addr = reinterpret_cast<uint64_t>(reinterpret_cast<uint8_t *>(o.c) +
+                                                         ((int64_t)split * o.M * o.N + (int64_t)tm0 * o.N + tn0) * ESZ);
+        const int bytes = min((int)o.M - tm0, BM) * row_bytes;   // < 2 GiB (checked by the caller)
         const v4i whole = {(int)(uint32_t)addr, (int)(uint32_t)(addr >> 32), bytes, 0x00020000};
-        return wave_inside(tm0, tn0) ? whole : empty;
+        return wave_inside(tm0, tn0, o) ? whole : empty;
     };
     // `us`: the slab's position in the wave tile's row, in slabs of 128 bytes
     auto store_slab = [](const u32x4 (&data)[4], int vo, const v4i &rsrc, int row_bytes, int t, int us) {
@@ -427,7 +437,10 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
     //   fp32: every sub-tile is a slab of 32 rows x 32 floats, read back at once and stored one MFMA later
     // EPI > 0: the wave's slices of the scale vectors (and of the bias) were brought to LDS by
     // `request_vectors`; those of sub-tile i + 1 are read while MFMA i runs.
-    auto phase_a_fold = [&](const uint8_t *sa_cur, const uint8_t *sb_cur, const v4i &rsrc_c) {
+    auto phase_a_fold = [&](const uint8_t *sa_cur, const uint8_t *sb_cur, const v4i &rsrc_c, const int done, const int done_n2) {
+        // GRP: the row length and the scale product of the tile that leaves, of product `done`
+        const int row_bytes = GRP ? done_n2 : n2;
+        const float scale = GRP ? sRatio[done] : s_tensor;
         // addresses are derived here (laundered ids), not kept in registers across the K loop
         int lane_e = lane, wave_e = wave;
         asm volatile("" : "+v"(lane_e));
@@ -435,7 +448,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         const uint32_t slab = lds_addr_of(sEpi) + wave_e * SLAB;
         const uint32_t epi_w = slab + (lane_e % 32) * PITCH + (lane_e / 32) * (F32 ? 16 : 8);
         const uint32_t epi_r = slab + (lane_e / 8) * PITCH + (lane_e % 8) * 16;
-        const int c_voff = c_off0 + (lane_e / 8) * n2 + (lane_e % 8) * 16;
+        const int c_voff = (GRP ? wm0 * row_bytes + wn0 * ESZ : c_off0) + (lane_e / 8) * row_bytes + (lane_e % 8) * 16;
         const uint32_t vec_row = lds_addr_of(sVec) + wave_e * VEC_BYTES + (lane_e % 32) * 4;          // sa of row lr
         const uint32_t vec_col = lds_addr_of(sVec) + wave_e * VEC_BYTES + 512 + (lane_e / 32) * 16;   // sb of columns 4 lg ..
         float sa_next = 0.0f;
@@ -464,7 +477,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
                     }
             } else {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) v[e] = acc[t][u][e] * s_tensor;
+                for (int e = 0; e < 16; ++e) v[e] = acc[t][u][e] * scale;
             }
             uint32_t pk[8];
             if constexpr (!F32) {
@@ -479,7 +492,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
                 if (i < 15) read_vectors((i + 1) / 4, (i + 1) % 4);
             }
             if constexpr (F32) {
-                if (i > 0) store_slab(back, c_voff, rsrc_c, n2, (i - 1) / 4, (i - 1) % 4);
+                if (i > 0) store_slab(back, c_voff, rsrc_c, row_bytes, (i - 1) / 4, (i - 1) % 4);
                 // lane (lr, lg) holds columns 8q + 4lg + {0..3} of row lr: 16 bytes at 32q + 16lg, as two 8-byte
                 // writes (the row pitch of 34 dwords spreads the 32 rows of a half-wave over all 64 banks)
 #pragma unroll
@@ -502,14 +515,14 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
 #pragma unroll
                     for (int j = 0; j < 4; ++j) back[j] = lds_r(epi_r + j * 8 * PITCH);
                 } else if (i > 0) {
-                    store_slab(back, c_voff, rsrc_c, n2, (i - 2) / 4, ((i - 2) % 4) / 2);   // completed one MFMA ago
+                    store_slab(back, c_voff, rsrc_c, row_bytes, (i - 2) / 4, ((i - 2) % 4) / 2);   // completed one MFMA ago
                 }
             }
             if (i < 4) a1[i] = read_a(sa_cur, i, 1);
             else if (i < 8) b1[i - 4] = read_b(sb_cur, i - 4, 1);
             __builtin_amdgcn_sched_barrier(0);
         }
-        store_slab(back, c_voff, rsrc_c, n2, 3, F32 ? 3 : 1);
+        store_slab(back, c_voff, rsrc_c, row_bytes, 3, F32 ? 3 : 1);
         __builtin_amdgcn_sched_barrier(0);
     };
     // EPI > 0: this wave's 128 row scales, 128 column scales (and 128 bias values) of the tile at (tm0, tn0)
@@ -524,7 +537,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         // the bounds of a descriptor cover the per-lane offset only, not the scalar one: a wave outside the matrix
         // must not request its (non-existent) slices at all, and the row goes into the per-lane offset (rows past the
         // end, in the last tile row of an M that is not a multiple of 128, read as zero)
-        const bool inside = wave_inside(tm0, tn0);
+        const bool inside = wave_inside(tm0, tn0, g);
         const v4i ra_ = inside ? rsrc_vec(g.sa, g.sa_vec ? g.M : 1) : empty, rb_ = inside ? rsrc_vec(g.sb, g.sb_vec ? g.N : 1) : empty;
         const int vb = lane * 4 * g.sb_vec;
 #pragma unroll
@@ -585,7 +598,8 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
     };
 
     // ---- first tile: steps 0 and 1 requested and awaited, then phase A of step 0
-    tile_origin(pid, m0, n0);
+    int member = member_of(pid);                  // GRP: the product that the current tile belongs to
+    tile_origin(pid, member, m0, n0);
     int seg = 0;                                  // SEG: the operand pair the block is on
     if constexpr (SEG) {
         KT = gp.k[0] / 128;                    // an even number of steps, at least 4 (checked by the caller)
@@ -594,8 +608,8 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
     } else {
         int first_step = 0;
         item_steps(pid, first_step, KT, padded);
-        rsrc_a = rsrc_for(g.a, m0, g.M, TA, first_step, (int)g.K);
-        rsrc_b = rsrc_for(g.b, n0, g.N, TB, first_step, (int)g.K);
+        rsrc_a = rsrc_for(args_of(member).a, m0, args_of(member).M, TA, first_step, (int)g.K);
+        rsrc_b = rsrc_for(args_of(member).b, n0, args_of(member).N, TB, first_step, (int)g.K);
         if constexpr (MX) scale_origin(m0, n0, first_step, sc_off_a, sc_off_b, sc_in_a, sc_in_b);
     }
     next_a = empty;
@@ -630,15 +644,17 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         const bool has_next = next_pid < pid_end;
         int next_m0 = 0, next_n0 = 0, next_first = 0, next_kt = 0;
         bool next_padded = false;
-        tile_origin(has_next ? next_pid : pid, next_m0, next_n0);
+        const int next_member = member_of(has_next ? next_pid : pid);
+        const GemmArgs &next_g = args_of(next_member);
+        tile_origin(has_next ? next_pid : pid, next_member, next_m0, next_n0);
         const int next_nk = SEG ? gp.k[next_seg] : (int)g.K;
         if constexpr (SEG) next_kt = next_nk / 128;
         else item_steps(has_next ? next_pid : pid, next_first, next_kt, next_padded);
-        const uint8_t *const base_a = SEG ? gp.a[next_seg] : g.a, *const base_b = SEG ? gp.b[next_seg] : g.b;
+        const uint8_t *const base_a = SEG ? gp.a[next_seg] : next_g.a, *const base_b = SEG ? gp.b[next_seg] : next_g.b;
 #ifdef ODL_EXP_SAME_PANELS            // experiment: every tile reads the operand panels of tile (0, 0): all traffic stays in the L2
-        const v4i na = rsrc_for(base_a, 0, g.M, TA, next_first, next_nk), nb = rsrc_for(base_b, 0, g.N, TB, next_first, next_nk);
+        const v4i na = rsrc_for(base_a, 0, next_g.M, TA, next_first, next_nk), nb = rsrc_for(base_b, 0, next_g.N, TB, next_first, next_nk);
 #else
-        const v4i na = rsrc_for(base_a, next_m0, g.M, TA, next_first, next_nk), nb = rsrc_for(base_b, next_n0, g.N, TB, next_first, next_nk);
+        const v4i na = rsrc_for(base_a, next_m0, next_g.M, TA, next_first, next_nk), nb = rsrc_for(base_b, next_n0, next_g.N, TB, next_first, next_nk);
 #endif
         next_a = has_next ? na : empty;
         next_b = has_next ? nb : empty;
@@ -669,7 +685,9 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         // ---- the tile is finished; buffer 0 already holds the next tile's first fragments.
         // Phase A of the next tile's step 0 stores this tile.  Without a next tile the same
         // phase runs on whatever the empty buffer delivered, only for its stores.
-        const v4i rsrc_c = rsrc_out(pid, m0, n0);
+        const int done = member, done_n2 = GRP ? (int)args_of(done).N * ESZ : n2;
+        const v4i rsrc_c = rsrc_out(pid, m0, n0, args_of(done), done_n2);
+        member = next_member;
         pid = next_pid;
         KT = next_kt;
         padded = next_padded;
@@ -683,7 +701,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         sc_in_b = sc_nin_b;
         const int pair = seg;
         seg = next_seg;
-        if constexpr (tile_ends) phase_a_fold(sA0, sB0, rsrc_c);
+        if constexpr (tile_ends) phase_a_fold(sA0, sB0, rsrc_c, done, done_n2);
         else phase_a_rescale(sA0, sB0, pair);
         return has_next;
     };
@@ -706,13 +724,19 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
 
 template <int FA, int FB, bool TA, bool TB, bool F32, int EPI, bool MX = false>
 __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs g) {
-    gemm_nt_stream_body<FA, FB, TA, TB, F32, EPI, MX, false>(g, GemmPairs{});
+    gemm_nt_stream_body<FA, FB, TA, TB, F32, EPI, MX, false, false>(g, GemmPairs{}, GemmGroup{});
 }
 
 // the same kernel over several operand pairs (see SEG above)
 template <int FA, int FB, bool F32>
 __global__ __launch_bounds__(256) void gemm_nt_stream_pairs_kernel(const GemmArgs g, const GemmPairs gp) {
-    gemm_nt_stream_body<FA, FB, false, false, F32, 0, false, true>(g, gp);
+    gemm_nt_stream_body<FA, FB, false, false, F32, 0, false, true, false>(g, gp, GemmGroup{});
+}
+
+// the same kernel over the tiles of several products (see GRP above)
+template <int FA, int FB, bool F32>
+__global__ __launch_bounds__(256) void gemm_nt_stream_group_kernel(const GemmGroup gg) {
+    gemm_nt_stream_body<FA, FB, false, false, F32, 0, false, false, true>(gg.m[0], GemmPairs{}, gg);
 }
 
 template <int FA, int FB, bool F32>
@@ -800,6 +824,35 @@ void launch_pairs_fmt(const GemmArgs &g, const GemmPairs &gp, int blocks_per_xcd
 }
 
 }  // namespace
+
+// One product of a group: as alone, with one scale per operand and no bias.
+bool gemm_stream_accepts_group(const GemmArgs &g) {
+    return gemm_stream_accepts(g) && !g.ta && !g.tb && !g.sa_vec && !g.sb_vec && !g.bias && !g.mx_sa && g.splits == 1;
+}
+
+namespace {
+
+template <int FA, int FB>
+void launch_group_fmt(const GemmGroup &gg, int blocks_per_xcd, hipStream_t stream) {
+    const dim3 grid((unsigned)(8 * blocks_per_xcd)), block(256);
+    if (gg.m[0].out_dtype == ODL_F32) hipLaunchKernelGGL((gemm_nt_stream_group_kernel<FA, FB, true>), grid, block, 0, stream, gg);
+    else hipLaunchKernelGGL((gemm_nt_stream_group_kernel<FA, FB, false>), grid, block, 0, stream, gg);
+}
+
+}  // namespace
+
+void launch_gemm_stream_group(int fa, int fb, const GemmGroup &group, int num_cus, hipStream_t stream) {
+    GemmGroup gg = group;
+    gg.m[0].splits = 1;
+    gg.m[0].split_steps = ((int)(gg.m[0].K / 128) + 1) & ~1;
+    const int per_xcd = (gg.total + 7) / 8;
+    int bpx = num_cus / 8;
+    if (bpx < 1) bpx = 1;
+    if (bpx > per_xcd) bpx = per_xcd;
+    if (fa == ODL_FP8_E4M3 && fb == ODL_FP8_E4M3) launch_group_fmt<ODL_FP8_E4M3, ODL_FP8_E4M3>(gg, bpx, stream);
+    else if (fa == ODL_FP8_E5M2 && fb == ODL_FP8_E4M3) launch_group_fmt<ODL_FP8_E5M2, ODL_FP8_E4M3>(gg, bpx, stream);
+    else launch_group_fmt<ODL_FP8_E5M2, ODL_FP8_E5M2>(gg, bpx, stream);
+}
 
 void launch_gemm_stream_pairs(int fa, int fb, const GemmArgs &args, const GemmPairs &gp, int num_cus, hipStream_t stream) {
     GemmArgs g = args;

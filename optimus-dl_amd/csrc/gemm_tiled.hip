@@ -30,8 +30,9 @@
 namespace odl {
 
 // ------------------------------------------------------------------ tiled kernel
-template <int BM, int BN, int WAVES_M, int WAVES_N, int FA, int FB, int STAGES = 2>
-__global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_nt_tiled_kernel(const GemmArgs g) {
+// Args: one product, or several (GemmGroup)
+template <int BM, int BN, int WAVES_M, int WAVES_N, int FA, int FB, int STAGES = 2, class Args = GemmArgs>
+__global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_nt_tiled_kernel(const Args args) {
     static_assert(STAGES == 2 || STAGES == 4, "two LDS stages, or four for launches of at most one block per compute unit");
     constexpr int NW = WAVES_M * WAVES_N;
     constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, TM = WM / 32, TN = WN / 32;
@@ -47,10 +48,11 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_nt_tiled_kernel(co
     __shared__ __attribute__((aligned(1024))) uint8_t lds3[STAGES == 4 ? STAGE : 1024];
 
     // ---- which tile (XCD-aware, grouped)
-    const int total = g.tiles_m * g.tiles_n;
+    const int total = tile_count(args);
     const int per_xcd = (total + 7) / 8;
-    const int pid = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
+    int pid = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (pid >= total) return;
+    const GemmArgs &g = product_of(args, pid);
     const int in_group = GM * g.tiles_n;
     const int first_m = (pid / in_group) * GM;
     const int group_rows = min(g.tiles_m - first_m, GM);
@@ -226,6 +228,19 @@ static void launch_tiled_fmt(int variant, const GemmArgs &g, hipStream_t stream)
             hipLaunchKernelGGL((gemm_nt_tiled_kernel<128, 128, 2, 2, FA, FB>), dim3(grid), dim3(256), 0, stream, g);
         break;
     }
+}
+
+template <int FA, int FB>
+static void launch_tiled_group_fmt(const GemmGroup &gg, hipStream_t stream) {
+    const dim3 grid((unsigned)((gg.total + 7) / 8 * 8));
+    if (gg.total <= device_cu_count()) hipLaunchKernelGGL((gemm_nt_tiled_kernel<128, 128, 2, 4, FA, FB, 4, GemmGroup>), grid, dim3(512), 0, stream, gg);
+    else hipLaunchKernelGGL((gemm_nt_tiled_kernel<128, 128, 2, 2, FA, FB, 2, GemmGroup>), grid, dim3(256), 0, stream, gg);
+}
+
+void launch_gemm_tiled_group(int fa, int fb, const GemmGroup &gg, hipStream_t stream) {
+    if (fa == ODL_FP8_E4M3 && fb == ODL_FP8_E4M3) launch_tiled_group_fmt<ODL_FP8_E4M3, ODL_FP8_E4M3>(gg, stream);
+    else if (fa == ODL_FP8_E5M2 && fb == ODL_FP8_E4M3) launch_tiled_group_fmt<ODL_FP8_E5M2, ODL_FP8_E4M3>(gg, stream);
+    else launch_tiled_group_fmt<ODL_FP8_E5M2, ODL_FP8_E5M2>(gg, stream);
 }
 
 void launch_gemm_tiled(int variant, int fa, int fb, const GemmArgs &g, hipStream_t stream) {

@@ -38,6 +38,8 @@ decltype(&odl_fp8_layernorm_bwd) layernorm_bwd_c;
 decltype(&odl_fp8_amax_rowcol) amax_rowcol_c;
 decltype(&odl_fp8_cast_rowcol_padded) cast_rowcol_c;
 decltype(&odl_fp8_gemm_nt_hinted) gemm_nt_c;
+decltype(&odl_fp8_gemm_group_route) group_route_c;
+decltype(&odl_fp8_gemm_nt_group) gemm_nt_group_c;
 decltype(&odl_fp8_gemm_layouts) gemm_layouts_c;
 decltype(&odl_fp8_gemm_runs) runs_c;
 decltype(&odl_fp8_mx_cast_padded) mx_cast_c;
@@ -65,6 +67,8 @@ void bind(const py::dict &d) {
     take(amax_rowcol_c, d, "odl_fp8_amax_rowcol");
     take(cast_rowcol_c, d, "odl_fp8_cast_rowcol_padded");
     take(gemm_nt_c, d, "odl_fp8_gemm_nt_hinted");
+    take(group_route_c, d, "odl_fp8_gemm_group_route");
+    take(gemm_nt_group_c, d, "odl_fp8_gemm_nt_group");
     take(gemm_layouts_c, d, "odl_fp8_gemm_layouts");
     take(runs_c, d, "odl_fp8_gemm_runs");
     take(mx_cast_c, d, "odl_fp8_mx_cast_padded");
@@ -283,6 +287,38 @@ py::object gemm_nt(const Tensor &a, const Tensor &b, int fa, int fb, const Tenso
     return rc ? status(rc) : py::cast(c);
 }
 
+bool group_in_one_launch(const std::vector<i64> &M, const std::vector<i64> &N, i64 K, int odt) {
+    return M.size() == N.size() && M.size() <= 4 && group_route_c((int)M.size(), M.data(), N.data(), K, odt) >= 0;
+}
+
+// Several products in one launch; None where they run one by one (each then in the way that is its own)
+py::object gemm_nt_group(const std::vector<Tensor> &a, const std::vector<Tensor> &b, int fa, int fb, const std::vector<Tensor> &sa,
+                         const std::vector<Tensor> &sb, int odt, bool fresh, i64 stream) {
+    const size_t n = a.size();
+    if (n < 2 || n > 4 || b.size() != n || sa.size() != n || sb.size() != n) return none();
+    const uint8_t *pa[4], *pb[4];
+    const float *psa[4], *psb[4];
+    void *pc[4];
+    i64 M[4], N[4];
+    for (size_t s = 0; s < n; ++s) {
+        if (!codes2d(a[s]) || !codes2d(b[s]) || a[s].size(1) != a[0].size(1) || b[s].size(1) != a[0].size(1) || !floats(sa[s], 1) || !floats(sb[s], 1) ||
+            !aligned(a[s]) || !aligned(b[s]))
+            return none();
+        M[s] = a[s].size(0); N[s] = b[s].size(0);
+        pa[s] = ptr(a[s]); pb[s] = ptr(b[s]); psa[s] = ptr(sa[s]); psb[s] = ptr(sb[s]);
+    }
+    const i64 K = a[0].size(1);
+    if (group_route_c((int)n, M, N, K, odt) < 0) return none();
+    py::list out;
+    for (size_t s = 0; s < n; ++s) {
+        Tensor c = result(OptTensor(), a[s], M[s], N[s], odt);
+        pc[s] = ptr(c);
+        out.append(c);
+    }
+    const int rc = call(gemm_nt_group_c, (int)n, pa, pb, M, N, K, fa, fb, psa, psb, pc, odt, fresh, str(stream));
+    return rc ? status(rc) : py::object(out);
+}
+
 // Not accumulating; whole tiles of the kernel that reads K-slow operands (the caller has checked: gemm_layouts_supported)
 py::object gemm_layouts(const Tensor &a, const Tensor &b, int fa, int fb, bool a_slow, bool b_slow, const Tensor &sa, const Tensor &sb,
                         const OptTensor &out, int odt, bool split, i64 stream) {
@@ -360,6 +396,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("layernorm_bwd", &layernorm_bwd);
     m.def("quantize_rowcol", &quantize_rowcol);
     m.def("gemm_nt", &gemm_nt);
+    m.def("group_in_one_launch", &group_in_one_launch);
+    m.def("gemm_nt_group", &gemm_nt_group);
     m.def("gemm_layouts", &gemm_layouts);
     m.def("mx_cast", &mx_cast);
     m.def("block_cast", &block_cast);

@@ -23,7 +23,8 @@ from .. import native
 from .amp import state as _state
 from .amp.fp8 import FP8Recipe
 from .calls import apply, no_graph, untraced
-from .fp8_linear import ROLE_G, ROLE_X, FP8Linear, _converted_input, _Fp8LinearFn, _Fp8LinearGroupFn, _MemberCtx
+from .fp8_linear import (ROLE_G, ROLE_X, FP8Linear, _converted_input, _Fp8LinearFn, _Fp8LinearGroupFn, _MemberCtx, _product_jobs,
+                         _run_jobs, _wgrad_jobs)
 
 
 def _bf16_cuda(*tensors: torch.Tensor) -> bool:
@@ -81,11 +82,11 @@ class _SwiGLUMLPFn(torch.autograd.Function):
         pol = recipe.recipe
         subs, saved = [], []
 
-        def member(x, module, weight, need_x, given=None):
+        def member(x, module, weight, need_x, given=None, jobs=None):
             sub = _MemberCtx((need_x, True, False, False, False, False))
-            sub.given_input = given
+            sub.given_input, sub.y_jobs = given, jobs
             y = _Fp8LinearFn.forward(sub, x, weight, None, module, recipe, torch.bfloat16)
-            sub.given_input = None
+            sub.given_input = sub.y_jobs = None
             sub.span = (len(saved), len(sub.saved_tensors))
             saved.extend(sub.saved_tensors)
             sub.saved_tensors = ()
@@ -93,7 +94,10 @@ class _SwiGLUMLPFn(torch.autograd.Function):
             return y
 
         w1, w2, down = modules
-        gate, up = member(x2d, w1, weights[0], ctx.needs_input_grad[0]), member(x2d, w2, weights[1], ctx.needs_input_grad[0])
+        jobs = _product_jobs(recipe, (w1, w2))
+        gate, up = (member(x2d, w, weight, ctx.needs_input_grad[0], jobs=jobs) for w, weight in ((w1, weights[0]), (w2, weights[1])))
+        if jobs is not None:
+            gate, up = _run_jobs(jobs, pol.fmt_fwd, pol.fmt_fwd, torch.bfloat16, fresh=True)
         if pol.kind == "mxfp8":
             h = native.swiglu_mx_cast(gate, up, pol.fmt_fwd, pol.mx_scale_rule)
         elif pol.kind == "blockwise":
@@ -131,18 +135,21 @@ class _SwiGLUMLPFn(torch.autograd.Function):
         dgate, dup = (gate, up) if given is not None else native.swiglu_bwd_amax_parts(dh, gate, up)[:2]
         pairs = _Fp8LinearGroupFn._dgrad_in_one_gemm(ctx, (dgate, dup))
         dx, grads = None, []
+        dw_jobs = _wgrad_jobs((sub_g, sub_u), (dgate, dup))
         for i, (sub, g) in enumerate(zip((sub_g, sub_u), (dgate, dup))):
             sub.given_grad = given[i] if given is not None else None
-            sub.dx_pairs = pairs
+            sub.dx_pairs, sub.dw_jobs = pairs, dw_jobs
             # (block scales: the GEMM that adds into what is there is not the streaming one; a sum of its own is cheaper)
             sub.dx_into = dx if dx is not None and pol.kind == "delayed" else None
             dxi, dw, *_ = _Fp8LinearFn.backward(sub, g)
-            sub.given_grad = sub.dx_pairs = sub.dx_into = None
+            sub.given_grad = sub.dx_pairs = sub.dx_into = sub.dw_jobs = None
             if dx is None:
                 dx = dxi
             elif dxi is not None and pol.kind != "delayed":
                 dx = dx + dxi
             grads.append(dw)
+        if dw_jobs:
+            grads = _run_jobs(dw_jobs, pol.fmt_bwd, pol.fmt_fwd, sub_g.w_dtype)
         if pairs:
             gqs, wq_ts, sg_invs, sw_invs = zip(*pairs)
             dx = native.gemm_nt_sum(list(gqs), list(wq_ts), pol.fmt_bwd, pol.fmt_fwd, list(sg_invs), list(sw_invs), out_dtype=sub_g.x_dtype)

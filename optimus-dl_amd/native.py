@@ -26,7 +26,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 25
+ABI_VERSION = 26
 _OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
@@ -72,6 +72,8 @@ EXPORTS = (
     "odl_fp8_gemm_nt",
     "odl_fp8_gemm_nt_hinted",
     "odl_fp8_gemm_nt_sum",
+    "odl_fp8_gemm_group_route",
+    "odl_fp8_gemm_nt_group",
     "odl_fp8_gemm_layouts",
     "odl_fp8_gemm_split_count",
     "odl_fp8_gemm_runs",
@@ -164,6 +166,8 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_cast_delayed.argtypes = [vp, i32, i64, i64, vp, i32, vp, vp, vp, vp, vp]
         L.odl_fp8_gemm_nt.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, i64, vp, i64, vp, i32, vp, i32, i32, vp]
         L.odl_fp8_gemm_nt_hinted.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, i64, vp, i64, vp, i32, vp, i32, i32, i32, vp]
+        L.odl_fp8_gemm_group_route.argtypes = [i32, vp, vp, i64, i32]
+        L.odl_fp8_gemm_nt_group.argtypes = [i32, vp, vp, vp, vp, i64, i32, i32, vp, vp, vp, i32, i32, vp]
         L.odl_fp8_gemm_nt_sum.argtypes = [i32, vp, vp, vp, i64, i64, i32, i32, vp, vp, vp, i32, vp]
         L.odl_fp8_gemm_layouts.argtypes = [vp, vp, i64, i64, i64, i32, i32, i32, i32, vp, vp, vp, i32, vp]
         L.odl_fp8_gemm_split_count.argtypes = [i64, i64, i64, i32]
@@ -997,6 +1001,26 @@ def gemm_nt_sum(a: "list[torch.Tensor]", b: "list[torch.Tensor]", fmt_a: int, fm
                                       ptrs(*[t.data_ptr() for t in sa_inv]), ptrs(*[t.data_ptr() for t in sb_inv]), out.data_ptr(),
                                       odt, _stream()), "odl_fp8_gemm_nt_sum")
     return out
+
+
+def gemm_group_in_one_launch(Ms: "list[int]", Ns: "list[int]", K: int, out_dtype: torch.dtype) -> bool:
+    """Whether :func:`gemm_nt_group` computes products of these sizes in one launch."""
+    odt = _OUT_DTYPES.get(out_dtype, -1)
+    load()
+    return odt >= 0 and len(Ms) >= 2 and bool(_host.group_in_one_launch(Ms, Ns, K, odt))
+
+
+def gemm_nt_group(a: "list[torch.Tensor]", b: "list[torch.Tensor]", fmt_a: int, fmt_b: int, sa_inv: "list[torch.Tensor]",
+                  sb_inv: "list[torch.Tensor]", out_dtype: torch.dtype = torch.bfloat16, fresh: bool = False) -> "list[torch.Tensor]":
+    """[gemm_nt(a[s], b[s], ...) for s]: products of one contraction length with one scale per operand, in one launch where that is
+    faster (``odl_fp8_gemm_group_route``)."""
+    odt = _OUT_DTYPES.get(out_dtype, -1)
+    if 2 <= len(a) <= 4 and odt >= 0 and all(t.is_cuda for t in a):
+        load()
+        r = _host.gemm_nt_group(a, b, fmt_a, fmt_b, sa_inv, sb_inv, odt, fresh, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_gemm_nt_group")
+    return [gemm_nt(x, y, fmt_a, fmt_b, s, t, out_dtype=out_dtype, fresh=fresh) for x, y, s, t in zip(a, b, sa_inv, sb_inv, strict=True)]
 
 
 def gemm_swiglu_pays(M: int, N: int, K: int) -> bool:
