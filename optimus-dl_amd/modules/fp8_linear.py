@@ -444,7 +444,7 @@ class _MemberCtx:
 def _product_jobs(recipe: FP8Recipe, modules) -> "list | None":
     """An empty list for members of a group to leave their forward products in (``native.gemm_nt_group``: in one launch where that
     is faster), or None: a recipe whose products have scale vectors or block scales, biases, one member or more than four."""
-    if recipe.recipe.kind not in ("tensorwise", "delayed") or not 2 <= len(modules) <= 4 or any(m.bias is not None for m in modules):
+    if not 2 <= len(modules) <= 4 or recipe.recipe.kind not in ("tensorwise", "delayed") or any(m.bias is not None for m in modules):
         return None
     return []
 
