@@ -22,7 +22,7 @@ LIB_NAME = "libodl_fp8.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 HOST_NAME = "_host"
 HOST_PATH = os.path.join(HERE, HOST_NAME + ".so")
-SOURCES = ["api.hip", "quant.hip", "gemm_fp8.hip", "gemm_tiled.hip", "gemm_thin.hip", "gemm_deep.hip", "gemm_pipe.hip", "gemm_stream.hip", "fused.hip", "mx.hip"]
+SOURCES = ["api.hip", "quant.hip", "gemm_fp8.hip", "gemm_tiled.hip", "gemm_thin.hip", "gemm_deep.hip", "gemm_deep_many.hip", "gemm_pipe.hip", "gemm_stream.hip", "fused.hip", "mx.hip"]
 
 # Per-source additions.  The compiler-scheduled tiled GEMMs: left to its own choice the compiler computes in vector
 # registers but parks the accumulators in the accumulation registers between K steps, 64 copies out and 64 back per

@@ -44,6 +44,7 @@ struct GemmPairs {
     int k[4] = {0, 0, 0, 0};
     const uint8_t *a[4] = {nullptr, nullptr, nullptr, nullptr}, *b[4] = {nullptr, nullptr, nullptr, nullptr};
     const float *sa[4] = {nullptr, nullptr, nullptr, nullptr}, *sb[4] = {nullptr, nullptr, nullptr, nullptr};
+    const uint8_t *mx_sa[4] = {nullptr, nullptr, nullptr, nullptr}, *mx_sb[4] = {nullptr, nullptr, nullptr, nullptr};   // block scales (GemmArgs)
 };
 
 // Several products of one contraction length in one launch: the tiles of member s are [first[s], first[s + 1]) of the launch's.
@@ -54,10 +55,18 @@ struct GemmGroup {
     __device__ __forceinline__ int member(int tile) const { return (tile >= first[1]) + (tile >= first[2]) + (tile >= first[3]); }
 };
 
+// Products of one output size that are added up (gemm_deep.h).
+struct GemmChain {
+    int count = 0;
+    GemmArgs m[4];                                        // the first one's output and tiles count
+};
+
 // What a kernel of one tile per block is launched with, one product (GemmArgs) or several: the tiles in all, and the product and
 // the tile of it that a block works on.
 __device__ __forceinline__ int tile_count(const GemmArgs &g) { return g.tiles_m * g.tiles_n; }
 __device__ __forceinline__ int tile_count(const GemmGroup &gg) { return gg.total; }
+__device__ __forceinline__ int tile_count(const GemmChain &gc) { return gc.m[0].tiles_m * gc.m[0].tiles_n; }
+__device__ __forceinline__ const GemmArgs &product_of(const GemmChain &gc, int &) { return gc.m[0]; }
 __device__ __forceinline__ const GemmArgs &product_of(const GemmArgs &g, int &) { return g; }
 __device__ __forceinline__ const GemmArgs &product_of(const GemmGroup &gg, int &tile) {
     const int s = __builtin_amdgcn_readfirstlane(gg.member(tile));
@@ -152,7 +161,8 @@ __device__ __forceinline__ void store_tile(const GemmArgs &g, const v16f &acc, i
 template <bool OUT_BF16, int TNS>
 constexpr int staged_epilogue_bytes() { return 32 * (TNS * 32 * (OUT_BF16 ? 2 : 4) + 16); }
 
-template <bool OUT_BF16, int TM, int TN, int TNS, bool RAGGED = false>
+// SCALED: the accumulators hold the values themselves.
+template <bool OUT_BF16, int TM, int TN, int TNS, bool RAGGED = false, bool SCALED = false>
 __device__ __forceinline__ void epilogue_staged(const GemmArgs &g, v16f (&acc)[TM][TN], uint8_t *wave_lds,
                                                 int64_t m_wave, int64_t n_wave, int lane) {
     static_assert(TN % TNS == 0, "slab width must divide the wave tile");
@@ -161,8 +171,8 @@ __device__ __forceinline__ void epilogue_staged(const GemmArgs &g, v16f (&acc)[T
     constexpr int LPR = ROW_BYTES / 16;            // lanes that cover one slab row with 16 bytes each
     constexpr int RPI = 64 / LPR;                  // rows per store instruction
     const int lr = lane % 32, lg = lane / 32;
-    const bool vec = g.sa_vec | g.sb_vec | (g.bias != nullptr);
-    const float s_tensor = g.sa[0] * g.sb[0];
+    const bool vec = !SCALED && (g.sa_vec | g.sb_vec | (g.bias != nullptr));
+    const float s_tensor = SCALED ? 1.0f : g.sa[0] * g.sb[0];
     const float *bias = reinterpret_cast<const float *>(g.bias);
     uint8_t *out = reinterpret_cast<uint8_t *>(g.c);
     const int rows = RAGGED ? (int)min(g.M - m_wave, (int64_t)(32 * TM)) : 32 * TM;          // of this wave tile
@@ -363,6 +373,7 @@ bool gemm_stream_accepts_pairs(const GemmArgs &g, const GemmPairs &pairs);
 bool gemm_stream_accepts_group(const GemmArgs &g);
 void launch_gemm_stream_group(int fa, int fb, const GemmGroup &gg, int num_cus, hipStream_t stream);
 void launch_gemm_deep_group(int bm, int bn, int fa, int fb, const GemmGroup &gg, int num_cus, hipStream_t stream);
+void launch_gemm_deep_chain(int bm, int bn, int fa, int fb, const GemmChain &gc, int num_cus, hipStream_t stream);
 void launch_gemm_tiled_group(int fa, int fb, const GemmGroup &gg, hipStream_t stream);
 void launch_gemm_stream_pairs(int fa, int fb, const GemmArgs &g, const GemmPairs &pairs, int num_cus, hipStream_t stream);
 // gemm_fp8.hip: hands the calling thread's clock-probe record (odl_fp8_gemm_set_clock_probe), if any, to a streaming launch

@@ -40,6 +40,8 @@ decltype(&odl_fp8_cast_rowcol_padded) cast_rowcol_c;
 decltype(&odl_fp8_gemm_nt_hinted) gemm_nt_c;
 decltype(&odl_fp8_gemm_group_route) group_route_c;
 decltype(&odl_fp8_gemm_nt_group) gemm_nt_group_c;
+decltype(&odl_fp8_gemm_chain_route) chain_route_c;
+decltype(&odl_fp8_gemm_nt_chain) gemm_nt_chain_c;
 decltype(&odl_fp8_gemm_layouts) gemm_layouts_c;
 decltype(&odl_fp8_gemm_runs) runs_c;
 decltype(&odl_fp8_mx_cast_padded) mx_cast_c;
@@ -69,6 +71,8 @@ void bind(const py::dict &d) {
     take(gemm_nt_c, d, "odl_fp8_gemm_nt_hinted");
     take(group_route_c, d, "odl_fp8_gemm_group_route");
     take(gemm_nt_group_c, d, "odl_fp8_gemm_nt_group");
+    take(chain_route_c, d, "odl_fp8_gemm_chain_route");
+    take(gemm_nt_chain_c, d, "odl_fp8_gemm_nt_chain");
     take(gemm_layouts_c, d, "odl_fp8_gemm_layouts");
     take(runs_c, d, "odl_fp8_gemm_runs");
     take(mx_cast_c, d, "odl_fp8_mx_cast_padded");
@@ -319,6 +323,37 @@ py::object gemm_nt_group(const std::vector<Tensor> &a, const std::vector<Tensor>
     return rc ? status(rc) : py::object(out);
 }
 
+bool chain_in_one_launch(const std::vector<i64> &K, i64 M, i64 N, bool block_scales) {
+    return K.size() <= 4 && chain_route_c((int)K.size(), K.data(), M, N, block_scales) >= 0;
+}
+
+// K-step-major scale bytes of codes [rows, K]
+bool kstep_scales(const Tensor &s, const Tensor &codes) {
+    return dense(s) && s.scalar_type() == at::kByte && s.dim() == 3 && s.size(0) * 128 == codes.size(1) && s.size(1) == codes.size(0) && s.size(2) == 4;
+}
+
+// The bf16 sum of several products in one launch
+py::object gemm_nt_chain(const std::vector<Tensor> &a, const std::vector<Tensor> &b, int fa, int fb, const std::vector<Tensor> &sa,
+                         const std::vector<Tensor> &sb, bool block_scales, i64 stream) {
+    const size_t n = a.size();
+    if (n < 2 || n > 4 || b.size() != n || sa.size() != n || sb.size() != n) return none();
+    const uint8_t *pa[4], *pb[4], *pma[4], *pmb[4];
+    const float *psa[4], *psb[4];
+    i64 K[4];
+    for (size_t s = 0; s < n; ++s) {
+        if (!codes2d(a[s]) || !codes2d(b[s]) || a[s].size(0) != a[0].size(0) || b[s].size(0) != b[0].size(0) || a[s].size(1) != b[s].size(1)) return none();
+        if (block_scales ? !kstep_scales(sa[s], a[s]) || !kstep_scales(sb[s], b[s]) : !floats(sa[s], 1) || !floats(sb[s], 1)) return none();
+        K[s] = a[s].size(1);
+        pa[s] = ptr(a[s]); pb[s] = ptr(b[s]);
+        if (block_scales) { pma[s] = ptr(sa[s]); pmb[s] = ptr(sb[s]); }
+        else { psa[s] = ptr(sa[s]); psb[s] = ptr(sb[s]); }
+    }
+    Tensor c = result(OptTensor(), a[0], a[0].size(0), b[0].size(0), 0);
+    const int rc = call(gemm_nt_chain_c, (int)n, pa, pb, K, a[0].size(0), b[0].size(0), fa, fb, psa, psb, block_scales ? pma : nullptr,
+                        block_scales ? pmb : nullptr, ptr(c), str(stream));
+    return rc ? status(rc) : py::cast(c);
+}
+
 // Not accumulating; whole tiles of the kernel that reads K-slow operands (the caller has checked: gemm_layouts_supported)
 py::object gemm_layouts(const Tensor &a, const Tensor &b, int fa, int fb, bool a_slow, bool b_slow, const Tensor &sa, const Tensor &sb,
                         const OptTensor &out, int odt, bool split, i64 stream) {
@@ -398,6 +433,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("gemm_nt", &gemm_nt);
     m.def("group_in_one_launch", &group_in_one_launch);
     m.def("gemm_nt_group", &gemm_nt_group);
+    m.def("chain_in_one_launch", &chain_in_one_launch);
+    m.def("gemm_nt_chain", &gemm_nt_chain);
     m.def("gemm_layouts", &gemm_layouts);
     m.def("mx_cast", &mx_cast);
     m.def("block_cast", &block_cast);

@@ -334,7 +334,10 @@ class _Fp8LinearFn(torch.autograd.Function):
             if ctx.need_dgrad or fp8_wgrad:
                 # one pass over dy: blocks along the output features for dgrad, along the tokens (transposed) for wgrad
                 gq, gs, gq_t, gs_t = given or _block_cast(pol, dy2d, pol.fmt_bwd, ctx.need_dgrad, fp8_wgrad)
-            if ctx.need_dgrad:
+            dx_pairs = getattr(ctx, "dx_pairs", None)
+            if ctx.need_dgrad and dx_pairs is not None:
+                dx_pairs.append((gq, saved["wq_t"], gs, saved["ws_t"]))
+            elif ctx.need_dgrad:
                 dx = native.mx_gemm_nt(gq, gs, saved["wq_t"], saved["ws_t"], pol.fmt_bwd, pol.fmt_fwd, out_dtype=ctx.x_dtype)
             if fp8_wgrad:
                 dw = native.mx_gemm_nt(gq_t, gs_t, saved["xq_t"], saved["xs_t"], pol.fmt_bwd, pol.fmt_fwd, out_dtype=ctx.w_dtype)
@@ -536,23 +539,30 @@ class _Fp8LinearGroupFn(torch.autograd.Function):
         return picked, torch.empty((rows, tokens), dtype=torch.uint8, device=xq_t.device), xq_t, sx_inv_t
 
     @staticmethod
-    def _dgrad_in_one_gemm(ctx, dys) -> "list | None":
+    def _dgrad_in_one_gemm(ctx, dys) -> "tuple[list, Any] | tuple[None, None]":
         """An empty list for the members to put their dgrad operands in (codes of dy, codes of W^T, the two inverse
-        scales) where ONE GEMM computes dx = sum over members of dy_s . W_s (``native.gemm_nt_sum``), else None: the
-        members then add into dx one by one.  One launch where per-tensor scales and the shapes allow: the k and v
-        shares of a grouped-query block (contractions of 1024) are, added into a cold 64 MB dx, bound by reading and
+        scales) and the call that makes dx = sum over members of dy_s . W_s of them in ONE launch, where there is one; else
+        (None, None): the members then add into dx one by one.  ``native.gemm_nt_sum`` (one rounding) where the shapes allow: the k
+        and v shares of a grouped-query block (contractions of 1024) are, added into a cold 64 MB dx, bound by reading and
         writing it (63 us each at 8192 tokens against 40 for the bare product); carried through one set of
-        accumulators they cost what their share of the contraction costs."""
+        accumulators they cost what their share of the contraction costs.  ``native.gemm_nt_chain`` where that is faster than
+        adding one by one, with the bits of it; under block scales, too, where a sum of the results is the other way."""
         recipe = ctx.subs[0].recipe
-        if not getattr(recipe, "fuse_dgrad_gemm", True) or recipe.recipe.kind not in ("tensorwise", "delayed"):
-            return None
+        kind = recipe.recipe.kind
+        if not recipe.fuse_dgrad_gemm or kind == "rowwise":
+            return None, None
         live = [sub for sub, dy in zip(ctx.subs, dys) if dy is not None and sub.need_dgrad]
         if len(live) < 2 or any(dy is not None and not sub.need_dgrad for sub, dy in zip(ctx.subs, dys)):
-            return None
+            return None, None
         tokens = next(dy for dy in dys if dy is not None).shape[0]
-        if not native.dgrad_sum_in_one_launch(tokens, live[0].module.in_features, [sub.module.out_features for sub in live]):
-            return None
-        return []
+        n_in, n_outs, dtype = live[0].module.in_features, [sub.module.out_features for sub in live], live[0].x_dtype
+        fmts = recipe.recipe.fmt_bwd, recipe.recipe.fmt_fwd
+        if kind in ("tensorwise", "delayed") and native.dgrad_sum_in_one_launch(tokens, n_in, n_outs):
+            return [], lambda a, b, sa, sb: native.gemm_nt_sum(a, b, *fmts, sa, sb, out_dtype=dtype)
+        block_scales = kind in ("mxfp8", "blockwise")
+        if dtype == torch.bfloat16 and native.gemm_chain_in_one_launch(n_outs, tokens, n_in, block_scales):
+            return [], lambda a, b, sa, sb: native.gemm_nt_chain(a, b, *fmts, sa, sb, block_scales)
+        return None, None
 
     @staticmethod
     def backward(ctx, *dys: torch.Tensor | None):
@@ -568,7 +578,7 @@ class _Fp8LinearGroupFn(torch.autograd.Function):
                 n = ctx.subs[i].module.out_features
                 ctx.subs[i].wgrad_joint = {"codes_t": joint[1][at:at + n], "rows": (at, at + n)}
                 at += n
-        dx_pairs = _Fp8LinearGroupFn._dgrad_in_one_gemm(ctx, dys)
+        dx_pairs, dx_of = _Fp8LinearGroupFn._dgrad_in_one_gemm(ctx, dys)
         for sub, (first, count), dy in zip(ctx.subs, ctx.spans, dys):
             if dy is None:                       # this member's output did not reach the loss
                 grads += [None, None]
@@ -586,10 +596,7 @@ class _Fp8LinearGroupFn(torch.autograd.Function):
                 dx = dxi
             grads += [dw, db]
         if dx_pairs:
-            pol = ctx.subs[0].recipe.recipe
-            gqs, wq_ts, sg_invs, sw_invs = zip(*dx_pairs)
-            dx = native.gemm_nt_sum(list(gqs), list(wq_ts), pol.fmt_bwd, pol.fmt_fwd, list(sg_invs), list(sw_invs),
-                                    out_dtype=ctx.subs[0].x_dtype)
+            dx = dx_of(*map(list, zip(*dx_pairs)))
         if dw_jobs:
             pol = ctx.subs[0].recipe.recipe
             for at, dw in zip(waiting, _run_jobs(dw_jobs, pol.fmt_bwd, pol.fmt_fwd, ctx.subs[0].w_dtype), strict=True):

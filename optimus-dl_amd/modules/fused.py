@@ -133,7 +133,7 @@ class _SwiGLUMLPFn(torch.autograd.Function):
         else:                                # put into eval mode since the forward: their histories are left alone
             given = None
         dgate, dup = (gate, up) if given is not None else native.swiglu_bwd_amax_parts(dh, gate, up)[:2]
-        pairs = _Fp8LinearGroupFn._dgrad_in_one_gemm(ctx, (dgate, dup))
+        pairs, dx_of = _Fp8LinearGroupFn._dgrad_in_one_gemm(ctx, (dgate, dup))
         dx, grads = None, []
         dw_jobs = _wgrad_jobs((sub_g, sub_u), (dgate, dup))
         for i, (sub, g) in enumerate(zip((sub_g, sub_u), (dgate, dup))):
@@ -151,8 +151,7 @@ class _SwiGLUMLPFn(torch.autograd.Function):
         if dw_jobs:
             grads = _run_jobs(dw_jobs, pol.fmt_bwd, pol.fmt_fwd, sub_g.w_dtype)
         if pairs:
-            gqs, wq_ts, sg_invs, sw_invs = zip(*pairs)
-            dx = native.gemm_nt_sum(list(gqs), list(wq_ts), pol.fmt_bwd, pol.fmt_fwd, list(sg_invs), list(sw_invs), out_dtype=sub_g.x_dtype)
+            dx = dx_of(*map(list, zip(*pairs)))
         for sub in ctx.subs:
             sub.saved_tensors = ()
         return dx, None, None, *grads, dw_d

@@ -74,6 +74,8 @@ EXPORTS = (
     "odl_fp8_gemm_nt_sum",
     "odl_fp8_gemm_group_route",
     "odl_fp8_gemm_nt_group",
+    "odl_fp8_gemm_chain_route",
+    "odl_fp8_gemm_nt_chain",
     "odl_fp8_gemm_layouts",
     "odl_fp8_gemm_split_count",
     "odl_fp8_gemm_runs",
@@ -166,6 +168,8 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_cast_delayed.argtypes = [vp, i32, i64, i64, vp, i32, vp, vp, vp, vp, vp]
         L.odl_fp8_gemm_nt.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, i64, vp, i64, vp, i32, vp, i32, i32, vp]
         L.odl_fp8_gemm_nt_hinted.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, i64, vp, i64, vp, i32, vp, i32, i32, i32, vp]
+        L.odl_fp8_gemm_chain_route.argtypes = [i32, vp, i64, i64, i32]
+        L.odl_fp8_gemm_nt_chain.argtypes = [i32, vp, vp, vp, i64, i64, i32, i32, vp, vp, vp, vp, vp, vp]
         L.odl_fp8_gemm_group_route.argtypes = [i32, vp, vp, i64, i32]
         L.odl_fp8_gemm_nt_group.argtypes = [i32, vp, vp, vp, vp, i64, i32, i32, vp, vp, vp, i32, i32, vp]
         L.odl_fp8_gemm_nt_sum.argtypes = [i32, vp, vp, vp, i64, i64, i32, i32, vp, vp, vp, i32, vp]
@@ -1001,6 +1005,26 @@ def gemm_nt_sum(a: "list[torch.Tensor]", b: "list[torch.Tensor]", fmt_a: int, fm
                                       ptrs(*[t.data_ptr() for t in sa_inv]), ptrs(*[t.data_ptr() for t in sb_inv]), out.data_ptr(),
                                       odt, _stream()), "odl_fp8_gemm_nt_sum")
     return out
+
+
+def gemm_chain_in_one_launch(Ks: "list[int]", M: int, N: int, block_scales: bool = False) -> bool:
+    """Whether :func:`gemm_nt_chain` takes products of these sizes."""
+    load()
+    return bool(_host.chain_in_one_launch(Ks, M, N, block_scales))
+
+
+def gemm_nt_chain(a: "list[torch.Tensor]", b: "list[torch.Tensor]", fmt_a: int, fmt_b: int, sa: "list[torch.Tensor]",
+                  sb: "list[torch.Tensor]", block_scales: bool = False) -> torch.Tensor:
+    """The bf16 sum of the products a[s] . b[s]^T in one launch: with one scale per operand what :func:`gemm_nt` and, for the second
+    and later ones, ``accumulate`` give; with block scales (K-step-major) rounded once.  Only where
+    :func:`gemm_chain_in_one_launch` says so."""
+    load()
+    if block_scales:
+        init_device(a[0].device)
+    r = _host.gemm_nt_chain(a, b, fmt_a, fmt_b, sa, sb, block_scales, _stream())
+    if r is None:
+        raise NativeError(f"gemm_nt_chain: operands {[tuple(t.shape) for t in (*a, *b)]} or their scales do not fit, are not dense or not aligned")
+    return _done(r, "odl_fp8_gemm_nt_chain")
 
 
 def gemm_group_in_one_launch(Ms: "list[int]", Ns: "list[int]", K: int, out_dtype: torch.dtype) -> bool:
