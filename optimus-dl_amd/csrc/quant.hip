@@ -899,9 +899,10 @@ __global__ __launch_bounds__(kThreads) void cast_transpose_kernel(const void *__
 }
 
 // ------------------------------------------------- current scaling of a small tensor, one launch
-// amax, scale and cast by one block that holds the tensor in registers in between: 16 pieces of 16 bytes a lane at most.  Bound
-// by what one compute unit reads, some 60 GB/s; it spares a launch (32 x 4096 bf16: 3.5 + 4.4 us and a launch of 4 us, here
-// 9.0).  Whole pieces, x and out 16-byte aligned.
+// amax, scale and cast by blocks that each read the whole tensor (16 pieces of 16 bytes a lane at most), find the same maximum, and
+// cast one piece per lane each.  Bound by what one compute unit reads, 60 - 70 bytes a nanosecond; nobody waits for another block, and
+// it spares a launch (32 x 4096 bf16: 3.5 + 4.4 us and a launch of 4 us; one block that casts everything 9.0, of which the
+// conversions were 5; here 7.0).  Whole pieces, x and out 16-byte aligned, not the same memory.
 constexpr int kSmallPieces = ODL_FP8_SMALL_BYTES / 16 / kFatThreads;
 template <int SRC, int FMT>
 __global__ __launch_bounds__(kFatThreads) void quantise_small_kernel(const void *__restrict__ x, int pieces, int margin, uint8_t *__restrict__ out,
@@ -909,7 +910,7 @@ __global__ __launch_bounds__(kFatThreads) void quantise_small_kernel(const void 
     __shared__ uint32_t red[kFatThreads / kWave];
     __shared__ float scale;
     const u32x4 *src = reinterpret_cast<const u32x4 *>(x);
-    u32x4 v[kSmallPieces];
+    u32x4 v[kSmallPieces], own = {0, 0, 0, 0};
 #pragma unroll
     for (int j = 0; j < kSmallPieces; ++j) {
         const int i = j * kFatThreads + (int)threadIdx.x;
@@ -918,6 +919,7 @@ __global__ __launch_bounds__(kFatThreads) void quantise_small_kernel(const void 
     uint32_t am = 0;
 #pragma unroll
     for (int j = 0; j < kSmallPieces; ++j) {
+        if (j == (int)blockIdx.x) own = v[j];
         const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -929,23 +931,22 @@ __global__ __launch_bounds__(kFatThreads) void quantise_small_kernel(const void 
     am = block_max_u32(am, red);
     if (threadIdx.x == 0) {
         const float amax = bits_to_float(am), s = scale_rule(amax, Fp8Lim<FMT>::max, margin, 1.0f);
-        dyn_out[0] = amax;
-        dyn_out[1] = s;
-        dyn_out[2] = __fdiv_rn(1.0f, s);
+        if (blockIdx.x == 0) {
+            dyn_out[0] = amax;
+            dyn_out[1] = s;
+            dyn_out[2] = __fdiv_rn(1.0f, s);
+        }
         scale = s;
     }
     __syncthreads();
     const float s = scale;
-#pragma unroll
-    for (int j = 0; j < kSmallPieces; ++j) {
-        const int i = j * kFatThreads + (int)threadIdx.x;
-        if (i >= pieces) break;
-        const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
-        if constexpr (SRC == ODL_BF16)
-            reinterpret_cast<u32x2 *>(out)[i] = u32x2{quantise4<FMT>(bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1]), s, s, s, s),
-                                                      quantise4<FMT>(bf16_lo(w[2]), bf16_hi(w[2]), bf16_lo(w[3]), bf16_hi(w[3]), s, s, s, s)};
-        else reinterpret_cast<uint32_t *>(out)[i] = quantise4<FMT>(bits_to_float(w[0]), bits_to_float(w[1]), bits_to_float(w[2]), bits_to_float(w[3]), s, s, s, s);
-    }
+    const int i = (int)blockIdx.x * kFatThreads + (int)threadIdx.x;
+    if (i >= pieces) return;
+    const uint32_t w[4] = {own.x, own.y, own.z, own.w};
+    if constexpr (SRC == ODL_BF16)
+        reinterpret_cast<u32x2 *>(out)[i] = u32x2{quantise4<FMT>(bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1]), s, s, s, s),
+                                                  quantise4<FMT>(bf16_lo(w[2]), bf16_hi(w[2]), bf16_lo(w[3]), bf16_hi(w[3]), s, s, s, s)};
+    else reinterpret_cast<uint32_t *>(out)[i] = quantise4<FMT>(bits_to_float(w[0]), bits_to_float(w[1]), bits_to_float(w[2]), bits_to_float(w[3]), s, s, s, s);
 }
 
 // ----------------------------------------------------------------- host helpers
@@ -1347,7 +1348,8 @@ extern "C" int odl_fp8_quantise_small(const void *x, int src_dtype, int64_t n, i
     if (margin < -64 || margin > 64) return set_error(ODL_ERR_ARG, "odl_fp8_quantise_small: margin %d", margin);
     if (!dyn_out || (n > 0 && (!x || !out))) return set_error(ODL_ERR_ARG, "odl_fp8_quantise_small: null pointer");
     if (!aligned16(x) || !aligned16(out)) return set_error(ODL_ERR_SHAPE, "odl_fp8_quantise_small: x and out must be 16-byte aligned");
-#define ODL_SMALL(S, F) hipLaunchKernelGGL((quantise_small_kernel<S, F>), dim3(1), dim3(kFatThreads), 0, stream, x, (int)(n * esz / 16), margin, out, dyn_out)
+    const int pieces = (int)(n * esz / 16), blocks = pieces > 0 ? (pieces + kFatThreads - 1) / kFatThreads : 1;
+#define ODL_SMALL(S, F) hipLaunchKernelGGL((quantise_small_kernel<S, F>), dim3((unsigned)blocks), dim3(kFatThreads), 0, stream, x, pieces, margin, out, dyn_out)
     if (src_dtype == ODL_BF16) { if (fmt == ODL_FP8_E4M3) ODL_SMALL(ODL_BF16, ODL_FP8_E4M3); else ODL_SMALL(ODL_BF16, ODL_FP8_E5M2); }
     else { if (fmt == ODL_FP8_E4M3) ODL_SMALL(ODL_F32, ODL_FP8_E4M3); else ODL_SMALL(ODL_F32, ODL_FP8_E5M2); }
 #undef ODL_SMALL

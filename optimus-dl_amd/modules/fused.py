@@ -205,7 +205,7 @@ def swiglu_mlp(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
 def swiglu_few_rows(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
     """``silu(w1 x) * w2 x`` of a decode step in one launch (``native.gemm_swiglu``), or None: only per-tensor current scaling,
     no graph, few rows (``native.gemm_swiglu_pays``), no biases, no hooks.  The value of the separate modules; to the last bit where
-    ``w1.in_features`` is 2048 or more (``native.gemm_swiglu``)."""
+    their products take the thin kernel (``native.gemm_swiglu``)."""
     recipe = _state.active_recipe()
     if recipe is None or recipe.recipe.kind != "tensorwise" or not no_graph() or _any_global_hook is None or _any_global_hook():
         return None

@@ -1048,24 +1048,20 @@ def gemm_nt_group(a: "list[torch.Tensor]", b: "list[torch.Tensor]", fmt_a: int, 
 
 
 def gemm_swiglu_pays(M: int, N: int, K: int) -> bool:
-    """Whether :func:`gemm_swiglu` takes a shape and is faster than two :func:`gemm_nt` and the SwiGLU kernel.  A block owns 16
-    columns and, from 33 rows on, has a compute unit to itself: rounds of blocks cost it more than they cost the separate
-    products.  Up to 32 rows four rounds (N <= 16384): 1.1 to 3.9 times as fast over K = 256 .. 8192 (N = 28672 0.8 to 1.2, 50304 0.6 to
-    1.0).  Up to 64 rows one round, below K = 2048 (where separate products run the kernel of few rows, too): 1.3 to 1.7
-    times as fast, where two rounds are 0.6 to 0.9, 14336 columns 0.4 to 0.7, and K = 2048 .. 8192 in one round 0.9 to 1.2.  us,
-    one launch / three, cold weights: 32 x 1024 -> 3072 6.0 / 18.3, 32 x 4096 -> 14336 37.2 / 44.8, 64 x 1024 -> 3072 11.5 / 18.8, 64 x
-    2048 -> 5632 33.0 / 22.7, 64 x 4096 -> 14336 79.4 / 49.4."""
+    """Whether :func:`gemm_swiglu` takes a shape and is faster than two :func:`gemm_nt` and the SwiGLU kernel.  us, one launch /
+    three, weights from memory: 32 rows 1024 -> 3072 4.9 / 18.4, 4096 -> 14336 28 / 40, 4096 -> 28672 48 / 67, but 1024 -> 50304 30 /
+    33; 64 rows 1024 -> 3072 5.6 / 18.9, 512 -> 8192 6.8 / 15.7, 4096 -> 16384 32 / 45, but 4096 -> 28672 62 / 70 and 1024 -> 28672 25 / 25.
+    From 33 rows on, contractions of less than 512 only up to 4096 columns, as far as they were measured first."""
     if not (0 < M <= 64 and N > 0 and N % 4 == 0 and K > 0 and K % 128 == 0 and N * K < 2**32 and M * K < 2**32):
         return False
-    columns = (N + 15) // 16
-    return columns <= 4 * 256 if M <= 32 else (columns <= 256 and K < 2048)
+    return N <= 28672 if M <= 32 else N <= 4096 or (K >= 512 and N <= 16384)
 
 
 def gemm_swiglu(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, fmt_x: int, fmt_w: int, sx_inv: torch.Tensor, sg_inv: torch.Tensor,
                 su_inv: torch.Tensor):
     """h = silu(x . gate^T) * (x . up^T) in bf16 for at most 64 rows (the roundings of two products and :func:`swiglu_amax_parts`),
     in one launch; x, gate, up uint8 FP8 codes [M, K], [N, K], [N, K] with one inverse scale each.  The products add up as the thin
-    kernel of :func:`gemm_nt` adds them: its bits from K = 2048 on, where it is chosen; below that the last places differ.
+    kernel of :func:`gemm_nt` adds them: its bits where that is chosen (K >= 2048, few rows); elsewhere the last places differ.
     -> (h, partial maxima of |h|)."""
     if x.is_cuda:
         load()
