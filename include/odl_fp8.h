@@ -46,7 +46,7 @@ enum odl_status {
 };
 
 /* ABI version of this header; bumped when a signature changes or an entry point is added. */
-#define ODL_FP8_ABI_VERSION 26
+#define ODL_FP8_ABI_VERSION 27
 int odl_fp8_abi_version(void);
 
 /*
@@ -479,6 +479,14 @@ int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t M, int64_t 
  * with an operand stored K-slow (a weight gradient that reads dY as stored) is added into C.
  * No counterpart in the reference, whose GEMMs are cuBLASLt's choice inside te.pytorch.Linear.
  */
+/*
+ * A weight gradient of that kind whose rows are no whole tiles (a vocabulary of 50304): dW [n_out, n_in] = dY^T . X from the codes of
+ * dY [tokens, n_out] as stored and of X^T [n_in, tokens].  n_out >= 256 and a multiple of 16, n_in and tokens of 128, tokens >= 512, everything
+ * 16-byte aligned and each operand under 2 GiB; the rest as for odl_fp8_gemm_layouts with layout_a = ODL_K_SLOW, layout_b = ODL_K_FAST.
+ */
+int odl_fp8_gemm_wgrad(const uint8_t *gy, const uint8_t *x_t, int64_t n_out, int64_t n_in, int64_t tokens, int fmt_g, int fmt_x,
+                       const float *sg_inv, const float *sx_inv, void *dw, int out_dtype, odl_stream_t stream);
+
 int odl_fp8_gemm_split_count(int64_t M, int64_t N, int64_t K, int k_slow);
 /*
  * The runs worth a workspace: odl_fp8_gemm_split_count, but 1 where one launch of odl_fp8_gemm_nt (or odl_fp8_mx_gemm_nt) in 128 x 192

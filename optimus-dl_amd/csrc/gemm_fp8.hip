@@ -419,18 +419,17 @@ extern "C" int odl_fp8_gemm_nt_sum(int pairs, const uint8_t *const *a, const uin
     return ODL_OK;
 }
 
-extern "C" int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b,
-                                    int layout_a, int layout_b, const float *sa_inv, const float *sb_inv, void *c,
-                                    int out_dtype, odl_stream_t stream_) {
-    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
-    if (!a || !b || !c || !sa_inv || !sb_inv) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_layouts: null pointer");
+// the launch of odl_fp8_gemm_layouts and odl_fp8_gemm_wgrad; `who` names the entry, `partial`: A need not be whole tiles
+static int gemm_as_stored(const char *who, const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b, int layout_a,
+                          int layout_b, const float *sa_inv, const float *sb_inv, void *c, int out_dtype, bool partial, hipStream_t stream) {
+    if (!a || !b || !c || !sa_inv || !sb_inv) return set_error(ODL_ERR_ARG, "%s: null pointer", who);
     if ((fmt_a != ODL_FP8_E4M3 && fmt_a != ODL_FP8_E5M2) || (fmt_b != ODL_FP8_E4M3 && fmt_b != ODL_FP8_E5M2))
-        return set_error(ODL_ERR_ARG, "odl_fp8_gemm_layouts: formats %d, %d", fmt_a, fmt_b);
+        return set_error(ODL_ERR_ARG, "%s: formats %d, %d", who, fmt_a, fmt_b);
     if ((layout_a != ODL_K_FAST && layout_a != ODL_K_SLOW) || (layout_b != ODL_K_FAST && layout_b != ODL_K_SLOW))
-        return set_error(ODL_ERR_ARG, "odl_fp8_gemm_layouts: layouts %d, %d", layout_a, layout_b);
-    if (out_dtype != ODL_BF16 && out_dtype != ODL_F32) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_layouts: out_dtype %d", out_dtype);
+        return set_error(ODL_ERR_ARG, "%s: layouts %d, %d", who, layout_a, layout_b);
+    if (out_dtype != ODL_BF16 && out_dtype != ODL_F32) return set_error(ODL_ERR_ARG, "%s: out_dtype %d", who, out_dtype);
     if ((reinterpret_cast<uintptr_t>(a) & 15) || (reinterpret_cast<uintptr_t>(b) & 15) || (reinterpret_cast<uintptr_t>(c) & 15))
-        return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_layouts: operands and output must be 16-byte aligned");
+        return set_error(ODL_ERR_SHAPE, "%s: operands and output must be 16-byte aligned", who);
     GemmArgs g;
     g.a = a; g.b = b; g.c = c; g.sa = sa_inv; g.sb = sb_inv; g.bias = nullptr;
     g.M = M; g.N = N; g.K = K;
@@ -438,14 +437,30 @@ extern "C" int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t 
     g.out_dtype = out_dtype;
     g.ta = layout_a == ODL_K_SLOW;
     g.tb = layout_b == ODL_K_SLOW;
-    const bool sizes_ok = M > 0 && N > 0 && K >= 512 && M % 256 == 0 && N % 256 == 0 && K % 128 == 0 &&
+    const int mult_m = partial ? 16 : 256, mult_n = partial ? 128 : 256;
+    const bool sizes_ok = M >= (partial ? 256 : 1) && N > 0 && K >= 512 && M % mult_m == 0 && N % mult_n == 0 && K % 128 == 0 &&
                           (double)(M + 256) * (double)K < 2147483648.0 && (double)(N + 256) * (double)K < 2147483648.0;
-    if (!sizes_ok) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_layouts: M, N must be multiples of 256, K of 128 (K >= 512) and each operand under 2 GiB; got %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
-    g.tiles_m = (int)(M / 256); g.tiles_n = (int)(N / 256);
-    if (!gemm_stream_accepts(g)) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_layouts: shape not taken by the streaming kernel");
+    if (!sizes_ok)
+        return set_error(ODL_ERR_SHAPE, "%s: M, N must be multiples of %s, K of 128 (K >= 512) and each operand under 2 GiB; got %lld x %lld x %lld",
+                         who, partial ? "16 (256 at least) and 128" : "256", (long long)M, (long long)N, (long long)K);
+    g.tiles_m = (int)((M + 255) / 256); g.tiles_n = (int)((N + 255) / 256);
+    if (!gemm_stream_accepts(g)) return set_error(ODL_ERR_SHAPE, "%s: shape not taken by the streaming kernel", who);
     attach_clock_probe(g);
     launch_gemm_stream(fmt_a, fmt_b, g, cu_count(), stream);
-    return check_launch("odl_fp8_gemm_layouts");
+    return check_launch(who);
+}
+
+extern "C" int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K, int fmt_a, int fmt_b,
+                                    int layout_a, int layout_b, const float *sa_inv, const float *sb_inv, void *c,
+                                    int out_dtype, odl_stream_t stream_) {
+    return gemm_as_stored("odl_fp8_gemm_layouts", a, b, M, N, K, fmt_a, fmt_b, layout_a, layout_b, sa_inv, sb_inv, c, out_dtype, false,
+                          reinterpret_cast<hipStream_t>(stream_));
+}
+
+extern "C" int odl_fp8_gemm_wgrad(const uint8_t *gy, const uint8_t *x_t, int64_t n_out, int64_t n_in, int64_t tokens, int fmt_g, int fmt_x,
+                                  const float *sg_inv, const float *sx_inv, void *dw, int out_dtype, odl_stream_t stream_) {
+    return gemm_as_stored("odl_fp8_gemm_wgrad", gy, x_t, n_out, n_in, tokens, fmt_g, fmt_x, ODL_K_SLOW, ODL_K_FAST, sg_inv, sx_inv, dw, out_dtype, true,
+                          reinterpret_cast<hipStream_t>(stream_));
 }
 
 // How many runs to cut K into for an output of few tiles (1 = do not split).  A model in microseconds, fitted to

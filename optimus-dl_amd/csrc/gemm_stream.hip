@@ -170,6 +170,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         const int group_rows = min(args_of(member).tiles_m - first_m, GM);
         // (integer division runs on the vector unit: readfirstlane states that the results are uniform)
         tm0 = __builtin_amdgcn_readfirstlane((first_m + (p % in_group) % group_rows) * BM);
+        if constexpr (TA) tm0 = min(tm0, (int)g.M - BM);          // a last tile that would be partial: see gemm_stream_accepts
         tn0 = __builtin_amdgcn_readfirstlane(((p % in_group) / group_rows) * BN);
     };
     // descriptor of an operand for the tile rows from row0 on and the K steps from first_step on
@@ -777,8 +778,10 @@ void launch_fmt(const GemmArgs &g, int blocks_per_xcd, hipStream_t stream) {
 }  // namespace
 
 // Shapes this kernel takes (the caller checks the 32-bit offset limits shared with gemm_pipe.hip).
-// An operand stored [K, rows] must fill whole tiles: the loads of a partial tile would run past the
-// end of its last K-row.  Stored [rows, K], A may end anywhere and B after half a tile (see wave_inside).
+// Stored [rows, K], A may end anywhere and B after half a tile (see wave_inside).  An operand stored [K, rows] must fill whole
+// tiles: the loads of a partial tile would run past the end of its last K-row, where no bound of a descriptor stops them (the scalar
+// offset that leads to a K step is not checked).  A with rows in whole 16-byte chunks does so by a last tile that begins BM rows before the
+// end: some rows are computed by two blocks, which store the same values.
 // Block scales are fetched for 128 rows at a time: behind the last row lie the next K step's, and what they scale is zero and
 // not stored.
 bool gemm_stream_accepts(const GemmArgs &g) {
@@ -786,7 +789,7 @@ bool gemm_stream_accepts(const GemmArgs &g) {
     const bool vectors = g.splits == 1 && (g.sa_vec || g.sb_vec || g.bias != nullptr);   // only with both operands stored [rows, K]
     if (g.mx_sa && (g.ta || g.tb || g.sa_vec || g.sb_vec || !g.mx_sb)) return false;
     return !g.accumulate && (g.out_dtype == ODL_BF16 || g.out_dtype == ODL_F32) && !(vectors && (g.ta || g.tb)) &&
-           g.M % (g.ta ? BM : 1) == 0 && g.N % (g.tb ? BN : WN) == 0 && g.K % 128 == 0 && g.K >= 512 && (double)g.N * esz * (BM + 8) < 2147483648.0;
+           g.M % (g.ta ? 16 : 1) == 0 && (!g.ta || g.M >= BM) && g.N % (g.tb ? BN : WN) == 0 && g.K % 128 == 0 && g.K >= 512 && (double)g.N * esz * (BM + 8) < 2147483648.0;
 }
 
 // Operand pairs: each a whole even number of K steps, four at least (the load pipeline is two steps deep and crosses

@@ -275,9 +275,10 @@ class _Fp8LinearFn(torch.autograd.Function):
             # accumulate, and the detour through a workspace costs what the fusion saves: measured 500 us against
             # 475 us unfused for a 14336 x 4096 fp32 gradient, where the transposed route with the flag takes 395)
             ctx.wgrad_direct = (fp8_wgrad and recipe.direct_layouts and not recipe.fuse_wgrad_accumulation
-                                and native.gemm_layouts_supported(n_out, n_in, tokens, weight.dtype)
-                                and (native.wgrad_direct_pays(n_out, n_in, tokens)
-                                     or (recipe.direct_layouts is True and n_out * n_in < 400_000)))
+                                and (native.gemm_layouts_supported(n_out, n_in, tokens, weight.dtype)
+                                     and (native.wgrad_direct_pays(n_out, n_in, tokens)
+                                          or (recipe.direct_layouts is True and n_out * n_in < 400_000))
+                                     or native.gemm_wgrad_pays(n_out, n_in, tokens, weight.dtype)))
             if pol.kind == "delayed":
                 # the histories see a forward only when it is part of training: the module in training mode AND
                 # grad mode on (the reference's backend refreshes its state on the same condition), so a validation
@@ -412,7 +413,10 @@ class _Fp8LinearFn(torch.autograd.Function):
                 grad_buf = module.weight.grad if recipe.fuse_wgrad_accumulation else None
                 into = grad_buf is not None and grad_buf.dtype == ctx.w_dtype and grad_buf.is_contiguous() and grad_buf.is_cuda \
                     and tuple(grad_buf.shape) == (module.out_features, module.in_features)
-                if ctx.wgrad_direct:        # dW = dY^T . X with dY [tokens, N] as stored, X^T from the forward
+                # wgrad_direct: dW = dY^T . X with dY [tokens, N] as stored, X^T from the forward
+                if ctx.wgrad_direct and module.out_features % 256:
+                    dw = native.gemm_wgrad(gq, saved["xq_t"], pol.fmt_bwd, pol.fmt_fwd, sg_inv, saved["sx_inv_t"], ctx.w_dtype)
+                elif ctx.wgrad_direct:
                     dw = native.gemm_layouts(gq, saved["xq_t"], pol.fmt_bwd, pol.fmt_fwd, native.K_SLOW, native.K_FAST,
                                              sg_inv, saved["sx_inv_t"], out=grad_buf if into else None,
                                              out_dtype=ctx.w_dtype, accumulate=into)

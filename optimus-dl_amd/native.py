@@ -26,7 +26,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 26
+ABI_VERSION = 27
 _OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
@@ -80,6 +80,7 @@ EXPORTS = (
     "odl_fp8_gemm_split_count",
     "odl_fp8_gemm_runs",
     "odl_fp8_gemm_splitk",
+    "odl_fp8_gemm_wgrad",
     "odl_fp8_delayed_update",
     "odl_fp8_gemm_num_variants",
     "odl_fp8_gemm_variant_name",
@@ -179,6 +180,7 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_gemm_runs.argtypes = [i64, i64, i64, i32]
         L.odl_fp8_gemm_runs.restype = i32
         L.odl_fp8_gemm_splitk.argtypes = [vp, vp, i64, i64, i64, i32, i32, i32, i32, vp, i64, vp, i64, vp, vp, i32, i32, i32, vp, i64, vp]
+        L.odl_fp8_gemm_wgrad.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, vp, vp, i32, vp]
         L.odl_fp8_delayed_update.argtypes = [vp, i64, i64, i64, vp, vp, vp, i32, i32, vp, vp]
         L.odl_fp8_gemm_num_variants.restype = i32
         L.odl_fp8_gemm_variant_name.argtypes = [i32]
@@ -1436,6 +1438,35 @@ def gemm_layouts(a: torch.Tensor, b: torch.Tensor, fmt_a: int, fmt_b: int, layou
     a, b = _as_2d(a), _as_2d(b)
     M, K = (a.shape[1], a.shape[0]) if layout_a == K_SLOW else a.shape
     N, K2 = (b.shape[1], b.shape[0]) if layout_b == K_SLOW else b.shape
+def gemm_wgrad_pays(n_out: int, n_in: int, tokens: int, out_dtype: torch.dtype = torch.bfloat16) -> bool:
+    """Whether :func:`gemm_wgrad` takes a weight gradient that :func:`gemm_layouts` does not (n_out no multiple of 256) and is faster
+    than the route over a transposed copy of dY: where its tiles fill the chip, as in :func:`wgrad_direct_pays`.  50304 x 768
+    fp32, product and cast of dY, this way / over the copy in us: 1024 tokens 88 / 99, 2048 142 / 159, 8192 589 / 704, 16384 1190 / 1417."""
+    return (n_out % 256 != 0 and n_out % 16 == 0 and n_in % 128 == 0 and tokens % 128 == 0 and tokens >= 512
+            and out_dtype in (torch.bfloat16, torch.float32) and -(-n_out // 256) * -(-n_in // 256) >= 192
+            and (n_out + 256) * tokens < 2**31 and (n_in + 256) * tokens < 2**31 and n_in * out_dtype.itemsize * 264 < 2**31)
+
+
+def gemm_wgrad(gy: torch.Tensor, x_t: torch.Tensor, fmt_g: int, fmt_x: int, sg_inv: torch.Tensor, sx_inv: torch.Tensor,
+               out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
+    """dW [n_out, n_in] = dY^T . X from the codes gy [tokens, n_out] of dY as stored and x_t [n_in, tokens] of X^T, as
+    :func:`gemm_layouts`, for any n_out >= 256 in multiples of 16 and n_in of 128."""
+    if gy.dtype != torch.uint8 or x_t.dtype != torch.uint8:
+        raise NativeError("gemm_wgrad operands must be uint8 FP8 codes")
+    gy, x_t = _as_2d(gy), _as_2d(x_t)
+    (tokens, n_out), (n_in, k) = gy.shape, x_t.shape
+    if k != tokens:
+        raise NativeError(f"gemm_wgrad: contraction sizes differ ({tokens} vs {k})")
+    if out_dtype not in _OUT_DTYPES:
+        raise NativeError(f"gemm_wgrad: {out_dtype} output")
+    _f32_dev(sg_inv, 1, "gemm_wgrad sg_inv")
+    _f32_dev(sx_inv, 1, "gemm_wgrad sx_inv")
+    dw = torch.empty((n_out, n_in), dtype=out_dtype, device=gy.device)
+    _check(load().odl_fp8_gemm_wgrad(gy.data_ptr(), x_t.data_ptr(), n_out, n_in, tokens, fmt_g, fmt_x, sg_inv.data_ptr(), sx_inv.data_ptr(),
+                                     dw.data_ptr(), _OUT_DTYPES[out_dtype], _stream()), "odl_fp8_gemm_wgrad")
+    return dw
+
+
     if K != K2:
         raise NativeError(f"gemm_layouts: contraction sizes differ ({K} vs {K2})")
     _f32_dev(sa_inv, 1, "gemm_layouts sa_inv")
