@@ -207,6 +207,17 @@ int odl_fp8_amax_parts_colsum(const void *x, int src_dtype, int64_t rows, int64_
                               float *colsum, float *workspace, odl_stream_t stream);
 
 /*
+ * The same in two halves around the cast that follows: odl_fp8_amax_parts_slabs leaves the partial maxima and, in the workspace, slabs
+ * of column sums; odl_fp8_cast_dynamic_colsum is odl_fp8_cast_dynamic_padded (both layouts; cols a multiple of 8, rows_out of 16, x and
+ * out_t 16-byte aligned) and adds the slabs up besides, to the sums of odl_fp8_amax_parts_colsum rounded to colsum_dtype
+ * (ODL_BF16 or ODL_F32).  src_dtype, rows and cols as in the first half.
+ */
+int odl_fp8_amax_parts_slabs(const void *x, int src_dtype, int64_t rows, int64_t cols, float *parts, float *workspace, odl_stream_t stream);
+int odl_fp8_cast_dynamic_colsum(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, const float *parts, int fmt,
+                                int margin, uint8_t *out, uint8_t *out_t, float *dyn_out, const float *workspace, void *colsum,
+                                int colsum_dtype, odl_stream_t stream);
+
+/*
  * The rowwise recipe needs every tensor twice: scaled per row for the GEMM that contracts
  * its columns, and scaled per column, transposed, for the GEMM that contracts its rows.
  *   odl_fp8_amax_rowcol: amax_row[rows] and amax_col[cols] in one pass over x;
@@ -313,6 +324,8 @@ int odl_fp8_layernorm_bwd(const void *dy, const void *x, int src_dtype, const fl
  *   odl_fp8_gelu_amax_parts     : y  = fwd[x];                  parts = partial maxima of |y|
  *   odl_fp8_gelu_bwd_amax_parts : dx = bf16( dy * bwd[x] );     parts = partial maxima of |dx|
  * rows * cols a multiple of 8, 16-byte aligned pointers.
+ *   odl_fp8_gelu_bwd_slabs      : the same, and the slabs of column sums of dx that odl_fp8_amax_parts_slabs(dx) leaves in its
+ *                                 workspace (cols a multiple of 8), for odl_fp8_cast_dynamic_colsum
  */
 #define ODL_FP8_GELU_TABLE_BYTES (65536 * 2 + 65536 * 4)
 int odl_fp8_gelu_table(void *table, odl_stream_t stream);
@@ -320,6 +333,8 @@ int odl_fp8_gelu_amax_parts(const void *x, int64_t rows, int64_t cols, const voi
                             float *parts, odl_stream_t stream);
 int odl_fp8_gelu_bwd_amax_parts(const void *dy, const void *x, int64_t rows, int64_t cols,
                                 const void *table, void *dx, float *parts, odl_stream_t stream);
+int odl_fp8_gelu_bwd_slabs(const void *dy, const void *x, int64_t rows, int64_t cols, const void *table, void *dx, float *parts,
+                           float *workspace, odl_stream_t stream);
 
 /*
  * out[r,c] = fp8( clamp( fp32(x[r,c]) * s , +-max ) ), s = scale[0] | scale[r] | scale[c].
@@ -465,6 +480,14 @@ int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t M, int64_t 
                          const float *sb_inv, void *c, int out_dtype, odl_stream_t stream);
 
 /*
+ * A weight gradient of that kind whose rows are no whole tiles (a vocabulary of 50304): dW [n_out, n_in] = dY^T . X from the codes of
+ * dY [tokens, n_out] as stored and of X^T [n_in, tokens].  n_out >= 256 and a multiple of 16, n_in and tokens of 128, tokens >= 512, everything
+ * 16-byte aligned and each operand under 2 GiB; the rest as for odl_fp8_gemm_layouts with layout_a = ODL_K_SLOW, layout_b = ODL_K_FAST.
+ */
+int odl_fp8_gemm_wgrad(const uint8_t *gy, const uint8_t *x_t, int64_t n_out, int64_t n_in, int64_t tokens, int fmt_g, int fmt_x,
+                       const float *sg_inv, const float *sx_inv, void *dw, int out_dtype, odl_stream_t stream);
+
+/*
  * The same product for an output of few 256 x 256 tiles and a long contraction (weight gradients of
  * small layers, the input gradient of a vocabulary-sized head): K is cut into `splits` runs that are
  * computed side by side as unscaled fp32 partial results in `workspace` ([splits, M, N] floats,
@@ -479,14 +502,6 @@ int odl_fp8_gemm_layouts(const uint8_t *a, const uint8_t *b, int64_t M, int64_t 
  * with an operand stored K-slow (a weight gradient that reads dY as stored) is added into C.
  * No counterpart in the reference, whose GEMMs are cuBLASLt's choice inside te.pytorch.Linear.
  */
-/*
- * A weight gradient of that kind whose rows are no whole tiles (a vocabulary of 50304): dW [n_out, n_in] = dY^T . X from the codes of
- * dY [tokens, n_out] as stored and of X^T [n_in, tokens].  n_out >= 256 and a multiple of 16, n_in and tokens of 128, tokens >= 512, everything
- * 16-byte aligned and each operand under 2 GiB; the rest as for odl_fp8_gemm_layouts with layout_a = ODL_K_SLOW, layout_b = ODL_K_FAST.
- */
-int odl_fp8_gemm_wgrad(const uint8_t *gy, const uint8_t *x_t, int64_t n_out, int64_t n_in, int64_t tokens, int fmt_g, int fmt_x,
-                       const float *sg_inv, const float *sx_inv, void *dw, int out_dtype, odl_stream_t stream);
-
 int odl_fp8_gemm_split_count(int64_t M, int64_t N, int64_t K, int k_slow);
 /*
  * The runs worth a workspace: odl_fp8_gemm_split_count, but 1 where one launch of odl_fp8_gemm_nt (or odl_fp8_mx_gemm_nt) in 128 x 192

@@ -167,4 +167,9 @@ __device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t *red) {
     return v;
 }
 
+// quant.hip: the cast of a gradient and the sum of its `nslab` slabs of column sums in one launch (both layouts; see there)
+bool cast_colsum_takes(const void *x, int64_t rows, int64_t cols, int64_t rows_out, const uint8_t *out, const uint8_t *out_t);
+void launch_cast_colsum(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, const float *parts, int fmt, int margin, uint8_t *out,
+                        uint8_t *out_t, float *dyn_out, const float *slabs, int nslab, void *colsum, int sum_dtype, hipStream_t stream);
+
 }  // namespace odl

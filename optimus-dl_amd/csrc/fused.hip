@@ -953,6 +953,64 @@ __global__ __launch_bounds__(kFusedThreads) void gelu_bwd_kernel(const u32x4 *__
         for (int j = (int)gridDim.x + threadIdx.x; j < kParts; j += kFusedThreads) parts[j] = 0.0f;
 }
 
+// The same for the gradient of a Linear with a bias: besides, the slabs of column sums of dx that amax_colsum_kernel would leave, in its
+// layout, order and bits, so that dx is not read again before its cast.  Blocks, rows and lanes as there.
+// 16384 x 3072: 60.4 us (5 TB/s; gelu_bwd_kernel 55.0 and that pass 19.0); 4096 x 3072: 21.3 (18.1 and 10.4); 512 x 3072: 7.4 (6.8 and 9.2).
+__global__ __launch_bounds__(kFusedThreads) void gelu_bwd_colsum_kernel(const uint16_t *__restrict__ dy, const uint16_t *__restrict__ x, int64_t rows,
+                                                                         int64_t cols, int rows_per_block, const float *__restrict__ bwd,
+                                                                         uint16_t *__restrict__ dx, float *__restrict__ parts,
+                                                                         float *__restrict__ slabs) {
+    constexpr int CW = 32 * 8;                    // columns per block
+    __shared__ float sums[32][CW + 1];
+    __shared__ uint32_t red[kFusedThreads / kWave];
+    __shared__ float win[2 * kGeluWin];
+    gelu_window_to_lds(bwd, win);
+    const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;
+    const int64_t c0 = (int64_t)blockIdx.x * CW + tx * 8;
+    const int64_t r0 = (int64_t)blockIdx.y * rows_per_block;
+    const int64_t r1 = r0 + rows_per_block < rows ? r0 + rows_per_block : rows;
+    float acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
+    uint32_t am = 0;
+    auto in = [&](const uint16_t *p, int64_t r) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p + r * cols + c0)); };
+    auto one = [&](const u32x4 v, const u32x4 d, int64_t r) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w}, dw[4] = {d.x, d.y, d.z, d.w};
+        uint32_t o[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            o[q] = pack2(__fmul_rn(bf16_lo(dw[q]), gelu_lookup(w[q] & 0xffffu, win, bwd)),
+                         __fmul_rn(bf16_hi(dw[q]), gelu_lookup(w[q] >> 16, win, bwd)));
+            am = max_u16x2(am, abs_bf16x2(o[q]));
+            acc[2 * q] = __fadd_rn(acc[2 * q], bf16_lo(o[q]));
+            acc[2 * q + 1] = __fadd_rn(acc[2 * q + 1], bf16_hi(o[q]));
+        }
+        *reinterpret_cast<u32x4 *>(dx + r * cols + c0) = u32x4{o[0], o[1], o[2], o[3]};
+    };
+    if (c0 + 8 <= cols) {                          // host guarantees cols % 8 == 0
+        int64_t r = r0 + ty;
+        for (; r + 32 < r1; r += 64) {
+            const u32x4 v0 = in(x, r), d0 = in(dy, r), v1 = in(x, r + 32), d1 = in(dy, r + 32);
+            one(v0, d0, r);
+            one(v1, d1, r + 32);
+        }
+        for (; r < r1; r += 32) one(in(x, r), in(dy, r), r);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sums[ty][tx * 8 + j] = acc[j];
+    am = block_max_u32(fold_u16x2_to_f32bits(am), red);        // has the barrier that also publishes sums[][]
+    for (int c = threadIdx.x; c < CW; c += kFusedThreads) {
+        float t = sums[0][c];
+#pragma unroll
+        for (int y = 1; y < 32; ++y) t = __fadd_rn(t, sums[y][c]);
+        const int64_t col = (int64_t)blockIdx.x * CW + c;
+        if (col < cols) slabs[(int64_t)blockIdx.y * cols + col] = t;
+    }
+    const int bid = blockIdx.y * gridDim.x + blockIdx.x, nblk = gridDim.x * gridDim.y;
+    if (threadIdx.x == 0) parts[bid] = bits_to_float(am);
+    if (bid == 0)
+        for (int j = nblk + threadIdx.x; j < kParts; j += kFusedThreads) parts[j] = 0.0f;
+}
 
 // at most two fat blocks per CU, and never more blocks than there are partial maxima
 static int grid_cap() {
@@ -1089,24 +1147,63 @@ extern "C" int odl_fp8_rmsnorm_bwd(const void *dy, const void *x, int src_dtype,
     return check_launch("odl_fp8_rmsnorm_bwd");
 }
 
-extern "C" int odl_fp8_amax_parts_colsum(const void *x, int src_dtype, int64_t rows, int64_t cols, float *parts, float *colsum,
-                                         float *workspace, odl_stream_t stream_) {
-    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
-    if (rows <= 0 || cols <= 0) return set_error(ODL_ERR_ARG, "odl_fp8_amax_parts_colsum: empty or negative shape");
-    if (!x || !parts || !colsum || !workspace) return set_error(ODL_ERR_ARG, "odl_fp8_amax_parts_colsum: null pointer");
-    if (src_dtype != ODL_BF16 && src_dtype != ODL_F32) return set_error(ODL_ERR_ARG, "odl_fp8_amax_parts_colsum: src_dtype %d", src_dtype);
+// rows of a slab of column sums, and how many slabs there are; one partial maximum per block of the pass
+static int64_t colsum_slab_rows(int src_dtype, int64_t rows, int64_t cols, int64_t *slabs_out) {
+    const int cw = 32 * (src_dtype == ODL_BF16 ? 8 : 4);
+    const int64_t slabs = kParts / ((cols + cw - 1) / cw);
+    int64_t rpb = (rows + slabs - 1) / slabs;
+    rpb = ((rpb + 31) / 32) * 32;
+    *slabs_out = (rows + rpb - 1) / rpb;
+    return rpb;
+}
+
+// the amax pass with column sums: partial maxima, and slabs of column sums in `workspace`
+static int amax_colsum_pass(const char *who, const void *x, int src_dtype, int64_t rows, int64_t cols, float *parts, float *workspace, hipStream_t stream) {
+    if (rows <= 0 || cols <= 0) return set_error(ODL_ERR_ARG, "%s: empty or negative shape", who);
+    if (!x || !parts || !workspace) return set_error(ODL_ERR_ARG, "%s: null pointer", who);
+    if (src_dtype != ODL_BF16 && src_dtype != ODL_F32) return set_error(ODL_ERR_ARG, "%s: src_dtype %d", who, src_dtype);
     const int cpl = src_dtype == ODL_BF16 ? 8 : 4, cw = 32 * cpl;
     const int64_t col_blocks = (cols + cw - 1) / cw;
     if (cols % cpl != 0 || !aligned16(x) || col_blocks > kParts)
-        return set_error(ODL_ERR_SHAPE, "odl_fp8_amax_parts_colsum: cols must be a multiple of %d and at most %d, x 16-byte aligned", cpl, kParts * cw);
-    int64_t slabs = kParts / col_blocks;                      // one partial maximum per block
-    int64_t rpb = (rows + slabs - 1) / slabs;
-    rpb = ((rpb + 31) / 32) * 32;
-    slabs = (rows + rpb - 1) / rpb;
+        return set_error(ODL_ERR_SHAPE, "%s: cols must be a multiple of %d and at most %d, x 16-byte aligned", who, cpl, kParts * cw);
+    int64_t slabs;
+    const int64_t rpb = colsum_slab_rows(src_dtype, rows, cols, &slabs);
     if (src_dtype == ODL_BF16) hipLaunchKernelGGL((amax_colsum_kernel<ODL_BF16>), dim3((unsigned)col_blocks, (unsigned)slabs), dim3(kFusedThreads), 0, stream, x, rows, cols, (int)rpb, parts, workspace);
     else hipLaunchKernelGGL((amax_colsum_kernel<ODL_F32>), dim3((unsigned)col_blocks, (unsigned)slabs), dim3(kFusedThreads), 0, stream, x, rows, cols, (int)rpb, parts, workspace);
+    return ODL_OK;
+}
+
+extern "C" int odl_fp8_amax_parts_colsum(const void *x, int src_dtype, int64_t rows, int64_t cols, float *parts, float *colsum,
+                                         float *workspace, odl_stream_t stream_) {
+    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+    if (!colsum) return set_error(ODL_ERR_ARG, "odl_fp8_amax_parts_colsum: null pointer");
+    if (const int rc = amax_colsum_pass("odl_fp8_amax_parts_colsum", x, src_dtype, rows, cols, parts, workspace, stream)) return rc;
+    int64_t slabs;
+    colsum_slab_rows(src_dtype, rows, cols, &slabs);
     launch_slab_reduce(workspace, (int)slabs, cols, colsum, stream);
     return check_launch("odl_fp8_amax_parts_colsum");
+}
+
+extern "C" int odl_fp8_amax_parts_slabs(const void *x, int src_dtype, int64_t rows, int64_t cols, float *parts, float *workspace, odl_stream_t stream_) {
+    if (const int rc = amax_colsum_pass("odl_fp8_amax_parts_slabs", x, src_dtype, rows, cols, parts, workspace, reinterpret_cast<hipStream_t>(stream_))) return rc;
+    return check_launch("odl_fp8_amax_parts_slabs");
+}
+
+extern "C" int odl_fp8_cast_dynamic_colsum(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, const float *parts, int fmt,
+                                           int margin, uint8_t *out, uint8_t *out_t, float *dyn_out, const float *workspace, void *colsum,
+                                           int colsum_dtype, odl_stream_t stream_) {
+    if (!parts || !dyn_out || !colsum || !workspace) return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic_colsum: null pointer");
+    if ((src_dtype != ODL_BF16 && src_dtype != ODL_F32) || (colsum_dtype != ODL_BF16 && colsum_dtype != ODL_F32))
+        return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic_colsum: src_dtype %d, colsum_dtype %d", src_dtype, colsum_dtype);
+    if (fmt != ODL_FP8_E4M3 && fmt != ODL_FP8_E5M2) return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic_colsum: fmt %d", fmt);
+    if (margin < -64 || margin > 64) return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic_colsum: margin %d", margin);
+    if (!cast_colsum_takes(x, rows, cols, rows_out, out, out_t) || (cols + 255) / 256 > kParts)
+        return set_error(ODL_ERR_SHAPE, "odl_fp8_cast_dynamic_colsum: both layouts, columns in multiples of 8, rows out of 16, 16-byte alignment");
+    int64_t slabs;
+    colsum_slab_rows(src_dtype, rows, cols, &slabs);
+    launch_cast_colsum(x, src_dtype, rows, cols, rows_out, parts, fmt, margin, out, out_t, dyn_out, workspace, (int)slabs, colsum, colsum_dtype,
+                       reinterpret_cast<hipStream_t>(stream_));
+    return check_launch("odl_fp8_cast_dynamic_colsum");
 }
 
 extern "C" int odl_fp8_layernorm_amax_parts(const void *x, int src_dtype, const float *weight, const float *bias, int64_t rows,
@@ -1225,4 +1322,21 @@ extern "C" int odl_fp8_gelu_bwd_amax_parts(const void *dy, const void *x, int64_
                        reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(table) + kGeluFwdBytes),
                        reinterpret_cast<u32x4 *>(dx), parts);
     return check_launch("odl_fp8_gelu_bwd_amax_parts");
+}
+
+extern "C" int odl_fp8_gelu_bwd_slabs(const void *dy, const void *x, int64_t rows, int64_t cols, const void *table, void *dx, float *parts,
+                                      float *workspace, odl_stream_t stream_) {
+    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+    if (rows <= 0 || cols <= 0) return set_error(ODL_ERR_ARG, "odl_fp8_gelu_bwd_slabs: empty or negative shape");
+    if (!dy || !x || !dx || !parts || !table || !workspace) return set_error(ODL_ERR_ARG, "odl_fp8_gelu_bwd_slabs: null pointer");
+    const int64_t col_blocks = (cols + 255) / 256;
+    if (cols % 8 != 0 || col_blocks > kParts || !aligned16(x) || !aligned16(dy) || !aligned16(dx) || !aligned16(table))
+        return set_error(ODL_ERR_SHAPE, "odl_fp8_gelu_bwd_slabs: cols must be a multiple of 8 and at most %d, pointers 16-byte aligned", kParts * 256);
+    int64_t slabs;
+    const int64_t rpb = colsum_slab_rows(ODL_BF16, rows, cols, &slabs);
+    hipLaunchKernelGGL(gelu_bwd_colsum_kernel, dim3((unsigned)col_blocks, (unsigned)slabs), dim3(kFusedThreads), 0, stream,
+                       reinterpret_cast<const uint16_t *>(dy), reinterpret_cast<const uint16_t *>(x), rows, cols, (int)rpb,
+                       reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(table) + kGeluFwdBytes), reinterpret_cast<uint16_t *>(dx),
+                       parts, workspace);
+    return check_launch("odl_fp8_gelu_bwd_slabs");
 }

@@ -27,10 +27,13 @@ decltype(&odl_fp8_quantise_small) quantise_small_c;
 decltype(&odl_fp8_gemm_swiglu) gemm_swiglu_c;
 decltype(&odl_fp8_cast_delayed_padded) cast_delayed_c;
 decltype(&odl_fp8_amax_parts_colsum) amax_colsum_c;
+decltype(&odl_fp8_amax_parts_slabs) amax_slabs_c;
+decltype(&odl_fp8_cast_dynamic_colsum) cast_colsum_c;
 decltype(&odl_fp8_swiglu_amax_parts) swiglu_c;
 decltype(&odl_fp8_swiglu_bwd_amax_parts) swiglu_bwd_c;
 decltype(&odl_fp8_gelu_amax_parts) gelu_c;
 decltype(&odl_fp8_gelu_bwd_amax_parts) gelu_bwd_c;
+decltype(&odl_fp8_gelu_bwd_slabs) gelu_bwd_slabs_c;
 decltype(&odl_fp8_rmsnorm_amax_parts) rmsnorm_c;
 decltype(&odl_fp8_rmsnorm_bwd) rmsnorm_bwd_c;
 decltype(&odl_fp8_layernorm_amax_parts) layernorm_c;
@@ -58,10 +61,13 @@ void bind(const py::dict &d) {
     take(gemm_swiglu_c, d, "odl_fp8_gemm_swiglu");
     take(cast_delayed_c, d, "odl_fp8_cast_delayed_padded");
     take(amax_colsum_c, d, "odl_fp8_amax_parts_colsum");
+    take(amax_slabs_c, d, "odl_fp8_amax_parts_slabs");
+    take(cast_colsum_c, d, "odl_fp8_cast_dynamic_colsum");
     take(swiglu_c, d, "odl_fp8_swiglu_amax_parts");
     take(swiglu_bwd_c, d, "odl_fp8_swiglu_bwd_amax_parts");
     take(gelu_c, d, "odl_fp8_gelu_amax_parts");
     take(gelu_bwd_c, d, "odl_fp8_gelu_bwd_amax_parts");
+    take(gelu_bwd_slabs_c, d, "odl_fp8_gelu_bwd_slabs");
     take(rmsnorm_c, d, "odl_fp8_rmsnorm_amax_parts");
     take(rmsnorm_bwd_c, d, "odl_fp8_rmsnorm_bwd");
     take(layernorm_c, d, "odl_fp8_layernorm_amax_parts");
@@ -171,11 +177,26 @@ py::object cast_delayed(const Tensor &x, const Tensor &scale, int fmt, const Opt
     return rc ? status(rc) : py::make_tuple(obj(q), obj(q_t), inv);
 }
 
-py::object amax_colsum(const Tensor &x, i64 stream) {
+py::object amax_colsum(const Tensor &x, bool finish, i64 stream) {
     if (!source2d(x)) return none();
+    if (!finish && x.size(1) % 8 == 0 && aligned(x)) {
+        Tensor parts = f32(x, {kParts}), ws = f32(x, {kParts, ODL_FP8_COLSUM_WORKSPACE / kParts});
+        const int rc = call(amax_slabs_c, ptr(x), src_of(x), x.size(0), x.size(1), ptr(parts), ptr(ws), str(stream));
+        return rc ? status(rc) : py::make_tuple(parts, ws);
+    }
     Tensor parts = f32(x, {kParts}), sums = f32(x, {x.size(1)}), ws = f32(x, {ODL_FP8_COLSUM_WORKSPACE});
     const int rc = call(amax_colsum_c, ptr(x), src_of(x), x.size(0), x.size(1), ptr(parts), ptr(sums), ptr(ws), str(stream));
     return rc ? status(rc) : py::make_tuple(parts, sums);
+}
+
+py::object cast_colsum(const Tensor &x, const Tensor &parts, const Tensor &slabs, int fmt, int margin, i64 rows_out, int odt, i64 stream) {
+    if (!source2d(x) || !aligned(x) || !floats(parts, kParts) || !floats(slabs, ODL_FP8_COLSUM_WORKSPACE) || x.size(1) % 8) return none();
+    const i64 rows = x.size(0), cols = x.size(1);
+    Tensor q = bytes(x, {rows_out, cols}), q_t = bytes(x, {cols, rows_out}), dyn = f32(x, {3});
+    Tensor sums = at::empty({cols}, x.options().dtype(odt ? at::kFloat : at::kBFloat16));
+    const int rc = call(cast_colsum_c, ptr(x), src_of(x), rows, cols, rows_out, ptr(parts), fmt, margin, ptr(q), ptr(q_t), ptr(dyn), ptr(slabs), ptr(sums),
+                        odt, str(stream));
+    return rc ? status(rc) : py::make_tuple(q, q_t, dyn.narrow(0, 2, 1), sums);
 }
 
 i64 last(const Tensor &t) { return t.dim() ? t.size(-1) : 1; }
@@ -211,6 +232,15 @@ py::object gelu_bwd(const Tensor &dy, const Tensor &x, const Tensor &table, i64 
     Tensor dx = at::empty_like(x), parts = f32(x, {kParts});
     const int rc = call(gelu_bwd_c, ptr(dy), ptr(x), rows, cols, ptr(table), ptr(dx), ptr(parts), str(stream));
     return rc ? status(rc) : py::make_tuple(dx, parts);
+}
+
+py::object gelu_bwd_slabs(const Tensor &dy, const Tensor &x, const Tensor &table, i64 stream) {
+    if (!bf16(dy) || !bf16(x) || dy.sizes() != x.sizes() || x.numel() == 0) return none();
+    const i64 cols = last(x), rows = x.numel() / cols;
+    if (cols % 8 || cols > kParts * 256) return none();
+    Tensor dx = at::empty_like(x), parts = f32(x, {kParts}), ws = f32(x, {kParts, ODL_FP8_COLSUM_WORKSPACE / kParts});
+    const int rc = call(gelu_bwd_slabs_c, ptr(dy), ptr(x), rows, cols, ptr(table), ptr(dx), ptr(parts), ptr(ws), str(stream));
+    return rc ? status(rc) : py::make_tuple(dx, parts, ws);
 }
 
 // rows of a norm: dense, aligned, with vectors of the row length in fp32 on the same device
@@ -421,10 +451,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("gemm_swiglu", &gemm_swiglu);
     m.def("cast_delayed", &cast_delayed);
     m.def("amax_colsum", &amax_colsum);
+    m.def("cast_colsum", &cast_colsum);
     m.def("swiglu", &swiglu);
     m.def("swiglu_bwd", &swiglu_bwd);
     m.def("gelu", &gelu);
     m.def("gelu_bwd", &gelu_bwd);
+    m.def("gelu_bwd_slabs", &gelu_bwd_slabs);
     m.def("rmsnorm", &rmsnorm);
     m.def("rmsnorm_bwd", &rmsnorm_bwd);
     m.def("layernorm", &layernorm);

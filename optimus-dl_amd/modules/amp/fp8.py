@@ -216,7 +216,7 @@ class FP8Recipe:
         self.direct_layouts: "bool | str" = "auto"
         # partial maxima handed over by the kernel that produced a tensor (SwiGLU, RMSNorm), so that
         # the Linear that quantises this very tensor skips its amax pass; a handful of entries
-        self.producer_parts: list[tuple[tuple, torch.Tensor, torch.Tensor]] = []
+        self.producer_parts: list[tuple[tuple, torch.Tensor, torch.Tensor, torch.Tensor | None]] = []
         # Linears fed by one tensor (q/k/v, gate/up) run as one autograd node whose data gradients are summed by the
         # GEMMs' accumulate flag (modules/fp8_linear.py: linear_group, SiblingGroup); False: every Linear on its own
         self.fuse_dgrad_sum = True
@@ -363,26 +363,30 @@ class FP8Recipe:
     def _tensor_key(t: torch.Tensor) -> tuple:
         return (t.data_ptr(), _state.tensor_version(t), t.numel(), t.dtype, t.device)
 
-    def offer_parts(self, tensor: torch.Tensor, parts: torch.Tensor) -> None:
-        """Record the partial maxima of |tensor| that its producer computed.  The entry keeps the
+    def offer_parts(self, tensor: torch.Tensor, parts: torch.Tensor, slabs: torch.Tensor | None = None) -> None:
+        """Record the partial maxima of |tensor| (and slabs of its column sums) that its producer computed.  The entry keeps the
         tensor alive (its address cannot be reused meanwhile); an in-place change bumps the
         version and the entry no longer matches."""
         if self._recipe.kind != "tensorwise":
             return
-        self.producer_parts.append((self._tensor_key(tensor), tensor, parts))
+        self.producer_parts.append((self._tensor_key(tensor), tensor, parts, slabs))
         if len(self.producer_parts) > 8:
             del self.producer_parts[0]
 
     def take_parts(self, tensor: torch.Tensor) -> torch.Tensor | None:
         """Partial maxima for exactly this tensor (or a view of all of it), if a producer left them."""
+        return self.take_parts_and_slabs(tensor)[0]
+
+    def take_parts_and_slabs(self, tensor: torch.Tensor) -> tuple[torch.Tensor | None, torch.Tensor | None]:
+        """The same, and the slabs of its column sums (``native.amax_parts_colsum(tensor, finish=False)``) if it left those too."""
         if not self.producer_parts:
-            return None
+            return None, None
         key = self._tensor_key(tensor)
-        for i, (k, _, parts) in enumerate(self.producer_parts):
+        for i, (k, made, parts, slabs) in enumerate(self.producer_parts):
             if k == key:
                 del self.producer_parts[i]
-                return parts
-        return None
+                return parts, slabs if made.shape[-1:] == tensor.shape[-1:] else None      # sums of other columns than a view's
+        return None, None
 
     # ---------------------------------------------------------------- contexts
     @contextmanager

@@ -378,15 +378,24 @@ class _Fp8LinearFn(torch.autograd.Function):
                                                          recipe=recipe, record=module.training, margin=pol.margin, out_t=gq_t_out,
                                                          rows_out=rows_out)
                 else:
-                    parts = recipe.take_parts(dy2d)
+                    parts, left = recipe.take_parts_and_slabs(dy2d)
+                    slabs = None
                     if ctx.has_bias and native.colsum_supported(dy2d):
                         # the amax pass also adds up the columns: the bias gradient costs no extra read of dy.  It
                         # runs for the column sums even when the producer of dy left its partial maxima (which are
-                        # the same numbers): one pass of this kernel is cheaper than a separate sum over the rows
-                        parts, colsum = native.amax_parts_colsum(dy2d)
-                        db = colsum.to(ctx.bias_dtype)
-                    gq, gq_t, sg_inv, _ = _quantise_dynamic(dy2d, pol.fmt_bwd, pol.margin, g_t_needed, g_rm_needed,
-                                                            parts=parts, out_t=gq_t_out, rows_out=rows_out)
+                        # the same numbers), unless that left the sums too: one pass of this kernel is cheaper than a separate
+                        # sum over the rows.  Slabs of sums are added up, and rounded, by blocks of the cast where that writes both layouts
+                        with_cast = g_t_needed and g_rm_needed and gq_t_out is None and ctx.bias_dtype in (torch.bfloat16, torch.float32)
+                        parts, sums = native.amax_parts_colsum(dy2d, finish=not with_cast, left=None if left is None else (parts, left))
+                        if sums.dim() == 2:
+                            slabs = sums
+                        else:
+                            db = sums.to(ctx.bias_dtype)
+                    if slabs is not None:
+                        gq, gq_t, sg_inv, db = native.cast_dynamic_colsum(dy2d, parts, slabs, pol.fmt_bwd, pol.margin, rows_out, ctx.bias_dtype)
+                    else:
+                        gq, gq_t, sg_inv, _ = _quantise_dynamic(dy2d, pol.fmt_bwd, pol.margin, g_t_needed, g_rm_needed,
+                                                                parts=parts, out_t=gq_t_out, rows_out=rows_out)
             if ctx.need_dgrad:
                 gq_rows = _rows(gq, tokens)
                 # a member of a group of Linears fed by one tensor leaves its operands to the group's one GEMM over

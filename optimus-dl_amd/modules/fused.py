@@ -434,8 +434,11 @@ class _GeluFn(torch.autograd.Function):
         (x,) = ctx.saved_tensors
         if dy.dtype != torch.bfloat16:
             dy = dy.to(torch.bfloat16)
-        dx, parts = native.gelu_bwd_amax_parts(dy, x)
-        ctx.recipe.offer_parts(dx, parts)
+        if ctx.recipe.recipe.kind == "tensorwise":         # c_fc has a bias as a rule
+            dx, parts, slabs = native.gelu_bwd_slabs(dy, x)
+            ctx.recipe.offer_parts(dx, parts, slabs)
+        else:
+            dx, _ = native.gelu_bwd_amax_parts(dy, x)
         return dx, None
 
 

@@ -55,6 +55,8 @@ EXPORTS = (
     "odl_fp8_multi_cast_dynamic",
     "odl_fp8_multi_cast_delayed",
     "odl_fp8_amax_parts_colsum",
+    "odl_fp8_amax_parts_slabs",
+    "odl_fp8_cast_dynamic_colsum",
     "odl_fp8_swiglu_amax_parts",
     "odl_fp8_swiglu_bwd_amax_parts",
     "odl_fp8_rmsnorm_amax_parts",
@@ -64,6 +66,7 @@ EXPORTS = (
     "odl_fp8_gelu_table",
     "odl_fp8_gelu_amax_parts",
     "odl_fp8_gelu_bwd_amax_parts",
+    "odl_fp8_gelu_bwd_slabs",
     "odl_fp8_amax_rowcol",
     "odl_fp8_cast_rowcol",
     "odl_fp8_cast",
@@ -77,10 +80,10 @@ EXPORTS = (
     "odl_fp8_gemm_chain_route",
     "odl_fp8_gemm_nt_chain",
     "odl_fp8_gemm_layouts",
+    "odl_fp8_gemm_wgrad",
     "odl_fp8_gemm_split_count",
     "odl_fp8_gemm_runs",
     "odl_fp8_gemm_splitk",
-    "odl_fp8_gemm_wgrad",
     "odl_fp8_delayed_update",
     "odl_fp8_gemm_num_variants",
     "odl_fp8_gemm_variant_name",
@@ -152,6 +155,8 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_multi_amax_parts.argtypes = [vp, vp, i64, vp]
         L.odl_fp8_multi_cast_dynamic.argtypes = [vp, vp, i64, i32, i32, vp]
         L.odl_fp8_multi_cast_delayed.argtypes = [vp, vp, i64, i32, vp]
+        L.odl_fp8_amax_parts_slabs.argtypes = [vp, i32, i64, i64, vp, vp, vp]
+        L.odl_fp8_cast_dynamic_colsum.argtypes = [vp, i32, i64, i64, i64, vp, i32, i32, vp, vp, vp, vp, vp, i32, vp]
         L.odl_fp8_amax_parts_colsum.argtypes = [vp, i32, i64, i64, vp, vp, vp, vp]
         L.odl_fp8_swiglu_amax_parts.argtypes = [vp, vp, i64, i64, vp, vp, vp]
         L.odl_fp8_swiglu_bwd_amax_parts.argtypes = [vp, vp, vp, i64, i64, vp, vp, vp, vp, vp]
@@ -161,6 +166,7 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_gelu_table.argtypes = [vp, vp]
         L.odl_fp8_gelu_amax_parts.argtypes = [vp, i64, i64, vp, vp, vp, vp]
         L.odl_fp8_gelu_bwd_amax_parts.argtypes = [vp, vp, i64, i64, vp, vp, vp, vp]
+        L.odl_fp8_gelu_bwd_slabs.argtypes = [vp, vp, i64, i64, vp, vp, vp, vp, vp]
         L.odl_fp8_layernorm_bwd.argtypes = [vp, vp, i32, vp, vp, vp, i64, i64, vp, vp, vp, vp, vp]
         L.odl_fp8_amax_rowcol.argtypes = [vp, i32, i64, i64, vp, vp, vp]
         L.odl_fp8_cast_rowcol.argtypes = [vp, i32, i64, i64, vp, vp, i32, i32, vp, vp, vp, vp, vp, vp, vp]
@@ -174,13 +180,13 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_gemm_group_route.argtypes = [i32, vp, vp, i64, i32]
         L.odl_fp8_gemm_nt_group.argtypes = [i32, vp, vp, vp, vp, i64, i32, i32, vp, vp, vp, i32, i32, vp]
         L.odl_fp8_gemm_nt_sum.argtypes = [i32, vp, vp, vp, i64, i64, i32, i32, vp, vp, vp, i32, vp]
+        L.odl_fp8_gemm_wgrad.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, vp, vp, i32, vp]
         L.odl_fp8_gemm_layouts.argtypes = [vp, vp, i64, i64, i64, i32, i32, i32, i32, vp, vp, vp, i32, vp]
         L.odl_fp8_gemm_split_count.argtypes = [i64, i64, i64, i32]
         L.odl_fp8_gemm_split_count.restype = i32
         L.odl_fp8_gemm_runs.argtypes = [i64, i64, i64, i32]
         L.odl_fp8_gemm_runs.restype = i32
         L.odl_fp8_gemm_splitk.argtypes = [vp, vp, i64, i64, i64, i32, i32, i32, i32, vp, i64, vp, i64, vp, vp, i32, i32, i32, vp, i64, vp]
-        L.odl_fp8_gemm_wgrad.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, vp, vp, i32, vp]
         L.odl_fp8_delayed_update.argtypes = [vp, i64, i64, i64, vp, vp, vp, i32, i32, vp, vp]
         L.odl_fp8_gemm_num_variants.restype = i32
         L.odl_fp8_gemm_variant_name.argtypes = [i32]
@@ -387,11 +393,15 @@ def colsum_supported(x: torch.Tensor) -> bool:
     return x.shape[1] % cpl == 0 and x.shape[1] <= AMAX_PARTS * 32 * cpl and x.is_contiguous() and x.data_ptr() % 16 == 0
 
 
-def amax_parts_colsum(x: torch.Tensor):
-    """Partial maxima of |x| and the fp32 column sums of x in one pass.  -> (parts, colsum[cols])."""
+def amax_parts_colsum(x: torch.Tensor, finish: bool = True, left: "tuple | None" = None):
+    """Partial maxima of |x| and the fp32 column sums of x in one pass.  -> (parts, colsum[cols]).  finish=False: the sums stay in
+    slabs, a 2-D tensor, for the cast that follows to add up (:func:`cast_dynamic_colsum`); where that cast does not take x they are
+    finished all the same.  left: (parts, slabs) of x that its producer left (:func:`gelu_bwd_slabs`); nothing is launched then."""
+    if left is not None and not finish:
+        return left
     if x.is_cuda:
         load()
-        r = _host.amax_colsum(x, _stream())
+        r = _host.amax_colsum(x, finish, _stream())
         if r is not None:
             return _done(r, "odl_fp8_amax_parts_colsum")
     x = _as_2d(x)
@@ -402,6 +412,17 @@ def amax_parts_colsum(x: torch.Tensor):
     _check(load().odl_fp8_amax_parts_colsum(x.data_ptr(), _src_dtype(x), rows, cols, parts.data_ptr(), colsum.data_ptr(),
                                             ws.data_ptr(), _stream()), "odl_fp8_amax_parts_colsum")
     return parts, colsum
+
+
+def cast_dynamic_colsum(x: torch.Tensor, parts: torch.Tensor, slabs: torch.Tensor, fmt: int, margin: int, rows_out: int,
+                        dtype: torch.dtype):
+    """Both layouts of :func:`cast_dynamic`, and the column sums that ``amax_parts_colsum(x, finish=False)`` left in slabs, rounded to
+    ``dtype`` (bf16 or fp32), in one launch.  -> (q, q_t, scale_inv, colsum[cols])."""
+    load()
+    r = _host.cast_colsum(x, parts, slabs, fmt, margin, rows_out, _OUT_DTYPES[dtype], _stream())
+    if r is None:
+        raise NativeError("cast_dynamic_colsum: x, its partial maxima or its slabs are not those of amax_parts_colsum(x, finish=False)")
+    return _done(r, "odl_fp8_cast_dynamic_colsum")
 
 
 def _codes_out(t: torch.Tensor, shape: tuple, device, what: str) -> torch.Tensor:
@@ -797,6 +818,17 @@ def gelu_amax_parts(x: torch.Tensor):
     _check(load().odl_fp8_gelu_amax_parts(x.data_ptr(), rows, cols, gelu_table(x.device).data_ptr(), y.data_ptr(), parts.data_ptr(),
                                           _stream()), "odl_fp8_gelu_amax_parts")
     return y, parts
+
+
+def gelu_bwd_slabs(dy: torch.Tensor, x: torch.Tensor):
+    """:func:`gelu_bwd_amax_parts`, and the slabs of column sums that ``amax_parts_colsum(dx, finish=False)`` would leave, where the
+    row length allows (else None).  -> (dx, parts, slabs)."""
+    if x.is_cuda:
+        load()
+        r = _host.gelu_bwd_slabs(dy, x, gelu_table(x.device), _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_gelu_bwd_slabs")
+    return (*gelu_bwd_amax_parts(dy, x), None)
 
 
 def gelu_bwd_amax_parts(dy: torch.Tensor, x: torch.Tensor):
@@ -1406,6 +1438,35 @@ def wgrad_direct_pays(n_out: int, n_in: int, tokens: int) -> bool:
     return tiles >= 192 or 262_144 <= elements < 1_800_000 and tokens >= (8192 if elements >= 400_000 else 16384)
 
 
+def gemm_wgrad_pays(n_out: int, n_in: int, tokens: int, out_dtype: torch.dtype = torch.bfloat16) -> bool:
+    """Whether :func:`gemm_wgrad` takes a weight gradient that :func:`gemm_layouts` does not (n_out no multiple of 256) and is faster
+    than the route over a transposed copy of dY: where its tiles fill the chip, as in :func:`wgrad_direct_pays`.  50304 x 768
+    fp32, product and cast of dY, this way / over the copy in us: 1024 tokens 88 / 99, 2048 142 / 159, 8192 589 / 704, 16384 1190 / 1417."""
+    return (n_out % 256 != 0 and n_out % 16 == 0 and n_in % 128 == 0 and tokens % 128 == 0 and tokens >= 512
+            and out_dtype in (torch.bfloat16, torch.float32) and -(-n_out // 256) * -(-n_in // 256) >= 192
+            and (n_out + 256) * tokens < 2**31 and (n_in + 256) * tokens < 2**31 and n_in * out_dtype.itemsize * 264 < 2**31)
+
+
+def gemm_wgrad(gy: torch.Tensor, x_t: torch.Tensor, fmt_g: int, fmt_x: int, sg_inv: torch.Tensor, sx_inv: torch.Tensor,
+               out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
+    """dW [n_out, n_in] = dY^T . X from the codes gy [tokens, n_out] of dY as stored and x_t [n_in, tokens] of X^T, as
+    :func:`gemm_layouts`, for any n_out >= 256 in multiples of 16 and n_in of 128."""
+    if gy.dtype != torch.uint8 or x_t.dtype != torch.uint8:
+        raise NativeError("gemm_wgrad operands must be uint8 FP8 codes")
+    gy, x_t = _as_2d(gy), _as_2d(x_t)
+    (tokens, n_out), (n_in, k) = gy.shape, x_t.shape
+    if k != tokens:
+        raise NativeError(f"gemm_wgrad: contraction sizes differ ({tokens} vs {k})")
+    if out_dtype not in _OUT_DTYPES:
+        raise NativeError(f"gemm_wgrad: {out_dtype} output")
+    _f32_dev(sg_inv, 1, "gemm_wgrad sg_inv")
+    _f32_dev(sx_inv, 1, "gemm_wgrad sx_inv")
+    dw = torch.empty((n_out, n_in), dtype=out_dtype, device=gy.device)
+    _check(load().odl_fp8_gemm_wgrad(gy.data_ptr(), x_t.data_ptr(), n_out, n_in, tokens, fmt_g, fmt_x, sg_inv.data_ptr(), sx_inv.data_ptr(),
+                                     dw.data_ptr(), _OUT_DTYPES[out_dtype], _stream()), "odl_fp8_gemm_wgrad")
+    return dw
+
+
 def dgrad_sum_in_one_launch(tokens: int, n_in: int, n_outs: "list[int]") -> bool:
     """Whether the data gradient of Linears fed by one tensor, dX [tokens, n_in] = sum_s dY_s [tokens, n_outs[s]] . W_s, runs
     as ONE launch of :func:`gemm_nt_sum` (the streaming kernel carrying its accumulators from one pair to the next): the
@@ -1438,35 +1499,6 @@ def gemm_layouts(a: torch.Tensor, b: torch.Tensor, fmt_a: int, fmt_b: int, layou
     a, b = _as_2d(a), _as_2d(b)
     M, K = (a.shape[1], a.shape[0]) if layout_a == K_SLOW else a.shape
     N, K2 = (b.shape[1], b.shape[0]) if layout_b == K_SLOW else b.shape
-def gemm_wgrad_pays(n_out: int, n_in: int, tokens: int, out_dtype: torch.dtype = torch.bfloat16) -> bool:
-    """Whether :func:`gemm_wgrad` takes a weight gradient that :func:`gemm_layouts` does not (n_out no multiple of 256) and is faster
-    than the route over a transposed copy of dY: where its tiles fill the chip, as in :func:`wgrad_direct_pays`.  50304 x 768
-    fp32, product and cast of dY, this way / over the copy in us: 1024 tokens 88 / 99, 2048 142 / 159, 8192 589 / 704, 16384 1190 / 1417."""
-    return (n_out % 256 != 0 and n_out % 16 == 0 and n_in % 128 == 0 and tokens % 128 == 0 and tokens >= 512
-            and out_dtype in (torch.bfloat16, torch.float32) and -(-n_out // 256) * -(-n_in // 256) >= 192
-            and (n_out + 256) * tokens < 2**31 and (n_in + 256) * tokens < 2**31 and n_in * out_dtype.itemsize * 264 < 2**31)
-
-
-def gemm_wgrad(gy: torch.Tensor, x_t: torch.Tensor, fmt_g: int, fmt_x: int, sg_inv: torch.Tensor, sx_inv: torch.Tensor,
-               out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
-    """dW [n_out, n_in] = dY^T . X from the codes gy [tokens, n_out] of dY as stored and x_t [n_in, tokens] of X^T, as
-    :func:`gemm_layouts`, for any n_out >= 256 in multiples of 16 and n_in of 128."""
-    if gy.dtype != torch.uint8 or x_t.dtype != torch.uint8:
-        raise NativeError("gemm_wgrad operands must be uint8 FP8 codes")
-    gy, x_t = _as_2d(gy), _as_2d(x_t)
-    (tokens, n_out), (n_in, k) = gy.shape, x_t.shape
-    if k != tokens:
-        raise NativeError(f"gemm_wgrad: contraction sizes differ ({tokens} vs {k})")
-    if out_dtype not in _OUT_DTYPES:
-        raise NativeError(f"gemm_wgrad: {out_dtype} output")
-    _f32_dev(sg_inv, 1, "gemm_wgrad sg_inv")
-    _f32_dev(sx_inv, 1, "gemm_wgrad sx_inv")
-    dw = torch.empty((n_out, n_in), dtype=out_dtype, device=gy.device)
-    _check(load().odl_fp8_gemm_wgrad(gy.data_ptr(), x_t.data_ptr(), n_out, n_in, tokens, fmt_g, fmt_x, sg_inv.data_ptr(), sx_inv.data_ptr(),
-                                     dw.data_ptr(), _OUT_DTYPES[out_dtype], _stream()), "odl_fp8_gemm_wgrad")
-    return dw
-
-
     if K != K2:
         raise NativeError(f"gemm_layouts: contraction sizes differ ({K} vs {K2})")
     _f32_dev(sa_inv, 1, "gemm_layouts sa_inv")

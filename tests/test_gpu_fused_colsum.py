@@ -1,0 +1,85 @@
+"""Column sums on the way to a cast (odl_fp8_amax_parts_slabs, odl_fp8_gelu_bwd_slabs, odl_fp8_cast_dynamic_colsum): the codes, the scale
+and the sums are those of the separate launches, bit for bit, at the edges of tiles, slabs and column blocks."""
+import pytest
+import torch
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 8, 16), (16, 16, 16), (33, 264, 48), (320, 768, 320), (500, 1032, 640), (1000, 3072, 1024), (16400, 256, 16512), (40, 131072, 48)]
+
+
+def parts_max(parts):
+    return parts.max().reshape(1)
+
+
+@pytest.mark.parametrize("fmt", [O.E4M3, O.E5M2])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols,rows_out", SHAPES)
+def test_sums_finished_by_the_cast(rows, cols, rows_out, dtype, fmt):
+    from optimus_dl_amd import native as N
+
+    x = torch.randn((rows, cols), generator=torch.Generator().manual_seed(rows + cols)).to(dtype).cuda()
+    if not N.colsum_supported(x):
+        pytest.skip("more columns than the pass takes in fp32")
+    want_parts, want_sums = N.amax_parts_colsum(x)
+    want_q, want_qt, _, _, want_inv = N.cast_dynamic(x, want_parts, fmt, 1, rows_out=rows_out)
+    for out in (torch.bfloat16, torch.float32):
+        parts, slabs = N.amax_parts_colsum(x, finish=False)
+        assert slabs.dim() == 2 and torch.equal(parts, want_parts)
+        q, qt, inv, sums = N.cast_dynamic_colsum(x, parts, slabs, fmt, 1, rows_out, out)
+        assert sums.dtype == out and torch.equal(sums, want_sums.to(out))
+        assert torch.equal(inv, want_inv) and torch.equal(qt, want_qt) and torch.equal(q, want_q)
+
+
+def test_sums_of_infinities_and_nan():
+    from optimus_dl_amd import native as N
+
+    x = torch.zeros((64, 32), dtype=torch.bfloat16)
+    x[3, 1], x[5, 2], x[6, 2], x[9, 4] = float("inf"), float("inf"), float("-inf"), float("nan")
+    x = x.cuda()
+    _, want = N.amax_parts_colsum(x)
+    parts, slabs = N.amax_parts_colsum(x, finish=False)
+    sums = N.cast_dynamic_colsum(x, parts, slabs, O.E5M2, 0, 64, torch.bfloat16)[3]
+    assert torch.equal(sums.isnan(), want.isnan()) and torch.equal(sums.nan_to_num(), want.to(torch.bfloat16).nan_to_num())
+    assert sums[1].item() == float("inf") and bool(sums[2].isnan()) and bool(sums[4].isnan())
+
+
+def test_columns_the_cast_does_not_take_are_finished_by_the_pass():
+    from optimus_dl_amd import native as N
+
+    x = torch.randn((48, 12), device="cuda")          # fp32: the pass takes multiples of four, the cast of eight
+    want = N.amax_parts_colsum(x)
+    got = N.amax_parts_colsum(x, finish=False)
+    assert got[1].dim() == 1 and all(torch.equal(a, b) for a, b in zip(got, want))
+    with pytest.raises(N.NativeError):
+        N.cast_dynamic_colsum(x, *got, O.E4M3, 0, 48, torch.float32)
+
+
+@pytest.mark.parametrize("rows,cols", [(r, c) for r, c, _ in SHAPES])
+def test_gelu_backward_leaves_the_slabs(rows, cols):
+    from optimus_dl_amd import native as N
+
+    g = torch.Generator().manual_seed(rows * cols)
+    x, dy = ((torch.randn((rows, cols), generator=g) * s).to(torch.bfloat16).cuda() for s in (2.0, 1e-2))
+    want, want_parts = N.gelu_bwd_amax_parts(dy, x)
+    dx, parts, slabs = N.gelu_bwd_slabs(dy, x)
+    assert torch.equal(dx, want) and torch.equal(parts_max(parts), parts_max(want_parts))
+    own_parts, own = N.amax_parts_colsum(dx, finish=False)
+    used = (-(-rows // max(32, -(-(-(-rows // (N.AMAX_PARTS // -(-cols // 256)))) // 32) * 32))) * cols      # slabs x columns
+    assert torch.equal(slabs.reshape(-1)[:used], own.reshape(-1)[:used])
+    assert N.amax_parts_colsum(dx, finish=False, left=(parts, slabs))[1] is slabs
+
+
+def test_slabs_are_not_handed_to_a_view_of_other_columns():
+    from optimus_dl_amd.modules import amp
+
+    recipe = amp.FP8Recipe(recipe_type="tensorwise")
+    t = torch.zeros((64, 32), dtype=torch.bfloat16, device="cuda")
+    parts, slabs = torch.zeros(4, device="cuda"), torch.zeros((2, 2), device="cuda")
+    recipe.offer_parts(t, parts, slabs)
+    assert recipe.take_parts_and_slabs(t.view(32, 64)) == (parts, None)
+    recipe.offer_parts(t.view(2, 32, 32), parts, slabs)
+    got = recipe.take_parts_and_slabs(t)
+    assert got[0] is parts and got[1] is slabs
