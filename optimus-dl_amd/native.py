@@ -1082,13 +1082,14 @@ def gemm_nt_group(a: "list[torch.Tensor]", b: "list[torch.Tensor]", fmt_a: int, 
 
 
 def gemm_swiglu_pays(M: int, N: int, K: int) -> bool:
-    """Whether :func:`gemm_swiglu` takes a shape and is faster than two :func:`gemm_nt` and the SwiGLU kernel.  us, one launch /
-    three, weights from memory: 32 rows 1024 -> 3072 4.9 / 18.4, 4096 -> 14336 28 / 40, 4096 -> 28672 48 / 67, but 1024 -> 50304 30 /
-    33; 64 rows 1024 -> 3072 5.6 / 18.9, 512 -> 8192 6.8 / 15.7, 4096 -> 16384 32 / 45, but 4096 -> 28672 62 / 70 and 1024 -> 28672 25 / 25.
-    From 33 rows on, contractions of less than 512 only up to 4096 columns, as far as they were measured first."""
+    """Whether a gated MLP takes :func:`gemm_swiglu` in place of two :func:`gemm_nt` and the SwiGLU kernel: four rounds of 16-column
+    blocks up to 32 rows, up to 64 one round below K = 2048.  Its last places differ from those of separate products that do not take the
+    thin kernel, so which sizes these are is part of the contract; it is faster beyond them too.  us, one launch / three, weights
+    from memory: 32 rows 1024 -> 3072 4.9 / 18.4, 4096 -> 14336 28 / 40, 4096 -> 28672 48 / 67, but 1024 -> 50304 30 / 33; 64 rows 1024 -> 3072
+    5.6 / 18.9, 512 -> 8192 6.8 / 15.7, 4096 -> 16384 32 / 45, but 4096 -> 28672 62 / 70 and 1024 -> 28672 25 / 25."""
     if not (0 < M <= 64 and N > 0 and N % 4 == 0 and K > 0 and K % 128 == 0 and N * K < 2**32 and M * K < 2**32):
         return False
-    return N <= 28672 if M <= 32 else N <= 4096 or (K >= 512 and N <= 16384)
+    return N <= 16384 if M <= 32 else (N <= 4096 and K < 2048)
 
 
 def gemm_swiglu(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, fmt_x: int, fmt_w: int, sx_inv: torch.Tensor, sg_inv: torch.Tensor,

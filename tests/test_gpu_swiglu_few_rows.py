@@ -33,11 +33,3 @@ def test_one_launch_has_the_bits_of_three(rows, cols, K):
     want, want_parts = N.swiglu_amax_parts(a.reshape(-1), b.reshape(-1))
     assert h.shape == (rows, cols) and torch.equal(h.reshape(-1), want)
     assert parts.numel() == N.AMAX_PARTS and parts.max().item() == want_parts.max().item()
-
-
-def test_where_one_launch_is_taken():
-    from optimus_dl_amd import native as N
-
-    yes = [(32, 14336, 4096), (16, 28672, 4096), (64, 3072, 1024), (48, 8192, 512), (64, 16384, 4096), (64, 2048, 256)]
-    no = [(32, 50304, 1024), (64, 28672, 4096), (64, 4352, 256), (65, 1024, 1024), (32, 1022, 1024), (32, 1024, 1000), (0, 1024, 1024)]
-    assert all(N.gemm_swiglu_pays(*c) for c in yes) and not any(N.gemm_swiglu_pays(*c) for c in no)
