@@ -24,9 +24,9 @@ owns the scaling policy itself:
 from __future__ import annotations
 
 import logging
+import sys
 import weakref
-from collections.abc import Iterator
-from contextlib import contextmanager
+from contextlib import ContextDecorator
 from dataclasses import dataclass
 from enum import Enum
 from typing import Any
@@ -389,45 +389,30 @@ class FP8Recipe:
         return None, None
 
     # ---------------------------------------------------------------- contexts
-    @contextmanager
-    def autocast(self) -> Iterator[None]:
+    def autocast(self) -> "_RecipeScope":
         """Forward context: FP8 Linears quantise while it is active.  Leaving the
         outermost one refreshes the forward scales (delayed scaling)."""
-        _state.push_recipe(self)
-        self._depth += 1
-        try:
-            yield
-        finally:
-            self._depth -= 1
-            _state.pop_recipe()
-            if self._depth == 0:
-                self.shared_input = None
-                self.producer_parts.clear()
-                for grp in list(self._sibling_groups):      # outputs made for siblings that were never asked for
-                    grp.clear()
-                self._sibling_groups.clear()
-                self.update_scales("fwd")
-                # gradients recorded by a backward that ran outside any backward()
-                # context are folded in here, one step late but never lost
-                self.update_scales("bwd")
+        return _RecipeScope(self, False)
 
-    @contextmanager
-    def backward(self) -> Iterator[None]:
+    def backward(self) -> "_RecipeScope":
         """Backward context: leaving it refreshes the gradient scales."""
-        _state.push_recipe(self)
-        self._depth += 1
-        try:
-            yield
-        finally:
-            self._depth -= 1
-            _state.pop_recipe()
-            if self._depth == 0:
-                self.shared_input = None          # a forward recomputed by activation checkpointing may have left one
-                self.producer_parts.clear()
-                for grp in list(self._sibling_groups):
-                    grp.clear()
-                self._sibling_groups.clear()
-                self.update_scales("bwd")
+        return _RecipeScope(self, True)
+
+    def _left(self, backward: bool) -> None:
+        """The outermost context of this recipe has been left."""
+        self.shared_input = None                  # (a backward's: a forward recomputed by activation checkpointing may have left one)
+        self.producer_parts.clear()
+        if len(self._sibling_groups):
+            for grp in list(self._sibling_groups):      # outputs made for siblings that were never asked for
+                grp.clear()
+            self._sibling_groups.clear()
+        if not self.is_delayed:
+            return
+        if not backward:
+            self.update_scales("fwd")
+        # (leaving a forward: gradients recorded by a backward that ran outside any backward()
+        # context are folded in here, one step late but never lost)
+        self.update_scales("bwd")
 
     def prepare_for_backward(self, *args: Any, **kwargs: Any) -> tuple[Any, ...]:
         return args
@@ -460,29 +445,84 @@ def create_fp8_recipe(
                      wgrad=wgrad, mx_scale_rule=mx_scale_rule)
 
 
-@contextmanager
+class _RecipeScope(ContextDecorator):
+    """An FP8 recipe in force.  The contexts of this module are classes, not generators: entering and leaving is host time of every
+    step, and what a decode step waits for (those of an evaluation forward 10.2 -> 7.9 us)."""
+
+    def __init__(self, recipe: FP8Recipe, backward: bool):
+        self._recipe, self._backward = recipe, backward
+
+    def _recreate_cm(self):
+        return _RecipeScope(self._recipe, self._backward)
+
+    def __enter__(self) -> None:
+        _state.push_recipe(self._recipe)
+        self._recipe._depth += 1
+
+    def __exit__(self, *exc) -> None:
+        recipe = self._recipe
+        recipe._depth -= 1
+        _state.pop_recipe()
+        if recipe._depth == 0:
+            recipe._left(self._backward)
+
+
+class NestedScopes(ContextDecorator):
+    """At most two contexts, one inside the other, made by ``_scopes()`` when this one is entered."""
+
+    def __init__(self, *args):
+        self._args, self._open = args, []
+
+    def _recreate_cm(self):
+        return type(self)(*self._args)
+
+    def _scopes(self, *args) -> tuple:
+        raise NotImplementedError
+
+    def __enter__(self) -> None:
+        scopes = self._scopes(*self._args)
+        if scopes:
+            scopes[0].__enter__()
+            if len(scopes) == 2:
+                try:
+                    scopes[1].__enter__()
+                except BaseException:
+                    scopes[0].__exit__(*sys.exc_info())
+                    raise
+        self._open.append(scopes)
+
+    def __exit__(self, *exc) -> None:
+        scopes = self._open.pop()
+        try:
+            if len(scopes) == 2:
+                scopes[1].__exit__(*exc)
+        finally:
+            if scopes:
+                scopes[0].__exit__(*exc)
+
+
+def autocast_scopes(device: torch.device, fp8_recipe: FP8Recipe | None, enabled: bool, dtype: torch.dtype | None) -> tuple:
+    if not enabled:
+        return ()
+    inner = torch.autocast(device.type, dtype=torch.bfloat16 if dtype is None else dtype, enabled=True)
+    return (fp8_recipe.autocast(), inner) if fp8_recipe is not None and device.type == "cuda" else (inner,)
+
+
+class _Fp8Autocast(NestedScopes):
+    _scopes = staticmethod(autocast_scopes)
+
+
+class _Fp8Backward(NestedScopes):
+    def _scopes(self, fp8_recipe, enabled):
+        return (fp8_recipe.backward(),) if enabled and fp8_recipe is not None else ()
+
+
 def fp8_autocast(device: torch.device, fp8_recipe: FP8Recipe | None, enabled: bool = True,
-                 dtype: torch.dtype | None = None) -> Iterator[None]:
+                 dtype: torch.dtype | None = None) -> ContextDecorator:
     """FP8 autocast outside, ordinary AMP autocast inside (for everything that is
     not an FP8 Linear); plain AMP when there is no recipe or no GPU."""
-    if not enabled:
-        yield
-        return
-    if dtype is None:
-        dtype = torch.bfloat16
-    if fp8_recipe is not None and device.type == "cuda":
-        with fp8_recipe.autocast():
-            with torch.autocast(device.type, dtype=dtype, enabled=True):
-                yield
-    else:
-        with torch.autocast(device.type, dtype=dtype, enabled=True):
-            yield
+    return _Fp8Autocast(device, fp8_recipe, enabled, dtype)
 
 
-@contextmanager
-def fp8_backward(fp8_recipe: FP8Recipe | None, enabled: bool = True) -> Iterator[None]:
-    if not enabled or fp8_recipe is None:
-        yield
-        return
-    with fp8_recipe.backward():
-        yield
+def fp8_backward(fp8_recipe: FP8Recipe | None, enabled: bool = True) -> ContextDecorator:
+    return _Fp8Backward(fp8_recipe, enabled)

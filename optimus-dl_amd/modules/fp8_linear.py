@@ -882,10 +882,13 @@ class FP8Linear(nn.Linear):
 
     # ------------------------------------------------------------------ forward
     def _fp8_eligible(self, x: torch.Tensor) -> bool:
-        if not self.fp8_enabled or not x.is_cuda or not self.weight.is_cuda:
+        if not self.fp8_enabled or not x.is_cuda:
             return False
-        if self.weight.dtype not in (torch.bfloat16, torch.float32):
-            _warn_once(f"FP8Linear: weight dtype {self.weight.dtype} is not bf16/fp32; running as a plain Linear")
+        weight = self.weight                 # (nn.Module.__getattr__ costs a third of a microsecond)
+        if not weight.is_cuda:
+            return False
+        if weight.dtype not in (torch.bfloat16, torch.float32):
+            _warn_once(f"FP8Linear: weight dtype {weight.dtype} is not bf16/fp32; running as a plain Linear")
             return False
         tokens = x.numel() // max(self.in_features, 1)
         recipe = _state.active_recipe()

@@ -162,7 +162,7 @@ _any_global_hook = getattr(torch.nn.modules.module, "_has_any_global_hook", None
 
 def _runs_as_written(m: FP8Linear) -> bool:
     """Nothing looks at this Linear's input, output or their gradients, and nothing stands in for its forward."""
-    return (type(m) is FP8Linear and m.fp8_enabled and m.bias is None and "forward" not in m.__dict__
+    return (type(m) is FP8Linear and m.fp8_enabled and m._parameters.get("bias", m) is None and "forward" not in m.__dict__
             and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
 
 
@@ -217,7 +217,8 @@ def swiglu_few_rows(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
         return None
     if (torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype) != torch.bfloat16:
         return None
-    if not (w1._fp8_eligible(x) and w2._fp8_eligible(x)):
+    w2_weight = w2.weight
+    if not w1._fp8_eligible(x) or not w2_weight.is_cuda or w2_weight.dtype not in (torch.bfloat16, torch.float32):
         return None
     x2d = x.reshape(-1, k)
     if x2d.dtype != torch.bfloat16 or not x2d.is_contiguous():
@@ -227,10 +228,10 @@ def swiglu_few_rows(mlp: nn.Module, x: torch.Tensor) -> torch.Tensor | None:
     xq, _, _, _, sx_inv = (native.quantise_small(x2d, pol.fmt_fwd, pol.margin) if parts is None
                            else native.cast_dynamic(x2d, parts, pol.fmt_fwd, pol.margin, want_transposed=False))
     codes = []
-    for m in (w1, w2):
+    for m, weight in ((w1, w1.weight), (w2, w2_weight)):
         m.__dict__["fp8_calls"] += 1
         m._note_grad_mode()
-        codes.append(m._tensor_weight(m.weight, recipe, need_t=recipe.cache_weights and x2d.requires_grad))
+        codes.append(m._tensor_weight(weight, recipe, need_t=recipe.cache_weights and x2d.requires_grad))
     (g, _, sg_inv), (u, _, su_inv) = codes
     h, parts = native.gemm_swiglu(xq, g, u, pol.fmt_fwd, pol.fmt_fwd, sx_inv, sg_inv, su_inv)
     h = h.reshape(*x.shape[:-1], w1.out_features)

@@ -117,7 +117,7 @@ class NativeError(RuntimeError):
 
 
 def is_built() -> bool:
-    return os.path.exists(LIB_PATH)
+    return _lib is not None or os.path.exists(LIB_PATH)
 
 
 def load() -> ctypes.CDLL:

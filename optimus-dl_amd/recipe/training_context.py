@@ -15,7 +15,7 @@ scales the training steps measured.
 from __future__ import annotations
 
 import logging
-from contextlib import contextmanager, nullcontext
+from contextlib import nullcontext
 from typing import Any
 
 import torch
@@ -23,6 +23,8 @@ import torch
 from ..core.dtype import get_fp8_format_from_dtype, is_fp8_dtype, str_to_dtype
 from ..modules.amp.fp8 import (
     FP8Recipe,
+    NestedScopes,
+    autocast_scopes,
     create_fp8_recipe,
     fp8_autocast,
     is_transformer_engine_available,
@@ -169,19 +171,21 @@ def _eval_recipe(f) -> FP8Recipe | None:
     return recipe
 
 
-@contextmanager
+class _ForwardContext(NestedScopes):
+    def _scopes(self, amp_cfg, device):
+        if not amp_cfg.enabled:
+            return ()
+        dtype = str_to_dtype(amp_cfg.dtype)
+        is_fp8 = is_fp8_dtype(dtype)
+        recipe = None
+        if is_fp8 and getattr(amp_cfg, "fp8", None) and amp_cfg.fp8.enabled and is_transformer_engine_available():
+            recipe = _eval_recipe(amp_cfg.fp8)
+        return autocast_scopes(device, recipe, True, torch.bfloat16 if is_fp8 else dtype)
+
+
 def forward_context(amp_cfg: AmpConfig, device: torch.device):
     """Evaluation forward (evaluation_manager.py:98-144): nothing when AMP is off; FP8 autocast with bf16
     inside when the AMP dtype is an FP8 dtype, ``fp8.enabled`` is set and the backend is there; ordinary
     autocast otherwise (bf16 standing in for an FP8 dtype).  Modules in eval mode use the delayed-scaling
     scales that training measured and leave the amax histories alone."""
-    if not amp_cfg.enabled:
-        yield
-        return
-    dtype = str_to_dtype(amp_cfg.dtype)
-    is_fp8 = is_fp8_dtype(dtype)
-    recipe = None
-    if is_fp8 and getattr(amp_cfg, "fp8", None) and amp_cfg.fp8.enabled and is_transformer_engine_available():
-        recipe = _eval_recipe(amp_cfg.fp8)
-    with fp8_autocast(device=device, fp8_recipe=recipe, enabled=True, dtype=torch.bfloat16 if is_fp8 else dtype):
-        yield
+    return _ForwardContext(amp_cfg, device)
