@@ -969,7 +969,9 @@ __global__ __launch_bounds__(kThreads) void cast_rowcol_kernel(const void *__res
     const int ty = threadIdx.x / 8;                 // 32 lane-rows, 4 rows each
     const int64_t tiles_c = (cols + kTileC - 1) / kTileC;
     int64_t tr, tc;
-    ct_tile_of(blockIdx.x, (rows_out + kTileR - 1) / kTileR, tiles_c, tr, tc);
+    // from the end on, which the pass that found the maxima left in the memory-side cache: both, 16384 x 14336 295 -> 276 us,
+    // 8192 x 28672 299 -> 292, 8192 x 4096 and below the same
+    ct_tile_of(gridDim.x - 1 - blockIdx.x, (rows_out + kTileR - 1) / kTileR, tiles_c, tr, tc);
     if (threadIdx.x < kTileR) {
         const int64_t r = tr * kTileR + threadIdx.x;
         const float sc = r < rows ? scale_rule(amax_row[r], Fp8Lim<FMT>::max, margin, 1.0f) : 1.0f;
