@@ -46,7 +46,7 @@ enum odl_status {
 };
 
 /* ABI version of this header; bumped when a signature changes or an entry point is added. */
-#define ODL_FP8_ABI_VERSION 27
+#define ODL_FP8_ABI_VERSION 28
 int odl_fp8_abi_version(void);
 
 /*
@@ -127,6 +127,11 @@ int odl_fp8_cast_dynamic_padded(const void *x, int src_dtype, int64_t rows, int6
 int odl_fp8_cast_delayed_padded(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out,
                                 const float *scale, int fmt, uint8_t *out, uint8_t *out_t, float *amax_parts,
                                 float *scale_inv_out, odl_stream_t stream);
+/* odl_fp8_cast_delayed_padded in both layouts for 1 to 4 scales at once (arrays on the host, of pointers on the device), x read once;
+ * cols a multiple of 8, rows_out of 16, x and out_t 16-byte aligned; a partial maximum may land in another entry of a strip. */
+int odl_fp8_cast_delayed_many(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, int count, const float *const *scale,
+                              int fmt, uint8_t *const *out, uint8_t *const *out_t, float *const *amax_parts, float *const *scale_inv_out,
+                              odl_stream_t stream);
 int odl_fp8_cast_rowcol_padded(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out,
                                const float *amax_row, const float *amax_col, int fmt, int margin, uint8_t *out,
                                uint8_t *out_t, float *s_row, float *s_row_inv, float *s_col, float *s_col_inv,

@@ -26,6 +26,7 @@ decltype(&odl_fp8_cast_dynamic_padded) cast_dynamic_c;
 decltype(&odl_fp8_quantise_small) quantise_small_c;
 decltype(&odl_fp8_gemm_swiglu) gemm_swiglu_c;
 decltype(&odl_fp8_cast_delayed_padded) cast_delayed_c;
+decltype(&odl_fp8_cast_delayed_many) cast_delayed_many_c;
 decltype(&odl_fp8_amax_parts_colsum) amax_colsum_c;
 decltype(&odl_fp8_amax_parts_slabs) amax_slabs_c;
 decltype(&odl_fp8_cast_dynamic_colsum) cast_colsum_c;
@@ -60,6 +61,7 @@ void bind(const py::dict &d) {
     take(quantise_small_c, d, "odl_fp8_quantise_small");
     take(gemm_swiglu_c, d, "odl_fp8_gemm_swiglu");
     take(cast_delayed_c, d, "odl_fp8_cast_delayed_padded");
+    take(cast_delayed_many_c, d, "odl_fp8_cast_delayed_many");
     take(amax_colsum_c, d, "odl_fp8_amax_parts_colsum");
     take(amax_slabs_c, d, "odl_fp8_amax_parts_slabs");
     take(cast_colsum_c, d, "odl_fp8_cast_dynamic_colsum");
@@ -175,6 +177,25 @@ py::object cast_delayed(const Tensor &x, const Tensor &scale, int fmt, const Opt
     Tensor inv = f32(x, {1});
     const int rc = call(cast_delayed_c, ptr(x), src_of(x), rows, cols, n, ptr(scale), fmt, ptr(q), ptr(q_t), ptr(parts), ptr(inv), str(stream));
     return rc ? status(rc) : py::make_tuple(obj(q), obj(q_t), inv);
+}
+
+py::object cast_delayed_many(const Tensor &x, const std::vector<Tensor> &scales, int fmt, const std::vector<Tensor> &parts, i64 rows_out, i64 stream) {
+    const size_t n = scales.size();
+    if (n < 1 || n > 4 || parts.size() != n || !source2d(x) || x.numel() == 0 || x.size(1) % 8 || rows_out % 16 || rows_out < x.size(0) || !aligned(x))
+        return none();
+    const float *s[4];
+    float *p[4], *inv[4];
+    uint8_t *q[4], *q_t[4];
+    py::list made(n);
+    Tensor invs = f32(x, {(i64)n});
+    for (size_t i = 0; i < n; ++i) {
+        if (!floats(scales[i], 1) || !floats(parts[i], kParts)) return none();
+        Tensor a = bytes(x, {rows_out, x.size(1)}), b = bytes(x, {x.size(1), rows_out});
+        s[i] = ptr(scales[i]), p[i] = ptr(parts[i]), inv[i] = static_cast<float *>(ptr(invs)) + i, q[i] = ptr(a), q_t[i] = ptr(b);
+        made[i] = py::make_tuple(a, b, invs.narrow(0, (i64)i, 1));
+    }
+    const int rc = call(cast_delayed_many_c, ptr(x), src_of(x), x.size(0), x.size(1), rows_out, (int)n, s, fmt, q, q_t, p, inv, str(stream));
+    return rc ? status(rc) : py::object(made);
 }
 
 py::object amax_colsum(const Tensor &x, bool finish, i64 stream) {
@@ -450,6 +471,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("quantise_small", &quantise_small);
     m.def("gemm_swiglu", &gemm_swiglu);
     m.def("cast_delayed", &cast_delayed);
+    m.def("cast_delayed_many", &cast_delayed_many);
     m.def("amax_colsum", &amax_colsum);
     m.def("cast_colsum", &cast_colsum);
     m.def("swiglu", &swiglu);

@@ -207,6 +207,20 @@ def _quantise_delayed(x2d: torch.Tensor, fmt: int, meta: "_state.ScalingMeta | N
                                want_transposed=need_t, out_t=out_t, rows_out=rows_out)
 
 
+def _quantise_delayed_for_all(recipe: FP8Recipe, x2d: torch.Tensor, modules, need_wgrad) -> list:
+    """Delayed scaling: the codes of x for Linears that are fed this one tensor, each with the scale of its own history, or None for each
+    that casts x by itself.  One launch reads x for all of them: 8192 x 4096 for q, k
+    and v 77.0 -> 48.5 us, 8192 x 1024 for gate and up 19.4 -> 12.4."""
+    pol = recipe.recipe
+    if pol.kind != "delayed" or not recipe.wgrad or not 2 <= len(modules) <= 4 or not all(need_wgrad) or not all(m._records() for m in modules):
+        return [None] * len(modules)
+    metas = [m._meta(recipe, x2d.device, "fwd", create=True) for m in modules]
+    for meta in metas:
+        meta.note_record(recipe._store)
+    return native.cast_delayed_many(x2d, [meta.scale_of(ROLE_X) for meta in metas], pol.fmt_fwd, [meta.amax_slot(ROLE_X) for meta in metas],
+                                    native.padded_rows(x2d.shape[0]))
+
+
 def _rows(codes: torch.Tensor, n: int) -> torch.Tensor:
     """The first n rows of codes that were cast with padding behind them."""
     return codes if codes.shape[0] == n else codes[:n]
@@ -503,16 +517,17 @@ class _Fp8LinearGroupFn(torch.autograd.Function):
         ctx.set_materialize_grads(False)         # an output that did not reach the loss arrives as None, not as zeros
         subs, outs, saved, spans = [], [], [], []
         jobs = _product_jobs(recipe, modules)
+        given = _quantise_delayed_for_all(recipe, x2d, modules, ctx.needs_input_grad[4::2])
         for i, mod in enumerate(modules):
             weight, bias = params[2 * i], params[2 * i + 1]
             sub = _MemberCtx((ctx.needs_input_grad[0], ctx.needs_input_grad[4 + 2 * i], ctx.needs_input_grad[5 + 2 * i],
                               False, False, False))
-            sub.y_jobs = jobs
+            sub.y_jobs, sub.given_input = jobs, given[i]
             outs.append(_Fp8LinearFn.forward(sub, x2d, weight, bias, mod, recipe, out_dtype))
             spans.append((len(saved), len(sub.saved_tensors)))
             saved.extend(sub.saved_tensors)
             sub.saved_tensors = ()
-            sub.y_jobs = None
+            sub.y_jobs = sub.given_input = None
             subs.append(sub)
         if jobs is not None:
             outs = _run_jobs(jobs, recipe.recipe.fmt_fwd, recipe.recipe.fmt_fwd, out_dtype, fresh=True)

@@ -24,7 +24,7 @@ from .amp import state as _state
 from .amp.fp8 import FP8Recipe
 from .calls import apply, no_graph, untraced
 from .fp8_linear import (ROLE_G, ROLE_X, FP8Linear, _converted_input, _Fp8LinearFn, _Fp8LinearGroupFn, _MemberCtx, _product_jobs,
-                         _run_jobs, _wgrad_jobs)
+                         _quantise_delayed_for_all, _run_jobs, _wgrad_jobs)
 
 
 def _bf16_cuda(*tensors: torch.Tensor) -> bool:
@@ -95,7 +95,9 @@ class _SwiGLUMLPFn(torch.autograd.Function):
 
         w1, w2, down = modules
         jobs = _product_jobs(recipe, (w1, w2))
-        gate, up = (member(x2d, w, weight, ctx.needs_input_grad[0], jobs=jobs) for w, weight in ((w1, weights[0]), (w2, weights[1])))
+        given = _quantise_delayed_for_all(recipe, x2d, (w1, w2), (True, True))
+        gate, up = (member(x2d, w, weight, ctx.needs_input_grad[0], given=g, jobs=jobs)
+                    for w, weight, g in ((w1, weights[0], given[0]), (w2, weights[1], given[1])))
         if jobs is not None:
             gate, up = _run_jobs(jobs, pol.fmt_fwd, pol.fmt_fwd, torch.bfloat16, fresh=True)
         if pol.kind == "mxfp8":

@@ -26,7 +26,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 27
+ABI_VERSION = 28
 _OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
@@ -56,6 +56,7 @@ EXPORTS = (
     "odl_fp8_multi_cast_delayed",
     "odl_fp8_amax_parts_colsum",
     "odl_fp8_amax_parts_slabs",
+    "odl_fp8_cast_delayed_many",
     "odl_fp8_cast_dynamic_colsum",
     "odl_fp8_swiglu_amax_parts",
     "odl_fp8_swiglu_bwd_amax_parts",
@@ -155,6 +156,7 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_multi_amax_parts.argtypes = [vp, vp, i64, vp]
         L.odl_fp8_multi_cast_dynamic.argtypes = [vp, vp, i64, i32, i32, vp]
         L.odl_fp8_multi_cast_delayed.argtypes = [vp, vp, i64, i32, vp]
+        L.odl_fp8_cast_delayed_many.argtypes = [vp, i32, i64, i64, i64, i32, vp, i32, vp, vp, vp, vp, vp]
         L.odl_fp8_amax_parts_slabs.argtypes = [vp, i32, i64, i64, vp, vp, vp]
         L.odl_fp8_cast_dynamic_colsum.argtypes = [vp, i32, i64, i64, i64, vp, i32, i32, vp, vp, vp, vp, vp, i32, vp]
         L.odl_fp8_amax_parts_colsum.argtypes = [vp, i32, i64, i64, vp, vp, vp, vp]
@@ -920,6 +922,17 @@ def cast_transpose(x: torch.Tensor, scale: torch.Tensor, fmt: int, mode: int = S
                                                 amax_out.data_ptr() if amax_out is not None else None, _stream()),
            "odl_fp8_cast_transpose")
     return out, out_t
+
+
+def cast_delayed_many(x: torch.Tensor, scales: "list[torch.Tensor]", fmt: int, amax_parts: "list[torch.Tensor]", rows_out: int) -> list:
+    """``[cast_delayed(x, s, fmt, p, want_transposed=True, rows_out=rows_out) for s, p in zip(scales, amax_parts)]``, in one launch that
+    reads x once where x has whole vectors."""
+    if x.is_cuda:
+        load()
+        r = _host.cast_delayed_many(x, scales, fmt, amax_parts, rows_out, _stream())
+        if r is not None:
+            return _done(r, "odl_fp8_cast_delayed_many")
+    return [cast_delayed(x, s, fmt, p, want_transposed=True, rows_out=rows_out) for s, p in zip(scales, amax_parts, strict=True)]
 
 
 def cast_delayed(x: torch.Tensor, scale: torch.Tensor, fmt: int, amax_parts: torch.Tensor | None = None,
