@@ -211,8 +211,8 @@ def _quantise_delayed_for_all(recipe: FP8Recipe, x2d: torch.Tensor, modules, nee
     """Delayed scaling: the codes of x for Linears that are fed this one tensor, each with the scale of its own history, or None for each
     that casts x by itself.  One launch reads x for all of them: 8192 x 4096 for q, k
     and v 77.0 -> 48.5 us, 8192 x 1024 for gate and up 19.4 -> 12.4."""
-    pol = recipe.recipe
-    if pol.kind != "delayed" or not recipe.wgrad or not 2 <= len(modules) <= 4 or not all(need_wgrad) or not all(m._records() for m in modules):
+    pol = recipe.recipe if 2 <= len(modules) <= 4 else None
+    if pol is None or pol.kind != "delayed" or not recipe.wgrad or not all(need_wgrad) or not all(m._records() for m in modules):
         return [None] * len(modules)
     metas = [m._meta(recipe, x2d.device, "fwd", create=True) for m in modules]
     for meta in metas:
