@@ -1197,8 +1197,8 @@ extern "C" int odl_fp8_cast_dynamic_colsum(const void *x, int src_dtype, int64_t
         return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic_colsum: src_dtype %d, colsum_dtype %d", src_dtype, colsum_dtype);
     if (fmt != ODL_FP8_E4M3 && fmt != ODL_FP8_E5M2) return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic_colsum: fmt %d", fmt);
     if (margin < -64 || margin > 64) return set_error(ODL_ERR_ARG, "odl_fp8_cast_dynamic_colsum: margin %d", margin);
-    if (!cast_colsum_takes(x, rows, cols, rows_out, out, out_t) || (cols + 255) / 256 > kParts)
-        return set_error(ODL_ERR_SHAPE, "odl_fp8_cast_dynamic_colsum: both layouts, columns in multiples of 8, rows out of 16, 16-byte alignment");
+    if (!cast_colsum_takes(x, rows, cols, rows_out, out, out_t) || cols > (int64_t)kParts * 32 * (src_dtype == ODL_BF16 ? 8 : 4))
+        return set_error(ODL_ERR_SHAPE, "odl_fp8_cast_dynamic_colsum: both layouts, columns in multiples of 8 (at most 131072, of fp32 65536), rows out of 16, 16-byte alignment");
     int64_t slabs;
     colsum_slab_rows(src_dtype, rows, cols, &slabs);
     launch_cast_colsum(x, src_dtype, rows, cols, rows_out, parts, fmt, margin, out, out_t, dyn_out, workspace, (int)slabs, colsum, colsum_dtype,

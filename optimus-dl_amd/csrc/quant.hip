@@ -940,10 +940,11 @@ __global__ __launch_bounds__(kThreads) void cast_transpose_kernel(const void *__
 // amax, scale and cast by blocks that each read the whole tensor (16 pieces of 16 bytes a lane at most), find the same maximum, and
 // cast one piece per lane each.  Bound by what one compute unit reads, 60 - 70 bytes a nanosecond; nobody waits for another block, and
 // it spares a launch (32 x 4096 bf16: 3.5 + 4.4 us and a launch of 4 us; one block that casts everything 9.0, of which the
-// conversions were 5; here 7.0).  Whole pieces, x and out 16-byte aligned, not the same memory.
+// conversions were 5; here 7.0).  Whole pieces, x and out 16-byte aligned.
 constexpr int kSmallPieces = ODL_FP8_SMALL_BYTES / 16 / kFatThreads;
-template <int SRC, int FMT>
-__global__ __launch_bounds__(kFatThreads) void quantise_small_kernel(const void *__restrict__ x, int pieces, int margin, uint8_t *__restrict__ out,
+// ONE: by one block, which has read all of x before it writes (out may then overlap x).
+template <int SRC, int FMT, bool ONE>
+__global__ __launch_bounds__(kFatThreads) void quantise_small_kernel(const void *x, int pieces, int margin, uint8_t *out,
                                                                      float *__restrict__ dyn_out) {
     __shared__ uint32_t red[kFatThreads / kWave];
     __shared__ float scale;
@@ -978,13 +979,20 @@ __global__ __launch_bounds__(kFatThreads) void quantise_small_kernel(const void 
     }
     __syncthreads();
     const float s = scale;
-    const int i = (int)blockIdx.x * kFatThreads + (int)threadIdx.x;
-    if (i >= pieces) return;
-    const uint32_t w[4] = {own.x, own.y, own.z, own.w};
-    if constexpr (SRC == ODL_BF16)
-        reinterpret_cast<u32x2 *>(out)[i] = u32x2{quantise4<FMT>(bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1]), s, s, s, s),
-                                                  quantise4<FMT>(bf16_lo(w[2]), bf16_hi(w[2]), bf16_lo(w[3]), bf16_hi(w[3]), s, s, s, s)};
-    else reinterpret_cast<uint32_t *>(out)[i] = quantise4<FMT>(bits_to_float(w[0]), bits_to_float(w[1]), bits_to_float(w[2]), bits_to_float(w[3]), s, s, s, s);
+    auto write = [&](const u32x4 piece, int i) {
+        if (i >= pieces) return;
+        const uint32_t w[4] = {piece.x, piece.y, piece.z, piece.w};
+        if constexpr (SRC == ODL_BF16)
+            reinterpret_cast<u32x2 *>(out)[i] = u32x2{quantise4<FMT>(bf16_lo(w[0]), bf16_hi(w[0]), bf16_lo(w[1]), bf16_hi(w[1]), s, s, s, s),
+                                                      quantise4<FMT>(bf16_lo(w[2]), bf16_hi(w[2]), bf16_lo(w[3]), bf16_hi(w[3]), s, s, s, s)};
+        else reinterpret_cast<uint32_t *>(out)[i] = quantise4<FMT>(bits_to_float(w[0]), bits_to_float(w[1]), bits_to_float(w[2]), bits_to_float(w[3]), s, s, s, s);
+    };
+    if constexpr (ONE) {
+#pragma unroll
+        for (int j = 0; j < kSmallPieces; ++j) write(v[j], j * kFatThreads + (int)threadIdx.x);
+    } else {
+        write(own, (int)blockIdx.x * kFatThreads + (int)threadIdx.x);
+    }
 }
 
 // ----------------------------------------------------------------- host helpers
@@ -1412,9 +1420,15 @@ extern "C" int odl_fp8_quantise_small(const void *x, int src_dtype, int64_t n, i
     if (!dyn_out || (n > 0 && (!x || !out))) return set_error(ODL_ERR_ARG, "odl_fp8_quantise_small: null pointer");
     if (!aligned16(x) || !aligned16(out)) return set_error(ODL_ERR_SHAPE, "odl_fp8_quantise_small: x and out must be 16-byte aligned");
     const int pieces = (int)(n * esz / 16), blocks = pieces > 0 ? (pieces + kFatThreads - 1) / kFatThreads : 1;
-#define ODL_SMALL(S, F) hipLaunchKernelGGL((quantise_small_kernel<S, F>), dim3((unsigned)blocks), dim3(kFatThreads), 0, stream, x, pieces, margin, out, dyn_out)
-    if (src_dtype == ODL_BF16) { if (fmt == ODL_FP8_E4M3) ODL_SMALL(ODL_BF16, ODL_FP8_E4M3); else ODL_SMALL(ODL_BF16, ODL_FP8_E5M2); }
-    else { if (fmt == ODL_FP8_E4M3) ODL_SMALL(ODL_F32, ODL_FP8_E4M3); else ODL_SMALL(ODL_F32, ODL_FP8_E5M2); }
+    const uintptr_t from = reinterpret_cast<uintptr_t>(x), to = reinterpret_cast<uintptr_t>(out);
+    const bool overlap = from < to + (uintptr_t)n && to < from + (uintptr_t)(n * esz);
+#define ODL_SMALL(S, F)                                                                                                                             \
+    if (overlap) hipLaunchKernelGGL((quantise_small_kernel<S, F, true>), dim3(1), dim3(kFatThreads), 0, stream, x, pieces, margin, out, dyn_out); \
+    else hipLaunchKernelGGL((quantise_small_kernel<S, F, false>), dim3((unsigned)blocks), dim3(kFatThreads), 0, stream, x, pieces, margin, out, dyn_out)
+    if (src_dtype == ODL_BF16 && fmt == ODL_FP8_E4M3) { ODL_SMALL(ODL_BF16, ODL_FP8_E4M3); }
+    else if (src_dtype == ODL_BF16) { ODL_SMALL(ODL_BF16, ODL_FP8_E5M2); }
+    else if (fmt == ODL_FP8_E4M3) { ODL_SMALL(ODL_F32, ODL_FP8_E4M3); }
+    else { ODL_SMALL(ODL_F32, ODL_FP8_E5M2); }
 #undef ODL_SMALL
     return check_launch("odl_fp8_quantise_small");
 }

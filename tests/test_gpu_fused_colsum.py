@@ -83,3 +83,16 @@ def test_slabs_are_not_handed_to_a_view_of_other_columns():
     recipe.offer_parts(t.view(2, 32, 32), parts, slabs)
     got = recipe.take_parts_and_slabs(t)
     assert got[0] is parts and got[1] is slabs
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [16, 16384, 48016])
+def test_small_tensor_quantised_in_its_own_place(n, dtype):
+    """Codes over the first bytes of x: the launch of one block, which reads everything first."""
+    from optimus_dl_amd import native as N
+
+    x = torch.randn((1, n), device="cuda").to(dtype)
+    want, _, _, _, inv = N.quantise_small(x, O.E4M3)
+    dyn, L = torch.empty(3, device="cuda"), N.load()
+    assert L.odl_fp8_quantise_small(x.data_ptr(), 0 if dtype == torch.bfloat16 else 1, n, O.E4M3, 0, x.data_ptr(), dyn.data_ptr(), N._stream()) == 0
+    assert torch.equal(x.view(torch.uint8).reshape(-1)[:n], want.reshape(-1)) and dyn[2].item() == inv.item()
