@@ -1056,6 +1056,17 @@ extern "C" int odl_fp8_swiglu_bwd_amax_parts(const void *dh, const void *gate, c
     return check_launch("odl_fp8_swiglu_bwd_amax_parts");
 }
 
+// Lanes of a block of the norms' forward kernels: the widest block of which there are `enough`, else narrower ones, four waves at least.
+// A row is a chain of a load, a reduction and a store; in wide blocks few rows leave units idle.  RMSNorm gains until there are two
+// blocks for every unit (grid_cap()), us, 1024 lanes / here: 8192 x 1024 fp32 18.0 / 12.9 (128 blocks before), 4016 x 2048 18.0 / 12.7, 512 x 768
+// 10.1 / 4.7, 4096 x 1024 bf16 8.9 / 7.0.  LayerNorm, whose two reductions want the waves of a wide block, only where those would fill
+// a third of that: 4096 x 768 fp32 9.2 / 7.5, 2048 x 2048 11.0 / 8.9, but with two blocks for every unit 4016 x 2048 bf16 9.3 / 11.7.
+static int norm_threads(int64_t rows, int rows_per_wave, int widest, int enough) {
+    int t = widest;
+    while (t > 256 && (rows + (t / kWave) * rows_per_wave - 1) / ((t / kWave) * rows_per_wave) < enough) t /= 2;
+    return t;
+}
+
 extern "C" int odl_fp8_rmsnorm_amax_parts(const void *x, int src_dtype, const float *weight, int64_t rows, int64_t cols, float eps,
                                           void *y, float *rstd, float *parts, odl_stream_t stream_) {
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
@@ -1082,17 +1093,21 @@ extern "C" int odl_fp8_rmsnorm_amax_parts(const void *x, int src_dtype, const fl
     // fp32 rows of 5 .. 8 chunks a lane (64 registers of input per row) allow four waves per SIMD: as 1024-lane blocks that
     // is one block per compute unit, which reads, then writes, then makes room for the next; two 512-lane blocks per unit
     // overlap one's stores with the other's loads (8192 x 4096: 43.4 -> 40.4 us; bf16 rows measured no difference)
-    const int threads = cpl <= 4 ? kFusedThreads : (cpl <= 8 ? (src_dtype == ODL_BF16 ? kFusedThreads : 512) : 256);
-    const int rows_per_block = (threads / kWave) * (cpl <= 2 ? 4 : (cpl <= 4 ? 2 : 1));   // RB rows per wave and trip
+    const int per_wave = cpl <= 2 ? 4 : (cpl <= 4 ? 2 : 1);   // rows per wave and trip
+    const int threads = norm_threads(rows, per_wave, cpl <= 8 ? (cpl > 4 && src_dtype == ODL_F32 ? 512 : kFusedThreads) : 256, grid_cap());
+    const int rows_per_block = (threads / kWave) * per_wave;
     int64_t g = (rows + rows_per_block - 1) / rows_per_block;
     g = g < 1 ? 1 : (g < grid_cap() ? g : grid_cap());
 #define ODL_RMS(SRC, CPL, THR) hipLaunchKernelGGL((rmsnorm_fwd_kernel<SRC, CPL, THR>), dim3((unsigned)g), dim3(THR), 0, stream, x, weight, rows, cols, eps, reinterpret_cast<uint16_t *>(y), rstd, parts)
 #define ODL_RMS_SRC(CPL, THR) do { if (src_dtype == ODL_BF16) ODL_RMS(ODL_BF16, CPL, THR); else ODL_RMS(ODL_F32, CPL, THR); } while (0)
-    if (cpl <= 2) ODL_RMS_SRC(2, kFusedThreads);
-    else if (cpl <= 4) ODL_RMS_SRC(4, kFusedThreads);
-    else if (cpl <= 8 && src_dtype == ODL_BF16) ODL_RMS(ODL_BF16, 8, kFusedThreads);
-    else if (cpl <= 8) ODL_RMS(ODL_F32, 8, 512);
-    else ODL_RMS_SRC(16, 256);
+#define ODL_RMS_THR(CPL) do { if (threads == 256) ODL_RMS_SRC(CPL, 256); else if (threads == 512) ODL_RMS_SRC(CPL, 512); else ODL_RMS_SRC(CPL, kFusedThreads); } while (0)
+    if (cpl <= 2) ODL_RMS_THR(2);
+    else if (cpl <= 4) ODL_RMS_THR(4);
+    else if (cpl > 8) ODL_RMS_SRC(16, 256);
+    else if (threads == 256) ODL_RMS_SRC(8, 256);
+    else if (threads == 512) ODL_RMS_SRC(8, 512);
+    else ODL_RMS(ODL_BF16, 8, kFusedThreads);
+#undef ODL_RMS_THR
 #undef ODL_RMS_SRC
 #undef ODL_RMS
     return check_launch("odl_fp8_rmsnorm_amax_parts");
@@ -1217,15 +1232,18 @@ extern "C" int odl_fp8_layernorm_amax_parts(const void *x, int src_dtype, const 
     if (cols < 8 || cols % 8 != 0 || cols > 4096 || !aligned16(x) || !aligned16(y) || !aligned16(weight) || !aligned16(bias))
         return set_error(ODL_ERR_SHAPE, "odl_fp8_layernorm_amax_parts: cols must be a multiple of 8 in [8, 4096] and the pointers 16-byte aligned");
     const int64_t cpl = (cols / 8 + kWave - 1) / kWave;
-    const int threads = cpl <= 4 ? kFusedThreads : 512;     // wider rows need more than the 128 registers of a 1024-lane block
-    const int rows_per_block = (threads / kWave) * (cpl <= 2 ? 2 : 1);   // RB rows per wave and trip
+    const int per_wave = cpl <= 2 ? 2 : 1;                  // rows per wave and trip
+    const int threads = cpl <= 4 ? norm_threads(rows, per_wave, kFusedThreads, grid_cap() / 3) : 512;     // wider rows need more than the 128 registers of a 1024-lane block
+    const int rows_per_block = (threads / kWave) * per_wave;
     int64_t g = (rows + rows_per_block - 1) / rows_per_block;
     g = g < 1 ? 1 : (g < grid_cap() ? g : grid_cap());
 #define ODL_LN(SRC, CPL, THR) hipLaunchKernelGGL((layernorm_fwd_kernel<SRC, CPL, THR>), dim3((unsigned)g), dim3(THR), 0, stream, x, weight, bias, rows, cols, eps, reinterpret_cast<uint16_t *>(y), mean, rstd, parts)
 #define ODL_LN_SRC(CPL, THR) do { if (src_dtype == ODL_BF16) ODL_LN(ODL_BF16, CPL, THR); else ODL_LN(ODL_F32, CPL, THR); } while (0)
-    if (cpl <= 2) ODL_LN_SRC(2, kFusedThreads);
-    else if (cpl <= 4) ODL_LN_SRC(4, kFusedThreads);
+#define ODL_LN_THR(CPL) do { if (threads == 256) ODL_LN_SRC(CPL, 256); else if (threads == 512) ODL_LN_SRC(CPL, 512); else ODL_LN_SRC(CPL, kFusedThreads); } while (0)
+    if (cpl <= 2) ODL_LN_THR(2);
+    else if (cpl <= 4) ODL_LN_THR(4);
     else ODL_LN_SRC(8, 512);
+#undef ODL_LN_THR
 #undef ODL_LN_SRC
 #undef ODL_LN
     return check_launch("odl_fp8_layernorm_amax_parts");
