@@ -46,7 +46,7 @@ enum odl_status {
 };
 
 /* ABI version of this header; bumped when a signature changes or an entry point is added. */
-#define ODL_FP8_ABI_VERSION 28
+#define ODL_FP8_ABI_VERSION 29
 int odl_fp8_abi_version(void);
 
 /*
@@ -454,15 +454,13 @@ int odl_fp8_gemm_nt_group(int count, const uint8_t *const *a, const uint8_t *con
 /*
  * C[M, N] = the bf16 sum of up to four products with the roundings of one odl_fp8_gemm_nt per product, the second and later ones
  * with accumulate set, in one launch: the data gradient of Linears fed one tensor, where odl_fp8_gemm_nt_sum has no launch for it or
- * its single rounding is not wanted.  sa_inv, sb_inv: one scale per operand.  With mx_sa and mx_sb given (then sa_inv and sb_inv are
- * not read) the operands carry block scales, K-step-major as odl_fp8_mx_gemm_nt takes them, and the sum is rounded once.
- * Only where odl_fp8_gemm_chain_route (mx: block scales or not) gives a variant, that is where it is faster, for 2 to 4 products,
+ * its single rounding is not wanted.  sa_inv, sb_inv: one scale per operand.
+ * Only where odl_fp8_gemm_chain_route gives a variant, that is where it is faster, for 2 to 4 products,
  * every K[s] a multiple of 256 and at least 512, N a multiple of 128, M at least 32, operands under 2 GiB; refused otherwise.
  */
-int odl_fp8_gemm_chain_route(int pairs, const int64_t *K, int64_t M, int64_t N, int mx);
+int odl_fp8_gemm_chain_route(int pairs, const int64_t *K, int64_t M, int64_t N);
 int odl_fp8_gemm_nt_chain(int pairs, const uint8_t *const *a, const uint8_t *const *b, const int64_t *K, int64_t M, int64_t N, int fmt_a,
-                          int fmt_b, const float *const *sa_inv, const float *const *sb_inv, const uint8_t *const *mx_sa,
-                          const uint8_t *const *mx_sb, void *c, odl_stream_t stream);
+                          int fmt_b, const float *const *sa_inv, const float *const *sb_inv, void *c, odl_stream_t stream);
 
 /*
  * The same product for operands that need no transposed copy.  layout_a / layout_b say how an

@@ -44,7 +44,6 @@ struct GemmPairs {
     int k[4] = {0, 0, 0, 0};
     const uint8_t *a[4] = {nullptr, nullptr, nullptr, nullptr}, *b[4] = {nullptr, nullptr, nullptr, nullptr};
     const float *sa[4] = {nullptr, nullptr, nullptr, nullptr}, *sb[4] = {nullptr, nullptr, nullptr, nullptr};
-    const uint8_t *mx_sa[4] = {nullptr, nullptr, nullptr, nullptr}, *mx_sb[4] = {nullptr, nullptr, nullptr, nullptr};   // block scales (GemmArgs)
 };
 
 // Several products of one contraction length in one launch: the tiles of member s are [first[s], first[s + 1]) of the launch's.

@@ -707,17 +707,17 @@ static double accumulate_us(int variant, const TileCounts &t, int64_t steps, dou
 
 // The kernel for C = sum of products [M, K_s] . [N, K_s]^T in bf16, or kNoVariant: a launch each.
 //
-// Tensor scales: gemm_deep.h keeps the sum so far in registers and rounds it behind each product, as launches that accumulate do; us a
-// launch each / together:
+// gemm_deep.h keeps the sum so far in registers and rounds it behind each product, as launches that accumulate do; us a launch
+// each / together:
 //   8192 x 1024 x (3072, 3072) 65.8 / 53.7    4016 x 2048 x (5632, 5632) 98.8 / 86.6    1024 x 1024 x (1024, 512, 512) 20.0 / 14.2
 //   5744 x 4096 x (4096, 1024, 1024) 198 / 136 (three rounds of 256 x 128 tiles against the 256 x 256 kernels that accumulate)
 //   8192 x 4096 x (14336, 14336) 718 / 804, 256 x 4096 x (14336, 14336) (thin tiles) 64 / 83: launches of their own
 // The model: 0.85 us a step of 256 x 128 tiles (operands from memory, the chip full), a last round that leaves units idle faster.
 // Where the streaming kernel takes the sum with one rounding (odl_fp8_gemm_nt_sum) callers ask it first.
 //
-// Block scales: the streaming kernel, the contractions as one (8192 x 2048 x (5632, 5632) 172 / 133 with the addition of the two results,
-// 8192 x 4096 x (14336, 14336) 754 / 738), for outputs it would take anyway; the deep kernel with block scales gained nothing.
-static int chain_variant(int pairs, const int64_t *K, int64_t M, int64_t N, bool mx) {
+// Block scales have no such launch: their results are rounded one by one and added in bf16, and the streaming kernel, which could
+// take them as one contraction (8192 x 2048 x (5632, 5632) 133 us against 172), would round once, other results by 2.9e-3.
+static int chain_variant(int pairs, const int64_t *K, int64_t M, int64_t N) {
     if (pairs < 2 || pairs > 4 || M < 32 || N < 128 || N % 128 != 0) return kNoVariant;
     const int cus = cu_count();
     const TileCounts t(M, N);
@@ -731,20 +731,16 @@ static int chain_variant(int pairs, const int64_t *K, int64_t M, int64_t N, bool
         if (t_forced_variant >= 0) continue;
         if (odl_fp8_gemm_runs(M, N, K[s], 0) > 1) return kNoVariant;
         const int64_t steps = K[s] / 128;
-        const Route route = route_of(M, N, K[s], ODL_BF16, s > 0 && !mx, -1);
+        const Route route = route_of(M, N, K[s], ODL_BF16, s > 0, -1);
         if (route.variant == kThinVariant) apart += 4.0 + 0.0027 * gemm_thin_rows(M, N, cus) * (double)steps + (s > 0 ? 0.4 * c_mb : 0.0);
-        else apart += s > 0 && !mx ? accumulate_us(route.variant, t, steps, c_mb, cus) : launch_us(route.variant, t, steps, cus) + (s > 0 ? 3.0 + 0.6 * c_mb : 0.0);
+        else apart += s > 0 ? accumulate_us(route.variant, t, steps, c_mb, cus) : launch_us(route.variant, t, steps, cus);
     }
     if (t.t128 > 0x7ffffff0LL || (double)N * 2.0 * 264.0 >= 2147483648.0) return kNoVariant;
-    if (t_forced_variant >= 0) return mx ? (t_forced_variant == kStreamVariant ? kStreamVariant : kNoVariant) : t_forced_variant >= kDeepWideVariant ? t_forced_variant : kNoVariant;
+    if (t_forced_variant >= 0) return t_forced_variant >= kDeepWideVariant ? t_forced_variant : kNoVariant;
     const double steps = (double)(total / 128);
     int best = kNoVariant;
     double cost = 0.97 * apart;
     auto offer = [&](int variant, double us) { if (us < cost) { cost = us; best = variant; } };
-    if (mx) {
-        if (t.t256 * 2 > cus) offer(kStreamVariant, launch_us(kStreamVariant, t, total / 128, cus));
-        return best;
-    }
     if (t.t128 <= cus) offer(kDeepVariant, launch_us(kDeepVariant, t, total / 128, cus));
     if (t.t192 <= cus) offer(kDeep192Variant, launch_us(kDeep192Variant, t, total / 128, cus));
     const double rest = (double)(t.wide % cus) / cus;
@@ -752,53 +748,38 @@ static int chain_variant(int pairs, const int64_t *K, int64_t M, int64_t N, bool
     return best;
 }
 
-extern "C" int odl_fp8_gemm_chain_route(int pairs, const int64_t *K, int64_t M, int64_t N, int mx) {
+extern "C" int odl_fp8_gemm_chain_route(int pairs, const int64_t *K, int64_t M, int64_t N) {
     if (!K) {
         set_error(ODL_ERR_ARG, "odl_fp8_gemm_chain_route: null pointer");
         return -1;
     }
-    return chain_variant(pairs, K, M, N, mx != 0);
+    return chain_variant(pairs, K, M, N);
 }
 
 extern "C" int odl_fp8_gemm_nt_chain(int pairs, const uint8_t *const *a, const uint8_t *const *b, const int64_t *K, int64_t M, int64_t N, int fmt_a,
-                                     int fmt_b, const float *const *sa_inv, const float *const *sb_inv, const uint8_t *const *mx_sa,
-                                     const uint8_t *const *mx_sb, void *c, odl_stream_t stream_) {
+                                     int fmt_b, const float *const *sa_inv, const float *const *sb_inv, void *c, odl_stream_t stream_) {
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
-    const bool mx = mx_sa != nullptr;
-    if (!a || !b || !K || !c || mx != (mx_sb != nullptr) || (!mx && (!sa_inv || !sb_inv))) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt_chain: null pointer");
-    const int variant = chain_variant(pairs, K, M, N, mx);
+    if (!a || !b || !K || !c || !sa_inv || !sb_inv) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt_chain: null pointer");
+    const int variant = chain_variant(pairs, K, M, N);
     if (variant == kNoVariant)
         return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt_chain: %d products of %lld x %lld do not run in one launch (odl_fp8_gemm_chain_route)", pairs, (long long)M, (long long)N);
     if (fmt_b == ODL_FP8_E4M3 ? fmt_a != ODL_FP8_E4M3 && fmt_a != ODL_FP8_E5M2 : fmt_b != ODL_FP8_E5M2 || fmt_a != ODL_FP8_E5M2)
         return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt_chain: formats %d, %d", fmt_a, fmt_b);
     const int bm = kVariants[variant].bm, bn = kVariants[variant].bn;
-    // (the kernels apply no tensor scale to block-scaled products; a valid one stands where they would read it)
-    const float *one = mx ? unit_scale_for_current_device("odl_fp8_gemm_nt_chain") : nullptr;
-    if (mx && !one) return ODL_ERR_LAUNCH;
     GemmChain gc;
-    GemmPairs gp;
-    gc.count = gp.count = pairs;
+    gc.count = pairs;
     if (reinterpret_cast<uintptr_t>(c) & 15) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt_chain: output must be 16-byte aligned");
     for (int s = 0; s < pairs; ++s) {
-        if (!a[s] || !b[s] || (mx ? !mx_sa[s] || !mx_sb[s] : !sa_inv[s] || !sb_inv[s])) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt_chain: null pointer in product %d", s);
-        if ((reinterpret_cast<uintptr_t>(a[s]) & 15) || (reinterpret_cast<uintptr_t>(b[s]) & 15) ||
-            (mx && ((reinterpret_cast<uintptr_t>(mx_sa[s]) & 3) || (reinterpret_cast<uintptr_t>(mx_sb[s]) & 3))))
-            return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt_chain: operands must be 16-byte aligned, block scales 4-byte (product %d)", s);
+        if (!a[s] || !b[s] || !sa_inv[s] || !sb_inv[s]) return set_error(ODL_ERR_ARG, "odl_fp8_gemm_nt_chain: null pointer in product %d", s);
+        if ((reinterpret_cast<uintptr_t>(a[s]) & 15) || (reinterpret_cast<uintptr_t>(b[s]) & 15))
+            return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt_chain: operands must be 16-byte aligned (product %d)", s);
         GemmArgs &g = gc.m[s];
-        g.a = a[s]; g.b = b[s]; g.c = c; g.sa = mx ? one : sa_inv[s]; g.sb = mx ? one : sb_inv[s]; g.bias = nullptr;
-        g.mx_sa = mx ? mx_sa[s] : nullptr; g.mx_sb = mx ? mx_sb[s] : nullptr;
+        g.a = a[s]; g.b = b[s]; g.c = c; g.sa = sa_inv[s]; g.sb = sb_inv[s]; g.bias = nullptr;
         g.M = M; g.N = N; g.K = K[s];
         g.sa_vec = g.sb_vec = 0;
         g.out_dtype = ODL_BF16;
         g.tiles_m = (int)((M + bm - 1) / bm); g.tiles_n = (int)((N + bn - 1) / bn);
-        gp.a[s] = a[s]; gp.b[s] = b[s]; gp.sa[s] = g.sa; gp.sb[s] = g.sb; gp.k[s] = (int)K[s]; gp.mx_sa[s] = g.mx_sa; gp.mx_sb[s] = g.mx_sb;
     }
-    if (variant != kStreamVariant) launch_gemm_deep_chain(bm, bn, fmt_a, fmt_b, gc, cu_count(), stream);
-    else {
-        GemmArgs g = gc.m[0];
-        g.mx_sa = g.mx_sb = nullptr;                       // (gp's)
-        if (!gemm_stream_accepts_pairs(g, gp)) return set_error(ODL_ERR_SHAPE, "odl_fp8_gemm_nt_chain: shape not taken by the streaming kernel");
-        launch_gemm_stream_pairs(fmt_a, fmt_b, g, gp, cu_count(), stream);
-    }
+    launch_gemm_deep_chain(bm, bn, fmt_a, fmt_b, gc, cu_count(), stream);
     return check_launch("odl_fp8_gemm_nt_chain");
 }

@@ -95,15 +95,14 @@ __device__ __forceinline__ v16f mma_step(const v8i &b, const v8i &a, const v16f 
 // pair to the next exactly as it crosses from one tile to the next (other descriptors, other row pitch), and where a tile
 // ends with a fold, a pair ends with the accumulators multiplied by (scale product of this pair) / (that of the next)
 // under the first MFMAs of the next pair.  After the last pair the fold applies the last pair's scale product, so
-// C = ((acc_0 r_0 + acc_1) r_1 + ...) s_last in fp32 with one rounding to the output type.  With block scales, which the MFMAs
-// apply, there is nothing to multiply by: the pairs are one long contraction.
+// C = ((acc_0 r_0 + acc_1) r_1 + ...) s_last in fp32 with one rounding to the output type.
 //
 // GRP: the tiles are those of up to four products (gg) with one contraction length and one scale per operand, g being the first:
 // where a tile begins or ends, its operands, output, row length and scale product are its own product's.
 template <int FA, int FB, bool TA, bool TB, bool F32, int EPI, bool MX, bool SEG, bool GRP>
 __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const GemmPairs &gp, const GemmGroup &gg) {
     static_assert(!MX || (!TA && !TB && EPI != 1), "block scales: both operands stored [rows, K], no scale vectors");
-    static_assert(!SEG || (!TA && !TB && EPI == 0), "operand pairs: both stored [rows, K], one scale each, or block scales");
+    static_assert(!SEG || (!TA && !TB && EPI == 0 && !MX), "operand pairs: both stored [rows, K], one scale each");
     static_assert(!GRP || (!TA && !TB && EPI == 0 && !MX && !SEG), "grouped products: operands stored [rows, K], one scale each");
     constexpr int ESZ = F32 ? 4 : 2;
     constexpr int VEC_BYTES = 3 * 128 * 4;     // per wave: 128 row scales, 128 column scales, 128 bias values
@@ -231,13 +230,11 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
     // gets the size field cleared.  Of each operand this wave fetches 64 dwords per step: LDS dword d = 64 wave + lane
     // holds tile row 128 (d / 128) + 32 (d % 4) + (d % 128) / 4, so that rows r, r + 32, r + 64, r + 96 of a wave tile
     // lie side by side.
-    auto whole_scales = [&](const uint8_t *p, int64_t rows, int nk) -> v4i {
+    auto whole_scales = [&](const uint8_t *p, int64_t rows) -> v4i {
         const uint64_t addr = reinterpret_cast<uint64_t>(p);
-        return v4i{(int)(uint32_t)addr, (int)(uint32_t)(addr >> 32), (int)((uint32_t)(nk / 128) * (uint32_t)rows * 4u), 0x00020000};
+        return v4i{(int)(uint32_t)addr, (int)(uint32_t)(addr >> 32), (int)((uint32_t)(g.K / 128) * (uint32_t)rows * 4u), 0x00020000};
     };
-    v4i whole_sa = MX ? whole_scales(SEG ? gp.mx_sa[0] : g.mx_sa, g.M, SEG ? gp.k[0] : (int)g.K) : empty,
-        whole_sb = MX ? whole_scales(SEG ? gp.mx_sb[0] : g.mx_sb, g.N, SEG ? gp.k[0] : (int)g.K) : empty;
-    v4i next_whole_sa = whole_sa, next_whole_sb = whole_sb;      // SEG: of the pair that the last two steps of this one request from
+    const v4i whole_sa = MX ? whole_scales(g.mx_sa, g.M) : empty, whole_sb = MX ? whole_scales(g.mx_sb, g.N) : empty;
     const int sc_d = 64 * wave + lane;
     const int sc_voff = (128 * (sc_d / 128) + 32 * (sc_d % 4) + (sc_d % 128) / 4) * 4;
     const int sc_region = 128 * (wave / 2);       // first tile row of the 128 rows this wave fetches from (both operands)
@@ -251,16 +248,16 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         ib = tn0 + sc_region < (int)g.N ? 1 : 0;
     };
     // one operand's 64 scale dwords of a K step (which: 0 = A, 1 = B)
-    auto issue_scale = [&](int which, int stage, int ok, int off, int kstep, bool of_next) {
-        v4i d = which ? (SEG && of_next ? next_whole_sb : whole_sb) : (SEG && of_next ? next_whole_sa : whole_sa);
+    auto issue_scale = [&](int which, int stage, int ok, int off, int kstep) {
+        v4i d = which ? whole_sb : whole_sa;
         d.z = __builtin_amdgcn_readfirstlane(d.z * ok);
         off = __builtin_amdgcn_readfirstlane(off);
         const uint32_t dst = lds_addr_of(reinterpret_cast<const uint8_t *>(sScale)) + (stage * 512 + which * 256 + 64 * wave) * 4;
         dma4(d, dst, sc_voff, off + kstep * (int)(which ? g.N : g.M) * 4);
     };
     auto issue_scales = [&](int stage, int ok_a, int ok_b, int off_a, int off_b, int kstep) {
-        issue_scale(0, stage, ok_a, off_a, kstep, false);
-        issue_scale(1, stage, ok_b, off_b, kstep, false);
+        issue_scale(0, stage, ok_a, off_a, kstep);
+        issue_scale(1, stage, ok_b, off_b, kstep);
     };
     int sca[2][4] = {}, scb[2][4] = {};           // [K step parity][fragment]: this lane's scale dwords, already shifted
     // in two parts, so that the shift (which waits for the data) can sit a few MFMAs after the read
@@ -342,7 +339,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
     auto uniform = [](float v) { return bits_to_float((uint32_t)__builtin_amdgcn_readfirstlane((int)float_to_bits(v))); };
     // SEG: between pair s and s + 1 the accumulators take sRatio[s] = (scale product of s) / (that of s + 1); kept in
     // LDS (read once per pair) rather than in scalar registers, of which the K loop leaves none to spare
-    if constexpr (SEG && !MX) {
+    if constexpr (SEG) {
         const int s = (int)threadIdx.x;
         if (s + 1 < gp.count) sRatio[s] = (gp.sa[s][0] * gp.sb[s][0]) / (gp.sa[s + 1][0] * gp.sb[s + 1][0]);
         // (first read after the K loop of the first pair, many barriers from here)
@@ -351,8 +348,7 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         const int s = (int)threadIdx.x;
         if (s <= member_of(tiles - 1)) sRatio[s] = gg.m[s].sa[0] * gg.m[s].sb[0];
     }
-    constexpr bool scaled = GRP || (SEG && MX);   // products of a group have scales of their own, block scales are in the accumulators
-    const float s_tensor = scaled || g.splits > 1 ? 1.0f :       // partial results leave unscaled
+    const float s_tensor = GRP || g.splits > 1 ? 1.0f :          // products of a group have scales of their own, partial results leave unscaled
         SEG ? uniform(gp.sa[gp.count - 1][0] * gp.sb[gp.count - 1][0]) : uniform(g.sa[0] * g.sb[0]);
     // N is a multiple of 128 = the width of a wave tile: in the last tile column a wave is either wholly inside or wholly
     // outside.  One that is outside computes on the zeros that the bounded operand loads deliver and stores through the
@@ -588,8 +584,8 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
                 // for about a dozen instructions beside its MFMA
                 const int live = pad && !nx ? 0 : 1;
                 if (i == 8) fetch_scales(par ^ 1);
-                if (i == 9) issue_scale(0, par, (nx ? sc_nin_a : sc_in_a) * live, nx ? sc_next_a : sc_off_a, koff, nx);
-                if (i == 10) issue_scale(1, par, (nx ? sc_nin_b : sc_in_b) * live, nx ? sc_next_b : sc_off_b, koff, nx);
+                if (i == 9) issue_scale(0, par, (nx ? sc_nin_a : sc_in_a) * live, nx ? sc_next_a : sc_off_a, koff);
+                if (i == 10) issue_scale(1, par, (nx ? sc_nin_b : sc_in_b) * live, nx ? sc_next_b : sc_off_b, koff);
                 if (i == 12) place_a(sca[par ^ 1]);
                 if (i == 14) place_b(scb[par ^ 1]);
             }
@@ -610,7 +606,6 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         KT = gp.k[0] / 128;                    // an even number of steps, at least 4 (checked by the caller)
         rsrc_a = rsrc_for(gp.a[0], m0, g.M, false, 0, gp.k[0]);
         rsrc_b = rsrc_for(gp.b[0], n0, g.N, false, 0, gp.k[0]);
-        if constexpr (MX) scale_origin(m0, n0, 0, sc_off_a, sc_off_b, sc_in_a, sc_in_b);
     } else {
         int first_step = 0;
         item_steps(pid, first_step, KT, padded);
@@ -668,10 +663,6 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
             scale_origin(next_m0, next_n0, next_first, sc_next_a, sc_next_b, sc_nin_a, sc_nin_b);
             sc_nin_a *= has_next ? 1 : 0;
             sc_nin_b *= has_next ? 1 : 0;
-            if constexpr (SEG) {
-                next_whole_sa = whole_scales(gp.mx_sa[next_seg], g.M, next_nk);
-                next_whole_sb = whole_scales(gp.mx_sb[next_seg], g.N, next_nk);
-            }
         }
 
         // ---- rest of step 0 (its phase A ran at the end of the previous trip), then steps 1 .. KT-1.
@@ -709,14 +700,9 @@ __device__ __forceinline__ void gemm_nt_stream_body(const GemmArgs &g, const Gem
         sc_off_b = sc_next_b;
         sc_in_a = sc_nin_a;
         sc_in_b = sc_nin_b;
-        if constexpr (SEG && MX) {
-            whole_sa = next_whole_sa;
-            whole_sb = next_whole_sb;
-        }
         const int pair = seg;
         seg = next_seg;
         if constexpr (tile_ends) phase_a_fold(sA0, sB0, rsrc_c, done, done_n2);
-        else if constexpr (MX) phase_a(sA0, sB0, 0);          // (the accumulators contain the scales and go on as they are)
         else phase_a_rescale(sA0, sB0, pair);
         return has_next;
     };
@@ -743,9 +729,9 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs g) {
 }
 
 // the same kernel over several operand pairs (see SEG above)
-template <int FA, int FB, bool F32, bool MX = false>
+template <int FA, int FB, bool F32>
 __global__ __launch_bounds__(256) void gemm_nt_stream_pairs_kernel(const GemmArgs g, const GemmPairs gp) {
-    gemm_nt_stream_body<FA, FB, false, false, F32, 0, MX, true, false>(g, gp, GemmGroup{});
+    gemm_nt_stream_body<FA, FB, false, false, F32, 0, false, true, false>(g, gp, GemmGroup{});
 }
 
 // the same kernel over the tiles of several products (see GRP above)
@@ -798,17 +784,14 @@ bool gemm_stream_accepts(const GemmArgs &g) {
 // 3e-3 (2-norm, bf16, contractions 4096 + 1024 + 1024) apart, and which of them a size gets is part of the contract.
 bool gemm_stream_accepts_pairs(const GemmArgs &g, const GemmPairs &gp) {
     const double esz = g.out_dtype == ODL_F32 ? 4.0 : 2.0;
-    const bool mx = gp.mx_sa[0] != nullptr;                  // block scales: bf16 only, and any M (there is no other route whose bits count)
     if (gp.count < 1 || gp.count > 4 || g.accumulate || g.ta || g.tb || g.sa_vec || g.sb_vec || g.bias || g.mx_sa || g.mx_sb || g.splits > 1)
         return false;
-    if (mx && g.out_dtype != ODL_BF16) return false;
     for (int s = 0; s < gp.count; ++s) {
         const int k = gp.k[s];
-        if (!gp.a[s] || !gp.b[s] || k < 512 || k % 256 != 0) return false;
-        if (mx ? !gp.mx_sa[s] || !gp.mx_sb[s] : !gp.sa[s] || !gp.sb[s]) return false;
+        if (!gp.a[s] || !gp.b[s] || !gp.sa[s] || !gp.sb[s] || k < 512 || k % 256 != 0) return false;
         if ((double)(g.M + 256) * k >= 2147483648.0 || (double)(g.N + 256) * k >= 2147483648.0) return false;
     }
-    return (g.out_dtype == ODL_BF16 || g.out_dtype == ODL_F32) && g.M > 0 && g.N > 0 && (mx || g.M % WM == 0) && g.N % WN == 0 &&
+    return (g.out_dtype == ODL_BF16 || g.out_dtype == ODL_F32) && g.M > 0 && g.N > 0 && g.M % WM == 0 && g.N % WN == 0 &&
            (double)g.N * esz * (BM + 8) < 2147483648.0;
 }
 
@@ -839,8 +822,7 @@ namespace {
 template <int FA, int FB>
 void launch_pairs_fmt(const GemmArgs &g, const GemmPairs &gp, int blocks_per_xcd, hipStream_t stream) {
     const dim3 grid((unsigned)(8 * blocks_per_xcd)), block(256);
-    if (gp.mx_sa[0]) hipLaunchKernelGGL((gemm_nt_stream_pairs_kernel<FA, FB, false, true>), grid, block, 0, stream, g, gp);
-    else if (g.out_dtype == ODL_F32) hipLaunchKernelGGL((gemm_nt_stream_pairs_kernel<FA, FB, true>), grid, block, 0, stream, g, gp);
+    if (g.out_dtype == ODL_F32) hipLaunchKernelGGL((gemm_nt_stream_pairs_kernel<FA, FB, true>), grid, block, 0, stream, g, gp);
     else hipLaunchKernelGGL((gemm_nt_stream_pairs_kernel<FA, FB, false>), grid, block, 0, stream, g, gp);
 }
 

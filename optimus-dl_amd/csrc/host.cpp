@@ -374,34 +374,24 @@ py::object gemm_nt_group(const std::vector<Tensor> &a, const std::vector<Tensor>
     return rc ? status(rc) : py::object(out);
 }
 
-bool chain_in_one_launch(const std::vector<i64> &K, i64 M, i64 N, bool block_scales) {
-    return K.size() <= 4 && chain_route_c((int)K.size(), K.data(), M, N, block_scales) >= 0;
-}
-
-// K-step-major scale bytes of codes [rows, K]
-bool kstep_scales(const Tensor &s, const Tensor &codes) {
-    return dense(s) && s.scalar_type() == at::kByte && s.dim() == 3 && s.size(0) * 128 == codes.size(1) && s.size(1) == codes.size(0) && s.size(2) == 4;
-}
+bool chain_in_one_launch(const std::vector<i64> &K, i64 M, i64 N) { return K.size() <= 4 && chain_route_c((int)K.size(), K.data(), M, N) >= 0; }
 
 // The bf16 sum of several products in one launch
 py::object gemm_nt_chain(const std::vector<Tensor> &a, const std::vector<Tensor> &b, int fa, int fb, const std::vector<Tensor> &sa,
-                         const std::vector<Tensor> &sb, bool block_scales, i64 stream) {
+                         const std::vector<Tensor> &sb, i64 stream) {
     const size_t n = a.size();
     if (n < 2 || n > 4 || b.size() != n || sa.size() != n || sb.size() != n) return none();
-    const uint8_t *pa[4], *pb[4], *pma[4], *pmb[4];
+    const uint8_t *pa[4], *pb[4];
     const float *psa[4], *psb[4];
     i64 K[4];
     for (size_t s = 0; s < n; ++s) {
         if (!codes2d(a[s]) || !codes2d(b[s]) || a[s].size(0) != a[0].size(0) || b[s].size(0) != b[0].size(0) || a[s].size(1) != b[s].size(1)) return none();
-        if (block_scales ? !kstep_scales(sa[s], a[s]) || !kstep_scales(sb[s], b[s]) : !floats(sa[s], 1) || !floats(sb[s], 1)) return none();
+        if (!floats(sa[s], 1) || !floats(sb[s], 1)) return none();
         K[s] = a[s].size(1);
-        pa[s] = ptr(a[s]); pb[s] = ptr(b[s]);
-        if (block_scales) { pma[s] = ptr(sa[s]); pmb[s] = ptr(sb[s]); }
-        else { psa[s] = ptr(sa[s]); psb[s] = ptr(sb[s]); }
+        pa[s] = ptr(a[s]); pb[s] = ptr(b[s]); psa[s] = ptr(sa[s]); psb[s] = ptr(sb[s]);
     }
     Tensor c = result(OptTensor(), a[0], a[0].size(0), b[0].size(0), 0);
-    const int rc = call(gemm_nt_chain_c, (int)n, pa, pb, K, a[0].size(0), b[0].size(0), fa, fb, psa, psb, block_scales ? pma : nullptr,
-                        block_scales ? pmb : nullptr, ptr(c), str(stream));
+    const int rc = call(gemm_nt_chain_c, (int)n, pa, pb, K, a[0].size(0), b[0].size(0), fa, fb, psa, psb, ptr(c), str(stream));
     return rc ? status(rc) : py::cast(c);
 }
 

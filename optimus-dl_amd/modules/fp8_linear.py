@@ -349,10 +349,7 @@ class _Fp8LinearFn(torch.autograd.Function):
             if ctx.need_dgrad or fp8_wgrad:
                 # one pass over dy: blocks along the output features for dgrad, along the tokens (transposed) for wgrad
                 gq, gs, gq_t, gs_t = given or _block_cast(pol, dy2d, pol.fmt_bwd, ctx.need_dgrad, fp8_wgrad)
-            dx_pairs = getattr(ctx, "dx_pairs", None)
-            if ctx.need_dgrad and dx_pairs is not None:
-                dx_pairs.append((gq, saved["wq_t"], gs, saved["ws_t"]))
-            elif ctx.need_dgrad:
+            if ctx.need_dgrad:
                 dx = native.mx_gemm_nt(gq, gs, saved["wq_t"], saved["ws_t"], pol.fmt_bwd, pol.fmt_fwd, out_dtype=ctx.x_dtype)
             if fp8_wgrad:
                 dw = native.mx_gemm_nt(gq_t, gs_t, saved["xq_t"], saved["xs_t"], pol.fmt_bwd, pol.fmt_fwd, out_dtype=ctx.w_dtype)
@@ -574,10 +571,9 @@ class _Fp8LinearGroupFn(torch.autograd.Function):
         and v shares of a grouped-query block (contractions of 1024) are, added into a cold 64 MB dx, bound by reading and
         writing it (63 us each at 8192 tokens against 40 for the bare product); carried through one set of
         accumulators they cost what their share of the contraction costs.  ``native.gemm_nt_chain`` where that is faster than
-        adding one by one, with the bits of it; under block scales, too, where a sum of the results is the other way."""
+        adding one by one, with the bits of it."""
         recipe = ctx.subs[0].recipe
-        kind = recipe.recipe.kind
-        if not recipe.fuse_dgrad_gemm or kind == "rowwise":
+        if not recipe.fuse_dgrad_gemm or recipe.recipe.kind not in ("tensorwise", "delayed"):
             return None, None
         live = [sub for sub, dy in zip(ctx.subs, dys) if dy is not None and sub.need_dgrad]
         if len(live) < 2 or any(dy is not None and not sub.need_dgrad for sub, dy in zip(ctx.subs, dys)):
@@ -585,11 +581,10 @@ class _Fp8LinearGroupFn(torch.autograd.Function):
         tokens = next(dy for dy in dys if dy is not None).shape[0]
         n_in, n_outs, dtype = live[0].module.in_features, [sub.module.out_features for sub in live], live[0].x_dtype
         fmts = recipe.recipe.fmt_bwd, recipe.recipe.fmt_fwd
-        if kind in ("tensorwise", "delayed") and native.dgrad_sum_in_one_launch(tokens, n_in, n_outs):
+        if native.dgrad_sum_in_one_launch(tokens, n_in, n_outs):
             return [], lambda a, b, sa, sb: native.gemm_nt_sum(a, b, *fmts, sa, sb, out_dtype=dtype)
-        block_scales = kind in ("mxfp8", "blockwise")
-        if dtype == torch.bfloat16 and native.gemm_chain_in_one_launch(n_outs, tokens, n_in, block_scales):
-            return [], lambda a, b, sa, sb: native.gemm_nt_chain(a, b, *fmts, sa, sb, block_scales)
+        if dtype == torch.bfloat16 and native.gemm_chain_in_one_launch(n_outs, tokens, n_in):
+            return [], lambda a, b, sa, sb: native.gemm_nt_chain(a, b, *fmts, sa, sb)
         return None, None
 
     @staticmethod

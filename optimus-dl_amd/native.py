@@ -26,7 +26,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 28
+ABI_VERSION = 29
 _OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
@@ -177,8 +177,8 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_cast_delayed.argtypes = [vp, i32, i64, i64, vp, i32, vp, vp, vp, vp, vp]
         L.odl_fp8_gemm_nt.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, i64, vp, i64, vp, i32, vp, i32, i32, vp]
         L.odl_fp8_gemm_nt_hinted.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, i64, vp, i64, vp, i32, vp, i32, i32, i32, vp]
-        L.odl_fp8_gemm_chain_route.argtypes = [i32, vp, i64, i64, i32]
-        L.odl_fp8_gemm_nt_chain.argtypes = [i32, vp, vp, vp, i64, i64, i32, i32, vp, vp, vp, vp, vp, vp]
+        L.odl_fp8_gemm_chain_route.argtypes = [i32, vp, i64, i64]
+        L.odl_fp8_gemm_nt_chain.argtypes = [i32, vp, vp, vp, i64, i64, i32, i32, vp, vp, vp, vp]
         L.odl_fp8_gemm_group_route.argtypes = [i32, vp, vp, i64, i32]
         L.odl_fp8_gemm_nt_group.argtypes = [i32, vp, vp, vp, vp, i64, i32, i32, vp, vp, vp, i32, i32, vp]
         L.odl_fp8_gemm_nt_sum.argtypes = [i32, vp, vp, vp, i64, i64, i32, i32, vp, vp, vp, i32, vp]
@@ -1054,21 +1054,18 @@ def gemm_nt_sum(a: "list[torch.Tensor]", b: "list[torch.Tensor]", fmt_a: int, fm
     return out
 
 
-def gemm_chain_in_one_launch(Ks: "list[int]", M: int, N: int, block_scales: bool = False) -> bool:
+def gemm_chain_in_one_launch(Ks: "list[int]", M: int, N: int) -> bool:
     """Whether :func:`gemm_nt_chain` takes products of these sizes."""
     load()
-    return bool(_host.chain_in_one_launch(Ks, M, N, block_scales))
+    return bool(_host.chain_in_one_launch(Ks, M, N))
 
 
 def gemm_nt_chain(a: "list[torch.Tensor]", b: "list[torch.Tensor]", fmt_a: int, fmt_b: int, sa: "list[torch.Tensor]",
-                  sb: "list[torch.Tensor]", block_scales: bool = False) -> torch.Tensor:
-    """The bf16 sum of the products a[s] . b[s]^T in one launch: with one scale per operand what :func:`gemm_nt` and, for the second
-    and later ones, ``accumulate`` give; with block scales (K-step-major) rounded once.  Only where
-    :func:`gemm_chain_in_one_launch` says so."""
+                  sb: "list[torch.Tensor]") -> torch.Tensor:
+    """The bf16 sum of the products a[s] . b[s]^T, one scale per operand, in one launch: what :func:`gemm_nt` and, for the second
+    and later ones, ``accumulate`` give.  Only where :func:`gemm_chain_in_one_launch` says so."""
     load()
-    if block_scales:
-        init_device(a[0].device)
-    r = _host.gemm_nt_chain(a, b, fmt_a, fmt_b, sa, sb, block_scales, _stream())
+    r = _host.gemm_nt_chain(a, b, fmt_a, fmt_b, sa, sb, _stream())
     if r is None:
         raise NativeError(f"gemm_nt_chain: operands {[tuple(t.shape) for t in (*a, *b)]} or their scales do not fit, are not dense or not aligned")
     return _done(r, "odl_fp8_gemm_nt_chain")
