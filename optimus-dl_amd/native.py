@@ -1453,7 +1453,7 @@ def gemm_wgrad_pays(n_out: int, n_in: int, tokens: int, out_dtype: torch.dtype =
     """Whether :func:`gemm_wgrad` takes a weight gradient that :func:`gemm_layouts` does not (n_out no multiple of 256) and is faster
     than the route over a transposed copy of dY: where its tiles fill the chip, as in :func:`wgrad_direct_pays`.  50304 x 768
     fp32, product and cast of dY, this way / over the copy in us: 1024 tokens 88 / 99, 2048 142 / 159, 8192 589 / 704, 16384 1190 / 1417."""
-    return (n_out % 256 != 0 and n_out % 16 == 0 and n_in % 128 == 0 and tokens % 128 == 0 and tokens >= 512
+    return (n_out > 256 and n_out % 256 != 0 and n_out % 16 == 0 and n_in % 128 == 0 and tokens % 128 == 0 and tokens >= 512
             and out_dtype in (torch.bfloat16, torch.float32) and -(-n_out // 256) * -(-n_in // 256) >= 192
             and (n_out + 256) * tokens < 2**31 and (n_in + 256) * tokens < 2**31 and n_in * out_dtype.itemsize * 264 < 2**31)
 

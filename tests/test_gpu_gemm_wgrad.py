@@ -67,3 +67,26 @@ def test_a_linear_takes_it_with_the_bits_of_the_copy(monkeypatch, recipe_name):
                 y.backward(dy)
         grads.append(lin.weight.grad)
     assert len(calls) == 2 and torch.equal(*grads) and grads[0].dtype == torch.float32
+
+
+@pytest.mark.parametrize("recipe_name", ["tensorwise", "delayed"])
+@pytest.mark.parametrize("n_out", [128, 240])
+def test_few_rows_of_a_wide_weight_keep_the_copy(n_out, recipe_name):
+    """50304 -> 128: 197 tiles of 256 x 256, but not a whole one of rows."""
+    from optimus_dl_amd.modules import amp
+    from optimus_dl_amd.modules.fp8_linear import FP8Linear
+
+    x, dy = torch.randn((512, 50304), device="cuda").bfloat16(), (torch.randn((512, n_out), device="cuda") * 1e-3).bfloat16()
+    lin = FP8Linear.from_linear(nn.Linear(50304, n_out, bias=False).cuda().bfloat16())
+    grads = []
+    for direct in ("auto", False):
+        recipe = amp.create_fp8_recipe(recipe_name, "hybrid", amax_history_len=4)
+        recipe.direct_layouts = direct
+        for _ in range(2):
+            lin.weight.grad = None
+            with recipe.autocast():
+                y = lin(x)
+            with recipe.backward():
+                y.backward(dy)
+        grads.append(lin.weight.grad)
+    assert torch.equal(*grads) and bool(grads[0].any())

@@ -3,6 +3,7 @@ their multiples, and column counts that leave no slab at all."""
 import ctypes
 
 import pytest
+import torch
 
 from optimus_dl_amd import native as N
 
@@ -48,3 +49,25 @@ def test_joint_cast_null_member(L):
 @pytest.mark.parametrize("n_out,n_in,tokens", [(240, 128, 512), (264, 128, 512), (272, 64, 512), (272, 128, 500), (272, 128, 384), (272, 128, 2**23), (0, 128, 512)])
 def test_weight_gradient_as_stored(L, n_out, n_in, tokens):
     assert L.odl_fp8_gemm_wgrad(P, P, n_out, n_in, tokens, 1, 0, P, P, P, 1, None) != 0
+
+
+@pytest.mark.parametrize("n_in,tokens", [(49152, 512), (50304, 512), (65536, 4096), (2**20, 512)])
+def test_few_rows_of_a_wide_weight_are_not_sent_to_what_refuses_them(L, n_in, tokens):
+    """Rows that leave no 256 x 256 tile, of so many columns that there are 192 tiles all the same."""
+    for n_out in range(16, 256, 16):
+        assert not N.gemm_wgrad_pays(n_out, n_in, tokens)
+        assert L.odl_fp8_gemm_wgrad(P, P, n_out, n_in, tokens, 1, 0, P, P, P, 1, None) != 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_what_pays_is_what_the_entry_takes(dtype):
+    """The sizes of odl_fp8.h: n_out >= 256 in sixteens, n_in and tokens of 128, 512 tokens, operands and 264 rows of dW under 2 GiB."""
+    taken = 0
+    for n_out in (*range(8, 600, 8), 1040, 12304, 50304, 128 * 1024 + 16):
+        for n_in in (64, 128, 700, 768, 4096, 25216, 50304, 2**20, 2**22):
+            for tokens in (128, 384, 512, 520, 640, 8192, 2**15):
+                if N.gemm_wgrad_pays(n_out, n_in, tokens, dtype):
+                    taken += 1
+                    assert n_out >= 256 and n_out % 16 == 0 and n_in % 128 == 0 and tokens % 128 == 0 and tokens >= 512
+                    assert (n_out + 256) * tokens < 2**31 and (n_in + 256) * tokens < 2**31 and n_in * dtype.itemsize * 264 < 2**31
+    assert taken > 100
