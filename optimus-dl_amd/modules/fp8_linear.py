@@ -435,6 +435,7 @@ class _Fp8LinearFn(torch.autograd.Function):
                     and tuple(grad_buf.shape) == (module.out_features, module.in_features)
                 # wgrad_direct: dW = dY^T . X with dY [tokens, N] as stored, X^T from the forward
                 if ctx.wgrad_direct and module.out_features % 256:
+                    into = False         # (the flag was set since the forward: this entry does not add, autograd does)
                     dw = native.gemm_wgrad(gq, saved["xq_t"], pol.fmt_bwd, pol.fmt_fwd, sg_inv, saved["sx_inv_t"], ctx.w_dtype)
                 elif ctx.wgrad_direct:
                     dw = native.gemm_layouts(gq, saved["xq_t"], pol.fmt_bwd, pol.fmt_fwd, native.K_SLOW, native.K_FAST,

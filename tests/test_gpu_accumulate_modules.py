@@ -209,6 +209,31 @@ def build_wide(group=True):
 
 
 @pytest.mark.parametrize("kind", ["tensorwise", "delayed"])
+@pytest.mark.parametrize("n_out", [512, 12288, 12304])
+def test_accumulation_switched_on_between_forward_and_backward(amp, n_out, kind):
+    """Whichever way the forward has chosen for the weight gradient (over the transposed copy, over dY as stored in whole tiles of rows or
+    not): the gradient of the pending graph reaches ``.grad``, with the bits of autograd's own addition (fp32)."""
+    from optimus_dl_amd.modules.fp8_linear import FP8Linear
+
+    def two_microbatches(switch):
+        torch.manual_seed(1)
+        lin = FP8Linear.from_linear(nn.Linear(1024, n_out, bias=False).cuda())
+        recipe = amp.create_fp8_recipe(kind, "hybrid", amax_history_len=4)
+        grads = []
+        for i in range(2):
+            with recipe.autocast():
+                y = lin(seeded_bf16((512, 1024), 1.0, 40 + i).cuda())
+            recipe.fuse_wgrad_accumulation = switch and i == 1
+            with recipe.backward():
+                y.backward(seeded_bf16((512, n_out), 1e-3, 50 + i).cuda())
+            grads.append(lin.weight.grad.clone())
+        return grads
+
+    (first, got), (first_want, want) = two_microbatches(True), two_microbatches(False)
+    assert torch.equal(first, first_want) and not torch.equal(got, first) and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("kind", ["tensorwise", "delayed"])
 def test_sibling_group_data_gradient_from_one_gemm(amp, kind, monkeypatch):
     """4096 tokens x 2304 features (144 tiles): the group's data gradient comes from ONE launch over the three members'
     operands (no GEMM with the accumulate flag, no dgrad of a member's own), outputs and weight gradients are the bits of
