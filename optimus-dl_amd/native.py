@@ -1451,10 +1451,17 @@ def wgrad_direct_pays(n_out: int, n_in: int, tokens: int) -> bool:
 
 def gemm_wgrad_pays(n_out: int, n_in: int, tokens: int, out_dtype: torch.dtype = torch.bfloat16) -> bool:
     """Whether :func:`gemm_wgrad` takes a weight gradient that :func:`gemm_layouts` does not (n_out no multiple of 256) and is faster
-    than the route over a transposed copy of dY: where its tiles fill the chip, as in :func:`wgrad_direct_pays`.  50304 x 768
-    fp32, product and cast of dY, this way / over the copy in us: 1024 tokens 88 / 99, 2048 142 / 159, 8192 589 / 704, 16384 1190 / 1417."""
-    return (n_out > 256 and n_out % 256 != 0 and n_out % 16 == 0 and n_in % 128 == 0 and tokens % 128 == 0 and tokens >= 512
-            and out_dtype in (torch.bfloat16, torch.float32) and -(-n_out // 256) * -(-n_in // 256) >= 192
+    than the route over a transposed copy of dY: for the output of a vocabulary, 48 tiles of rows or more and four times as many rows as
+    columns.  It spares writing that copy, n_out x tokens bytes, which is 1 / n_in of what the product does; the product itself is a
+    little slower over dY as stored, and the copy's has other kernels for a last round of few tiles.  Product and cast of dY, both
+    layouts where dY is copied, this way / over the copy in us, 2048 and 8192 tokens: 50304 x 768 fp32 142 / 166 and 534 / 676, 12304 x
+    1024 bf16 45 / 53 and 135 / 171, 12304 x 3072 96 / 102 and 305 / 319, 32016 x 5632 321 / 337 and 1207 / 1263, 20496 x 5120 204 / 213 and
+    698 / 741 (512 tokens fp32 115.5 / 113.9, the one loss of 90 measured).  On the other side of the line 32016 x 8192 448 / 456 and 1688 /
+    1721, 6160 x 2048 40.5 / 41.2 and 115 / 128, but 8208 x 4096 91 / 89 and 286 / 271, 4112 x 4096 60 / 52 and 183 / 155, 1040 x 14336 54 / 44
+    and 169 / 133, 272 x 50304 55 / 49 and 206 / 199.  Where nobody asks for the data gradient both ways cast one layout and are equal
+    within 5 %."""
+    return (n_out >= 12288 and n_out >= 4 * n_in and n_out % 256 != 0 and n_out % 16 == 0 and n_in % 128 == 0 and tokens % 128 == 0
+            and tokens >= 512 and out_dtype in (torch.bfloat16, torch.float32) and -(-n_out // 256) * -(-n_in // 256) >= 192
             and (n_out + 256) * tokens < 2**31 and (n_in + 256) * tokens < 2**31 and n_in * out_dtype.itemsize * 264 < 2**31)
 
 
