@@ -46,7 +46,7 @@ enum odl_status {
 };
 
 /* ABI version of this header; bumped when a signature changes or an entry point is added. */
-#define ODL_FP8_ABI_VERSION 29
+#define ODL_FP8_ABI_VERSION 30
 int odl_fp8_abi_version(void);
 
 /*
@@ -215,12 +215,14 @@ int odl_fp8_amax_parts_colsum(const void *x, int src_dtype, int64_t rows, int64_
  * The same in two halves around the cast that follows: odl_fp8_amax_parts_slabs leaves the partial maxima and, in the workspace, slabs
  * of column sums; odl_fp8_cast_dynamic_colsum is odl_fp8_cast_dynamic_padded (both layouts; cols a multiple of 8, rows_out of 16, x and
  * out_t 16-byte aligned) and adds the slabs up besides, to the sums of odl_fp8_amax_parts_colsum rounded to colsum_dtype
- * (ODL_BF16 or ODL_F32).  src_dtype, rows and cols as in the first half.
+ * (ODL_BF16 or ODL_F32).  src_dtype, rows and cols as in the first half.  odl_fp8_slabs_colsum adds the slabs up by themselves, to
+ * the very sums of odl_fp8_amax_parts_colsum (colsum[cols], fp32).
  */
 int odl_fp8_amax_parts_slabs(const void *x, int src_dtype, int64_t rows, int64_t cols, float *parts, float *workspace, odl_stream_t stream);
 int odl_fp8_cast_dynamic_colsum(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, const float *parts, int fmt,
                                 int margin, uint8_t *out, uint8_t *out_t, float *dyn_out, const float *workspace, void *colsum,
                                 int colsum_dtype, odl_stream_t stream);
+int odl_fp8_slabs_colsum(const float *workspace, int src_dtype, int64_t rows, int64_t cols, float *colsum, odl_stream_t stream);
 
 /*
  * The rowwise recipe needs every tensor twice: scaled per row for the GEMM that contracts
@@ -330,7 +332,7 @@ int odl_fp8_layernorm_bwd(const void *dy, const void *x, int src_dtype, const fl
  *   odl_fp8_gelu_bwd_amax_parts : dx = bf16( dy * bwd[x] );     parts = partial maxima of |dx|
  * rows * cols a multiple of 8, 16-byte aligned pointers.
  *   odl_fp8_gelu_bwd_slabs      : the same, and the slabs of column sums of dx that odl_fp8_amax_parts_slabs(dx) leaves in its
- *                                 workspace (cols a multiple of 8), for odl_fp8_cast_dynamic_colsum
+ *                                 workspace (cols a multiple of 8), for odl_fp8_cast_dynamic_colsum or odl_fp8_slabs_colsum
  */
 #define ODL_FP8_GELU_TABLE_BYTES (65536 * 2 + 65536 * 4)
 int odl_fp8_gelu_table(void *table, odl_stream_t stream);

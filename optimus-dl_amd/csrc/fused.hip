@@ -1204,6 +1204,19 @@ extern "C" int odl_fp8_amax_parts_slabs(const void *x, int src_dtype, int64_t ro
     return check_launch("odl_fp8_amax_parts_slabs");
 }
 
+extern "C" int odl_fp8_slabs_colsum(const float *workspace, int src_dtype, int64_t rows, int64_t cols, float *colsum, odl_stream_t stream_) {
+    if (!workspace || !colsum) return set_error(ODL_ERR_ARG, "odl_fp8_slabs_colsum: null pointer");
+    if (src_dtype != ODL_BF16 && src_dtype != ODL_F32) return set_error(ODL_ERR_ARG, "odl_fp8_slabs_colsum: src_dtype %d", src_dtype);
+    if (rows <= 0 || cols <= 0) return set_error(ODL_ERR_ARG, "odl_fp8_slabs_colsum: empty or negative shape");
+    const int cpl = src_dtype == ODL_BF16 ? 8 : 4;
+    if (cols % cpl != 0 || cols > (int64_t)kParts * 32 * cpl)
+        return set_error(ODL_ERR_SHAPE, "odl_fp8_slabs_colsum: cols must be a multiple of %d and at most %d", cpl, kParts * 32 * cpl);
+    int64_t slabs;
+    colsum_slab_rows(src_dtype, rows, cols, &slabs);
+    launch_slab_reduce(workspace, (int)slabs, cols, colsum, reinterpret_cast<hipStream_t>(stream_));
+    return check_launch("odl_fp8_slabs_colsum");
+}
+
 extern "C" int odl_fp8_cast_dynamic_colsum(const void *x, int src_dtype, int64_t rows, int64_t cols, int64_t rows_out, const float *parts, int fmt,
                                            int margin, uint8_t *out, uint8_t *out_t, float *dyn_out, const float *workspace, void *colsum,
                                            int colsum_dtype, odl_stream_t stream_) {

@@ -29,6 +29,7 @@ decltype(&odl_fp8_cast_delayed_padded) cast_delayed_c;
 decltype(&odl_fp8_cast_delayed_many) cast_delayed_many_c;
 decltype(&odl_fp8_amax_parts_colsum) amax_colsum_c;
 decltype(&odl_fp8_amax_parts_slabs) amax_slabs_c;
+decltype(&odl_fp8_slabs_colsum) slabs_colsum_c;
 decltype(&odl_fp8_cast_dynamic_colsum) cast_colsum_c;
 decltype(&odl_fp8_swiglu_amax_parts) swiglu_c;
 decltype(&odl_fp8_swiglu_bwd_amax_parts) swiglu_bwd_c;
@@ -64,6 +65,7 @@ void bind(const py::dict &d) {
     take(cast_delayed_many_c, d, "odl_fp8_cast_delayed_many");
     take(amax_colsum_c, d, "odl_fp8_amax_parts_colsum");
     take(amax_slabs_c, d, "odl_fp8_amax_parts_slabs");
+    take(slabs_colsum_c, d, "odl_fp8_slabs_colsum");
     take(cast_colsum_c, d, "odl_fp8_cast_dynamic_colsum");
     take(swiglu_c, d, "odl_fp8_swiglu_amax_parts");
     take(swiglu_bwd_c, d, "odl_fp8_swiglu_bwd_amax_parts");
@@ -208,6 +210,14 @@ py::object amax_colsum(const Tensor &x, bool finish, i64 stream) {
     Tensor parts = f32(x, {kParts}), sums = f32(x, {x.size(1)}), ws = f32(x, {ODL_FP8_COLSUM_WORKSPACE});
     const int rc = call(amax_colsum_c, ptr(x), src_of(x), x.size(0), x.size(1), ptr(parts), ptr(sums), ptr(ws), str(stream));
     return rc ? status(rc) : py::make_tuple(parts, sums);
+}
+
+// the column sums of x from the slabs that amax_colsum(x, false) or the producer of x left
+py::object slabs_colsum(const Tensor &x, const Tensor &slabs, i64 stream) {
+    if (!source2d(x) || x.numel() == 0 || !floats(slabs, ODL_FP8_COLSUM_WORKSPACE)) return none();
+    Tensor sums = f32(x, {x.size(1)});
+    const int rc = call(slabs_colsum_c, ptr(slabs), src_of(x), x.size(0), x.size(1), ptr(sums), str(stream));
+    return rc ? status(rc) : py::cast(sums);
 }
 
 py::object cast_colsum(const Tensor &x, const Tensor &parts, const Tensor &slabs, int fmt, int margin, i64 rows_out, int odt, i64 stream) {
@@ -463,6 +473,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("cast_delayed", &cast_delayed);
     m.def("cast_delayed_many", &cast_delayed_many);
     m.def("amax_colsum", &amax_colsum);
+    m.def("slabs_colsum", &slabs_colsum);
     m.def("cast_colsum", &cast_colsum);
     m.def("swiglu", &swiglu);
     m.def("swiglu_bwd", &swiglu_bwd);

@@ -395,7 +395,8 @@ class _Fp8LinearFn(torch.autograd.Function):
                         # the amax pass also adds up the columns: the bias gradient costs no extra read of dy.  It
                         # runs for the column sums even when the producer of dy left its partial maxima (which are
                         # the same numbers), unless that left the sums too: one pass of this kernel is cheaper than a separate
-                        # sum over the rows.  Slabs of sums are added up, and rounded, by blocks of the cast where that writes both layouts
+                        # sum over the rows.  Slabs of sums are added up, and rounded, by blocks of the cast where that writes both
+                        # layouts, else in a launch of their own
                         with_cast = g_t_needed and g_rm_needed and gq_t_out is None and ctx.bias_dtype in (torch.bfloat16, torch.float32)
                         parts, sums = native.amax_parts_colsum(dy2d, finish=not with_cast, left=None if left is None else (parts, left))
                         if sums.dim() == 2:
@@ -450,8 +451,10 @@ class _Fp8LinearFn(torch.autograd.Function):
             dw = (dy2d.t().to(saved["x_hp"].dtype) @ saved["x_hp"]).to(ctx.w_dtype)
         if ctx.has_bias and db is None:
             if dy2d.is_cuda and native.colsum_supported(dy2d):
-                # delayed and rowwise scaling have no amax pass to ride on: the same kernel, for its column sums only
-                db = native.amax_parts_colsum(dy2d)[1].to(ctx.bias_dtype)
+                # delayed and rowwise scaling have no amax pass to ride on: the same kernel, for its column sums only.  (Sums that
+                # the producer of dy left are still there where nobody has quantised dy: a frozen weight, no data gradient.)
+                parts, left = recipe.take_parts_and_slabs(dy2d)
+                db = native.amax_parts_colsum(dy2d, left=None if left is None else (parts, left))[1].to(ctx.bias_dtype)
             else:
                 db = dy2d.sum(dim=0, dtype=torch.float32).to(ctx.bias_dtype)
         return dx, dw, db, None, None, None

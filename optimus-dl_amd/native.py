@@ -26,7 +26,7 @@ DT_BF16, DT_F32 = 0, 1
 AMAX_MAX, AMAX_MOST_RECENT = 0, 1
 FP8_MAX = {E4M3: 448.0, E5M2: 57344.0}
 TORCH_FP8 = {E4M3: torch.float8_e4m3fn, E5M2: torch.float8_e5m2}
-ABI_VERSION = 29
+ABI_VERSION = 30
 _OUT_DTYPES = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 AMAX_PARTS = 512                       # ODL_FP8_AMAX_PARTS
 
@@ -58,6 +58,7 @@ EXPORTS = (
     "odl_fp8_amax_parts_slabs",
     "odl_fp8_cast_delayed_many",
     "odl_fp8_cast_dynamic_colsum",
+    "odl_fp8_slabs_colsum",
     "odl_fp8_swiglu_amax_parts",
     "odl_fp8_swiglu_bwd_amax_parts",
     "odl_fp8_rmsnorm_amax_parts",
@@ -158,6 +159,7 @@ def load() -> ctypes.CDLL:
         L.odl_fp8_multi_cast_delayed.argtypes = [vp, vp, i64, i32, vp]
         L.odl_fp8_cast_delayed_many.argtypes = [vp, i32, i64, i64, i64, i32, vp, i32, vp, vp, vp, vp, vp]
         L.odl_fp8_amax_parts_slabs.argtypes = [vp, i32, i64, i64, vp, vp, vp]
+        L.odl_fp8_slabs_colsum.argtypes = [vp, i32, i64, i64, vp, vp]
         L.odl_fp8_cast_dynamic_colsum.argtypes = [vp, i32, i64, i64, i64, vp, i32, i32, vp, vp, vp, vp, vp, i32, vp]
         L.odl_fp8_amax_parts_colsum.argtypes = [vp, i32, i64, i64, vp, vp, vp, vp]
         L.odl_fp8_swiglu_amax_parts.argtypes = [vp, vp, i64, i64, vp, vp, vp]
@@ -398,9 +400,15 @@ def colsum_supported(x: torch.Tensor) -> bool:
 def amax_parts_colsum(x: torch.Tensor, finish: bool = True, left: "tuple | None" = None):
     """Partial maxima of |x| and the fp32 column sums of x in one pass.  -> (parts, colsum[cols]).  finish=False: the sums stay in
     slabs, a 2-D tensor, for the cast that follows to add up (:func:`cast_dynamic_colsum`); where that cast does not take x they are
-    finished all the same.  left: (parts, slabs) of x that its producer left (:func:`gelu_bwd_slabs`); nothing is launched then."""
-    if left is not None and not finish:
-        return left
+    finished all the same.  left: (parts, slabs) of x that its producer left (:func:`gelu_bwd_slabs`); x is not read then: nothing is
+    launched, or what adds up the slabs (16384 x 8192: 4.5 us, the pass over x 41)."""
+    if left is not None:
+        if not finish:
+            return left
+        r = _host.slabs_colsum(x, left[1], _stream())
+        if r is None:
+            raise NativeError("amax_parts_colsum: the slabs are not those of x")
+        return left[0], _done(r, "odl_fp8_slabs_colsum")
     if x.is_cuda:
         load()
         r = _host.amax_colsum(x, finish, _stream())

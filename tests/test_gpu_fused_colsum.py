@@ -1,5 +1,5 @@
-"""Column sums on the way to a cast (odl_fp8_amax_parts_slabs, odl_fp8_gelu_bwd_slabs, odl_fp8_cast_dynamic_colsum): the codes, the scale
-and the sums are those of the separate launches, bit for bit, at the edges of tiles, slabs and column blocks."""
+"""Column sums on the way to a cast (odl_fp8_amax_parts_slabs, odl_fp8_gelu_bwd_slabs, odl_fp8_cast_dynamic_colsum, odl_fp8_slabs_colsum): the
+codes, the scale and the sums are those of the separate launches, bit for bit, at the edges of tiles, slabs and column blocks."""
 import pytest
 import torch
 
@@ -96,3 +96,66 @@ def test_small_tensor_quantised_in_its_own_place(n, dtype):
     dyn, L = torch.empty(3, device="cuda"), N.load()
     assert L.odl_fp8_quantise_small(x.data_ptr(), 0 if dtype == torch.bfloat16 else 1, n, O.E4M3, 0, x.data_ptr(), dyn.data_ptr(), N._stream()) == 0
     assert torch.equal(x.view(torch.uint8).reshape(-1)[:n], want.reshape(-1)) and dyn[2].item() == inv.item()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols", [(r, c) for r, c, _ in SHAPES])
+def test_sums_finished_by_themselves(rows, cols, dtype):
+    from optimus_dl_amd import native as N
+
+    x = torch.randn((rows, cols), generator=torch.Generator().manual_seed(rows + 2 * cols)).to(dtype).cuda()
+    if not N.colsum_supported(x):
+        pytest.skip("more columns than the pass takes in fp32")
+    _, want = N.amax_parts_colsum(x)
+    left = N.amax_parts_colsum(x, finish=False)
+    parts, sums = N.amax_parts_colsum(x, left=left)
+    assert parts is left[0] and sums.shape == (cols,) and sums.dtype == torch.float32 and torch.equal(sums, want)
+    with pytest.raises(N.NativeError):
+        N.amax_parts_colsum(x, left=(parts, left[1][:1]))
+
+
+@pytest.mark.parametrize("how", ["as stored", "both layouts", "frozen weight", "frozen weight and input", "wgrad off", "no bias", "bf16 Linear"])
+def test_gelu_backward_makes_sums_where_they_are_used(monkeypatch, how):
+    """c_fc behind its GELU: the slabs are made where c_fc has a bias and quantises its gradient or sums it, and used whichever layouts its
+    cast writes; the gradients have the bits they have without them."""
+    from optimus_dl_amd import native as N
+    from optimus_dl_amd.modules import amp, fused
+    from optimus_dl_amd.modules.model.blocks import GELUMLP
+    from optimus_dl_amd.modules.model_transforms import build_model_transform
+
+    n_in, n_out = (2048, 8192) if how == "as stored" else (256, 1024)
+    torch.manual_seed(0)
+    m = build_model_transform({"_name": "fp8_linear"}).apply(GELUMLP(n_in, n_out, bias=how != "no bias").to("cuda", torch.bfloat16))
+    m.c_fc.weight.requires_grad_(not how.startswith("frozen"))
+    m.c_fc.fp8_enabled = how != "bf16 Linear"
+    recipe = amp.FP8Recipe(recipe_type="tensorwise", wgrad=how != "wgrad off")
+    slabs_of, passes = [], []
+    real_slabs, real_pass = N.gelu_bwd_slabs, N.amax_parts_colsum
+
+    def counted(x, *a, left=None, **k):
+        if left is None:
+            passes.append(tuple(x.shape))
+        return real_pass(x, *a, left=left, **k)
+
+    monkeypatch.setattr(N, "gelu_bwd_slabs", lambda *a: (slabs_of.append(1), real_slabs(*a))[1])
+    monkeypatch.setattr(N, "amax_parts_colsum", counted)
+
+    def step():
+        x = (torch.randn((4, 96, n_in), generator=torch.Generator().manual_seed(5))).bfloat16().cuda().requires_grad_("input" not in how)
+        dy = (torch.randn((4, 96, n_in), generator=torch.Generator().manual_seed(6)) * 1e-2).bfloat16().cuda()
+        for p in m.parameters():
+            p.grad = None
+        slabs_of.clear(); passes.clear()
+        with recipe.autocast(), torch.autocast("cuda", torch.bfloat16):
+            y = m(x)
+        with recipe.backward():
+            y.backward(dy)
+        return [x.grad, *(p.grad for p in m.parameters())], len(slabs_of), passes.count((384, n_out))
+
+    got, made, read_again = step()
+    used = how not in ("no bias", "bf16 Linear")
+    assert made == int(used) and read_again == 0
+    monkeypatch.setattr(fused, "_gradient_is_summed", lambda x, recipe: False)
+    want, made, read_again = step()
+    assert made == 0 and read_again == int(used)
+    assert all(a is b is None or torch.equal(a, b) for a, b in zip(got, want, strict=True))

@@ -22,7 +22,13 @@ def test_cast_with_sums(L, src, cols, rows_out, fmt):
     assert L.odl_fp8_cast_dynamic_colsum(P, src, 16, cols, rows_out, P, fmt, 0, P, P, P, P, P, 1, None) != 0
 
 
+@pytest.mark.parametrize("src,rows,cols", [(0, 0, 16), (0, 16, 0), (0, 16, 12), (0, 16, 131080), (1, 16, 6), (1, 16, 65540), (2, 16, 16)])
+def test_sums_of_slabs(L, src, rows, cols):
+    assert L.odl_fp8_slabs_colsum(P, src, rows, cols, P, None) != 0
+
+
 def test_null_pointers(L):
+    assert L.odl_fp8_slabs_colsum(None, 0, 16, 16, P, None) != 0 and L.odl_fp8_slabs_colsum(P, 0, 16, 16, None, None) != 0
     for i in range(5):
         a = [P] * 5
         a[i] = None
