@@ -624,6 +624,7 @@ class _Fp8LinearGroupFn(torch.autograd.Function):
             grads += [dw, db]
         if dx_pairs:
             dx = dx_of(*map(list, zip(*dx_pairs)))
+            dx_pairs.clear()                     # the codes of dy as stored: their memory is free for the weight gradients
         if dw_jobs:
             pol = ctx.subs[0].recipe.recipe
             for at, dw in zip(waiting, _run_jobs(dw_jobs, pol.fmt_bwd, pol.fmt_fwd, ctx.subs[0].w_dtype), strict=True):

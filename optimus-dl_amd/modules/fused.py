@@ -150,10 +150,12 @@ class _SwiGLUMLPFn(torch.autograd.Function):
             elif dxi is not None and pol.kind != "delayed":
                 dx = dx + dxi
             grads.append(dw)
-        if dw_jobs:
-            grads = _run_jobs(dw_jobs, pol.fmt_bwd, pol.fmt_fwd, sub_g.w_dtype)
+        given = None
         if pairs:
             dx = dx_of(*map(list, zip(*pairs)))
+            pairs.clear()                    # the codes of the gradients as stored: their memory is free for the weight gradients
+        if dw_jobs:
+            grads = _run_jobs(dw_jobs, pol.fmt_bwd, pol.fmt_fwd, sub_g.w_dtype)
         for sub in ctx.subs:
             sub.saved_tensors = ()
         return dx, None, None, *grads, dw_d

@@ -120,3 +120,34 @@ def test_mlp_with_its_data_gradient_in_one_launch(N, monkeypatch, kind, tokens):
         assert torch.equal(dx, want)
     else:
         assert (dx.float() - want.float()).abs().max() <= 2.0 ** -7 * want.float().abs().max()
+
+
+@pytest.mark.parametrize("kind", ["tensorwise", "delayed"])
+def test_codes_of_the_data_gradient_are_gone_before_the_weight_gradients(N, monkeypatch, kind):
+    """Both are one launch for gate and up, so the codes of both are there; those as stored are given back behind the first."""
+    from optimus_dl_amd.modules import amp
+    from optimus_dl_amd.modules.model.blocks import SwiGLUMLP
+    from optimus_dl_amd.modules.model_transforms import build_model_transform
+
+    mlp = build_model_transform({"_name": "fp8_linear"}).apply(SwiGLUMLP(1024, 3072).to("cuda", torch.bfloat16))
+    recipe = amp.create_fp8_recipe(kind, "hybrid", amax_history_len=4)
+    seen, chain, group = {}, N.gemm_nt_chain, N.gemm_nt_group
+
+    def data_gradient(a, *args):
+        dx = chain(a, *args)
+        seen["codes"], seen["held"] = sum(t.numel() for t in a), torch.cuda.memory_allocated()
+        return dx
+
+    def products(a, b, fmt_a, *args):
+        if fmt_a == O.E5M2:
+            seen["left"] = torch.cuda.memory_allocated()
+        return group(a, b, fmt_a, *args)
+
+    monkeypatch.setattr(N, "gemm_nt_chain", data_gradient)
+    monkeypatch.setattr(N, "gemm_nt_group", products)
+    x = seeded_bf16((1024, 1024), 1.0, 31).cuda().requires_grad_(True)
+    with recipe.autocast():
+        y = mlp(x)
+    with recipe.backward():
+        y.backward(seeded_bf16(tuple(y.shape), 1e-3, 32).cuda())
+    assert seen["codes"] == 2 * 1024 * 3072 and seen["left"] <= seen["held"] - seen["codes"]
