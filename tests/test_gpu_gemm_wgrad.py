@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n_out,n_in,tokens", [(256, 128, 512), (272, 128, 640), (496, 384, 512), (528, 256, 1152), (12304, 1024, 640), (50304, 768, 1024)])
 def test_weight_gradient_of_rows_that_are_no_whole_tiles(n_out, n_in, tokens, out_dtype):
     """Against the tiled kernel over the transposed copy, which walks K in the same order; what lies behind each operand is NaN, and
-    nothing behind the output is written."""
+    nothing in front of or behind the output is written."""
     from optimus_dl_amd import native as N
 
     g = torch.Generator(device="cuda").manual_seed(n_out + tokens)
@@ -31,6 +31,12 @@ def test_weight_gradient_of_rows_that_are_no_whole_tiles(n_out, n_in, tokens, ou
     finally:
         N.gemm_set_variant(-1)
     assert torch.equal(N.gemm_wgrad(gy, x_t, O.E5M2, O.E4M3, *one, out_dtype), want)
+
+    room = torch.full((n_out + 512, n_in), 3.0, dtype=out_dtype, device="cuda")           # 256 rows each side: a tile's
+    dw = room[256:256 + n_out]
+    assert N.load().odl_fp8_gemm_wgrad(gy.data_ptr(), x_t.data_ptr(), n_out, n_in, tokens, O.E5M2, O.E4M3, one[0].data_ptr(), one[1].data_ptr(),
+                                       dw.data_ptr(), N._OUT_DTYPES[out_dtype], N._stream()) == 0
+    assert torch.equal(dw, want) and bool((room[:256] == 3.0).all()) and bool((room[256 + n_out:] == 3.0).all())
 
 
 def test_weight_gradient_refusals():
