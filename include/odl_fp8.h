@@ -456,7 +456,8 @@ int odl_fp8_gemm_nt_group(int count, const uint8_t *const *a, const uint8_t *con
 /*
  * C[M, N] = the bf16 sum of up to four products with the roundings of one odl_fp8_gemm_nt per product, the second and later ones
  * with accumulate set, in one launch: the data gradient of Linears fed one tensor, where odl_fp8_gemm_nt_sum has no launch for it or
- * its single rounding is not wanted.  sa_inv, sb_inv: one scale per operand.
+ * its single rounding is not wanted.  sa_inv, sb_inv: one scale per operand.  As for odl_fp8_gemm_nt_group the last place of an fp32 sum
+ * in front of a rounding may differ where a product alone takes the thin kernel.
  * Only where odl_fp8_gemm_chain_route gives a variant, that is where it is faster, for 2 to 4 products,
  * every K[s] a multiple of 256 and at least 512, N a multiple of 128, M at least 32, operands under 2 GiB; refused otherwise.
  */

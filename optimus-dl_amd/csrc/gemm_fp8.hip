@@ -613,7 +613,7 @@ static int variant_of(FewTiles few) {
 // Products that a Linear's siblings need side by side (q / k / v, gate / up, and their weight gradients) each leave a last round of
 // tiles part empty, or are too small to fill the chip at all, and each pays a launch's fill and drain.  Together they are one
 // launch of gemm_few_tiles's kernel for all their tiles.  Same K order as alone, so the same bits (fp32 sums of products
-// that alone take the thin kernel add in that kernel's order instead: its error, gemm_fp8.hip).  us one by one / in one launch:
+// that alone take the thin kernel, few rows of a long K, add in this kernel's order instead, to the same error).  us one by one / in one launch:
 //   8192 x (4096, 1024, 1024) x 4096 160.7 / 146.9   2048 x (4096, 1024, 1024) x 4096 64.4 / 44.3   256 x the same 32.1 / 15.7
 //   4016 x (5632, 5632) x 2048 93.2 / 76.9           8192 x (3072, 3072) x 1024 59.8 / 49.9        1024 x the same 14.4 / 11.0
 //   (3072, 3072) x 1024 x 8192 fp32 61.8 / 51.4      (5632, 5632) x 2048 x 4096 fp32 91.3 / 89.9   (14336 x 2) x 4096 x 4096 395 / 369
@@ -698,8 +698,10 @@ extern "C" int odl_fp8_gemm_nt_group(int count, const uint8_t *const *a, const u
 }
 
 // ------------------------------------------------------- products that are added up in one launch
-// What a launch costs that adds its product to C in bf16.  C is read and written once more: 0.45 us a MB where tiles end in an output
-// phase of their own beside other blocks' steps, 0.8 and 1.5 us a step in the 256 x 256 kernels that have one.
+// What a launch costs that adds its product to C in bf16.  C is read once more, in an output phase that nothing overlaps but other
+// blocks: charged with 1 us and 0.4 us a MB in the kernels of 128 rows and 256 x 128 tiles (accumulating less plain, C of 16 to 67 MB, two
+// 128 x 128 blocks a unit 0.2 - 0.5 us a MB, the deep kernels 0.25 - 0.6 and up to 1 at 8192 x 4096 x 3072; under 10 MB 1 - 6 us in all).  The
+// 256 x 256 kernels that have such a phase take 1.5 us a step with cold operands, and 0.8 us a MB.
 static double accumulate_us(int variant, const TileCounts &t, int64_t steps, double c_mb, int cus) {
     if (variant == 4 || variant >= kDeepWideVariant) return launch_us(variant, t, steps, cus) + 1.0 + 0.4 * c_mb;
     return (double)((t.t256 + cus - 1) / cus) * (double)steps * 1.5 + 8.0 + 0.8 * c_mb;
@@ -707,8 +709,8 @@ static double accumulate_us(int variant, const TileCounts &t, int64_t steps, dou
 
 // The kernel for C = sum of products [M, K_s] . [N, K_s]^T in bf16, or kNoVariant: a launch each.
 //
-// gemm_deep.h keeps the sum so far in registers and rounds it behind each product, as launches that accumulate do; us a launch
-// each / together:
+// gemm_deep.h keeps the sum so far in registers and rounds it behind each product, as launches that accumulate do, so the bits are
+// theirs (but where one alone takes the thin kernel: see group_variant); us a launch each / together:
 //   8192 x 1024 x (3072, 3072) 65.8 / 53.7    4016 x 2048 x (5632, 5632) 98.8 / 86.6    1024 x 1024 x (1024, 512, 512) 20.0 / 14.2
 //   5744 x 4096 x (4096, 1024, 1024) 198 / 136 (three rounds of 256 x 128 tiles against the 256 x 256 kernels that accumulate)
 //   8192 x 4096 x (14336, 14336) 718 / 804, 256 x 4096 x (14336, 14336) (thin tiles) 64 / 83: launches of their own

@@ -345,7 +345,9 @@ void launch_gemm_thin(int fa, int fb, const GemmArgs &g, int num_cus, hipStream_
     else launch_thin_fmt<ODL_FP8_E5M2, ODL_FP8_E5M2>(mt, nt, g, stream);
 }
 
-// The columns of a block (eight times nt) with the least operand rows fetched by the busiest compute unit.
+// The columns of a block (eight times nt) with the least operand rows fetched by the busiest compute unit.  The choices are what the
+// widths it was measured at want (3072, 5632, 14336) and steps between; six is not built, though 12288 columns would fill 256 units with
+// it (they take seven: 144 operand rows a step in 220 blocks in place of 128).
 static int swiglu_nt(int mt, int64_t M, int64_t N, int num_cus) {
     static const int choices[] = {1, 2, 3, 4, 5, 7};
     int64_t best = INT64_MAX;

@@ -1464,7 +1464,7 @@ def gemm_wgrad_pays(n_out: int, n_in: int, tokens: int, out_dtype: torch.dtype =
     little slower over dY as stored, and the copy's has other kernels for a last round of few tiles.  Product and cast of dY, both
     layouts where dY is copied, this way / over the copy in us, 2048 and 8192 tokens: 50304 x 768 fp32 142 / 166 and 534 / 676, 12304 x
     1024 bf16 45 / 53 and 135 / 171, 12304 x 3072 96 / 102 and 305 / 319, 32016 x 5632 321 / 337 and 1207 / 1263, 20496 x 5120 204 / 213 and
-    698 / 741 (512 tokens fp32 115.5 / 113.9, the one loss of 90 measured).  On the other side of the line 32016 x 8192 448 / 456 and 1688 /
+    698 / 741 (512 tokens fp32 115.5 / 113.9, the largest loss of 166 measured).  On the other side of the line 32016 x 8192 448 / 456 and 1688 /
     1721, 6160 x 2048 40.5 / 41.2 and 115 / 128, but 8208 x 4096 91 / 89 and 286 / 271, 4112 x 4096 60 / 52 and 183 / 155, 1040 x 14336 54 / 44
     and 169 / 133, 272 x 50304 55 / 49 and 206 / 199.  Where nobody asks for the data gradient both ways cast one layout and are equal
     within 5 %."""
